@@ -20,7 +20,7 @@ inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 inline size_t dtype_bytes(int dtype) { return dtype == JTMOE_F32 ? 4 : 2; }
 inline bool dtype_ok(int dtype) { return dtype == JTMOE_BF16 || dtype == JTMOE_F32; }
 inline bool score_func_ok(int f) { return f == JTMOE_SCORE_SIGMOID || f == JTMOE_SCORE_SOFTMAX; }
-inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+__host__ __device__ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // ---- optional per-stage timing (only jtmoe_moe_forward_timed installs a timer) ----
 enum Stage {
