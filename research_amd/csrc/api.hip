@@ -590,9 +590,10 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
     return fail(JTMOE_EWORKSPACE, "moe_forward: workspace %zu < %zu bytes", workspace_bytes, w.total);
   // where the GEMM can apply the permutation while it fetches its A tiles, the permuted copy of
   // x is never written: dispatch then only computes the histogram, offsets and permutation
-  const bool gather = train || (T > 0 && jtmoe_grouped_swiglu_gather_supported(T, H, I, dtype));
+  const bool no_copy = !train && T > 0 && jtmoe_grouped_swiglu_gather_supported(T, H, I, dtype);
+  const bool gather = train || no_copy || (T > 0 && T * H * (int64_t)dtype_bytes(dtype) < ((int64_t)1 << 30));
   // the workspace of such a shape holds no permuted copy of x to fall back on
-  if (gather && !train &&
+  if (no_copy &&
       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up) |
         reinterpret_cast<uintptr_t>(down)) & 15u) != 0)
     return fail(JTMOE_EINVAL, "moe_forward: x and the expert matrices must be 16-byte aligned");
@@ -633,8 +634,8 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
       rc = jtmoe_grouped_swiglu_train(x, source_order, gate, up, down, group_sizes, offsets, T, K, H, I, E, dtype,
                                       gate_pre, up_pre, w.act, w.packed_y, stream);
     else if (gather)
-      rc = jtmoe_grouped_swiglu_gather(x, source_order, gate, up, down, group_sizes, offsets, T, K, H, I, E, dtype,
-                                       w.act, w.packed_y, stream);
+      rc = launch_swiglu_gather(x, source_order, gate, up, down, group_sizes, offsets, T, K, H, I, E, dtype, w.act,
+                                w.packed_y, main_stream);
     else
       rc = jtmoe_grouped_swiglu(w.packed_x, gate, up, down, group_sizes, offsets, T * K, H, I, E, dtype, w.act,
                                 w.packed_y, stream);

@@ -136,6 +136,12 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
                      int score_func, bool* stats_done, bool* plan_done, hipStream_t stream);
 
 
+// grouped_gemm.hip: the two grouped launches on packed rows fetched through the permutation (packed row j is
+// row source_order[j] / K of x), any shape and alignment as long as x is smaller than 1 GiB.
+int launch_swiglu_gather(const void* x, const int32_t* source_order, const void* gate, const void* up,
+                         const void* down, const int32_t* group_sizes, const int32_t* offsets, int64_t T, int64_t K,
+                         int64_t H, int64_t I, int64_t E, int dtype, void* act, void* packed_y, hipStream_t stream);
+
 // The decode path of the layer (a handful of tokens, nearly every expert chosen by some token).  A tile is
 // 64 rows tall whether it holds an expert's few routed rows or all T <= 64 tokens, so ONE launch runs every
 // token through every expert's gate and up matrices -- act_full [E][T][I], which needs nothing of the

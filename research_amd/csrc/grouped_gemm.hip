@@ -240,7 +240,7 @@ int launch_stream(const void* a, const void* b0, const void* b1, void* c, const 
 // divisor of at most 32
 template <typename Cfg>
 inline bool stream_ok(int64_t rows, int64_t Kdim, int64_t N, const int32_t* row_map, int row_div) {
-  return Kdim % Cfg::BK == 0 && Kdim / Cfg::BK >= 2 * Cfg::NSTAGE && rows * N * 2 <= (int64_t)0x7ffe0000 &&
+  return ((Cfg::OPT & 65536) != 0 || Kdim % Cfg::BK == 0) && (Kdim + Cfg::BK - 1) / Cfg::BK >= 2 * Cfg::NSTAGE && rows * N * 2 <= (int64_t)0x7ffe0000 &&
          (row_map == nullptr || (rows < ((int64_t)1 << 27) && row_div >= 1 && row_div <= 32));
 }
 
@@ -253,7 +253,7 @@ constexpr int64_t kTinyGroupRows = 32;
 inline bool tiny_groups(int64_t rows, int64_t E) { return rows <= kTinyGroupRows * E; }
 
 inline bool fast_ok(const void* a, const void* b0, const void* b1, const void* c, int64_t Kdim, int64_t N) {
-  return Kdim % 64 == 0 && N % 8 == 0 && Kdim * N < ((int64_t)1 << 30) && aligned16(a) && aligned16(b0) && (b1 == nullptr || aligned16(b1)) &&
+  return Kdim % 8 == 0 && N % 8 == 0 && Kdim * N < ((int64_t)1 << 30) && aligned16(a) && aligned16(b0) && (b1 == nullptr || aligned16(b1)) &&
          aligned16(c);
 }
 
@@ -275,8 +275,14 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
          : stream_ok<GateUpStreamCfg>(rows, H, I, row_map, row_div)
              ? launch_stream<GateUpStreamCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
                                               row_div, x_rows, save_gate, save_up)
-             : launch_fast<GateUpCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
-                                      row_div, x_rows, save_gate, save_up);
+         : stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div)
+             ? launch_stream<GateUpStreamTailCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
+                                                  row_div, x_rows, save_gate, save_up)
+         : H % 64 == 0
+             ? launch_fast<GateUpCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map, row_div,
+                                      x_rows, save_gate, save_up)
+             : launch_fast<GateUpTailCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
+                                          row_div, x_rows, save_gate, save_up);
   else
     rc = launch_generic<T, true>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map, row_div,
                                  save_gate, save_up);
@@ -285,7 +291,8 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
   if (Elem<T>::is_bf16 && fast_ok(act, down, nullptr, y, I, H))
     rc = tiny    ? launch_fast<DownTinyCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream)
          : small ? launch_fast<DownSmallCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream)
-                 : launch_fast<DownCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream);
+         : I % 64 == 0 ? launch_fast<DownCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream)
+                       : launch_fast<DownTailCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream);
   else
     rc = launch_generic<T, false>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream);
   if (rc) return rc;
@@ -312,6 +319,19 @@ int launch_down_from_all_tokens(const void* act_full, const void* down, const in
     return fail(JTMOE_EINVAL, "moe_forward: operands must be 16-byte aligned");
   return launch_fast<DownTinyCfg>(act_full, down, nullptr, packed_y, group_sizes, offsets, T * K, I, H, E, stream,
                                   source_order, (int)K, T, nullptr, nullptr, 0, /*a_group_rows=*/T);
+}
+
+// ---- the gathering launch pair as the layer uses it (declared in common.hpp) ----
+int launch_swiglu_gather(const void* x, const int32_t* source_order, const void* gate, const void* up,
+                         const void* down, const int32_t* group_sizes, const int32_t* offsets, int64_t T, int64_t K,
+                         int64_t H, int64_t I, int64_t E, int dtype, void* act, void* packed_y, hipStream_t stream) {
+  const int rc = validate_gemm("grouped_swiglu_gather", T * K, H, I, E, dtype);
+  if (rc) return rc;
+  if (dtype == JTMOE_BF16)
+    return launch_pair<bf16_raw>(x, gate, up, down, group_sizes, offsets, T * K, H, I, E, act, packed_y, stream,
+                                 kStageGateUp, source_order, (int)K, T);
+  return launch_pair<float>(x, gate, up, down, group_sizes, offsets, T * K, H, I, E, act, packed_y, stream,
+                            kStageGateUp, source_order, (int)K, T);
 }
 
 }  // namespace jtmoe
@@ -371,8 +391,8 @@ extern "C" int jtmoe_grouped_swiglu_gather(const void* x, const int32_t* source_
     return fail(JTMOE_EUNSUPPORTED,
                 "grouped_swiglu_gather: needs bf16, H and I multiples of 64 and 16-byte aligned rows "
                 "(use jtmoe_dispatch + jtmoe_grouped_swiglu otherwise)");
-  return launch_pair<bf16_raw>(x, gate, up, down, group_sizes, offsets, A, H, I, E, act, packed_y, as_stream(stream),
-                               kStageGateUp, source_order, (int)K, T);
+  return launch_swiglu_gather(x, source_order, gate, up, down, group_sizes, offsets, T, K, H, I, E, dtype, act,
+                              packed_y, as_stream(stream));
 }
 
 // Forward pass that keeps what the backward pass needs: the two rounded products

@@ -144,6 +144,29 @@ hipError_t allow_lds(Kernel kernel, size_t bytes) {
 
 constexpr int64_t kOperandLimit = (int64_t)1 << 30;  // elements: byte offsets stay below 2^31
 
+template <typename Cfg>
+int launch_nt_fast(const void* a0, const void* a1, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
+                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, const int32_t* row_map,
+                   int row_div, int64_t a_rows, int segs, hipStream_t stream) {
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  auto kernel = grouped_gemm_nt_kernel<Cfg>;
+  std::call_once(once, [&] { attr_err = allow_lds(kernel, Cfg::SMEM_BYTES); });
+  if (attr_err != hipSuccess)
+    return fail(JTMOE_ELAUNCH, "grouped gemm (nt): hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
+  const int64_t mtiles = group_sizes == nullptr ? (rows + Cfg::BM - 1) / Cfg::BM : max_m_tiles(rows, E, Cfg::BM);
+  const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
+  const int64_t tiles_grid = gemm_grid(mtiles, nt);
+  if (tiles_grid >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");
+  // persistent workgroups: one per CU, each walking its share of the tiles
+  const int64_t grid = tiles_grid > persistent_grid_size() ? persistent_grid_size() : tiles_grid;
+  kernel<<<(unsigned)grid, Cfg::NT, Cfg::SMEM_BYTES, stream>>>(
+      static_cast<const uint16_t*>(a0), static_cast<const uint16_t*>(a1), static_cast<const uint16_t*>(b0),
+      static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim,
+      (int)N, (int)mtiles, (int)nt, row_map, row_div, (int)a_rows, segs);
+  return JTMOE_OK;
+}
+
 }  // namespace
 
 int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, const void* b1, void* c,
@@ -151,29 +174,15 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
                    int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream) {
   if (rows == 0) return JTMOE_OK;
   const bool dense = group_sizes == nullptr;
-  const bool fast = dtype == JTMOE_BF16 && Kdim % 64 == 0 && N % 8 == 0 && N * Kdim < kOperandLimit &&
+  const bool fast = dtype == JTMOE_BF16 && Kdim % 8 == 0 && N % 8 == 0 && N * Kdim < kOperandLimit &&
                     (row_map ? a_rows : rows) * Kdim < kOperandLimit && aligned16(a0) && aligned16(b0) &&
                     (segs == 1 || (aligned16(a1) && aligned16(b1))) && aligned16(c);
-  if (fast) {
-    using Cfg = DgradCfg;
-    static std::once_flag once;
-    static hipError_t attr_err = hipSuccess;
-    auto kernel = grouped_gemm_nt_kernel<Cfg>;
-    std::call_once(once, [&] { attr_err = allow_lds(kernel, Cfg::SMEM_BYTES); });
-    if (attr_err != hipSuccess)
-      return fail(JTMOE_ELAUNCH, "grouped gemm (nt): hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
-    const int64_t mtiles = dense ? (rows + Cfg::BM - 1) / Cfg::BM : max_m_tiles(rows, E, Cfg::BM);
-    const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
-    const int64_t tiles_grid = gemm_grid(mtiles, nt);
-    if (tiles_grid >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");
-    // persistent workgroups: one per CU, each walking its share of the tiles
-    const int64_t grid = tiles_grid > persistent_grid_size() ? persistent_grid_size() : tiles_grid;
-    kernel<<<(unsigned)grid, Cfg::NT, Cfg::SMEM_BYTES, stream>>>(
-        static_cast<const uint16_t*>(a0), static_cast<const uint16_t*>(a1), static_cast<const uint16_t*>(b0),
-        static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows,
-        (int)Kdim, (int)N, (int)mtiles, (int)nt, row_map, row_div, (int)a_rows, segs);
-    return JTMOE_OK;
-  }
+  if (fast && Kdim % 64 == 0)
+    return launch_nt_fast<DgradCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div,
+                                    a_rows, segs, stream);
+  if (fast)
+    return launch_nt_fast<DgradTailCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div,
+                                        a_rows, segs, stream);
   const int64_t mtiles = dense ? (rows + QB - 1) / QB : max_m_tiles(rows, E, QB);
   const int64_t nt = (N + QB - 1) / QB;
   if (mtiles * nt >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");

@@ -18,7 +18,9 @@
 // row_map[j] / row_div), the way the forward gate/up launch does, so neither the
 // permuted activations nor the permuted output gradient are ever written to memory.
 //
-// Requirements: bf16, K % 64 == 0 (NT), row lengths multiples of 8, 16-byte aligned
+// NT: with OPT & 65536 K need not be a multiple of the 64-deep step (chunks past the end of a row read as zeros).
+//
+// Requirements: bf16, K % 8 == 0 (NT), row lengths multiples of 8, 16-byte aligned
 // pointers, every operand smaller than 2 GiB.
 #pragma once
 
@@ -141,7 +143,8 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_nt_kernel(
   };
   const unsigned lds0 = lds_byte_addr(smem_raw);
   const unsigned wave_lds = lds0 + wave * 1024;
-  const int nk1 = Kdim / BK;
+  constexpr bool kTail = (Cfg::OPT & 65536) != 0;  // K may end inside a step
+  const int nk1 = kTail ? (Kdim + BK - 1) / BK : Kdim / BK;
   const int nk = nk1 * segs;
 
   auto issue = [&](int kt) {
@@ -150,11 +153,15 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_nt_kernel(
     const int k0 = (second ? kt - nk1 : kt) * BK;
     const i32x4_t ar = second ? a_rsrc[1] : a_rsrc[0];
     const i32x4_t br = second ? b_rsrc[1] : b_rsrc[0];
+    // the last step of a K that is no multiple of 64: this lane's chunk lies past the end of the row
+    const bool outside = kTail && k0 + BK > Kdim && k0 + l_c * 8 >= Kdim;
 #pragma unroll
-    for (int j = 0; j < Cfg::A_LOADS; ++j) buffer_load_lds16(ar, base + j * NT * 16, a_voff[j], k0 * 2);
+    for (int j = 0; j < Cfg::A_LOADS; ++j)
+      buffer_load_lds16(ar, base + j * NT * 16, outside ? kOutside : a_voff[j], k0 * 2);
 #pragma unroll
     for (int j = 0; j < Cfg::B_LOADS; ++j)
-      buffer_load_lds16(br, base + Cfg::A_BYTES + j * NT * 16, b_voff + j * (NT / 8) * Kdim * 2, k0 * 2);
+      buffer_load_lds16(br, base + Cfg::A_BYTES + j * NT * 16, outside ? kOutside : b_voff + j * (NT / 8) * Kdim * 2,
+                        k0 * 2);
   };
 
   const int sw = ((lane & 31) >> 1) & 7;
@@ -734,6 +741,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_tn_kernel(
 
 // Configurations the library launches.
 using DgradCfg = NtGemmCfg<256, 256, 2, 4, 16 + 64 + 32768>;   // data gradients: 256 x 256 tiles
+using DgradTailCfg = NtGemmCfg<256, 256, 2, 4, 16 + 64 + 32768 + 65536>;  // the same for K % 64 != 0
 // narrow LDS blocks: the fastest layout when the operands are streamed (1.52 vs 1.60 ms for the
 // gate/up product of the C3 shape); the wide blocks pay off only when rows are gathered.
 // Four stages of 32 rows against two of 64 (the same LDS): 1.39-1.43 against 1.47-1.49 ms for the gate/up

@@ -25,7 +25,14 @@
 // and computes.  The loads are issued from inline assembly because the compiler
 // would otherwise drain every outstanding load before each LDS read.
 //
-// Requirements: K % BK == 0, N % 8 == 0, 16-byte aligned pointers, K*N*2 < 2^31.
+// K need not be a multiple of the step: the chunks of A past the end of a row are not fetched but read as
+// zeros (they would be the next row's first elements), and B has no rows there (its descriptor ends with
+// the matrix).  The 64-row kernel checks once per step; the persistent and the stream kernel have variants of
+// their own (OPT & 65536), because the check costs registers that the others do not have to spare.  Before,
+// such widths ran element by element in the generic kernel: 2931 x 3 rows, 1000 x 2664, 24 experts with a
+// shared expert took 1122 + 967 us (routed) and 415 + 464 us (shared), now 122 + 81 and 36 + 64 us.
+//
+// Requirements: K % 8 == 0, N % 8 == 0, 16-byte aligned pointers, K*N*2 < 2^31.
 #pragma once
 
 #include "gemm_common.hpp"
@@ -85,6 +92,9 @@ __device__ __forceinline__ float silu_rcp(float g) {
   return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
 }
 
+// a byte offset outside every operand (all are smaller than 2 GiB): such a load stores zeros
+constexpr int kOutside = (int)0x80000000u;
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -106,7 +116,8 @@ struct DmaGemmCfg {
   // scheduling options: 16 = request the fragments of MFMA step kk+1 before issuing step kk,
   // 32 = raise the wave priority around the MFMA burst, 64 = ask the scheduler to interleave
   // one MFMA with up to three LDS reads, 128 = B tiles in 4 x 64 blocks, 2048 = (persistent kernel) results written
-  // straight from transposed accumulators instead of through LDS, 4096 = non-temporal loads of B, 8192 / 16384 = 8 / 2 m-tiles per group of the tile order instead of 4, 32768 = non-temporal stores of the result
+  // straight from transposed accumulators instead of through LDS, 4096 = non-temporal loads of B, 8192 / 16384 = 8 / 2 m-tiles per group of the tile order instead of 4, 32768 = non-temporal stores of the result,
+  // 65536 = (persistent and stream kernels) K may end inside a step
   static constexpr int OPT = OPT_;
   static constexpr bool kDual = kDual_;
   static constexpr int BNE = kDual ? 2 * BN : BN;  // columns of the B tile in LDS
@@ -333,19 +344,23 @@ __device__ __forceinline__ void grouped_gemm_dma_tile(
   auto issue = [&](int kt) {
     const unsigned base = wave_lds + (kt % NSTAGE) * Cfg::STAGE_BYTES;
     const int k0 = kt * BK;
+    const bool ragged = k0 + BK > Kdim;  // uniform: the last step of a K that is no multiple of BK
+    const bool a_outside = ragged && k0 + a_c * 8 >= Kdim;
 #pragma unroll
     for (int j = 0; j < Cfg::A_LOADS; ++j)
-      buffer_load_lds16(a_rsrc, base + j * NT * 16, a_voff[j], k0 * 2);
+      buffer_load_lds16(a_rsrc, base + j * NT * 16, a_outside ? kOutside : a_voff[j], k0 * 2);
+    // (the whole offset in the vector part where rows past the end of B have to be recognised)
+    const int b_soff = ragged ? 0 : k0 * N * 2, b_extra = ragged ? k0 * N * 2 : 0;
 #pragma unroll
     for (int u = 0; u < Cfg::NSUB; ++u)
 #pragma unroll
       for (int j = 0; j < Cfg::BSUB_LOADS; ++j) {
         if (Cfg::OPT & 4096)
           buffer_load_lds16_nt(b_rsrc[u], base + Cfg::A_BYTES + u * Cfg::BSUB_BYTES + j * NT * 16,
-                               b_voff[u] + j * (NT / 16) * N * 2, k0 * N * 2);
+                               b_voff[u] + j * (NT / 16) * N * 2 + b_extra, b_soff);
         else
           buffer_load_lds16(b_rsrc[u], base + Cfg::A_BYTES + u * Cfg::BSUB_BYTES + j * NT * 16,
-                            b_voff[u] + j * (NT / 16) * N * 2, k0 * N * 2);
+                            b_voff[u] + j * (NT / 16) * N * 2 + b_extra, b_soff);
       }
   };
 
@@ -398,7 +413,7 @@ __device__ __forceinline__ void grouped_gemm_dma_tile(
     }
   };
 
-  const int nk = Kdim / BK;
+  const int nk = (Kdim + BK - 1) / BK;
   // The last tile of a group is usually partly empty.  A wave whose WM rows all lie past the end of
   // the group (or whose columns all lie past N) still takes part in the loads and the barriers but
   // skips its fragment reads and MFMAs.
@@ -541,6 +556,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_dma_persistent_kernel(
   static_assert(Cfg::NSTAGE == 2, "two stages");
   // results straight from (transposed) accumulators: the weight fragment is the MFMA's first operand
   constexpr bool kDirect = (Cfg::OPT & 2048) != 0;
+  constexpr bool kTail = (Cfg::OPT & 65536) != 0;  // K may end inside a step (costs registers: 11 spilled in DownCfg)
   extern __shared__ __align__(16) unsigned char smem_raw[];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -632,14 +648,18 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_dma_persistent_kernel(
   auto issue = [&](int kt) {
     const unsigned base = wave_lds + (kt & 1) * Cfg::STAGE_BYTES;
     const int k0 = kt * BK;
+    const bool ragged = kTail && k0 + BK > Kdim;
+    const bool a_outside = ragged && k0 + a_c * 8 >= Kdim;
 #pragma unroll
-    for (int j = 0; j < Cfg::A_LOADS; ++j) buffer_load_lds16(a_rsrc, base + j * NT * 16, a_voff[j], k0 * 2);
+    for (int j = 0; j < Cfg::A_LOADS; ++j)
+      buffer_load_lds16(a_rsrc, base + j * NT * 16, a_outside ? kOutside : a_voff[j], k0 * 2);
+    const int b_soff = ragged ? 0 : k0 * N * 2, b_extra = ragged ? k0 * N * 2 : 0;
 #pragma unroll
     for (int u = 0; u < Cfg::NSUB; ++u)
 #pragma unroll
       for (int j = 0; j < Cfg::BSUB_LOADS; ++j)
         buffer_load_lds16(b_rsrc[u], base + Cfg::A_BYTES + u * Cfg::BSUB_BYTES + j * NT * 16,
-                          b_voff[u] + j * (NT / 16) * N * 2, k0 * N * 2);
+                          b_voff[u] + j * (NT / 16) * N * 2 + b_extra, b_soff);
   };
 
   // ---- fragment addresses of this lane (the same for every tile) ----
@@ -680,7 +700,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_dma_persistent_kernel(
     }
   };
 
-  const int nk = Kdim / BK;
+  const int nk = kTail ? (Kdim + BK - 1) / BK : Kdim / BK;
   constexpr int TNO = Cfg::TNO, WNO = Cfg::WNO, CS = Cfg::CS;
   // Epilogue staging lives above the first stage buffer, which the next tile's first loads fill
   // while the epilogue runs.  If a wave's block does not fit its share, it goes out in two halves.
@@ -815,12 +835,14 @@ inline PersistentSchedule persistent_schedule(int64_t tiles_grid, int cus, int t
 // tile: 128 + 128 columns), 64-deep k steps, two LDS stages, 8 waves, B tiles in 4 x 64 blocks
 // (whole 128-byte lines per eight lanes; about 1 % faster than 4 x 16 blocks at 131072 rows).
 using GateUpCfg = DmaGemmCfg<256, 128, 64, 4, 2, true, 2, 16 + 128>;
+using GateUpTailCfg = DmaGemmCfg<256, 128, 64, 4, 2, true, 2, 16 + 128 + 65536>;  // for K % 64 != 0
 // tiles per workgroup of a persistent launch (0: one workgroup per CU walks them all).  The down
 // projection measures 0.8 % faster fully persistent (and sheds 7 % of its L2 misses with 4); gate/up
 // runs as fast either way and sheds a quarter of them.
 template <typename Cfg>
 constexpr int kTilesPerWorkgroup = Cfg::kDual ? 4 : 0;
 using DownCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 64 + 128 + 32768>;  // 537 MB of results at C3: streamed out
+using DownTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 64 + 128 + 32768 + 65536>;
 // Few rows per group (decode-sized batches): the layer streams every expert matrix once and
 // is bound by HBM, so the tiles are only 64 rows tall to keep the padded-row MFMA work below
 // the time the weights take to arrive, and the k steps 32 deep so that four workgroups of four

@@ -16,7 +16,7 @@
 //     row map of the next tile arrives by LDS-DMA as well, group sizes and offsets are read from a copy
 //     in LDS), so the compiler never inserts a wait that drains the operand loads.
 //
-// Requirements: those of grouped_gemm_dma.hpp, and K / BK >= 2 * NSTAGE, a result of at most 0x7ffe0000
+// Requirements: those of grouped_gemm_dma.hpp, K % BK == 0 unless OPT & 65536, K / BK >= 2 * NSTAGE, a result of at most 0x7ffe0000
 // bytes, with a row map fewer than 2^27 rows and row_div <= 32; launch with a multiple of 8 workgroups
 // (persistent schedule).
 #pragma once
@@ -66,6 +66,9 @@ __device__ __forceinline__ void stream_gemm_body(
   static_assert(KK % 2 == 0, "fragment double buffer wants an even number of sub-steps");
   static_assert(kNT || (Cfg::OPT & 128) != 0, "weight tiles in 4 x 64 blocks");
   static_assert(!kNT || !kDual, "the transposed-B form has one output per tile");
+  // K may end inside a step (the interleaved steady part leaves no room for a branch: every load checks)
+  constexpr bool kTail = (Cfg::OPT & 65536) != 0;
+  static_assert(!kTail || !kNT, "the transposed-B form takes whole steps");
   static_assert(!kNT || (BN * CPRA) % NT == 0, "the B tile must divide evenly over the threads");
   // Timing experiments of the stand-alone check's time_ablation mode, which bounds what any schedule of
   // this loop can reach (wrong results by construction, never launched by the library): OPT & 256 leaves out the operand loads of the steady part of the k loop, OPT & 512 its
@@ -80,7 +83,7 @@ __device__ __forceinline__ void stream_gemm_body(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WAVES_N, wn = wave - wm * Cfg::WAVES_N;
   const bool gather = row_map != nullptr;
-  const int nk1 = Kdim / BK;               // k steps of one segment
+  const int nk1 = kTail ? (Kdim + BK - 1) / BK : Kdim / BK;  // k steps of one segment
   const int nk = kNT ? nk1 * segs : nk1;   // k steps of a tile
 
   // ---- schedule (as in grouped_gemm_dma_persistent_kernel) ----
@@ -207,11 +210,12 @@ __device__ __forceinline__ void stream_gemm_body(
     } else {
       const int k0 = kt * BK;
       if (i < Cfg::A_LOADS) {
-        buffer_load_lds16(p.a_rsrc[0], base + i * NT * 16, p.a_voff[i], k0 * 2);
+        buffer_load_lds16(p.a_rsrc[0], base + i * NT * 16, kTail && k0 + a_c * 8 >= Kdim ? kOutside : p.a_voff[i],
+                          k0 * 2);
       } else {
         const int u = (i - Cfg::A_LOADS) / Cfg::BSUB_LOADS, jb = (i - Cfg::A_LOADS) % Cfg::BSUB_LOADS;
         buffer_load_lds16(p.b_rsrc[u], base + Cfg::A_BYTES + u * Cfg::BSUB_BYTES + jb * NT * 16,
-                          p.b_voff[u] + jb * (NT / 16) * N * 2, k0 * N * 2);
+                          p.b_voff[u] + jb * (NT / 16) * N * 2 + (kTail ? k0 * N * 2 : 0), kTail ? 0 : k0 * N * 2);
       }
     }
   };
@@ -440,6 +444,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_nt_kernel(
 // (alternating in one process): 1.306 ms against 1.400-1.409 ms for grouped_gemm_dma_persistent_kernel
 // and 1.315-1.320 ms for 64-deep steps with two stages.
 using GateUpStreamCfg = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128>;
+using GateUpStreamTailCfg = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 65536>;  // for K % 32 != 0
 // Variants kept for the stand-alone check and its timings (time_stream, time_down): 64-deep steps with
 // two stages, and the down projection's tile (within 2 % of grouped_gemm_dma_persistent_kernel, which
 // the library keeps for that launch, at 12, 22 and 44 k steps per tile).
