@@ -26,4 +26,20 @@ int launch_gemm_tn(int dtype, const void* p, const void* d0, const void* d1, voi
                    hipStream_t stream, void* split_ws = nullptr);
 size_t gemm_tn_split_bytes(int dtype, int64_t rows, int64_t KA, int64_t N, bool dual);
 
+// Single precision on the matrix cores (grouped_gemm_f32.hip): K and N multiples of 4, 16-byte aligned
+// operands (null ones count as aligned), operands below 2 GiB.  a_rows: rows of the gathered matrix with a row
+// map, else `rows`.  NN with b1: gate and up with the SwiGLU (and the two products in save0 / save1).
+bool f32_gemm_supported(const void* a0, const void* a1, const void* b0, const void* b1, const void* c, int64_t a_rows,
+                        int64_t Kdim, int64_t N);
+int launch_f32_nn(const void* a, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
+                  const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, const int32_t* row_map,
+                  int row_div, int64_t a_rows, void* save0, void* save1, hipStream_t stream);
+int launch_f32_nt(const void* a0, const void* a1, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
+                  const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, const int32_t* row_map,
+                  int row_div, int64_t a_rows, int segs, hipStream_t stream);
+int launch_f32_tn(const void* p, const void* d0, const void* d1, void* c0, void* c1, const int32_t* group_sizes,
+                  const int32_t* offsets, int64_t rows, int64_t KA, int64_t N, int64_t E, void* split_ws,
+                  hipStream_t stream);
+size_t f32_tn_split_bytes(int64_t rows, int64_t KA, int64_t N, bool dual);
+
 }  // namespace jtmoe

@@ -10,6 +10,7 @@
 // are accumulated in fp32 on the matrix cores (v_mfma_f32_32x32x16_bf16 for
 // bf16, v_mfma_f32_32x32x2_f32 for fp32).
 #include "common.hpp"
+#include "gemm_launch.hpp"
 #include "grouped_gemm_dma.hpp"
 #include "grouped_gemm_stream.hpp"
 
@@ -283,6 +284,10 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
                                       x_rows, save_gate, save_up)
              : launch_fast<GateUpTailCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
                                           row_div, x_rows, save_gate, save_up);
+  else if (!Elem<T>::is_bf16 && f32_gemm_supported(x, save_gate, gate, up, act, row_map ? x_rows : rows, H, I) &&
+           aligned16(save_up))
+    rc = launch_f32_nn(x, gate, up, act, group_sizes, offsets, rows, H, I, E, row_map, row_div, x_rows, save_gate,
+                       save_up, stream);
   else
     rc = launch_generic<T, true>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map, row_div,
                                  save_gate, save_up);
@@ -293,6 +298,9 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
          : small ? launch_fast<DownSmallCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream)
          : I % 64 == 0 ? launch_fast<DownCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream)
                        : launch_fast<DownTailCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream);
+  else if (!Elem<T>::is_bf16 && f32_gemm_supported(act, nullptr, down, nullptr, y, rows, I, H))
+    rc = launch_f32_nn(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, nullptr, 1, 0, nullptr, nullptr,
+                       stream);
   else
     rc = launch_generic<T, false>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream);
   if (rc) return rc;

@@ -183,6 +183,10 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
   if (fast)
     return launch_nt_fast<DgradTailCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div,
                                         a_rows, segs, stream);
+  if (dtype == JTMOE_F32 && f32_gemm_supported(a0, a1, b0, b1, c, row_map ? a_rows : rows, Kdim, N) &&
+      !(row_map && segs > 1))
+    return launch_f32_nt(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div, a_rows, segs,
+                         stream);
   const int64_t mtiles = dense ? (rows + QB - 1) / QB : max_m_tiles(rows, E, QB);
   const int64_t nt = (N + QB - 1) / QB;
   if (mtiles * nt >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");
@@ -341,6 +345,9 @@ int launch_gemm_tn(int dtype, const void* p, const void* d0, const void* d1, voi
     return launch_tn_fast<WgradCfg>(p, d0, nullptr, c0, nullptr, group_sizes, offsets, rows, KA, N, E, nullptr, 1,
                                     false, false, 0, stream, split_ws);
   }
+  if (dtype == JTMOE_F32 && !p_gather && !d_gather && f32_gemm_supported(p, d0, d1, c0, c1, rows, KA, N) &&
+      rows * N < ((int64_t)1 << 29))
+    return launch_f32_tn(p, d0, d1, c0, c1, group_sizes, offsets, rows, KA, N, E, split_ws, stream);
   const int64_t mt = (KA + QB - 1) / QB, nt = (N + QB - 1) / QB;
   if (E * mt * nt >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (tn): grid too large");
   for (int i = 0; i < (dual ? 2 : 1); ++i) {
@@ -359,7 +366,8 @@ int launch_gemm_tn(int dtype, const void* p, const void* d0, const void* d1, voi
 }
 
 size_t gemm_tn_split_bytes(int dtype, int64_t rows, int64_t KA, int64_t N, bool dual) {
-  if (dtype != JTMOE_BF16 || KA % 8 != 0 || N % 8 != 0) return 0;
+  if (dtype == JTMOE_F32) return f32_tn_split_bytes(rows, KA, N, dual);
+  if (KA % 8 != 0 || N % 8 != 0) return 0;
   const SplitPlan plan = dual ? split_plan<WgradDualCfg>(rows, KA, N) : split_plan<WgradCfg>(rows, KA, N);
   if (plan.splits == 0) return 0;
   return align_up((size_t)plan.splits * KA * N * sizeof(float) * (dual ? 2 : 1), 256);

@@ -1,0 +1,319 @@
+// Single-precision grouped GEMMs on v_mfma_f32_32x32x2_f32 (inputs, sums and results in fp32):
+//
+//   "NN"  C[rows of e, :] = A[rows of e, :] @ B[e]            B[e] [K, N]      (forward products; kDual: gate and
+//         up share the A tile and the SwiGLU runs in the epilogue)
+//   "NT"  C[rows of e, :] = sum over segments A_s[rows of e, :] @ B_s[e]^T,    B_s[e] [N, K]   (data gradients)
+//   "TN"  C[e] = P[rows of e, :]^T @ D[rows of e, :]                           (weight gradients)
+//
+// Bound: the fp32 matrix rate (157 TFLOP/s: 64 cycles per 32 x 32 x 2 product), sixteen times below bf16's, so
+// operand traffic is cheap by comparison and the design only has to keep every SIMD's matrix core busy: four
+// waves (2 x 2) per workgroup, 32-deep k steps, two LDS stages filled by buffer_load ... lds while the other is
+// multiplied, and two to four workgroups per CU so that one's barrier runs under another's products.  A step
+// of a 64 x 64 wave tile is 4096 matrix cycles against 16 ds_read_b128 and 64 ds_read_b32.
+// k-contiguous tiles (A, and B of NT) hold rows of eight 16-byte chunks, chunk c of row r in slot
+// c ^ ((r / 2) % 8), and one ds_read_b128 feeds four MFMAs (lane half h takes k = 8 q + 4 h + i in product i:
+// any assignment of k to products serves as long as both operands use it).  Row-major tiles ([k][n]) are read
+// one word per MFMA, 32 consecutive words per half wave.
+// Two tile heights and widths (128 and 64): the launcher takes the one with the fewer rounds over the CUs.
+// Three or four stages instead of two measured the same or slower (101 / 108 / 129 us for the gate/up product
+// below): the loads arrive in time, and the LDS is better spent on more workgroups per CU.
+// Measured at 4096 rows in 8 groups, 512 x 1024: gate/up 199 -> 100 us, down 211 -> 61, data gradients
+// 143 -> 54 and 424 -> 115, weight gradients 147 -> 47 and 154 + 145 -> 83 (one launch); 52 to 103 TFLOP/s of
+// matrix work where the element-wise staged kernels, which still take other widths, reached 10 to 59.  What is
+// left is the last, partly filled round and the fixed cost of launches this short.
+//
+// Requirements: K, N (KA) multiples of 4, 16-byte aligned pointers, operands of a group below 2 GiB.
+#pragma once
+
+#include "grouped_gemm_dma.hpp"
+
+namespace jtmoe {
+
+template <int BM_, int BN_, bool kDual_, bool kBT_>
+struct F32Cfg {
+  static constexpr int BM = BM_, BN = BN_, BK = 32, NT = 256;
+  static constexpr bool kDual = kDual_, kBT = kBT_;
+  static constexpr int NSUB = kDual ? 2 : 1;           // matrices per B tile
+  static constexpr int TM = BM / 64, TN = NSUB * BN / 64;  // 32 x 32 blocks per wave
+  static constexpr int A_BYTES = BM * BK * 4, B_BYTES = BN * BK * 4;
+  static constexpr int STAGE_BYTES = A_BYTES + NSUB * B_BYTES;
+  static constexpr int SMEM_BYTES = 2 * STAGE_BYTES;
+  static constexpr int A_LOADS = BM * 8 / NT, B_LOADS = BN * 8 / NT;
+  static constexpr int GROUP_M = 4;
+  static_assert(BM % 64 == 0 && BN % 64 == 0 && !(kDual && (kBT || BN != 64)), "2 x 2 waves of 32 x 32 blocks");
+};
+
+// 16 bytes per lane into LDS at base + lane * 16; the whole offset in the vector part (ends of rows and
+// matrices are recognised by the descriptor's bound)
+__device__ __forceinline__ void f32_load(i32x4_t rsrc, unsigned base, int voffset) {
+  buffer_load_lds16(rsrc, base, voffset, 0);
+}
+
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) void grouped_gemm_f32_kernel(
+    const float* __restrict__ A0, const float* __restrict__ A1, const float* __restrict__ B0,
+    const float* __restrict__ B1, float* __restrict__ C, const int32_t* __restrict__ group_sizes,
+    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n,
+    const int32_t* __restrict__ row_map, int row_div, int a_rows, int segs, float* __restrict__ save0,
+    float* __restrict__ save1) {
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, TM = Cfg::TM, TN = Cfg::TN;
+  constexpr bool kDual = Cfg::kDual, kBT = Cfg::kBT;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+
+  TileCoord tc;
+  TileRows tr;
+  if (group_sizes) {
+    const GroupScan scan = group_scan(BM, group_sizes, E);
+    tc = xcd_tile_order_balanced(scan.total, ntiles_n, Cfg::GROUP_M);
+    if (tc.mt < 0) return;
+    tr = locate_tile(scan, tc.mt, BM, offsets);
+  } else {
+    tc = xcd_tile_order(mtiles, ntiles_n, Cfg::GROUP_M);
+    if (tc.mt < 0) return;
+    tr = find_tile_wave(tc.mt, BM, nullptr, nullptr, E, dense_rows);
+  }
+  tr.expert = __builtin_amdgcn_readfirstlane(tr.expert);
+  tr.row0 = __builtin_amdgcn_readfirstlane(tr.row0);
+  tr.rows = __builtin_amdgcn_readfirstlane(tr.rows);
+  if (tr.rows <= 0) return;
+  const int n0 = tc.nt * BN;
+  const size_t wofs = (size_t)tr.expert * Kdim * N;
+
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const bool gather = row_map != nullptr;
+
+  // ---- load plan ----
+  const i32x4_t a_rsrc0 = gather ? make_rsrc(A0, a_rows * Kdim * 4) : make_rsrc(A0 + (size_t)tr.row0 * Kdim, tr.rows * Kdim * 4);
+  const i32x4_t a_rsrc1 = segs > 1 ? make_rsrc(A1 + (size_t)tr.row0 * Kdim, tr.rows * Kdim * 4) : a_rsrc0;
+  const i32x4_t b_rsrc0 = make_rsrc(B0 + wofs, Kdim * N * 4);
+  const i32x4_t b_rsrc1 = (kDual || segs > 1) ? make_rsrc(B1 + wofs, Kdim * N * 4) : b_rsrc0;
+  // k-contiguous tiles: load j of this thread is row l_r + 32 j, source chunk l_c
+  const int l_r = tid >> 3, l_c = (tid & 7) ^ ((l_r >> 1) & 7);
+  int a_voff[Cfg::A_LOADS];
+#pragma unroll
+  for (int j = 0; j < Cfg::A_LOADS; ++j) {
+    const int r = l_r + j * 32;
+    const int src = gather && r < tr.rows ? row_map[tr.row0 + r] / row_div : r;
+    a_voff[j] = r < tr.rows ? (src * Kdim + l_c * 4) * 4 : kOutside;
+  }
+  const unsigned wave_lds = lds_byte_addr(smem_raw) + wave * 1024;
+  const int nk1 = (Kdim + BK - 1) / BK, nk = nk1 * segs;
+  auto issue = [&](int kt) {
+    const unsigned base = wave_lds + (kt & 1) * Cfg::STAGE_BYTES;
+    const bool second = kt >= nk1;
+    const int k0 = (second ? kt - nk1 : kt) * BK;
+    const bool past_k = k0 + l_c * 4 >= Kdim;  // this lane's chunk lies past the end of a row
+#pragma unroll
+    for (int j = 0; j < Cfg::A_LOADS; ++j)
+      f32_load(second ? a_rsrc1 : a_rsrc0, base + j * NT * 16, past_k ? kOutside : a_voff[j] + k0 * 4);
+    if constexpr (kBT) {
+#pragma unroll
+      for (int j = 0; j < Cfg::B_LOADS; ++j)
+        f32_load(second ? b_rsrc1 : b_rsrc0, base + Cfg::A_BYTES + j * NT * 16,
+                 past_k ? kOutside : ((n0 + l_r + j * 32) * Kdim + k0 + l_c * 4) * 4);
+    } else {
+#pragma unroll
+      for (int u = 0; u < Cfg::NSUB; ++u)
+#pragma unroll
+        for (int j = 0; j < Cfg::B_LOADS; ++j) {
+          const int s = tid + j * NT, k = s / (BN / 4), c = s % (BN / 4);
+          f32_load(u ? b_rsrc1 : b_rsrc0, base + Cfg::A_BYTES + u * Cfg::B_BYTES + j * NT * 16,
+                   ((k0 + k) * N + n0 + c * 4) * 4);
+        }
+    }
+  };
+
+  f32x16_t acc[TM][TN];
+#pragma unroll
+  for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+    for (int jj = 0; jj < TN; ++jj)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mi][jj][i] = 0.0f;
+
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  const int sw = ((lane & 31) >> 1) & 7;
+  const int a_off = (wm * 32 * TM + (lane & 31)) * (BK * 4);
+  const int bt_off = Cfg::A_BYTES + (wn * 32 * TN + (lane & 31)) * (BK * 4);
+  // fragments of an 8-deep sub-step: value i of this lane belongs to k = 8 q + 4 half + i
+  auto load_frags = [&](const unsigned char* st, int q, f32x4* a, f32x4* b) {
+    const int chunk = ((2 * q + half) ^ sw) << 4;
+#pragma unroll
+    for (int mi = 0; mi < TM; ++mi)
+      a[mi] = *reinterpret_cast<const f32x4*>(st + a_off + mi * 32 * BK * 4 + chunk);
+#pragma unroll
+    for (int jj = 0; jj < TN; ++jj) {
+      if constexpr (kBT) {
+        b[jj] = *reinterpret_cast<const f32x4*>(st + bt_off + jj * 32 * BK * 4 + chunk);
+      } else {
+        const int u = kDual ? jj : 0, col = (kDual ? wn : wn * TN + jj) * 32 + (lane & 31);
+        const float* p = reinterpret_cast<const float*>(st + Cfg::A_BYTES + u * Cfg::B_BYTES) + (8 * q + 4 * half) * BN + col;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[jj][i] = p[i * BN];
+      }
+    }
+  };
+  // (the fragments of the next sub-step are requested before the products of this one are issued, and the
+  // scheduling barriers keep it so: left alone the compiler reads each sub-step's fragments right in front of
+  // its products and the wave waits for the LDS every time, 1 to 4 % of the run time)
+  auto compute = [&](int kt) {
+    const unsigned char* st = smem_raw + (kt & 1) * Cfg::STAGE_BYTES;
+    f32x4 a[2][TM], b[2][TN];
+    load_frags(st, 0, a[0], b[0]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < BK / 8; ++q) {
+      if (q + 1 < BK / 8) load_frags(st, q + 1, a[(q + 1) & 1], b[(q + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+          for (int jj = 0; jj < TN; ++jj)
+            acc[mi][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q & 1][mi][i], b[q & 1][jj][i], acc[mi][jj], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  const bool wave_has_work = wm * 32 * TM < tr.rows;  // rows past the end of the group: loads and barriers only
+  issue(0);
+  for (int kt = 0; kt < nk; ++kt) {
+    wait_vmcnt<0>();
+    __syncthreads();
+    if (kt + 1 < nk) issue(kt + 1);
+    if (wave_has_work) compute(kt);
+  }
+
+  // value i of lane l of a block is row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32: the 32 lanes of a
+  // half wave store 128 contiguous bytes
+#pragma unroll
+  for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+    for (int jj = 0; jj < (kDual ? 1 : TN); ++jj) {
+      const int col = n0 + (kDual ? wn : wn * TN + jj) * 32 + (lane & 31);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int r = (wm * TM + mi) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+        if (r < tr.rows && col < N) {
+          const size_t at = (size_t)(tr.row0 + r) * N + col;
+          if constexpr (kDual) {
+            const float g = acc[mi][0][i], u = acc[mi][1][i];
+            C[at] = silu_fast(g) * u;
+            if (save0) {
+              save0[at] = g;
+              save1[at] = u;
+            }
+          } else {
+            C[at] = acc[mi][jj][i];
+          }
+        }
+      }
+    }
+}
+
+// Weight gradients.  One workgroup per (matrix, group, tile); D1 / C1 (if `matrices` is 2) is a second
+// product with the same P.  split_chunk > 0 (one dense group): "group" e is the e-th run of split_chunk rows
+// and C holds partial sums [matrix][E][KA, N] that the caller adds up in order.
+template <int BMO, int BNO>
+__global__ __launch_bounds__(256) void grouped_gemm_f32_tn_kernel(
+    const float* __restrict__ P, const float* __restrict__ D0, const float* __restrict__ D1, float* __restrict__ C0,
+    float* __restrict__ C1, const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E,
+    int dense_rows, int KA, int N, int mtiles_o, int ntiles_o, int split_chunk) {
+  constexpr int BK = 32, NT = 256, TM = BMO / 64, TN = BNO / 64;
+  constexpr int P_BYTES = BK * BMO * 4, STAGE_BYTES = P_BYTES + BK * BNO * 4;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int per_group = mtiles_o * ntiles_o;
+  int block = (int)blockIdx.x;
+  const int which = block / (E * per_group);
+  block -= which * E * per_group;
+  const int e = block / per_group;
+  const int in_e = block - e * per_group;
+  const int nt = in_e / mtiles_o, m0 = (in_e - nt * mtiles_o) * BMO, n0 = nt * BNO;
+  int row0 = 0, rows = dense_rows;
+  if (group_sizes) {
+    row0 = __builtin_amdgcn_readfirstlane(offsets[e]);
+    rows = __builtin_amdgcn_readfirstlane(group_sizes[e]);
+  } else if (split_chunk > 0) {
+    row0 = e * split_chunk;
+    rows = max(0, min(split_chunk, dense_rows - row0));
+  }
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  // rows past the end of the group lie outside the descriptors and read as zeros
+  const i32x4_t p_rsrc = make_rsrc(P + (size_t)row0 * KA, rows * KA * 4);
+  const i32x4_t d_rsrc = make_rsrc((which ? D1 : D0) + (size_t)row0 * N, rows * N * 4);
+  const unsigned wave_lds = lds_byte_addr(smem_raw) + wave * 1024;
+  auto issue = [&](int kt) {
+    const unsigned base = wave_lds + (kt & 1) * STAGE_BYTES;
+#pragma unroll
+    for (int j = 0; j < BMO / 32; ++j) {
+      const int s = tid + j * NT, k = s / (BMO / 4), c = s % (BMO / 4);
+      f32_load(p_rsrc, base + j * NT * 16, ((kt * BK + k) * KA + m0 + c * 4) * 4);
+    }
+#pragma unroll
+    for (int j = 0; j < BNO / 32; ++j) {
+      const int s = tid + j * NT, k = s / (BNO / 4), c = s % (BNO / 4);
+      f32_load(d_rsrc, base + P_BYTES + j * NT * 16, ((kt * BK + k) * N + n0 + c * 4) * 4);
+    }
+  };
+  f32x16_t acc[TM][TN];
+#pragma unroll
+  for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+    for (int jj = 0; jj < TN; ++jj)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mi][jj][i] = 0.0f;
+  const int nk = (rows + BK - 1) / BK;
+  if (nk > 0) issue(0);
+  for (int kt = 0; kt < nk; ++kt) {
+    wait_vmcnt<0>();
+    __syncthreads();
+    if (kt + 1 < nk) issue(kt + 1);
+    const float* ps = reinterpret_cast<const float*>(smem_raw + (kt & 1) * STAGE_BYTES) + half * BMO + wm * 32 * TM + (lane & 31);
+    const float* ds = reinterpret_cast<const float*>(smem_raw + (kt & 1) * STAGE_BYTES + P_BYTES) + half * BNO + wn * 32 * TN + (lane & 31);
+    // two k rows (one per half wave) per product, four products' worth of fragments ahead
+    constexpr int KS = 4;
+    float a[2][KS][TM], b[2][KS][TN];
+    auto load_frags = [&](int set, int k2) {
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi) a[set][i][mi] = ps[2 * (k2 + i) * BMO + mi * 32];
+#pragma unroll
+        for (int jj = 0; jj < TN; ++jj) b[set][i][jj] = ds[2 * (k2 + i) * BNO + jj * 32];
+      }
+    };
+    load_frags(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < BK / 2 / KS; ++g) {
+      if (g + 1 < BK / 2 / KS) load_frags((g + 1) & 1, (g + 1) * KS);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < KS; ++i)
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+          for (int jj = 0; jj < TN; ++jj)
+            acc[mi][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g & 1][i][mi], b[g & 1][i][jj], acc[mi][jj], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  float* const Ce = (which ? C1 : C0) + (size_t)e * KA * N;
+#pragma unroll
+  for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+    for (int jj = 0; jj < TN; ++jj) {
+      const int col = n0 + (wn * TN + jj) * 32 + (lane & 31);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int r = m0 + (wm * TM + mi) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+        if (r < KA && col < N) Ce[(size_t)r * N + col] = acc[mi][jj][i];
+      }
+    }
+}
+
+}  // namespace jtmoe

@@ -1,0 +1,60 @@
+"""The single-precision matrix-core products at the edges of their tiles (64 and 128 rows and columns, k steps
+of 32, chunks of 4), against the oracle.
+
+Bars: the forward's f32_tol.  Gradients: max|g - ref| / max|ref| <= 2^-23 * sqrt(n) * 8 for sums of n terms --
+each of two summation orders is off by about sqrt(n) roundings of 2^-24 of the terms' size, and a factor of
+eight covers the largest of the elements and the chain of three products.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import test_gpu_grad as G
+import test_gpu_parity as P
+from oracle import moe_grad_oracle as GO
+from oracle import moe_oracle as O
+from research_amd import grad
+from test_gpu_parity import dev, host, random_problem
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,top_k,inter", [
+    (1, 4, 1, 1, 4),          # one row, one chunk
+    (65, 36, 3, 2, 68),       # a second 32-deep step of one chunk, tiles with one row
+    (400, 128, 2, 2, 192),    # whole tiles with gathered rows
+    (600, 260, 3, 1, 132),    # columns and steps that end one chunk in
+    (2500, 64, 4, 2, 256),    # enough tiles for the 128-row forms
+])
+def test_f32_experts_at_tile_edges(gpu, tokens, hidden, experts, top_k, inter):
+    P.test_grouped_swiglu_matches_oracle(gpu, tokens, hidden, experts, top_k, inter, "f32")
+    x, gate, up, down, ids, w = random_problem(7 + tokens, tokens, hidden, experts, top_k, inter, 0.1)
+    dy = np.random.default_rng(tokens).standard_normal((tokens, hidden)).astype(np.float32)
+    want = GO.experts_backward(x, ids, w, gate, up, down, dy)
+    got, _ = G.expert_grads(gpu, x, ids, w, gate, up, down, dy, "f32")
+    bar = 2.0 ** -23 * 8 * np.sqrt(max(hidden, inter, tokens * top_k))
+    for name in ("dx", "d_weights", "d_gate", "d_up", "d_down"):
+        assert P.report(f"f32 {name}", host(getattr(got, name)), getattr(want, name).astype(np.float32)) <= bar, name
+
+
+@pytest.mark.parametrize("tokens,hidden,inter", [(130, 68, 36), (1000, 128, 64), (4100, 256, 4)])
+def test_f32_shared_experts_with_split_reductions(gpu, tokens, hidden, inter):
+    """One group: the weight gradients are cut into runs of rows whose partial sums are added in order."""
+    rng = np.random.default_rng(tokens)
+    x, dy = (rng.standard_normal((tokens, hidden)).astype(np.float32) for _ in range(2))
+    mats = [(rng.standard_normal(s) * 0.1).astype(np.float32) for s in ((hidden, inter), (hidden, inter), (inter, hidden))]
+    md = [dev(m, gpu) for m in mats]
+    y, res = grad.shared_swiglu_train(dev(x, gpu), *md)
+    np.testing.assert_allclose(host(y), O.shared_swiglu(x, *mats, "f32"), **P.f32_tol(O.shared_swiglu(x, *mats, "f32")))
+    got = grad.shared_backward(dev(x, gpu), dev(dy, gpu), *md, res)
+    again = grad.shared_backward(dev(x, gpu), dev(dy, gpu), *md, res)
+    leaves = [torch.from_numpy(a.astype(np.float64)).requires_grad_() for a in (x, *mats)]
+    h = torch.nn.functional.silu(leaves[0] @ leaves[1]) * (leaves[0] @ leaves[2])
+    want = torch.autograd.grad(h @ leaves[3], leaves, torch.from_numpy(dy.astype(np.float64)))
+    bar = 2.0 ** -23 * 8 * np.sqrt(max(hidden, inter, tokens))
+    for g, a, ref in zip(got, again, want):
+        assert torch.equal(g, a)
+        assert P.report("f32 shared", host(g), ref.numpy().astype(np.float32)) <= bar
