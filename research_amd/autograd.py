@@ -27,6 +27,8 @@ class MoeLayerFunction(torch.autograd.Function):
         ctx.route_scale = route_scale
         ctx.score_func = score_func
         ctx.has_shared = shared is not None
+        # no zero-filled cotangents for the outputs nothing depends on (the ids always, often the scores)
+        ctx.set_materialize_grads(False)
         # Everything the backward pass reads goes through save_for_backward (which knows how to hold an
         # output such as the scores without a reference cycle); y itself is not needed again.
         shared_res = residuals.shared
