@@ -28,7 +28,8 @@ ARCH = "gfx950"
 SOURCE_FILES = (
     "api.hip", "router.hip", "dispatch.hip", "combine.hip", "norm.hip", "grouped_gemm.hip", "grouped_gemm_bwd.hip",
     "grouped_gemm_f32.hip", "backward.hip", "common.hpp", "gemm_common.hpp", "gemm_launch.hpp", "grouped_gemm_dma.hpp",
-    "grouped_gemm_stream.hpp", "grouped_gemm_bwd.hpp", "grouped_gemm_f32.hpp", "dispatch_small.hpp", "native/gemm_check.hip",
+    "grouped_gemm_stream.hpp", "grouped_gemm_bwd.hpp", "grouped_gemm_f32.hpp",
+    "grouped_gemm_skinny.hpp", "dispatch_small.hpp", "native/gemm_check.hip",
 )
 
 

@@ -12,7 +12,11 @@
 #include "common.hpp"
 #include "gemm_launch.hpp"
 #include "grouped_gemm_dma.hpp"
+#include "grouped_gemm_skinny.hpp"
 #include "grouped_gemm_stream.hpp"
+
+#include <algorithm>
+#include <cmath>
 
 #include <mutex>
 
@@ -211,7 +215,8 @@ int launch_fast(const void* a, const void* b0, const void* b1, void* c, const in
 template <typename Cfg>
 int launch_stream(const void* a, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, hipStream_t stream,
-                  const int32_t* row_map, int row_div, int64_t a_rows, void* save0, void* save1) {
+                  const int32_t* row_map, int row_div, int64_t a_rows, void* save0, void* save1,
+                  int workgroups_per_cu = 1) {
   using L = StreamLayout<Cfg>;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
@@ -227,7 +232,7 @@ int launch_stream(const void* a, const void* b0, const void* b1, void* c, const 
   const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles_grid = gemm_grid(mtiles, nt);
   if (tiles_grid >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: grid too large");
-  const PersistentSchedule ps = persistent_schedule(tiles_grid, persistent_grid_size(), kTilesPerWorkgroup<Cfg>);
+  const PersistentSchedule ps = persistent_schedule(tiles_grid, workgroups_per_cu * persistent_grid_size(), 4);
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes, stream>>>(
       static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
       static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim, (int)N, (int)mtiles, (int)nt,
@@ -245,17 +250,143 @@ inline bool stream_ok(int64_t rows, int64_t Kdim, int64_t N, const int32_t* row_
          (row_map == nullptr || (rows < ((int64_t)1 << 27) && row_div >= 1 && row_div <= 32));
 }
 
-// Mean rows per group below which the 64-row tiles are used.
-constexpr int64_t kSmallGroupRows = 128;
-inline bool small_groups(int64_t rows, int64_t E) { return rows < kSmallGroupRows * E; }
-// Mean rows per group up to which nearly every group is a single tile tall, so that no workgroup
-// reads an expert matrix after another has: its loads are then marked non-temporal.
-constexpr int64_t kTinyGroupRows = 32;
-inline bool tiny_groups(int64_t rows, int64_t E) { return rows <= kTinyGroupRows * E; }
+template <typename Cfg>
+int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
+                  const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, hipStream_t stream,
+                  const int32_t* row_map = nullptr, int row_div = 1, int64_t a_rows = 0, void* save0 = nullptr,
+                  void* save1 = nullptr, int64_t a_group_rows = 0) {
+  if constexpr (Cfg::SMEM_BYTES > 64 * 1024) {
+    static std::once_flag once;
+    static hipError_t attr_err = hipSuccess;
+    std::call_once(once, [] {
+      attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&grouped_gemm_skinny_kernel<Cfg>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::SMEM_BYTES);
+    });
+    if (attr_err != hipSuccess)
+      return fail(JTMOE_ELAUNCH, "grouped gemm: kernel set-up: %s", hipGetErrorString(attr_err));
+  }
+  const int64_t mtiles = group_sizes == nullptr ? (rows + Cfg::BM - 1) / Cfg::BM : max_m_tiles(rows, E, Cfg::BM);
+  const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
+  const int64_t grid = gemm_grid(mtiles, nt);
+  if (grid >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: grid too large");
+  const SkinnyProblem p{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
+                        static_cast<uint16_t*>(c), static_cast<uint16_t*>(save0), static_cast<uint16_t*>(save1),
+                        group_sizes, offsets, row_map, (int)E, (int)rows, (int)Kdim, (int)N, (int)mtiles, (int)nt, row_div,
+                        (int)a_rows, (int)a_group_rows};
+  grouped_gemm_skinny_kernel<Cfg><<<(unsigned)grid, Cfg::NT, Cfg::SMEM_BYTES, stream>>>(p);
+  return JTMOE_OK;
+}
+
+// ---- which kernel takes a product ------------------------------------------------------------------------
+// All times below: rows of T tokens in E groups by a balanced top-k, matrices cold, launch overhead included.
+enum class Tiles { kSkinny11, kSkinny12, kSkinny21, kSkinny22, kSkinny41, kTiny, kHalf, kHalfDeep, kFull };
+
+// m-tiles of BM rows to be expected: exact for one dense group; otherwise the groups that a balanced choice
+// leaves with a row, and half a tile of padding in each once groups outgrow half a tile
+inline double expected_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
+  if (dense) return (double)((rows + BM - 1) / BM);
+  const double groups = (double)E * (1.0 - std::exp(-(double)rows / (double)E)), mean = (double)rows / groups;
+  return groups * (mean > BM / 2 ? mean / BM + 0.5 : 1.0);
+}
+
+// Streaming tiles (grouped_gemm_skinny.hpp) while they find a CU each: of the shapes with at most one tile per CU
+// the one with the most tiles, so that the matrices are drawn through as many CUs as possible.  us at 1 token,
+// 64 experts top-8, 2048 -> 1408: gate/up 21 (64-column tiles, 176 of them; 128 columns 27, the 64-row LDS tiles
+// 49), down 14 (15; 38); shared experts of 2816: 20 and 12 (25 and 21; 62 and 86) at 1 token, 20 and 16 (30 and
+// 21; 62 and 86) at 64, 27 and 21 in 32-row tiles at 128 (31 and 22 in 16-row ones).  With more than 256
+// tiles, while groups hold a row or four: 73 against 77 and 41 against 45 us at 8 tokens; from 16 tokens on
+// (mean 2.3 of 64 groups) the two are equal within 2 %.  Beyond, a group's second tile reads its matrix again:
+// 154 against 111 us for gate/up at 128 tokens.
+inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dual, Tiles* out) {
+  struct Shape {
+    Tiles id;
+    int RB, BN;
+  };
+  constexpr Shape shapes[] = {{Tiles::kSkinny12, 1, 64}, {Tiles::kSkinny22, 2, 64}, {Tiles::kSkinny11, 1, 128},
+                              {Tiles::kSkinny21, 2, 128}, {Tiles::kSkinny41, 4, 128}};
+  const double cus = (double)persistent_grid_size();
+  double most = 0.0;
+  for (const Shape& s : shapes) {
+    if (s.id == Tiles::kSkinny41 && dual) continue;  // 512 tokens, shared 2816: 45 us against 41 in half tiles
+    const double tiles = expected_mtiles(rows, E, dense, 16 * s.RB) * (double)((N + s.BN - 1) / s.BN);
+    if (tiles <= cus && tiles > most) {
+      most = tiles;
+      *out = s.id;
+    }
+  }
+  if (most == 0.0 && !dense && (double)rows <= 4.0 * expected_mtiles(rows, E, false, 16)) {
+    *out = Tiles::kSkinny11;
+    return true;
+  }
+  return most > 0.0;
+}
+
+// Rows per group up to which 64-row LDS tiles hold nearly every group in one tile: each expert matrix is then
+// read by one row of workgroups, with non-temporal loads.  us for gate/up and down, 64 experts: mean 48 rows 121
+// and 61 (256-row tiles 141 and 77), mean 64 rows, where half of the groups need a second tile, 203 and 103 (148
+// and 78).
+constexpr int64_t kTinyGroupRows = 52;  // four or fewer in a hundred groups above 64
+
+// With fewer 128-row tiles than CUs: gate/up of 1024 tokens, shared 2816: 41 us against 50 in 256-row tiles;
+// with more, two rounds of half tiles: 2048 tokens 77 against 52.
+// Down: one half tile per CU 40 us against 63 (2048 tokens, shared 2816; 64-deep steps 41), two per CU with
+// 64-deep steps 55 against 64 (4096 tokens; 32-deep 69), and so on by rounds: a round of 512 half tiles takes
+// 0.57 of a round of 256 whole ones, a last round of at most 256 of them 0.42, the launch 0.12 more; half tiles
+// read their operands twice as often, so they are taken only where that is 15 % less.  8192 rows x 2048 -> 1024 in
+// 8 groups: 57 against 56 (576 tiles, whole ones kept); 16384 rows: 84 against 100 (1088 against 272 tiles: the
+// whole ones start a second round for 16 of them).
+inline Tiles pick_large(int64_t rows, int64_t E, bool dense, int64_t N, bool dual) {
+  const double cus = (double)persistent_grid_size();
+  const double half = expected_mtiles(rows, E, dense, 128) * (double)((N + 127) / 128);
+  if (half <= cus) return Tiles::kHalf;
+  if (dual) return Tiles::kFull;
+  const double full = expected_mtiles(rows, E, dense, 256) * (double)((N + 255) / 256);
+  const double rounds = std::floor(half / (2 * cus)), rest = half - rounds * 2 * cus;
+  const double half_cost = 0.12 + 0.57 * rounds + (rest <= 0.0 ? 0.0 : (rest <= cus ? 0.42 : 0.57));
+  return 1.15 * half_cost < std::ceil(full / cus) ? Tiles::kHalfDeep : Tiles::kFull;
+}
+
+inline Tiles pick_tiles(int64_t rows, int64_t Kdim, int64_t E, bool dense, int64_t N, bool dual) {
+  Tiles t;
+  // Where the layer's decode path may run every token through every expert (router.hip), gate/up keeps the
+  // 64-row LDS tiles, whose sums that launch reproduces bit for bit.
+  const bool decode_shape = dual && !dense && (E == 16 || E == 32 || E == 64) && rows >= 2 * E && Kdim % 128 == 0 && N % 64 == 0;
+  if (!decode_shape && pick_skinny(rows, E, dense, N, dual, &t)) return t;
+  if (!dense && rows <= kTinyGroupRows * E) return Tiles::kTiny;
+  return pick_large(rows, E, dense, N, dual);
+}
 
 inline bool fast_ok(const void* a, const void* b0, const void* b1, const void* c, int64_t Kdim, int64_t N) {
   return Kdim % 8 == 0 && N % 8 == 0 && Kdim * N < ((int64_t)1 << 30) && aligned16(a) && aligned16(b0) && (b1 == nullptr || aligned16(b1)) &&
          aligned16(c);
+}
+
+// y = act Wd[e] on the matrix cores (fast_ok holds); with a map, packed row j reads row row_map[j] / row_div of
+// its group's block of a_group_rows rows (the decode path)
+int launch_down_fast(const void* act, const void* down, const int32_t* group_sizes, const int32_t* offsets,
+                     int64_t rows, int64_t H, int64_t I, int64_t E, void* y, hipStream_t stream,
+                     const int32_t* row_map = nullptr, int row_div = 1, int64_t a_group_rows = 0) {
+#define JT_DOWN(LAUNCH, CFG) LAUNCH<CFG>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream, row_map, row_div, a_group_rows, nullptr, nullptr
+  using S11 = SkinnyCfg<1, 1, false>;
+  using S12 = SkinnyCfg<1, 2, false>;
+  using S21 = SkinnyCfg<2, 1, false>;
+  using S22 = SkinnyCfg<2, 2, false>;
+  using S41 = SkinnyCfg<4, 1, false>;
+  const Tiles t = pick_tiles(rows, I, E, group_sizes == nullptr, H, false);
+  switch (t) {
+    case Tiles::kSkinny11: return JT_DOWN(launch_skinny, S11), a_group_rows);
+    case Tiles::kSkinny12: return JT_DOWN(launch_skinny, S12), a_group_rows);
+    case Tiles::kSkinny21: return JT_DOWN(launch_skinny, S21), a_group_rows);
+    case Tiles::kSkinny22: return JT_DOWN(launch_skinny, S22), a_group_rows);
+    case Tiles::kSkinny41: return JT_DOWN(launch_skinny, S41), a_group_rows);
+    case Tiles::kTiny: return JT_DOWN(launch_fast, DownTinyCfg), 0, a_group_rows);
+    default: break;
+  }
+  if (a_group_rows > 0) return JT_DOWN(launch_fast, DownTinyCfg), 0, a_group_rows);
+  if (t == Tiles::kHalf && stream_ok<DownHalfCfg>(rows, I, H, nullptr, 1)) return JT_DOWN(launch_stream, DownHalfCfg), 2);
+  if (t != Tiles::kFull && stream_ok<DownHalfDeepCfg>(rows, I, H, nullptr, 1)) return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
+  return I % 64 == 0 ? JT_DOWN(launch_fast, DownCfg)) : JT_DOWN(launch_fast, DownTailCfg));
+#undef JT_DOWN
 }
 
 template <typename T>
@@ -265,25 +396,37 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
                 int64_t x_rows = 0, void* save_gate = nullptr, void* save_up = nullptr) {
   if (rows == 0) return JTMOE_OK;
   int rc;
-  const bool small = small_groups(rows, E), tiny = tiny_groups(rows, E);
+  const bool dense = group_sizes == nullptr;
   const bool gather_ok = row_map == nullptr || x_rows * H < ((int64_t)1 << 30);
   const bool saves_ok = save_gate == nullptr || (aligned16(save_gate) && aligned16(save_up));
-  if (Elem<T>::is_bf16 && fast_ok(x, gate, up, act, H, I) && gather_ok && saves_ok)
-    rc = tiny    ? launch_fast<GateUpTinyCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
-                                              row_div, x_rows, save_gate, save_up)
-         : small ? launch_fast<GateUpSmallCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
-                                               row_div, x_rows, save_gate, save_up)
-         : stream_ok<GateUpStreamCfg>(rows, H, I, row_map, row_div)
-             ? launch_stream<GateUpStreamCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
-                                              row_div, x_rows, save_gate, save_up)
-         : stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div)
-             ? launch_stream<GateUpStreamTailCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
-                                                  row_div, x_rows, save_gate, save_up)
-         : H % 64 == 0
-             ? launch_fast<GateUpCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map, row_div,
-                                      x_rows, save_gate, save_up)
-             : launch_fast<GateUpTailCfg>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map,
-                                          row_div, x_rows, save_gate, save_up);
+#define JT_GATE_UP(LAUNCH, CFG, ...)                                                                               \
+  LAUNCH<CFG>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map, row_div, x_rows, save_gate,  \
+              save_up __VA_ARGS__)
+  if (Elem<T>::is_bf16 && fast_ok(x, gate, up, act, H, I) && gather_ok && saves_ok) {
+    using S11 = SkinnyCfg<1, 1, true>;
+    using S12 = SkinnyCfg<1, 2, true>;
+    using S21 = SkinnyCfg<2, 1, true>;
+    using S22 = SkinnyCfg<2, 2, true>;
+    switch (pick_tiles(rows, H, E, dense, I, true)) {
+      case Tiles::kSkinny11: rc = JT_GATE_UP(launch_skinny, S11); break;
+      case Tiles::kSkinny12: rc = JT_GATE_UP(launch_skinny, S12); break;
+      case Tiles::kSkinny21: rc = JT_GATE_UP(launch_skinny, S21); break;
+      case Tiles::kSkinny22: rc = JT_GATE_UP(launch_skinny, S22); break;
+      case Tiles::kTiny: rc = JT_GATE_UP(launch_fast, GateUpTinyCfg); break;
+      case Tiles::kHalf:
+        if (stream_ok<GateUpHalfCfg>(rows, H, I, row_map, row_div)) {
+          rc = JT_GATE_UP(launch_stream, GateUpHalfCfg);
+          break;
+        }
+        [[fallthrough]];
+      default:
+        rc = stream_ok<GateUpStreamCfg>(rows, H, I, row_map, row_div)       ? JT_GATE_UP(launch_stream, GateUpStreamCfg)
+             : stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div) ? JT_GATE_UP(launch_stream, GateUpStreamTailCfg)
+             : H % 64 == 0                                                  ? JT_GATE_UP(launch_fast, GateUpCfg)
+                                                                            : JT_GATE_UP(launch_fast, GateUpTailCfg);
+    }
+  }
+#undef JT_GATE_UP
   else if (!Elem<T>::is_bf16 && f32_gemm_supported(x, save_gate, gate, up, act, row_map ? x_rows : rows, H, I) &&
            aligned16(save_up))
     rc = launch_f32_nn(x, gate, up, act, group_sizes, offsets, rows, H, I, E, row_map, row_div, x_rows, save_gate,
@@ -294,10 +437,7 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
   if (rc) return rc;
   stage_mark(first_stage, stream);
   if (Elem<T>::is_bf16 && fast_ok(act, down, nullptr, y, I, H))
-    rc = tiny    ? launch_fast<DownTinyCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream)
-         : small ? launch_fast<DownSmallCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream)
-         : I % 64 == 0 ? launch_fast<DownCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream)
-                       : launch_fast<DownTailCfg>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream);
+    rc = launch_down_fast(act, down, group_sizes, offsets, rows, H, I, E, y, stream);
   else if (!Elem<T>::is_bf16 && f32_gemm_supported(act, nullptr, down, nullptr, y, rows, I, H))
     rc = launch_f32_nn(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, nullptr, 1, 0, nullptr, nullptr,
                        stream);
@@ -325,8 +465,8 @@ int launch_down_from_all_tokens(const void* act_full, const void* down, const in
                                 int64_t I, int64_t E, void* packed_y, hipStream_t stream) {
   if (!fast_ok(act_full, down, nullptr, packed_y, I, H))
     return fail(JTMOE_EINVAL, "moe_forward: operands must be 16-byte aligned");
-  return launch_fast<DownTinyCfg>(act_full, down, nullptr, packed_y, group_sizes, offsets, T * K, I, H, E, stream,
-                                  source_order, (int)K, T, nullptr, nullptr, 0, /*a_group_rows=*/T);
+  return launch_down_fast(act_full, down, group_sizes, offsets, T * K, H, I, E, packed_y, stream, source_order, (int)K,
+                          /*a_group_rows=*/T);
 }
 
 // ---- the gathering launch pair as the layer uses it (declared in common.hpp) ----

@@ -849,11 +849,9 @@ using DownTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 64 + 128 + 327
 // waves fit a CU: at 64 experts x 11 column tiles every workgroup of the launch is then resident
 // at once and all of them stream together (with 64-deep steps and two workgroups per CU the
 // last third of the workgroups ran alone on a mostly idle memory system: 0.140 vs 0.126 ms).
-using GateUpSmallCfg = DmaGemmCfg<64, 128, 32, 1, 4, true, 2, 16 + 128>;
-using DownSmallCfg = DmaGemmCfg<64, 256, 32, 1, 4, false, 2, 16>;
-// The same tiles when nearly every group fits one tile (a decode step): each expert matrix is then
-// read by exactly one row of workgroups, and non-temporal loads stream it past the L2
-// (64 tokens, 64 experts: gate/up 0.126 -> 0.110 ms = 6.7 TB/s, down 0.061 -> 0.054 ms = 6.8 TB/s).
+// Nearly every group fits one such tile, so each expert matrix is read by exactly one row of workgroups, and
+// non-temporal loads stream it past the L2 (64 tokens, 64 experts: gate/up 0.126 -> 0.110 ms = 6.7 TB/s, down
+// 0.061 -> 0.054 ms = 6.8 TB/s; at 387 tokens 137 -> 121 and 68 -> 61 us).
 using GateUpTinyCfg = DmaGemmCfg<64, 128, 32, 1, 4, true, 2, 16 + 128 + 4096>;
 using DownTinyCfg = DmaGemmCfg<64, 256, 32, 1, 4, false, 2, 16 + 4096>;
 

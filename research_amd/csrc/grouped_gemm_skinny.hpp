@@ -1,0 +1,220 @@
+// bf16 grouped GEMM for groups of a few rows (a decode step, the shared experts of a small batch): the
+// matrices stream straight from memory into MFMA operands, no LDS and no barrier in the k loop.
+//
+//   C[rows of e, :] = A[rows of e, :] @ B[e]                          (kDual = false)
+//   C = silu(round(A @ B0[e])) * round(A @ B1[e])                     (kDual = true)
+//
+// Bound: HBM (a matrix element is used by a handful of rows), through what one CU can draw: 50 to 60 GB/s from
+// memory and twice that from the L2, however many loads its waves have in flight, so that the chip's 6 TB/s
+// take the greater part of its CUs.  A launch of the LDS kernels at these sizes has 8 to 100 tiles, and a
+// 32-deep step of a tile costs 0.65 us whatever the depth of its pipeline (wait, barrier, LDS reads and
+// products of 64 mostly empty rows with one wave per SIMD: 1500 cycles for 16 KB).  Hence here
+//   * narrow tiles: 128 / FOLD columns of one matrix, or of each of two (kDual);
+//   * a wave owns its loads: a lane fetches 16 bytes (8 columns) of eight consecutive k rows, the wave a block
+//     of the matrix as it is stored, and 32 byte permutes turn it into the B operands of eight
+//     v_mfma_f32_16x16x32_bf16 (operand j: column 8 (lane % 16) + j, whose eight k values the lane holds);
+//   * FOLD = 2: the upper eight of sixteen lanes hold the same columns 32 k rows further on.  An MFMA takes its
+//     A operand for all columns, so the block is multiplied once with either half's rows of A into accumulators
+//     of its own, and each half's columns are taken from the right one at the end: twice the products, which
+//     there is time for, and whole 128-byte lines with half as many columns per tile;
+//   * D blocks of 8 KB are in flight per wave in a ring of registers;
+//   * the four waves of a workgroup share out the k range (two of them per matrix when kDual), and add
+//     their sums up in wave order through LDS at the end.
+// RB = blocks of 16 rows per tile.  Rows past the end of a group, columns past N and k past K read as zeros.
+//
+// Requirements: K % 8 == 0, N % 8 == 0, 16-byte aligned pointers, K*N*2 < 2^31, a_rows*K*2 < 2^31.
+#pragma once
+
+#include "grouped_gemm_dma.hpp"
+
+namespace jtmoe {
+
+template <int RB_, int FOLD_, bool kDual_>
+struct SkinnyCfg {
+  static constexpr int RB = RB_, FOLD = FOLD_, BM = 16 * RB, BN = 128 / FOLD, NT = 256, BK = 32 * FOLD;
+  static constexpr bool kDual = kDual_;
+  static constexpr int D = RB == 1 ? 4 : 3;                    // blocks in flight per wave
+  static constexpr int KWAVES = kDual ? 2 : 4;                 // waves that share out the k range of a matrix
+  static constexpr int MIN_WAVES_PER_EU = RB * FOLD <= 2 ? 2 : 1;
+  static constexpr int GROUP_M = 4;
+  static constexpr int PAD = 4;                                // floats per row of the exchange, against bank conflicts
+  static constexpr int SMEM_BYTES = 4 * BM * (BN + PAD) * 4;   // one block of sums per wave
+  static_assert(FOLD == 1 || FOLD == 2, "columns per tile");
+};
+
+struct SkinnyProblem {
+  const uint16_t *A, *B0, *B1;
+  uint16_t *C, *save0, *save1;  // save0 / save1: the two rounded products of a dual launch, or null
+  const int32_t *group_sizes, *offsets;  // null: one group of dense_rows rows
+  const int32_t* row_map;  // tile row j reads row row_map[j] / row_div of A (a_rows rows), or null
+  int E, dense_rows, Kdim, N, mtiles, ntiles_n, row_div, a_rows;
+  int a_group_rows;  // > 0: A holds a block of a_group_rows rows per group, and the map's rows are rows of it
+};
+
+template <typename Cfg>
+__device__ __forceinline__ void grouped_gemm_skinny_tile(const SkinnyProblem& pr, int block, int launch_blocks) {
+  constexpr int RB = Cfg::RB, FOLD = Cfg::FOLD, BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, D = Cfg::D;
+  constexpr int LF = 16 / FOLD;  // lanes (of sixteen) that hold different columns
+  constexpr bool kDual = Cfg::kDual;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+
+  const int Kdim = pr.Kdim, N = pr.N;
+  TileCoord tc;
+  TileRows tr;
+  if (pr.group_sizes) {
+    const GroupScan scan = group_scan(BM, pr.group_sizes, pr.E);
+    tc = xcd_tile_order_balanced(scan.total, pr.ntiles_n, Cfg::GROUP_M, block);
+    if (tc.mt < 0) return;
+    tr = locate_tile(scan, tc.mt, BM, pr.offsets);
+  } else {
+    tc = xcd_tile_order(pr.mtiles, pr.ntiles_n, Cfg::GROUP_M, block, launch_blocks);
+    if (tc.mt < 0) return;
+    tr = find_tile_wave(tc.mt, BM, nullptr, nullptr, pr.E, pr.dense_rows);
+  }
+  tr.expert = __builtin_amdgcn_readfirstlane(tr.expert);
+  tr.row0 = __builtin_amdgcn_readfirstlane(tr.row0);
+  tr.rows = __builtin_amdgcn_readfirstlane(tr.rows);
+  if (tr.rows <= 0) return;
+  const int n0 = tc.nt * BN;
+  const size_t wofs = (size_t)tr.expert * Kdim * N;
+
+  const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int which = kDual ? wave & 1 : 0, kw = kDual ? wave >> 1 : wave;  // matrix, and share of the k range
+
+  const bool gather = pr.row_map != nullptr;
+  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(pr.A + (gather ? (size_t)tr.expert * pr.a_group_rows : (size_t)tr.row0) * Kdim), 0,
+      (gather ? pr.a_rows : tr.rows) * Kdim * 2, kBufferFlags);
+  const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>((which ? pr.B1 : pr.B0) + wofs), 0, Kdim * N * 2, kBufferFlags);
+  int a_voff[RB];
+#pragma unroll
+  for (int b = 0; b < RB; ++b) {
+    const int r = b * 16 + c16;
+    const int src = gather && r < tr.rows ? pr.row_map[tr.row0 + r] / pr.row_div : r;
+    a_voff[b] = r < tr.rows ? (src * Kdim + g * 8) * 2 : kOutside;
+  }
+  const int col = n0 + c16 % LF * 8, b_k = c16 / LF * 32 + g * 8;  // this lane's columns, and first k row of a block
+  const int b_voff = col < N ? (b_k * N + col) * 2 : kOutside;
+
+  const int blocks = (Kdim + BK - 1) / BK;
+  const int per = (blocks + Cfg::KWAVES - 1) / Cfg::KWAVES;
+  const int first = min(blocks, kw * per), count = min(blocks - first, per);
+
+  u32x4_t b_ring[D][8], a_ring[D][FOLD][RB];
+  // Every load is issued on every path (a block past this wave's share, like a chunk past the end of K, takes
+  // an offset outside the operand: zeros, no traffic), so that the compiler's wait counts stay exact: with the
+  // loads of the last blocks behind a branch it waits for all loads in flight in front of every block.
+  auto load = [&](int slot, int i) {
+    const int k0 = (first + i) * BK;
+#pragma unroll
+    for (int f = 0; f < FOLD; ++f) {
+      const bool past = i >= count || k0 + f * 32 + g * 8 >= Kdim;
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+        a_ring[slot][f][b] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, past ? kOutside : a_voff[b], (k0 + f * 32) * 2, 0);
+    }
+    const bool past = i >= count || k0 + b_k >= Kdim;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)  // non-temporal: few other workgroups read these bytes
+      b_ring[slot][r] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, past ? kOutside : b_voff, (k0 + r) * N * 2, 2);
+  };
+  typedef __attribute__((ext_vector_type(4))) float f32x4;
+  f32x4 acc[FOLD][RB][8];
+#pragma unroll
+  for (int f = 0; f < FOLD; ++f)
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[f][b][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    load(d, d);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int i0 = 0; i0 < count; i0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {  // (blocks past the wave's share multiply zeros)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        u32x4_t frag;
+#pragma unroll
+        for (int p = 0; p < 4; ++p)  // k = 8 g + 2 p (low half) and 2 p + 1 of column 8 c16 + j
+          frag[p] = __builtin_amdgcn_perm(b_ring[d][2 * p + 1][j / 2], b_ring[d][2 * p][j / 2],
+                                          j % 2 ? 0x07060302u : 0x05040100u);
+#pragma unroll
+        for (int f = 0; f < FOLD; ++f)
+#pragma unroll
+          for (int b = 0; b < RB; ++b)
+            acc[f][b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a_ring[d][f][b]),
+                                                                   __builtin_bit_cast(bf16x8_t, frag), acc[f][b][j], 0, 0, 0);
+      }
+      load(d, i0 + d + D);
+      __builtin_amdgcn_sched_barrier(0);  // (else the loads of all D blocks gather at the end of the loop body)
+    }
+  }
+
+  // value i of lane (c16, g) in acc[f][b][j] is row 16 b + 4 g + i, column 8 (c16 % LF) + j, and belongs to the
+  // product if f is the half of the block that the lane holds; the other half's lanes add theirs up here
+  float* const mine = reinterpret_cast<float*>(smem_raw) + wave * (BM * (BN + Cfg::PAD));
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[j] = acc[0][b][j][i];
+        if (FOLD == 2) v[j] += __shfl_xor(acc[FOLD - 1][b][j][i], 8);
+      }
+      float* p = mine + (16 * b + 4 * g + i) * (BN + Cfg::PAD) + c16 % LF * 8;
+      if (c16 < LF) {
+        *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
+      }
+    }
+  __syncthreads();
+  const float* const sums = reinterpret_cast<const float*>(smem_raw);
+  constexpr int kPlane = BM * (BN + Cfg::PAD);
+  for (int c = tid; c < BM * (BN / 8); c += Cfg::NT) {  // one 16-byte piece of a result row per thread
+    const int r = c / (BN / 8), c8 = (c - r * (BN / 8)) * 8;
+    if (r >= tr.rows || n0 + c8 >= N) continue;
+    const float* p = sums + r * (BN + Cfg::PAD) + c8;
+    float v[2][8];  // the two products, or the only one
+#pragma unroll
+    for (int m = 0; m < (kDual ? 2 : 1); ++m)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float t = p[m * kPlane + j];
+#pragma unroll
+        for (int w = 1; w < Cfg::KWAVES; ++w) t += p[(w * (kDual ? 2 : 1) + m) * kPlane + j];
+        v[m][j] = t;
+      }
+    const size_t at = (size_t)(tr.row0 + r) * N + n0 + c8;
+    auto store8 = [&](uint16_t* out, const float* f) {
+      const u32x4_t q = {pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7])};
+      *reinterpret_cast<u32x4_t*>(out + at) = q;
+    };
+    if (kDual) {
+      float h[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) h[j] = silu_rcp(bf16_round_fast(v[0][j])) * bf16_round_fast(v[1][j]);
+      store8(pr.C, h);
+      if (pr.save0) {
+        store8(pr.save0, v[0]);
+        store8(pr.save1, v[1]);
+      }
+    } else {
+      store8(pr.C, v[0]);
+    }
+  }
+}
+
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) __attribute__((amdgpu_waves_per_eu(Cfg::MIN_WAVES_PER_EU))) void grouped_gemm_skinny_kernel(
+    SkinnyProblem p) {
+  grouped_gemm_skinny_tile<Cfg>(p, (int)blockIdx.x, (int)gridDim.x);
+}
+
+}  // namespace jtmoe

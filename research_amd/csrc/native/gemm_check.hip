@@ -594,9 +594,7 @@ static void time_decode() {
   timeit<GateUpCfg>("gate/up 64 groups, 256-row tiles", g, 20);
   timeit<DownCfg>("down 64 groups, 256-row tiles", d, 20);
   for (int rep = 0; rep < 3; ++rep) {
-    timeit<GateUpSmallCfg>("gate/up 64 groups, 64-row tiles", g, 50);
     timeit<GateUpTinyCfg>("gate/up 64 groups, 64-row tiles, weights non-temporal", g, 50);
-    timeit<DownSmallCfg>("down 64 groups, 64-row tiles", d, 50);
     timeit<DownTinyCfg>("down 64 groups, 64-row tiles, weights non-temporal", d, 50);
   }
   release(g);
@@ -627,13 +625,12 @@ int main(int argc, char** argv) {
   }
   {
     Problem p = make(16, 150, 512, 392, 6, true, 0, 1.0f);  // a handful of rows per group: the 64-row tiles
-    ok &= check<GateUpSmallCfg>("gate/up few rows per group", p);
-    ok &= check<DownSmallCfg>("down few rows per group", p);
+    ok &= check<GateUpTinyCfg>("gate/up few rows per group", p);
+    ok &= check<DownTinyCfg>("down few rows per group", p);
     release(p);
   }
   {
     Problem p = make(5, 300, 512, 384, 7, true, 3, 1.0f);
-    ok &= check<GateUpSmallCfg>("gate/up few rows, gather on load", p);
     ok &= check<GateUpTinyCfg>("gate/up few rows, gather, streamed weights", p);
     release(p);
     Problem q = make(16, 150, 512, 392, 8, true, 0, 1.0f);
