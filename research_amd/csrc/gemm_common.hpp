@@ -4,6 +4,8 @@
 
 #include "common.hpp"
 
+#include <cmath>
+
 namespace jtmoe {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -205,6 +207,33 @@ inline int persistent_grid_size() {
     return cus / 8 * 8;
   }();
   return size;
+}
+
+// m-tiles of BM rows to be expected: exact for one dense group; otherwise the groups that a balanced choice
+// leaves with a row, and half a tile of padding in each once groups outgrow half a tile
+inline double expected_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
+  if (dense) return (double)((rows + BM - 1) / BM);
+  const double groups = (double)E * (1.0 - std::exp(-(double)rows / (double)E)), mean = (double)rows / groups;
+  return groups * (mean > BM / 2 ? mean / BM + 0.5 : 1.0);
+}
+
+// 128 x 128 tiles against 256 x 256 ones, by rounds over the CUs: a round of 512 half tiles takes 0.57 of a round of
+// 256 whole ones, a last round of at most 256 of them 0.42, the launch 0.12 more; half tiles read their operands
+// twice as often, so beyond one per CU they are taken only where that is 15 % less.  Down products: one half tile
+// per CU 40 us against 63 (2048 tokens, shared 2816; 64-deep steps 41), two per CU with 64-deep steps 55 against 64
+// (4096 tokens; 32-deep 69); 8192 rows x 2048 -> 1024 in 8 groups: 57 against 56 (576 tiles, whole ones kept);
+// 16384 rows: 84 against 100 (1088 against 272 tiles: the whole ones start a second round for 16 of them).  The data
+// gradients follow the same line (figures at DgradHalfCfg and DgradHalfDeepCfg); on the wrong side of it 32768
+// rows in 64 groups x 2048 -> 1408 would take 262 us against 228.
+enum class HalfTiles { kNone, kOnePerCu, kRounds };
+inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N) {
+  const double cus = (double)persistent_grid_size();
+  const double half = expected_mtiles(rows, E, dense, 128) * (double)((N + 127) / 128);
+  if (half <= cus) return HalfTiles::kOnePerCu;
+  const double full = expected_mtiles(rows, E, dense, 256) * (double)((N + 255) / 256);
+  const double rounds = std::floor(half / (2 * cus)), rest = half - rounds * 2 * cus;
+  const double half_cost = 0.12 + 0.57 * rounds + (rest <= 0.0 ? 0.0 : (rest <= cus ? 0.42 : 0.57));
+  return 1.15 * half_cost < std::ceil(full / cus) ? HalfTiles::kRounds : HalfTiles::kNone;
 }
 
 }  // namespace jtmoe

@@ -16,8 +16,6 @@
 #include "grouped_gemm_stream.hpp"
 
 #include <algorithm>
-#include <cmath>
-
 #include <mutex>
 
 namespace jtmoe {
@@ -281,14 +279,6 @@ int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const 
 // All times below: rows of T tokens in E groups by a balanced top-k, matrices cold, launch overhead included.
 enum class Tiles { kSkinny11, kSkinny12, kSkinny21, kSkinny22, kSkinny41, kTiny, kHalf, kHalfDeep, kFull };
 
-// m-tiles of BM rows to be expected: exact for one dense group; otherwise the groups that a balanced choice
-// leaves with a row, and half a tile of padding in each once groups outgrow half a tile
-inline double expected_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
-  if (dense) return (double)((rows + BM - 1) / BM);
-  const double groups = (double)E * (1.0 - std::exp(-(double)rows / (double)E)), mean = (double)rows / groups;
-  return groups * (mean > BM / 2 ? mean / BM + 0.5 : 1.0);
-}
-
 // Streaming tiles (grouped_gemm_skinny.hpp) while they find a CU each: of the shapes with at most one tile per CU
 // the one with the most tiles, so that the matrices are drawn through as many CUs as possible.  us at 1 token,
 // 64 experts top-8, 2048 -> 1408: gate/up 21 (64-column tiles, 176 of them; 128 columns 27, the 64-row LDS tiles
@@ -327,23 +317,12 @@ inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dua
 // and 78).
 constexpr int64_t kTinyGroupRows = 52;  // four or fewer in a hundred groups above 64
 
-// With fewer 128-row tiles than CUs: gate/up of 1024 tokens, shared 2816: 41 us against 50 in 256-row tiles;
-// with more, two rounds of half tiles: 2048 tokens 77 against 52.
-// Down: one half tile per CU 40 us against 63 (2048 tokens, shared 2816; 64-deep steps 41), two per CU with
-// 64-deep steps 55 against 64 (4096 tokens; 32-deep 69), and so on by rounds: a round of 512 half tiles takes
-// 0.57 of a round of 256 whole ones, a last round of at most 256 of them 0.42, the launch 0.12 more; half tiles
-// read their operands twice as often, so they are taken only where that is 15 % less.  8192 rows x 2048 -> 1024 in
-// 8 groups: 57 against 56 (576 tiles, whole ones kept); 16384 rows: 84 against 100 (1088 against 272 tiles: the
-// whole ones start a second round for 16 of them).
+// Half tiles where they pay (half_tiles); gate/up only with at most one per CU: 1024 tokens, shared 2816: 41 us
+// against 50 in 256-row tiles; with more, two rounds of half tiles: 2048 tokens 77 against 52.
 inline Tiles pick_large(int64_t rows, int64_t E, bool dense, int64_t N, bool dual) {
-  const double cus = (double)persistent_grid_size();
-  const double half = expected_mtiles(rows, E, dense, 128) * (double)((N + 127) / 128);
-  if (half <= cus) return Tiles::kHalf;
-  if (dual) return Tiles::kFull;
-  const double full = expected_mtiles(rows, E, dense, 256) * (double)((N + 255) / 256);
-  const double rounds = std::floor(half / (2 * cus)), rest = half - rounds * 2 * cus;
-  const double half_cost = 0.12 + 0.57 * rounds + (rest <= 0.0 ? 0.0 : (rest <= cus ? 0.42 : 0.57));
-  return 1.15 * half_cost < std::ceil(full / cus) ? Tiles::kHalfDeep : Tiles::kFull;
+  const HalfTiles half = half_tiles(rows, E, dense, N);
+  if (half == HalfTiles::kOnePerCu) return Tiles::kHalf;
+  return half == HalfTiles::kNone || dual ? Tiles::kFull : Tiles::kHalfDeep;
 }
 
 inline Tiles pick_tiles(int64_t rows, int64_t Kdim, int64_t E, bool dense, int64_t N, bool dual) {

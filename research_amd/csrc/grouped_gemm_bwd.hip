@@ -4,6 +4,7 @@
 // of their own, see grouped_gemm_bwd.hpp.
 #include "gemm_launch.hpp"
 #include "grouped_gemm_bwd.hpp"
+#include "grouped_gemm_stream.hpp"
 
 #include <algorithm>
 #include <mutex>
@@ -158,12 +159,37 @@ int launch_nt_fast(const void* a0, const void* a1, const void* b0, const void* b
   const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles_grid = gemm_grid(mtiles, nt);
   if (tiles_grid >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");
-  // persistent workgroups: one per CU, each walking its share of the tiles
-  const int64_t grid = tiles_grid > persistent_grid_size() ? persistent_grid_size() : tiles_grid;
+  // persistent workgroups: one per CU (two with half the LDS), each walking its share of the tiles
+  const int64_t most = (2 * Cfg::SMEM_BYTES <= 160 * 1024 ? 2 : 1) * persistent_grid_size();
+  const int64_t grid = std::min(tiles_grid, most);
   kernel<<<(unsigned)grid, Cfg::NT, Cfg::SMEM_BYTES, stream>>>(
       static_cast<const uint16_t*>(a0), static_cast<const uint16_t*>(a1), static_cast<const uint16_t*>(b0),
       static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim,
       (int)N, (int)mtiles, (int)nt, row_map, row_div, (int)a_rows, segs);
+  return JTMOE_OK;
+}
+
+// needs (K / 64, rounded up) * segs >= 2 * NSTAGE and a result of at most 0x7ffe0000 bytes
+template <typename Cfg>
+int launch_nt_stream(const void* a0, const void* a1, const void* b0, const void* b1, void* c,
+                     const int32_t* group_sizes, const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N,
+                     int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream) {
+  using L = StreamLayout<Cfg>;
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  auto kernel = grouped_gemm_stream_nt_kernel<Cfg>;
+  std::call_once(once, [&] { attr_err = allow_lds(kernel, L::kSmemBytes); });
+  if (attr_err != hipSuccess)
+    return fail(JTMOE_ELAUNCH, "grouped gemm (nt): hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
+  const int64_t mtiles = group_sizes == nullptr ? (rows + Cfg::BM - 1) / Cfg::BM : max_m_tiles(rows, E, Cfg::BM);
+  const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
+  const int64_t tiles_grid = gemm_grid(mtiles, nt);
+  if (tiles_grid >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");
+  const PersistentSchedule ps = persistent_schedule(tiles_grid, persistent_grid_size(), 4);
+  kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes, stream>>>(
+      static_cast<const uint16_t*>(a0), static_cast<const uint16_t*>(a1), static_cast<const uint16_t*>(b0),
+      static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim,
+      (int)N, (int)mtiles, (int)nt, row_map, row_div, (int)a_rows, segs, ps.window, ps.chunk);
   return JTMOE_OK;
 }
 
@@ -177,6 +203,13 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
   const bool fast = dtype == JTMOE_BF16 && Kdim % 8 == 0 && N % 8 == 0 && N * Kdim < kOperandLimit &&
                     (row_map ? a_rows : rows) * Kdim < kOperandLimit && aligned16(a0) && aligned16(b0) &&
                     (segs == 1 || (aligned16(a1) && aligned16(b1))) && aligned16(c);
+  const HalfTiles half = fast && rows * N * 2 <= (int64_t)0x7ffe0000 ? half_tiles(rows, E, dense, N) : HalfTiles::kNone;
+  if (half == HalfTiles::kOnePerCu && (Kdim + 63) / 64 * segs >= 2 * DgradHalfDeepCfg::NSTAGE)
+    return launch_nt_stream<DgradHalfDeepCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map,
+                                              row_div, a_rows, segs, stream);
+  if (half != HalfTiles::kNone)
+    return launch_nt_fast<DgradHalfCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div,
+                                        a_rows, segs, stream);
   if (fast && Kdim % 64 == 0)
     return launch_nt_fast<DgradCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div,
                                     a_rows, segs, stream);

@@ -742,6 +742,11 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_tn_kernel(
 // Configurations the library launches.
 using DgradCfg = NtGemmCfg<256, 256, 2, 4, 16 + 64 + 32768>;   // data gradients: 256 x 256 tiles
 using DgradTailCfg = NtGemmCfg<256, 256, 2, 4, 16 + 64 + 32768 + 65536>;  // the same for K % 64 != 0
+// half tiles, two workgroups per CU, by the rule of half_tiles (gemm_common.hpp): 16384 rows in 64 groups x 2048 ->
+// 1408 (1760 half tiles): 158 us against 171; 8192 rows in 8 groups x 1024 -> 2048 (1088): 53 against 59; 16384
+// rows in 8 groups x 4096 -> 1024 (1056): 174 against 190; 4096 rows x 1024 -> 2048 in one group (512): 21
+// against 30.  The streaming kernel in the same tiles, two stages or four, is 2 to 20 % slower on these.
+using DgradHalfCfg = NtGemmCfg<128, 128, 2, 2, 16 + 64 + 32768 + 65536>;
 // narrow LDS blocks: the fastest layout when the operands are streamed (1.52 vs 1.60 ms for the
 // gate/up product of the C3 shape); the wide blocks pay off only when rows are gathered.
 // Four stages of 32 rows against two of 64 (the same LDS): 1.39-1.43 against 1.47-1.49 ms for the gate/up

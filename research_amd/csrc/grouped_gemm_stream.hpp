@@ -68,7 +68,6 @@ __device__ __forceinline__ void stream_gemm_body(
   static_assert(!kNT || !kDual, "the transposed-B form has one output per tile");
   // K may end inside a step (the interleaved steady part leaves no room for a branch: every load checks)
   constexpr bool kTail = (Cfg::OPT & 65536) != 0;
-  static_assert(!kTail || !kNT, "the transposed-B form takes whole steps");
   static_assert(!kNT || (BN * CPRA) % NT == 0, "the B tile must divide evenly over the threads");
   // Timing experiments of the stand-alone check's time_ablation mode, which bounds what any schedule of
   // this loop can reach (wrong results by construction, never launched by the library): OPT & 256 leaves out the operand loads of the steady part of the k loop, OPT & 512 its
@@ -202,11 +201,13 @@ __device__ __forceinline__ void stream_gemm_body(
     if constexpr (kNT) {
       const bool second = kt >= nk1;  // uniform: the step belongs to the second segment
       const int k0 = (second ? kt - nk1 : kt) * BK;
+      const bool outside = kTail && k0 + a_c * 8 >= Kdim;  // both tiles: this lane's chunk lies past the end of the row
       if (i < Cfg::A_LOADS)
-        buffer_load_lds16(second ? p.a_rsrc[1] : p.a_rsrc[0], base + i * NT * 16, p.a_voff[i], k0 * 2);
+        buffer_load_lds16(second ? p.a_rsrc[1] : p.a_rsrc[0], base + i * NT * 16, outside ? kOutside : p.a_voff[i],
+                          k0 * 2);
       else
         buffer_load_lds16(second ? p.b_rsrc[1] : p.b_rsrc[0], base + Cfg::A_BYTES + (i - Cfg::A_LOADS) * NT * 16,
-                          p.b_voff[i - Cfg::A_LOADS], k0 * 2);
+                          outside ? kOutside : p.b_voff[i - Cfg::A_LOADS], k0 * 2);
     } else {
       const int k0 = kt * BK;
       if (i < Cfg::A_LOADS) {
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_kernel(
 }
 
 // The transposed-B form: the arguments of grouped_gemm_nt_kernel (grouped_gemm_bwd.hpp) plus the schedule.
-// Requirements: (Kdim / BK) * segs >= 2 * NSTAGE, and those of the kernel above.
+// Requirements: (Kdim / BK, rounded up with OPT & 65536) * segs >= 2 * NSTAGE, and those of the kernel above.
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_nt_kernel(
     const uint16_t* __restrict__ A0, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
@@ -462,5 +463,9 @@ using DownStream2Cfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 32768
 // Checked and timed by the stand-alone check (time_stream_nt) against grouped_gemm_nt_kernel, which
 // the library launches: the transposed-B form measures equal or slower there.
 using DgradStreamCfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128>;
+// The same in half tiles, launched where a data gradient has at most one of them per CU: nothing else runs on the CU,
+// so four 64-deep stages (131 KB) keep its loads going.  4096 rows x 4096 -> 1024: 40 us, two 64-deep stages with
+// two workgroups per CU 59, four 32-deep ones 49, 256 x 256 tiles 93; 2048 rows x 5632 -> 2048: 55, 79, 67 and 124.
+using DgradHalfDeepCfg = DmaGemmCfg<128, 128, 64, 2, 2, false, 4, 16 + 128 + 65536>;
 
 }  // namespace jtmoe

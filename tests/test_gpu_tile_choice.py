@@ -29,6 +29,7 @@ pytestmark = pytest.mark.gpu
     (350, 264, 40, 4, 136),      # 64-row LDS tiles
     (700, 296, 4, 2, 520),       # 128-row tiles with gathered rows, ten 32-deep steps and one chunk
     (2600, 328, 8, 2, 264),      # 128-row tiles of the down product, several per workgroup
+    (512, 72, 64, 8, 1416),      # 128-row tiles of a data gradient, several per workgroup, a ragged second k step
 ])
 def test_grouped_products_on_every_kernel(gpu, tokens, hidden, experts, top_k, inter):
     P.test_grouped_swiglu_matches_oracle(gpu, tokens, hidden, experts, top_k, inter, "bf16")
