@@ -605,7 +605,7 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
   // the dispatch plan; the down launch then picks the routed rows.
   hipStream_t main_stream = as_stream(stream);
   const bool decode = !train && decode_dense_supported(T, H, E, K, I, dtype);
-  bool stats_done = false, plan_done = false;
+  bool stats_done = false, plan_done = false, shared_done = false;
   int rc;
   if (decode) {
     rc = launch_decode_gate_up_router(x, w_router, expert_bias, gate, up, w.act, T, H, E, K, I, route_scale,
@@ -619,9 +619,12 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
     stage_mark(kStageDown, main_stream);
     rc = check_launch("grouped gemm");
   } else {
+    const SharedExperts shared{shared_gate, shared_up, shared_down, Is, w.shared_act, w.shared_y, shared_gate_pre,
+                               shared_up_pre};
     rc = router_for_layer(x, w_router, expert_bias, T, H, E, K, route_scale, dtype, expert_ids, weights, scores,
                           expert_counts, importance, group_sizes, offsets, source_order, inverse, w.router,
-                          w.router_bytes, score_func, &stats_done, &plan_done, main_stream);
+                          w.router_bytes, score_func, &stats_done, &plan_done, main_stream, Is > 0 ? &shared : nullptr,
+                          &shared_done);
     if (rc) return rc;
     stage_mark(kStageRouter, main_stream);
     rc = dispatch_for_layer(expert_ids, weights, (T > 0 && !gather) ? x : nullptr, T, H, E, K, dtype, group_sizes,
@@ -641,7 +644,7 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
                                 w.packed_y, stream);
     if (rc) return rc;
   }
-  if (Is > 0) {
+  if (Is > 0 && !shared_done) {
     if (train)
       rc = jtmoe_shared_swiglu_train(x, shared_gate, shared_up, shared_down, T, H, Is, dtype, shared_gate_pre,
                                      shared_up_pre, w.shared_act, w.shared_y, stream);

@@ -123,6 +123,15 @@ int dispatch_for_layer(const int32_t* expert_ids, const void* weights, const voi
                        int32_t* inverse, void* packed_x, float* expert_counts, float* importance, void* workspace,
                        bool want_stats, bool plan_done, hipStream_t stream);
 
+// The shared experts of a layer call.  A router of a few tokens takes them along in its own two launches
+// (*shared_done): neither needs the other's results, and the router's workgroups leave most CUs idle.
+// gate_pre / up_pre: where a training forward keeps the two rounded products, or null.
+struct SharedExperts {
+  const void *gate, *up, *down;
+  int64_t Is;
+  void *act, *y, *gate_pre, *up_pre;
+};
+
 // router.hip: the router as the layer runs it, with the dispatch plan behind it where that is free.
 // On return *stats_done says whether expert_counts / importance have been written (the small-batch
 // path gets them from its one finishing workgroup); if not, the caller's dispatch computes them from
@@ -133,8 +142,11 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
                      int64_t K, double route_scale, int dtype, int32_t* expert_ids, void* weights, float* scores,
                      float* expert_counts, float* importance, int32_t* group_sizes, int32_t* offsets,
                      int32_t* source_order, int32_t* inverse, void* workspace, size_t workspace_bytes,
-                     int score_func, bool* stats_done, bool* plan_done, hipStream_t stream);
-
+                     int score_func, bool* stats_done, bool* plan_done, hipStream_t stream,
+                     const SharedExperts* shared = nullptr, bool* shared_done = nullptr);
+// grouped_gemm.hip: whether both products of the shared experts run in the streaming tiles of 16 rows x 64 columns
+// (the ones that can share the router's launches) at these sizes and pointers.
+bool shared_in_skinny_tiles(const void* x, const SharedExperts& shared, int64_t T, int64_t H);
 
 // grouped_gemm.hip: the two grouped launches on packed rows fetched through the permutation (packed row j is
 // row source_order[j] / K of x), any shape and alignment as long as x is smaller than 1 GiB.

@@ -448,6 +448,12 @@ int launch_down_from_all_tokens(const void* act_full, const void* down, const in
                           /*a_group_rows=*/T);
 }
 
+bool shared_in_skinny_tiles(const void* x, const SharedExperts& s, int64_t T, int64_t H) {
+  return fast_ok(x, s.gate, s.up, s.act, H, s.Is) && fast_ok(s.act, s.down, nullptr, s.y, s.Is, H) &&
+         aligned16(s.gate_pre) && aligned16(s.up_pre) && pick_tiles(T, H, 1, true, s.Is, true) == Tiles::kSkinny12 &&
+         pick_tiles(T, s.Is, 1, true, H, false) == Tiles::kSkinny12;
+}
+
 // ---- the gathering launch pair as the layer uses it (declared in common.hpp) ----
 int launch_swiglu_gather(const void* x, const int32_t* source_order, const void* gate, const void* up,
                          const void* down, const int32_t* group_sizes, const int32_t* offsets, int64_t T, int64_t K,
