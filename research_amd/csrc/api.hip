@@ -434,6 +434,7 @@ struct LayerWorkspace {
   size_t dispatch_bytes;
   void* packed_x;
   void* act;
+  size_t act_bytes;
   void* packed_y;
   void* shared_act;
   void* shared_y;
@@ -454,7 +455,8 @@ LayerWorkspace carve_layer(void* base, int64_t T, int64_t H, int64_t E, int64_t 
   w.packed_x = jtmoe_grouped_swiglu_gather_supported(T, H, I, dtype) ? nullptr : c.take(A * (size_t)H * b);
   // (the decode path keeps the activations of all tokens through every expert)
   const size_t act_rows = decode_dense_supported(T, H, E, K, I, dtype) ? (size_t)E * (size_t)T : A;
-  w.act = c.take((act_rows > A ? act_rows : A) * (size_t)I * b);
+  w.act_bytes = (act_rows > A ? act_rows : A) * (size_t)I * b;
+  w.act = c.take(w.act_bytes);
   w.packed_y = c.take(A * (size_t)H * b);
   w.shared_act = Is > 0 ? c.take((size_t)T * (size_t)Is * b) : nullptr;
   w.shared_y = Is > 0 ? c.take((size_t)T * (size_t)H * b) : nullptr;
@@ -623,8 +625,8 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
                                shared_up_pre};
     rc = router_for_layer(x, w_router, expert_bias, T, H, E, K, route_scale, dtype, expert_ids, weights, scores,
                           expert_counts, importance, group_sizes, offsets, source_order, inverse, w.router,
-                          w.router_bytes, score_func, &stats_done, &plan_done, main_stream, Is > 0 ? &shared : nullptr,
-                          &shared_done);
+                          w.router_bytes, score_func, &stats_done, &plan_done, main_stream, w.act, w.act_bytes,
+                          Is > 0 ? &shared : nullptr, &shared_done);
     if (rc) return rc;
     stage_mark(kStageRouter, main_stream);
     rc = dispatch_for_layer(expert_ids, weights, (T > 0 && !gather) ? x : nullptr, T, H, E, K, dtype, group_sizes,

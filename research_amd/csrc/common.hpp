@@ -137,13 +137,13 @@ struct SharedExperts {
 // path gets them from its one finishing workgroup); if not, the caller's dispatch computes them from
 // the ids and weights.  *plan_done says whether group_sizes / offsets / source_order / inverse have
 // been written as well (the finishing workgroup of the small-batch router goes on to the plan while
-// it still holds the ids in LDS).
+// it still holds the ids in LDS).  scratch: memory that nothing else uses until the router is done.
 int router_for_layer(const void* x, const void* w_router, const float* expert_bias, int64_t T, int64_t H, int64_t E,
                      int64_t K, double route_scale, int dtype, int32_t* expert_ids, void* weights, float* scores,
                      float* expert_counts, float* importance, int32_t* group_sizes, int32_t* offsets,
                      int32_t* source_order, int32_t* inverse, void* workspace, size_t workspace_bytes,
-                     int score_func, bool* stats_done, bool* plan_done, hipStream_t stream,
-                     const SharedExperts* shared = nullptr, bool* shared_done = nullptr);
+                     int score_func, bool* stats_done, bool* plan_done, hipStream_t stream, void* scratch = nullptr,
+                     size_t scratch_bytes = 0, const SharedExperts* shared = nullptr, bool* shared_done = nullptr);
 // grouped_gemm.hip: whether both products of the shared experts run in the streaming tiles of 16 rows x 64 columns
 // (the ones that can share the router's launches) at these sizes and pointers.
 bool shared_in_skinny_tiles(const void* x, const SharedExperts& shared, int64_t T, int64_t H);

@@ -711,6 +711,7 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
 // make a workgroup, so small batches spread over more CUs.
 // ---------------------------------------------------------------------------
 constexpr int kSplitMaxTokens = 256;
+constexpr int kMidMaxTokens = 2560;  // with the slices in workgroups of their own, a layer call (launch_router)
 
 __host__ __device__ inline size_t router_split_smem_bytes(int E, int K) {
   const size_t w = (size_t)2 * kSplitKC * router_w_stride(E) * 2;
@@ -879,6 +880,26 @@ __global__ __launch_bounds__(256) void router_mfma_split_kernel(
                                   partial_out, score_func, (int)blockIdx.x, (int)blockIdx.y);
 }
 
+// the slices of partial sums of n tokens, added in slice order and rounded to bf16 (the projection's output dtype),
+// into the score tile
+template <int kThreads>
+__device__ __forceinline__ void add_slices(const RouterSmem& sm, const float* __restrict__ partial, int slices,
+                                           size_t plane, int n, int E) {
+  const int stride = E + 1;
+#pragma unroll 4
+  for (int idx = threadIdx.x; idx < n * E; idx += kThreads) {
+    const int t = idx / E, e = idx - t * E;
+    float part[kPartialMaxSlices];  // all slices requested before the first is needed
+#pragma unroll
+    for (int sl = 0; sl < kPartialMaxSlices; ++sl) part[sl] = sl < slices ? partial[sl * plane + idx] : 0.0f;
+    float v = part[0];
+#pragma unroll
+    for (int sl = 1; sl < kPartialMaxSlices; ++sl)
+      if (sl < slices) v += part[sl];
+    sm.tile[t * stride + e] = round_to_bf16(v);
+  }
+}
+
 // Second half of the small-batch router: one workgroup adds the slices of partial sums in slice
 // order, rounds to bf16 (the projection's output dtype) and runs the epilogue for every token of
 // the call, so the statistics need neither the zeroing nor the finalising launch.
@@ -896,20 +917,7 @@ __device__ __forceinline__ void router_finish_body(
     int32_t* __restrict__ inverse, int score_func) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   RouterSmem sm = router_smem(smem_raw, E, K, kTok);
-  const int stride = E + 1;
-  const size_t plane = (size_t)tokens * E;
-#pragma unroll 4
-  for (int idx = threadIdx.x; idx < tokens * E; idx += 4 * kTok) {
-    const int t = idx / E, e = idx - t * E;
-    float part[kPartialMaxSlices];  // all slices requested before the first is needed
-#pragma unroll
-    for (int sl = 0; sl < kPartialMaxSlices; ++sl) part[sl] = sl < slices ? partial[sl * plane + idx] : 0.0f;
-    float v = part[0];
-#pragma unroll
-    for (int sl = 1; sl < kPartialMaxSlices; ++sl)
-      if (sl < slices) v += part[sl];
-    sm.tile[t * stride + e] = round_to_bf16(v);
-  }
+  add_slices<4 * kTok>(sm, partial, slices, (size_t)tokens * E, tokens, E);
   __syncthreads();
   router_epilogue<bf16_raw, kTok, 4 * kTok>(sm, bias, 0, tokens, E, K, route_scale, ids, weights, scores, logits_out,
                                             RouterScratch{}, score_func, counts, importance);
@@ -930,6 +938,22 @@ __global__ __launch_bounds__(4 * kTok) void router_finish_kernel(
     int32_t* __restrict__ inverse, int score_func) {
   router_finish_body<kTok, kPlan>(partial, slices, bias, tokens, E, K, route_scale, ids, weights, scores, logits_out,
                                   counts, importance, group_sizes, offsets, source_order, inverse, score_func);
+}
+
+// Second half of a middle-sized layer call: a workgroup per 16 tokens adds up their slices and runs the epilogue
+// (the statistics and the plan are the dispatch's).
+template <int kTok, int kThreads>
+__global__ __launch_bounds__(kThreads) void router_finish_blocks_kernel(
+    const float* __restrict__ partial, int slices, const float* __restrict__ bias, int tokens, int E, int K,
+    float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights, float* __restrict__ scores,
+    int score_func) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  RouterSmem sm = router_smem(smem_raw, E, K, kTok);
+  const int t0 = (int)blockIdx.x * kTok;
+  add_slices<kThreads>(sm, partial + (size_t)t0 * E, slices, (size_t)tokens * E, min(kTok, tokens - t0), E);
+  __syncthreads();
+  router_epilogue<bf16_raw, kTok, kThreads>(sm, bias, t0, tokens, E, K, route_scale, ids, weights, scores, nullptr,
+                                            RouterScratch{}, score_func);
 }
 
 inline size_t router_arrivals_offset(int64_t E) {
@@ -1020,7 +1044,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
 // The two launches of the small-batch router with the shared experts beside it: the gate/up tiles next to the
 // workgroups of the partial sums, the down tiles next to the finishing workgroup.  Each launch is bound by one
 // workgroup's own chain of dependent steps, on a few dozen CUs, and nothing of one is needed by the other.
-// One token, 2048 wide, 64 experts, shared 2816: 4.4 + 10.6 us (router) and 18 + 13.5 us (shared) in four launches.
+// One token, 2048 wide, 64 experts, shared 2816: 17.8 + 14.3 us, against 4.4 + 10.6 (router) and 18 + 13.5 (shared) in
+// four launches.
 // ---------------------------------------------------------------------------
 using SharedGateUpCfg = SkinnyCfg<1, 2, true>;
 using SharedDownCfg = SkinnyCfg<1, 2, false>;
@@ -1072,6 +1097,8 @@ struct LayerPlan {
   int32_t* inverse;
   bool stats_done;
   bool plan_done;
+  void* scratch;  // memory of the layer that nothing uses until the router is done
+  size_t scratch_bytes;
 };
 
 template <typename T, bool kFromLogits>
@@ -1168,6 +1195,44 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
       }
       if (stats) router_finalize_kernel<<<1, 256, 0, stream>>>(ws, (int)E, counts, importance);
       return check_launch("router");
+    }
+    // Middle-sized layer calls: a 64-token workgroup walks all of H, 26 us (E = 64) and 40 us (E = 128) whether
+    // there are 300 tokens or 8000; up to kMidMaxTokens the slices are computed in workgroups of their own, in the
+    // layer's memory, and a workgroup per 16 tokens finishes.  us at 2048 columns, split + finish against one
+    // launch: E = 64: 300 tokens 4.4 + 9.9 / 23.6, 1024: 5.7 + 10.2 / 26.1, 2048: 9.1 + 10.6 / 25.9, 4096: 16.1 + 11.4
+    // / 27.7; E = 128: 5.7 + 15.6 / 37.6, 7.9 + 15.9 / 40.4, 13.5 + 16.5 / 40.0, 24.4 + 16.8 / 41.3.  E = 16 at 1024
+    // columns: 4.4 + 4.3 / 10.1, which the gap between the launches takes back.
+    const int slice_rows = router_slice_rows((int)H);
+    const int slices = (int)((H + slice_rows - 1) / slice_rows);
+    if (layer && tokens <= kMidMaxTokens && (E == 64 || E == 128) && H % kSplitKC == 0 && H >= 2048 &&
+        (size_t)slices * tokens * E * sizeof(float) <= layer->scratch_bytes) {
+      const size_t smem = (size_t)2 * kSplitKC * router_w_stride((int)E) * 2;
+      const size_t fsmem = router_smem_bytes((int)E, (int)K, 16);
+      if (fsmem <= 160 * 1024) {
+        float* const partial = static_cast<float*>(layer->scratch);
+        const int blocks = (int)((tokens + 15) / 16);
+#define JT_PARTIAL_CASE(NB)                                                                                  \
+  case NB * 16: {                                                                                            \
+    auto kernel = router_mfma_split_kernel<NB, true>;                                                        \
+    const int rc = set_max_smem(kernel, smem);                                                               \
+    if (rc) return rc;                                                                                       \
+    kernel<<<dim3(blocks, slices), 256, smem, stream>>>(                                                     \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
+        (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, nullptr, partial,      \
+        score_func);                                                                                         \
+  } break;
+        switch ((int)E) {
+          JT_PARTIAL_CASE(4)
+          JT_PARTIAL_CASE(8)
+        }
+#undef JT_PARTIAL_CASE
+        auto finish = router_finish_blocks_kernel<16, 256>;
+        const int rc = set_max_smem(finish, fsmem);
+        if (rc) return rc;
+        finish<<<blocks, 256, fsmem, stream>>>(partial, slices, bias, (int)tokens, (int)E, (int)K, (float)route_scale,
+                                               ids, static_cast<bf16_raw*>(weights), scores, score_func);
+        return check_launch("router");
+      }
     }
     // four waves (64 tokens) per workgroup: the waves share the work of bringing in the router
     // matrix, which every workgroup reads in full
@@ -1383,8 +1448,8 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
                      int64_t K, double route_scale, int dtype, int32_t* expert_ids, void* weights, float* scores,
                      float* expert_counts, float* importance, int32_t* group_sizes, int32_t* offsets,
                      int32_t* source_order, int32_t* inverse, void* workspace, size_t workspace_bytes,
-                     int score_func, bool* stats_done, bool* plan_done, hipStream_t s, const SharedExperts* shared,
-                     bool* shared_done) {
+                     int score_func, bool* stats_done, bool* plan_done, hipStream_t s, void* scratch,
+                     size_t scratch_bytes, const SharedExperts* shared, bool* shared_done) {
   int rc = validate_router(T, H, E, K, route_scale, dtype, true);
   if (rc) return rc;
   JT_REQUIRE(score_func_ok(score_func), "router: unknown score function %d", score_func);
@@ -1393,7 +1458,7 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
   JT_REQUIRE(group_sizes && offsets && (T == 0 || (source_order && inverse)), "router: null pointer argument");
   if (workspace_bytes < jtmoe_router_workspace_bytes(E))
     return fail(JTMOE_EWORKSPACE, "router: workspace %zu < %zu bytes", workspace_bytes, jtmoe_router_workspace_bytes(E));
-  LayerPlan layer{group_sizes, offsets, source_order, inverse, false, false};
+  LayerPlan layer{group_sizes, offsets, source_order, inverse, false, false, scratch, scratch_bytes};
   if (shared && router_takes_shared(x, w_router, *shared, T, H, E, K, dtype)) {
     *stats_done = *plan_done = *shared_done = true;
     return launch_router_with_shared(x, w_router, expert_bias, *shared, T, H, E, K, route_scale, score_func, expert_ids,
