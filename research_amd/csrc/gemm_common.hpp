@@ -217,6 +217,22 @@ inline double expected_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
   return groups * (mean > BM / 2 ? mean / BM + 0.5 : 1.0);
 }
 
+// The same where the tiles are as tall as a group is: rows per group spread evenly over mean +- 3 sqrt(mean) (top-k
+// groups of random rows lie within that), so that groups of 162 rows count as one 256-row tile and two of 128, and
+// not as 1.13 and 1.77.  From the latter the half tiles looked like 15 % less than three rounds where the whole
+// ones need two: 1300 tokens top-8, 64 experts of 1408, 2048 wide 332 us a layer call against 311 without them.
+// How far the groups really spread is not known on the host, so half tiles have to pay by either estimate.
+inline double spread_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
+  if (dense) return (double)((rows + BM - 1) / BM);
+  const double groups = (double)E * (1.0 - std::exp(-(double)rows / (double)E)), mean = (double)rows / groups;
+  const double hi = mean + 3.0 * std::sqrt(mean), lo = std::fmax(0.0, mean - 3.0 * std::sqrt(mean));
+  auto tiles_upto = [BM](double x) {  // integral of ceil(n / BM) over n from 0 to x
+    const double q = std::floor(x / BM);
+    return BM * q * (q + 1.0) / 2.0 + (x - q * BM) * (q + 1.0);
+  };
+  return groups * (tiles_upto(hi) - tiles_upto(lo)) / (hi - lo);
+}
+
 // 128 x 128 tiles against 256 x 256 ones, by rounds over the CUs: a round of 512 half tiles takes 0.57 of a round of
 // 256 whole ones, a last round of at most 256 of them 0.42, the launch 0.12 more; half tiles read their operands
 // twice as often, so beyond one per CU they are taken only where that is 15 % less.  Down products: one half tile
@@ -228,12 +244,17 @@ inline double expected_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
 enum class HalfTiles { kNone, kOnePerCu, kRounds };
 inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N) {
   const double cus = (double)persistent_grid_size();
-  const double half = expected_mtiles(rows, E, dense, 128) * (double)((N + 127) / 128);
-  if (half <= cus) return HalfTiles::kOnePerCu;
-  const double full = expected_mtiles(rows, E, dense, 256) * (double)((N + 255) / 256);
-  const double rounds = std::floor(half / (2 * cus)), rest = half - rounds * 2 * cus;
-  const double half_cost = 0.12 + 0.57 * rounds + (rest <= 0.0 ? 0.0 : (rest <= cus ? 0.42 : 0.57));
-  return 1.15 * half_cost < std::ceil(full / cus) ? HalfTiles::kRounds : HalfTiles::kNone;
+  const double half_n = (double)((N + 127) / 128), full_n = (double)((N + 255) / 256);
+  if (expected_mtiles(rows, E, dense, 128) * half_n <= cus) return HalfTiles::kOnePerCu;
+  auto pays = [cus](double half, double full) {
+    const double rounds = std::floor(half / (2 * cus)), rest = half - rounds * 2 * cus;
+    const double half_cost = 0.12 + 0.57 * rounds + (rest <= 0.0 ? 0.0 : (rest <= cus ? 0.42 : 0.57));
+    return 1.15 * half_cost < std::ceil(full / cus);
+  };
+  return pays(expected_mtiles(rows, E, dense, 128) * half_n, expected_mtiles(rows, E, dense, 256) * full_n) &&
+                 pays(spread_mtiles(rows, E, dense, 128) * half_n, spread_mtiles(rows, E, dense, 256) * full_n)
+             ? HalfTiles::kRounds
+             : HalfTiles::kNone;
 }
 
 }  // namespace jtmoe
