@@ -253,16 +253,7 @@ int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const 
                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, hipStream_t stream,
                   const int32_t* row_map = nullptr, int row_div = 1, int64_t a_rows = 0, void* save0 = nullptr,
                   void* save1 = nullptr, int64_t a_group_rows = 0) {
-  if constexpr (Cfg::SMEM_BYTES > 64 * 1024) {
-    static std::once_flag once;
-    static hipError_t attr_err = hipSuccess;
-    std::call_once(once, [] {
-      attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&grouped_gemm_skinny_kernel<Cfg>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::SMEM_BYTES);
-    });
-    if (attr_err != hipSuccess)
-      return fail(JTMOE_ELAUNCH, "grouped gemm: kernel set-up: %s", hipGetErrorString(attr_err));
-  }
+  static_assert(Cfg::SMEM_BYTES <= 64 * 1024, "launched without a raised limit");
   const int64_t mtiles = group_sizes == nullptr ? (rows + Cfg::BM - 1) / Cfg::BM : max_m_tiles(rows, E, Cfg::BM);
   const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t grid = gemm_grid(mtiles, nt);
@@ -277,34 +268,33 @@ int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const 
 
 // ---- which kernel takes a product ------------------------------------------------------------------------
 // All times below: rows of T tokens in E groups by a balanced top-k, matrices cold, launch overhead included.
-enum class Tiles { kSkinny11, kSkinny12, kSkinny21, kSkinny22, kSkinny41, kTiny, kHalf, kHalfDeep, kFull };
+enum class Tiles { kSkinny11, kSkinny12, kSkinny22, kTiny, kHalf, kHalfDeep, kFull };
 
 // Streaming tiles (grouped_gemm_skinny.hpp) while they find a CU each: of the shapes with at most one tile per CU
-// the one with the most tiles, so that the matrices are drawn through as many CUs as possible.  us at 1 token,
-// 64 experts top-8, 2048 -> 1408: gate/up 21 (64-column tiles, 176 of them; 128 columns 27, the 64-row LDS tiles
-// 49), down 14 (15; 38); shared experts of 2816: 20 and 12 (25 and 21; 62 and 86) at 1 token, 20 and 16 (30 and
-// 21; 62 and 86) at 64, 27 and 21 in 32-row tiles at 128 (31 and 22 in 16-row ones).  With more than 256
-// tiles, while groups hold a row or four: 73 against 77 and 41 against 45 us at 8 tokens; from 16 tokens on
-// (mean 2.3 of 64 groups) the two are equal within 2 %.  Beyond, a group's second tile reads its matrix again:
-// 154 against 111 us for gate/up at 128 tokens.
-inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dual, Tiles* out) {
+// the one with the most tiles, so that the matrices are drawn through as many CUs as possible.  us for gate/up and
+// down together, 2048 -> 1408, 64 experts top-8, 1 token: 35 against 87 in 64-row LDS tiles; shared experts of 2816:
+// 34 at 1 token, 36 at 64 (148 in 64-row LDS tiles), 43 at 130 with 32-row tiles (58 without them).  Tiles of 128
+// columns and 32 or 64 rows do not pay where half tiles can be had: 68 against 53 at 387 tokens, 91 against 63 at 700.
+// With more tiles than CUs they pay while few groups need a second product's worth of rows, up to a mean of two
+// per group reached: 64 experts 100 against 127 at 4 tokens, 130 against 138 at 8 (mean 1.6), but 177 against
+// 166 at 15 (2.2) and 187 against 174 at 28 (3.6); 128 experts of 768: 163 against 166 at 20 (1.75), equal within
+// 1 % from 30 on.
+inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, Tiles* out) {
   struct Shape {
     Tiles id;
     int RB, BN;
   };
-  constexpr Shape shapes[] = {{Tiles::kSkinny12, 1, 64}, {Tiles::kSkinny22, 2, 64}, {Tiles::kSkinny11, 1, 128},
-                              {Tiles::kSkinny21, 2, 128}, {Tiles::kSkinny41, 4, 128}};
+  constexpr Shape shapes[] = {{Tiles::kSkinny12, 1, 64}, {Tiles::kSkinny22, 2, 64}, {Tiles::kSkinny11, 1, 128}};
   const double cus = (double)persistent_grid_size();
   double most = 0.0;
   for (const Shape& s : shapes) {
-    if (s.id == Tiles::kSkinny41 && dual) continue;  // 512 tokens, shared 2816: 45 us against 41 in half tiles
     const double tiles = expected_mtiles(rows, E, dense, 16 * s.RB) * (double)((N + s.BN - 1) / s.BN);
     if (tiles <= cus && tiles > most) {
       most = tiles;
       *out = s.id;
     }
   }
-  if (most == 0.0 && !dense && (double)rows <= 4.0 * expected_mtiles(rows, E, false, 16)) {
+  if (most == 0.0 && !dense && (double)rows <= 2.0 * expected_mtiles(rows, E, false, 16)) {
     *out = Tiles::kSkinny11;
     return true;
   }
@@ -325,12 +315,9 @@ inline Tiles pick_large(int64_t rows, int64_t E, bool dense, int64_t N, bool dua
   return half == HalfTiles::kNone || dual ? Tiles::kFull : Tiles::kHalfDeep;
 }
 
-inline Tiles pick_tiles(int64_t rows, int64_t Kdim, int64_t E, bool dense, int64_t N, bool dual) {
+inline Tiles pick_tiles(int64_t rows, int64_t E, bool dense, int64_t N, bool dual) {
   Tiles t;
-  // Where the layer's decode path may run every token through every expert (router.hip), gate/up keeps the
-  // 64-row LDS tiles, whose sums that launch reproduces bit for bit.
-  const bool decode_shape = dual && !dense && (E == 16 || E == 32 || E == 64) && rows >= 2 * E && Kdim % 128 == 0 && N % 64 == 0;
-  if (!decode_shape && pick_skinny(rows, E, dense, N, dual, &t)) return t;
+  if (pick_skinny(rows, E, dense, N, &t)) return t;
   if (!dense && rows <= kTinyGroupRows * E) return Tiles::kTiny;
   return pick_large(rows, E, dense, N, dual);
 }
@@ -348,16 +335,12 @@ int launch_down_fast(const void* act, const void* down, const int32_t* group_siz
 #define JT_DOWN(LAUNCH, CFG) LAUNCH<CFG>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream, row_map, row_div, a_group_rows, nullptr, nullptr
   using S11 = SkinnyCfg<1, 1, false>;
   using S12 = SkinnyCfg<1, 2, false>;
-  using S21 = SkinnyCfg<2, 1, false>;
   using S22 = SkinnyCfg<2, 2, false>;
-  using S41 = SkinnyCfg<4, 1, false>;
-  const Tiles t = pick_tiles(rows, I, E, group_sizes == nullptr, H, false);
+  const Tiles t = pick_tiles(rows, E, group_sizes == nullptr, H, false);
   switch (t) {
     case Tiles::kSkinny11: return JT_DOWN(launch_skinny, S11), a_group_rows);
     case Tiles::kSkinny12: return JT_DOWN(launch_skinny, S12), a_group_rows);
-    case Tiles::kSkinny21: return JT_DOWN(launch_skinny, S21), a_group_rows);
     case Tiles::kSkinny22: return JT_DOWN(launch_skinny, S22), a_group_rows);
-    case Tiles::kSkinny41: return JT_DOWN(launch_skinny, S41), a_group_rows);
     case Tiles::kTiny: return JT_DOWN(launch_fast, DownTinyCfg), 0, a_group_rows);
     default: break;
   }
@@ -384,12 +367,10 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
   if (Elem<T>::is_bf16 && fast_ok(x, gate, up, act, H, I) && gather_ok && saves_ok) {
     using S11 = SkinnyCfg<1, 1, true>;
     using S12 = SkinnyCfg<1, 2, true>;
-    using S21 = SkinnyCfg<2, 1, true>;
     using S22 = SkinnyCfg<2, 2, true>;
-    switch (pick_tiles(rows, H, E, dense, I, true)) {
+    switch (pick_tiles(rows, E, dense, I, true)) {
       case Tiles::kSkinny11: rc = JT_GATE_UP(launch_skinny, S11); break;
       case Tiles::kSkinny12: rc = JT_GATE_UP(launch_skinny, S12); break;
-      case Tiles::kSkinny21: rc = JT_GATE_UP(launch_skinny, S21); break;
       case Tiles::kSkinny22: rc = JT_GATE_UP(launch_skinny, S22); break;
       case Tiles::kTiny: rc = JT_GATE_UP(launch_fast, GateUpTinyCfg); break;
       case Tiles::kHalf:
@@ -450,8 +431,8 @@ int launch_down_from_all_tokens(const void* act_full, const void* down, const in
 
 bool shared_in_skinny_tiles(const void* x, const SharedExperts& s, int64_t T, int64_t H) {
   return fast_ok(x, s.gate, s.up, s.act, H, s.Is) && fast_ok(s.act, s.down, nullptr, s.y, s.Is, H) &&
-         aligned16(s.gate_pre) && aligned16(s.up_pre) && pick_tiles(T, H, 1, true, s.Is, true) == Tiles::kSkinny12 &&
-         pick_tiles(T, s.Is, 1, true, H, false) == Tiles::kSkinny12;
+         aligned16(s.gate_pre) && aligned16(s.up_pre) && pick_tiles(T, 1, true, s.Is, true) == Tiles::kSkinny12 &&
+         pick_tiles(T, 1, true, H, false) == Tiles::kSkinny12;
 }
 
 // ---- the gathering launch pair as the layer uses it (declared in common.hpp) ----

@@ -1,5 +1,5 @@
 // bf16 grouped GEMM for groups of a few rows (a decode step, the shared experts of a small batch): the
-// matrices stream straight from memory into MFMA operands, no LDS and no barrier in the k loop.
+// matrices stream straight from memory into MFMA operands, without LDS in between.
 //
 //   C[rows of e, :] = A[rows of e, :] @ B[e]                          (kDual = false)
 //   C = silu(round(A @ B0[e])) * round(A @ B1[e])                     (kDual = true)
@@ -13,13 +13,22 @@
 //   * a wave owns its loads: a lane fetches 16 bytes (8 columns) of eight consecutive k rows, the wave a block
 //     of the matrix as it is stored, and 32 byte permutes turn it into the B operands of eight
 //     v_mfma_f32_16x16x32_bf16 (operand j: column 8 (lane % 16) + j, whose eight k values the lane holds);
-//   * FOLD = 2: the upper eight of sixteen lanes hold the same columns 32 k rows further on.  An MFMA takes its
-//     A operand for all columns, so the block is multiplied once with either half's rows of A into accumulators
-//     of its own, and each half's columns are taken from the right one at the end: twice the products, which
-//     there is time for, and whole 128-byte lines with half as many columns per tile;
-//   * D blocks of 8 KB are in flight per wave in a ring of registers;
-//   * the four waves of a workgroup share out the k range (two of them per matrix when kDual), and add
-//     their sums up in wave order through LDS at the end.
+//   * FOLD = 2: the upper eight of sixteen lanes hold the same columns 32 k rows further on, so that a tile of half
+//     the columns still reads whole 128-byte lines.  Operands 0 .. 3 then take columns j of the lower lanes and
+//     j + 4 of the upper ones, for either half of the k rows, the other half's values a lane rotation away;
+//   * D = 2 blocks of 8 KB are in flight per wave in a ring of registers, up to three workgroups to a CU.  (Four
+//     blocks leave room for one workgroup per CU, and longer turns: 10 to 20 % slower throughout; the next
+//     blocks requested before the turn instead of in it, with registers for both: as fast with one workgroup to
+//     a CU, 5 to 30 % slower with more.)
+//   * the four waves of a workgroup (two of them per matrix when kDual) take turns of D blocks on the k range and
+//     hand the accumulators on through LDS, so that every sum is ONE chain in k order, as in the LDS kernels: a row's
+//     result has the same bits whichever kernel takes it, and does not depend on what shares its call.  (A
+//     16x16x32 instruction adds its 32 products as two 32x32x16 ones in a row do: no bit of 2048-deep chains
+//     differed on operands of 12, 24 and 48 bits of range.)  A wave turns its blocks into operands before its
+//     turn comes, which leaves 8 D products and 16 bytes per lane and accumulator each way in it.
+//     The turns cost 0 to 6 % against partial sums of each wave's own (shared experts of 2816 at 64 tokens 36 us
+//     against 34, 64 experts at 4 tokens 100 against 100); only tiles of 32 rows and 128 columns, with twice the
+//     accumulators to hand on, lost more (gate/up at 256 tokens 6 us) and are gone.
 // RB = blocks of 16 rows per tile.  Rows past the end of a group, columns past N and k past K read as zeros.
 //
 // Requirements: K % 8 == 0, N % 8 == 0, 16-byte aligned pointers, K*N*2 < 2^31, a_rows*K*2 < 2^31.
@@ -33,12 +42,12 @@ template <int RB_, int FOLD_, bool kDual_>
 struct SkinnyCfg {
   static constexpr int RB = RB_, FOLD = FOLD_, BM = 16 * RB, BN = 128 / FOLD, NT = 256, BK = 32 * FOLD;
   static constexpr bool kDual = kDual_;
-  static constexpr int D = RB == 1 ? 4 : 3;                    // blocks in flight per wave
-  static constexpr int KWAVES = kDual ? 2 : 4;                 // waves that share out the k range of a matrix
-  static constexpr int MIN_WAVES_PER_EU = RB * FOLD <= 2 ? 2 : 1;
+  static constexpr int D = 2;                                  // blocks per turn, and in flight per wave
+  static constexpr int KWAVES = kDual ? 2 : 4;                 // waves that take turns on the k range of a matrix
+  static constexpr int NJ = 8 / FOLD;                          // accumulators per 16 rows
+  static constexpr int MIN_WAVES_PER_EU = RB == 1 ? 2 : 1;
   static constexpr int GROUP_M = 4;
-  static constexpr int PAD = 4;                                // floats per row of the exchange, against bank conflicts
-  static constexpr int SMEM_BYTES = 4 * BM * (BN + PAD) * 4;   // one block of sums per wave
+  static constexpr int SMEM_BYTES = (kDual ? 2 : 1) * RB * NJ * 64 * 16;  // the accumulators of each matrix
   static_assert(FOLD == 1 || FOLD == 2, "columns per tile");
 };
 
@@ -98,99 +107,105 @@ __device__ __forceinline__ void grouped_gemm_skinny_tile(const SkinnyProblem& pr
   const int col = n0 + c16 % LF * 8, b_k = c16 / LF * 32 + g * 8;  // this lane's columns, and first k row of a block
   const int b_voff = col < N ? (b_k * N + col) * 2 : kOutside;
 
+  constexpr int KW = Cfg::KWAVES, NJ = Cfg::NJ;
   const int blocks = (Kdim + BK - 1) / BK;
-  const int per = (blocks + Cfg::KWAVES - 1) / Cfg::KWAVES;
-  const int first = min(blocks, kw * per), count = min(blocks - first, per);
+  const int rounds = (blocks + KW * D - 1) / (KW * D);  // turns of every wave
 
   u32x4_t b_ring[D][8], a_ring[D][FOLD][RB];
-  // Every load is issued on every path (a block past this wave's share, like a chunk past the end of K, takes
-  // an offset outside the operand: zeros, no traffic), so that the compiler's wait counts stay exact: with the
-  // loads of the last blocks behind a branch it waits for all loads in flight in front of every block.
-  auto load = [&](int slot, int i) {
-    const int k0 = (first + i) * BK;
+  // Every load is issued on every path (a block past the end, like a chunk past the end of K, takes an offset
+  // outside the operand: zeros, no traffic), so that the compiler's wait counts stay exact: with the loads of the
+  // last blocks behind a branch it waits for all loads in flight in front of every block.
+  auto load = [&](int slot, int block) {
+    const int k0 = block < blocks ? block * BK : 0;
+    const int k_end = block < blocks ? Kdim - k0 : 0;  // k rows from k0 on
 #pragma unroll
-    for (int f = 0; f < FOLD; ++f) {
-      const bool past = i >= count || k0 + f * 32 + g * 8 >= Kdim;
+    for (int f = 0; f < FOLD; ++f)
 #pragma unroll
       for (int b = 0; b < RB; ++b)
-        a_ring[slot][f][b] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, past ? kOutside : a_voff[b], (k0 + f * 32) * 2, 0);
-    }
-    const bool past = i >= count || k0 + b_k >= Kdim;
+        a_ring[slot][f][b] = __builtin_amdgcn_raw_buffer_load_b128(
+            a_rsrc, f * 32 + g * 8 >= k_end ? kOutside : a_voff[b], (k0 + f * 32) * 2, 0);
 #pragma unroll
     for (int r = 0; r < 8; ++r)  // non-temporal: few other workgroups read these bytes
-      b_ring[slot][r] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, past ? kOutside : b_voff, (k0 + r) * N * 2, 2);
+      b_ring[slot][r] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, b_k >= k_end ? kOutside : b_voff, (k0 + r) * N * 2, 2);
+  };
+  // operand jj for k half f of the block in `slot`: column 8 (c16 % LF) + jj (+ 4 in the upper lanes of a folded one)
+  auto operand = [&](int slot, int j) {
+    u32x4_t v;
+#pragma unroll
+    for (int p = 0; p < 4; ++p)  // k = 8 g + 2 p (low half) and 2 p + 1 of column j of the lane's eight
+      v[p] = __builtin_amdgcn_perm(b_ring[slot][2 * p + 1][j / 2], b_ring[slot][2 * p][j / 2],
+                                   j % 2 ? 0x07060302u : 0x05040100u);
+    return v;
+  };
+  u32x4_t frag[D][FOLD][NJ];
+  auto prepare = [&](int slot) {
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj) {
+      const u32x4_t lo = operand(slot, jj);
+      if constexpr (FOLD == 1) {
+        frag[slot][0][jj] = lo;
+      } else {
+        const u32x4_t hi = operand(slot, jj + 4);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {  // rotations by 8 of 16 lanes, into the upper eight and into the lower eight
+          frag[slot][0][jj][p] = __builtin_amdgcn_update_dpp(lo[p], hi[p], 0x128, 0xf, 0xc, false);
+          frag[slot][FOLD - 1][jj][p] = __builtin_amdgcn_update_dpp(hi[p], lo[p], 0x128, 0xf, 0x3, false);
+        }
+      }
+    }
   };
   typedef __attribute__((ext_vector_type(4))) float f32x4;
-  f32x4 acc[FOLD][RB][8];
+  f32x4* const sums = reinterpret_cast<f32x4*>(smem_raw);  // [matrix][16-row block][operand][lane]
+  f32x4* const mine = sums + which * (RB * NJ * 64) + lane;
+  auto turn_ends = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  if (kw == 0)
 #pragma unroll
-  for (int f = 0; f < FOLD; ++f)
-#pragma unroll
-    for (int b = 0; b < RB; ++b)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) acc[f][b][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < RB * NJ; ++i) mine[i * 64] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    load(d, d);
+    load(d, kw * D + d);
     __builtin_amdgcn_sched_barrier(0);
   }
-  for (int i0 = 0; i0 < count; i0 += D) {
+  for (int round = 0; round < rounds; ++round) {
 #pragma unroll
-    for (int d = 0; d < D; ++d) {  // (blocks past the wave's share multiply zeros)
+    for (int d = 0; d < D; ++d) {
+      prepare(d);
+      __builtin_amdgcn_sched_barrier(0);  // (one block's operands at a time: mixed, they do not fit the registers)
+    }
+    for (int w = 0; w < kw; ++w) turn_ends();  // the waves before this one
+    f32x4 acc[RB][NJ];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        u32x4_t frag;
+    for (int i = 0; i < RB * NJ; ++i) acc[i / NJ][i % NJ] = mine[i * 64];
 #pragma unroll
-        for (int p = 0; p < 4; ++p)  // k = 8 g + 2 p (low half) and 2 p + 1 of column 8 c16 + j
-          frag[p] = __builtin_amdgcn_perm(b_ring[d][2 * p + 1][j / 2], b_ring[d][2 * p][j / 2],
-                                          j % 2 ? 0x07060302u : 0x05040100u);
+    for (int d = 0; d < D; ++d) {  // (blocks past the end multiply zeros)
 #pragma unroll
-        for (int f = 0; f < FOLD; ++f)
+      for (int f = 0; f < FOLD; ++f)
 #pragma unroll
-          for (int b = 0; b < RB; ++b)
-            acc[f][b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a_ring[d][f][b]),
-                                                                   __builtin_bit_cast(bf16x8_t, frag), acc[f][b][j], 0, 0, 0);
-      }
-      load(d, i0 + d + D);
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+          for (int jj = 0; jj < NJ; ++jj)
+            acc[b][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a_ring[d][f][b]),
+                                                                 __builtin_bit_cast(bf16x8_t, frag[d][f][jj]), acc[b][jj], 0, 0, 0);
+      load(d, ((round + 1) * KW + kw) * D + d);
       __builtin_amdgcn_sched_barrier(0);  // (else the loads of all D blocks gather at the end of the loop body)
     }
+#pragma unroll
+    for (int i = 0; i < RB * NJ; ++i) mine[i * 64] = acc[i / NJ][i % NJ];
+    for (int w = kw; w < KW; ++w) turn_ends();  // this wave, and those behind it
   }
 
-  // value i of lane (c16, g) in acc[f][b][j] is row 16 b + 4 g + i, column 8 (c16 % LF) + j, and belongs to the
-  // product if f is the half of the block that the lane holds; the other half's lanes add theirs up here
-  float* const mine = reinterpret_cast<float*>(smem_raw) + wave * (BM * (BN + Cfg::PAD));
-#pragma unroll
-  for (int b = 0; b < RB; ++b)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        v[j] = acc[0][b][j][i];
-        if (FOLD == 2) v[j] += __shfl_xor(acc[FOLD - 1][b][j][i], 8);
-      }
-      float* p = mine + (16 * b + 4 * g + i) * (BN + Cfg::PAD) + c16 % LF * 8;
-      if (c16 < LF) {
-        *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
-      }
-    }
-  __syncthreads();
-  const float* const sums = reinterpret_cast<const float*>(smem_raw);
-  constexpr int kPlane = BM * (BN + Cfg::PAD);
+  // value i of lane (c16, g) of accumulator (b, jj) is row 16 b + 4 g + i, column 8 (c16 % LF) + jj (+ 4 in the
+  // upper lanes of a folded tile)
+  const float* const values = reinterpret_cast<const float*>(smem_raw);
   for (int c = tid; c < BM * (BN / 8); c += Cfg::NT) {  // one 16-byte piece of a result row per thread
-    const int r = c / (BN / 8), c8 = (c - r * (BN / 8)) * 8;
+    const int r = c / (BN / 8), q = c - r * (BN / 8), c8 = q * 8;
     if (r >= tr.rows || n0 + c8 >= N) continue;
-    const float* p = sums + r * (BN + Cfg::PAD) + c8;
+    const float* p = values + ((r / 16) * NJ * 64 + r % 16 / 4 * 16 + q) * 4 + r % 4;
     float v[2][8];  // the two products, or the only one
 #pragma unroll
     for (int m = 0; m < (kDual ? 2 : 1); ++m)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float t = p[m * kPlane + j];
-#pragma unroll
-        for (int w = 1; w < Cfg::KWAVES; ++w) t += p[(w * (kDual ? 2 : 1) + m) * kPlane + j];
-        v[m][j] = t;
-      }
+      for (int j = 0; j < 8; ++j) v[m][j] = p[(m * RB * NJ * 64 + j % NJ * 64 + j / NJ * LF) * 4];
     const size_t at = (size_t)(tr.row0 + r) * N + n0 + c8;
     auto store8 = [&](uint16_t* out, const float* f) {
       const u32x4_t q = {pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7])};

@@ -1,0 +1,79 @@
+"""A row of the expert products has the same bits whichever kernel takes it.
+
+The reference's invariant is prefill + decode == full forward (tests/jaxtitan/test_infer.py:270-301).  Which kernel
+takes a product depends on the size of the call, so all of them add up a result in one order: 16 k values per
+instruction, chained in k order, one rounding at the end.  The sizes below stand on either side of the rules that
+choose: streaming tiles of 16 and 32 rows, 64-row LDS tiles, half tiles, 256-row tiles, the decode launch, shared
+experts beside the router.  Equal means equal: no tolerance.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from research_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+WIDTHS = [(1024, 704), (512, 2816), (2048, 192)]
+
+
+def drawer(gpu, seed):
+    generator = torch.Generator(device=gpu).manual_seed(seed)
+
+    def normal(*shape, std=1.0):
+        return (torch.randn(shape, generator=generator, device=gpu) * std).to(torch.bfloat16)
+
+    return normal
+
+
+@pytest.mark.parametrize("hidden,inter", WIDTHS)
+def test_shared_rows_do_not_depend_on_the_call(gpu, hidden, inter):
+    normal = drawer(gpu, hidden)
+    x = normal(2600, hidden)
+    matrices = normal(hidden, inter, std=0.05), normal(hidden, inter, std=0.05), normal(inter, hidden, std=0.05)
+    whole = ops.shared_swiglu(x, *matrices)
+    for rows in (1, 3, 16, 17, 64, 65, 130, 260, 520, 1030):
+        part = ops.shared_swiglu(x[:rows].contiguous(), *matrices)
+        assert torch.equal(part, whole[:rows]), f"{rows} rows: {int((part != whole[:rows]).sum())} values differ"
+
+
+@pytest.mark.parametrize("hidden,inter", WIDTHS)
+@pytest.mark.parametrize("experts", [5, 64])
+def test_routed_rows_do_not_depend_on_the_call(gpu, hidden, inter, experts):
+    """Rows of every group: the first few of each alone against all of them."""
+    normal = drawer(gpu, hidden + experts)
+    per_group = 6000 // experts
+    x = normal(experts * per_group, hidden)
+    matrices = (normal(experts, hidden, inter, std=0.05), normal(experts, hidden, inter, std=0.05),
+                normal(experts, inter, hidden, std=0.05))
+
+    def run(rows):
+        sizes = torch.full((experts,), rows, dtype=torch.int32, device=gpu)
+        offsets = (torch.cumsum(sizes, 0) - sizes).to(torch.int32)
+        part = x.view(experts, per_group, hidden)[:, :rows].reshape(-1, hidden).contiguous()
+        return ops.grouped_swiglu(part, *matrices, sizes, offsets).view(experts, rows, hidden)
+
+    whole = run(per_group)
+    for rows in (1, 2, 3, 9, 20, 40, 70):
+        part = run(rows)
+        assert torch.equal(part, whole[:, :rows]), f"{rows} rows: {int((part != whole[:, :rows]).sum())} values differ"
+
+
+@pytest.mark.parametrize("hidden,inter,experts,top_k,shared", [
+    (512, 704, 64, 8, 1408),  # streaming tiles and shared experts beside the router at the small sizes
+    (1024, 192, 16, 2, 0),    # the decode launch from 16 tokens on
+    (2048, 64, 128, 2, 128),  # the sliced router in between
+])
+def test_layer_rows_do_not_depend_on_the_call(gpu, hidden, inter, experts, top_k, shared):
+    normal = drawer(gpu, experts)
+    x, bias = normal(2700, hidden), torch.zeros(experts, device=gpu)
+    weights = (normal(hidden, experts, std=0.05), bias, normal(experts, hidden, inter, std=0.05),
+               normal(experts, hidden, inter, std=0.05), normal(experts, inter, hidden, std=0.05))
+    extra = (normal(hidden, shared, std=0.05), normal(hidden, shared, std=0.05), normal(shared, hidden, std=0.05)) if shared else None
+    whole = ops.moe_forward(x, *weights, top_k, 1.0, shared=extra)
+    for rows in (1, 2, 7, 16, 33, 64, 65, 200, 257, 700, 1300):
+        part = ops.moe_forward(x[:rows].contiguous(), *weights, top_k, 1.0, shared=extra)
+        assert torch.equal(part.expert_ids, whole.expert_ids[:rows])
+        assert torch.equal(part.y, whole.y[:rows]), f"{rows} rows: {int((part.y != whole.y[:rows]).sum())} values differ"
