@@ -372,18 +372,20 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
       case Tiles::kSkinny11: rc = JT_GATE_UP(launch_skinny, S11); break;
       case Tiles::kSkinny12: rc = JT_GATE_UP(launch_skinny, S12); break;
       case Tiles::kSkinny22: rc = JT_GATE_UP(launch_skinny, S22); break;
-      case Tiles::kTiny: rc = JT_GATE_UP(launch_fast, GateUpTinyCfg); break;
+      case Tiles::kTiny:
+        rc = H % 64 == 0 ? JT_GATE_UP(launch_fast, GateUpTinyCfg) : JT_GATE_UP(launch_fast, GateUpTinyTailCfg);
+        break;
       case Tiles::kHalf:
-        if (stream_ok<GateUpHalfCfg>(rows, H, I, row_map, row_div)) {
-          rc = JT_GATE_UP(launch_stream, GateUpHalfCfg);
+        if (stream_ok<GateUpHalfTailCfg>(rows, H, I, row_map, row_div)) {
+          rc = H % 64 == 0 ? JT_GATE_UP(launch_stream, GateUpHalfCfg) : JT_GATE_UP(launch_stream, GateUpHalfTailCfg);
           break;
         }
         [[fallthrough]];
       default:
-        rc = stream_ok<GateUpStreamCfg>(rows, H, I, row_map, row_div)       ? JT_GATE_UP(launch_stream, GateUpStreamCfg)
-             : stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div) ? JT_GATE_UP(launch_stream, GateUpStreamTailCfg)
-             : H % 64 == 0                                                  ? JT_GATE_UP(launch_fast, GateUpCfg)
-                                                                            : JT_GATE_UP(launch_fast, GateUpTailCfg);
+        if (stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div))
+          rc = H % 64 == 0 ? JT_GATE_UP(launch_stream, GateUpStreamCfg) : JT_GATE_UP(launch_stream, GateUpStreamTailCfg);
+        else
+          rc = H % 64 == 0 ? JT_GATE_UP(launch_fast, GateUpCfg) : JT_GATE_UP(launch_fast, GateUpTailCfg);
     }
   }
 #undef JT_GATE_UP

@@ -27,7 +27,7 @@
 //
 // K need not be a multiple of the step: the chunks of A past the end of a row are not fetched but read as
 // zeros (they would be the next row's first elements), and B has no rows there (its descriptor ends with
-// the matrix).  The 64-row kernel checks once per step; the persistent and the stream kernel have variants of
+// the matrix).  The 64-row kernel always checks, once per step; the persistent and the stream kernel have variants of
 // their own (OPT & 65536), because the check costs registers that the others do not have to spare.  Before,
 // such widths ran element by element in the generic kernel: 2931 x 3 rows, 1000 x 2664, 24 experts with a
 // shared expert took 1122 + 967 us (routed) and 415 + 464 us (shared), now 122 + 81 and 36 + 64 us.
@@ -91,6 +91,13 @@ __device__ __forceinline__ float bf16_round_fast(float f) { return (float)(__bf1
 __device__ __forceinline__ float silu_rcp(float g) {
   return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
 }
+// Gate/up products whose reduction is no multiple of 64 divide, like the general kernel, which alone took them once:
+// the reciprocal's last bit puts 1.2 times as many of their results on the other side of a bf16 rounding.  One rule
+// for every kernel, so that a row's bits do not depend on which of them takes it.
+template <bool kDivide>
+__device__ __forceinline__ float silu_gate(float g) {
+  return kDivide ? silu_fast(g) : silu_rcp(g);
+}
 
 // a byte offset outside every operand (all are smaller than 2 GiB): such a load stores zeros
 constexpr int kOutside = (int)0x80000000u;
@@ -117,7 +124,7 @@ struct DmaGemmCfg {
   // 32 = raise the wave priority around the MFMA burst, 64 = ask the scheduler to interleave
   // one MFMA with up to three LDS reads, 128 = B tiles in 4 x 64 blocks, 2048 = (persistent kernel) results written
   // straight from transposed accumulators instead of through LDS, 4096 = non-temporal loads of B, 8192 / 16384 = 8 / 2 m-tiles per group of the tile order instead of 4, 32768 = non-temporal stores of the result,
-  // 65536 = (persistent and stream kernels) K may end inside a step
+  // 65536 = (persistent and stream kernels) K may end inside a step; dual ones are for K % 64 != 0 only (silu_gate)
   static constexpr int OPT = OPT_;
   static constexpr bool kDual = kDual_;
   static constexpr int BNE = kDual ? 2 * BN : BN;  // columns of the B tile in LDS
@@ -178,7 +185,7 @@ __device__ __forceinline__ void store_transposed_accumulators(const f32x16_t (&a
                                                               uint16_t* __restrict__ C, uint16_t* __restrict__ save0,
                                                               uint16_t* __restrict__ save1) {
   constexpr int TM = Cfg::TM, TN = Cfg::TN, WM = Cfg::WM, TNO = Cfg::TNO, WNO = Cfg::WNO;
-  constexpr bool kDual = Cfg::kDual;
+  constexpr bool kDual = Cfg::kDual, kTail = (Cfg::OPT & 65536) != 0;
   // (the lane id is taken afresh so that nothing of the epilogue's addressing is kept in registers
   // through the k loops, where every register is spoken for)
   int lane_e;
@@ -211,7 +218,7 @@ __device__ __forceinline__ void store_transposed_accumulators(const f32x16_t (&a
                 if (pass == 0) {
                   const float g0 = __uint_as_float(gb << 16), g1 = __uint_as_float(gb & 0xffff0000u);
                   const float u0 = __uint_as_float(ub << 16), u1 = __uint_as_float(ub & 0xffff0000u);
-                  pk[dq][tp] = pack_bf16x2(silu_rcp(g0) * u0, silu_rcp(g1) * u1);
+                  pk[dq][tp] = pack_bf16x2(silu_gate<kTail>(g0) * u0, silu_gate<kTail>(g1) * u1);
                 } else {
                   pk[dq][tp] = pass == 1 ? gb : ub;
                 }
@@ -480,6 +487,7 @@ __device__ __forceinline__ void grouped_gemm_dma_tile(
   uint16_t* const cw = reinterpret_cast<uint16_t*>(smem_raw) + wave * (WM * CS);
   const int col0 = n0 + wn * WNO;
   const int row_base = wm * WM;
+  constexpr bool kTail = (Cfg::OPT & 65536) != 0;
   const int passes = (kDual && save0 != nullptr) ? 3 : 1;
   for (int pass = 0; pass < passes; ++pass) {
 #pragma unroll
@@ -493,7 +501,7 @@ __device__ __forceinline__ void grouped_gemm_dma_tile(
           if (kDual) {
             const float g = bf16_round_fast(acc[mi][jj][i]);
             const float u = bf16_round_fast(acc[mi][jj + TN / 2][i]);
-            v = pass == 0 ? silu_rcp(g) * u : (pass == 1 ? g : u);
+            v = pass == 0 ? silu_gate<kTail>(g) * u : (pass == 1 ? g : u);
           } else {
             v = acc[mi][jj][i];
           }
@@ -795,7 +803,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_dma_persistent_kernel(
               if (kDual) {
                 const float g = bf16_round_fast(acc[mi][jj][i]);
                 const float u = bf16_round_fast(acc[mi][jj + TN / 2][i]);
-                v = pass == 0 ? silu_rcp(g) * u : (pass == 1 ? g : u);
+                v = pass == 0 ? silu_gate<kTail>(g) * u : (pass == 1 ? g : u);
               } else {
                 v = acc[mi][jj][i];
               }
@@ -853,6 +861,7 @@ using DownTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 64 + 128 + 327
 // non-temporal loads stream it past the L2 (64 tokens, 64 experts: gate/up 0.126 -> 0.110 ms = 6.7 TB/s, down
 // 0.061 -> 0.054 ms = 6.8 TB/s; at 387 tokens 137 -> 121 and 68 -> 61 us).
 using GateUpTinyCfg = DmaGemmCfg<64, 128, 32, 1, 4, true, 2, 16 + 128 + 4096>;
+using GateUpTinyTailCfg = DmaGemmCfg<64, 128, 32, 1, 4, true, 2, 16 + 128 + 4096 + 65536>;  // for K % 64 != 0
 using DownTinyCfg = DmaGemmCfg<64, 256, 32, 1, 4, false, 2, 16 + 4096>;
 
 }  // namespace jtmoe

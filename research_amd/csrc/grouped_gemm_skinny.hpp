@@ -214,7 +214,10 @@ __device__ __forceinline__ void grouped_gemm_skinny_tile(const SkinnyProblem& pr
     if (kDual) {
       float h[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) h[j] = silu_rcp(bf16_round_fast(v[0][j])) * bf16_round_fast(v[1][j]);
+      for (int j = 0; j < 8; ++j) {
+        const float gate = bf16_round_fast(v[0][j]);
+        h[j] = (Kdim % 64 != 0 ? silu_gate<true>(gate) : silu_gate<false>(gate)) * bf16_round_fast(v[1][j]);
+      }
       store8(pr.C, h);
       if (pr.save0) {
         store8(pr.save0, v[0]);

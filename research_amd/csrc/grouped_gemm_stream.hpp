@@ -445,12 +445,13 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_nt_kernel(
 // (alternating in one process): 1.306 ms against 1.400-1.409 ms for grouped_gemm_dma_persistent_kernel
 // and 1.315-1.320 ms for 64-deep steps with two stages.
 using GateUpStreamCfg = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128>;
-using GateUpStreamTailCfg = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 65536>;  // for K % 32 != 0
+using GateUpStreamTailCfg = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 65536>;  // for K % 64 != 0
 // Half-size tiles in four-wave workgroups for launches that would leave CUs without a 256-row tile: gate/up with
 // one workgroup per CU (99 KB of LDS), down with two.  The dispatch rules and what they measured stand in
-// grouped_gemm.hip.  (With the check for a ragged last step, so that one variant serves every width: 33.3 against
-// 33.7 us without it for gate/up, 39.8 against 40.4 for down, that is nothing.)
-using GateUpHalfCfg = DmaGemmCfg<128, 128, 32, 2, 2, true, 4, 16 + 128 + 65536>;
+// grouped_gemm.hip.  (The check for a ragged last step costs nothing: 33.3 against 33.7 us without it for gate/up,
+// 39.8 against 40.4 for down, so that one variant of the latter serves every width.)
+using GateUpHalfCfg = DmaGemmCfg<128, 128, 32, 2, 2, true, 4, 16 + 128>;
+using GateUpHalfTailCfg = DmaGemmCfg<128, 128, 32, 2, 2, true, 4, 16 + 128 + 65536>;  // for K % 64 != 0
 using DownHalfCfg = DmaGemmCfg<128, 128, 32, 2, 2, false, 4, 16 + 128 + 65536>;
 using DownHalfDeepCfg = DmaGemmCfg<128, 128, 64, 2, 2, false, 2, 16 + 128 + 65536>;
 // Variants kept for the stand-alone check and its timings (time_stream, time_down): 64-deep steps with

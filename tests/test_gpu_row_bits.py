@@ -12,11 +12,11 @@ from __future__ import annotations
 import pytest
 import torch
 
-from research_amd import ops
+from research_amd import grad, ops
 
 pytestmark = pytest.mark.gpu
 
-WIDTHS = [(1024, 704), (512, 2816), (2048, 192)]
+WIDTHS = [(1024, 704), (512, 2816), (2048, 192), (1000, 264), (264, 1352), (72, 2056)]
 
 
 def drawer(gpu, seed):
@@ -77,3 +77,33 @@ def test_layer_rows_do_not_depend_on_the_call(gpu, hidden, inter, experts, top_k
         part = ops.moe_forward(x[:rows].contiguous(), *weights, top_k, 1.0, shared=extra)
         assert torch.equal(part.expert_ids, whole.expert_ids[:rows])
         assert torch.equal(part.y, whole.y[:rows]), f"{rows} rows: {int((part.y != whole.y[:rows]).sum())} values differ"
+
+
+def off_by_one_element(t):
+    """The same values at an address that is no multiple of 16: only the general kernel takes such an operand."""
+    room = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    moved = room[1:].view(t.shape)
+    moved.copy_(t)
+    return moved
+
+
+@pytest.mark.parametrize("tokens,experts,top_k,hidden,inter", [
+    (2, 3, 1, 200, 72), (40, 2, 1, 264, 1352), (30, 64, 8, 1000, 264), (350, 40, 4, 264, 1352), (900, 2, 2, 1000, 328),
+    (2931, 24, 3, 264, 1352), (2600, 8, 2, 104, 520), (700, 3, 1, 72, 136),
+])
+def test_ragged_widths_have_the_bits_of_the_general_kernel(gpu, tokens, experts, top_k, hidden, inter):
+    """Routed and shared products, and the two products that a training forward keeps."""
+    normal = drawer(gpu, tokens)
+    x = normal(tokens, hidden)
+    matrices = (normal(experts, hidden, inter, std=0.05), normal(experts, hidden, inter, std=0.05),
+                normal(experts, inter, hidden, std=0.05))
+    ids = torch.rand(tokens, experts, device=gpu).topk(top_k, dim=1).indices.to(torch.int32)
+    plan = ops.dispatch(ids, experts, x)
+    general = [off_by_one_element(m) for m in matrices]
+    groups = plan.group_sizes, plan.offsets
+    assert torch.equal(ops.grouped_swiglu(plan.packed_x, *matrices, *groups), ops.grouped_swiglu(plan.packed_x, *general, *groups))
+    one = [m[0].contiguous() for m in matrices]
+    want, kept_by_general = grad.shared_swiglu_train(x, *(off_by_one_element(m) for m in one))
+    got, kept = grad.shared_swiglu_train(x, *one)
+    assert torch.equal(got, want)
+    assert torch.equal(kept.gate_pre, kept_by_general.gate_pre) and torch.equal(kept.up_pre, kept_by_general.up_pre)
