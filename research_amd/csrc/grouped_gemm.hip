@@ -275,11 +275,16 @@ enum class Tiles { kSkinny11, kSkinny12, kSkinny22, kTiny, kHalf, kHalfDeep, kFu
 // down together, 2048 -> 1408, 64 experts top-8, 1 token: 35 against 87 in 64-row LDS tiles; shared experts of 2816:
 // 34 at 1 token, 36 at 64 (148 in 64-row LDS tiles), 43 at 130 with 32-row tiles (58 without them).  Tiles of 128
 // columns and 32 or 64 rows do not pay where half tiles can be had: 68 against 53 at 387 tokens, 91 against 63 at 700.
-// With more tiles than CUs they pay while few groups need a second product's worth of rows, up to a mean of two
-// per group reached: 64 experts 100 against 127 at 4 tokens, 130 against 138 at 8 (mean 1.6), but 177 against
-// 166 at 15 (2.2) and 187 against 174 at 28 (3.6); 128 experts of 768: 163 against 166 at 20 (1.75), equal within
-// 1 % from 30 on.
-inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, Tiles* out) {
+// With more tiles than CUs, and up to four rows per group reached (a group's second tile reads its matrix again),
+// they compete with the 64-row LDS tiles over the number that is resident at once.  Gate/up: the LDS tiles are as
+// wide, three to a CU; streaming pays up to two tiles per CU: 74 against 76 us at 12 tokens top-8 of 128 experts,
+// 2048 -> 768 (426 tiles expected), 77 against 84 at 8 tokens of 64 experts, 2048 -> 1408 (448), but 104 against 98 at
+// 20 tokens (546) and 104 against 102 at 15 (605).  Down: the LDS tiles are 256 wide, two to a CU, and a second
+// round of them costs as much as the first (33 us for 480 tiles, 55 for 528); streaming pays while all of its
+// tiles are resident, three to a CU (8 tokens, 64 experts 48 against 56), and where the LDS tiles start that round (12
+// and 20 tokens, 128 experts 41 and 52 against 56 and 58; 37 with two thirds of the experts reached 39 against 55;
+// balanced 63 against 62), but not in between (15 tokens, 64 experts 63 against 54).
+inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dual, Tiles* out) {
   struct Shape {
     Tiles id;
     int RB, BN;
@@ -294,9 +299,11 @@ inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, Tiles* o
       *out = s.id;
     }
   }
-  if (most == 0.0 && !dense && (double)rows <= 2.0 * expected_mtiles(rows, E, false, 16)) {
+  if (most == 0.0 && !dense && (double)rows <= 4.0 * expected_mtiles(rows, E, false, 16)) {
+    const double tiles = expected_mtiles(rows, E, false, 16) * (double)((N + 127) / 128);
+    const double lds_tiles = expected_mtiles(rows, E, false, 64) * (double)((N + 255) / 256);
     *out = Tiles::kSkinny11;
-    return true;
+    return dual ? tiles <= 2.0 * cus : tiles <= 3.0 * cus || lds_tiles > 2.0 * cus;
   }
   return most > 0.0;
 }
@@ -317,7 +324,7 @@ inline Tiles pick_large(int64_t rows, int64_t E, bool dense, int64_t N, bool dua
 
 inline Tiles pick_tiles(int64_t rows, int64_t E, bool dense, int64_t N, bool dual) {
   Tiles t;
-  if (pick_skinny(rows, E, dense, N, &t)) return t;
+  if (pick_skinny(rows, E, dense, N, dual, &t)) return t;
   if (!dense && rows <= kTinyGroupRows * E) return Tiles::kTiny;
   return pick_large(rows, E, dense, N, dual);
 }
