@@ -41,7 +41,8 @@ namespace {
 // wave).  Forward: partial sums per chunk, then one workgroup adds them in chunk order.  Backward: each
 // workgroup counts its whole sequence's ids itself (they are a fraction of the scores and come from the
 // L2), which needs neither scratch nor a second launch.  Every sum has a fixed order.
-// Measured there: forward 406 + 5 -> 14 + 8 us, backward 274 -> 15 us.
+// Measured there: forward 406 + 5 -> 14 + 8 us, backward 274 -> 15 us.  Many short sequences (16384 of 8 tokens, 256
+// experts): forward 785 -> 37 us, of which one launch adds up the sequences' shares; backward 49 -> 48.
 constexpr int kBalThreads = 256;
 constexpr int kBalWaves = kBalThreads / kWave;
 constexpr int kBalFinalThreads = 1024;
@@ -51,8 +52,13 @@ inline int bal_clamp(int64_t v, int64_t lo, int64_t hi) { return (int)(v < lo ? 
 // chunks per sequence of the forward pass: one workgroup per CU, and at most 64 partial sums for the
 // finishing workgroup to add up
 inline int bal_max_chunks(int64_t B) { return bal_clamp((256 + B - 1) / B, 1, 64); }
-inline int bal_chunks(int64_t B, int64_t S) {
-  return bal_clamp((S + kBalMinTokens - 1) / kBalMinTokens, 1, bal_max_chunks(B));
+// A step of a workgroup's tokens takes 0.45 us, 1024 partial sums 0.4 us of the
+// finishing one: where the latter is more a sequence stays whole and its workgroup writes one number (us at 64 and
+// 200 sequences of 64 tokens, 256 experts: 16 and 16 whole, 28 and 49 in chunks; 32 of 512: 67 and 33).
+inline int bal_chunks(int64_t B, int64_t S, int64_t E) {
+  const int chunks = bal_clamp((S + kBalMinTokens - 1) / kBalMinTokens, 1, bal_max_chunks(B));
+  const int64_t tokens_per_step = kBalWaves * (E <= 8 ? 8 : E <= 16 ? 4 : E <= 32 ? 2 : 1);
+  return S * 1024 <= B * E * chunks * tokens_per_step ? 1 : chunks;
 }
 // ... of the backward pass: two workgroups per CU (no finishing step), but no more than 8 E / K, beyond
 // which counting the sequence's S K ids in every chunk would move more bytes than half of the chunk's own
@@ -71,8 +77,9 @@ __device__ __forceinline__ float bal_row_sum(float v) {
 }
 
 // psum[chunk][b][e] = sum over the chunk's tokens of scores / max(row sum, 1e-20), pcnt = the ids' histogram.
-// W lanes per token, PL experts per lane (W * PL >= E).
-template <int W, int PL>
+// W lanes per token, PL experts per lane (W * PL >= E).  kWhole: the chunk is the whole sequence, and psum[b] is its
+// share of the loss, sum over e of f[b,e] P[b,e]; nothing else is written.
+template <int W, int PL, bool kWhole>
 __global__ __launch_bounds__(kBalThreads) void balance_partial_kernel(const int32_t* __restrict__ ids,
                                                                       const float* __restrict__ scores, int B, int S,
                                                                       int E, int K, int chunk_tokens,
@@ -115,11 +122,43 @@ __global__ __launch_bounds__(kBalThreads) void balance_partial_kernel(const int3
     if (e < E) part[row * E + e] = acc[j];
   }
   __syncthreads();
+  const float fscale = (float)E / ((float)K * (float)S);
+  float local = 0.0f;
   for (int e = tid; e < E; e += kBalThreads) {
     float t = 0.0f;
     for (int r = 0; r < kRows; ++r) t += part[r * E + e];
-    psum[((size_t)chunk * B + b) * E + e] = t;
-    pcnt[((size_t)chunk * B + b) * E + e] = cnt[e];
+    if constexpr (kWhole) {
+      local += fscale * (float)cnt[e] * (t / (float)S);
+    } else {
+      psum[((size_t)chunk * B + b) * E + e] = t;
+      pcnt[((size_t)chunk * B + b) * E + e] = cnt[e];
+    }
+  }
+  if constexpr (kWhole) {
+    __shared__ float red[kBalWaves];
+    local = bal_row_sum<kWave>(local);
+    if ((tid & (kWave - 1)) == 0) red[tid / kWave] = local;
+    __syncthreads();
+    if (tid == 0) psum[b] = (red[0] + red[1]) + (red[2] + red[3]);
+  }
+}
+
+// loss = mean of the sequences' shares.  A thread keeps eight loads in flight and adds them in order.
+__global__ __launch_bounds__(kBalFinalThreads) void balance_mean_kernel(const float* __restrict__ share, int B,
+                                                                        float* __restrict__ loss) {
+  __shared__ float red[kBalFinalThreads / kWave];
+  const int tid = threadIdx.x;
+  float local = 0.0f;
+#pragma unroll 8
+  for (int b = tid; b < B; b += kBalFinalThreads) local += share[b];
+  local = bal_row_sum<kWave>(local);
+  if ((tid & (kWave - 1)) == 0) red[tid / kWave] = local;
+  __syncthreads();
+  if (tid == 0) {
+    float t = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kBalFinalThreads / kWave; ++w) t += red[w];
+    loss[0] = t / (float)B;
   }
 }
 
@@ -191,16 +230,19 @@ __global__ __launch_bounds__(kBalThreads) void balance_backward_kernel(const int
                                                                        float* __restrict__ d_scores) {
   extern __shared__ float smem[];
   constexpr int kRows = kBalWaves * (kWave / W);
-  int* cnt = reinterpret_cast<int*>(smem);  // [kBalWaves][E]: a histogram per wave, fewer lanes per counter
+  // [sets][E]: a histogram per wave, fewer lanes per counter; a single one where it takes longer to clear and to add
+  // up than to fill (16384 sequences of 8 tokens, 256 experts: 52 -> 47 us)
+  int* cnt = reinterpret_cast<int*>(smem);
   const int b = blockIdx.y, tid = threadIdx.x, wave = tid / kWave;
   const int row = tid / W, e0 = tid % W;
   const int s_lo = blockIdx.x * chunk_tokens, s_hi = min(S, s_lo + chunk_tokens);
-  for (int e = tid; e < kBalWaves * E; e += kBalThreads) cnt[e] = 0;
+  const int n = S * K, sets = n >= 4 * E ? kBalWaves : 1;
+  for (int e = tid; e < sets * E; e += kBalThreads) cnt[e] = 0;
   __syncthreads();
   const int32_t* ids_b = ids + (size_t)b * S * K;
-  const int n = S * K;
+  int* const mine = cnt + (sets > 1 ? wave * E : 0);
   auto count = [&](int id) {
-    if (id >= 0 && id < E) atomicAdd(&cnt[wave * E + id], 1);
+    if (id >= 0 && id < E) atomicAdd(&mine[id], 1);
   };
   int done = 0;
   if (aligned16(ids_b)) {  // four ids per load: the loop is a chain of load latencies
@@ -224,9 +266,12 @@ __global__ __launch_bounds__(kBalThreads) void balance_backward_kernel(const int
   for (int j = 0; j < PL; ++j) {
     const int e = e0 + j * W;
     int c = 0;
-    if (e < E)
+    if (e < E) {
+      c = cnt[e];
+      if (sets > 1)
 #pragma unroll
-      for (int w = 0; w < kBalWaves; ++w) c += cnt[w * E + e];
+        for (int w = 1; w < kBalWaves; ++w) c += cnt[w * E + e];
+    }
     f[j] = fscale * (float)c;
   }
 #pragma unroll 4
@@ -475,6 +520,7 @@ extern "C" const char* jtmoe_last_error(void) { return g_error; }
 
 extern "C" size_t jtmoe_balance_workspace_bytes(int64_t B, int64_t E) {
   if (B <= 0) return 0;
+  if (bal_max_chunks(B) == 1) return align_up((size_t)B * sizeof(float), 256);
   return align_up((size_t)bal_max_chunks(B) * B * (E > 0 ? E : 1) * (sizeof(float) + sizeof(int)), 256);
 }
 
@@ -492,19 +538,28 @@ extern "C" int jtmoe_sequence_balance_loss(const int32_t* expert_ids, const floa
     return fail(JTMOE_EWORKSPACE, "sequence_balance_loss: workspace %zu < %zu bytes", workspace_bytes,
                 jtmoe_balance_workspace_bytes(B, E));
   hipStream_t s = as_stream(stream);
-  const int chunks = bal_chunks(B, S);
+  const int chunks = bal_chunks(B, S, E);
   const int chunk_tokens = (int)((S + chunks - 1) / chunks);
   float* psum = static_cast<float*>(workspace);
-  int* pcnt = reinterpret_cast<int*>(psum + (size_t)chunks * B * E);
-#define JT_LAUNCH(W, PL)                                                                                     \
-  for (int64_t b0 = 0; b0 < B; b0 += 65535)                                                                  \
-  balance_partial_kernel<W, PL><<<dim3(chunks, (unsigned)(B - b0 < 65535 ? B - b0 : 65535)), kBalThreads,    \
-                                  (size_t)(kBalThreads / W + 1) * E * sizeof(float), s>>>(                   \
-      expert_ids + b0 * S * K, scores + b0 * S * E, (int)B, (int)S, (int)E, (int)K, chunk_tokens,            \
-      psum + b0 * E, pcnt + b0 * E)
-  JT_BALANCE_WIDTHS(JT_LAUNCH);
-#undef JT_LAUNCH
-  balance_final_kernel<<<1, kBalFinalThreads, 0, s>>>(psum, pcnt, chunks, (int)B, (int)S, (int)E, (int)K, loss);
+  int* pcnt = reinterpret_cast<int*>(psum + (size_t)chunks * B * E);  // (without a use where a chunk is a sequence)
+#define JT_LAUNCH_CHUNKS(W, PL, WHOLE)                                                                              \
+  for (int64_t b0 = 0; b0 < B; b0 += 65535)                                                                         \
+  balance_partial_kernel<W, PL, WHOLE><<<dim3(chunks, (unsigned)(B - b0 < 65535 ? B - b0 : 65535)), kBalThreads,    \
+                                         (size_t)(kBalThreads / W + 1) * E * sizeof(float), s>>>(                   \
+      expert_ids + b0 * S * K, scores + b0 * S * E, (int)B, (int)S, (int)E, (int)K, chunk_tokens,                   \
+      psum + (WHOLE ? b0 : b0 * E), pcnt + (WHOLE ? 0 : b0 * E))
+#define JT_LAUNCH_WHOLE(W, PL) JT_LAUNCH_CHUNKS(W, PL, true)
+#define JT_LAUNCH_PARTS(W, PL) JT_LAUNCH_CHUNKS(W, PL, false)
+  if (chunks == 1) {
+    JT_BALANCE_WIDTHS(JT_LAUNCH_WHOLE);
+    balance_mean_kernel<<<1, kBalFinalThreads, 0, s>>>(psum, (int)B, loss);
+  } else {
+    JT_BALANCE_WIDTHS(JT_LAUNCH_PARTS);
+    balance_final_kernel<<<1, kBalFinalThreads, 0, s>>>(psum, pcnt, chunks, (int)B, (int)S, (int)E, (int)K, loss);
+  }
+#undef JT_LAUNCH_PARTS
+#undef JT_LAUNCH_WHOLE
+#undef JT_LAUNCH_CHUNKS
   return check_launch("sequence_balance_loss");
 }
 
