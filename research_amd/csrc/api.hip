@@ -676,12 +676,14 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
     stage_mark(kStageDown, main_stream);
     rc = check_launch("grouped gemm");
   } else {
+    // (a timed call keeps the shared experts in launches of their own: their stages would read as the router's)
+    const bool offer_shared = Is > 0 && g_stage_timer == nullptr;
     const SharedExperts shared{shared_gate, shared_up, shared_down, Is, w.shared_act, w.shared_y, shared_gate_pre,
                                shared_up_pre};
     rc = router_for_layer(x, w_router, expert_bias, T, H, E, K, route_scale, dtype, expert_ids, weights, scores,
                           expert_counts, importance, group_sizes, offsets, source_order, inverse, w.router,
                           w.router_bytes, score_func, &stats_done, &plan_done, main_stream, w.act, w.act_bytes,
-                          Is > 0 ? &shared : nullptr, &shared_done);
+                          offer_shared ? &shared : nullptr, &shared_done);
     if (rc) return rc;
     stage_mark(kStageRouter, main_stream);
     rc = dispatch_for_layer(expert_ids, weights, (T > 0 && !gather) ? x : nullptr, T, H, E, K, dtype, group_sizes,

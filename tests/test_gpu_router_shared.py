@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 import torch
 
-from research_amd import grad
+from research_amd import _ffi, grad, ops
 from test_gpu_layer_paths import test_decode_path_equals_the_stand_alone_operators as check_layer
 from test_gpu_parity import dev
 
@@ -46,3 +46,19 @@ def test_training_forward_keeps_the_shared_products(gpu, tokens):
     _, alone = grad.shared_swiglu_train(x, *shared)
     assert torch.equal(kept.shared.gate_pre, alone.gate_pre)
     assert torch.equal(kept.shared.up_pre, alone.up_pre)
+
+
+@pytest.mark.parametrize("tokens", [1, 20])
+def test_a_timed_call_times_the_shared_experts_as_such(gpu, tokens):
+    generator = torch.Generator(device=gpu).manual_seed(tokens)
+
+    def normal(*shape):
+        return (torch.randn(shape, generator=generator, device=gpu) * 0.05).to(torch.bfloat16)
+
+    args = (normal(tokens, 512), normal(512, 64), None, normal(64, 512, 64), normal(64, 512, 64), normal(64, 64, 512), 4, 1.0)
+    shared = normal(512, 1024), normal(512, 1024), normal(1024, 512)
+    stage_ms = []
+    timed = ops.moe_forward(*args, shared=shared, stage_ms=stage_ms)
+    assert torch.equal(timed.y, ops.moe_forward(*args, shared=shared).y)
+    stages = dict(zip(_ffi.STAGE_NAMES, stage_ms))
+    assert stages["shared_gate_up"] > 0.0 and stages["shared_down"] > 0.0, stages
