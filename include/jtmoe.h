@@ -176,6 +176,16 @@ int jtmoe_grouped_swiglu(const void* packed_x, const void* gate, const void* up,
  *   x [T,H] dtype; source_order [T*K] i32; others as jtmoe_grouped_swiglu.
  */
 int jtmoe_grouped_swiglu_gather_supported(int64_t T, int64_t H, int64_t I, int dtype);
+
+/*
+ * Which bf16 kernel takes a product of `rows` rows in E groups (0: one dense group) with a reduction of K
+ * and N columns, for 16-byte aligned operands below 2 GiB: host arithmetic only, no counterpart in the
+ * reference.  product: 0 gate/up, 1 down, 2 data gradient, 3 the sum of two data gradients.
+ * compute_units: of the device to answer for, 0: the current one.  The names ("stream_16x64", "rows64",
+ * "half", "rows256_tail", "general", ...) are for tests and tools and may change with the rules; "" for
+ * sizes out of range.
+ */
+const char* jtmoe_product_kernel(int product, int64_t rows, int64_t K, int64_t N, int64_t E, int compute_units);
 int jtmoe_grouped_swiglu_gather(const void* x, const int32_t* source_order,
                                 const void* gate, const void* up, const void* down,
                                 const int32_t* group_sizes, const int32_t* offsets,

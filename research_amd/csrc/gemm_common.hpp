@@ -242,8 +242,7 @@ inline double spread_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
 // gradients follow the same line (figures at DgradHalfCfg and DgradHalfDeepCfg); on the wrong side of it 32768
 // rows in 64 groups x 2048 -> 1408 would take 262 us against 228.
 enum class HalfTiles { kNone, kOnePerCu, kRounds };
-inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N) {
-  const double cus = (double)persistent_grid_size();
+inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, double cus) {
   const double half_n = (double)((N + 127) / 128), full_n = (double)((N + 255) / 256);
   if (expected_mtiles(rows, E, dense, 128) * half_n <= cus) return HalfTiles::kOnePerCu;
   auto pays = [cus](double half, double full) {

@@ -7,12 +7,32 @@
 
 namespace jtmoe {
 
+// The bf16 kernel of a product, as the dispatch rules choose it (jtmoe_product_kernel names them).  "Tail": K ends
+// inside a step, or a gate/up product that divides (silu_gate).
+enum class ProductKernel {
+  kGeneral,
+  kStream16x128,  // grouped_gemm_skinny.hpp: tiles of 16 or 32 rows
+  kStream16x64,
+  kStream32x64,
+  kRows64,        // 64-row LDS tiles, non-temporal loads of the matrix
+  kRows64Tail,
+  kHalf,          // 128 x 128 tiles
+  kHalfTail,
+  kHalfDeep,
+  kRows256,       // 256-row tiles: gate/up in the four-stage kernel, the others persistent with two stages
+  kRows256Tail,
+  kRows256Short,  // gate/up whose reduction is too short for four stages
+  kRows256ShortTail,
+};
+
 // C[rows of group e, :] = sum over s < segs of A_s[rows of e, :] @ B_s[e]^T
 //   A_s: [rows, Kdim], or [a_rows, Kdim] read through row_map (row j -> row_map[j] / row_div)
 //   B_s: [E, N, Kdim]      C: [rows, N]      group_sizes == nullptr: one group holding every row
 int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, const void* b1, void* c,
                    const int32_t* group_sizes, const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N,
                    int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream);
+// ... and the kernel it takes for bf16 operands (16-byte aligned, below 2 GiB) on `cus` compute units
+ProductKernel data_gradient_kernel(int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense, int segs, double cus);
 
 // C_i[e] = P[rows of group e, :]^T @ D_i[rows of group e, :]     (i = 0, and 1 if d1 is given)
 //   P: [rows, KA], D_i: [rows, N]; either may instead be [gathered_rows, .] read through row_map

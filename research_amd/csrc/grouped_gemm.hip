@@ -268,8 +268,6 @@ int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const 
 
 // ---- which kernel takes a product ------------------------------------------------------------------------
 // All times below: rows of T tokens in E groups by a balanced top-k, matrices cold, launch overhead included.
-enum class Tiles { kSkinny11, kSkinny12, kSkinny22, kTiny, kHalf, kHalfDeep, kFull };
-
 // Streaming tiles (grouped_gemm_skinny.hpp) while they find a CU each: of the shapes with at most one tile per CU
 // the one with the most tiles, so that the matrices are drawn through as many CUs as possible.  us for gate/up and
 // down together, 2048 -> 1408, 64 experts top-8, 1 token: 35 against 87 in 64-row LDS tiles; shared experts of 2816:
@@ -284,13 +282,13 @@ enum class Tiles { kSkinny11, kSkinny12, kSkinny22, kTiny, kHalf, kHalfDeep, kFu
 // tiles are resident, three to a CU (8 tokens, 64 experts 48 against 56), and where the LDS tiles start that round (12
 // and 20 tokens, 128 experts 41 and 52 against 56 and 58; 37 with two thirds of the experts reached 39 against 55;
 // balanced 63 against 62), but not in between (15 tokens, 64 experts 63 against 54).
-inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dual, Tiles* out) {
+inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dual, double cus, ProductKernel* out) {
   struct Shape {
-    Tiles id;
+    ProductKernel id;
     int RB, BN;
   };
-  constexpr Shape shapes[] = {{Tiles::kSkinny12, 1, 64}, {Tiles::kSkinny22, 2, 64}, {Tiles::kSkinny11, 1, 128}};
-  const double cus = (double)persistent_grid_size();
+  constexpr Shape shapes[] = {{ProductKernel::kStream16x64, 1, 64}, {ProductKernel::kStream32x64, 2, 64},
+                              {ProductKernel::kStream16x128, 1, 128}};
   double most = 0.0;
   for (const Shape& s : shapes) {
     const double tiles = expected_mtiles(rows, E, dense, 16 * s.RB) * (double)((N + s.BN - 1) / s.BN);
@@ -302,7 +300,7 @@ inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dua
   if (most == 0.0 && !dense && (double)rows <= 4.0 * expected_mtiles(rows, E, false, 16)) {
     const double tiles = expected_mtiles(rows, E, false, 16) * (double)((N + 127) / 128);
     const double lds_tiles = expected_mtiles(rows, E, false, 64) * (double)((N + 255) / 256);
-    *out = Tiles::kSkinny11;
+    *out = ProductKernel::kStream16x128;
     return dual ? tiles <= 2.0 * cus : tiles <= 3.0 * cus || lds_tiles > 2.0 * cus;
   }
   return most > 0.0;
@@ -314,19 +312,30 @@ inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dua
 // and 78).
 constexpr int64_t kTinyGroupRows = 52;  // four or fewer in a hundred groups above 64
 
-// Half tiles where they pay (half_tiles); gate/up only with at most one per CU: 1024 tokens, shared 2816: 41 us
+// Then half tiles where they pay (half_tiles); gate/up only with at most one per CU: 1024 tokens, shared 2816: 41 us
 // against 50 in 256-row tiles; with more, two rounds of half tiles: 2048 tokens 77 against 52.
-inline Tiles pick_large(int64_t rows, int64_t E, bool dense, int64_t N, bool dual) {
-  const HalfTiles half = half_tiles(rows, E, dense, N);
-  if (half == HalfTiles::kOnePerCu) return Tiles::kHalf;
-  return half == HalfTiles::kNone || dual ? Tiles::kFull : Tiles::kHalfDeep;
+ProductKernel gate_up_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, bool dense, double cus,
+                             const int32_t* row_map = nullptr, int row_div = 1) {
+  const bool tail = H % 64 != 0;
+  ProductKernel k;
+  if (pick_skinny(rows, E, dense, I, true, cus, &k)) return k;
+  if (!dense && rows <= kTinyGroupRows * E) return tail ? ProductKernel::kRows64Tail : ProductKernel::kRows64;
+  if (half_tiles(rows, E, dense, I, cus) == HalfTiles::kOnePerCu &&
+      stream_ok<GateUpHalfTailCfg>(rows, H, I, row_map, row_div))
+    return tail ? ProductKernel::kHalfTail : ProductKernel::kHalf;
+  if (stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div))
+    return tail ? ProductKernel::kRows256Tail : ProductKernel::kRows256;
+  return tail ? ProductKernel::kRows256ShortTail : ProductKernel::kRows256Short;
 }
 
-inline Tiles pick_tiles(int64_t rows, int64_t E, bool dense, int64_t N, bool dual) {
-  Tiles t;
-  if (pick_skinny(rows, E, dense, N, dual, &t)) return t;
-  if (!dense && rows <= kTinyGroupRows * E) return Tiles::kTiny;
-  return pick_large(rows, E, dense, N, dual);
+ProductKernel down_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, bool dense, double cus) {
+  ProductKernel k;
+  if (pick_skinny(rows, E, dense, H, false, cus, &k)) return k;
+  if (!dense && rows <= kTinyGroupRows * E) return ProductKernel::kRows64;
+  const HalfTiles half = half_tiles(rows, E, dense, H, cus);
+  if (half == HalfTiles::kOnePerCu && stream_ok<DownHalfCfg>(rows, I, H, nullptr, 1)) return ProductKernel::kHalf;
+  if (half != HalfTiles::kNone && stream_ok<DownHalfDeepCfg>(rows, I, H, nullptr, 1)) return ProductKernel::kHalfDeep;
+  return I % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
 }
 
 inline bool fast_ok(const void* a, const void* b0, const void* b1, const void* c, int64_t Kdim, int64_t N) {
@@ -343,18 +352,22 @@ int launch_down_fast(const void* act, const void* down, const int32_t* group_siz
   using S11 = SkinnyCfg<1, 1, false>;
   using S12 = SkinnyCfg<1, 2, false>;
   using S22 = SkinnyCfg<2, 2, false>;
-  const Tiles t = pick_tiles(rows, E, group_sizes == nullptr, H, false);
-  switch (t) {
-    case Tiles::kSkinny11: return JT_DOWN(launch_skinny, S11), a_group_rows);
-    case Tiles::kSkinny12: return JT_DOWN(launch_skinny, S12), a_group_rows);
-    case Tiles::kSkinny22: return JT_DOWN(launch_skinny, S22), a_group_rows);
-    case Tiles::kTiny: return JT_DOWN(launch_fast, DownTinyCfg), 0, a_group_rows);
+  const ProductKernel k = down_kernel(rows, H, I, E, group_sizes == nullptr, persistent_grid_size());
+  switch (k) {
+    case ProductKernel::kStream16x128: return JT_DOWN(launch_skinny, S11), a_group_rows);
+    case ProductKernel::kStream16x64: return JT_DOWN(launch_skinny, S12), a_group_rows);
+    case ProductKernel::kStream32x64: return JT_DOWN(launch_skinny, S22), a_group_rows);
+    case ProductKernel::kRows64: return JT_DOWN(launch_fast, DownTinyCfg), 0, a_group_rows);
     default: break;
   }
-  if (a_group_rows > 0) return JT_DOWN(launch_fast, DownTinyCfg), 0, a_group_rows);
-  if (t == Tiles::kHalf && stream_ok<DownHalfCfg>(rows, I, H, nullptr, 1)) return JT_DOWN(launch_stream, DownHalfCfg), 2);
-  if (t != Tiles::kFull && stream_ok<DownHalfDeepCfg>(rows, I, H, nullptr, 1)) return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
-  return I % 64 == 0 ? JT_DOWN(launch_fast, DownCfg)) : JT_DOWN(launch_fast, DownTailCfg));
+  // (at most half a tile of rows per group on the decode path: the rules above take all of it)
+  if (row_map) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: no down kernel reads blocks of rows per group at this size");
+  switch (k) {
+    case ProductKernel::kHalf: return JT_DOWN(launch_stream, DownHalfCfg), 2);
+    case ProductKernel::kHalfDeep: return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
+    case ProductKernel::kRows256: return JT_DOWN(launch_fast, DownCfg));
+    default: return JT_DOWN(launch_fast, DownTailCfg));
+  }
 #undef JT_DOWN
 }
 
@@ -375,24 +388,18 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
     using S11 = SkinnyCfg<1, 1, true>;
     using S12 = SkinnyCfg<1, 2, true>;
     using S22 = SkinnyCfg<2, 2, true>;
-    switch (pick_tiles(rows, E, dense, I, true)) {
-      case Tiles::kSkinny11: rc = JT_GATE_UP(launch_skinny, S11); break;
-      case Tiles::kSkinny12: rc = JT_GATE_UP(launch_skinny, S12); break;
-      case Tiles::kSkinny22: rc = JT_GATE_UP(launch_skinny, S22); break;
-      case Tiles::kTiny:
-        rc = H % 64 == 0 ? JT_GATE_UP(launch_fast, GateUpTinyCfg) : JT_GATE_UP(launch_fast, GateUpTinyTailCfg);
-        break;
-      case Tiles::kHalf:
-        if (stream_ok<GateUpHalfTailCfg>(rows, H, I, row_map, row_div)) {
-          rc = H % 64 == 0 ? JT_GATE_UP(launch_stream, GateUpHalfCfg) : JT_GATE_UP(launch_stream, GateUpHalfTailCfg);
-          break;
-        }
-        [[fallthrough]];
-      default:
-        if (stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div))
-          rc = H % 64 == 0 ? JT_GATE_UP(launch_stream, GateUpStreamCfg) : JT_GATE_UP(launch_stream, GateUpStreamTailCfg);
-        else
-          rc = H % 64 == 0 ? JT_GATE_UP(launch_fast, GateUpCfg) : JT_GATE_UP(launch_fast, GateUpTailCfg);
+    switch (gate_up_kernel(rows, H, I, E, dense, persistent_grid_size(), row_map, row_div)) {
+      case ProductKernel::kStream16x128: rc = JT_GATE_UP(launch_skinny, S11); break;
+      case ProductKernel::kStream16x64: rc = JT_GATE_UP(launch_skinny, S12); break;
+      case ProductKernel::kStream32x64: rc = JT_GATE_UP(launch_skinny, S22); break;
+      case ProductKernel::kRows64: rc = JT_GATE_UP(launch_fast, GateUpTinyCfg); break;
+      case ProductKernel::kRows64Tail: rc = JT_GATE_UP(launch_fast, GateUpTinyTailCfg); break;
+      case ProductKernel::kHalf: rc = JT_GATE_UP(launch_stream, GateUpHalfCfg); break;
+      case ProductKernel::kHalfTail: rc = JT_GATE_UP(launch_stream, GateUpHalfTailCfg); break;
+      case ProductKernel::kRows256: rc = JT_GATE_UP(launch_stream, GateUpStreamCfg); break;
+      case ProductKernel::kRows256Tail: rc = JT_GATE_UP(launch_stream, GateUpStreamTailCfg); break;
+      case ProductKernel::kRows256Short: rc = JT_GATE_UP(launch_fast, GateUpCfg); break;
+      default: rc = JT_GATE_UP(launch_fast, GateUpTailCfg); break;
     }
   }
 #undef JT_GATE_UP
@@ -440,8 +447,9 @@ int launch_down_from_all_tokens(const void* act_full, const void* down, const in
 
 bool shared_in_skinny_tiles(const void* x, const SharedExperts& s, int64_t T, int64_t H) {
   return fast_ok(x, s.gate, s.up, s.act, H, s.Is) && fast_ok(s.act, s.down, nullptr, s.y, s.Is, H) &&
-         aligned16(s.gate_pre) && aligned16(s.up_pre) && pick_tiles(T, 1, true, s.Is, true) == Tiles::kSkinny12 &&
-         pick_tiles(T, 1, true, H, false) == Tiles::kSkinny12;
+         aligned16(s.gate_pre) && aligned16(s.up_pre) &&
+         gate_up_kernel(T, H, s.Is, 1, true, persistent_grid_size()) == ProductKernel::kStream16x64 &&
+         down_kernel(T, H, s.Is, 1, true, persistent_grid_size()) == ProductKernel::kStream16x64;
 }
 
 // ---- the gathering launch pair as the layer uses it (declared in common.hpp) ----
@@ -488,6 +496,25 @@ extern "C" int jtmoe_shared_swiglu(const void* x, const void* gate, const void* 
   if (dtype == JTMOE_BF16)
     return launch_pair<bf16_raw>(x, gate, up, down, nullptr, nullptr, T, H, Is, 1, act, shared_y, s, kStageSharedGateUp);
   return launch_pair<float>(x, gate, up, down, nullptr, nullptr, T, H, Is, 1, act, shared_y, s, kStageSharedGateUp);
+}
+
+// the kernel that the rules above choose, by name
+extern "C" const char* jtmoe_product_kernel(int product, int64_t rows, int64_t K, int64_t N, int64_t E, int compute_units) {
+  static const char* const names[] = {"general", "stream_16x128", "stream_16x64", "stream_32x64", "rows64", "rows64_tail",
+                                      "half", "half_tail", "half_deep", "rows256", "rows256_tail", "rows256_short",
+                                      "rows256_short_tail"};
+  const bool dense = E == 0;
+  if (product < 0 || product > 3 || rows <= 0 || K <= 0 || N <= 0 || E < 0 || K >= ((int64_t)1 << 24) ||
+      N >= ((int64_t)1 << 24) || rows >= ((int64_t)1 << 31) || compute_units < 0)
+    return "";
+  const double cus = compute_units > 0 ? compute_units : persistent_grid_size();
+  const int64_t groups = dense ? 1 : E;
+  ProductKernel k = ProductKernel::kGeneral;
+  if (product >= 2)
+    k = data_gradient_kernel(rows, K, N, groups, dense, product - 1, cus);
+  else if (fast_ok(nullptr, nullptr, nullptr, nullptr, K, N))
+    k = product == 0 ? gate_up_kernel(rows, K, N, groups, dense, cus) : down_kernel(rows, N, K, groups, dense, cus);
+  return names[(int)k];
 }
 
 extern "C" int jtmoe_grouped_swiglu_gather_supported(int64_t T, int64_t H, int64_t I, int dtype) {

@@ -195,27 +195,32 @@ int launch_nt_stream(const void* a0, const void* a1, const void* b0, const void*
 
 }  // namespace
 
+ProductKernel data_gradient_kernel(int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense, int segs, double cus) {
+  if (Kdim % 8 != 0 || N % 8 != 0 || N * Kdim >= kOperandLimit) return ProductKernel::kGeneral;
+  const HalfTiles half = rows * N * 2 <= (int64_t)0x7ffe0000 ? half_tiles(rows, E, dense, N, cus) : HalfTiles::kNone;
+  if (half == HalfTiles::kOnePerCu && (Kdim + 63) / 64 * segs >= 2 * DgradHalfDeepCfg::NSTAGE)
+    return ProductKernel::kHalfDeep;
+  if (half != HalfTiles::kNone) return ProductKernel::kHalf;
+  return Kdim % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
+}
+
 int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, const void* b1, void* c,
                    const int32_t* group_sizes, const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N,
                    int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream) {
   if (rows == 0) return JTMOE_OK;
   const bool dense = group_sizes == nullptr;
-  const bool fast = dtype == JTMOE_BF16 && Kdim % 8 == 0 && N % 8 == 0 && N * Kdim < kOperandLimit &&
-                    (row_map ? a_rows : rows) * Kdim < kOperandLimit && aligned16(a0) && aligned16(b0) &&
-                    (segs == 1 || (aligned16(a1) && aligned16(b1))) && aligned16(c);
-  const HalfTiles half = fast && rows * N * 2 <= (int64_t)0x7ffe0000 ? half_tiles(rows, E, dense, N) : HalfTiles::kNone;
-  if (half == HalfTiles::kOnePerCu && (Kdim + 63) / 64 * segs >= 2 * DgradHalfDeepCfg::NSTAGE)
-    return launch_nt_stream<DgradHalfDeepCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map,
-                                              row_div, a_rows, segs, stream);
-  if (half != HalfTiles::kNone)
-    return launch_nt_fast<DgradHalfCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div,
-                                        a_rows, segs, stream);
-  if (fast && Kdim % 64 == 0)
-    return launch_nt_fast<DgradCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div,
-                                    a_rows, segs, stream);
-  if (fast)
-    return launch_nt_fast<DgradTailCfg>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div,
-                                        a_rows, segs, stream);
+  const bool fast = dtype == JTMOE_BF16 && (row_map ? a_rows : rows) * Kdim < kOperandLimit && aligned16(a0) &&
+                    aligned16(b0) && (segs == 1 || (aligned16(a1) && aligned16(b1))) && aligned16(c);
+#define JT_NT(LAUNCH, CFG) \
+  LAUNCH<CFG>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div, a_rows, segs, stream)
+  switch (fast ? data_gradient_kernel(rows, Kdim, N, E, dense, segs, persistent_grid_size()) : ProductKernel::kGeneral) {
+    case ProductKernel::kHalfDeep: return JT_NT(launch_nt_stream, DgradHalfDeepCfg);
+    case ProductKernel::kHalf: return JT_NT(launch_nt_fast, DgradHalfCfg);
+    case ProductKernel::kRows256: return JT_NT(launch_nt_fast, DgradCfg);
+    case ProductKernel::kRows256Tail: return JT_NT(launch_nt_fast, DgradTailCfg);
+    default: break;
+  }
+#undef JT_NT
   if (dtype == JTMOE_F32 && f32_gemm_supported(a0, a1, b0, b1, c, row_map ? a_rows : rows, Kdim, N) &&
       !(row_map && segs > 1))
     return launch_f32_nt(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div, a_rows, segs,

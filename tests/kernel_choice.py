@@ -1,0 +1,23 @@
+"""Which kernel the library's rules choose for the expert products, for tests that name the kernels they are about."""
+
+from __future__ import annotations
+
+from research_amd import _ffi
+
+GATE_UP, DOWN, DATA_GRADIENT, DATA_GRADIENT_PAIR = range(4)
+MI355X_CUS = 256
+
+
+def chosen(product, rows, reduction, columns, experts, cus=0):
+    """Name of the bf16 kernel (experts = 0: a dense product; cus = 0: on the current device)."""
+    return _ffi.load_library().jtmoe_product_kernel(product, rows, reduction, columns, experts, cus).decode()
+
+
+def forward_kernels(rows, hidden, inter, experts=0, cus=0):
+    return chosen(GATE_UP, rows, hidden, inter, experts, cus), chosen(DOWN, rows, inter, hidden, experts, cus)
+
+
+def gradient_kernels(rows, hidden, inter, experts=0, cus=0):
+    """Those of dZ = dY Wd^T and of dX = dG Wg^T + dU Wu^T."""
+    return (chosen(DATA_GRADIENT, rows, hidden, inter, experts, cus),
+            chosen(DATA_GRADIENT_PAIR, rows, inter, hidden, experts, cus))

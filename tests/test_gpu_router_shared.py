@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 import torch
 
+from kernel_choice import forward_kernels
 from research_amd import _ffi, grad, ops
 from test_gpu_layer_paths import test_decode_path_equals_the_stand_alone_operators as check_layer
 from test_gpu_parity import dev
@@ -17,17 +18,22 @@ from test_gpu_parity import dev
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tokens,hidden,experts,top_k,d_ff,shared_width", [
-    (1, 2048, 64, 8, 1408, 2816),  # the benchmark's model
-    (1, 128, 16, 1, 64, 8),        # one slice, one 8-wide column tile, a reduction of one chunk
-    (3, 384, 16, 1, 64, 200),      # three slices, a ragged last column tile
-    (15, 256, 64, 8, 64, 1000),    # the last row of a 16-row tile missing
-    (17, 2176, 256, 1, 64, 72),    # two token blocks, the second of one token; 256 experts
-    (64, 1024, 128, 2, 64, 2816),  # the largest batch
-    (65, 1024, 128, 1, 64, 2816),  # a token more: launches of their own
-    (64, 128, 128, 1, 64, 8200),   # more tiles than CUs: launches of their own
-])
-def test_layer_equals_the_stand_alone_operators(gpu, tokens, hidden, experts, top_k, d_ff, shared_width):
+SHAPES = [
+    # tokens, hidden, experts, top_k, d_ff, shared width, whether the router takes the shared experts along
+    (1, 2048, 64, 8, 1408, 2816, True),   # the benchmark's model
+    (1, 128, 16, 1, 64, 8, True),         # one slice, one 8-wide column tile, a reduction of one chunk
+    (3, 384, 16, 1, 64, 200, True),       # three slices, a ragged last column tile
+    (15, 256, 64, 8, 64, 1000, True),     # the last row of a 16-row tile missing
+    (17, 2176, 256, 1, 64, 72, True),     # two token blocks, the second of one token; 256 experts
+    (64, 1024, 128, 2, 64, 2816, True),   # the largest batch
+    (65, 1024, 128, 1, 64, 2816, False),  # a token more: launches of their own
+    (64, 128, 128, 1, 64, 8200, False),   # more tiles than CUs: launches of their own
+]
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,top_k,d_ff,shared_width,beside", SHAPES)
+def test_layer_equals_the_stand_alone_operators(gpu, tokens, hidden, experts, top_k, d_ff, shared_width, beside):
+    assert beside == (tokens <= 64 and forward_kernels(tokens, hidden, shared_width) == ("stream_16x64", "stream_16x64"))
     check_layer(gpu, tokens, hidden, experts, top_k, d_ff, shared_width)
 
 

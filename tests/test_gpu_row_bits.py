@@ -17,6 +17,9 @@ from research_amd import grad, ops
 pytestmark = pytest.mark.gpu
 
 WIDTHS = [(1024, 704), (512, 2816), (2048, 192), (1000, 264), (264, 1352), (72, 2056)]
+DENSE_ROWS = (1, 3, 16, 17, 64, 65, 130, 260, 520, 1030, 2600)
+EXPERTS = (5, 64)
+GROUP_ROWS, MOST_ROWS = (1, 2, 3, 9, 20, 40, 70), 6000
 
 
 def drawer(gpu, seed):
@@ -31,20 +34,20 @@ def drawer(gpu, seed):
 @pytest.mark.parametrize("hidden,inter", WIDTHS)
 def test_shared_rows_do_not_depend_on_the_call(gpu, hidden, inter):
     normal = drawer(gpu, hidden)
-    x = normal(2600, hidden)
+    x = normal(DENSE_ROWS[-1], hidden)
     matrices = normal(hidden, inter, std=0.05), normal(hidden, inter, std=0.05), normal(inter, hidden, std=0.05)
     whole = ops.shared_swiglu(x, *matrices)
-    for rows in (1, 3, 16, 17, 64, 65, 130, 260, 520, 1030):
+    for rows in DENSE_ROWS[:-1]:
         part = ops.shared_swiglu(x[:rows].contiguous(), *matrices)
         assert torch.equal(part, whole[:rows]), f"{rows} rows: {int((part != whole[:rows]).sum())} values differ"
 
 
 @pytest.mark.parametrize("hidden,inter", WIDTHS)
-@pytest.mark.parametrize("experts", [5, 64])
+@pytest.mark.parametrize("experts", EXPERTS)
 def test_routed_rows_do_not_depend_on_the_call(gpu, hidden, inter, experts):
     """Rows of every group: the first few of each alone against all of them."""
     normal = drawer(gpu, hidden + experts)
-    per_group = 6000 // experts
+    per_group = MOST_ROWS // experts
     x = normal(experts * per_group, hidden)
     matrices = (normal(experts, hidden, inter, std=0.05), normal(experts, hidden, inter, std=0.05),
                 normal(experts, inter, hidden, std=0.05))
@@ -56,7 +59,7 @@ def test_routed_rows_do_not_depend_on_the_call(gpu, hidden, inter, experts):
         return ops.grouped_swiglu(part, *matrices, sizes, offsets).view(experts, rows, hidden)
 
     whole = run(per_group)
-    for rows in (1, 2, 3, 9, 20, 40, 70):
+    for rows in GROUP_ROWS:
         part = run(rows)
         assert torch.equal(part, whole[:, :rows]), f"{rows} rows: {int((part != whole[:, :rows]).sum())} values differ"
 

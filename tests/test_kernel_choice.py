@@ -1,0 +1,62 @@
+"""The rules that deal the expert products to kernels, asked on the CPU for a device of 256 compute units.
+
+What the GPU tests say about the kernels they exercise is checked here without a GPU, and that between them they
+exercise every kernel, so that a change of a rule cannot take a kernel's last test away unseen.
+"""
+
+from __future__ import annotations
+
+import pytest
+
+import test_gpu_ragged_widths as ragged
+import test_gpu_row_bits as row_bits
+import test_gpu_tile_choice as tiles
+from kernel_choice import DOWN, GATE_UP, MI355X_CUS, chosen, forward_kernels, gradient_kernels
+
+GATE_UP_KERNELS = {"stream_16x128", "stream_16x64", "stream_32x64", "rows64", "rows64_tail", "half", "half_tail", "rows256",
+                   "rows256_tail", "rows256_short", "rows256_short_tail"}
+DOWN_KERNELS = {"stream_16x128", "stream_16x64", "stream_32x64", "rows64", "half", "half_deep", "rows256", "rows256_tail"}
+GRADIENT_KERNELS = {"half", "half_deep", "rows256", "rows256_tail"}
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,top_k,inter,forward,gradients", tiles.GROUPED + ragged.SHAPES)
+def test_grouped_shapes_take_the_kernels_they_name(tokens, hidden, experts, top_k, inter, forward, gradients):
+    assert " ".join(forward_kernels(tokens * top_k, hidden, inter, experts, MI355X_CUS)) == forward
+    assert " ".join(gradient_kernels(tokens * top_k, hidden, inter, experts, MI355X_CUS)) == gradients
+
+
+@pytest.mark.parametrize("tokens,hidden,inter,forward,gradients", tiles.DENSE)
+def test_dense_shapes_take_the_kernels_they_name(tokens, hidden, inter, forward, gradients):
+    assert " ".join(forward_kernels(tokens, hidden, inter, cus=MI355X_CUS)) == forward
+    assert " ".join(gradient_kernels(tokens, hidden, inter, cus=MI355X_CUS)) == gradients
+
+
+@pytest.mark.parametrize("tokens,hidden,inter,experts,kernels", ragged.LAST_ROWS)
+def test_last_row_shapes_take_the_kernels_they_name(tokens, hidden, inter, experts, kernels):
+    assert " ".join(forward_kernels(tokens, hidden, inter, experts, MI355X_CUS)) == kernels
+
+
+def test_every_kernel_is_checked_against_the_oracle():
+    forward = [case[5].split() for case in tiles.GROUPED + ragged.SHAPES] + [case[3].split() for case in tiles.DENSE]
+    gradients = [case[6].split() for case in tiles.GROUPED + ragged.SHAPES] + [case[4].split() for case in tiles.DENSE]
+    assert {gate_up for gate_up, _ in forward} == GATE_UP_KERNELS
+    assert {down for _, down in forward} == DOWN_KERNELS
+    assert {dz for dz, _ in gradients} == GRADIENT_KERNELS
+    assert {dx for _, dx in gradients} == GRADIENT_KERNELS
+
+
+def test_every_kernel_is_held_to_the_bits_of_the_others():
+    seen = set()
+    for hidden, inter in row_bits.WIDTHS:
+        for rows in row_bits.DENSE_ROWS:
+            seen.update(zip((GATE_UP, DOWN), forward_kernels(rows, hidden, inter, cus=MI355X_CUS)))
+        for experts in row_bits.EXPERTS:
+            for rows in (*row_bits.GROUP_ROWS, row_bits.MOST_ROWS // experts):
+                seen.update(zip((GATE_UP, DOWN), forward_kernels(rows * experts, hidden, inter, experts, MI355X_CUS)))
+    assert {kernel for product, kernel in seen if product == GATE_UP} >= GATE_UP_KERNELS - {"rows256_short"}
+    assert {kernel for product, kernel in seen if product == DOWN} >= DOWN_KERNELS
+
+
+def test_sizes_out_of_range_have_no_kernel():
+    assert chosen(GATE_UP, 0, 64, 64, 1, MI355X_CUS) == chosen(4, 1, 64, 64, 1, MI355X_CUS) == ""
+    assert chosen(GATE_UP, 1, 63, 64, 1, MI355X_CUS) == chosen(DOWN, 1, 64, 12, 1, MI355X_CUS) == "general"
