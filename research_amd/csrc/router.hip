@@ -1196,15 +1196,17 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
       if (stats) router_finalize_kernel<<<1, 256, 0, stream>>>(ws, (int)E, counts, importance);
       return check_launch("router");
     }
-    // Middle-sized layer calls: a 64-token workgroup walks all of H, 26 us (E = 64) and 40 us (E = 128) whether
-    // there are 300 tokens or 8000; up to kMidMaxTokens the slices are computed in workgroups of their own, in the
-    // layer's memory, and a workgroup per 16 tokens finishes.  us at 2048 columns, split + finish against one
-    // launch: E = 64: 300 tokens 4.4 + 9.9 / 23.6, 1024: 5.7 + 10.2 / 26.1, 2048: 9.1 + 10.6 / 25.9, 4096: 16.1 + 11.4
-    // / 27.7; E = 128: 5.7 + 15.6 / 37.6, 7.9 + 15.9 / 40.4, 13.5 + 16.5 / 40.0, 24.4 + 16.8 / 41.3.  E = 16 at 1024
-    // columns: 4.4 + 4.3 / 10.1, which the gap between the launches takes back.
+    // Middle-sized layer calls: a 64-token workgroup walks all of H, 26 us (E = 64) and 40 us (E = 128) at 2048 columns
+    // whether there are 300 tokens or 8000; up to kMidMaxTokens the slices are computed in workgroups of their own, in
+    // the layer's memory, and a workgroup per 16 tokens finishes.  us, split + finish against one launch, E = 64: 300
+    // tokens 4.4 + 9.9 / 23.6, 1024: 5.7 + 10.2 / 26.1, 2048: 9.1 + 10.6 / 25.9, 4096: 16.1 + 11.4 / 27.7; E = 128:
+    // 5.7 + 15.6 / 37.6, 7.9 + 15.9 / 40.4, 13.5 + 16.5 / 40.0, 24.4 + 16.8 / 41.3.
+    // The walk grows with H and E, the second launch does not: a layer call gains, at 300 and 2560 tokens, E = 16: 5.4
+    // and 4.0 us at 2048 columns, 1.7 and 1.6 at 1024, 0.8 and 0.2 at 768, 0 and -0.3 at 512; E = 256: 40 and 18, 20 and
+    // 7, 13 and 6, 8 and 3.  The line is drawn where every expert count gains.
     const int slice_rows = router_slice_rows((int)H);
     const int slices = (int)((H + slice_rows - 1) / slice_rows);
-    if (layer && tokens <= kMidMaxTokens && (E == 64 || E == 128) && H % kSplitKC == 0 && H >= 2048 &&
+    if (layer && tokens <= kMidMaxTokens && H % kSplitKC == 0 && H >= 1024 &&
         (size_t)slices * tokens * E * sizeof(float) <= layer->scratch_bytes) {
       const size_t smem = (size_t)2 * kSplitKC * router_w_stride((int)E) * 2;
       const size_t fsmem = router_smem_bytes((int)E, (int)K, 16);
@@ -1222,8 +1224,11 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
         score_func);                                                                                         \
   } break;
         switch ((int)E) {
+          JT_PARTIAL_CASE(1)
+          JT_PARTIAL_CASE(2)
           JT_PARTIAL_CASE(4)
           JT_PARTIAL_CASE(8)
+          JT_PARTIAL_CASE(16)
         }
 #undef JT_PARTIAL_CASE
         auto finish = router_finish_blocks_kernel<16, 256>;

@@ -16,6 +16,10 @@ pytestmark = pytest.mark.gpu
     (2561, 2048, 64, 2),  # a token more: 64-token workgroups
     (1000, 2048, 128, 8),
     (600, 2048, 128, 1),
+    (257, 1024, 16, 2),   # the narrowest rows: eight slices of one chunk
+    (700, 1152, 32, 4),   # nine chunks: slices of two, the last of one
+    (2560, 1024, 256, 8), # the most experts
+    (700, 896, 256, 2),   # narrower: 64-token workgroups
     (512, 128, 16, 8),    # 4096 assignments: one workgroup
     (513, 128, 16, 8),    # 4104: histogram and rank passes
 ])
