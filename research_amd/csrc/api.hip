@@ -495,8 +495,9 @@ LayerWorkspace carve_layer(void* base, int64_t T, int64_t H, int64_t E, int64_t 
   w.router = c.take(w.router_bytes);
   w.dispatch_bytes = dispatch_layer_workspace_bytes((int64_t)A, E);
   w.dispatch = c.take(w.dispatch_bytes);
-  // the permuted copy of x exists only where the grouped GEMM cannot fetch its rows through the
-  // permutation itself (a third of the workspace at 64 experts x top-8 x 2048)
+  // Room for a permuted copy of x (a third of the workspace at 64 experts x top-8 x 2048) for every shape that the
+  // gathering entry point refuses, as the size of the workspace has always been; the layer itself fetches the rows
+  // through the permutation up to 1 GiB of x and writes the copy only beyond.
   w.packed_x = jtmoe_grouped_swiglu_gather_supported(T, H, I, dtype) ? nullptr : c.take(A * (size_t)H * b);
   // (the decode path keeps the activations of all tokens through every expert)
   const size_t act_rows = decode_dense_supported(T, H, E, K, I, dtype) ? (size_t)E * (size_t)T : A;

@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void combine_bf16_vec_kernel(const uint4* __re
 
 // fp32 rows of a multiple of 4 elements, 16-byte aligned, without the norm: one wave per token, one 16-byte
 // vector per lane and step, the rows of four slots in flight.  (One element per lane took 11 us at 2048 tokens x
-// top-2 x 512, 4.2 MB each way; this takes 5, as long as the profiler
+// top-2 x 512, 8.4 MB in and 4.2 out; this takes 5, as long as the profiler
 // shows for an empty launch.)
 __global__ __launch_bounds__(256) void combine_f32_vec_kernel(const float4* __restrict__ packed_y,
                                                               const int32_t* __restrict__ inverse,

@@ -238,7 +238,8 @@ inline double spread_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
 // twice as often, so beyond one per CU they are taken only where that is 15 % less.  Down products: one half tile
 // per CU 40 us against 63 (2048 tokens, shared 2816; 64-deep steps 41), two per CU with 64-deep steps 55 against 64
 // (4096 tokens; 32-deep 69); 8192 rows x 2048 -> 1024 in 8 groups: 57 against 56 (576 tiles, whole ones kept);
-// 16384 rows: 84 against 100 (1088 against 272 tiles: the whole ones start a second round for 16 of them).  The data
+// 16384 rows in 16 groups x 2816 -> 1024 (1088 against 288 tiles: the whole ones start a second round for 32 of them):
+// 145 against 152 inside the layer call, whose gate/up launch then clocks lower: 372 against 374 for the call.  The data
 // gradients follow the same line (figures at DgradHalfCfg and DgradHalfDeepCfg); on the wrong side of it 32768
 // rows in 64 groups x 2048 -> 1408 would take 262 us against 228.
 enum class HalfTiles { kNone, kOnePerCu, kRounds };

@@ -30,7 +30,7 @@
 // the matrix).  The 64-row kernel always checks, once per step; the persistent and the stream kernel have variants of
 // their own (OPT & 65536), because the check costs registers that the others do not have to spare.  Before,
 // such widths ran element by element in the generic kernel: 2931 x 3 rows, 1000 x 2664, 24 experts with a
-// shared expert took 1122 + 967 us (routed) and 415 + 464 us (shared), now 122 + 81 and 36 + 64 us.
+// shared expert took 1122 + 967 us (routed) and 415 + 464 us (shared), now 130 + 79 and 38 + 46 us.
 //
 // Requirements: K % 8 == 0, N % 8 == 0, 16-byte aligned pointers, K*N*2 < 2^31.
 #pragma once

@@ -6,7 +6,7 @@
 //
 // Bound: HBM (a matrix element is used by a handful of rows), through what one CU can draw: 50 to 60 GB/s from
 // memory and twice that from the L2, however many loads its waves have in flight, so that the chip's 6 TB/s
-// take the greater part of its CUs.  A launch of the LDS kernels at these sizes has 8 to 100 tiles, and a
+// take a hundred of its CUs or more.  A launch of the LDS kernels at these sizes has 8 to 100 tiles, and a
 // 32-deep step of a tile costs 0.65 us whatever the depth of its pipeline (wait, barrier, LDS reads and
 // products of 64 mostly empty rows with one wave per SIMD: 1500 cycles for 16 KB).  Hence here
 //   * narrow tiles: 128 / FOLD columns of one matrix, or of each of two (kDual);

@@ -1044,7 +1044,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
 // The two launches of the small-batch router with the shared experts beside it: the gate/up tiles next to the
 // workgroups of the partial sums, the down tiles next to the finishing workgroup.  Each launch is bound by one
 // workgroup's own chain of dependent steps, on a few dozen CUs, and nothing of one is needed by the other.
-// One token, 2048 wide, 64 experts, shared 2816: 17.8 + 14.3 us, against 4.4 + 10.6 (router) and 18 + 13.5 (shared) in
+// One token, 2048 wide, 64 experts, shared 2816: 17.5 + 14.9 us, against 4.4 + 10.6 (router) and 18 + 13.5 (shared) in
 // four launches.
 // ---------------------------------------------------------------------------
 using SharedGateUpCfg = SkinnyCfg<1, 2, true>;
