@@ -27,7 +27,9 @@ pytestmark = pytest.mark.gpu
     (65, 36, 3, 2, 68),       # a second 32-deep step of one chunk, tiles with one row
     (400, 128, 2, 2, 192),    # whole tiles with gathered rows
     (600, 260, 3, 1, 132),    # columns and steps that end one chunk in
-    (2500, 64, 4, 2, 256),    # enough tiles for the 128-row forms
+    (2500, 64, 4, 2, 256),    # enough tiles for 128-row gate/up tiles: 168 of them against 324 in two rounds of 256
+    (2500, 644, 4, 2, 652),   # ... and 128 x 128 down products and data gradients (252 against 891 tiles), ragged ends
+    (1200, 508, 8, 2, 1020),  # ... and weight gradients, single (256 against 1024) and dual
 ])
 def test_f32_experts_at_tile_edges(gpu, tokens, hidden, experts, top_k, inter):
     P.test_grouped_swiglu_matches_oracle(gpu, tokens, hidden, experts, top_k, inter, "f32")
