@@ -186,6 +186,12 @@ int jtmoe_grouped_swiglu_gather_supported(int64_t T, int64_t H, int64_t I, int d
  * sizes out of range.
  */
 const char* jtmoe_product_kernel(int product, int64_t rows, int64_t K, int64_t N, int64_t E, int compute_units);
+/*
+ * Which bf16 kernel takes a product of the routed experts and the same product of the shared ones (width Is) in one
+ * launch of a layer call, forward (0, 1) or backward (2, 3); "separate": launches of their own.  Otherwise as above.
+ */
+const char* jtmoe_joint_kernel(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is, int64_t E,
+                               int compute_units);
 int jtmoe_grouped_swiglu_gather(const void* x, const int32_t* source_order,
                                 const void* gate, const void* up, const void* down,
                                 const int32_t* group_sizes, const int32_t* offsets,

@@ -664,6 +664,10 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
   hipStream_t main_stream = as_stream(stream);
   const bool decode = !train && decode_dense_supported(T, H, E, K, I, dtype);
   bool stats_done = false, plan_done = false, shared_done = false;
+  // (a timed call keeps the shared experts in launches of their own, so that their stages are theirs)
+  const bool offer_shared = Is > 0 && g_stage_timer == nullptr;
+  const SharedExperts shared{shared_gate, shared_up, shared_down, Is, w.shared_act, w.shared_y, shared_gate_pre,
+                             shared_up_pre};
   int rc;
   if (decode) {
     rc = launch_decode_gate_up_router(x, w_router, expert_bias, gate, up, w.act, T, H, E, K, I, route_scale,
@@ -677,10 +681,6 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
     stage_mark(kStageDown, main_stream);
     rc = check_launch("grouped gemm");
   } else {
-    // (a timed call keeps the shared experts in launches of their own: their stages would read as the router's)
-    const bool offer_shared = Is > 0 && g_stage_timer == nullptr;
-    const SharedExperts shared{shared_gate, shared_up, shared_down, Is, w.shared_act, w.shared_y, shared_gate_pre,
-                               shared_up_pre};
     rc = router_for_layer(x, w_router, expert_bias, T, H, E, K, route_scale, dtype, expert_ids, weights, scores,
                           expert_counts, importance, group_sizes, offsets, source_order, inverse, w.router,
                           w.router_bytes, score_func, &stats_done, &plan_done, main_stream, w.act, w.act_bytes,
@@ -693,12 +693,12 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
   }
   if (rc) return rc;
   if (!decode) {  // (the decode path has enqueued both of its GEMM launches above)
-    if (train)
-      rc = jtmoe_grouped_swiglu_train(x, source_order, gate, up, down, group_sizes, offsets, T, K, H, I, E, dtype,
-                                      gate_pre, up_pre, w.act, w.packed_y, stream);
-    else if (gather)
+    if (train || gather) {
+      const bool take = offer_shared && !shared_done && T > 0;
       rc = launch_swiglu_gather(x, source_order, gate, up, down, group_sizes, offsets, T, K, H, I, E, dtype, w.act,
-                                w.packed_y, main_stream);
+                                w.packed_y, main_stream, take ? &shared : nullptr, gate_pre, up_pre);
+      shared_done = shared_done || take;
+    }
     else
       rc = jtmoe_grouped_swiglu(w.packed_x, gate, up, down, group_sizes, offsets, T * K, H, I, E, dtype, w.act,
                                 w.packed_y, stream);

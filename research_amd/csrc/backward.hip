@@ -280,13 +280,48 @@ RouterBwdWs carve_router(void* base, int64_t T, int64_t H, int64_t E, int dtype)
   return w;
 }
 
-// steps of the routed experts up to dXp (in ws.dxp) and d_weights; dx itself is one combine away
+// The shared experts' part of the layer's backward pass.
+struct SharedBackward {
+  const void *gate, *up, *down, *gate_pre, *up_pre;
+  int64_t Is;
+  void *dx, *d_gate, *d_up, *d_down;
+  SharedBwdWs ws;
+};
+
+// dZ (with_z), the SwiGLU, the three weight gradients and dx (with_dx) of the shared experts
+int shared_backward_steps(const void* x, const void* dy, const SharedBackward& sh, int64_t T, int64_t H, int dtype,
+                          bool with_z, bool with_dx, hipStream_t s) {
+  const SharedBwdWs& ws = sh.ws;
+  const int64_t Is = sh.Is;
+  int rc = JTMOE_OK;
+  if (with_z)
+    rc = launch_gemm_nt(dtype, dy, nullptr, sh.down, nullptr, ws.dg, nullptr, nullptr, T, H, Is, 1, nullptr, 1, 0, 1, s);
+  if (rc) return rc;
+  rc = dtype == JTMOE_BF16
+           ? run_swiglu_backward<bf16_raw>(ws.dg, sh.gate_pre, sh.up_pre, nullptr, nullptr, T, Is, ws.du, ws.hw, nullptr, s)
+           : run_swiglu_backward<float>(ws.dg, sh.gate_pre, sh.up_pre, nullptr, nullptr, T, Is, ws.du, ws.hw, nullptr, s);
+  if (rc) return rc;
+  rc = launch_gemm_tn(dtype, ws.hw, dy, nullptr, sh.d_down, nullptr, nullptr, nullptr, T, Is, H, 1, nullptr, 1, false,
+                      false, 0, s, ws.split);
+  if (rc) return rc;
+  rc = launch_gemm_tn(dtype, x, ws.dg, ws.du, sh.d_gate, sh.d_up, nullptr, nullptr, T, H, Is, 1, nullptr, 1, false,
+                      false, 0, s, ws.split);
+  if (rc || !with_dx) return rc;
+  rc = launch_gemm_nt(dtype, ws.dg, ws.du, sh.gate, sh.up, sh.dx, nullptr, nullptr, T, Is, H, 1, nullptr, 1, 0, 2, s);
+  return rc ? rc : check_launch("shared backward");
+}
+
+// the steps up to dXp (in ws.dxp) and d_weights; dx of the routed experts is one combine away.  With `shared` the
+// shared experts' gradients, their dx among them, as well.
 int experts_backward_core(const void* x, const void* dy, const int32_t* source_order, const int32_t* inverse,
                           const void* weights, const int32_t* group_sizes, const int32_t* offsets, const void* gate,
                           const void* up, const void* down, const void* gate_pre, const void* up_pre, int64_t T,
                           int64_t K, int64_t H, int64_t I, int64_t E, int dtype, void* d_weights, void* d_gate,
-                          void* d_up, void* d_down, const ExpertsBwdWs& ws, hipStream_t s) {
+                          void* d_up, void* d_down, const ExpertsBwdWs& ws, hipStream_t s,
+                          const SharedBackward* shared = nullptr) {
   const int64_t A = T * K;
+  const NtProblem routed_z{ws.packed_dy, nullptr, down, nullptr, ws.dg, A, H, I};
+  const NtProblem routed_dx{ws.dg, ws.du, gate, up, ws.dxp, A, I, H};
   int rc;
   // The weight-gradient products walk the rows of a group 64 at a time; fetching those rows through
   // the permutation (64 fresh token rows every step) costs more than writing the permuted copies of
@@ -296,9 +331,20 @@ int experts_backward_core(const void* x, const void* dy, const int32_t* source_o
   launch_dispatch_rows(dy, inverse, T, K, H, dtype, ws.packed_dy, s);
   rc = check_launch("experts backward (row scatter)");
   if (rc) return rc;
+  // The shared experts' dZ and dx run in the launches of the routed ones where that is faster; what is left of their
+  // pass follows the routed one (kept apart entirely, either finds its own intermediate results in the caches).
+  NtProblem shared_z{}, shared_dx{};
+  bool joint_z = false, joint_dx = false;
+  if (shared) {
+    shared_z = {dy, nullptr, shared->down, nullptr, shared->ws.dg, T, H, shared->Is};
+    shared_dx = {shared->ws.dg, shared->ws.du, shared->gate, shared->up, shared->dx, T, shared->Is, H};
+    joint_z = gemm_nt_joint(dtype, routed_z, E, shared_z, 1) != ProductKernel::kGeneral;
+    joint_dx = gemm_nt_joint(dtype, routed_dx, E, shared_dx, 2) != ProductKernel::kGeneral;
+  }
   // Z = dYp @ Wd[e]^T
-  rc = launch_gemm_nt(dtype, ws.packed_dy, nullptr, down, nullptr, ws.dg, group_sizes, offsets, A, H, I, E, nullptr, 1,
-                      0, 1, s);
+  rc = joint_z ? launch_gemm_nt_joint(dtype, routed_z, group_sizes, offsets, E, shared_z, 1, s)
+               : launch_gemm_nt(dtype, ws.packed_dy, nullptr, down, nullptr, ws.dg, group_sizes, offsets, A, H, I, E,
+                                nullptr, 1, 0, 1, s);
   if (rc) return rc;
   rc = dtype == JTMOE_BF16 ? run_swiglu_backward<bf16_raw>(ws.dg, gate_pre, up_pre, source_order, weights, A, I, ws.du,
                                                            ws.hw, d_weights, s, group_sizes, offsets, E)
@@ -313,9 +359,19 @@ int experts_backward_core(const void* x, const void* dy, const int32_t* source_o
   rc = launch_gemm_tn(dtype, ws.packed_x, ws.dg, ws.du, d_gate, d_up, group_sizes, offsets, A, H, I, E, nullptr, 1,
                       false, false, 0, s);
   if (rc) return rc;
+  if (joint_dx) {
+    rc = shared_backward_steps(x, dy, *shared, T, H, dtype, !joint_z, false, s);
+    if (rc) return rc;
+  }
   // dXp = dG @ Wg[e]^T + dU @ Wu[e]^T
-  rc = launch_gemm_nt(dtype, ws.dg, ws.du, gate, up, ws.dxp, group_sizes, offsets, A, I, H, E, nullptr, 1, 0, 2, s);
+  rc = joint_dx ? launch_gemm_nt_joint(dtype, routed_dx, group_sizes, offsets, E, shared_dx, 2, s)
+                : launch_gemm_nt(dtype, ws.dg, ws.du, gate, up, ws.dxp, group_sizes, offsets, A, I, H, E, nullptr, 1, 0,
+                                 2, s);
   if (rc) return rc;
+  if (shared && !joint_dx) {
+    rc = shared_backward_steps(x, dy, *shared, T, H, dtype, !joint_z, true, s);
+    if (rc) return rc;
+  }
   if (A == 0) return JTMOE_OK;
   const unsigned grid = (unsigned)((A + 255) / 256);
   if (dtype == JTMOE_BF16)
@@ -325,26 +381,6 @@ int experts_backward_core(const void* x, const void* dy, const int32_t* source_o
     fill_one_kernel<float><<<grid, 256, 0, s>>>(static_cast<float*>(ws.ones), (int)A, inverse,
                                                 static_cast<float*>(d_weights));
   return check_launch("experts backward");
-}
-
-int shared_backward_impl(const void* x, const void* dy, const void* gate, const void* up, const void* down,
-                         const void* gate_pre, const void* up_pre, int64_t T, int64_t H, int64_t Is, int dtype,
-                         void* dx, void* d_gate, void* d_up, void* d_down, const SharedBwdWs& ws, hipStream_t s) {
-  int rc = launch_gemm_nt(dtype, dy, nullptr, down, nullptr, ws.dg, nullptr, nullptr, T, H, Is, 1, nullptr, 1, 0, 1, s);
-  if (rc) return rc;
-  rc = dtype == JTMOE_BF16
-           ? run_swiglu_backward<bf16_raw>(ws.dg, gate_pre, up_pre, nullptr, nullptr, T, Is, ws.du, ws.hw, nullptr, s)
-           : run_swiglu_backward<float>(ws.dg, gate_pre, up_pre, nullptr, nullptr, T, Is, ws.du, ws.hw, nullptr, s);
-  if (rc) return rc;
-  rc = launch_gemm_tn(dtype, ws.hw, dy, nullptr, d_down, nullptr, nullptr, nullptr, T, Is, H, 1, nullptr, 1, false,
-                      false, 0, s, ws.split);
-  if (rc) return rc;
-  rc = launch_gemm_tn(dtype, x, ws.dg, ws.du, d_gate, d_up, nullptr, nullptr, T, H, Is, 1, nullptr, 1, false, false, 0,
-                      s, ws.split);
-  if (rc) return rc;
-  rc = launch_gemm_nt(dtype, ws.dg, ws.du, gate, up, dx, nullptr, nullptr, T, Is, H, 1, nullptr, 1, 0, 2, s);
-  if (rc) return rc;
-  return check_launch("shared backward");
 }
 
 int router_backward_impl(const void* x, const void* router_weight, const float* scores, const int32_t* ids,
@@ -469,8 +505,8 @@ extern "C" int jtmoe_shared_backward(const void* x, const void* dy, const void* 
   if (T > 0 && (workspace == nullptr || workspace_bytes < ws.total))
     return fail(JTMOE_EWORKSPACE, "shared_backward: workspace of %zu bytes given, %zu needed", workspace_bytes,
                 ws.total);
-  return shared_backward_impl(x, dy, gate, up, down, gate_pre, up_pre, T, H, Is, dtype, dx, d_gate, d_up, d_down, ws,
-                              as_stream(stream));
+  return shared_backward_steps(x, dy, {gate, up, down, gate_pre, up_pre, Is, dx, d_gate, d_up, d_down, ws}, T, H, dtype,
+                               true, true, as_stream(stream));
 }
 
 extern "C" size_t jtmoe_router_backward_workspace_bytes(int64_t T, int64_t H, int64_t E, int dtype) {
@@ -577,14 +613,12 @@ extern "C" int jtmoe_moe_backward_sf(const void* x, const void* dy, const float*
   void* dx_sum = c.take(th);
   void* d_weights = c.take((size_t)T * K * dtype_bytes(dtype));
 
+  const SharedBackward shared{shared_gate, shared_up, shared_down, shared_gate_pre, shared_up_pre, Is, dx_shared,
+                              d_shared_gate, d_shared_up, d_shared_down, sws};
   rc = experts_backward_core(x, dy, source_order, inverse, weights, group_sizes, offsets, gate, up, down, gate_pre,
-                             up_pre, T, K, H, I, E, dtype, d_weights, d_gate, d_up, d_down, ews, s);
+                             up_pre, T, K, H, I, E, dtype, d_weights, d_gate, d_up, d_down, ews, s,
+                             Is > 0 ? &shared : nullptr);
   if (rc) return rc;
-  if (Is > 0) {
-    rc = shared_backward_impl(x, dy, shared_gate, shared_up, shared_down, shared_gate_pre, shared_up_pre, T, H, Is,
-                              dtype, dx_shared, d_shared_gate, d_shared_up, d_shared_down, sws, s);
-    if (rc) return rc;
-  }
   rc = router_backward_impl(x, router_weight, scores, expert_ids, d_weights, d_scores, route_scale, T, H, E, K, dtype,
                             dx_router, d_router_weight, rws, s, score_func);
   if (rc) return rc;

@@ -149,10 +149,13 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
 bool shared_in_skinny_tiles(const void* x, const SharedExperts& shared, int64_t T, int64_t H);
 
 // grouped_gemm.hip: the two grouped launches on packed rows fetched through the permutation (packed row j is
-// row source_order[j] / K of x), any shape and alignment as long as x is smaller than 1 GiB.
+// row source_order[j] / K of x), any shape and alignment as long as x is smaller than 1 GiB (with gate_pre / up_pre,
+// where the two rounded products are kept, any size).  With `shared` the shared experts' products of the T rows of x
+// run as well, in the same launches where that is faster.
 int launch_swiglu_gather(const void* x, const int32_t* source_order, const void* gate, const void* up,
                          const void* down, const int32_t* group_sizes, const int32_t* offsets, int64_t T, int64_t K,
-                         int64_t H, int64_t I, int64_t E, int dtype, void* act, void* packed_y, hipStream_t stream);
+                         int64_t H, int64_t I, int64_t E, int dtype, void* act, void* packed_y, hipStream_t stream,
+                         const SharedExperts* shared = nullptr, void* gate_pre = nullptr, void* up_pre = nullptr);
 
 // The decode path of the layer (a handful of tokens, nearly every expert chosen by some token).  A tile is
 // 64 rows tall whether it holds an expert's few routed rows or all T <= 64 tokens, so ONE launch runs every

@@ -243,18 +243,50 @@ inline double spread_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
 // gradients follow the same line (figures at DgradHalfCfg and DgradHalfDeepCfg); on the wrong side of it 32768
 // rows in 64 groups x 2048 -> 1408 would take 262 us against 228.
 enum class HalfTiles { kNone, kOnePerCu, kRounds };
+// what `half` half tiles take, in rounds of whole ones
+inline double half_tile_rounds(double half, double cus) {
+  const double rounds = std::floor(half / (2 * cus)), rest = half - rounds * 2 * cus;
+  return 0.12 + 0.57 * rounds + (rest <= 0.0 ? 0.0 : (rest <= cus ? 0.42 : 0.57));
+}
 inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, double cus) {
   const double half_n = (double)((N + 127) / 128), full_n = (double)((N + 255) / 256);
   if (expected_mtiles(rows, E, dense, 128) * half_n <= cus) return HalfTiles::kOnePerCu;
-  auto pays = [cus](double half, double full) {
-    const double rounds = std::floor(half / (2 * cus)), rest = half - rounds * 2 * cus;
-    const double half_cost = 0.12 + 0.57 * rounds + (rest <= 0.0 ? 0.0 : (rest <= cus ? 0.42 : 0.57));
-    return 1.15 * half_cost < std::ceil(full / cus);
-  };
+  auto pays = [cus](double half, double full) { return 1.15 * half_tile_rounds(half, cus) < std::ceil(full / cus); };
   return pays(expected_mtiles(rows, E, dense, 128) * half_n, expected_mtiles(rows, E, dense, 256) * full_n) &&
                  pays(spread_mtiles(rows, E, dense, 128) * half_n, spread_mtiles(rows, E, dense, 256) * full_n)
              ? HalfTiles::kRounds
              : HalfTiles::kNone;
+}
+
+// ---- routed and shared experts in one launch ----
+// Alone, the shared experts' products are a part of a round behind the routed ones; as more tiles of the routed
+// launch they fill its last round.  `rows` routed rows in E groups times N columns, T shared rows times N1 columns with
+// a reduction `longer` times as long (dual: gate/up, tiles 128 columns wide whatever their height).  kOnePerCu: half
+// tiles hold both products at once; kRounds: 256-row tiles; kNone: launches of their own.
+// Estimates in full rounds of routed 256-row tiles; a launch of half tiles with a CU each is one_per_cu of them times
+// its reduction (measured beside full rounds, at the power limit: shared down of 2816 at 2048 tokens 40 us, a round of
+// routed tiles of 1408 53; gate/up at 1024 tokens 41 and 57; dx of 2048 at 4096 tokens 41 and 99).  At equal
+// rounds a call gains or loses up to 3 % with few of them (less of a last round idle against a higher clock in two part-filled
+// ones) and gains up to 1 % from six on.  As for half tiles it has to pay by two estimates of how the groups spread (1300
+// tokens, 64 experts top-8: two rounds of routed tiles by one, 2.3 by the other; down jointly 3 % more a call).
+inline HalfTiles joint_tiles(int64_t rows, int64_t E, int64_t N, int64_t T, int64_t N1, double longer, double cus,
+                             double one_per_cu, bool dual = false) {
+  auto across = [dual](int64_t n, int bn) { return (double)(dual ? (n + 127) / 128 : (n + bn - 1) / bn); };
+  auto dense_tiles = [&](int bm) { return (double)((T + bm - 1) / bm) * across(N1, bm); };
+  auto alone = [&](HalfTiles h, double half, double full) {
+    if (h == HalfTiles::kOnePerCu) return one_per_cu;
+    return h == HalfTiles::kRounds && !dual ? half_tile_rounds(half, cus) : std::ceil(full / cus);
+  };
+  if (expected_mtiles(rows, E, false, 128) * across(N, 128) + dense_tiles(128) <= cus) return HalfTiles::kOnePerCu;
+  const HalfTiles routed = half_tiles(rows, E, false, N, cus);
+  const double shared = longer * alone(half_tiles(T, 1, true, N1, cus), dense_tiles(128), dense_tiles(256));
+  auto pays = [&](auto mtiles) {
+    const double full = mtiles(rows, E, false, 256) * across(N, 256), half = mtiles(rows, E, false, 128) * across(N, 128);
+    const double both = std::fmax(longer, std::ceil((full + longer * dense_tiles(256)) / cus));
+    const double apart = alone(routed, half, full) + shared;
+    return both < apart || (both == apart && both > 6.0);
+  };
+  return pays(expected_mtiles) && pays(spread_mtiles) ? HalfTiles::kRounds : HalfTiles::kNone;
 }
 
 }  // namespace jtmoe

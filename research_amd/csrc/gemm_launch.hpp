@@ -34,6 +34,22 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
 // ... and the kernel it takes for bf16 operands (16-byte aligned, below 2 GiB) on `cus` compute units
 ProductKernel data_gradient_kernel(int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense, int segs, double cus);
 
+// The routed product above and the shared experts' one (one dense group of s.rows rows) in one launch.  Operands as in
+// launch_gemm_nt, without a row map; gemm_nt_joint: the kernel, or kGeneral where launches of their own are faster or
+// the operands ask for them.
+struct NtProblem {
+  const void *a0, *a1, *b0, *b1;
+  void* c;
+  int64_t rows, Kdim, N;
+};
+ProductKernel gemm_nt_joint(int dtype, const NtProblem& p, int64_t E, const NtProblem& s, int segs);
+int launch_gemm_nt_joint(int dtype, const NtProblem& p, const int32_t* group_sizes, const int32_t* offsets, int64_t E,
+                         const NtProblem& s, int segs, hipStream_t stream);
+// ... by the sizes alone, for segs = 1 (dZ: reduction H, width I or Is) and 2 (dX: reduction I or Is, width H); kGeneral:
+// launches of their own
+ProductKernel joint_data_gradient_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t T, int64_t Is, int segs,
+                                         double cus);
+
 // C_i[e] = P[rows of group e, :]^T @ D_i[rows of group e, :]     (i = 0, and 1 if d1 is given)
 //   P: [rows, KA], D_i: [rows, N]; either may instead be [gathered_rows, .] read through row_map
 //   C_i: [E, KA, N]; an empty group yields zeros

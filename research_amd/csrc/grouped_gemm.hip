@@ -238,6 +238,46 @@ int launch_stream(const void* a, const void* b0, const void* b1, void* c, const 
   return JTMOE_OK;
 }
 
+// A routed product and the shared experts' one in the same launch.  Routed operands as in launch_fast; `dp` without its
+// tile counts.
+struct RoutedProblem {
+  const void *a, *b0, *b1;
+  void *c, *save0, *save1;
+  const int32_t *group_sizes, *offsets, *row_map;
+  int64_t rows, K, N, E, a_rows, a_group_rows;
+  int row_div;
+};
+
+DenseProblem dense_problem(const RoutedProblem& s) {
+  return {static_cast<const uint16_t*>(s.a), nullptr, static_cast<const uint16_t*>(s.b0), static_cast<const uint16_t*>(s.b1),
+          static_cast<uint16_t*>(s.c), static_cast<uint16_t*>(s.save0), static_cast<uint16_t*>(s.save1), (int)s.rows,
+          (int)s.K, (int)s.N, 0, 0};
+}
+
+template <typename Cfg>
+int launch_joint(const RoutedProblem& r, DenseProblem dp, hipStream_t stream) {
+  constexpr int kSmem = (int)StreamLayout<Cfg>::kSmemBytes;
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  auto kernel = &grouped_gemm_joint_kernel<Cfg>;
+  std::call_once(once, [&] {
+    attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
+  });
+  if (attr_err != hipSuccess)
+    return fail(JTMOE_ELAUNCH, "grouped gemm: kernel set-up: %s", hipGetErrorString(attr_err));
+  const int64_t mtiles = max_m_tiles(r.rows, r.E, Cfg::BM), nt = (r.N + Cfg::BN - 1) / Cfg::BN;
+  dp.mtiles = (dp.rows + Cfg::BM - 1) / Cfg::BM;
+  dp.ntiles = (dp.n + Cfg::BN - 1) / Cfg::BN;
+  const int64_t tiles_grid = gemm_grid(mtiles, nt) + gemm_grid(dp.mtiles, dp.ntiles);
+  if (tiles_grid >= ((int64_t)1 << 28)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: grid too large");
+  const int64_t grid = std::min<int64_t>(tiles_grid, persistent_grid_size());
+  kernel<<<(unsigned)grid, Cfg::NT, kSmem, stream>>>(
+      static_cast<const uint16_t*>(r.a), static_cast<const uint16_t*>(r.b0), static_cast<const uint16_t*>(r.b1),
+      static_cast<uint16_t*>(r.c), r.group_sizes, r.offsets, (int)r.E, (int)r.rows, (int)r.K, (int)r.N, (int)mtiles,
+      (int)nt, r.row_map, r.row_div, (int)r.a_rows, static_cast<uint16_t*>(r.save0), static_cast<uint16_t*>(r.save1), dp);
+  return JTMOE_OK;
+}
+
 // what the stream kernel needs beyond fast_ok: enough k steps to fill its pipeline, a result of at most
 // 0x7ffe0000 bytes (32-bit store offsets; the kernel drops a store by giving it the offset 0x7fff0000,
 // which must lie past the end of every admitted result) and, with a row map, fewer than 2^27 rows and a
@@ -338,6 +378,44 @@ ProductKernel down_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, bool de
   return I % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
 }
 
+inline bool streaming_or_rows64(ProductKernel k) {
+  return k == ProductKernel::kStream16x128 || k == ProductKernel::kStream16x64 || k == ProductKernel::kStream32x64 ||
+         k == ProductKernel::kRows64 || k == ProductKernel::kRows64Tail;
+}
+
+// Routed and shared experts in one launch (joint_tiles): the kernel of both, or kGeneral for launches of their own.
+// Not with routed rows in streaming tiles, which a few rows per group are too few to give up.
+// Not with the routed rows in 64-row tiles: those are resident all at once and share the memory's rate, and the shared
+// tiles, whose matrices every 64 rows read again, take their share of it (387 tokens, 64 experts top-8 of 1408, shared
+// 2816, 2048 wide: 158 us for gate/up together, 119 + 28 apart, 111 against 66 + 25 for down).
+// Measured (us, gate/up and down, routed + shared apart against joint): 2048 tokens of that model 293 + 58 and
+// 173 + 40 against 306 and 182; 2931 tokens, 1000 wide, 24 experts top-3 of 2664 and one shared, down 81 + 45
+// against 94; 4096 tokens, 1024 wide, 8 experts top-2 of 2048 and one shared, down 55 + 29 against 62.
+ProductKernel joint_gate_up(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t T, int64_t Is, double cus,
+                            const int32_t* row_map = nullptr, int row_div = 1) {
+  const ProductKernel routed = gate_up_kernel(rows, H, I, E, false, cus, row_map, row_div);
+  if (streaming_or_rows64(routed) || !stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div) ||
+      !stream_ok<GateUpStreamTailCfg>(T, H, Is, nullptr, 1))
+    return ProductKernel::kGeneral;
+  const bool tail = H % 64 != 0;
+  switch (joint_tiles(rows, E, I, T, Is, 1.0, cus, 0.72, /*dual=*/true)) {
+    case HalfTiles::kOnePerCu: return tail ? ProductKernel::kHalfTail : ProductKernel::kHalf;
+    case HalfTiles::kRounds: return tail ? ProductKernel::kRows256Tail : ProductKernel::kRows256;
+    default: return ProductKernel::kGeneral;
+  }
+}
+
+ProductKernel joint_down(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t T, int64_t Is, double cus) {
+  if (streaming_or_rows64(down_kernel(rows, H, I, E, false, cus)) ||
+      !stream_ok<DownStreamTailCfg>(rows, I, H, nullptr, 1) || !stream_ok<DownStreamTailCfg>(T, Is, H, nullptr, 1))
+    return ProductKernel::kGeneral;
+  switch (joint_tiles(rows, E, H, T, H, (double)Is / (double)I, cus, 0.4)) {
+    case HalfTiles::kOnePerCu: return ProductKernel::kHalf;
+    case HalfTiles::kRounds: return I % 64 == 0 && Is % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
+    default: return ProductKernel::kGeneral;
+  }
+}
+
 inline bool fast_ok(const void* a, const void* b0, const void* b1, const void* c, int64_t Kdim, int64_t N) {
   return Kdim % 8 == 0 && N % 8 == 0 && Kdim * N < ((int64_t)1 << 30) && aligned16(a) && aligned16(b0) && (b1 == nullptr || aligned16(b1)) &&
          aligned16(c);
@@ -372,53 +450,117 @@ int launch_down_fast(const void* act, const void* down, const int32_t* group_siz
 }
 
 template <typename T>
-int launch_pair(const void* x, const void* gate, const void* up, const void* down, const int32_t* group_sizes,
-                const int32_t* offsets, int64_t rows, int64_t H, int64_t I, int64_t E, void* act, void* y,
-                hipStream_t stream, int first_stage, const int32_t* row_map = nullptr, int row_div = 1,
-                int64_t x_rows = 0, void* save_gate = nullptr, void* save_up = nullptr) {
-  if (rows == 0) return JTMOE_OK;
-  int rc;
-  const bool dense = group_sizes == nullptr;
-  const bool gather_ok = row_map == nullptr || x_rows * H < ((int64_t)1 << 30);
-  const bool saves_ok = save_gate == nullptr || (aligned16(save_gate) && aligned16(save_up));
-#define JT_GATE_UP(LAUNCH, CFG, ...)                                                                               \
-  LAUNCH<CFG>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map, row_div, x_rows, save_gate,  \
-              save_up __VA_ARGS__)
-  if (Elem<T>::is_bf16 && fast_ok(x, gate, up, act, H, I) && gather_ok && saves_ok) {
+int launch_gate_up(const RoutedProblem& p, hipStream_t stream) {
+  const bool dense = p.group_sizes == nullptr;
+  const bool gather_ok = p.row_map == nullptr || p.a_rows * p.K < ((int64_t)1 << 30);
+  const bool saves_ok = aligned16(p.save0) && aligned16(p.save1);
+#define JT_GATE_UP(LAUNCH, CFG)                                                                                  \
+  LAUNCH<CFG>(p.a, p.b0, p.b1, p.c, p.group_sizes, p.offsets, p.rows, p.K, p.N, p.E, stream, p.row_map, p.row_div, \
+              p.a_rows, p.save0, p.save1)
+  if (Elem<T>::is_bf16 && fast_ok(p.a, p.b0, p.b1, p.c, p.K, p.N) && gather_ok && saves_ok) {
     using S11 = SkinnyCfg<1, 1, true>;
     using S12 = SkinnyCfg<1, 2, true>;
     using S22 = SkinnyCfg<2, 2, true>;
-    switch (gate_up_kernel(rows, H, I, E, dense, persistent_grid_size(), row_map, row_div)) {
-      case ProductKernel::kStream16x128: rc = JT_GATE_UP(launch_skinny, S11); break;
-      case ProductKernel::kStream16x64: rc = JT_GATE_UP(launch_skinny, S12); break;
-      case ProductKernel::kStream32x64: rc = JT_GATE_UP(launch_skinny, S22); break;
-      case ProductKernel::kRows64: rc = JT_GATE_UP(launch_fast, GateUpTinyCfg); break;
-      case ProductKernel::kRows64Tail: rc = JT_GATE_UP(launch_fast, GateUpTinyTailCfg); break;
-      case ProductKernel::kHalf: rc = JT_GATE_UP(launch_stream, GateUpHalfCfg); break;
-      case ProductKernel::kHalfTail: rc = JT_GATE_UP(launch_stream, GateUpHalfTailCfg); break;
-      case ProductKernel::kRows256: rc = JT_GATE_UP(launch_stream, GateUpStreamCfg); break;
-      case ProductKernel::kRows256Tail: rc = JT_GATE_UP(launch_stream, GateUpStreamTailCfg); break;
-      case ProductKernel::kRows256Short: rc = JT_GATE_UP(launch_fast, GateUpCfg); break;
-      default: rc = JT_GATE_UP(launch_fast, GateUpTailCfg); break;
+    switch (gate_up_kernel(p.rows, p.K, p.N, p.E, dense, persistent_grid_size(), p.row_map, p.row_div)) {
+      case ProductKernel::kStream16x128: return JT_GATE_UP(launch_skinny, S11);
+      case ProductKernel::kStream16x64: return JT_GATE_UP(launch_skinny, S12);
+      case ProductKernel::kStream32x64: return JT_GATE_UP(launch_skinny, S22);
+      case ProductKernel::kRows64: return JT_GATE_UP(launch_fast, GateUpTinyCfg);
+      case ProductKernel::kRows64Tail: return JT_GATE_UP(launch_fast, GateUpTinyTailCfg);
+      case ProductKernel::kHalf: return JT_GATE_UP(launch_stream, GateUpHalfCfg);
+      case ProductKernel::kHalfTail: return JT_GATE_UP(launch_stream, GateUpHalfTailCfg);
+      case ProductKernel::kRows256: return JT_GATE_UP(launch_stream, GateUpStreamCfg);
+      case ProductKernel::kRows256Tail: return JT_GATE_UP(launch_stream, GateUpStreamTailCfg);
+      case ProductKernel::kRows256Short: return JT_GATE_UP(launch_fast, GateUpCfg);
+      default: return JT_GATE_UP(launch_fast, GateUpTailCfg);
     }
   }
 #undef JT_GATE_UP
-  else if (!Elem<T>::is_bf16 && f32_gemm_supported(x, save_gate, gate, up, act, row_map ? x_rows : rows, H, I) &&
-           aligned16(save_up))
-    rc = launch_f32_nn(x, gate, up, act, group_sizes, offsets, rows, H, I, E, row_map, row_div, x_rows, save_gate,
-                       save_up, stream);
-  else
-    rc = launch_generic<T, true>(x, gate, up, act, group_sizes, offsets, rows, H, I, E, stream, row_map, row_div,
-                                 save_gate, save_up);
+  if (!Elem<T>::is_bf16 && f32_gemm_supported(p.a, p.save0, p.b0, p.b1, p.c, p.row_map ? p.a_rows : p.rows, p.K, p.N) &&
+      aligned16(p.save1))
+    return launch_f32_nn(p.a, p.b0, p.b1, p.c, p.group_sizes, p.offsets, p.rows, p.K, p.N, p.E, p.row_map, p.row_div,
+                         p.a_rows, p.save0, p.save1, stream);
+  return launch_generic<T, true>(p.a, p.b0, p.b1, p.c, p.group_sizes, p.offsets, p.rows, p.K, p.N, p.E, stream,
+                                 p.row_map, p.row_div, p.save0, p.save1);
+}
+
+template <typename T>
+int launch_down(const RoutedProblem& p, hipStream_t stream) {
+  if (Elem<T>::is_bf16 && fast_ok(p.a, p.b0, nullptr, p.c, p.K, p.N))
+    return launch_down_fast(p.a, p.b0, p.group_sizes, p.offsets, p.rows, p.N, p.K, p.E, p.c, stream);
+  if (!Elem<T>::is_bf16 && f32_gemm_supported(p.a, nullptr, p.b0, nullptr, p.c, p.rows, p.K, p.N))
+    return launch_f32_nn(p.a, p.b0, nullptr, p.c, p.group_sizes, p.offsets, p.rows, p.K, p.N, p.E, nullptr, 1, 0,
+                         nullptr, nullptr, stream);
+  return launch_generic<T, false>(p.a, p.b0, nullptr, p.c, p.group_sizes, p.offsets, p.rows, p.K, p.N, p.E, stream);
+}
+
+// A product of the routed experts and of the shared ones in one launch: the kernel that the rules above choose, or
+// kGeneral where they or the operands ask for launches of their own.
+ProductKernel joint_gate_up_of(const RoutedProblem& p, const RoutedProblem& s) {
+  const bool ok = (p.row_map == nullptr || p.a_rows * p.K < ((int64_t)1 << 30)) && fast_ok(p.a, p.b0, p.b1, p.c, p.K, p.N) &&
+                  fast_ok(s.a, s.b0, s.b1, s.c, s.K, s.N) && aligned16(p.save0) && aligned16(p.save1) &&
+                  aligned16(s.save0) && aligned16(s.save1);
+  return ok ? joint_gate_up(p.rows, p.K, p.N, p.E, s.rows, s.N, persistent_grid_size(), p.row_map, p.row_div)
+            : ProductKernel::kGeneral;
+}
+
+ProductKernel joint_down_of(const RoutedProblem& p, const RoutedProblem& s) {
+  const bool ok = fast_ok(p.a, p.b0, nullptr, p.c, p.K, p.N) && fast_ok(s.a, s.b0, nullptr, s.c, s.K, s.N);
+  return ok ? joint_down(p.rows, p.N, p.K, p.E, s.rows, s.K, persistent_grid_size()) : ProductKernel::kGeneral;
+}
+
+// Gate/up and down of both kinds of experts.  In launches of their own the shared pair follows the routed one, whose
+// activations are then read while the caches hold them (800 and 1300 tokens, 64 experts top-8: 1.5 % of a call).
+template <typename T>
+int launch_with_shared(const RoutedProblem& gu, const RoutedProblem& dn, const RoutedProblem& sgu,
+                       const RoutedProblem& sdn, hipStream_t stream) {
+  const ProductKernel jg = Elem<T>::is_bf16 ? joint_gate_up_of(gu, sgu) : ProductKernel::kGeneral;
+  const ProductKernel jd = Elem<T>::is_bf16 ? joint_down_of(dn, sdn) : ProductKernel::kGeneral;
+  const bool joint_gu = jg != ProductKernel::kGeneral, joint_dn = jd != ProductKernel::kGeneral;
+  const DenseProblem dgu = dense_problem(sgu), ddn = dense_problem(sdn);
+  int rc;
+  switch (jg) {
+    case ProductKernel::kGeneral: rc = launch_gate_up<T>(gu, stream); break;
+    case ProductKernel::kHalf: rc = launch_joint<GateUpHalfCfg>(gu, dgu, stream); break;
+    case ProductKernel::kHalfTail: rc = launch_joint<GateUpHalfTailCfg>(gu, dgu, stream); break;
+    case ProductKernel::kRows256: rc = launch_joint<GateUpStreamCfg>(gu, dgu, stream); break;
+    default: rc = launch_joint<GateUpStreamTailCfg>(gu, dgu, stream); break;
+  }
+  if (!rc && !joint_gu && joint_dn) rc = launch_gate_up<T>(sgu, stream);
+  if (rc) return rc;
+  switch (jd) {
+    case ProductKernel::kGeneral: rc = launch_down<T>(dn, stream); break;
+    case ProductKernel::kHalf: rc = launch_joint<DownHalfCfg>(dn, ddn, stream); break;
+    case ProductKernel::kRows256: rc = launch_joint<DownStreamCfg>(dn, ddn, stream); break;
+    default: rc = launch_joint<DownStreamTailCfg>(dn, ddn, stream); break;
+  }
+  if (!rc && !joint_gu && !joint_dn) rc = launch_gate_up<T>(sgu, stream);
+  if (!rc && !joint_dn) rc = launch_down<T>(sdn, stream);
+  return rc;
+}
+
+template <typename T>
+int launch_pair(const void* x, const void* gate, const void* up, const void* down, const int32_t* group_sizes,
+                const int32_t* offsets, int64_t rows, int64_t H, int64_t I, int64_t E, void* act, void* y,
+                hipStream_t stream, int first_stage, const int32_t* row_map = nullptr, int row_div = 1,
+                int64_t x_rows = 0, void* save_gate = nullptr, void* save_up = nullptr,
+                const SharedExperts* shared = nullptr) {
+  if (rows == 0) return JTMOE_OK;
+  const RoutedProblem gu{x, gate, up, act, save_gate, save_up, group_sizes, offsets, row_map, rows, H, I, E, x_rows, 0, row_div};
+  const RoutedProblem dn{act, down, nullptr, y, nullptr, nullptr, group_sizes, offsets, nullptr, rows, I, H, E, 0, 0, 1};
+  int rc = JTMOE_OK;
+  if (shared != nullptr) {
+    const RoutedProblem sgu{x, shared->gate, shared->up, shared->act, shared->gate_pre, shared->up_pre, nullptr, nullptr,
+                            nullptr, x_rows, H, shared->Is, 1, 0, 0, 1};
+    const RoutedProblem sdn{shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, nullptr, nullptr, nullptr,
+                            x_rows, shared->Is, H, 1, 0, 0, 1};
+    rc = launch_with_shared<T>(gu, dn, sgu, sdn, stream);
+    return rc ? rc : check_launch("grouped gemm");
+  }
+  rc = launch_gate_up<T>(gu, stream);
   if (rc) return rc;
   stage_mark(first_stage, stream);
-  if (Elem<T>::is_bf16 && fast_ok(act, down, nullptr, y, I, H))
-    rc = launch_down_fast(act, down, group_sizes, offsets, rows, H, I, E, y, stream);
-  else if (!Elem<T>::is_bf16 && f32_gemm_supported(act, nullptr, down, nullptr, y, rows, I, H))
-    rc = launch_f32_nn(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, nullptr, 1, 0, nullptr, nullptr,
-                       stream);
-  else
-    rc = launch_generic<T, false>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream);
+  rc = launch_down<T>(dn, stream);
   if (rc) return rc;
   stage_mark(first_stage + 1, stream);
   return check_launch("grouped gemm");
@@ -455,14 +597,23 @@ bool shared_in_skinny_tiles(const void* x, const SharedExperts& s, int64_t T, in
 // ---- the gathering launch pair as the layer uses it (declared in common.hpp) ----
 int launch_swiglu_gather(const void* x, const int32_t* source_order, const void* gate, const void* up,
                          const void* down, const int32_t* group_sizes, const int32_t* offsets, int64_t T, int64_t K,
-                         int64_t H, int64_t I, int64_t E, int dtype, void* act, void* packed_y, hipStream_t stream) {
-  const int rc = validate_gemm("grouped_swiglu_gather", T * K, H, I, E, dtype);
+                         int64_t H, int64_t I, int64_t E, int dtype, void* act, void* packed_y, hipStream_t stream,
+                         const SharedExperts* shared, void* gate_pre, void* up_pre) {
+  int rc = validate_gemm("grouped_swiglu_gather", T * K, H, I, E, dtype);
   if (rc) return rc;
+  if (T > 0)
+    JT_REQUIRE(x && source_order && gate && up && down && group_sizes && offsets && act && packed_y,
+               "grouped_swiglu_gather: null pointer argument");
+  if (shared != nullptr) {
+    rc = validate_gemm("shared_swiglu", T, H, shared->Is, 1, dtype);
+    if (rc) return rc;
+    JT_REQUIRE(shared->gate && shared->up && shared->down && shared->act && shared->y, "shared_swiglu: null pointer argument");
+  }
   if (dtype == JTMOE_BF16)
     return launch_pair<bf16_raw>(x, gate, up, down, group_sizes, offsets, T * K, H, I, E, act, packed_y, stream,
-                                 kStageGateUp, source_order, (int)K, T);
+                                 kStageGateUp, source_order, (int)K, T, gate_pre, up_pre, shared);
   return launch_pair<float>(x, gate, up, down, group_sizes, offsets, T * K, H, I, E, act, packed_y, stream,
-                            kStageGateUp, source_order, (int)K, T);
+                            kStageGateUp, source_order, (int)K, T, gate_pre, up_pre, shared);
 }
 
 }  // namespace jtmoe
@@ -498,11 +649,12 @@ extern "C" int jtmoe_shared_swiglu(const void* x, const void* gate, const void* 
   return launch_pair<float>(x, gate, up, down, nullptr, nullptr, T, H, Is, 1, act, shared_y, s, kStageSharedGateUp);
 }
 
-// the kernel that the rules above choose, by name
+// the kernels that the rules above choose, by name
+static const char* const kProductKernelNames[] = {"general", "stream_16x128", "stream_16x64", "stream_32x64", "rows64",
+                                                  "rows64_tail", "half", "half_tail", "half_deep", "rows256",
+                                                  "rows256_tail", "rows256_short", "rows256_short_tail"};
+
 extern "C" const char* jtmoe_product_kernel(int product, int64_t rows, int64_t K, int64_t N, int64_t E, int compute_units) {
-  static const char* const names[] = {"general", "stream_16x128", "stream_16x64", "stream_32x64", "rows64", "rows64_tail",
-                                      "half", "half_tail", "half_deep", "rows256", "rows256_tail", "rows256_short",
-                                      "rows256_short_tail"};
   const bool dense = E == 0;
   if (product < 0 || product > 3 || rows <= 0 || K <= 0 || N <= 0 || E < 0 || K >= ((int64_t)1 << 24) ||
       N >= ((int64_t)1 << 24) || rows >= ((int64_t)1 << 31) || compute_units < 0)
@@ -514,7 +666,22 @@ extern "C" const char* jtmoe_product_kernel(int product, int64_t rows, int64_t K
     k = data_gradient_kernel(rows, K, N, groups, dense, product - 1, cus);
   else if (fast_ok(nullptr, nullptr, nullptr, nullptr, K, N))
     k = product == 0 ? gate_up_kernel(rows, K, N, groups, dense, cus) : down_kernel(rows, N, K, groups, dense, cus);
-  return names[(int)k];
+  return kProductKernelNames[(int)k];
+}
+
+extern "C" const char* jtmoe_joint_kernel(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is,
+                                          int64_t E, int compute_units) {
+  const int64_t limit = (int64_t)1 << 24;
+  if (product < 0 || product > 3 || T <= 0 || top_k <= 0 || H <= 0 || I <= 0 || Is <= 0 || E <= 0 || H >= limit ||
+      I >= limit || Is >= limit || T * top_k >= ((int64_t)1 << 31) || compute_units < 0)
+    return "";
+  const double cus = compute_units > 0 ? compute_units : persistent_grid_size();
+  ProductKernel k = ProductKernel::kGeneral;
+  if (product >= 2)
+    k = joint_data_gradient_kernel(T * top_k, H, I, E, T, Is, product - 1, cus);
+  else if (fast_ok(nullptr, nullptr, nullptr, nullptr, H, I) && fast_ok(nullptr, nullptr, nullptr, nullptr, H, Is))
+    k = product == 0 ? joint_gate_up(T * top_k, H, I, E, T, Is, cus) : joint_down(T * top_k, H, I, E, T, Is, cus);
+  return k == ProductKernel::kGeneral ? "separate" : kProductKernelNames[(int)k];
 }
 
 extern "C" int jtmoe_grouped_swiglu_gather_supported(int64_t T, int64_t H, int64_t I, int dtype) {

@@ -204,6 +204,72 @@ ProductKernel data_gradient_kernel(int64_t rows, int64_t Kdim, int64_t N, int64_
   return Kdim % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
 }
 
+// 256-row tiles of the joint launch: 64-deep steps in two stages (as fast as grouped_gemm_nt_kernel there, see
+// DgradStreamCfg).  Both reductions fill its pipeline and both results stay below its limit.
+ProductKernel joint_data_gradient_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t T, int64_t Is, int segs,
+                                         double cus) {
+  const int64_t k0 = segs == 1 ? H : I, k1 = segs == 1 ? H : Is, n0 = segs == 1 ? I : H, n1 = segs == 1 ? Is : H;
+  auto steps = [segs](int64_t k) { return (k + 63) / 64 * segs; };
+  if (k0 % 8 != 0 || k1 % 8 != 0 || n0 % 8 != 0 || n1 % 8 != 0 || n0 * k0 >= kOperandLimit || n1 * k1 >= kOperandLimit ||
+      rows * n0 * 2 > (int64_t)0x7ffe0000 || T * n1 * 2 > (int64_t)0x7ffe0000 || rows * k0 >= kOperandLimit ||
+      T * k1 >= kOperandLimit)
+    return ProductKernel::kGeneral;
+  const int64_t least = std::min(steps(k0), steps(k1));
+  switch (joint_tiles(rows, E, n0, T, n1, (double)k1 / (double)k0, cus, 0.43)) {
+    case HalfTiles::kOnePerCu:
+      return least >= 2 * DgradHalfDeepCfg::NSTAGE ? ProductKernel::kHalfDeep : ProductKernel::kGeneral;
+    case HalfTiles::kRounds:
+      if (least < 2 * DgradJointCfg::NSTAGE) return ProductKernel::kGeneral;
+      return k0 % 64 == 0 && k1 % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
+    default: return ProductKernel::kGeneral;
+  }
+}
+
+namespace {
+template <typename Cfg>
+int launch_nt_joint(const NtProblem& p, const int32_t* group_sizes, const int32_t* offsets, int64_t E,
+                    const NtProblem& s, int segs, hipStream_t stream) {
+  using L = StreamLayout<Cfg>;
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  auto kernel = grouped_gemm_joint_nt_kernel<Cfg>;
+  std::call_once(once, [&] { attr_err = allow_lds(kernel, L::kSmemBytes); });
+  if (attr_err != hipSuccess)
+    return fail(JTMOE_ELAUNCH, "grouped gemm (nt): hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
+  const int64_t mtiles = max_m_tiles(p.rows, E, Cfg::BM), nt = (p.N + Cfg::BN - 1) / Cfg::BN;
+  const int64_t mt1 = (s.rows + Cfg::BM - 1) / Cfg::BM, nt1 = (s.N + Cfg::BN - 1) / Cfg::BN;
+  const int64_t tiles_grid = gemm_grid(mtiles, nt) + gemm_grid(mt1, nt1);
+  if (tiles_grid >= ((int64_t)1 << 28)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");
+  const int64_t grid = std::min<int64_t>(tiles_grid, persistent_grid_size());
+  auto in = [](const void* q) { return static_cast<const uint16_t*>(q); };
+  const DenseProblem dp{in(s.a0), in(s.a1), in(s.b0), in(s.b1), static_cast<uint16_t*>(s.c), nullptr, nullptr,
+                        (int)s.rows, (int)s.Kdim, (int)s.N, (int)mt1, (int)nt1};
+  kernel<<<(unsigned)grid, Cfg::NT, L::kSmemBytes, stream>>>(
+      in(p.a0), in(p.a1), in(p.b0), in(p.b1), static_cast<uint16_t*>(p.c), group_sizes, offsets, (int)E, (int)p.rows,
+      (int)p.Kdim, (int)p.N, (int)mtiles, (int)nt, segs, dp);
+  return JTMOE_OK;
+}
+}  // namespace
+
+ProductKernel gemm_nt_joint(int dtype, const NtProblem& p, int64_t E, const NtProblem& s, int segs) {
+  auto aligned = [segs](const NtProblem& q) {
+    return aligned16(q.a0) && aligned16(q.b0) && (segs == 1 || (aligned16(q.a1) && aligned16(q.b1))) && aligned16(q.c);
+  };
+  if (dtype != JTMOE_BF16 || p.rows <= 0 || s.rows <= 0 || !aligned(p) || !aligned(s)) return ProductKernel::kGeneral;
+  return segs == 1 ? joint_data_gradient_kernel(p.rows, p.Kdim, p.N, E, s.rows, s.N, 1, persistent_grid_size())
+                   : joint_data_gradient_kernel(p.rows, p.N, p.Kdim, E, s.rows, s.Kdim, 2, persistent_grid_size());
+}
+
+int launch_gemm_nt_joint(int dtype, const NtProblem& p, const int32_t* group_sizes, const int32_t* offsets, int64_t E,
+                         const NtProblem& s, int segs, hipStream_t stream) {
+  switch (gemm_nt_joint(dtype, p, E, s, segs)) {
+    case ProductKernel::kHalfDeep: return launch_nt_joint<DgradHalfDeepCfg>(p, group_sizes, offsets, E, s, segs, stream);
+    case ProductKernel::kRows256: return launch_nt_joint<DgradJointCfg>(p, group_sizes, offsets, E, s, segs, stream);
+    case ProductKernel::kRows256Tail: return launch_nt_joint<DgradJointTailCfg>(p, group_sizes, offsets, E, s, segs, stream);
+    default: return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): no joint launch at this size");
+  }
+}
+
 int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, const void* b1, void* c,
                    const int32_t* group_sizes, const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N,
                    int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream) {

@@ -46,18 +46,47 @@ struct StreamLayout {
   static_assert(Cfg::BM <= Cfg::NT, "one row-map entry per thread");
 };
 
+// A second product in the same launch: one dense group with its own matrices, width and reduction length, as the
+// shared experts are beside the routed ones.
+struct DenseProblem {
+  const uint16_t *a0, *a1, *b0, *b1;  // a1 / b1: the up matrix or the second segment
+  uint16_t *c, *save0, *save1;
+  int rows, k, n, mtiles, ntiles;
+};
+
+// How the workgroups of an XCD share out the tiles of two products (kJoint): the dense product's tiles first, dealt
+// round, then the grouped product's, of which the workgroups without the last round of dense tiles take `lead` rounds
+// more than the others -- as many grouped tiles as last as long as one dense tile.  Workgroup w of W takes in place p
+// (p = 0, 1, ...) the tile with the returned index among n1 dense tiles followed by n0 grouped ones, or -1 at its end.
+// Every index from 0 to n0 + n1 - 1 is returned exactly once.
+__host__ __device__ inline int joint_tile(int w, int W, int p, int n1, int n0, int lead) {
+  const int full = n1 / W, longer = n1 - full * W;  // `longer` workgroups have one dense tile more
+  const int mine = full + (w < longer ? 1 : 0);
+  if (p < mine) return p * W + w;
+  const int q = p - mine, rest = W - longer;
+  int i;
+  if (longer == 0)
+    i = q * W + w;
+  else if (w < longer)
+    i = lead * rest + q * W + w;
+  else
+    i = q < lead ? q * rest + (w - longer) : lead * rest + (q - lead) * W + w;
+  return i < n0 ? n1 + i : -1;
+}
+
 // kNT = false: C = A @ B[e] with B[e] stored [K, N] (the forward products; kDual: two of them sharing the A tile).
 // kNT = true:  C = sum over segs segments of A_s @ B_s[e]^T with B_s[e] stored [N, K] (the data gradients of
 //              the backward pass, grouped_gemm_bwd.hpp): the B tile is then k-contiguous like the A tile,
 //              lives in LDS in the same swizzled row layout and is read with ds_read_b128; the k loop
 //              runs through the segments one after the other.
-template <typename Cfg, bool kNT>
+// kJoint: the tiles of `dp` run in the same launch (fully persistent workgroups, chunk 0).
+template <typename Cfg, bool kNT, bool kJoint = false>
 __device__ __forceinline__ void stream_gemm_body(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes,
     const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n,
     const int32_t* __restrict__ row_map, int row_div, int a_rows, uint16_t* __restrict__ save0,
-    uint16_t* __restrict__ save1, int segs, int window, int chunk) {
+    uint16_t* __restrict__ save1, int segs, int window, int chunk, const DenseProblem& dp) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, NS = Cfg::NSTAGE;
   constexpr int TM = Cfg::TM, TN = Cfg::TN, WM = Cfg::WM, WN = Cfg::WN;
   constexpr int CPRA = Cfg::CPRA, KK = BK / 16, LPS = Cfg::LPS;
@@ -82,8 +111,8 @@ __device__ __forceinline__ void stream_gemm_body(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WAVES_N, wn = wave - wm * Cfg::WAVES_N;
   const bool gather = row_map != nullptr;
-  const int nk1 = kTail ? (Kdim + BK - 1) / BK : Kdim / BK;  // k steps of one segment
-  const int nk = kNT ? nk1 * segs : nk1;   // k steps of a tile
+  auto seg_steps = [](int k) { return kTail ? (k + BK - 1) / BK : k / BK; };  // k steps of one segment
+  const int nk_segs = kNT ? segs : 1;
 
   // ---- schedule (as in grouped_gemm_dma_persistent_kernel) ----
   // Group sizes and first rows are copied into LDS once; every tile look-up scans them from there, so
@@ -103,6 +132,12 @@ __device__ __forceinline__ void stream_gemm_body(
   const int per_xcd = (total + 7) >> 3;
   const int xcd = (int)blockIdx.x & 7;
   int idx = (int)blockIdx.x >> 3, stride = max(1, (int)gridDim.x >> 3), left = 0x7fffffff;
+  // kJoint: this XCD's range of either product, the odd tiles of the two at opposite ends of the XCDs
+  const int total1 = kJoint ? dp.mtiles * dp.ntiles : 0;
+  const int first0 = (xcd * total) >> 3, count0 = (((xcd + 1) * total) >> 3) - first0;
+  const int first1 = (xcd * total1 + 7) >> 3, count1 = (((xcd + 1) * total1 + 7) >> 3) - first1;
+  const int lead = kJoint ? max(1, (2 * dp.k + Kdim) / (2 * Kdim)) : 0;
+  int place = 0;  // kJoint: how many tiles this workgroup has looked up
   if (chunk > 0) {
     idx = (idx / window) * (window * chunk) + idx % window;
     stride = window;
@@ -110,20 +145,34 @@ __device__ __forceinline__ void stream_gemm_body(
   }
 
   struct Tile {
-    int expert, row0, rows, n0;
+    int expert, row0, rows, n0;  // expert < 0: a tile of `dp`
   };
   auto locate = [&](int i) -> Tile {
     Tile t;
     t.expert = 0; t.row0 = 0; t.rows = 0; t.n0 = 0;
-    const int logical = xcd * per_xcd + i;
-    if (i >= per_xcd || logical >= total) return t;
-    const int group_span = Cfg::GROUP_M * ntiles_n;
+    bool second = false;
+    int logical = xcd * per_xcd + i, mts = real_mtiles, nts = ntiles_n;
+    if constexpr (kJoint) {
+      const int j = joint_tile(idx, stride, place++, count1, count0, lead);
+      if (j < 0) return t;
+      second = j < count1;
+      logical = second ? first1 + j : first0 + (j - count1);
+      mts = second ? dp.mtiles : real_mtiles;
+      nts = second ? dp.ntiles : ntiles_n;
+    } else if (i >= per_xcd || logical >= total) {
+      return t;
+    }
+    const int group_span = Cfg::GROUP_M * nts;
     const int group = logical / group_span;
     const int in_group = logical - group * group_span;
-    const int gm = min(Cfg::GROUP_M, real_mtiles - group * Cfg::GROUP_M);
+    const int gm = min(Cfg::GROUP_M, mts - group * Cfg::GROUP_M);
     const int nt = in_group / gm;
     const int mt = group * Cfg::GROUP_M + (in_group - nt * gm);
-    if (group_sizes) {
+    if (second) {
+      t.expert = -1;
+      t.row0 = mt * BM;
+      t.rows = min(BM, dp.rows - mt * BM);
+    } else if (group_sizes) {
       const TileRows tr = locate_tile(group_scan(BM, gs_l, JTMOE_MAX_EXPERTS), mt, BM, row0_l);
       t.expert = __builtin_amdgcn_readfirstlane(tr.expert);
       t.row0 = __builtin_amdgcn_readfirstlane(tr.row0);
@@ -148,7 +197,12 @@ __device__ __forceinline__ void stream_gemm_body(
     i32x4_t b_rsrc[NBD];
     int a_voff[Cfg::A_LOADS];
     int b_voff[B_LOADS];
+    int k, n, nk1;  // of the tile's product (constants of the launch unless kJoint)
   };
+  // the tile's product, seen from the tile
+  auto second_product = [](const Tile& t) { return kJoint && t.expert < 0; };
+  auto tile_k = [&](const Tile& t) { return second_product(t) ? dp.k : Kdim; };
+  auto tile_n = [&](const Tile& t) { return second_product(t) ? dp.n : N; };
   const int a_r = tid / CPRA, a_slot = tid - a_r * CPRA;
   const int a_c = a_slot ^ ((a_r / (16 / CPRA)) % CPRA);
   const int b_blk_id = tid >> 5;
@@ -160,27 +214,33 @@ __device__ __forceinline__ void stream_gemm_body(
 
   // everything of a plan but the A row offsets
   auto plan_tile = [&](Plan& p, const Tile& t) {
-    const size_t wofs = (size_t)t.expert * Kdim * N;
+    const bool second = second_product(t), gathered = gather && !second;
+    p.k = tile_k(t);
+    p.n = tile_n(t);
+    p.nk1 = seg_steps(p.k);
+    const size_t wofs = second ? 0 : (size_t)t.expert * Kdim * N;
+    const uint16_t *a0 = second ? dp.a0 : A, *b0 = second ? dp.b0 : B0, *b1 = second ? dp.b1 : B1;
     if constexpr (kNT) {
+      const uint16_t* a1 = second ? dp.a1 : A1;
 #pragma unroll
       for (int sg = 0; sg < 2; ++sg) {
-        const uint16_t* a = (sg == 1 && segs > 1) ? A1 : A;
-        const uint16_t* b = (sg == 1 && segs > 1) ? B1 : B0;
-        p.a_rsrc[sg] = gather ? make_rsrc(a, a_rows * Kdim * 2) : make_rsrc(a + (size_t)t.row0 * Kdim, t.rows * Kdim * 2);
-        p.b_rsrc[sg] = make_rsrc(b + wofs, N * Kdim * 2);  // rows of B past N lie outside it and read as zeros
+        const uint16_t* a = (sg == 1 && segs > 1) ? a1 : a0;
+        const uint16_t* b = (sg == 1 && segs > 1) ? b1 : b0;
+        p.a_rsrc[sg] = gathered ? make_rsrc(a, a_rows * Kdim * 2) : make_rsrc(a + (size_t)t.row0 * p.k, t.rows * p.k * 2);
+        p.b_rsrc[sg] = make_rsrc(b + wofs, p.n * p.k * 2);  // rows of B past N lie outside it and read as zeros
       }
       // the B tile's rows are output columns: row n0 + r of B[e], the same slots and swizzle as the A tile
 #pragma unroll
-      for (int j = 0; j < B_LOADS; ++j) p.b_voff[j] = ((t.n0 + a_r + j * (NT / CPRA)) * Kdim + a_c * 8) * 2;
+      for (int j = 0; j < B_LOADS; ++j) p.b_voff[j] = ((t.n0 + a_r + j * (NT / CPRA)) * p.k + a_c * 8) * 2;
     } else {
 #pragma unroll
-      for (int u = 0; u < Cfg::NSUB; ++u) p.b_rsrc[u] = make_rsrc((kDual && u == 1 ? B1 : B0) + wofs, Kdim * N * 2);
-      p.a_rsrc[0] = gather ? make_rsrc(A, a_rows * Kdim * 2) : make_rsrc(A + (size_t)t.row0 * Kdim, t.rows * Kdim * 2);
+      for (int u = 0; u < Cfg::NSUB; ++u) p.b_rsrc[u] = make_rsrc((kDual && u == 1 ? b1 : b0) + wofs, p.k * p.n * 2);
+      p.a_rsrc[0] = gathered ? make_rsrc(a0, a_rows * Kdim * 2) : make_rsrc(a0 + (size_t)t.row0 * p.k, t.rows * p.k * 2);
 #pragma unroll
-      for (int u = 0; u < Cfg::NSUB; ++u) p.b_voff[u] = (b_k * N + t.n0 + (kDual ? 0 : u * 128) + b_c * 8) * 2;
+      for (int u = 0; u < Cfg::NSUB; ++u) p.b_voff[u] = (b_k * p.n + t.n0 + (kDual ? 0 : u * 128) + b_c * 8) * 2;
     }
 #pragma unroll
-    for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = ((a_r + j * (NT / CPRA)) * Kdim + a_c * 8) * 2;
+    for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = ((a_r + j * (NT / CPRA)) * p.k + a_c * 8) * 2;
   };
   // gathered rows: the offsets come from row ids (rows past the end of the group read as zeros)
   // row_map entries are divided by row_div (the top-k of the routing) with a multiply: for
@@ -199,9 +259,9 @@ __device__ __forceinline__ void stream_gemm_body(
   auto issue_one = [&](const Plan& p, int kt, int stage, int i) {
     const unsigned base = wave_lds + stage * Cfg::STAGE_BYTES;
     if constexpr (kNT) {
-      const bool second = kt >= nk1;  // uniform: the step belongs to the second segment
-      const int k0 = (second ? kt - nk1 : kt) * BK;
-      const bool outside = kTail && k0 + a_c * 8 >= Kdim;  // both tiles: this lane's chunk lies past the end of the row
+      const bool second = kt >= p.nk1;  // uniform: the step belongs to the second segment
+      const int k0 = (second ? kt - p.nk1 : kt) * BK;
+      const bool outside = kTail && k0 + a_c * 8 >= p.k;  // both tiles: this lane's chunk lies past the end of the row
       if (i < Cfg::A_LOADS)
         buffer_load_lds16(second ? p.a_rsrc[1] : p.a_rsrc[0], base + i * NT * 16, outside ? kOutside : p.a_voff[i],
                           k0 * 2);
@@ -211,12 +271,12 @@ __device__ __forceinline__ void stream_gemm_body(
     } else {
       const int k0 = kt * BK;
       if (i < Cfg::A_LOADS) {
-        buffer_load_lds16(p.a_rsrc[0], base + i * NT * 16, kTail && k0 + a_c * 8 >= Kdim ? kOutside : p.a_voff[i],
+        buffer_load_lds16(p.a_rsrc[0], base + i * NT * 16, kTail && k0 + a_c * 8 >= p.k ? kOutside : p.a_voff[i],
                           k0 * 2);
       } else {
         const int u = (i - Cfg::A_LOADS) / Cfg::BSUB_LOADS, jb = (i - Cfg::A_LOADS) % Cfg::BSUB_LOADS;
         buffer_load_lds16(p.b_rsrc[u], base + Cfg::A_BYTES + u * Cfg::BSUB_BYTES + jb * NT * 16,
-                          p.b_voff[u] + jb * (NT / 16) * N * 2 + (kTail ? k0 * N * 2 : 0), kTail ? 0 : k0 * N * 2);
+                          p.b_voff[u] + jb * (NT / 16) * p.n * 2 + (kTail ? k0 * p.n * 2 : 0), kTail ? 0 : k0 * p.n * 2);
       }
     }
   };
@@ -276,7 +336,8 @@ __device__ __forceinline__ void stream_gemm_body(
   Plan pl;
   plan_tile(pl, cur);
   // (a partial tile's rows past the group end are not read: the map may end with the group)
-  if (gather) plan_rows(pl, cur, [&](int r) { return r < cur.rows ? row_map[cur.row0 + r] : 0; });
+  if (gather && !second_product(cur)) plan_rows(pl, cur, [&](int r) { return r < cur.rows ? row_map[cur.row0 + r] : 0; });
+  int nk = pl.nk1 * nk_segs;  // k steps of the current tile
 #pragma unroll
   for (int s = 0; s < NS; ++s) issue(pl, s, s);
   f32x16_t acc[TM][TN];
@@ -287,16 +348,18 @@ __device__ __forceinline__ void stream_gemm_body(
   int cs = 0;  // stage of the current k step
 
   while (true) {
-    const bool wave_has_rows = wm * WM < cur.rows && cur.n0 + wn * Cfg::WNO < N;
-    idx += stride;
+    const int cur_n = tile_n(cur);
+    const bool wave_has_rows = wm * WM < cur.rows && cur.n0 + wn * Cfg::WNO < cur_n;
+    if constexpr (!kJoint) idx += stride;
     --left;
     const Tile nxt = locate(left > 0 ? idx : 0x3fffffff);
     const bool have_next = nxt.rows > 0;
+    const int nk_next = kJoint ? seg_steps(tile_k(nxt)) * nk_segs : nk;
 
     // row ids of the next tile: one LDS-DMA dword per thread, requested now and read NS steps before
     // this tile ends (it is older than every operand load issued from here on, so the waits below
     // cover it)
-    if (gather && have_next) {
+    if (gather && have_next && !second_product(nxt)) {
       const i32x4_t map_rsrc = make_rsrc(row_map + nxt.row0, nxt.rows * 4);
       buffer_load_lds4(map_rsrc, lds0 + L::kRowBufBase + wave * 256, lane * 4 + wave * 256);
     }
@@ -387,7 +450,7 @@ __device__ __forceinline__ void stream_gemm_body(
       if (wave_has_rows) leading_substeps(std::false_type{});
       // k steps of this workgroup's stream after this one (only the next tile counts: a load is
       // never issued more than NS <= nk steps ahead)
-      const int rem = (nk - 1 - j) + (have_next ? nk : 0);
+      const int rem = (nk - 1 - j) + (have_next ? nk_next : 0);
       if (rem > 0) {
         if (rem >= NS - 1)
           wait_and_barrier<(NS - 2) * LPS>();
@@ -399,7 +462,7 @@ __device__ __forceinline__ void stream_gemm_body(
           const int kt = j + NS - nk;  // a step of the next tile
           if (kt == 0) {               // from here on the plan is the next tile's
             plan_tile(pl, nxt);
-            if (gather) plan_rows(pl, nxt, [&](int r) { return rowbuf[r]; });
+            if (gather && !second_product(nxt)) plan_rows(pl, nxt, [&](int r) { return rowbuf[r]; });
           }
           issue(pl, kt, cs);
         }
@@ -412,9 +475,12 @@ __device__ __forceinline__ void stream_gemm_body(
     }
 
     // ---- epilogue: straight from the accumulators to memory (no LDS, no barrier) ----
-    store_transposed_accumulators<Cfg>(acc, wm, wn, cur.row0, cur.rows, cur.n0, N, dense_rows, C, save0, save1);
+    const bool second = second_product(cur);
+    store_transposed_accumulators<Cfg>(acc, wm, wn, cur.row0, cur.rows, cur.n0, cur_n, second ? dp.rows : dense_rows,
+                                       second ? dp.c : C, second ? dp.save0 : save0, second ? dp.save1 : save1);
     if (!have_next) break;
     cur = nxt;
+    nk = nk_next;
   }
 }
 
@@ -425,7 +491,19 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_kernel(
     int dense_rows, int Kdim, int N, int mtiles, int ntiles_n, const int32_t* __restrict__ row_map, int row_div,
     int a_rows, uint16_t* __restrict__ save0, uint16_t* __restrict__ save1, int window, int chunk) {
   stream_gemm_body<Cfg, false>(A, nullptr, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, mtiles, ntiles_n,
-                               row_map, row_div, a_rows, save0, save1, 1, window, chunk);
+                               row_map, row_div, a_rows, save0, save1, 1, window, chunk, DenseProblem{});
+}
+
+// A grouped and a dense product in one launch of persistent workgroups (a multiple of 8, chunk 0).  The requirements
+// above hold for both.
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) void grouped_gemm_joint_kernel(
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
+    uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E,
+    int dense_rows, int Kdim, int N, int mtiles, int ntiles_n, const int32_t* __restrict__ row_map, int row_div,
+    int a_rows, uint16_t* __restrict__ save0, uint16_t* __restrict__ save1, DenseProblem dp) {
+  stream_gemm_body<Cfg, false, true>(A, nullptr, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, mtiles,
+                                     ntiles_n, row_map, row_div, a_rows, save0, save1, 1, 0, 0, dp);
 }
 
 // The transposed-B form: the arguments of grouped_gemm_nt_kernel (grouped_gemm_bwd.hpp) plus the schedule.
@@ -437,7 +515,17 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_nt_kernel(
     const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n,
     const int32_t* __restrict__ row_map, int row_div, int a_rows, int segs, int window, int chunk) {
   stream_gemm_body<Cfg, true>(A0, A1, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, mtiles, ntiles_n,
-                              row_map, row_div, a_rows, nullptr, nullptr, segs, window, chunk);
+                              row_map, row_div, a_rows, nullptr, nullptr, segs, window, chunk, DenseProblem{});
+}
+
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) void grouped_gemm_joint_nt_kernel(
+    const uint16_t* __restrict__ A0, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
+    const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes,
+    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n, int segs,
+    DenseProblem dp) {
+  stream_gemm_body<Cfg, true, true>(A0, A1, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, mtiles, ntiles_n,
+                                    nullptr, 1, 0, nullptr, nullptr, segs, 0, 0, dp);
 }
 
 // The configuration the library launches for gate/up (routed and shared experts): the tile of GateUpCfg
@@ -459,11 +547,15 @@ using DownHalfDeepCfg = DmaGemmCfg<128, 128, 64, 2, 2, false, 2, 16 + 128 + 6553
 // the library keeps for that launch, at 12, 22 and 44 k steps per tile).
 using GateUpStream2Cfg = DmaGemmCfg<256, 128, 64, 4, 2, true, 2, 16 + 128>;
 using DownStreamCfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768>;
+using DownStreamTailCfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + 65536>;
 using DownStream2Cfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 32768>;
 // The data-gradient products of the backward pass (transposed-B form): 256 x 256 tiles, 2 x 4 waves.
 // Checked and timed by the stand-alone check (time_stream_nt) against grouped_gemm_nt_kernel, which
 // the library launches: the transposed-B form measures equal or slower there.
 using DgradStreamCfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128>;
+// The 256-row tiles of the joint launch of routed and shared data gradients.
+using DgradJointCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128>;
+using DgradJointTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 65536>;
 // The same in half tiles, launched where a data gradient has at most one of them per CU: nothing else runs on the CU,
 // so four 64-deep stages (131 KB) keep its loads going.  4096 rows x 4096 -> 1024: 40 us, two 64-deep stages with
 // two workgroups per CU 59, four 32-deep ones 49, 256 x 256 tiles 93; 2048 rows x 5632 -> 2048: 55, 79, 67 and 124.

@@ -21,3 +21,10 @@ def gradient_kernels(rows, hidden, inter, experts=0, cus=0):
     """Those of dZ = dY Wd^T and of dX = dG Wg^T + dU Wu^T."""
     return (chosen(DATA_GRADIENT, rows, hidden, inter, experts, cus),
             chosen(DATA_GRADIENT_PAIR, rows, inter, hidden, experts, cus))
+
+
+def joint_kernels(tokens, top_k, hidden, inter, shared, experts, cus=0):
+    """Those of gate/up, down, dZ and dX of routed and shared experts in one launch ("separate": in two)."""
+    joint = _ffi.load_library().jtmoe_joint_kernel
+    return [joint(product, tokens, top_k, hidden, inter, shared, experts, cus).decode()
+            for product in (GATE_UP, DOWN, DATA_GRADIENT, DATA_GRADIENT_PAIR)]

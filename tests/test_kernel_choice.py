@@ -8,10 +8,11 @@ from __future__ import annotations
 
 import pytest
 
+import test_gpu_joint_products as joint
 import test_gpu_ragged_widths as ragged
 import test_gpu_row_bits as row_bits
 import test_gpu_tile_choice as tiles
-from kernel_choice import DOWN, GATE_UP, MI355X_CUS, chosen, forward_kernels, gradient_kernels
+from kernel_choice import DOWN, GATE_UP, MI355X_CUS, chosen, forward_kernels, gradient_kernels, joint_kernels
 
 GATE_UP_KERNELS = {"stream_16x128", "stream_16x64", "stream_32x64", "rows64", "rows64_tail", "half", "half_tail", "rows256",
                    "rows256_tail", "rows256_short", "rows256_short_tail"}
@@ -55,6 +56,20 @@ def test_every_kernel_is_held_to_the_bits_of_the_others():
                 seen.update(zip((GATE_UP, DOWN), forward_kernels(rows * experts, hidden, inter, experts, MI355X_CUS)))
     assert {kernel for product, kernel in seen if product == GATE_UP} >= GATE_UP_KERNELS - {"rows256_short"}
     assert {kernel for product, kernel in seen if product == DOWN} >= DOWN_KERNELS
+
+
+JOINT_KERNELS = ({"separate", "half", "half_tail", "rows256", "rows256_tail"}, {"separate", "half", "rows256", "rows256_tail"},
+                 {"separate", "half_deep", "rows256", "rows256_tail"}, {"separate", "half_deep", "rows256", "rows256_tail"})
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,top_k,inter,shared,kernels", joint.SHAPES)
+def test_joint_shapes_take_the_kernels_they_name(tokens, hidden, experts, top_k, inter, shared, kernels):
+    assert " ".join(joint_kernels(tokens, top_k, hidden, inter, shared, experts, MI355X_CUS)) == kernels
+
+
+def test_every_joint_kernel_is_held_to_separate_launches():
+    for product, names in enumerate(zip(*(case[6].split() for case in joint.SHAPES))):
+        assert set(names) == JOINT_KERNELS[product]
 
 
 def test_sizes_out_of_range_have_no_kernel():
