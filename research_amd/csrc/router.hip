@@ -150,6 +150,18 @@ __device__ __forceinline__ int order_key(float v) {
   return v != v ? kNanKey : bits ^ ((bits >> 31) & 0x7fffffff);
 }
 
+// The largest of a row of sixteen lanes, in all of them.
+__device__ __forceinline__ int row_max_i32(int v) {
+  int o = quad_xor_i32<1>(v);
+  v = o > v ? o : v;
+  o = quad_xor_i32<2>(v);
+  v = o > v ? o : v;
+  o = __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true);  // row_half_mirror: lane i of 8 from lane 7 - i
+  v = o > v ? o : v;
+  o = __builtin_amdgcn_mov_dpp(v, 0x140, 0xf, 0xf, true);  // row_mirror: lane i of 16 from lane 15 - i
+  return o > v ? o : v;
+}
+
 // K rounds of "largest remaining score + bias, lower index on ties" for one token, by its four
 // lanes: lane q owns experts [e_begin, e_begin + EQ) and keeps their keys in registers; a taken
 // expert's key becomes kTakenKey, below every real value.  A round: the largest key of the token (a run
@@ -192,47 +204,88 @@ __device__ __forceinline__ void select_from_registers(const RouterSmem& sm, cons
   }
 }
 
-// The same selection (same keys, same comparisons) for any expert count: the lane re-reads its quarter
-// from LDS in every round.
-__device__ __forceinline__ void select_from_lds(const RouterSmem& sm, const float* row, int e_begin, int eq, int E,
-                                                bool row_ok, int t, int q, int K) {
+// The same selection (same keys, same comparisons) by sixteen lanes to a token, for any expert count: lane l owns experts
+// [EQ l, EQ l + EQ).  A round: the largest key (in the lane, then four exchanges in the row of lanes), the lowest lane
+// that holds it (a ballot), which writes the lowest of its experts with that key and retires it.
+template <int EQ>
+__device__ __forceinline__ void select_by_rows(const RouterSmem& sm, int t, bool row_ok, int E, int K) {
 #pragma clang fp contract(off)
-  unsigned long long taken = 0ull;
-  for (int r = 0; r < K; ++r) {
-    int best_k = kTakenKey, best_e = -1;
-    if (row_ok) {
-      for (int j = 0; j < eq; ++j) {
-        const int e = e_begin + j;
-        if (e < E && !((taken >> j) & 1ull)) {
-          const int k = order_key(row[e] + sm.bias[e]);
-          if (k > best_k) {  // strictly: the lower index keeps a tie
-            best_k = k;
-            best_e = e;
-          }
-        }
-      }
-    }
+  const int l = threadIdx.x & 15;
+  const unsigned row_shift = threadIdx.x & 48;
+  const float* const row = sm.tile + t * (E + 1) + l * EQ;
+  int key[EQ];
 #pragma unroll
-    for (int m = 1; m <= 2; m <<= 1) {
-      const int ok = __shfl_xor(best_k, m, 4);
-      const int oe = __shfl_xor(best_e, m, 4);
-      const bool take = oe >= 0 && (best_e < 0 || ok > best_k || (ok == best_k && oe < best_e));
-      if (take) {
-        best_k = ok;
-        best_e = oe;
-      }
+  for (int j = 0; j < EQ; ++j) key[j] = row_ok && l * EQ + j < E ? order_key(row[j] + sm.bias[l * EQ + j]) : kTakenKey;
+  for (int r = 0; r < K; ++r) {
+    int best = key[0];
+#pragma unroll
+    for (int j = 1; j < EQ; ++j) best = key[j] > best ? key[j] : best;
+    best = row_max_i32(best);
+    int own = EQ;
+#pragma unroll
+    for (int j = EQ - 1; j >= 0; --j) own = key[j] == best ? j : own;
+    const unsigned holders = (unsigned)(__ballot(own < EQ) >> row_shift) & 0xffffu;
+    const bool mine = (holders & (0u - holders)) == (1u << l);
+#pragma unroll
+    for (int j = 0; j < EQ; ++j) key[j] = mine && j == own ? kTakenKey : key[j];
+    if (mine && row_ok) sm.top_id[t * K + r] = l * EQ + own;
+  }
+}
+
+// A round is bound by its dependent steps, whose number grows with the experts of a lane (four lanes to a token: eight
+// rounds of 64 experts 5.1 us, of 128 9.6), so sixteen lanes take a token where a workgroup has them to spare.  Finishing
+// workgroup of 1024 threads: 37 tokens, 128 experts 20.3 -> 13.0 us, 14 tokens, 64 experts 13.2 -> 9.4; of 256 threads
+// and 16 tokens: 17.5 -> 12.3 and 12.0 -> 9.0 (the sigmoid without a pass of its own among it, see add_slices).  Four
+// passes cost what one of four lanes does where waves fill each other's latency (1024 threads, 200 tokens: 28.5 and
+// 28.2) and more with a wave per SIMD (64-token workgroups 31.0 against 33.6 us), which therefore keep four lanes from
+// three passes on.
+template <int kRouterTokens, int kRouterThreads>
+__device__ __forceinline__ void select_all(const RouterSmem& sm, int nrows, int E, int K) {
+  constexpr int kGroups = kRouterThreads / 16;
+  static_assert(4 * kRouterTokens <= kRouterThreads, "four lanes to a token");
+  const int tid = threadIdx.x;
+  if (kRouterTokens > 2 * kGroups && kRouterThreads < 1024 && nrows > 2 * kGroups &&
+      (E == 16 || E == 32 || E == 64 || E == 128 || E == 256)) {
+    const int t = tid >> 2, q = tid & 3, e_begin = q * (E >> 2);
+    const bool row_ok = t < nrows;
+    const float* const row = sm.tile + t * (E + 1);
+    switch (E) {
+      case 16: select_from_registers<4>(sm, row, e_begin, row_ok, t, q, K); break;
+      case 32: select_from_registers<8>(sm, row, e_begin, row_ok, t, q, K); break;
+      case 64: select_from_registers<16>(sm, row, e_begin, row_ok, t, q, K); break;
+      case 128: select_from_registers<32>(sm, row, e_begin, row_ok, t, q, K); break;
+      default: select_from_registers<64>(sm, row, e_begin, row_ok, t, q, K); break;
     }
-    if (row_ok) {
-      const int j = best_e - e_begin;
-      if (j >= 0 && j < eq) taken |= 1ull << j;
-      if (q == 0) sm.top_id[t * K + r] = best_e;
-    }
+    return;
+  }
+  for (int t0 = 0; t0 < nrows; t0 += kGroups) {
+    const int t = t0 + (tid >> 4);
+    const bool row_ok = t < nrows;
+    if (E <= 16)
+      select_by_rows<1>(sm, t, row_ok, E, K);
+    else if (E <= 32)
+      select_by_rows<2>(sm, t, row_ok, E, K);
+    else if (E <= 64)
+      select_by_rows<4>(sm, t, row_ok, E, K);
+    else if (E <= 128)
+      select_by_rows<8>(sm, t, row_ok, E, K);
+    else
+      select_by_rows<16>(sm, t, row_ok, E, K);
+  }
+}
+
+__device__ __forceinline__ void router_clear(const RouterSmem& sm, const float* __restrict__ bias, int E, int threads) {
+  for (int e = threadIdx.x; e < E; e += threads) {
+    sm.bias[e] = bias ? bias[e] : 0.0f;
+    sm.cnt[e] = 0;
+    sm.imp[e] = 0ull;
   }
 }
 
 // Everything after the logits tile is in LDS.  `T` is the output element type of
-// the weights.
-template <typename T, int kRouterTokens, int kRouterThreads>
+// the weights.  kSummed: behind router_clear and add_slices, which has written the logits (and, for the sigmoid, turned
+// the tile into scores and written these).
+template <typename T, int kRouterTokens, int kRouterThreads, bool kSummed = false>
 __device__ void router_epilogue(const RouterSmem& sm, const float* __restrict__ bias_g, int t0, int tokens,
                                 int E, int K, float route_scale, int32_t* __restrict__ ids_out,
                                 T* __restrict__ weights_out, float* __restrict__ scores_out,
@@ -245,17 +298,13 @@ __device__ void router_epilogue(const RouterSmem& sm, const float* __restrict__ 
   const int nrows = min(kRouterTokens, tokens - t0);
   const bool softmax = score_func == JTMOE_SCORE_SOFTMAX;
 
-  for (int e = tid; e < E; e += kRouterThreads) {
-    sm.bias[e] = bias_g ? bias_g[e] : 0.0f;
-    sm.cnt[e] = 0;
-    sm.imp[e] = 0ull;
-  }
+  if (!kSummed) router_clear(sm, bias_g, E, kRouterThreads);
   if (softmax) {
     // Softmax over the experts of every token, in place, by the token's four lanes (lane q owns the
     // run of ceil(E/4) consecutive experts that it owns in the selection below):
     // m = max z;  p_e = exp(max(z_e - m, -86));  the four run sums, each added in index order, are
     // combined as (s0 + s1) + (s2 + s3);  score_e = p_e / sum.  A fixed sequence of fp32 operations.
-    if (logits_out)
+    if (!kSummed && logits_out)
       for (int idx = tid; idx < nrows * E; idx += kRouterThreads) {
         const int t = idx / E, e = idx - t * E;
         logits_out[(size_t)(t0 + t) * E + e] = sm.tile[t * stride + e];
@@ -287,41 +336,24 @@ __device__ void router_epilogue(const RouterSmem& sm, const float* __restrict__ 
     __syncthreads();
   }
   // logits -> scores (in place), both written out row-major
-  for (int idx = tid; idx < nrows * E; idx += kRouterThreads) {
-    const int t = idx / E, e = idx - t * E;
-    const float z = sm.tile[t * stride + e];
-    if (logits_out && !softmax) logits_out[(size_t)(t0 + t) * E + e] = z;
-    const float s = softmax ? z : sigmoid_fixed(z);
-    sm.tile[t * stride + e] = s;
-    scores_out[(size_t)(t0 + t) * E + e] = s;
-  }
+  if (!kSummed || softmax)
+    for (int idx = tid; idx < nrows * E; idx += kRouterThreads) {
+      const int t = idx / E, e = idx - t * E;
+      const float z = sm.tile[t * stride + e];
+      if (!kSummed && logits_out && !softmax) logits_out[(size_t)(t0 + t) * E + e] = z;
+      const float s = softmax ? z : sigmoid_fixed(z);
+      sm.tile[t * stride + e] = s;
+      scores_out[(size_t)(t0 + t) * E + e] = s;
+    }
   __syncthreads();
 
-  // selection: 4 lanes per token, each owning a contiguous quarter of the experts
-  // (sixteen lanes per token, where a workgroup has them to spare, measured no faster: a round costs
-  // its chain of dependent steps, not its compares)
+  select_all<kRouterTokens, kRouterThreads>(sm, nrows, E, K);
+  __syncthreads();
+  // renormalise: four lanes to a token (as in the softmax), which share out its K slots; each adds up the
+  // denominator itself, in slot order
   const int t = tid >> 2, q = tid & 3;
-  const int eq = (E + 3) >> 2;
-  const int e_begin = q * eq;
-  const bool row_ok = t < nrows;
-  const float* row = sm.tile + t * stride;
-  // For the usual expert counts the lane keeps its quarter (score + bias) in registers, so that a
-  // round is a run of compares instead of a chain of LDS reads; same scan order, same comparisons.
-  if (E == 64 || E == 128 || E == 32 || E == 256 || E == 16) {
-    switch (E) {
-      case 16: select_from_registers<4>(sm, row, e_begin, row_ok, t, q, K); break;
-      case 32: select_from_registers<8>(sm, row, e_begin, row_ok, t, q, K); break;
-      case 64: select_from_registers<16>(sm, row, e_begin, row_ok, t, q, K); break;
-      case 128: select_from_registers<32>(sm, row, e_begin, row_ok, t, q, K); break;
-      default: select_from_registers<64>(sm, row, e_begin, row_ok, t, q, K); break;
-    }
-  } else {
-    select_from_lds(sm, row, e_begin, eq, E, row_ok, t, q, K);
-  }
-  __syncthreads();  // the selection of a token was written by its lane 0 and is read by all its lanes
-  // renormalise: the lanes of a token share out its K slots; each adds up the denominator itself, in
-  // slot order
-  if (row_ok) {
+  const float* const row = sm.tile + t * stride;
+  if (t < nrows) {
     float denom = row[sm.top_id[t * K]];
     for (int r = 1; r < K; ++r) denom = denom + row[sm.top_id[t * K + r]];
     denom = denom + 1e-20f;
@@ -880,15 +912,18 @@ __global__ __launch_bounds__(256) void router_mfma_split_kernel(
                                   partial_out, score_func, (int)blockIdx.x, (int)blockIdx.y);
 }
 
-// the slices of partial sums of n tokens, added in slice order and rounded to bf16 (the projection's output dtype),
-// into the score tile
+// The slices of partial sums of n tokens, added in slice order and rounded to bf16 (the projection's output dtype),
+// into the score tile, as scores already where these are sigmoids (both E and the sums' layout are a power of two wide).
+// `logits` / `scores`: rows of these tokens, or null logits.
 template <int kThreads>
 __device__ __forceinline__ void add_slices(const RouterSmem& sm, const float* __restrict__ partial, int slices,
-                                           size_t plane, int n, int E) {
-  const int stride = E + 1;
+                                           size_t plane, int n, int E, int score_func, float* __restrict__ logits,
+                                           float* __restrict__ scores) {
+  const int stride = E + 1, log2e = 31 - __clz(E);
+  const bool softmax = score_func == JTMOE_SCORE_SOFTMAX;
 #pragma unroll 4
   for (int idx = threadIdx.x; idx < n * E; idx += kThreads) {
-    const int t = idx / E, e = idx - t * E;
+    const int t = idx >> log2e, e = idx & (E - 1);
     float part[kPartialMaxSlices];  // all slices requested before the first is needed
 #pragma unroll
     for (int sl = 0; sl < kPartialMaxSlices; ++sl) part[sl] = sl < slices ? partial[sl * plane + idx] : 0.0f;
@@ -896,7 +931,13 @@ __device__ __forceinline__ void add_slices(const RouterSmem& sm, const float* __
 #pragma unroll
     for (int sl = 1; sl < kPartialMaxSlices; ++sl)
       if (sl < slices) v += part[sl];
-    sm.tile[t * stride + e] = round_to_bf16(v);
+    v = round_to_bf16(v);
+    if (logits) logits[idx] = v;
+    if (!softmax) {
+      v = sigmoid_fixed(v);
+      scores[idx] = v;
+    }
+    sm.tile[t * stride + e] = v;
   }
 }
 
@@ -917,10 +958,11 @@ __device__ __forceinline__ void router_finish_body(
     int32_t* __restrict__ inverse, int score_func) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   RouterSmem sm = router_smem(smem_raw, E, K, kTok);
-  add_slices<4 * kTok>(sm, partial, slices, (size_t)tokens * E, tokens, E);
+  router_clear(sm, bias, E, 4 * kTok);
+  add_slices<4 * kTok>(sm, partial, slices, (size_t)tokens * E, tokens, E, score_func, logits_out, scores);
   __syncthreads();
-  router_epilogue<bf16_raw, kTok, 4 * kTok>(sm, bias, 0, tokens, E, K, route_scale, ids, weights, scores, logits_out,
-                                            RouterScratch{}, score_func, counts, importance);
+  router_epilogue<bf16_raw, kTok, 4 * kTok, true>(sm, bias, 0, tokens, E, K, route_scale, ids, weights, scores,
+                                                  logits_out, RouterScratch{}, score_func, counts, importance);
   if (kPlan) {
     static_assert(kTok >= 1 + 4 * kTok / kWave, "the plan's tables fit into the score tile");
     dispatch_small_body<4 * kTok, false, bf16_raw>(sm.top_id, nullptr, tokens * K, E, group_sizes, offsets,
@@ -950,10 +992,12 @@ __global__ __launch_bounds__(kThreads) void router_finish_blocks_kernel(
   extern __shared__ __align__(16) unsigned char smem_raw[];
   RouterSmem sm = router_smem(smem_raw, E, K, kTok);
   const int t0 = (int)blockIdx.x * kTok;
-  add_slices<kThreads>(sm, partial + (size_t)t0 * E, slices, (size_t)tokens * E, min(kTok, tokens - t0), E);
+  router_clear(sm, bias, E, kThreads);
+  add_slices<kThreads>(sm, partial + (size_t)t0 * E, slices, (size_t)tokens * E, min(kTok, tokens - t0), E, score_func,
+                       nullptr, scores + (size_t)t0 * E);
   __syncthreads();
-  router_epilogue<bf16_raw, kTok, kThreads>(sm, bias, t0, tokens, E, K, route_scale, ids, weights, scores, nullptr,
-                                            RouterScratch{}, score_func);
+  router_epilogue<bf16_raw, kTok, kThreads, true>(sm, bias, t0, tokens, E, K, route_scale, ids, weights, scores, nullptr,
+                                                  RouterScratch{}, score_func);
 }
 
 inline size_t router_arrivals_offset(int64_t E) {
