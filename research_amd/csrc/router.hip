@@ -25,8 +25,7 @@
 namespace jtmoe {
 namespace {
 
-// A workgroup of NW waves routes 16*NW tokens with 64*NW threads (4 lanes per token in the
-// selection phase).
+// A workgroup of NW waves routes 16*NW tokens with 64*NW threads.
 
 // ---- fully specified fp32 sigmoid ------------------------------------------
 __device__ __forceinline__ float exp_fixed(float x) {
@@ -409,8 +408,8 @@ __global__ __launch_bounds__(256) void router_from_logits_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Projection for everything the matrix-core kernels below do not take (single precision, expert counts
-// other than 16 / 32 / 64 / 128 / 256, hidden sizes that are no multiple of 64): one logit per thread, a
+// Projection for everything the matrix-core kernels below do not take (single precision, expert counts or hidden
+// sizes that are no multiples of 8, unaligned operands): one logit per thread, a
 // chain of fused multiply-adds in k order, so a row's logits do not depend on the batch.
 //
 // The chain (H dependent steps) bounds it, so everything else is kept out of its way: a workgroup takes
@@ -418,8 +417,7 @@ __global__ __launch_bounds__(256) void router_from_logits_kernel(
 // time -- one 16-byte vector of x and NL vectors of the matrix per thread, requested D chunks ahead into a
 // ring of registers -- and are read back four k values at a time (x broadcast among a token's threads, the
 // matrix transposed, rows padded by four words).  When every thread walked H elements of x and of a matrix
-// column in global memory by itself, with 64 tokens to a workgroup, this took 158 us at 4096 x 1024 x 8 in
-// bf16 and 98 us at 2048 x 512 x 8 in fp32; now 18 and 11 us.
+// column in global memory by itself, with 64 tokens to a workgroup, this took 98 us at 2048 x 512 x 8 in fp32; now 11.
 // NL = logits per thread >= E / 16; kVec: rows of x and the matrix are whole, aligned 16-byte vectors.
 // ---------------------------------------------------------------------------
 constexpr int kStagedTokens = 16, kStagedThreads = 256;
@@ -575,7 +573,7 @@ __global__ __launch_bounds__(kStagedThreads) void router_staged_kernel(
 // (each lane two 16-byte pieces per 64-wide k chunk, the four lane groups of a token together whole
 // 128-byte lines per token row); the router matrix [H,E] is staged chunk by chunk through LDS as it
 // is stored and read with the transposing ds_read_b64_tr_b16.
-// Requires H % 64 == 0 and E in {16, 32, 64, 128, 256}.
+// H % 64 == 0 and E in {16, 32, 64, 128, 256}; with kPad H and E multiples of 8.
 // ---------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 constexpr int kRouterKC = 64;  // k rows of the router matrix per LDS stage
@@ -596,18 +594,27 @@ __host__ __device__ inline size_t router_mfma_smem_bytes(int E, int K, int token
   return w > ep ? w : ep;
 }
 
-template <int NB, int NW>
+// kPad kernels: expert counts below the 16 NB columns of the tiles (a multiple of 8: whole 16-byte pieces) and rows that
+// end inside a chunk (H a multiple of 8).  What lies outside the matrix or the row reads as zeros.  Byte offset of piece
+// c of a stage that starts at row k0:
+__device__ __forceinline__ int router_pad_w(int c, int pieces_per_row, int k0, int E) {
+  const int kr = c / pieces_per_row, nc = c - kr * pieces_per_row;
+  return nc * 8 < E ? ((k0 + kr) * E + nc * 8) * 2 : kOutside;
+}
+
+template <int NB, int NW, bool kPad>
 __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens,
-    int H, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
+    int H, int width, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ logits_out, void* ws, int score_func) {
   constexpr int kRouterTokens = 16 * NW, kRouterThreads = 64 * NW;
-  const int slice_chunks = router_slice_rows(H) / kRouterKC;  // 64-row chunks per slice
-  constexpr int E = NB * 16;
-  constexpr int WS = E + 32;                      // LDS row stride of the staged matrix (elements)
-  constexpr int W_CHUNKS = kRouterKC * E / 8;     // 16-byte chunks per stage
+  const int slice_chunks = (router_slice_rows(H) + kRouterKC - 1) / kRouterKC;  // 64-row chunks per slice
+  constexpr int EC = NB * 16;
+  const int E = kPad ? width : EC;
+  constexpr int WS = EC + 32;                     // LDS row stride of the staged matrix (elements)
+  constexpr int W_CHUNKS = kRouterKC * EC / 8;     // 16-byte chunks per stage
   constexpr int CW = (W_CHUNKS + kRouterThreads - 1) / kRouterThreads;
-  constexpr int CPR = E / 8;                      // chunks per k row
+  constexpr int CPR = EC / 8;                      // chunks per k row
   extern __shared__ __align__(16) unsigned char smem_raw[];
   uint16_t* const Ws = reinterpret_cast<uint16_t*>(smem_raw);  // [2][kRouterKC][WS]; reused by the epilogue
 
@@ -644,7 +651,8 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
   _Pragma("unroll") for (int i = 0; i < CW; ++i) {                                           \
     const int c = tid + i * kRouterThreads;                                                  \
     if (W_CHUNKS % kRouterThreads == 0 || c < W_CHUNKS)                                      \
-      w_ring[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, c * 16, (k0)*E * 2, 0); \
+      w_ring[slot][i] = kPad ? __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, router_pad_w(c, CPR, k0, E), 0, 0)   \
+                             : __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, c * 16, (k0)*E * 2, 0);              \
   }
 #define JT_STORE_W(slot, stage)                                                              \
   _Pragma("unroll") for (int i = 0; i < CW; ++i) {                                           \
@@ -656,13 +664,15 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
   }
 #define JT_LOAD_X(slot, k0)                                                                  \
   {                                                                                          \
-    a_ring[slot][0] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff, (k0)*2, 0);      \
-    a_ring[slot][1] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff + 64, (k0)*2, 0); \
+    _Pragma("unroll") for (int n = 0; n < 2; ++n) a_ring[slot][n] =                          \
+        kPad ? __builtin_amdgcn_raw_buffer_load_b128(                                        \
+                   x_rsrc, (k0) + n * 32 + (lane >> 4) * 8 < H ? x_voff + n * 64 + (k0)*2 : kOutside, 0, 0) \
+             : __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff + n * 64, (k0)*2, 0);    \
   }
 
   // transposing read of this lane: 16-lane group g = lane/16 reads rows 32*s + 8*g + 4*h + i/4
   const int w_lane = ((lane >> 4) * 8 + ((lane & 15) >> 2)) * WS + 4 * (lane & 3);
-  const int nchunks = H / kRouterKC;
+  const int nchunks = (H + kRouterKC - 1) / kRouterKC;
   int in_slice = 0;  // chunks of the current slice done
 #pragma unroll
   for (int d = 0; d < D; ++d)
@@ -729,7 +739,8 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
   for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      sm.tile[(wave * 16 + 4 * (lane >> 4) + i) * stride + nb * 16 + (lane & 15)] = round_to_bf16(total[nb][i]);
+      if (!kPad || nb * 16 + (lane & 15) < E)
+        sm.tile[(wave * 16 + 4 * (lane >> 4) + i) * stride + nb * 16 + (lane & 15)] = round_to_bf16(total[nb][i]);
   __syncthreads();
   router_epilogue<bf16_raw, 16 * NW, 64 * NW>(sm, bias, t0, tokens, E, K, route_scale, ids, weights, scores,
                                               logits_out, router_scratch(ws, E), score_func);
@@ -743,6 +754,12 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
 // make a workgroup, so small batches spread over more CUs.
 // ---------------------------------------------------------------------------
 constexpr int kSplitMaxTokens = 256;
+// From this many scores on a layer call of a small batch finishes in a workgroup per 16 tokens, as the middle-sized ones
+// do, and leaves the plan to the dispatch: one finishing workgroup takes longer with every score, the blocks and the
+// dispatch do not.  us a call, one workgroup against blocks: 128 experts, 37 tokens 142.9 / 143.4, 48 153.8 / 153.6, 66
+// 177.9 / 173.4, 250 255.9 / 227.9; 64 experts, 66 tokens 189.9 / 188.1, 128 193.9 / 188.1, 250 211.5 / 197.2; 8 experts,
+// 128 tokens 86.2 / 86.0.
+constexpr int64_t kFinishInBlocks = 6144;
 constexpr int kMidMaxTokens = 2560;  // with the slices in workgroups of their own, a layer call (launch_router)
 
 __host__ __device__ inline size_t router_split_smem_bytes(int E, int K) {
@@ -756,18 +773,19 @@ __host__ __device__ inline size_t router_split_smem_bytes(int E, int K) {
 // order and does the rest.  Otherwise the workgroup walks all slices itself.
 // (token_block / slice: the workgroup's place in the launch's grid -- blockIdx.x / blockIdx.y in
 // router_mfma_split_kernel; the decode launch hands them out among its own workgroups)
-template <int NB, bool kPartial>
+template <int NB, bool kPartial, bool kPad>
 __device__ __forceinline__ void router_split_body(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens,
-    int H, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
+    int H, int width, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ logits_out, void* ws, float* __restrict__ partial_out,
     int score_func, int token_block, int slice) {
   constexpr int kThreads = 256, kTokens = 16;
-  constexpr int E = NB * 16;
-  constexpr int WS = E + 32;
-  constexpr int W_CHUNKS = kSplitKC * E / 8;
+  constexpr int EC = NB * 16;
+  const int E = kPad ? width : EC;
+  constexpr int WS = EC + 32;
+  constexpr int W_CHUNKS = kSplitKC * EC / 8;
   constexpr int CW = (W_CHUNKS + kThreads - 1) / kThreads;
-  constexpr int CPR = E / 8;
+  constexpr int CPR = EC / 8;
   constexpr int NBW = (NB + 3) / 4;  // column blocks per wave
   extern __shared__ __align__(16) unsigned char smem_raw[];
   uint16_t* const Ws = reinterpret_cast<uint16_t*>(smem_raw);  // [2][kSplitKC][WS]
@@ -798,7 +816,8 @@ __device__ __forceinline__ void router_split_body(
     _Pragma("unroll") for (int i = 0; i < CW; ++i) {                                          \
       const int c = tid + i * kThreads;                                                       \
       if (W_CHUNKS % kThreads == 0 || c < W_CHUNKS)                                           \
-        w_ring[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, c * 16, (k0)*E * 2, 0); \
+        w_ring[slot][i] = kPad ? __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, router_pad_w(c, CPR, k0, E), 0, 0) \
+                               : __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, c * 16, (k0)*E * 2, 0);             \
     }                                                                                         \
     if (has_cols) {                                                                           \
       _Pragma("unroll") for (int n = 0; n < 4; ++n)                                           \
@@ -879,7 +898,7 @@ __device__ __forceinline__ void router_split_body(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int t = 4 * (lane >> 4) + i;
-          if (t < nrows && wave + 4 * b < NB)
+          if (t < nrows && wave + 4 * b < NB && (!kPad || (wave + 4 * b) * 16 + (lane & 15) < E))
             partial_out[((size_t)slice * tokens + t0 + t) * E + (wave + 4 * b) * 16 + (lane & 15)] = acc[b][i];
         }
     }
@@ -894,7 +913,7 @@ __device__ __forceinline__ void router_split_body(
     for (int b = 0; b < NBW; ++b)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (wave + 4 * b < NB)
+        if (wave + 4 * b < NB && (!kPad || (wave + 4 * b) * 16 + (lane & 15) < E))
           sm.tile[(4 * (lane >> 4) + i) * stride + (wave + 4 * b) * 16 + (lane & 15)] = round_to_bf16(total[b][i]);
   }
   __syncthreads();
@@ -902,28 +921,29 @@ __device__ __forceinline__ void router_split_body(
                                                logits_out, router_scratch(ws, E), score_func);
 }
 
-template <int NB, bool kPartial>
+template <int NB, bool kPartial, bool kPad>
 __global__ __launch_bounds__(256) void router_mfma_split_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens,
-    int H, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
+    int H, int width, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ logits_out, void* ws, float* __restrict__ partial_out,
     int score_func) {
-  router_split_body<NB, kPartial>(x, w, bias, tokens, H, K, route_scale, ids, weights, scores, logits_out, ws,
+  router_split_body<NB, kPartial, kPad>(x, w, bias, tokens, H, width, K, route_scale, ids, weights, scores, logits_out, ws,
                                   partial_out, score_func, (int)blockIdx.x, (int)blockIdx.y);
 }
 
 // The slices of partial sums of n tokens, added in slice order and rounded to bf16 (the projection's output dtype),
-// into the score tile, as scores already where these are sigmoids (both E and the sums' layout are a power of two wide).
+// into the score tile, as scores already where these are sigmoids.
 // `logits` / `scores`: rows of these tokens, or null logits.
 template <int kThreads>
 __device__ __forceinline__ void add_slices(const RouterSmem& sm, const float* __restrict__ partial, int slices,
                                            size_t plane, int n, int E, int score_func, float* __restrict__ logits,
                                            float* __restrict__ scores) {
   const int stride = E + 1, log2e = 31 - __clz(E);
+  const bool pow2 = (E & (E - 1)) == 0;
   const bool softmax = score_func == JTMOE_SCORE_SOFTMAX;
 #pragma unroll 4
   for (int idx = threadIdx.x; idx < n * E; idx += kThreads) {
-    const int t = idx >> log2e, e = idx & (E - 1);
+    const int t = pow2 ? idx >> log2e : idx / E, e = idx - t * E;
     float part[kPartialMaxSlices];  // all slices requested before the first is needed
 #pragma unroll
     for (int sl = 0; sl < kPartialMaxSlices; ++sl) part[sl] = sl < slices ? partial[sl * plane + idx] : 0.0f;
@@ -1055,7 +1075,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
   }
   __shared__ int is_last;
   const int token_block = (int)blockIdx.x % token_blocks, slice = (int)blockIdx.x / token_blocks;
-  router_split_body<NB, true>(x, w_router, bias, T, H, K, route_scale, ids, weights, scores, nullptr, nullptr, partial,
+  router_split_body<NB, true, false>(x, w_router, bias, T, H, E, K, route_scale, ids, weights, scores, nullptr, nullptr, partial,
                               score_func, token_block, slice);
   // Hand-over.  Every thread waits until its own stores have reached the L2 (on this part stores count in
   // vmcnt); after the barrier one thread releases them to the device (the fence writes the L2's dirty
@@ -1095,16 +1115,16 @@ using SharedGateUpCfg = SkinnyCfg<1, 2, true>;
 using SharedDownCfg = SkinnyCfg<1, 2, false>;
 constexpr int kSharedFinishTokens = 64;  // the finishing workgroup has the tiles' 256 threads
 
-template <int NB>
+template <int NB, bool kPad>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void router_shared_gate_up_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int tokens, int H, int K, float* __restrict__ partial,
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int tokens, int H, int E, int K, float* __restrict__ partial,
     int token_blocks, int router_blocks, SkinnyProblem shared) {
   const int block = (int)blockIdx.x;
   if (block >= router_blocks) {
     grouped_gemm_skinny_tile<SharedGateUpCfg>(shared, block - router_blocks, (int)gridDim.x - router_blocks);
     return;
   }
-  router_split_body<NB, true>(x, w, nullptr, tokens, H, K, 1.0f, nullptr, nullptr, nullptr, nullptr, nullptr, partial, 0,
+  router_split_body<NB, true, kPad>(x, w, nullptr, tokens, H, E, K, 1.0f, nullptr, nullptr, nullptr, nullptr, nullptr, partial, 0,
                               block % token_blocks, block / token_blocks);
 }
 
@@ -1145,6 +1165,22 @@ struct LayerPlan {
   size_t scratch_bytes;
 };
 
+// bf16 routers whose experts and columns are multiples of 8 run on the matrix cores, in tiles of 16, 32, 64, 128 or 256
+// columns; where these do not fit exactly, in kernels that check (kPad).  The staged kernel, a chain of H dependent steps,
+// takes what is left: where it took those too, a router call
+// of 2000 x 1384 x 96 took 127 us (now 36), 2931 x 1000 x 24 30 (17.5), 4096 x 1024 x 8 18.4 (12.8), 300 x 1024 x 8
+// 17 (3.6 + 4.2), and a layer call of one token at 1024 x 8 66 (49.5: the plan and the shared experts share its launches).
+inline bool router_on_matrix_cores(const void* x, const void* w, int64_t H, int64_t E) {
+  return H % 8 == 0 && E % 8 == 0 && E <= 256 && H * E < ((int64_t)1 << 30) && aligned16(x) && aligned16(w);
+}
+inline bool router_padded(int64_t H, int64_t E) { return H % kRouterKC != 0 || E < 16 || (E & (E - 1)) != 0; }
+// column blocks of 16 in the tiles: 1, 2, 4, 8 or 16
+inline int router_column_blocks(int64_t E) {
+  int nb = 1;
+  while (nb * 16 < E) nb *= 2;
+  return nb;
+}
+
 template <typename T, bool kFromLogits>
 int launch_router(const void* x, const void* w, const float* logits_in, const float* bias, int64_t tokens,
                   int64_t H, int64_t E, int64_t K, double route_scale, int32_t* ids, void* weights,
@@ -1154,8 +1190,8 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
   const bool stats = layer == nullptr;
   void* const ws_stats = stats ? ws : nullptr;
   if (layer) layer->stats_done = layer->plan_done = false;
-  const bool mfma = Elem<T>::is_bf16 && !kFromLogits && H % kRouterKC == 0 && H * E < ((int64_t)1 << 30) &&
-                    (E == 16 || E == 32 || E == 64 || E == 128 || E == 256) && aligned16(x) && aligned16(w);
+  const bool mfma = Elem<T>::is_bf16 && !kFromLogits && router_on_matrix_cores(x, w, H, E);
+  const bool pad = router_padded(H, E);
   if (mfma) {
     // Up to a few hundred tokens the whole call is a handful of workgroups, each waiting on its own
     // chain of chunks: the k-split kernel (16 tokens per workgroup, half as many and shorter
@@ -1163,7 +1199,7 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
     // less often per token and win.
     if (H % kSplitKC == 0 && tokens <= kSplitMaxTokens) {
       const int blocks = (int)((tokens + 15) / 16);
-      const size_t smem = router_split_smem_bytes((int)E, (int)K);
+      const size_t smem = std::max(router_split_smem_bytes((int)E, (int)K), router_split_smem_bytes(16 * router_column_blocks(E), 1));
       if (smem > 160 * 1024)
         return fail(JTMOE_EUNSUPPORTED, "router: E=%lld K=%lld needs %zu bytes of LDS", (long long)E, (long long)K, smem);
       // Two launches when one workgroup can hold the epilogue of the whole call: partial sums over
@@ -1174,16 +1210,16 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
         const int slices = (int)((H + slice_rows - 1) / slice_rows);
         float* partial = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + router_scratch_bytes(E));
 #define JT_PARTIAL_CASE(NB)                                                                                   \
-  case NB * 16: {                                                                                            \
-    auto kernel = router_mfma_split_kernel<NB, true>;                                                        \
+  case NB: {                                                                                                 \
+    auto kernel = pad ? &router_mfma_split_kernel<NB, true, true> : &router_mfma_split_kernel<NB, true, false>; \
     int rc = set_max_smem(kernel, smem);                                                                     \
     if (rc) return rc;                                                                                       \
     kernel<<<dim3(blocks, slices), 256, smem, stream>>>(                                                     \
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K, \
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, ws, partial,           \
         score_func);                                                                                         \
   } break;
-        switch ((int)E) {
+        switch (router_column_blocks(E)) {
           JT_PARTIAL_CASE(1)
           JT_PARTIAL_CASE(2)
           JT_PARTIAL_CASE(4)
@@ -1191,6 +1227,15 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
           JT_PARTIAL_CASE(16)
         }
 #undef JT_PARTIAL_CASE
+        if (layer && tokens * E >= kFinishInBlocks) {
+          const size_t bsmem = router_smem_bytes((int)E, (int)K, 16);
+          auto finish = router_finish_blocks_kernel<16, 256>;
+          const int rc = set_max_smem(finish, bsmem);
+          if (rc) return rc;
+          finish<<<blocks, 256, bsmem, stream>>>(partial, slices, bias, (int)tokens, (int)E, (int)K, (float)route_scale,
+                                                 ids, static_cast<bf16_raw*>(weights), scores, score_func);
+          return check_launch("router");
+        }
         const size_t fsmem = router_smem_bytes((int)E, (int)K, finish_tok);
         const bool plan = layer != nullptr && tokens * K <= kSmallMaxAssignments && E <= 4 * finish_tok;
 #define JT_FINISH(TOK, PLAN)                                                                                       \
@@ -1219,16 +1264,16 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
       if (stats) router_zero_kernel<<<1, 256, 0, stream>>>(ws, (int)E);
       if (tokens > 0) {
 #define JT_SPLIT_CASE(NB)                                                                                     \
-  case NB * 16: {                                                                                            \
-    auto kernel = router_mfma_split_kernel<NB, false>;                                                       \
+  case NB: {                                                                                                 \
+    auto kernel = pad ? &router_mfma_split_kernel<NB, false, true> : &router_mfma_split_kernel<NB, false, false>; \
     int rc = set_max_smem(kernel, smem);                                                                     \
     if (rc) return rc;                                                                                       \
     kernel<<<blocks, 256, smem, stream>>>(                                                                   \
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K, \
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, ws_stats, nullptr,     \
         score_func);                                                                                         \
   } break;
-        switch ((int)E) {
+        switch (router_column_blocks(E)) {
           JT_SPLIT_CASE(1)
           JT_SPLIT_CASE(2)
           JT_SPLIT_CASE(4)
@@ -1252,22 +1297,22 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
     const int slices = (int)((H + slice_rows - 1) / slice_rows);
     if (layer && tokens <= kMidMaxTokens && H % kSplitKC == 0 && H >= 1024 &&
         (size_t)slices * tokens * E * sizeof(float) <= layer->scratch_bytes) {
-      const size_t smem = (size_t)2 * kSplitKC * router_w_stride((int)E) * 2;
+      const size_t smem = (size_t)2 * kSplitKC * router_w_stride(16 * router_column_blocks(E)) * 2;
       const size_t fsmem = router_smem_bytes((int)E, (int)K, 16);
       if (fsmem <= 160 * 1024) {
         float* const partial = static_cast<float*>(layer->scratch);
         const int blocks = (int)((tokens + 15) / 16);
 #define JT_PARTIAL_CASE(NB)                                                                                  \
-  case NB * 16: {                                                                                            \
-    auto kernel = router_mfma_split_kernel<NB, true>;                                                        \
+  case NB: {                                                                                                 \
+    auto kernel = pad ? &router_mfma_split_kernel<NB, true, true> : &router_mfma_split_kernel<NB, true, false>; \
     const int rc = set_max_smem(kernel, smem);                                                               \
     if (rc) return rc;                                                                                       \
     kernel<<<dim3(blocks, slices), 256, smem, stream>>>(                                                     \
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K, \
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, nullptr, partial,      \
         score_func);                                                                                         \
   } break;
-        switch ((int)E) {
+        switch (router_column_blocks(E)) {
           JT_PARTIAL_CASE(1)
           JT_PARTIAL_CASE(2)
           JT_PARTIAL_CASE(4)
@@ -1288,24 +1333,24 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
     constexpr int nw = 4;
     const int tok = 16 * nw;
     const int blocks = (int)((tokens + tok - 1) / tok);
-    const size_t smem = router_mfma_smem_bytes((int)E, (int)K, tok);
+    const size_t smem = std::max(router_mfma_smem_bytes((int)E, (int)K, tok), router_mfma_smem_bytes(16 * router_column_blocks(E), 1, 1));
     if (smem > 160 * 1024) return fail(JTMOE_EUNSUPPORTED, "router: E=%lld K=%lld needs %zu bytes of LDS", (long long)E, (long long)K, smem);
     if (stats) router_zero_kernel<<<1, 256, 0, stream>>>(ws, (int)E);
     if (tokens > 0) {
 #define JT_ROUTER_LAUNCH(NB, NW)                                                                             \
   {                                                                                                          \
-    auto kernel = router_mfma_kernel<NB, NW>;                                                                \
+    auto kernel = pad ? &router_mfma_kernel<NB, NW, true> : &router_mfma_kernel<NB, NW, false>;               \
     int rc = set_max_smem(kernel, smem);                                                                     \
     if (rc) return rc;                                                                                       \
     kernel<<<blocks, 64 * NW, smem, stream>>>(                                                               \
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K, \
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, ws_stats, score_func); \
   }
 #define JT_ROUTER_CASE(NB)    \
-  case NB * 16:               \
+  case NB:                    \
     JT_ROUTER_LAUNCH(NB, nw)  \
     break;
-      switch ((int)E) {
+      switch (router_column_blocks(E)) {
         JT_ROUTER_CASE(1)
         JT_ROUTER_CASE(2)
         JT_ROUTER_CASE(4)
@@ -1439,8 +1484,8 @@ int launch_decode_gate_up_router(const void* x, const void* w_router, const floa
 static bool router_takes_shared(const void* x, const void* w_router, const SharedExperts& shared, int64_t T, int64_t H,
                                 int64_t E, int64_t K, int dtype) {
   return dtype == JTMOE_BF16 && T > 0 && T <= kSharedFinishTokens && T * K <= kSmallMaxAssignments &&
-         H % kSplitKC == 0 && H * E < ((int64_t)1 << 30) && (E == 16 || E == 32 || E == 64 || E == 128 || E == 256) &&
-         aligned16(x) && aligned16(w_router) && router_split_smem_bytes((int)E, (int)K) <= 160 * 1024 &&
+         H % kSplitKC == 0 && router_on_matrix_cores(x, w_router, H, E) &&
+         router_split_smem_bytes((int)E, (int)K) <= 160 * 1024 &&
          router_smem_bytes((int)E, (int)K, kSharedFinishTokens) <= 160 * 1024 && shared_in_skinny_tiles(x, shared, T, H);
 }
 
@@ -1463,19 +1508,21 @@ static int launch_router_with_shared(const void* x, const void* w_router, const 
                                         SharedGateUpCfg::BN);
   const SkinnyProblem down = problem(sh.act, sh.down, nullptr, sh.y, nullptr, nullptr, sh.Is, H, SharedDownCfg::BM,
                                      SharedDownCfg::BN);
-  const size_t smem = std::max(router_split_smem_bytes((int)E, (int)K), (size_t)SharedGateUpCfg::SMEM_BYTES);
+  const bool pad = router_padded(H, E);
+  const size_t smem = std::max({router_split_smem_bytes((int)E, (int)K), router_split_smem_bytes(16 * router_column_blocks(E), 1),
+                                (size_t)SharedGateUpCfg::SMEM_BYTES});
   const int router_blocks = token_blocks * slices;
   const int64_t grid = router_blocks + gemm_grid(gate_up.mtiles, gate_up.ntiles_n);
 #define JT_SHARED_CASE(NB)                                                                                       \
-  case NB * 16: {                                                                                                \
-    auto kernel = router_shared_gate_up_kernel<NB>;                                                              \
+  case NB: {                                                                                                     \
+    auto kernel = pad ? &router_shared_gate_up_kernel<NB, true> : &router_shared_gate_up_kernel<NB, false>;      \
     const int rc = set_max_smem(kernel, smem);                                                                   \
     if (rc) return rc;                                                                                           \
     kernel<<<(unsigned)grid, 256, smem, stream>>>(static_cast<const uint16_t*>(x),                               \
-                                                  static_cast<const uint16_t*>(w_router), (int)T, (int)H, (int)K, \
+                                                  static_cast<const uint16_t*>(w_router), (int)T, (int)H, (int)E, (int)K, \
                                                   partial, token_blocks, router_blocks, gate_up);                \
   } break;
-  switch ((int)E) {
+  switch (router_column_blocks(E)) {
     JT_SHARED_CASE(1)
     JT_SHARED_CASE(2)
     JT_SHARED_CASE(4)
