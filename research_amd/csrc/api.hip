@@ -663,28 +663,30 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
   // the dispatch plan; the down launch then picks the routed rows.
   hipStream_t main_stream = as_stream(stream);
   const bool decode = !train && decode_dense_supported(T, H, E, K, I, dtype);
-  bool stats_done = false, plan_done = false, shared_done = false;
+  bool stats_done = false, plan_done = false, shared_done = Is == 0;
   // (a timed call keeps the shared experts in launches of their own, so that their stages are theirs)
   const bool offer_shared = Is > 0 && g_stage_timer == nullptr;
-  const SharedExperts shared{shared_gate, shared_up, shared_down, Is, w.shared_act, w.shared_y, shared_gate_pre,
-                             shared_up_pre};
+  SharedExperts shared{shared_gate, shared_up, shared_down, Is, w.shared_act, w.shared_y, shared_gate_pre,
+                       shared_up_pre, false};
   int rc;
   if (decode) {
     rc = launch_decode_gate_up_router(x, w_router, expert_bias, gate, up, w.act, T, H, E, K, I, route_scale,
                                       score_func, expert_ids, weights, scores, expert_counts, importance, group_sizes,
-                                      offsets, source_order, inverse, w.router, main_stream);
+                                      offsets, source_order, inverse, w.router, main_stream,
+                                      offer_shared ? &shared : nullptr);
     if (rc) return rc;
     stage_mark(kStageGateUp, main_stream);
     rc = launch_down_from_all_tokens(w.act, down, group_sizes, offsets, source_order, T, K, H, I, E, w.packed_y,
-                                     main_stream);
+                                     main_stream, shared.gate_up_done ? &shared : nullptr);
     if (rc) return rc;
+    shared_done = shared_done || shared.gate_up_done;
     stage_mark(kStageDown, main_stream);
     rc = check_launch("grouped gemm");
   } else {
     rc = router_for_layer(x, w_router, expert_bias, T, H, E, K, route_scale, dtype, expert_ids, weights, scores,
                           expert_counts, importance, group_sizes, offsets, source_order, inverse, w.router,
                           w.router_bytes, score_func, &stats_done, &plan_done, main_stream, w.act, w.act_bytes,
-                          offer_shared ? &shared : nullptr, &shared_done);
+                          offer_shared ? &shared : nullptr);
     if (rc) return rc;
     stage_mark(kStageRouter, main_stream);
     rc = dispatch_for_layer(expert_ids, weights, (T > 0 && !gather) ? x : nullptr, T, H, E, K, dtype, group_sizes,
@@ -694,7 +696,7 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
   if (rc) return rc;
   if (!decode) {  // (the decode path has enqueued both of its GEMM launches above)
     if (train || gather) {
-      const bool take = offer_shared && !shared_done && T > 0;
+      const bool take = offer_shared && T > 0;
       rc = launch_swiglu_gather(x, source_order, gate, up, down, group_sizes, offsets, T, K, H, I, E, dtype, w.act,
                                 w.packed_y, main_stream, take ? &shared : nullptr, gate_pre, up_pre);
       shared_done = shared_done || take;
@@ -704,7 +706,7 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
                                 w.packed_y, stream);
     if (rc) return rc;
   }
-  if (Is > 0 && !shared_done) {
+  if (!shared_done) {
     if (train)
       rc = jtmoe_shared_swiglu_train(x, shared_gate, shared_up, shared_down, T, H, Is, dtype, shared_gate_pre,
                                      shared_up_pre, w.shared_act, w.shared_y, stream);

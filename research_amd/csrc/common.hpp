@@ -123,13 +123,14 @@ int dispatch_for_layer(const int32_t* expert_ids, const void* weights, const voi
                        int32_t* inverse, void* packed_x, float* expert_counts, float* importance, void* workspace,
                        bool want_stats, bool plan_done, hipStream_t stream);
 
-// The shared experts of a layer call.  A router of a few tokens takes them along in its own two launches
-// (*shared_done): neither needs the other's results, and the router's workgroups leave most CUs idle.
+// The shared experts of a layer call.  A router of a few tokens takes their gate/up product along in its launch (and sets
+// gate_up_done), the routed products then the down one: neither needs the other's results.
 // gate_pre / up_pre: where a training forward keeps the two rounded products, or null.
 struct SharedExperts {
   const void *gate, *up, *down;
   int64_t Is;
   void *act, *y, *gate_pre, *up_pre;
+  bool gate_up_done;
 };
 
 // router.hip: the router as the layer runs it, with the dispatch plan behind it where that is free.
@@ -143,7 +144,7 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
                      float* expert_counts, float* importance, int32_t* group_sizes, int32_t* offsets,
                      int32_t* source_order, int32_t* inverse, void* workspace, size_t workspace_bytes,
                      int score_func, bool* stats_done, bool* plan_done, hipStream_t stream, void* scratch = nullptr,
-                     size_t scratch_bytes = 0, const SharedExperts* shared = nullptr, bool* shared_done = nullptr);
+                     size_t scratch_bytes = 0, SharedExperts* shared = nullptr);
 // grouped_gemm.hip: whether both products of the shared experts run in the streaming tiles of 16 rows x 64 columns
 // (the ones that can share the router's launches) at these sizes and pointers.
 bool shared_in_skinny_tiles(const void* x, const SharedExperts& shared, int64_t T, int64_t H);
@@ -170,9 +171,11 @@ int launch_decode_gate_up_router(const void* x, const void* w_router, const floa
                                  const void* up, void* act_full, int64_t T, int64_t H, int64_t E, int64_t K, int64_t I,
                                  double route_scale, int score_func, int32_t* expert_ids, void* weights, float* scores,
                                  float* expert_counts, float* importance, int32_t* group_sizes, int32_t* offsets,
-                                 int32_t* source_order, int32_t* inverse, void* router_workspace, hipStream_t stream);
+                                 int32_t* source_order, int32_t* inverse, void* router_workspace, hipStream_t stream,
+                                 SharedExperts* shared = nullptr);
 int launch_down_from_all_tokens(const void* act_full, const void* down, const int32_t* group_sizes,
                                 const int32_t* offsets, const int32_t* source_order, int64_t T, int64_t K, int64_t H,
-                                int64_t I, int64_t E, void* packed_y, hipStream_t stream);
+                                int64_t I, int64_t E, void* packed_y, hipStream_t stream,
+                                const SharedExperts* shared = nullptr);
 
 }  // namespace jtmoe

@@ -162,7 +162,8 @@ template <typename Cfg>
 int launch_fast(const void* a, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
                 const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, hipStream_t stream,
                 const int32_t* row_map = nullptr, int row_div = 1, int64_t a_rows = 0, void* save0 = nullptr,
-                void* save1 = nullptr, int64_t uniform_rows = 0, int64_t a_group_rows = 0) {
+                void* save1 = nullptr, int64_t uniform_rows = 0, int64_t a_group_rows = 0,
+                const Beside* beside = nullptr) {
   // the 256-row configurations run as persistent workgroups (see persistent_schedule), the others one
   // tile per workgroup
   constexpr bool kPersistent = Cfg::BM == 256 && Cfg::NSTAGE == 2 && Cfg::BK == 64;
@@ -197,6 +198,16 @@ int launch_fast(const void* a, const void* b0, const void* b1, void* c, const in
         row_map, row_div, (int)a_rows, static_cast<uint16_t*>(save0), static_cast<uint16_t*>(save1), ps.window,
         ps.chunk);
   } else {
+    // (the shared experts come beside a router of whole 128-row chunks: never with a ragged reduction here)
+    constexpr bool kBeside = (Cfg::OPT & 65536) == 0;
+    if constexpr (kBeside) if (beside) {
+      grouped_gemm_dma_beside_kernel<Cfg><<<(unsigned)(tiles_grid + beside->blocks), Cfg::NT, Cfg::SMEM_BYTES, stream>>>(
+          static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
+          static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim, (int)N, (int)mtiles, (int)nt,
+          row_map, row_div, (int)a_rows, static_cast<uint16_t*>(save0), static_cast<uint16_t*>(save1),
+          (int)a_group_rows, *beside);
+      return JTMOE_OK;
+    }
     kernel<<<(unsigned)tiles_grid, Cfg::NT, Cfg::SMEM_BYTES, stream>>>(
         static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
         static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim, (int)N, (int)mtiles, (int)nt,
@@ -292,7 +303,7 @@ template <typename Cfg>
 int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, hipStream_t stream,
                   const int32_t* row_map = nullptr, int row_div = 1, int64_t a_rows = 0, void* save0 = nullptr,
-                  void* save1 = nullptr, int64_t a_group_rows = 0) {
+                  void* save1 = nullptr, int64_t a_group_rows = 0, const Beside* beside = nullptr) {
   static_assert(Cfg::SMEM_BYTES <= 64 * 1024, "launched without a raised limit");
   const int64_t mtiles = group_sizes == nullptr ? (rows + Cfg::BM - 1) / Cfg::BM : max_m_tiles(rows, E, Cfg::BM);
   const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
@@ -302,7 +313,11 @@ int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const 
                         static_cast<uint16_t*>(c), static_cast<uint16_t*>(save0), static_cast<uint16_t*>(save1),
                         group_sizes, offsets, row_map, (int)E, (int)rows, (int)Kdim, (int)N, (int)mtiles, (int)nt, row_div,
                         (int)a_rows, (int)a_group_rows};
-  grouped_gemm_skinny_kernel<Cfg><<<(unsigned)grid, Cfg::NT, Cfg::SMEM_BYTES, stream>>>(p);
+  if (beside)
+    grouped_gemm_skinny_beside_kernel<Cfg><<<(unsigned)(grid + beside->blocks), Cfg::NT,
+                                             std::max<int>(Cfg::SMEM_BYTES, BesideCfg::SMEM_BYTES), stream>>>(p, *beside);
+  else
+    grouped_gemm_skinny_kernel<Cfg><<<(unsigned)grid, Cfg::NT, Cfg::SMEM_BYTES, stream>>>(p);
   return JTMOE_OK;
 }
 
@@ -346,6 +361,11 @@ inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dua
   return most > 0.0;
 }
 
+inline bool streaming_or_rows64(ProductKernel k) {
+  return k == ProductKernel::kStream16x128 || k == ProductKernel::kStream16x64 || k == ProductKernel::kStream32x64 ||
+         k == ProductKernel::kRows64 || k == ProductKernel::kRows64Tail;
+}
+
 // Rows per group up to which 64-row LDS tiles hold nearly every group in one tile: each expert matrix is then
 // read by one row of workgroups, with non-temporal loads.  us for gate/up and down, 64 experts: mean 48 rows 121
 // and 61 (256-row tiles 141 and 77), mean 64 rows, where half of the groups need a second tile, 203 and 103 (148
@@ -376,11 +396,6 @@ ProductKernel down_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, bool de
   if (half == HalfTiles::kOnePerCu && stream_ok<DownHalfCfg>(rows, I, H, nullptr, 1)) return ProductKernel::kHalf;
   if (half != HalfTiles::kNone && stream_ok<DownHalfDeepCfg>(rows, I, H, nullptr, 1)) return ProductKernel::kHalfDeep;
   return I % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
-}
-
-inline bool streaming_or_rows64(ProductKernel k) {
-  return k == ProductKernel::kStream16x128 || k == ProductKernel::kStream16x64 || k == ProductKernel::kStream32x64 ||
-         k == ProductKernel::kRows64 || k == ProductKernel::kRows64Tail;
 }
 
 // Routed and shared experts in one launch (joint_tiles): the kernel of both, or kGeneral for launches of their own.
@@ -425,17 +440,19 @@ inline bool fast_ok(const void* a, const void* b0, const void* b1, const void* c
 // its group's block of a_group_rows rows (the decode path)
 int launch_down_fast(const void* act, const void* down, const int32_t* group_sizes, const int32_t* offsets,
                      int64_t rows, int64_t H, int64_t I, int64_t E, void* y, hipStream_t stream,
-                     const int32_t* row_map = nullptr, int row_div = 1, int64_t a_group_rows = 0) {
+                     const int32_t* row_map = nullptr, int row_div = 1, int64_t a_group_rows = 0,
+                     const Beside* beside = nullptr, bool* beside_taken = nullptr) {
 #define JT_DOWN(LAUNCH, CFG) LAUNCH<CFG>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream, row_map, row_div, a_group_rows, nullptr, nullptr
   using S11 = SkinnyCfg<1, 1, false>;
   using S12 = SkinnyCfg<1, 2, false>;
   using S22 = SkinnyCfg<2, 2, false>;
   const ProductKernel k = down_kernel(rows, H, I, E, group_sizes == nullptr, persistent_grid_size());
+  if (beside) *beside_taken = streaming_or_rows64(k);
   switch (k) {
-    case ProductKernel::kStream16x128: return JT_DOWN(launch_skinny, S11), a_group_rows);
-    case ProductKernel::kStream16x64: return JT_DOWN(launch_skinny, S12), a_group_rows);
-    case ProductKernel::kStream32x64: return JT_DOWN(launch_skinny, S22), a_group_rows);
-    case ProductKernel::kRows64: return JT_DOWN(launch_fast, DownTinyCfg), 0, a_group_rows);
+    case ProductKernel::kStream16x128: return JT_DOWN(launch_skinny, S11), a_group_rows, beside);
+    case ProductKernel::kStream16x64: return JT_DOWN(launch_skinny, S12), a_group_rows, beside);
+    case ProductKernel::kStream32x64: return JT_DOWN(launch_skinny, S22), a_group_rows, beside);
+    case ProductKernel::kRows64: return JT_DOWN(launch_fast, DownTinyCfg), 0, a_group_rows, beside);
     default: break;
   }
   // (at most half a tile of rows per group on the decode path: the rules above take all of it)
@@ -449,23 +466,29 @@ int launch_down_fast(const void* act, const void* down, const int32_t* group_siz
 #undef JT_DOWN
 }
 
+// (`beside`: streaming and 64-row tiles take these tiles along, and say so)
 template <typename T>
-int launch_gate_up(const RoutedProblem& p, hipStream_t stream) {
+int launch_gate_up(const RoutedProblem& p, hipStream_t stream, const Beside* beside = nullptr,
+                   bool* beside_taken = nullptr) {
   const bool dense = p.group_sizes == nullptr;
   const bool gather_ok = p.row_map == nullptr || p.a_rows * p.K < ((int64_t)1 << 30);
   const bool saves_ok = aligned16(p.save0) && aligned16(p.save1);
-#define JT_GATE_UP(LAUNCH, CFG)                                                                                  \
+#define JT_GATE_UP(LAUNCH, CFG, ...)                                                                             \
   LAUNCH<CFG>(p.a, p.b0, p.b1, p.c, p.group_sizes, p.offsets, p.rows, p.K, p.N, p.E, stream, p.row_map, p.row_div, \
-              p.a_rows, p.save0, p.save1)
+              p.a_rows, p.save0, p.save1 __VA_ARGS__)
+#define JT_BESIDE , 0, beside
+#define JT_BESIDE64 , 0, 0, beside
   if (Elem<T>::is_bf16 && fast_ok(p.a, p.b0, p.b1, p.c, p.K, p.N) && gather_ok && saves_ok) {
     using S11 = SkinnyCfg<1, 1, true>;
     using S12 = SkinnyCfg<1, 2, true>;
     using S22 = SkinnyCfg<2, 2, true>;
-    switch (gate_up_kernel(p.rows, p.K, p.N, p.E, dense, persistent_grid_size(), p.row_map, p.row_div)) {
-      case ProductKernel::kStream16x128: return JT_GATE_UP(launch_skinny, S11);
-      case ProductKernel::kStream16x64: return JT_GATE_UP(launch_skinny, S12);
-      case ProductKernel::kStream32x64: return JT_GATE_UP(launch_skinny, S22);
-      case ProductKernel::kRows64: return JT_GATE_UP(launch_fast, GateUpTinyCfg);
+    const ProductKernel k = gate_up_kernel(p.rows, p.K, p.N, p.E, dense, persistent_grid_size(), p.row_map, p.row_div);
+    if (beside) *beside_taken = streaming_or_rows64(k) && k != ProductKernel::kRows64Tail;
+    switch (k) {
+      case ProductKernel::kStream16x128: return JT_GATE_UP(launch_skinny, S11, JT_BESIDE);
+      case ProductKernel::kStream16x64: return JT_GATE_UP(launch_skinny, S12, JT_BESIDE);
+      case ProductKernel::kStream32x64: return JT_GATE_UP(launch_skinny, S22, JT_BESIDE);
+      case ProductKernel::kRows64: return JT_GATE_UP(launch_fast, GateUpTinyCfg, JT_BESIDE64);
       case ProductKernel::kRows64Tail: return JT_GATE_UP(launch_fast, GateUpTinyTailCfg);
       case ProductKernel::kHalf: return JT_GATE_UP(launch_stream, GateUpHalfCfg);
       case ProductKernel::kHalfTail: return JT_GATE_UP(launch_stream, GateUpHalfTailCfg);
@@ -475,6 +498,8 @@ int launch_gate_up(const RoutedProblem& p, hipStream_t stream) {
       default: return JT_GATE_UP(launch_fast, GateUpTailCfg);
     }
   }
+#undef JT_BESIDE64
+#undef JT_BESIDE
 #undef JT_GATE_UP
   if (!Elem<T>::is_bf16 && f32_gemm_supported(p.a, p.save0, p.b0, p.b1, p.c, p.row_map ? p.a_rows : p.rows, p.K, p.N) &&
       aligned16(p.save1))
@@ -554,6 +579,17 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
                             nullptr, x_rows, H, shared->Is, 1, 0, 0, 1};
     const RoutedProblem sdn{shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, nullptr, nullptr, nullptr,
                             x_rows, shared->Is, H, 1, 0, 0, 1};
+    if (shared->gate_up_done) {
+      // (a few tokens: the router has run the shared gate/up product, its down product goes beside the routed gate/up)
+      const SkinnyProblem down_p = dense_skinny(shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, x_rows,
+                                                shared->Is, H, BesideCfg::BM, BesideCfg::BN);
+      const Beside beside{down_p, (int)gemm_grid(down_p.mtiles, down_p.ntiles_n)};
+      bool taken = false;
+      rc = launch_gate_up<T>(gu, stream, &beside, &taken);
+      if (!rc) rc = launch_down<T>(dn, stream);
+      if (!rc && !taken) rc = launch_down<T>(sdn, stream);
+      return rc ? rc : check_launch("grouped gemm");
+    }
     rc = launch_with_shared<T>(gu, dn, sgu, sdn, stream);
     return rc ? rc : check_launch("grouped gemm");
   }
@@ -580,11 +616,21 @@ int validate_gemm(const char* what, int64_t rows, int64_t H, int64_t I, int64_t 
 // ---- the down launch of the layer's decode path (declared in common.hpp) ----
 int launch_down_from_all_tokens(const void* act_full, const void* down, const int32_t* group_sizes,
                                 const int32_t* offsets, const int32_t* source_order, int64_t T, int64_t K, int64_t H,
-                                int64_t I, int64_t E, void* packed_y, hipStream_t stream) {
+                                int64_t I, int64_t E, void* packed_y, hipStream_t stream, const SharedExperts* shared) {
   if (!fast_ok(act_full, down, nullptr, packed_y, I, H))
     return fail(JTMOE_EINVAL, "moe_forward: operands must be 16-byte aligned");
-  return launch_down_fast(act_full, down, group_sizes, offsets, T * K, H, I, E, packed_y, stream, source_order, (int)K,
-                          /*a_group_rows=*/T);
+  if (!shared)
+    return launch_down_fast(act_full, down, group_sizes, offsets, T * K, H, I, E, packed_y, stream, source_order, (int)K,
+                            /*a_group_rows=*/T);
+  const SkinnyProblem p = dense_skinny(shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, T, shared->Is, H,
+                                       BesideCfg::BM, BesideCfg::BN);
+  const Beside beside{p, (int)gemm_grid(p.mtiles, p.ntiles_n)};
+  bool taken = false;
+  const int rc = launch_down_fast(act_full, down, group_sizes, offsets, T * K, H, I, E, packed_y, stream, source_order,
+                                  (int)K, /*a_group_rows=*/T, &beside, &taken);
+  // (every kernel that reads blocks of rows per group takes the shared tiles along)
+  if (rc || taken) return rc;
+  return launch_down_fast(shared->act, shared->down, nullptr, nullptr, T, H, shared->Is, 1, shared->y, stream);
 }
 
 bool shared_in_skinny_tiles(const void* x, const SharedExperts& s, int64_t T, int64_t H) {

@@ -235,4 +235,45 @@ __global__ __launch_bounds__(Cfg::NT) __attribute__((amdgpu_waves_per_eu(Cfg::MI
   grouped_gemm_skinny_tile<Cfg>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
+// The shared experts' down product of a few tokens beside a routed product: its tiles are the launch's first
+// beside_blocks workgroups.  Neither needs the other's result, and either alone leaves CUs or bandwidth idle.
+using BesideCfg = SkinnyCfg<1, 2, false>;
+struct Beside {
+  SkinnyProblem p;
+  int blocks;  // a multiple of 8
+};
+
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) __attribute__((amdgpu_waves_per_eu(Cfg::MIN_WAVES_PER_EU))) void grouped_gemm_skinny_beside_kernel(
+    SkinnyProblem p, Beside beside) {
+  if ((int)blockIdx.x < beside.blocks)
+    grouped_gemm_skinny_tile<BesideCfg>(beside.p, (int)blockIdx.x, beside.blocks);
+  else
+    grouped_gemm_skinny_tile<Cfg>(p, (int)blockIdx.x - beside.blocks, (int)gridDim.x - beside.blocks);
+}
+
+// (three workgroups per CU: the streaming tile takes more registers than the 64-row one)
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) __attribute__((amdgpu_waves_per_eu(3))) void grouped_gemm_dma_beside_kernel(
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
+    uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E,
+    int rows, int Kdim, int N, int mtiles, int ntiles_n, const int32_t* __restrict__ row_map, int row_div, int a_rows,
+    uint16_t* __restrict__ save0, uint16_t* __restrict__ save1, int a_group_rows, Beside beside) {
+  if ((int)blockIdx.x < beside.blocks)
+    grouped_gemm_skinny_tile<BesideCfg>(beside.p, (int)blockIdx.x, beside.blocks);
+  else
+    grouped_gemm_dma_tile<Cfg>(A, B0, B1, C, group_sizes, offsets, E, rows, Kdim, N, mtiles, ntiles_n, row_map, row_div,
+                               a_rows, save0, save1, 0, a_group_rows, (int)blockIdx.x - beside.blocks,
+                               (int)gridDim.x - beside.blocks);
+}
+
+// One dense group of T rows.
+inline SkinnyProblem dense_skinny(const void* a, const void* b0, const void* b1, void* c, void* save0, void* save1,
+                                  int64_t T, int64_t Kdim, int64_t N, int BM, int BN) {
+  return SkinnyProblem{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b0),
+                       static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), static_cast<uint16_t*>(save0),
+                       static_cast<uint16_t*>(save1), nullptr, nullptr, nullptr, 1, (int)T, (int)Kdim, (int)N,
+                       (int)((T + BM - 1) / BM), (int)((N + BN - 1) / BN), 1, 0, 0};
+}
+
 }  // namespace jtmoe

@@ -1040,44 +1040,28 @@ inline size_t router_arrivals_offset(int64_t E) {
 // same at every replay, starts from zero as well.  No state outside the workspace: calls are as
 // re-entrant as their workspaces are distinct.
 // ---------------------------------------------------------------------------
-std::atomic<unsigned long long> g_decode_tag{0};
+std::atomic<unsigned long long> g_launch_tag{0};
 
-unsigned long long next_decode_tag() {
-  unsigned long long t = g_decode_tag.load(std::memory_order_relaxed);
+unsigned long long next_launch_tag() {
+  unsigned long long t = g_launch_tag.load(std::memory_order_relaxed);
   if (t == 0) {  // first use in this process
     std::random_device rd;
     unsigned long long seed = ((unsigned long long)rd() << 32) ^ rd() ^
                               (unsigned long long)std::chrono::steady_clock::now().time_since_epoch().count();
     unsigned long long expected = 0;
-    g_decode_tag.compare_exchange_strong(expected, seed | 1ull, std::memory_order_relaxed);
+    g_launch_tag.compare_exchange_strong(expected, seed | 1ull, std::memory_order_relaxed);
   }
-  t = g_decode_tag.fetch_add(1ull, std::memory_order_relaxed) & 0x00ffffffffffffffull;
+  t = g_launch_tag.fetch_add(1ull, std::memory_order_relaxed) & 0x00ffffffffffffffull;
   return (t == 0 ? 1ull : t) << 8;
 }
 
-template <int NB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void decode_gate_up_router_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ gate, const uint16_t* __restrict__ up,
-    uint16_t* __restrict__ act_full, int T, int H, int I, int mtiles, int ntiles_n,
-    const uint16_t* __restrict__ w_router, const float* __restrict__ bias, int K, float route_scale, int score_func,
-    int32_t* __restrict__ ids, bf16_raw* __restrict__ weights, float* __restrict__ scores,
-    float* __restrict__ counts, float* __restrict__ importance, int32_t* __restrict__ group_sizes,
-    int32_t* __restrict__ offsets, int32_t* __restrict__ source_order, int32_t* __restrict__ inverse,
-    float* __restrict__ partial, int token_blocks, int slices, unsigned long long* __restrict__ arrivals,
-    unsigned long long tag) {
-  constexpr int E = NB * 16;
-  const int router_blocks = token_blocks * slices;
-  if ((int)blockIdx.x >= router_blocks) {
-    grouped_gemm_dma_tile<GateUpTinyCfg>(x, gate, up, act_full, nullptr, nullptr, E, E * T, H, I, mtiles, ntiles_n,
-                                         nullptr, 1, 0, nullptr, nullptr, /*uniform_rows=*/T, 0,
-                                         (int)blockIdx.x - router_blocks, (int)gridDim.x - router_blocks);
-    return;
-  }
+using SharedGateUpCfg = SkinnyCfg<1, 2, true>;
+constexpr int kSharedFinishTokens = 64;  // the finishing workgroup has the tiles' 256 threads
+
+// Hand-over of the partial sums: true in all threads of the one workgroup that finds all others counted.
+__device__ __forceinline__ bool last_to_arrive(unsigned long long* arrivals, unsigned long long tag, int expected) {
   __shared__ int is_last;
-  const int token_block = (int)blockIdx.x % token_blocks, slice = (int)blockIdx.x / token_blocks;
-  router_split_body<NB, true, false>(x, w_router, bias, T, H, E, K, route_scale, ids, weights, scores, nullptr, nullptr, partial,
-                              score_func, token_block, slice);
-  // Hand-over.  Every thread waits until its own stores have reached the L2 (on this part stores count in
+  // Every thread waits until its own stores have reached the L2 (on this part stores count in
   // vmcnt); after the barrier one thread releases them to the device (the fence writes the L2's dirty
   // lines back, so that the other XCDs can see them) and counts the workgroup in.  The workgroup that
   // finds everyone else counted acquires with one fence (it invalidates this CU's L1 and the stale lines
@@ -1094,53 +1078,70 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
       count = (assumed >> 8) == (tag >> 8) ? (unsigned)(assumed & 0xffull) : 0u;
       seen = atomicCAS(arrivals, assumed, tag | (unsigned long long)(count + 1u));
     } while (seen != assumed);
-    is_last = count + 1u == (unsigned)router_blocks;
+    is_last = count + 1u == (unsigned)expected;
     if (is_last) __threadfence();
   }
   __syncthreads();
-  if (!is_last) return;
+  return is_last != 0;
+}
+
+template <int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void decode_gate_up_router_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ gate, const uint16_t* __restrict__ up,
+    uint16_t* __restrict__ act_full, int T, int H, int I, int mtiles, int ntiles_n,
+    const uint16_t* __restrict__ w_router, const float* __restrict__ bias, int K, float route_scale, int score_func,
+    int32_t* __restrict__ ids, bf16_raw* __restrict__ weights, float* __restrict__ scores,
+    float* __restrict__ counts, float* __restrict__ importance, int32_t* __restrict__ group_sizes,
+    int32_t* __restrict__ offsets, int32_t* __restrict__ source_order, int32_t* __restrict__ inverse,
+    float* __restrict__ partial, int token_blocks, int slices, unsigned long long* __restrict__ arrivals,
+    unsigned long long tag, SkinnyProblem shared, int shared_blocks) {
+  constexpr int E = NB * 16;
+  const int router_blocks = token_blocks * slices, block = (int)blockIdx.x - router_blocks;
+  if (block >= shared_blocks) {
+    grouped_gemm_dma_tile<GateUpTinyCfg>(x, gate, up, act_full, nullptr, nullptr, E, E * T, H, I, mtiles, ntiles_n,
+                                         nullptr, 1, 0, nullptr, nullptr, /*uniform_rows=*/T, 0,
+                                         block - shared_blocks, (int)gridDim.x - router_blocks - shared_blocks);
+    return;
+  }
+  if (block >= 0) {  // the shared experts' gate/up tiles
+    grouped_gemm_skinny_tile<SharedGateUpCfg>(shared, block, shared_blocks);
+    return;
+  }
+  const int token_block = (int)blockIdx.x % token_blocks, slice = (int)blockIdx.x / token_blocks;
+  router_split_body<NB, true, false>(x, w_router, bias, T, H, E, K, route_scale, ids, weights, scores, nullptr, nullptr, partial,
+                              score_func, token_block, slice);
+  if (!last_to_arrive(arrivals, tag, router_blocks)) return;
   router_finish_body<64, true>(partial, slices, bias, T, E, K, route_scale, ids, weights, scores, nullptr, counts,
                                importance, group_sizes, offsets, source_order, inverse, score_func);
   if (threadIdx.x == 0) *arrivals = 0ull;
 }
 
 // ---------------------------------------------------------------------------
-// The two launches of the small-batch router with the shared experts beside it: the gate/up tiles next to the
-// workgroups of the partial sums, the down tiles next to the finishing workgroup.  Each launch is bound by one
-// workgroup's own chain of dependent steps, on a few dozen CUs, and nothing of one is needed by the other.
-// One token, 2048 wide, 64 experts, shared 2816: 17.5 + 14.9 us, against 4.4 + 10.6 (router) and 18 + 13.5 (shared) in
-// four launches.
+// The small-batch router in one launch with the shared experts' gate/up tiles beside it.  The launch is bound by the
+// shared tiles (one token, 2048 wide, shared 2816: 17 us), under which both halves of the router fit (4.4 + 5 us; as
+// in the decode launch, the last workgroup to arrive finishes); the shared down tiles go beside the routed gate/up product
+// (BesideCfg).  As two launches, the finishing workgroup beside the shared down tiles, it took 17.5 + 14.9 us there.
 // ---------------------------------------------------------------------------
-using SharedGateUpCfg = SkinnyCfg<1, 2, true>;
-using SharedDownCfg = SkinnyCfg<1, 2, false>;
-constexpr int kSharedFinishTokens = 64;  // the finishing workgroup has the tiles' 256 threads
-
 template <int NB, bool kPad>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void router_shared_gate_up_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int tokens, int H, int E, int K, float* __restrict__ partial,
-    int token_blocks, int router_blocks, SkinnyProblem shared) {
-  const int block = (int)blockIdx.x;
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens, int H,
+    int E, int K, float route_scale, int score_func, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
+    float* __restrict__ scores, float* __restrict__ counts, float* __restrict__ importance,
+    int32_t* __restrict__ group_sizes, int32_t* __restrict__ offsets, int32_t* __restrict__ source_order,
+    int32_t* __restrict__ inverse, float* __restrict__ partial, int token_blocks, int slices,
+    unsigned long long* __restrict__ arrivals, unsigned long long tag, SkinnyProblem shared) {
+  const int block = (int)blockIdx.x, router_blocks = token_blocks * slices;
   if (block >= router_blocks) {
     grouped_gemm_skinny_tile<SharedGateUpCfg>(shared, block - router_blocks, (int)gridDim.x - router_blocks);
     return;
   }
-  router_split_body<NB, true, kPad>(x, w, nullptr, tokens, H, E, K, 1.0f, nullptr, nullptr, nullptr, nullptr, nullptr, partial, 0,
-                              block % token_blocks, block / token_blocks);
-}
-
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void router_finish_shared_down_kernel(
-    const float* __restrict__ partial, int slices, const float* __restrict__ bias, int tokens, int E, int K,
-    float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights, float* __restrict__ scores,
-    float* __restrict__ counts, float* __restrict__ importance, int32_t* __restrict__ group_sizes,
-    int32_t* __restrict__ offsets, int32_t* __restrict__ source_order, int32_t* __restrict__ inverse, int score_func,
-    SkinnyProblem shared) {
-  if (blockIdx.x > 0) {
-    grouped_gemm_skinny_tile<SharedDownCfg>(shared, (int)blockIdx.x - 1, (int)gridDim.x - 1);
-    return;
-  }
+  router_split_body<NB, true, kPad>(x, w, bias, tokens, H, E, K, route_scale, ids, weights, scores, nullptr, nullptr,
+                                    partial, score_func, block % token_blocks, block / token_blocks);
+  if (!last_to_arrive(arrivals, tag, router_blocks)) return;
   router_finish_body<kSharedFinishTokens, true>(partial, slices, bias, tokens, E, K, route_scale, ids, weights, scores,
                                                 nullptr, counts, importance, group_sizes, offsets, source_order,
                                                 inverse, score_func);
+  if (threadIdx.x == 0) *arrivals = 0ull;
 }
 
 template <typename KernelT>
@@ -1438,7 +1439,8 @@ int launch_decode_gate_up_router(const void* x, const void* w_router, const floa
                                  const void* up, void* act_full, int64_t T, int64_t H, int64_t E, int64_t K, int64_t I,
                                  double route_scale, int score_func, int32_t* expert_ids, void* weights, float* scores,
                                  float* expert_counts, float* importance, int32_t* group_sizes, int32_t* offsets,
-                                 int32_t* source_order, int32_t* inverse, void* router_workspace, hipStream_t stream) {
+                                 int32_t* source_order, int32_t* inverse, void* router_workspace, hipStream_t stream,
+                                 SharedExperts* shared) {
   if (!(aligned16(x) && aligned16(w_router) && aligned16(gate) && aligned16(up) && aligned16(act_full)))
     return fail(JTMOE_EINVAL, "moe_forward: operands must be 16-byte aligned");
   const int token_blocks = (int)((T + 15) / 16);
@@ -1451,11 +1453,19 @@ int launch_decode_gate_up_router(const void* x, const void* w_router, const floa
   if (smem > 53 * 1024) return fail(JTMOE_EUNSUPPORTED, "moe_forward: decode launch needs %zu bytes of LDS", smem);
   const int64_t mtiles = E * ((T + GateUpTinyCfg::BM - 1) / GateUpTinyCfg::BM);
   const int64_t nt = (I + GateUpTinyCfg::BN - 1) / GateUpTinyCfg::BN;
-  const int64_t grid = (int64_t)token_blocks * slices + gemm_grid(mtiles, nt);
+  SkinnyProblem shared_gu{};
+  int64_t shared_blocks = 0;
+  if (shared && shared_in_skinny_tiles(x, *shared, T, H)) {
+    shared_gu = dense_skinny(x, shared->gate, shared->up, shared->act, shared->gate_pre, shared->up_pre, T, H, shared->Is,
+                             SharedGateUpCfg::BM, SharedGateUpCfg::BN);
+    shared_blocks = gemm_grid(shared_gu.mtiles, shared_gu.ntiles_n);
+    shared->gate_up_done = true;
+  }
+  const int64_t grid = (int64_t)token_blocks * slices + shared_blocks + gemm_grid(mtiles, nt);
   if (token_blocks * slices > 255) return fail(JTMOE_EUNSUPPORTED, "moe_forward: decode launch with %d router workgroups", token_blocks * slices);
   unsigned long long* const arrivals = reinterpret_cast<unsigned long long*>(
       static_cast<unsigned char*>(router_workspace) + router_arrivals_offset(E));
-  const unsigned long long tag = next_decode_tag();
+  const unsigned long long tag = next_launch_tag();
 #define JT_DECODE_CASE(NB)                                                                                       \
   case NB * 16: {                                                                                                \
     auto kernel = decode_gate_up_router_kernel<NB>;                                                              \
@@ -1466,7 +1476,7 @@ int launch_decode_gate_up_router(const void* x, const void* w_router, const floa
         static_cast<uint16_t*>(act_full), (int)T, (int)H, (int)I, (int)mtiles, (int)nt,                          \
         static_cast<const uint16_t*>(w_router), expert_bias, (int)K, (float)route_scale, score_func, expert_ids, \
         static_cast<bf16_raw*>(weights), scores, expert_counts, importance, group_sizes, offsets, source_order,  \
-        inverse, partial, token_blocks, slices, arrivals, tag);                                                  \
+        inverse, partial, token_blocks, slices, arrivals, tag, shared_gu, (int)shared_blocks);                   \
   } break;
   switch ((int)E) {
     JT_DECODE_CASE(1)
@@ -1489,7 +1499,7 @@ static bool router_takes_shared(const void* x, const void* w_router, const Share
          router_smem_bytes((int)E, (int)K, kSharedFinishTokens) <= 160 * 1024 && shared_in_skinny_tiles(x, shared, T, H);
 }
 
-static int launch_router_with_shared(const void* x, const void* w_router, const float* bias, const SharedExperts& sh,
+static int launch_router_with_shared(const void* x, const void* w_router, const float* bias, SharedExperts& sh,
                                      int64_t T, int64_t H, int64_t E, int64_t K, double route_scale, int score_func,
                                      int32_t* ids, void* weights, float* scores, float* counts, float* importance,
                                      const LayerPlan& plan, void* ws, hipStream_t stream) {
@@ -1497,30 +1507,25 @@ static int launch_router_with_shared(const void* x, const void* w_router, const 
   const int slice_rows = router_slice_rows((int)H);
   const int slices = (int)((H + slice_rows - 1) / slice_rows);
   float* const partial = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + router_scratch_bytes(E));
-  auto problem = [&](const void* a, const void* b0, const void* b1, void* c, void* save0, void* save1, int64_t Kdim,
-                     int64_t N, int BM, int BN) {
-    return SkinnyProblem{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b0),
-                         static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), static_cast<uint16_t*>(save0),
-                         static_cast<uint16_t*>(save1), nullptr, nullptr, nullptr, 1, (int)T, (int)Kdim, (int)N,
-                         (int)((T + BM - 1) / BM), (int)((N + BN - 1) / BN), 1, 0, 0};
-  };
-  const SkinnyProblem gate_up = problem(x, sh.gate, sh.up, sh.act, sh.gate_pre, sh.up_pre, H, sh.Is, SharedGateUpCfg::BM,
-                                        SharedGateUpCfg::BN);
-  const SkinnyProblem down = problem(sh.act, sh.down, nullptr, sh.y, nullptr, nullptr, sh.Is, H, SharedDownCfg::BM,
-                                     SharedDownCfg::BN);
+  unsigned long long* const arrivals =
+      reinterpret_cast<unsigned long long*>(static_cast<unsigned char*>(ws) + router_arrivals_offset(E));
+  const SkinnyProblem gate_up = dense_skinny(x, sh.gate, sh.up, sh.act, sh.gate_pre, sh.up_pre, T, H, sh.Is,
+                                             SharedGateUpCfg::BM, SharedGateUpCfg::BN);
   const bool pad = router_padded(H, E);
   const size_t smem = std::max({router_split_smem_bytes((int)E, (int)K), router_split_smem_bytes(16 * router_column_blocks(E), 1),
-                                (size_t)SharedGateUpCfg::SMEM_BYTES});
-  const int router_blocks = token_blocks * slices;
-  const int64_t grid = router_blocks + gemm_grid(gate_up.mtiles, gate_up.ntiles_n);
-#define JT_SHARED_CASE(NB)                                                                                       \
-  case NB: {                                                                                                     \
-    auto kernel = pad ? &router_shared_gate_up_kernel<NB, true> : &router_shared_gate_up_kernel<NB, false>;      \
-    const int rc = set_max_smem(kernel, smem);                                                                   \
-    if (rc) return rc;                                                                                           \
-    kernel<<<(unsigned)grid, 256, smem, stream>>>(static_cast<const uint16_t*>(x),                               \
-                                                  static_cast<const uint16_t*>(w_router), (int)T, (int)H, (int)E, (int)K, \
-                                                  partial, token_blocks, router_blocks, gate_up);                \
+                                router_smem_bytes((int)E, (int)K, kSharedFinishTokens), (size_t)SharedGateUpCfg::SMEM_BYTES});
+  const int64_t grid = token_blocks * slices + gemm_grid(gate_up.mtiles, gate_up.ntiles_n);
+  const unsigned long long tag = next_launch_tag();
+#define JT_SHARED_CASE(NB)                                                                                        \
+  case NB: {                                                                                                      \
+    auto kernel = pad ? &router_shared_gate_up_kernel<NB, true> : &router_shared_gate_up_kernel<NB, false>;       \
+    const int rc = set_max_smem(kernel, smem);                                                                    \
+    if (rc) return rc;                                                                                            \
+    kernel<<<(unsigned)grid, 256, smem, stream>>>(                                                                \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w_router), bias, (int)T, (int)H, (int)E,    \
+        (int)K, (float)route_scale, score_func, ids, static_cast<bf16_raw*>(weights), scores, counts, importance, \
+        plan.group_sizes, plan.offsets, plan.source_order, plan.inverse, partial, token_blocks, slices, arrivals, \
+        tag, gate_up);                                                                                            \
   } break;
   switch (router_column_blocks(E)) {
     JT_SHARED_CASE(1)
@@ -1530,13 +1535,7 @@ static int launch_router_with_shared(const void* x, const void* w_router, const 
     JT_SHARED_CASE(16)
   }
 #undef JT_SHARED_CASE
-  const size_t fsmem =
-      std::max(router_smem_bytes((int)E, (int)K, kSharedFinishTokens), (size_t)SharedDownCfg::SMEM_BYTES);
-  const int rc = set_max_smem(&router_finish_shared_down_kernel, fsmem);
-  if (rc) return rc;
-  router_finish_shared_down_kernel<<<(unsigned)(1 + gemm_grid(down.mtiles, down.ntiles_n)), 256, fsmem, stream>>>(
-      partial, slices, bias, (int)T, (int)E, (int)K, (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores,
-      counts, importance, plan.group_sizes, plan.offsets, plan.source_order, plan.inverse, score_func, down);
+  sh.gate_up_done = true;
   return check_launch("router and shared experts");
 }
 
@@ -1545,7 +1544,7 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
                      float* expert_counts, float* importance, int32_t* group_sizes, int32_t* offsets,
                      int32_t* source_order, int32_t* inverse, void* workspace, size_t workspace_bytes,
                      int score_func, bool* stats_done, bool* plan_done, hipStream_t s, void* scratch,
-                     size_t scratch_bytes, const SharedExperts* shared, bool* shared_done) {
+                     size_t scratch_bytes, SharedExperts* shared) {
   int rc = validate_router(T, H, E, K, route_scale, dtype, true);
   if (rc) return rc;
   JT_REQUIRE(score_func_ok(score_func), "router: unknown score function %d", score_func);
@@ -1556,7 +1555,7 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
     return fail(JTMOE_EWORKSPACE, "router: workspace %zu < %zu bytes", workspace_bytes, jtmoe_router_workspace_bytes(E));
   LayerPlan layer{group_sizes, offsets, source_order, inverse, false, false, scratch, scratch_bytes};
   if (shared && router_takes_shared(x, w_router, *shared, T, H, E, K, dtype)) {
-    *stats_done = *plan_done = *shared_done = true;
+    *stats_done = *plan_done = true;
     return launch_router_with_shared(x, w_router, expert_bias, *shared, T, H, E, K, route_scale, score_func, expert_ids,
                                      weights, scores, expert_counts, importance, layer, workspace, s);
   }
