@@ -15,12 +15,22 @@
 // any assignment of k to products serves as long as both operands use it).  Row-major tiles ([k][n]) are read
 // one word per MFMA, 32 consecutive words per half wave.
 // Two tile heights and widths (128 and 64): the launcher takes the one with the fewer rounds over the CUs.
-// Three or four stages instead of two measured the same or slower (101 / 108 / 129 us for the gate/up product
-// below): the loads arrive in time, and the LDS is better spent on more workgroups per CU.
-// Measured at 4096 rows in 8 groups, 512 x 1024: gate/up 199 -> 100 us, down 211 -> 61, data gradients
-// 143 -> 54 and 424 -> 115, weight gradients 147 -> 47 and 154 + 145 -> 83 (one launch); 52 to 103 TFLOP/s of
-// matrix work where the element-wise staged kernels, which still take other widths, reached 10 to 59.  What is
-// left is the last, partly filled round and the fixed cost of launches this short.
+// Three stages instead of two measured the same (46.4 against 45.6 us for a product of 4096 rows in one group, K = 1024,
+// N = 512): the loads arrive in time, and the LDS is better spent on more workgroups per CU.
+// What costs rate beside the products, and what is done about it in the two forms with a row per group row:
+//   - the accumulators have to stay where they are.  A wave that skips its products inside the step loop makes the
+//     compiler carry them through ordinary registers, a write and a read of each per step: 16 to 64 writes among 16 to 64
+//     products.  The waves without rows have a loop of their own instead (4096 rows in one group, K = 4096, N = 512:
+//     168.9 -> 162.5 us; gate/up with K = 2048, N = 1024: 270.7 -> 253.4).
+//   - the first fragments of a step are requested in front of the last products of the one before (162.5 -> 159.8).
+//   - 64-row tiles, whose steps are short: the loads lie between those products.  In one piece behind the barrier the
+//     loads of all waves queue up and hold the products back (159.8 -> 150.9).  In the tiles with four blocks per wave
+//     that costs 2 % (gate/up above 253 -> 259).
+// Measured at 4096 rows in 8 groups, 512 x 1024: gate/up 100.5 -> 95.4 us, down 60.8 -> 56.1, data gradients 54.2 -> 52.1
+// and 114.6 -> 107.9, weight gradients 47 and 83 (one launch); the element-wise staged kernels, which still take other
+// widths, 143 to 424.  What is left is the last, partly filled round (2.1 rounds of tiles for the down product) and
+// the fixed cost of launches this short; with long reductions the large tiles reach 136 TFLOP/s of the 154 that the
+// matrix cores reach from registers.
 //
 // Requirements: K, N (KA) multiples of 4, 16-byte aligned pointers, operands of a group below 2 GiB.
 #pragma once
@@ -40,6 +50,7 @@ struct F32Cfg {
   static constexpr int SMEM_BYTES = 2 * STAGE_BYTES;
   static constexpr int A_LOADS = BM * 8 / NT, B_LOADS = BN * 8 / NT;
   static constexpr int GROUP_M = 4;
+  static constexpr bool kSpread = BM == 64;  // the loads lie between the products
   static_assert(BM % 64 == 0 && BN % 64 == 0 && !(kDual && (kBT || BN != 64)), "2 x 2 waves of 32 x 32 blocks");
 };
 
@@ -98,31 +109,31 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_f32_kernel(
     const int src = gather && r < tr.rows ? row_map[tr.row0 + r] / row_div : r;
     a_voff[j] = r < tr.rows ? (src * Kdim + l_c * 4) * 4 : kOutside;
   }
+  int b_voff[Cfg::B_LOADS];
+#pragma unroll
+  for (int j = 0; j < Cfg::B_LOADS; ++j) {
+    const int c = tid + j * NT;
+    b_voff[j] = kBT ? ((n0 + l_r + j * 32) * Kdim + l_c * 4) * 4 : (c / (BN / 4) * N + n0 + c % (BN / 4) * 4) * 4;
+  }
   const unsigned wave_lds = lds_byte_addr(smem_raw) + wave * 1024;
-  const int nk1 = (Kdim + BK - 1) / BK, nk = nk1 * segs;
-  auto issue = [&](int kt) {
-    const unsigned base = wave_lds + (kt & 1) * Cfg::STAGE_BYTES;
+  const int nk1 = (Kdim + BK - 1) / BK, nk = max(nk1 * segs, 1);
+  constexpr int LOADS = Cfg::A_LOADS + Cfg::NSUB * Cfg::B_LOADS;
+  // load `i` of step kt; past the last step everything lies outside and reads as zeros
+  auto issue = [&](int kt, int i) {
+    const unsigned base = __builtin_amdgcn_readfirstlane(wave_lds + (kt & 1) * Cfg::STAGE_BYTES);
     const bool second = kt >= nk1;
     const int k0 = (second ? kt - nk1 : kt) * BK;
-    const bool past_k = k0 + l_c * 4 >= Kdim;  // this lane's chunk lies past the end of a row
-#pragma unroll
-    for (int j = 0; j < Cfg::A_LOADS; ++j)
-      f32_load(second ? a_rsrc1 : a_rsrc0, base + j * NT * 16, past_k ? kOutside : a_voff[j] + k0 * 4);
-    if constexpr (kBT) {
-#pragma unroll
-      for (int j = 0; j < Cfg::B_LOADS; ++j)
-        f32_load(second ? b_rsrc1 : b_rsrc0, base + Cfg::A_BYTES + j * NT * 16,
-                 past_k ? kOutside : ((n0 + l_r + j * 32) * Kdim + k0 + l_c * 4) * 4);
-    } else {
-#pragma unroll
-      for (int u = 0; u < Cfg::NSUB; ++u)
-#pragma unroll
-        for (int j = 0; j < Cfg::B_LOADS; ++j) {
-          const int s = tid + j * NT, k = s / (BN / 4), c = s % (BN / 4);
-          f32_load(u ? b_rsrc1 : b_rsrc0, base + Cfg::A_BYTES + u * Cfg::B_BYTES + j * NT * 16,
-                   ((k0 + k) * N + n0 + c * 4) * 4);
-        }
+    const bool past_k = kt >= nk || k0 + l_c * 4 >= Kdim;  // this lane's chunk lies past the end of a row
+    if (i < Cfg::A_LOADS) {
+      f32_load(second ? a_rsrc1 : a_rsrc0, base + i * NT * 16, past_k ? kOutside : a_voff[i] + k0 * 4);
+      return;
     }
+    const int u = (i - Cfg::A_LOADS) / Cfg::B_LOADS, j = (i - Cfg::A_LOADS) % Cfg::B_LOADS;
+    const unsigned to = base + Cfg::A_BYTES + u * Cfg::B_BYTES + j * NT * 16;
+    if (kBT)
+      f32_load(second ? b_rsrc1 : b_rsrc0, to, past_k ? kOutside : b_voff[j] + k0 * 4);
+    else
+      f32_load(u ? b_rsrc1 : b_rsrc0, to, kt >= nk ? kOutside : b_voff[j] + k0 * N * 4);
   };
 
   f32x16_t acc[TM][TN];
@@ -155,36 +166,69 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_f32_kernel(
       }
     }
   };
-  // (the fragments of the next sub-step are requested before the products of this one are issued, and the
-  // scheduling barriers keep it so: left alone the compiler reads each sub-step's fragments right in front of
-  // its products and the wave waits for the LDS every time, 1 to 4 % of the run time)
-  auto compute = [&](int kt) {
-    const unsigned char* st = smem_raw + (kt & 1) * Cfg::STAGE_BYTES;
-    f32x4 a[2][TM], b[2][TN];
-    load_frags(st, 0, a[0], b[0]);
+  // (the scheduling barriers keep the fragments' requests in front of the products, under which they arrive, and spread
+  // loads between them)
+  f32x4 a[2][TM], b[2][TN];
+  auto products = [&](int set, bool loads, int kt) {  // with `loads`: and the loads of step kt
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < BK / 8; ++q) {
-      if (q + 1 < BK / 8) load_frags(st, q + 1, a[(q + 1) & 1], b[(q + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < 4; ++i) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
-        for (int mi = 0; mi < TM; ++mi)
+        for (int jj = 0; jj < TN; ++jj)
+          acc[mi][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[set][mi][i], b[set][jj][i], acc[mi][jj], 0, 0, 0);
+      if (loads) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int jj = 0; jj < TN; ++jj)
-            acc[mi][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q & 1][mi][i], b[q & 1][jj][i], acc[mi][jj], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int j = LOADS * i / 4; j < LOADS * (i + 1) / 4; ++j) issue(kt, j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  const bool wave_has_work = wm * 32 * TM < tr.rows;  // rows past the end of the group: loads and barriers only
-  issue(0);
-  for (int kt = 0; kt < nk; ++kt) {
+  constexpr int QS = BK / 8;
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) issue(0, i);
+  wait_and_barrier<0>();
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) issue(1, i);
+  if (wm * 32 * TM >= tr.rows) {  // rows past the end of the group: loads and barriers only
+    for (int kt = 0; kt + 1 < nk; ++kt) {
+      wait_and_barrier<0>();
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) issue(kt + 2, i);
+    }
     wait_vmcnt<0>();
-    __syncthreads();
-    if (kt + 1 < nk) issue(kt + 1);
-    if (wave_has_work) compute(kt);
+    return;
   }
+  load_frags(smem_raw, 0, a[0], b[0]);
+  for (int kt = 0; kt + 1 < nk; ++kt) {
+    const unsigned char* st = smem_raw + (kt & 1) * Cfg::STAGE_BYTES;
+#pragma unroll
+    for (int q = 0; q < QS - 1; ++q) {
+      load_frags(st, q + 1, a[(q + 1) & 1], b[(q + 1) & 1]);
+      products(q & 1, false, 0);
+    }
+    // all waves have read stage kt and their loads of stage kt + 1 are there: its first fragments are on their way
+    // while the last products of this step run
+    wait_and_barrier<0>();
+    if (!Cfg::kSpread && kt + 2 < nk) {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) issue(kt + 2, i);
+    }
+    load_frags(smem_raw + ((kt + 1) & 1) * Cfg::STAGE_BYTES, 0, a[0], b[0]);
+    products((QS - 1) & 1, Cfg::kSpread, kt + 2);
+  }
+  {
+    const unsigned char* st = smem_raw + ((nk - 1) & 1) * Cfg::STAGE_BYTES;
+#pragma unroll
+    for (int q = 0; q < QS; ++q) {
+      if (q + 1 < QS) load_frags(st, q + 1, a[(q + 1) & 1], b[(q + 1) & 1]);
+      products(q & 1, false, 0);
+    }
+  }
+  wait_vmcnt<0>();  // the loads past the last step
 
   // value i of lane l of a block is row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32: the 32 lanes of a
   // half wave store 128 contiguous bytes
