@@ -351,23 +351,29 @@ int experts_backward_core(const void* x, const void* dy, const int32_t* source_o
                            : run_swiglu_backward<float>(ws.dg, gate_pre, up_pre, source_order, weights, A, I, ws.du,
                                                         ws.hw, d_weights, s, group_sizes, offsets, E);
   if (rc) return rc;
-  // dWd[e] = (w Hh)^T @ dYp
-  rc = launch_gemm_tn(dtype, ws.hw, ws.packed_dy, nullptr, d_down, nullptr, group_sizes, offsets, A, I, H, E, nullptr,
-                      1, false, false, 0, s);
-  if (rc) return rc;
-  // dWg[e], dWu[e] = Xp^T @ (dG, dU)
-  rc = launch_gemm_tn(dtype, ws.packed_x, ws.dg, ws.du, d_gate, d_up, group_sizes, offsets, A, H, I, E, nullptr, 1,
-                      false, false, 0, s);
-  if (rc) return rc;
-  if (joint_dx) {
-    rc = shared_backward_steps(x, dy, *shared, T, H, dtype, !joint_z, false, s);
+  const F32Backward products{ws.dg, ws.du, ws.hw, ws.packed_x, ws.packed_dy, gate, up, ws.dxp, d_gate, d_up, d_down};
+  if (dtype == JTMOE_F32 && f32_backward_products_supported(products, A, H, I, E)) {
+    rc = launch_f32_backward_products(products, group_sizes, offsets, A, H, I, E, s);
+    if (rc) return rc;
+  } else {
+    // dWd[e] = (w Hh)^T @ dYp
+    rc = launch_gemm_tn(dtype, ws.hw, ws.packed_dy, nullptr, d_down, nullptr, group_sizes, offsets, A, I, H, E, nullptr,
+                        1, false, false, 0, s);
+    if (rc) return rc;
+    // dWg[e], dWu[e] = Xp^T @ (dG, dU)
+    rc = launch_gemm_tn(dtype, ws.packed_x, ws.dg, ws.du, d_gate, d_up, group_sizes, offsets, A, H, I, E, nullptr, 1,
+                        false, false, 0, s);
+    if (rc) return rc;
+    if (joint_dx) {
+      rc = shared_backward_steps(x, dy, *shared, T, H, dtype, !joint_z, false, s);
+      if (rc) return rc;
+    }
+    // dXp = dG @ Wg[e]^T + dU @ Wu[e]^T
+    rc = joint_dx ? launch_gemm_nt_joint(dtype, routed_dx, group_sizes, offsets, E, shared_dx, 2, s)
+                  : launch_gemm_nt(dtype, ws.dg, ws.du, gate, up, ws.dxp, group_sizes, offsets, A, I, H, E, nullptr, 1, 0,
+                                   2, s);
     if (rc) return rc;
   }
-  // dXp = dG @ Wg[e]^T + dU @ Wu[e]^T
-  rc = joint_dx ? launch_gemm_nt_joint(dtype, routed_dx, group_sizes, offsets, E, shared_dx, 2, s)
-                : launch_gemm_nt(dtype, ws.dg, ws.du, gate, up, ws.dxp, group_sizes, offsets, A, I, H, E, nullptr, 1, 0,
-                                 2, s);
-  if (rc) return rc;
   if (shared && !joint_dx) {
     rc = shared_backward_steps(x, dy, *shared, T, H, dtype, !joint_z, true, s);
     if (rc) return rc;

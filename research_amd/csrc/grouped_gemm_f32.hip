@@ -142,4 +142,43 @@ int launch_f32_tn(const void* p_, const void* d0_, const void* d1_, void* c0_, v
   return launch_f32_tn<64, 64>(p, d0, d1, c0, c1, group_sizes, offsets, rows, KA, N, E, 0, stream);
 }
 
+// One launch where it saves work in the last rounds of three.  Cost in k steps of a 64 x 64 tile per CU: the launches of
+// their own in whole rounds of the tiles they take, the joint one spread evenly, but no shorter than its longest tile.
+// The weight gradients' large tiles are the faster ones as long as rounds are full (131 against 114 TFLOP/s), so a tenth
+// has to be saved.  4096 rows in 8 groups, 512 x 1024 (10496 against 12288 steps): 192 us against 238 for the three;
+// twice the rows (20736 against 22528) keep launches of their own.
+bool f32_backward_joint(int64_t rows, int64_t H, int64_t I, int64_t E) {
+  const int64_t cus = persistent_grid_size(), depth = std::max<int64_t>(rows / std::max<int64_t>(E, 1), 1);
+  const auto tn = [&](int64_t matrices) {
+    const int64_t big = matrices * E * ((H + 127) / 128) * ((I + 127) / 128);
+    const int64_t small = matrices * E * ((H + 63) / 64) * ((I + 63) / 64);
+    return std::min((big + cus - 1) / cus * 4, (small + cus - 1) / cus) * depth;
+  };
+  const int64_t apart =
+      std::min(f32_cost(false, rows, E, H, 128, 128, 4), f32_cost(false, rows, E, H, 64, 64, 1)) * 2 * I + tn(2) + tn(1);
+  const int64_t mt = (rows + 63) / 64 + std::min(E, rows) / 2, th = (H + 63) / 64, ti = (I + 63) / 64;
+  const int64_t joint = std::max((mt * th * 2 * I + 3 * E * th * ti * depth + cus - 1) / cus, 2 * I);
+  return joint * 10 <= apart * 9;
+}
+
+bool f32_backward_products_supported(const F32Backward& b, int64_t rows, int64_t H, int64_t I, int64_t E) {
+  const int64_t grid = gemm_grid(f32_mtiles(false, rows, E, 64), (H + 63) / 64) + 3 * E * ((H + 63) / 64) * ((I + 63) / 64);
+  return rows > 0 && rows * H < kF32Limit && grid < ((int64_t)1 << 31) && aligned16(b.hw) && aligned16(b.dyp) &&
+         f32_gemm_supported(b.dg, b.du, b.gate, b.up, b.dxp, rows, I, H) &&
+         f32_gemm_supported(b.xp, b.d_gate, b.d_up, b.d_down, nullptr, rows, H, I) && f32_backward_joint(rows, H, I, E);
+}
+
+int launch_f32_backward_products(const F32Backward& b, const int32_t* group_sizes, const int32_t* offsets, int64_t rows,
+                                 int64_t H, int64_t I, int64_t E, hipStream_t stream) {
+  const int64_t th = (H + 63) / 64, ti = (I + 63) / 64, mtiles = f32_mtiles(false, rows, E, 64);
+  const int64_t dx_blocks = gemm_grid(mtiles, th), grid = dx_blocks + 3 * E * th * ti;
+  const auto in = [](const void* p) { return static_cast<const float*>(p); };
+  const auto out = [](void* p) { return static_cast<float*>(p); };
+  const F32BackwardProducts p{in(b.dg),   in(b.du),      in(b.hw),    in(b.xp),     in(b.dyp),   in(b.gate), in(b.up),
+                              out(b.dxp), out(b.d_gate), out(b.d_up), out(b.d_down), group_sizes, offsets,    (int)rows,
+                              (int)H,     (int)I,        (int)E,      (int)mtiles,  (int)dx_blocks};
+  grouped_gemm_f32_backward_kernel<<<(unsigned)grid, 256, F32Cfg<64, 64, false, true>::SMEM_BYTES, stream>>>(p);
+  return check_launch("experts backward (f32 products)");
+}
+
 }  // namespace jtmoe

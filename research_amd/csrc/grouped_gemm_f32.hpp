@@ -27,7 +27,7 @@
 //     loads of all waves queue up and hold the products back (159.8 -> 150.9).  In the tiles with four blocks per wave
 //     that costs 2 % (gate/up above 253 -> 259).
 // Measured at 4096 rows in 8 groups, 512 x 1024: gate/up 100.5 -> 95.4 us, down 60.8 -> 56.1, data gradients 54.2 -> 52.1
-// and 114.6 -> 107.9, weight gradients 47 and 83 (one launch); the element-wise staged kernels, which still take other
+// and 114.6 -> 107.9, weight gradients 47 and 83 in launches of their own; the element-wise staged kernels, which still take other
 // widths, 143 to 424.  What is left is the last, partly filled round (2.1 rounds of tiles for the down product) and
 // the fixed cost of launches this short; with long reductions the large tiles reach 136 TFLOP/s of the 154 that the
 // matrix cores reach from registers.
@@ -60,26 +60,26 @@ __device__ __forceinline__ void f32_load(i32x4_t rsrc, unsigned base, int voffse
   buffer_load_lds16(rsrc, base, voffset, 0);
 }
 
+// (block / blocks: this workgroup's index among those that share out the tiles, and their number, a multiple of 8)
 template <typename Cfg>
-__global__ __launch_bounds__(Cfg::NT) void grouped_gemm_f32_kernel(
-    const float* __restrict__ A0, const float* __restrict__ A1, const float* __restrict__ B0,
-    const float* __restrict__ B1, float* __restrict__ C, const int32_t* __restrict__ group_sizes,
-    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n,
-    const int32_t* __restrict__ row_map, int row_div, int a_rows, int segs, float* __restrict__ save0,
-    float* __restrict__ save1) {
+__device__ __forceinline__ void f32_rows_body(
+    int block, int blocks, unsigned char* smem_raw, const float* __restrict__ A0, const float* __restrict__ A1,
+    const float* __restrict__ B0, const float* __restrict__ B1, float* __restrict__ C,
+    const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N,
+    int mtiles, int ntiles_n, const int32_t* __restrict__ row_map, int row_div, int a_rows, int segs,
+    float* __restrict__ save0, float* __restrict__ save1) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, TM = Cfg::TM, TN = Cfg::TN;
   constexpr bool kDual = Cfg::kDual, kBT = Cfg::kBT;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
 
   TileCoord tc;
   TileRows tr;
   if (group_sizes) {
     const GroupScan scan = group_scan(BM, group_sizes, E);
-    tc = xcd_tile_order_balanced(scan.total, ntiles_n, Cfg::GROUP_M);
+    tc = xcd_tile_order_balanced(scan.total, ntiles_n, Cfg::GROUP_M, block);
     if (tc.mt < 0) return;
     tr = locate_tile(scan, tc.mt, BM, offsets);
   } else {
-    tc = xcd_tile_order(mtiles, ntiles_n, Cfg::GROUP_M);
+    tc = xcd_tile_order(mtiles, ntiles_n, Cfg::GROUP_M, block, blocks);
     if (tc.mt < 0) return;
     tr = find_tile_wave(tc.mt, BM, nullptr, nullptr, E, dense_rows);
   }
@@ -257,19 +257,31 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_f32_kernel(
     }
 }
 
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) void grouped_gemm_f32_kernel(
+    const float* __restrict__ A0, const float* __restrict__ A1, const float* __restrict__ B0,
+    const float* __restrict__ B1, float* __restrict__ C, const int32_t* __restrict__ group_sizes,
+    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n,
+    const int32_t* __restrict__ row_map, int row_div, int a_rows, int segs, float* __restrict__ save0,
+    float* __restrict__ save1) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  f32_rows_body<Cfg>((int)blockIdx.x, (int)gridDim.x, smem_raw, A0, A1, B0, B1, C, group_sizes, offsets, E, dense_rows,
+                     Kdim, N, mtiles, ntiles_n, row_map, row_div, a_rows, segs, save0, save1);
+}
+
 // Weight gradients.  One workgroup per (matrix, group, tile); D1 / C1 (if `matrices` is 2) is a second
 // product with the same P.  split_chunk > 0 (one dense group): "group" e is the e-th run of split_chunk rows
 // and C holds partial sums [matrix][E][KA, N] that the caller adds up in order.
 template <int BMO, int BNO>
-__global__ __launch_bounds__(256) void grouped_gemm_f32_tn_kernel(
-    const float* __restrict__ P, const float* __restrict__ D0, const float* __restrict__ D1, float* __restrict__ C0,
-    float* __restrict__ C1, const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E,
-    int dense_rows, int KA, int N, int mtiles_o, int ntiles_o, int split_chunk) {
+__device__ __forceinline__ void f32_tn_body(int block, unsigned char* smem_raw, const float* __restrict__ P,
+                                            const float* __restrict__ D0, const float* __restrict__ D1,
+                                            float* __restrict__ C0, float* __restrict__ C1,
+                                            const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets,
+                                            int E, int dense_rows, int KA, int N, int mtiles_o, int ntiles_o,
+                                            int split_chunk) {
   constexpr int BK = 32, NT = 256, TM = BMO / 64, TN = BNO / 64;
   constexpr int P_BYTES = BK * BMO * 4, STAGE_BYTES = P_BYTES + BK * BNO * 4;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
   const int per_group = mtiles_o * ntiles_o;
-  int block = (int)blockIdx.x;
   const int which = block / (E * per_group);
   block -= which * E * per_group;
   const int e = block / per_group;
@@ -358,6 +370,45 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_tn_kernel(
         if (r < KA && col < N) Ce[(size_t)r * N + col] = acc[mi][jj][i];
       }
     }
+}
+
+template <int BMO, int BNO>
+__global__ __launch_bounds__(256) void grouped_gemm_f32_tn_kernel(
+    const float* __restrict__ P, const float* __restrict__ D0, const float* __restrict__ D1, float* __restrict__ C0,
+    float* __restrict__ C1, const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E,
+    int dense_rows, int KA, int N, int mtiles_o, int ntiles_o, int split_chunk) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  f32_tn_body<BMO, BNO>((int)blockIdx.x, smem_raw, P, D0, D1, C0, C1, group_sizes, offsets, E, dense_rows, KA, N,
+                        mtiles_o, ntiles_o, split_chunk);
+}
+
+// The three products behind the SwiGLU's backward pass, none of which needs another's result, in one launch of 64 x 64
+// tiles: dXp = dG Wg^T + dU Wu^T first, whose tiles are the longest, then dWg = Xp^T dG, dWu = Xp^T dU and
+// dWd = HW^T dYp.  Launches of their own each end in a round that is partly empty: at 4096 rows in 8 groups, 512 x 1024,
+// 108 + 83 + 47 us (2.1 rounds of tiles for dXp, and two and one of the large tiles of the weight gradients at 102 and
+// 92 TFLOP/s), 192 us in one.
+struct F32BackwardProducts {
+  const float *dg, *du, *hw, *xp, *dyp, *gate, *up;  // [rows, I] x 3, [rows, H] x 2, [E, H, I] x 2
+  float *dxp, *d_gate, *d_up, *d_down;               // [rows, H], [E, H, I] x 2, [E, I, H]
+  const int32_t *group_sizes, *offsets;
+  int rows, H, I, E, mtiles, dx_blocks;  // m-tiles and workgroups of dXp
+};
+
+__global__ __launch_bounds__(256) void grouped_gemm_f32_backward_kernel(F32BackwardProducts p) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int th = (p.H + 63) / 64, ti = (p.I + 63) / 64, per_matrix = p.E * th * ti;
+  int block = (int)blockIdx.x;
+  if (block < p.dx_blocks) {
+    f32_rows_body<F32Cfg<64, 64, false, true>>(block, p.dx_blocks, smem_raw, p.dg, p.du, p.gate, p.up, p.dxp,
+                                               p.group_sizes, p.offsets, p.E, p.rows, p.I, p.H, p.mtiles, th, nullptr, 1,
+                                               0, 2, nullptr, nullptr);
+    return;
+  }
+  block -= p.dx_blocks;
+  const bool down = block >= 2 * per_matrix;
+  f32_tn_body<64, 64>(down ? block - 2 * per_matrix : block, smem_raw, down ? p.hw : p.xp, down ? p.dyp : p.dg, p.du,
+                      down ? p.d_down : p.d_gate, p.d_up, p.group_sizes, p.offsets, p.E, p.rows, down ? p.I : p.H,
+                      down ? p.H : p.I, down ? ti : th, down ? th : ti, 0);
 }
 
 }  // namespace jtmoe

@@ -60,3 +60,36 @@ def test_f32_shared_experts_with_split_reductions(gpu, tokens, hidden, inter):
     for g, a, ref in zip(got, again, want):
         assert torch.equal(g, a)
         assert P.report("f32 shared", host(g), ref.numpy().astype(np.float32)) <= bar
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,inter,joint", [
+    (3, 4, 5, 4, True),         # one chunk, groups of at most three rows, two of them empty
+    (300, 260, 5, 132, True),   # columns one chunk past a tile; a group without rows between groups with some
+    (700, 132, 16, 68, True),   # short reductions, most tiles partly filled
+    (2048, 512, 8, 1024, True),
+    (8192, 512, 8, 1024, False),  # the launches of their own, whose rounds are nearly full
+])
+def test_f32_backward_products_in_one_launch(gpu, tokens, hidden, experts, inter, joint):
+    """dXp and the three weight gradients with uneven groups and empty ones, against float64; each gradient has the
+    bits that the data gradients and weight gradients of a second call have."""
+    rng = np.random.default_rng(tokens + hidden)
+    share = np.where(np.arange(experts) % 4 == 1, 0.0, 1.0 + np.arange(experts) ** 2)
+    first = rng.choice(experts, tokens, p=share / share.sum())
+    ids = first.astype(np.int32)[:, None]
+    x, dy = (rng.standard_normal((tokens, hidden)).astype(np.float32) for _ in range(2))
+    w = rng.uniform(0.5, 1.0, (tokens, 1)).astype(np.float32)
+    gate, up = ((rng.standard_normal((experts, hidden, inter)) * 0.1).astype(np.float32) for _ in range(2))
+    down = (rng.standard_normal((experts, inter, hidden)) * 0.1).astype(np.float32)
+    got, _ = G.expert_grads(gpu, x, ids, w, gate, up, down, dy, "f32")
+    again, _ = G.expert_grads(gpu, x, ids, w, gate, up, down, dy, "f32")
+    leaves = [torch.from_numpy(a.astype(np.float64)).requires_grad_() for a in (x, gate, up, down)]
+    y = torch.zeros(tokens, hidden, dtype=torch.float64)
+    for e in range(experts):
+        rows = torch.from_numpy(np.flatnonzero(first == e))
+        h = torch.nn.functional.silu(leaves[0][rows] @ leaves[1][e]) * (leaves[0][rows] @ leaves[2][e])
+        y = y.index_put((rows,), (h @ leaves[3][e]) * torch.from_numpy(w[rows].astype(np.float64)))
+    want = torch.autograd.grad(y, leaves, torch.from_numpy(dy.astype(np.float64)))
+    bar = 2.0 ** -23 * 8 * np.sqrt(max(hidden, inter, tokens))
+    for name, ref in zip(("dx", "d_gate", "d_up", "d_down"), want):
+        assert torch.equal(getattr(got, name), getattr(again, name)), name
+        assert P.report(f"f32 {name}", host(getattr(got, name)), ref.numpy().astype(np.float32)) <= bar, name
