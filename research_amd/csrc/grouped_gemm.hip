@@ -337,6 +337,8 @@ int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const 
 // tiles are resident, three to a CU (8 tokens, 64 experts 48 against 56), and where the LDS tiles start that round (12
 // and 20 tokens, 128 experts 41 and 52 against 56 and 58; 37 with two thirds of the experts reached 39 against 55;
 // balanced 63 against 62), but not in between (15 tokens, 64 experts 63 against 54).
+// (These lines were drawn with three and two of the 64-row LDS tiles on a CU; four are resident now.
+// They have not been drawn again; what the fourth gave, the LDS tiles' side of them gained.)
 inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dual, double cus, ProductKernel* out) {
   struct Shape {
     ProductKernel id;
