@@ -243,7 +243,7 @@ __device__ __forceinline__ void select_all(const RouterSmem& sm, int nrows, int 
   constexpr int kGroups = kRouterThreads / 16;
   static_assert(4 * kRouterTokens <= kRouterThreads, "four lanes to a token");
   const int tid = threadIdx.x;
-  if (kRouterTokens > 2 * kGroups && kRouterThreads < 1024 && nrows > 2 * kGroups &&
+  if (kRouterTokens > 2 * kGroups && kRouterThreads < 1024 &&
       (E == 16 || E == 32 || E == 64 || E == 128 || E == 256)) {
     const int t = tid >> 2, q = tid & 3, e_begin = q * (E >> 2);
     const bool row_ok = t < nrows;
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
     int H, int width, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ logits_out, void* ws, int score_func) {
   constexpr int kRouterTokens = 16 * NW, kRouterThreads = 64 * NW;
-  const int slice_chunks = (router_slice_rows(H) + kRouterKC - 1) / kRouterKC;  // 64-row chunks per slice
+  const int slice_chunks = (router_slice_rows(H) + (kPad ? kRouterKC - 1 : 0)) / kRouterKC;  // 64-row chunks per slice
   constexpr int EC = NB * 16;
   const int E = kPad ? width : EC;
   constexpr int WS = EC + 32;                     // LDS row stride of the staged matrix (elements)
@@ -664,15 +664,20 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
   }
 #define JT_LOAD_X(slot, k0)                                                                  \
   {                                                                                          \
-    _Pragma("unroll") for (int n = 0; n < 2; ++n) a_ring[slot][n] =                          \
-        kPad ? __builtin_amdgcn_raw_buffer_load_b128(                                        \
-                   x_rsrc, (k0) + n * 32 + (lane >> 4) * 8 < H ? x_voff + n * 64 + (k0)*2 : kOutside, 0, 0) \
-             : __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff + n * 64, (k0)*2, 0);    \
+    /* (the whole-chunk form without the offsets' sum: it cost the kernel 2 to 4 us) */       \
+    if constexpr (kPad) {                                                                    \
+      _Pragma("unroll") for (int n = 0; n < 2; ++n) a_ring[slot][n] =                        \
+          __builtin_amdgcn_raw_buffer_load_b128(                                             \
+              x_rsrc, (k0) + n * 32 + (lane >> 4) * 8 < H ? x_voff + n * 64 + (k0)*2 : kOutside, 0, 0); \
+    } else {                                                                                 \
+      a_ring[slot][0] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff, (k0)*2, 0);    \
+      a_ring[slot][1] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff + 64, (k0)*2, 0); \
+    }                                                                                        \
   }
 
   // transposing read of this lane: 16-lane group g = lane/16 reads rows 32*s + 8*g + 4*h + i/4
   const int w_lane = ((lane >> 4) * 8 + ((lane & 15) >> 2)) * WS + 4 * (lane & 3);
-  const int nchunks = (H + kRouterKC - 1) / kRouterKC;
+  const int nchunks = (H + (kPad ? kRouterKC - 1 : 0)) / kRouterKC;
   int in_slice = 0;  // chunks of the current slice done
 #pragma unroll
   for (int d = 0; d < D; ++d)
@@ -1030,8 +1035,8 @@ inline size_t router_arrivals_offset(int64_t E) {
 // and the first token_blocks * slices workgroups are the small-batch router: each computes the partial
 // sums of its (token block, slice), counts itself in, and the last of them to arrive adds the slices up
 // in slice order and runs the epilogue and the dispatch plan (router_finish_body) -- the same arithmetic
-// in the same order as the two-launch form, so the same bits.  The router's 21 us of dependent steps
-// then run beside the 115 us of weight streaming instead of in front of it, with no second stream and
+// in the same order as the two-launch form, so the same bits.  The router's dependent steps, 11 to 17 us
+// alone, then run beside the 115 us of weight streaming instead of in front of it, with no second stream and
 // no dependency between launches other than the stream's own order.
 // The arrival counter is a 64-bit word of the caller's workspace: the low byte counts, the rest is a tag
 // the host draws per launch.  A word whose tag is not this launch's counts as zero, so the word needs no
