@@ -557,7 +557,7 @@ __global__ __launch_bounds__(kStagedThreads) void router_staged_kernel(
 // ONE summation order for every batch size.  A token's logits must not depend on how many tokens
 // share its call (a decode step of 64 tokens and a prefill of 16 384 have to route a row the same
 // way), although small batches want the k range shared out over many workgroups and large ones want
-// it walked by one.  All the matrix-core kernels below therefore add up a logit in this order:
+// it walked by one.  All the kernels with bf16 products therefore add up a logit in this order:
 //   * H is cut into slices of router_slice_rows(H) consecutive k rows (eight slices, or as many
 //     128-row chunks as there are, when H is a multiple of 128; one slice otherwise);
 //   * inside a slice, v_mfma_f32_16x16x32_bf16 instructions are chained in k order, the first onto a
@@ -573,7 +573,7 @@ __global__ __launch_bounds__(kStagedThreads) void router_staged_kernel(
 // (each lane two 16-byte pieces per 64-wide k chunk, the four lane groups of a token together whole
 // 128-byte lines per token row); the router matrix [H,E] is staged chunk by chunk through LDS as it
 // is stored and read with the transposing ds_read_b64_tr_b16.
-// H % 64 == 0 and E in {16, 32, 64, 128, 256}; with kPad H and E multiples of 8.
+// Requires H % 64 == 0 and E in {16, 32, 64, 128, 256}.
 // ---------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 constexpr int kRouterKC = 64;  // k rows of the router matrix per LDS stage
@@ -594,27 +594,18 @@ __host__ __device__ inline size_t router_mfma_smem_bytes(int E, int K, int token
   return w > ep ? w : ep;
 }
 
-// kPad kernels: expert counts below the 16 NB columns of the tiles (a multiple of 8: whole 16-byte pieces) and rows that
-// end inside a chunk (H a multiple of 8).  What lies outside the matrix or the row reads as zeros.  Byte offset of piece
-// c of a stage that starts at row k0:
-__device__ __forceinline__ int router_pad_w(int c, int pieces_per_row, int k0, int E) {
-  const int kr = c / pieces_per_row, nc = c - kr * pieces_per_row;
-  return nc * 8 < E ? ((k0 + kr) * E + nc * 8) * 2 : kOutside;
-}
-
-template <int NB, int NW, bool kPad>
+template <int NB, int NW>
 __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens,
-    int H, int width, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
+    int H, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ logits_out, void* ws, int score_func) {
   constexpr int kRouterTokens = 16 * NW, kRouterThreads = 64 * NW;
-  const int slice_chunks = (router_slice_rows(H) + (kPad ? kRouterKC - 1 : 0)) / kRouterKC;  // 64-row chunks per slice
-  constexpr int EC = NB * 16;
-  const int E = kPad ? width : EC;
-  constexpr int WS = EC + 32;                     // LDS row stride of the staged matrix (elements)
-  constexpr int W_CHUNKS = kRouterKC * EC / 8;     // 16-byte chunks per stage
+  const int slice_chunks = router_slice_rows(H) / kRouterKC;  // 64-row chunks per slice
+  constexpr int E = NB * 16;
+  constexpr int WS = E + 32;                      // LDS row stride of the staged matrix (elements)
+  constexpr int W_CHUNKS = kRouterKC * E / 8;     // 16-byte chunks per stage
   constexpr int CW = (W_CHUNKS + kRouterThreads - 1) / kRouterThreads;
-  constexpr int CPR = EC / 8;                      // chunks per k row
+  constexpr int CPR = E / 8;                      // chunks per k row
   extern __shared__ __align__(16) unsigned char smem_raw[];
   uint16_t* const Ws = reinterpret_cast<uint16_t*>(smem_raw);  // [2][kRouterKC][WS]; reused by the epilogue
 
@@ -651,8 +642,7 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
   _Pragma("unroll") for (int i = 0; i < CW; ++i) {                                           \
     const int c = tid + i * kRouterThreads;                                                  \
     if (W_CHUNKS % kRouterThreads == 0 || c < W_CHUNKS)                                      \
-      w_ring[slot][i] = kPad ? __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, router_pad_w(c, CPR, k0, E), 0, 0)   \
-                             : __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, c * 16, (k0)*E * 2, 0);              \
+      w_ring[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, c * 16, (k0)*E * 2, 0); \
   }
 #define JT_STORE_W(slot, stage)                                                              \
   _Pragma("unroll") for (int i = 0; i < CW; ++i) {                                           \
@@ -664,20 +654,13 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
   }
 #define JT_LOAD_X(slot, k0)                                                                  \
   {                                                                                          \
-    /* (the whole-chunk form without the offsets' sum: it cost the kernel 2 to 4 us) */       \
-    if constexpr (kPad) {                                                                    \
-      _Pragma("unroll") for (int n = 0; n < 2; ++n) a_ring[slot][n] =                        \
-          __builtin_amdgcn_raw_buffer_load_b128(                                             \
-              x_rsrc, (k0) + n * 32 + (lane >> 4) * 8 < H ? x_voff + n * 64 + (k0)*2 : kOutside, 0, 0); \
-    } else {                                                                                 \
-      a_ring[slot][0] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff, (k0)*2, 0);    \
-      a_ring[slot][1] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff + 64, (k0)*2, 0); \
-    }                                                                                        \
+    a_ring[slot][0] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff, (k0)*2, 0);      \
+    a_ring[slot][1] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff + 64, (k0)*2, 0); \
   }
 
   // transposing read of this lane: 16-lane group g = lane/16 reads rows 32*s + 8*g + 4*h + i/4
   const int w_lane = ((lane >> 4) * 8 + ((lane & 15) >> 2)) * WS + 4 * (lane & 3);
-  const int nchunks = (H + (kPad ? kRouterKC - 1 : 0)) / kRouterKC;
+  const int nchunks = H / kRouterKC;
   int in_slice = 0;  // chunks of the current slice done
 #pragma unroll
   for (int d = 0; d < D; ++d)
@@ -744,8 +727,7 @@ __global__ __launch_bounds__(64 * NW) void router_mfma_kernel(
   for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (!kPad || nb * 16 + (lane & 15) < E)
-        sm.tile[(wave * 16 + 4 * (lane >> 4) + i) * stride + nb * 16 + (lane & 15)] = round_to_bf16(total[nb][i]);
+      sm.tile[(wave * 16 + 4 * (lane >> 4) + i) * stride + nb * 16 + (lane & 15)] = round_to_bf16(total[nb][i]);
   __syncthreads();
   router_epilogue<bf16_raw, 16 * NW, 64 * NW>(sm, bias, t0, tokens, E, K, route_scale, ids, weights, scores,
                                               logits_out, router_scratch(ws, E), score_func);
@@ -778,19 +760,18 @@ __host__ __device__ inline size_t router_split_smem_bytes(int E, int K) {
 // order and does the rest.  Otherwise the workgroup walks all slices itself.
 // (token_block / slice: the workgroup's place in the launch's grid -- blockIdx.x / blockIdx.y in
 // router_mfma_split_kernel; the decode launch hands them out among its own workgroups)
-template <int NB, bool kPartial, bool kPad>
+template <int NB, bool kPartial>
 __device__ __forceinline__ void router_split_body(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens,
-    int H, int width, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
+    int H, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ logits_out, void* ws, float* __restrict__ partial_out,
     int score_func, int token_block, int slice) {
   constexpr int kThreads = 256, kTokens = 16;
-  constexpr int EC = NB * 16;
-  const int E = kPad ? width : EC;
-  constexpr int WS = EC + 32;
-  constexpr int W_CHUNKS = kSplitKC * EC / 8;
+  constexpr int E = NB * 16;
+  constexpr int WS = E + 32;
+  constexpr int W_CHUNKS = kSplitKC * E / 8;
   constexpr int CW = (W_CHUNKS + kThreads - 1) / kThreads;
-  constexpr int CPR = EC / 8;
+  constexpr int CPR = E / 8;
   constexpr int NBW = (NB + 3) / 4;  // column blocks per wave
   extern __shared__ __align__(16) unsigned char smem_raw[];
   uint16_t* const Ws = reinterpret_cast<uint16_t*>(smem_raw);  // [2][kSplitKC][WS]
@@ -821,8 +802,7 @@ __device__ __forceinline__ void router_split_body(
     _Pragma("unroll") for (int i = 0; i < CW; ++i) {                                          \
       const int c = tid + i * kThreads;                                                       \
       if (W_CHUNKS % kThreads == 0 || c < W_CHUNKS)                                           \
-        w_ring[slot][i] = kPad ? __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, router_pad_w(c, CPR, k0, E), 0, 0) \
-                               : __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, c * 16, (k0)*E * 2, 0);             \
+        w_ring[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, c * 16, (k0)*E * 2, 0); \
     }                                                                                         \
     if (has_cols) {                                                                           \
       _Pragma("unroll") for (int n = 0; n < 4; ++n)                                           \
@@ -903,7 +883,7 @@ __device__ __forceinline__ void router_split_body(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int t = 4 * (lane >> 4) + i;
-          if (t < nrows && wave + 4 * b < NB && (!kPad || (wave + 4 * b) * 16 + (lane & 15) < E))
+          if (t < nrows && wave + 4 * b < NB)
             partial_out[((size_t)slice * tokens + t0 + t) * E + (wave + 4 * b) * 16 + (lane & 15)] = acc[b][i];
         }
     }
@@ -918,7 +898,7 @@ __device__ __forceinline__ void router_split_body(
     for (int b = 0; b < NBW; ++b)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (wave + 4 * b < NB && (!kPad || (wave + 4 * b) * 16 + (lane & 15) < E))
+        if (wave + 4 * b < NB)
           sm.tile[(4 * (lane >> 4) + i) * stride + (wave + 4 * b) * 16 + (lane & 15)] = round_to_bf16(total[b][i]);
   }
   __syncthreads();
@@ -926,13 +906,13 @@ __device__ __forceinline__ void router_split_body(
                                                logits_out, router_scratch(ws, E), score_func);
 }
 
-template <int NB, bool kPartial, bool kPad>
+template <int NB, bool kPartial>
 __global__ __launch_bounds__(256) void router_mfma_split_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens,
-    int H, int width, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
+    int H, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ logits_out, void* ws, float* __restrict__ partial_out,
     int score_func) {
-  router_split_body<NB, kPartial, kPad>(x, w, bias, tokens, H, width, K, route_scale, ids, weights, scores, logits_out, ws,
+  router_split_body<NB, kPartial>(x, w, bias, tokens, H, K, route_scale, ids, weights, scores, logits_out, ws,
                                   partial_out, score_func, (int)blockIdx.x, (int)blockIdx.y);
 }
 
@@ -1025,6 +1005,226 @@ __global__ __launch_bounds__(kThreads) void router_finish_blocks_kernel(
                                                   RouterScratch{}, score_func);
 }
 
+// ---------------------------------------------------------------------------
+// bf16 projection on the fp32 matrix cores, for whole 16-byte rows that the kernels above do not take (H and E multiples
+// of 8; experts that do not fill their tiles, rows that end inside their chunks).
+//
+// A logit is ONE chain of H fused multiply-adds in k order, as in the staged kernel, and has its bits: a chain of
+// v_mfma_f32_16x16x4_f32, element g of a step (g = lane / 16) at k = 4 j + g, rounds after every product in that order
+// (compared with fmaf over 70000 sums, among them denormals, overflows, infinities and NaN).  So a row's logits depend
+// neither on the batch nor on the alignment that chooses between the two.
+//
+// The chain bounds it, H / 4 steps of 32 cycles (3.5 us at H = 1024; measured 5.6 ns a k value with the staging, where
+// 3.4 are the products), NBW chains side by side in a wave; a workgroup takes 16 tokens, wave w the 16-column blocks w,
+// w + 4, ... of its columns.  Both operands pass through LDS as bf16, KC rows of k at a time, requested D chunks ahead;
+// a chunk is parked between the products of the one before.  A row of LDS holds k in the order [k / 32][k % 4][k % 32 / 4],
+// so that one 16-byte read is a lane's operand of eight steps; rows are padded by 16 bytes and every eight of them by
+// another 16, which keeps the two-byte writes of the transposed matrix at two lanes to a bank.
+// What lies outside the row or the matrix reads as zeros; columns of LDS past the last expert hold anything, and their
+// sums go nowhere.
+// Router calls, us, staged kernel -> here: 2000 x 1384 x 96 118 -> 41, 2931 x 1000 x 24 31 -> 18, 4096 x 1024 x 8 22 -> 16,
+// 300 x 1024 x 8 19 -> 13, 1 x 1024 x 8 19 -> 12, 16384 x 1024 x 8 44 -> 31.  bf16 products in slices of k take 35, 17, 15, 14,
+// 6 and 18, with other last bits in one to three of ten thousand logits.
+// ---------------------------------------------------------------------------
+constexpr int kChainColumns = 64;  // of a workgroup that only writes sums: a chain to a wave
+template <int NBW>
+constexpr int kChainKC = NBW == 1 ? 128 : 64;  // (the same pieces of the matrix per thread for one and two blocks)
+template <int NBW>
+constexpr int kChainRow = 2 * kChainKC<NBW> + 16;  // bytes
+template <int NBW>
+inline size_t router_chain_smem_bytes(int cols) {
+  return (size_t)2 * (24 + (cols + 15) / 16 * 16) * (kChainRow<NBW> + 2);  // (16 bytes to eight rows)
+}
+
+template <int NBW, int NL>
+__device__ __forceinline__ void router_chain(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int t0,
+                                             int nrows, int H, int E, int col0, int cols, unsigned char* smem,
+                                             f32x4_t (&acc)[NBW]) {
+  constexpr int kThreads = 256, KC = kChainKC<NBW>, RS = kChainRow<NBW>, XP = KC / 8;  // XP pieces of a token's row
+  constexpr int D = NL == 1 ? 8 : (NL == 2 ? 4 : (NL <= 4 ? 3 : 2)), UNROLL = D % 2 ? 2 * D : D;
+  static_assert(16 * XP <= kThreads, "a piece of x per thread");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int blocks = (cols + 15) >> 4, stage_bytes = (24 + 16 * blocks) * (RS + 2);
+  const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(x + (size_t)t0 * H), 0, nrows * H * 2, kBufferFlags);
+  const __amdgpu_buffer_rsrc_t w_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w), 0, H * E * 2, kBufferFlags);
+  auto row_at = [](int r) { return r * RS + (r >> 3) * 16; };  // token r, or column r - 16
+  auto k_at = [](int k) { return (k >> 5) * 64 + (k & 3) * 16 + ((k & 31) >> 2) * 2; };
+
+  const int x_k = tid % XP * 8, x_voff = (tid / XP * H + x_k) * 2;
+  const bool has_x = 16 * XP == kThreads || tid < 16 * XP;
+  const int x_lds = row_at(tid / XP) + k_at(x_k);
+  const int per_row = cols >> 3;
+  int w_voff[NL], w_lds[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int c = tid + i * kThreads, k = c / per_row, n = (c - k * per_row) * 8;
+    w_voff[i] = k < KC ? (k * E + col0 + n) * 2 : kOutside;
+    // (eight columns lie RS bytes apart; a thread without a piece writes behind the last ones: a branch around the write
+    // would let the compiler move the load into it)
+    w_lds[i] = k < KC ? row_at(16 + n) + k_at(k) : row_at(16 + 16 * blocks) + k_at(tid % KC);
+  }
+  u32x4_t x_ring[D], w_ring[D][NL];
+  auto load = [&](int slot, int k0) {
+    x_ring[slot] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, has_x && k0 + x_k < H ? x_voff + k0 * 2 : kOutside, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      w_ring[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(
+          w_rsrc, w_voff[i] != kOutside ? (int)((unsigned)w_voff[i] + (unsigned)(k0 * 2) * (unsigned)E) : kOutside, 0, 0);
+  };
+  auto park = [&](int slot, int stage, int j) {  // in eight parts
+    unsigned char* const base = smem + stage * stage_bytes;
+    if (j < 4 && has_x) {  // k and k + 4 side by side
+      const uint32_t lo = x_ring[slot][j >> 1], hi = x_ring[slot][2 + (j >> 1)];
+      *reinterpret_cast<uint32_t*>(base + x_lds + j * 16) = j & 1 ? (lo >> 16) | (hi & 0xffff0000u) : (lo & 0xffffu) | (hi << 16);
+    }
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      *reinterpret_cast<uint16_t*>(base + w_lds[i] + j * RS) = (uint16_t)(w_ring[slot][i][j >> 1] >> (j & 1) * 16);
+  };
+  const int a_lds = row_at(lane & 15) + (lane >> 4) * 16, b_lds = row_at(16 + wave * 16 + (lane & 15)) + (lane >> 4) * 16;
+  auto value = [](const u32x4_t& v, int j) {
+    return __builtin_bit_cast(float, j & 1 ? v[j >> 1] & 0xffff0000u : v[j >> 1] << 16);
+  };
+  // Eight steps at a time, two sets of operands: those of the next block are requested in front of a block's products and
+  // unpacked between them.  An operand is kept until the next ones are written: a write into a register that a product
+  // in flight reads waits for the product (58 instead of 33 cycles a step).
+  u32x4_t a_words, b_words[NBW];
+  float a[2][8], b[2][NBW][8];
+  auto request = [&](int stage, int kb) {
+    const unsigned char* const base = smem + stage * stage_bytes + kb * 64;
+    a_words = *reinterpret_cast<const u32x4_t*>(base + a_lds);
+#pragma unroll
+    for (int n = 0; n < NBW; ++n)
+      if (wave + 4 * n < blocks) b_words[n] = *reinterpret_cast<const u32x4_t*>(base + b_lds + n * (64 * RS + 128));
+  };
+  auto unpack = [&](int set, int j) {
+    a[set][j] = value(a_words, j);
+#pragma unroll
+    for (int n = 0; n < NBW; ++n) b[set][n][j] = value(b_words[n], j);
+  };
+  auto products = [&](int set, auto&& between) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+      for (int n = 0; n < NBW; ++n)
+        if (wave + 4 * n < blocks) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][j], b[set][n][j], acc[n], 0, 0, 0);
+      between(j);
+      if (j >= 4) {  // (the words have arrived)
+        unpack(set ^ 1, 2 * j - 8);
+        unpack(set ^ 1, 2 * j - 7);
+      }
+      asm volatile("" ::"v"(a[set][j]));
+#pragma unroll
+      for (int n = 0; n < NBW; ++n) asm volatile("" ::"v"(b[set][n][j]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  constexpr int KB = KC / 32;
+  static_assert(KB % 2 == 0, "the first block of a chunk in the first set");
+  const int nchunks = (H + KC - 1) / KC;
+#pragma unroll
+  for (int n = 0; n < NBW; ++n)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[n][i] = 0.0f;
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d * KC);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) park(0, 0, j);
+  __syncthreads();
+  // Nothing in it depends on whether a chunk follows (past the last one loads lie outside and move nothing, and zeros are
+  // parked): the compiler then counts the loads in flight, and a chunk waits for its own alone.
+  auto walk = [&](auto with_products) {
+    constexpr bool kProducts = decltype(with_products)::value;
+    if constexpr (kProducts) {
+      request(0, 0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) unpack(0, j);
+    }
+    for (int c = 0; c < nchunks;) {
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        const int next = (u + 1) & 1;
+        if constexpr (kProducts) {
+#pragma unroll
+          for (int kb = 0; kb + 1 < KB; ++kb) {
+            request(u & 1, kb + 1);
+            products(kb & 1, [&](int j) {
+              if (kb == 0 && j == 0) load(u % D, (c + D) * KC);  // (parked before the last barrier)
+              if (kb == KB - 2) park((u + 1) % D, next, j);
+            });
+          }
+        } else {
+          load(u % D, (c + D) * KC);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) park((u + 1) % D, next, j);
+        }
+        __syncthreads();
+        if constexpr (kProducts) {
+          request(next, 0);
+          products((KB - 1) & 1, [](int) {});
+        }
+        if (++c == nchunks) break;  // uniform over the workgroup
+      }
+    }
+  };
+  if (wave < blocks)
+    walk(std::true_type{});
+  else
+    walk(std::false_type{});
+  __syncthreads();  // all stages read
+}
+
+// The unrounded sums of 16 tokens and up to 64 experts, partial[token][expert]: a call's only slice (see router_finish_body).
+template <int NL>
+__device__ __forceinline__ void router_chain_sums(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                  int tokens, int H, int E, float* __restrict__ partial, int token_block,
+                                                  int column_block) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int t0 = token_block * 16, nrows = min(16, tokens - t0), col0 = column_block * kChainColumns;
+  const int lane = threadIdx.x & 63, col = col0 + ((int)threadIdx.x >> 6) * 16 + (lane & 15);
+  f32x4_t acc[1];
+  router_chain<1, NL>(x, w, t0, nrows, H, E, col0, min(kChainColumns, E - col0), smem_raw, acc);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = 4 * (lane >> 4) + i;
+    if (t < nrows && col < E) partial[(size_t)(t0 + t) * E + col] = acc[0][i];
+  }
+}
+
+template <int NL>
+__global__ __launch_bounds__(256) void router_chain_sums_kernel(const uint16_t* __restrict__ x,
+                                                                const uint16_t* __restrict__ w, int tokens, int H, int E,
+                                                                float* __restrict__ partial) {
+  router_chain_sums<NL>(x, w, tokens, H, E, partial, (int)blockIdx.x, (int)blockIdx.y);
+}
+
+// Projection and epilogue of 16 tokens.
+template <int NBW, int NL>
+__global__ __launch_bounds__(256) void router_chain_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens, int H,
+    int E, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
+    float* __restrict__ scores, float* __restrict__ logits_out, void* ws, int score_func) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int t0 = (int)blockIdx.x * 16, lane = threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  f32x4_t acc[NBW];
+  router_chain<NBW, NL>(x, w, t0, min(16, tokens - t0), H, E, 0, E, smem_raw, acc);
+  RouterSmem sm = router_smem(smem_raw, E, K, 16);  // (the stages are dead: the loop ends with a barrier)
+#pragma unroll
+  for (int b = 0; b < NBW; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int col = (wave + 4 * b) * 16 + (lane & 15);
+      if (col < E) sm.tile[(4 * (lane >> 4) + i) * (E + 1) + col] = round_to_bf16(acc[b][i]);
+    }
+  __syncthreads();
+  router_epilogue<bf16_raw, 16, 256>(sm, bias, t0, tokens, E, K, route_scale, ids, weights, scores, logits_out,
+                                     router_scratch(ws, E), score_func);
+}
+
 inline size_t router_arrivals_offset(int64_t E) {
   return router_scratch_bytes(E) + align_up((size_t)kPartialMaxSlices * kSplitMaxTokens * E * sizeof(float), 256);
 }
@@ -1113,7 +1313,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
     return;
   }
   const int token_block = (int)blockIdx.x % token_blocks, slice = (int)blockIdx.x / token_blocks;
-  router_split_body<NB, true, false>(x, w_router, bias, T, H, E, K, route_scale, ids, weights, scores, nullptr, nullptr, partial,
+  router_split_body<NB, true>(x, w_router, bias, T, H, K, route_scale, ids, weights, scores, nullptr, nullptr, partial,
                               score_func, token_block, slice);
   if (!last_to_arrive(arrivals, tag, router_blocks)) return;
   router_finish_body<64, true>(partial, slices, bias, T, E, K, route_scale, ids, weights, scores, nullptr, counts,
@@ -1127,23 +1327,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
 // in the decode launch, the last workgroup to arrive finishes); the shared down tiles go beside the routed gate/up product
 // (BesideCfg).  As two launches, the finishing workgroup beside the shared down tiles, it took 17.5 + 14.9 us there.
 // ---------------------------------------------------------------------------
-template <int NB, bool kPad>
+// NB < 0: the chained projection (chain_pieces: -NB), a workgroup per 16 tokens and 64 experts, its sums the only slice.
+template <int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void router_shared_gate_up_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens, int H,
     int E, int K, float route_scale, int score_func, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ counts, float* __restrict__ importance,
     int32_t* __restrict__ group_sizes, int32_t* __restrict__ offsets, int32_t* __restrict__ source_order,
-    int32_t* __restrict__ inverse, float* __restrict__ partial, int token_blocks, int slices,
+    int32_t* __restrict__ inverse, float* __restrict__ partial, int token_blocks, int parts,
     unsigned long long* __restrict__ arrivals, unsigned long long tag, SkinnyProblem shared) {
-  const int block = (int)blockIdx.x, router_blocks = token_blocks * slices;
+  const int block = (int)blockIdx.x, router_blocks = token_blocks * parts;
   if (block >= router_blocks) {
     grouped_gemm_skinny_tile<SharedGateUpCfg>(shared, block - router_blocks, (int)gridDim.x - router_blocks);
     return;
   }
-  router_split_body<NB, true, kPad>(x, w, bias, tokens, H, E, K, route_scale, ids, weights, scores, nullptr, nullptr,
-                                    partial, score_func, block % token_blocks, block / token_blocks);
+  if constexpr (NB < 0)
+    router_chain_sums<-NB>(x, w, tokens, H, E, partial, block % token_blocks, block / token_blocks);
+  else
+    router_split_body<NB, true>(x, w, bias, tokens, H, K, route_scale, ids, weights, scores, nullptr, nullptr, partial,
+                                score_func, block % token_blocks, block / token_blocks);
   if (!last_to_arrive(arrivals, tag, router_blocks)) return;
-  router_finish_body<kSharedFinishTokens, true>(partial, slices, bias, tokens, E, K, route_scale, ids, weights, scores,
+  router_finish_body<kSharedFinishTokens, true>(partial, NB < 0 ? 1 : parts, bias, tokens, E, K, route_scale, ids, weights, scores,
                                                 nullptr, counts, importance, group_sizes, offsets, source_order,
                                                 inverse, score_func);
   if (threadIdx.x == 0) *arrivals = 0ull;
@@ -1171,20 +1375,41 @@ struct LayerPlan {
   size_t scratch_bytes;
 };
 
-// bf16 routers whose experts and columns are multiples of 8 run on the matrix cores, in tiles of 16, 32, 64, 128 or 256
-// columns; where these do not fit exactly, in kernels that check (kPad).  The staged kernel, a chain of H dependent steps,
-// takes what is left: where it took those too, a router call
-// of 2000 x 1384 x 96 took 127 us (now 36), 2931 x 1000 x 24 30 (17.5), 4096 x 1024 x 8 18.4 (12.8), 300 x 1024 x 8
-// 17 (3.6 + 4.2), and a layer call of one token at 1024 x 8 66 (49.5: the plan and the shared experts share its launches).
+// bf16 routers whose experts and columns are multiples of 8 run on the matrix cores: those that fill the tiles with bf16
+// products in slices of k, the others (router_chained) as one chain in fp32.  The staged kernel takes what is left.
 inline bool router_on_matrix_cores(const void* x, const void* w, int64_t H, int64_t E) {
   return H % 8 == 0 && E % 8 == 0 && E <= 256 && H * E < ((int64_t)1 << 30) && aligned16(x) && aligned16(w);
 }
-inline bool router_padded(int64_t H, int64_t E) { return H % kRouterKC != 0 || E < 16 || (E & (E - 1)) != 0; }
-// column blocks of 16 in the tiles: 1, 2, 4, 8 or 16
-inline int router_column_blocks(int64_t E) {
-  int nb = 1;
-  while (nb * 16 < E) nb *= 2;
-  return nb;
+inline bool router_chained(int64_t H, int64_t E) { return H % kRouterKC != 0 || E < 16 || (E & (E - 1)) != 0; }
+
+// pieces of the matrix per thread and chunk of a workgroup with at most 64 experts
+inline int chain_pieces(int64_t E) { return E <= 16 ? 1 : (E <= 32 ? 2 : 4); }
+
+// (ws: the statistics' accumulators, null where the caller leaves them to the dispatch)
+int launch_router_chain(const void* x, const void* w, const float* bias, int64_t tokens, int64_t H, int64_t E, int64_t K,
+                        double route_scale, int32_t* ids, void* weights, float* scores, float* counts, float* importance,
+                        float* logits_out, void* ws, hipStream_t stream, int score_func) {
+  if (ws) router_zero_kernel<<<1, 256, 0, stream>>>(ws, (int)E);
+  if (tokens > 0) {
+    const int nbw = (int)((E + 63) / 64);
+    const size_t stages = nbw == 1 ? router_chain_smem_bytes<1>((int)E) : router_chain_smem_bytes<2>((int)E);
+    const size_t smem = std::max(stages, router_smem_bytes((int)E, (int)K, 16));
+    if (smem > 160 * 1024) return fail(JTMOE_EUNSUPPORTED, "router: E=%lld K=%lld needs %zu bytes of LDS", (long long)E, (long long)K, smem);
+    const int pieces = chain_pieces(E);
+    auto kernel = pieces == 1   ? &router_chain_kernel<1, 1>
+                  : pieces == 2 ? &router_chain_kernel<1, 2>
+                  : nbw == 1    ? &router_chain_kernel<1, 4>
+                  : nbw == 2    ? &router_chain_kernel<2, 4>
+                  : nbw == 3    ? &router_chain_kernel<3, 6>
+                                : &router_chain_kernel<4, 8>;
+    const int rc = set_max_smem(kernel, smem);
+    if (rc) return rc;
+    kernel<<<(unsigned)((tokens + 15) / 16), 256, smem, stream>>>(
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K,
+        (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, ws, score_func);
+  }
+  if (ws) router_finalize_kernel<<<1, 256, 0, stream>>>(ws, (int)E, counts, importance);
+  return check_launch("router");
 }
 
 template <typename T, bool kFromLogits>
@@ -1197,15 +1422,16 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
   void* const ws_stats = stats ? ws : nullptr;
   if (layer) layer->stats_done = layer->plan_done = false;
   const bool mfma = Elem<T>::is_bf16 && !kFromLogits && router_on_matrix_cores(x, w, H, E);
-  const bool pad = router_padded(H, E);
+  const bool chained = mfma && router_chained(H, E);
   if (mfma) {
     // Up to a few hundred tokens the whole call is a handful of workgroups, each waiting on its own
     // chain of chunks: the k-split kernel (16 tokens per workgroup, half as many and shorter
     // iterations) is used; beyond that the 64-token workgroups stage the router matrix four times
     // less often per token and win.
-    if (H % kSplitKC == 0 && tokens <= kSplitMaxTokens) {
+    if ((chained || H % kSplitKC == 0) && tokens <= kSplitMaxTokens) {
       const int blocks = (int)((tokens + 15) / 16);
-      const size_t smem = std::max(router_split_smem_bytes((int)E, (int)K), router_split_smem_bytes(16 * router_column_blocks(E), 1));
+      const size_t smem = chained ? router_chain_smem_bytes<1>(std::min((int)E, kChainColumns))
+                                  : router_split_smem_bytes((int)E, (int)K);
       if (smem > 160 * 1024)
         return fail(JTMOE_EUNSUPPORTED, "router: E=%lld K=%lld needs %zu bytes of LDS", (long long)E, (long long)K, smem);
       // Two launches when one workgroup can hold the epilogue of the whole call: partial sums over
@@ -1213,19 +1439,27 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
       const int finish_tok = router_smem_bytes((int)E, (int)K, 256) <= 160 * 1024 ? 256 : 64;
       if (tokens > 0 && tokens <= finish_tok && router_smem_bytes((int)E, (int)K, finish_tok) <= 160 * 1024) {
         const int slice_rows = router_slice_rows((int)H);
-        const int slices = (int)((H + slice_rows - 1) / slice_rows);
+        const int slices = chained ? 1 : (int)((H + slice_rows - 1) / slice_rows);
         float* partial = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + router_scratch_bytes(E));
+        if (chained) {
+          const int pieces = chain_pieces(E);
+          auto kernel = pieces == 1   ? &router_chain_sums_kernel<1>
+                        : pieces == 2 ? &router_chain_sums_kernel<2>
+                                      : &router_chain_sums_kernel<4>;
+          kernel<<<dim3(blocks, (unsigned)((E + kChainColumns - 1) / kChainColumns)), 256, smem, stream>>>(
+              static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), (int)tokens, (int)H, (int)E, partial);
+        } else
 #define JT_PARTIAL_CASE(NB)                                                                                   \
-  case NB: {                                                                                                 \
-    auto kernel = pad ? &router_mfma_split_kernel<NB, true, true> : &router_mfma_split_kernel<NB, true, false>; \
+  case NB * 16: {                                                                                            \
+    auto kernel = router_mfma_split_kernel<NB, true>;                                                        \
     int rc = set_max_smem(kernel, smem);                                                                     \
     if (rc) return rc;                                                                                       \
     kernel<<<dim3(blocks, slices), 256, smem, stream>>>(                                                     \
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K, \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, ws, partial,           \
         score_func);                                                                                         \
   } break;
-        switch (router_column_blocks(E)) {
+        switch ((int)E) {
           JT_PARTIAL_CASE(1)
           JT_PARTIAL_CASE(2)
           JT_PARTIAL_CASE(4)
@@ -1267,19 +1501,22 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
         }
         return check_launch("router");
       }
+      if (chained)
+        return launch_router_chain(x, w, bias, tokens, H, E, K, route_scale, ids, weights, scores, counts, importance,
+                                   logits_out, ws_stats, stream, score_func);
       if (stats) router_zero_kernel<<<1, 256, 0, stream>>>(ws, (int)E);
       if (tokens > 0) {
 #define JT_SPLIT_CASE(NB)                                                                                     \
-  case NB: {                                                                                                 \
-    auto kernel = pad ? &router_mfma_split_kernel<NB, false, true> : &router_mfma_split_kernel<NB, false, false>; \
+  case NB * 16: {                                                                                            \
+    auto kernel = router_mfma_split_kernel<NB, false>;                                                       \
     int rc = set_max_smem(kernel, smem);                                                                     \
     if (rc) return rc;                                                                                       \
     kernel<<<blocks, 256, smem, stream>>>(                                                                   \
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K, \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, ws_stats, nullptr,     \
         score_func);                                                                                         \
   } break;
-        switch (router_column_blocks(E)) {
+        switch ((int)E) {
           JT_SPLIT_CASE(1)
           JT_SPLIT_CASE(2)
           JT_SPLIT_CASE(4)
@@ -1291,6 +1528,9 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
       if (stats) router_finalize_kernel<<<1, 256, 0, stream>>>(ws, (int)E, counts, importance);
       return check_launch("router");
     }
+    if (chained)
+      return launch_router_chain(x, w, bias, tokens, H, E, K, route_scale, ids, weights, scores, counts, importance,
+                                 logits_out, ws_stats, stream, score_func);
     // Middle-sized layer calls: a 64-token workgroup walks all of H, 26 us (E = 64) and 40 us (E = 128) at 2048 columns
     // whether there are 300 tokens or 8000; up to kMidMaxTokens the slices are computed in workgroups of their own, in
     // the layer's memory, and a workgroup per 16 tokens finishes.  us, split + finish against one launch, E = 64: 300
@@ -1303,22 +1543,22 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
     const int slices = (int)((H + slice_rows - 1) / slice_rows);
     if (layer && tokens <= kMidMaxTokens && H % kSplitKC == 0 && H >= 1024 &&
         (size_t)slices * tokens * E * sizeof(float) <= layer->scratch_bytes) {
-      const size_t smem = (size_t)2 * kSplitKC * router_w_stride(16 * router_column_blocks(E)) * 2;
+      const size_t smem = (size_t)2 * kSplitKC * router_w_stride((int)E) * 2;
       const size_t fsmem = router_smem_bytes((int)E, (int)K, 16);
       if (fsmem <= 160 * 1024) {
         float* const partial = static_cast<float*>(layer->scratch);
         const int blocks = (int)((tokens + 15) / 16);
 #define JT_PARTIAL_CASE(NB)                                                                                  \
-  case NB: {                                                                                                 \
-    auto kernel = pad ? &router_mfma_split_kernel<NB, true, true> : &router_mfma_split_kernel<NB, true, false>; \
+  case NB * 16: {                                                                                            \
+    auto kernel = router_mfma_split_kernel<NB, true>;                                                        \
     const int rc = set_max_smem(kernel, smem);                                                               \
     if (rc) return rc;                                                                                       \
     kernel<<<dim3(blocks, slices), 256, smem, stream>>>(                                                     \
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K, \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, nullptr, partial,      \
         score_func);                                                                                         \
   } break;
-        switch (router_column_blocks(E)) {
+        switch ((int)E) {
           JT_PARTIAL_CASE(1)
           JT_PARTIAL_CASE(2)
           JT_PARTIAL_CASE(4)
@@ -1339,24 +1579,24 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
     constexpr int nw = 4;
     const int tok = 16 * nw;
     const int blocks = (int)((tokens + tok - 1) / tok);
-    const size_t smem = std::max(router_mfma_smem_bytes((int)E, (int)K, tok), router_mfma_smem_bytes(16 * router_column_blocks(E), 1, 1));
+    const size_t smem = router_mfma_smem_bytes((int)E, (int)K, tok);
     if (smem > 160 * 1024) return fail(JTMOE_EUNSUPPORTED, "router: E=%lld K=%lld needs %zu bytes of LDS", (long long)E, (long long)K, smem);
     if (stats) router_zero_kernel<<<1, 256, 0, stream>>>(ws, (int)E);
     if (tokens > 0) {
 #define JT_ROUTER_LAUNCH(NB, NW)                                                                             \
   {                                                                                                          \
-    auto kernel = pad ? &router_mfma_kernel<NB, NW, true> : &router_mfma_kernel<NB, NW, false>;               \
+    auto kernel = router_mfma_kernel<NB, NW>;                                                                \
     int rc = set_max_smem(kernel, smem);                                                                     \
     if (rc) return rc;                                                                                       \
     kernel<<<blocks, 64 * NW, smem, stream>>>(                                                               \
-        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)E, (int)K, \
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias, (int)tokens, (int)H, (int)K, \
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, ws_stats, score_func); \
   }
 #define JT_ROUTER_CASE(NB)    \
-  case NB:                    \
+  case NB * 16:               \
     JT_ROUTER_LAUNCH(NB, nw)  \
     break;
-      switch (router_column_blocks(E)) {
+      switch ((int)E) {
         JT_ROUTER_CASE(1)
         JT_ROUTER_CASE(2)
         JT_ROUTER_CASE(4)
@@ -1510,29 +1750,33 @@ static int launch_router_with_shared(const void* x, const void* w_router, const 
                                      const LayerPlan& plan, void* ws, hipStream_t stream) {
   const int token_blocks = (int)((T + 15) / 16);
   const int slice_rows = router_slice_rows((int)H);
-  const int slices = (int)((H + slice_rows - 1) / slice_rows);
   float* const partial = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + router_scratch_bytes(E));
   unsigned long long* const arrivals =
       reinterpret_cast<unsigned long long*>(static_cast<unsigned char*>(ws) + router_arrivals_offset(E));
   const SkinnyProblem gate_up = dense_skinny(x, sh.gate, sh.up, sh.act, sh.gate_pre, sh.up_pre, T, H, sh.Is,
                                              SharedGateUpCfg::BM, SharedGateUpCfg::BN);
-  const bool pad = router_padded(H, E);
-  const size_t smem = std::max({router_split_smem_bytes((int)E, (int)K), router_split_smem_bytes(16 * router_column_blocks(E), 1),
+  const bool chained = router_chained(H, E);
+  const int parts = chained ? (int)((E + kChainColumns - 1) / kChainColumns) : (int)((H + slice_rows - 1) / slice_rows);
+  const size_t smem = std::max({chained ? router_chain_smem_bytes<1>(std::min((int)E, kChainColumns))
+                                        : router_split_smem_bytes((int)E, (int)K),
                                 router_smem_bytes((int)E, (int)K, kSharedFinishTokens), (size_t)SharedGateUpCfg::SMEM_BYTES});
-  const int64_t grid = token_blocks * slices + gemm_grid(gate_up.mtiles, gate_up.ntiles_n);
+  const int64_t grid = token_blocks * parts + gemm_grid(gate_up.mtiles, gate_up.ntiles_n);
   const unsigned long long tag = next_launch_tag();
 #define JT_SHARED_CASE(NB)                                                                                        \
-  case NB: {                                                                                                      \
-    auto kernel = pad ? &router_shared_gate_up_kernel<NB, true> : &router_shared_gate_up_kernel<NB, false>;       \
+  case NB * 16: {                                                                                                 \
+    auto kernel = router_shared_gate_up_kernel<NB>;                                                               \
     const int rc = set_max_smem(kernel, smem);                                                                    \
     if (rc) return rc;                                                                                            \
     kernel<<<(unsigned)grid, 256, smem, stream>>>(                                                                \
         static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w_router), bias, (int)T, (int)H, (int)E,    \
         (int)K, (float)route_scale, score_func, ids, static_cast<bf16_raw*>(weights), scores, counts, importance, \
-        plan.group_sizes, plan.offsets, plan.source_order, plan.inverse, partial, token_blocks, slices, arrivals, \
+        plan.group_sizes, plan.offsets, plan.source_order, plan.inverse, partial, token_blocks, parts, arrivals, \
         tag, gate_up);                                                                                            \
   } break;
-  switch (router_column_blocks(E)) {
+  switch (chained ? -16 * chain_pieces(E) : (int)E) {
+    JT_SHARED_CASE(-1)
+    JT_SHARED_CASE(-2)
+    JT_SHARED_CASE(-4)
     JT_SHARED_CASE(1)
     JT_SHARED_CASE(2)
     JT_SHARED_CASE(4)
