@@ -192,6 +192,11 @@ const char* jtmoe_product_kernel(int product, int64_t rows, int64_t K, int64_t N
  */
 const char* jtmoe_joint_kernel(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is, int64_t E,
                                int compute_units);
+/*
+ * Whether the single-precision backward pass of `rows` routed rows in E groups runs dXp and the three weight gradients
+ * in one launch ("joint") or in launches of their own ("separate").  Otherwise as above.
+ */
+const char* jtmoe_f32_backward_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, int compute_units);
 int jtmoe_grouped_swiglu_gather(const void* x, const int32_t* source_order,
                                 const void* gate, const void* up, const void* down,
                                 const int32_t* group_sizes, const int32_t* offsets,

@@ -79,11 +79,13 @@ int launch_f32_tn(const void* p, const void* d0, const void* d1, void* c0, void*
 size_t f32_tn_split_bytes(int64_t rows, int64_t KA, int64_t N, bool dual);
 
 // dXp and the three weight gradients of the routed experts in one launch, where that is supported and faster
+// (compute_units: of the device to answer for, 0: the current one)
 struct F32Backward {
   const void *dg, *du, *hw, *xp, *dyp, *gate, *up;
   void *dxp, *d_gate, *d_up, *d_down;
 };
-bool f32_backward_products_supported(const F32Backward& b, int64_t rows, int64_t H, int64_t I, int64_t E);
+bool f32_backward_products_supported(const F32Backward& b, int64_t rows, int64_t H, int64_t I, int64_t E,
+                                     int compute_units = 0);
 int launch_f32_backward_products(const F32Backward& b, const int32_t* group_sizes, const int32_t* offsets, int64_t rows,
                                  int64_t H, int64_t I, int64_t E, hipStream_t stream);
 

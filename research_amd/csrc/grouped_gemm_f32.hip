@@ -18,9 +18,10 @@ inline int64_t f32_mtiles(bool dense, int64_t rows, int64_t E, int BM) {
 // tile per group is padding.  At 4096 rows in 8 groups, 512 x 1024 the rule takes the small tiles; when it was drawn,
 // before either lost 5 to 9 % of its time: gate/up 101 against 120 us, down 62 (544 tiles, three units) against 81 (144 tiles,
 // four units), data gradients 55 and 118 against 74 and 151 us.
-inline int64_t f32_cost(bool dense, int64_t rows, int64_t E, int64_t N, int BM, int BN, int units) {
+inline int64_t f32_cost(bool dense, int64_t rows, int64_t E, int64_t N, int BM, int BN, int units,
+                        int64_t cus = persistent_grid_size()) {
   const int64_t mt = (rows + BM - 1) / BM + (dense ? 0 : std::min(E, rows) / 2);
-  const int64_t tiles = mt * ((N + BN - 1) / BN), cus = persistent_grid_size();
+  const int64_t tiles = mt * ((N + BN - 1) / BN);
   return (tiles + cus - 1) / cus * units;
 }
 
@@ -147,25 +148,28 @@ int launch_f32_tn(const void* p_, const void* d0_, const void* d1_, void* c0_, v
 // The weight gradients' large tiles are the faster ones as long as rounds are full (131 against 114 TFLOP/s), so a tenth
 // has to be saved.  4096 rows in 8 groups, 512 x 1024 (10496 against 12288 steps): 192 us against 238 for the three;
 // twice the rows (20736 against 22528) keep launches of their own.
-bool f32_backward_joint(int64_t rows, int64_t H, int64_t I, int64_t E) {
-  const int64_t cus = persistent_grid_size(), depth = std::max<int64_t>(rows / std::max<int64_t>(E, 1), 1);
+bool f32_backward_joint(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t cus) {
+  const int64_t depth = std::max<int64_t>(rows / std::max<int64_t>(E, 1), 1);
   const auto tn = [&](int64_t matrices) {
     const int64_t big = matrices * E * ((H + 127) / 128) * ((I + 127) / 128);
     const int64_t small = matrices * E * ((H + 63) / 64) * ((I + 63) / 64);
     return std::min((big + cus - 1) / cus * 4, (small + cus - 1) / cus) * depth;
   };
   const int64_t apart =
-      std::min(f32_cost(false, rows, E, H, 128, 128, 4), f32_cost(false, rows, E, H, 64, 64, 1)) * 2 * I + tn(2) + tn(1);
+      std::min(f32_cost(false, rows, E, H, 128, 128, 4, cus), f32_cost(false, rows, E, H, 64, 64, 1, cus)) * 2 * I +
+      tn(2) + tn(1);
   const int64_t mt = (rows + 63) / 64 + std::min(E, rows) / 2, th = (H + 63) / 64, ti = (I + 63) / 64;
   const int64_t joint = std::max((mt * th * 2 * I + 3 * E * th * ti * depth + cus - 1) / cus, 2 * I);
   return joint * 10 <= apart * 9;
 }
 
-bool f32_backward_products_supported(const F32Backward& b, int64_t rows, int64_t H, int64_t I, int64_t E) {
+bool f32_backward_products_supported(const F32Backward& b, int64_t rows, int64_t H, int64_t I, int64_t E,
+                                     int compute_units) {
   const int64_t grid = gemm_grid(f32_mtiles(false, rows, E, 64), (H + 63) / 64) + 3 * E * ((H + 63) / 64) * ((I + 63) / 64);
   return rows > 0 && rows * H < kF32Limit && grid < ((int64_t)1 << 31) && aligned16(b.hw) && aligned16(b.dyp) &&
          f32_gemm_supported(b.dg, b.du, b.gate, b.up, b.dxp, rows, I, H) &&
-         f32_gemm_supported(b.xp, b.d_gate, b.d_up, b.d_down, nullptr, rows, H, I) && f32_backward_joint(rows, H, I, E);
+         f32_gemm_supported(b.xp, b.d_gate, b.d_up, b.d_down, nullptr, rows, H, I) &&
+         f32_backward_joint(rows, H, I, E, compute_units > 0 ? compute_units : persistent_grid_size());
 }
 
 int launch_f32_backward_products(const F32Backward& b, const int32_t* group_sizes, const int32_t* offsets, int64_t rows,
@@ -182,3 +186,13 @@ int launch_f32_backward_products(const F32Backward& b, const int32_t* group_size
 }
 
 }  // namespace jtmoe
+
+// what the rule above says of these sizes
+extern "C" const char* jtmoe_f32_backward_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, int compute_units) {
+  using namespace jtmoe;
+  const int64_t limit = (int64_t)1 << 24;
+  if (rows <= 0 || rows >= ((int64_t)1 << 31) || H <= 0 || H >= limit || I <= 0 || I >= limit || E <= 0 ||
+      E > JTMOE_MAX_EXPERTS || compute_units < 0)
+    return "";
+  return f32_backward_products_supported({}, rows, H, I, E, compute_units) ? "joint" : "separate";
+}

@@ -23,6 +23,11 @@ def gradient_kernels(rows, hidden, inter, experts=0, cus=0):
             chosen(DATA_GRADIENT_PAIR, rows, inter, hidden, experts, cus))
 
 
+def f32_backward_kernel(rows, hidden, inter, experts, cus=0):
+    """Whether the single-precision gradients of the routed experts run in one launch ("joint") or in three."""
+    return _ffi.load_library().jtmoe_f32_backward_kernel(rows, hidden, inter, experts, cus).decode()
+
+
 def joint_kernels(tokens, top_k, hidden, inter, shared, experts, cus=0):
     """Those of gate/up, down, dZ and dX of routed and shared experts in one launch ("separate": in two)."""
     joint = _ffi.load_library().jtmoe_joint_kernel

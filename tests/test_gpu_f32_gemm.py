@@ -14,6 +14,7 @@ import torch
 
 import test_gpu_grad as G
 import test_gpu_parity as P
+from kernel_choice import MI355X_CUS, f32_backward_kernel
 from oracle import moe_grad_oracle as GO
 from oracle import moe_oracle as O
 from research_amd import grad
@@ -62,16 +63,24 @@ def test_f32_shared_experts_with_split_reductions(gpu, tokens, hidden, inter):
         assert P.report("f32 shared", host(g), ref.numpy().astype(np.float32)) <= bar
 
 
-@pytest.mark.parametrize("tokens,hidden,experts,inter,joint", [
-    (3, 4, 5, 4, True),         # one chunk, groups of at most three rows, two of them empty
-    (300, 260, 5, 132, True),   # columns one chunk past a tile; a group without rows between groups with some
-    (700, 132, 16, 68, True),   # short reductions, most tiles partly filled
-    (2048, 512, 8, 1024, True),
-    (8192, 512, 8, 1024, False),  # the launches of their own, whose rounds are nearly full
-])
-def test_f32_backward_products_in_one_launch(gpu, tokens, hidden, experts, inter, joint):
-    """dXp and the three weight gradients with uneven groups and empty ones, against float64; each gradient has the
-    bits that the data gradients and weight gradients of a second call have."""
+# tokens, hidden, experts, d_ff, how the products of the backward pass run, and (tokens, experts) of a larger call whose
+# first groups are these and whose products have launches of their own
+BACKWARD_SHAPES = [
+    (3, 4, 5, 4, "joint", (4099, 250)),         # one chunk, groups of at most three rows, two of them empty
+    (300, 260, 5, 132, "joint", (1200, 64)),    # columns one chunk past a tile; a group without rows between groups with some
+    (700, 132, 16, 68, "joint", (1700, 250)),   # short reductions, most tiles partly filled
+    (2048, 512, 8, 1024, "joint", (3048, 10)),
+    (8192, 512, 8, 1024, "separate", (9192, 10)),  # rounds of the launches of their own are nearly full
+]
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,inter,launches,larger", BACKWARD_SHAPES)
+def test_f32_backward_products_in_one_launch(gpu, tokens, hidden, experts, inter, launches, larger):
+    """dXp and the three weight gradients with uneven groups and empty ones, against float64.  The same groups among the
+    first of a larger call, whose products run in launches of their own, have the same bits."""
+    if torch.cuda.get_device_properties(gpu).multi_processor_count == MI355X_CUS:
+        assert f32_backward_kernel(tokens, hidden, inter, experts) == launches
+        assert f32_backward_kernel(larger[0], hidden, inter, larger[1]) == "separate"
     rng = np.random.default_rng(tokens + hidden)
     share = np.where(np.arange(experts) % 4 == 1, 0.0, 1.0 + np.arange(experts) ** 2)
     first = rng.choice(experts, tokens, p=share / share.sum())
@@ -81,7 +90,13 @@ def test_f32_backward_products_in_one_launch(gpu, tokens, hidden, experts, inter
     gate, up = ((rng.standard_normal((experts, hidden, inter)) * 0.1).astype(np.float32) for _ in range(2))
     down = (rng.standard_normal((experts, inter, hidden)) * 0.1).astype(np.float32)
     got, _ = G.expert_grads(gpu, x, ids, w, gate, up, down, dy, "f32")
-    again, _ = G.expert_grads(gpu, x, ids, w, gate, up, down, dy, "f32")
+
+    def extended(a, n, scale):
+        return np.concatenate([a, (rng.standard_normal((n - len(a), *a.shape[1:])) * scale).astype(np.float32)])
+
+    more = rng.integers(experts, larger[1], (larger[0] - tokens, 1)).astype(np.int32)
+    alone, _ = G.expert_grads(gpu, extended(x, larger[0], 1.0), np.concatenate([ids, more]), extended(w, larger[0], 1.0),
+                              *(extended(m, larger[1], 0.1) for m in (gate, up, down)), extended(dy, larger[0], 1.0), "f32")
     leaves = [torch.from_numpy(a.astype(np.float64)).requires_grad_() for a in (x, gate, up, down)]
     y = torch.zeros(tokens, hidden, dtype=torch.float64)
     for e in range(experts):
@@ -91,5 +106,5 @@ def test_f32_backward_products_in_one_launch(gpu, tokens, hidden, experts, inter
     want = torch.autograd.grad(y, leaves, torch.from_numpy(dy.astype(np.float64)))
     bar = 2.0 ** -23 * 8 * np.sqrt(max(hidden, inter, tokens))
     for name, ref in zip(("dx", "d_gate", "d_up", "d_down"), want):
-        assert torch.equal(getattr(got, name), getattr(again, name)), name
+        assert torch.equal(getattr(got, name), getattr(alone, name)[:len(ref)]), name
         assert P.report(f"f32 {name}", host(getattr(got, name)), ref.numpy().astype(np.float32)) <= bar, name

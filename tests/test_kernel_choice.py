@@ -8,11 +8,13 @@ from __future__ import annotations
 
 import pytest
 
+import test_gpu_f32_gemm as f32
 import test_gpu_joint_products as joint
 import test_gpu_ragged_widths as ragged
 import test_gpu_row_bits as row_bits
 import test_gpu_tile_choice as tiles
-from kernel_choice import DOWN, GATE_UP, MI355X_CUS, chosen, forward_kernels, gradient_kernels, joint_kernels
+from kernel_choice import (DOWN, GATE_UP, MI355X_CUS, chosen, f32_backward_kernel, forward_kernels, gradient_kernels,
+                           joint_kernels)
 
 GATE_UP_KERNELS = {"stream_16x128", "stream_16x64", "stream_32x64", "rows64", "rows64_tail", "half", "half_tail", "rows256",
                    "rows256_tail", "rows256_short", "rows256_short_tail"}
@@ -70,6 +72,12 @@ def test_joint_shapes_take_the_kernels_they_name(tokens, hidden, experts, top_k,
 def test_every_joint_kernel_is_held_to_separate_launches():
     for product, names in enumerate(zip(*(case[6].split() for case in joint.SHAPES))):
         assert set(names) == JOINT_KERNELS[product]
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,inter,launches,larger", f32.BACKWARD_SHAPES)
+def test_f32_backward_shapes_take_the_launches_they_name(tokens, hidden, experts, inter, launches, larger):
+    assert f32_backward_kernel(tokens, hidden, inter, experts, MI355X_CUS) == launches
+    assert f32_backward_kernel(larger[0], hidden, inter, larger[1], MI355X_CUS) == "separate"
 
 
 def test_sizes_out_of_range_have_no_kernel():
