@@ -601,7 +601,41 @@ static void time_decode() {
   release(d);
 }
 
+// "deal": host arithmetic only.  The workgroups of an XCD take every tile of the two products of a joint launch exactly
+// once, each workgroup the dense ones first, in rising order, and have no tile after their last.
+bool check_deal() {
+  srand(1);
+  const int cases = 20000;
+  for (int c = 0; c < cases; ++c) {
+    const int W = 1 + rand() % 40, n1 = rand() % (c % 3 == 0 ? 4 : 200), n0 = rand() % (c % 5 == 0 ? 4 : 400), lead = 1 + rand() % 6;
+    std::vector<int> seen(n0 + n1, 0);
+    for (int w = 0; w < W; ++w) {
+      int last = -1, p = 0;
+      for (int i = joint_tile(w, W, p, n1, n0, lead); i >= 0; i = joint_tile(w, W, ++p, n1, n0, lead)) {
+        if (i <= last || i >= n0 + n1 || seen[i]++) {
+          printf("deal: W=%d n1=%d n0=%d lead=%d: workgroup %d, place %d: tile %d\n", W, n1, n0, lead, w, p, i);
+          return false;
+        }
+        last = i;
+      }
+      for (int q = p; q < p + 10; ++q)
+        if (joint_tile(w, W, q, n1, n0, lead) >= 0) {
+          printf("deal: W=%d n1=%d n0=%d lead=%d: workgroup %d goes on after its end\n", W, n1, n0, lead, w);
+          return false;
+        }
+    }
+    for (int i = 0; i < n0 + n1; ++i)
+      if (!seen[i]) {
+        printf("deal: W=%d n1=%d n0=%d lead=%d: tile %d of none\n", W, n1, n0, lead, i);
+        return false;
+      }
+  }
+  printf("deal: %d cases\nPASS\n", cases);
+  return true;
+}
+
 int main(int argc, char** argv) {
+  if (argc > 1 && !strcmp(argv[1], "deal")) return check_deal() ? 0 : 1;
   bool ok = true;
   // "<mode> nocheck": only the timing mode (for counter collection); otherwise every check runs first
   const bool nocheck = argc > 2 && !strcmp(argv[2], "nocheck");

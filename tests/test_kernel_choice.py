@@ -6,6 +6,8 @@ exercise every kernel, so that a change of a rule cannot take a kernel's last te
 
 from __future__ import annotations
 
+import subprocess
+
 import pytest
 
 import test_gpu_f32_gemm as f32
@@ -15,6 +17,7 @@ import test_gpu_row_bits as row_bits
 import test_gpu_tile_choice as tiles
 from kernel_choice import (DOWN, GATE_UP, MI355X_CUS, chosen, f32_backward_kernel, forward_kernels, gradient_kernels,
                            joint_kernels)
+from research_amd import build
 
 GATE_UP_KERNELS = {"stream_16x128", "stream_16x64", "stream_32x64", "rows64", "rows64_tail", "half", "half_tail", "rows256",
                    "rows256_tail", "rows256_short", "rows256_short_tail"}
@@ -78,6 +81,13 @@ def test_every_joint_kernel_is_held_to_separate_launches():
 def test_f32_backward_shapes_take_the_launches_they_name(tokens, hidden, experts, inter, launches, larger):
     assert f32_backward_kernel(tokens, hidden, inter, experts, MI355X_CUS) == launches
     assert f32_backward_kernel(larger[0], hidden, inter, larger[1], MI355X_CUS) == "separate"
+
+
+def test_joint_launches_deal_every_tile_once():
+    binary = build.cache_dir() / build.NATIVE_TEST_NAME
+    assert binary.exists(), "run __graft_entry__.build() first"
+    proc = subprocess.run([binary.as_posix(), "deal"], capture_output=True, text=True, timeout=110)
+    assert proc.returncode == 0 and proc.stdout.strip().endswith("PASS"), proc.stdout + proc.stderr
 
 
 def test_sizes_out_of_range_have_no_kernel():
