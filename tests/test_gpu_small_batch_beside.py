@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from kernel_choice import MI355X_CUS, forward_kernels
-from research_amd import _ffi, graph, ops
+from research_amd import _ffi, grad, graph, ops
 from test_gpu_layer_paths import test_decode_path_equals_the_stand_alone_operators as check_layer
 
 pytestmark = pytest.mark.gpu
@@ -38,6 +38,37 @@ def test_layer_equals_the_stand_alone_operators(gpu, tokens, hidden, experts, to
     if not decode:
         assert forward_kernels(tokens * top_k, hidden, d_ff, experts, MI355X_CUS)[0] == kernel
     check_layer(gpu, tokens, hidden, experts, top_k, d_ff, shared_width)
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,top_k,d_ff,shared_width,kernel", [
+    (2, 256, 32, 2, 64, 136, "stream_16x64"),
+    (64, 1024, 8, 2, 2048, 2048, "stream_32x64"),
+    (64, 384, 24, 8, 2048, 64, "rows64"),
+    (24, 512, 16, 2, 396, 264, "general"),  # takes no tiles along: the shared down product in a launch of its own
+])
+def test_training_forward_keeps_every_product(gpu, tokens, hidden, experts, top_k, d_ff, shared_width, kernel):
+    """The training forward, whose routed gate/up beside the shared down tiles keeps its two products, and the inference
+    call, against the operators one by one."""
+    assert forward_kernels(tokens, hidden, shared_width, cus=MI355X_CUS) == ("stream_16x64", "stream_16x64")
+    assert forward_kernels(tokens * top_k, hidden, d_ff, experts, MI355X_CUS)[0] == kernel
+    generator = torch.Generator(device=gpu).manual_seed(tokens + d_ff)
+
+    def normal(*shape, std=0.05):
+        return (torch.randn(shape, generator=generator, device=gpu) * std).to(torch.bfloat16)
+
+    x, weights = normal(tokens, hidden, std=1.0), (normal(hidden, experts), torch.zeros(experts, device=gpu),
+                                                   normal(experts, hidden, d_ff), normal(experts, hidden, d_ff),
+                                                   normal(experts, d_ff, hidden))
+    shared = normal(hidden, shared_width), normal(hidden, shared_width), normal(shared_width, hidden)
+    trained, kept = grad.moe_forward_train(x, *weights, top_k, 1.0, shared=shared)
+    plan = ops.dispatch(trained.expert_ids, experts, x)
+    packed_y, _, routed = grad.grouped_swiglu_train(plan.packed_x, None, top_k, *weights[2:], plan.group_sizes, plan.offsets)
+    shared_y, dense = grad.shared_swiglu_train(x, *shared)
+    want = ops.combine(packed_y, plan.inverse, trained.weights, shared_y)
+    assert torch.equal(trained.y, want)
+    assert torch.equal(ops.moe_forward(x, *weights, top_k, 1.0, shared=shared).y, want)
+    for got, alone in ((kept.routed, routed), (kept.shared, dense)):
+        assert torch.equal(got.gate_pre, alone.gate_pre) and torch.equal(got.up_pre, alone.up_pre)
 
 
 @pytest.mark.parametrize("tokens,hidden,experts,top_k,d_ff,shared_width", [(1, 1024, 8, 2, 512, 264), (9, 512, 64, 8, 704, 1408),
