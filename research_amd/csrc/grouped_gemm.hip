@@ -255,7 +255,7 @@ struct RoutedProblem {
   const void *a, *b0, *b1;
   void *c, *save0, *save1;
   const int32_t *group_sizes, *offsets, *row_map;
-  int64_t rows, K, N, E, a_rows, a_group_rows;
+  int64_t rows, K, N, E, a_rows;
   int row_div;
 };
 
@@ -439,17 +439,16 @@ inline bool fast_ok(const void* a, const void* b0, const void* b1, const void* c
 }
 
 // y = act Wd[e] on the matrix cores (fast_ok holds); with a map, packed row j reads row row_map[j] / row_div of
-// its group's block of a_group_rows rows (the decode path)
+// its group's block of a_group_rows rows (the decode path), and the tiles of `beside` run in the same launch
 int launch_down_fast(const void* act, const void* down, const int32_t* group_sizes, const int32_t* offsets,
                      int64_t rows, int64_t H, int64_t I, int64_t E, void* y, hipStream_t stream,
                      const int32_t* row_map = nullptr, int row_div = 1, int64_t a_group_rows = 0,
-                     const Beside* beside = nullptr, bool* beside_taken = nullptr) {
+                     const Beside* beside = nullptr) {
 #define JT_DOWN(LAUNCH, CFG) LAUNCH<CFG>(act, down, nullptr, y, group_sizes, offsets, rows, I, H, E, stream, row_map, row_div, a_group_rows, nullptr, nullptr
   using S11 = SkinnyCfg<1, 1, false>;
   using S12 = SkinnyCfg<1, 2, false>;
   using S22 = SkinnyCfg<2, 2, false>;
   const ProductKernel k = down_kernel(rows, H, I, E, group_sizes == nullptr, persistent_grid_size());
-  if (beside) *beside_taken = streaming_or_rows64(k);
   switch (k) {
     case ProductKernel::kStream16x128: return JT_DOWN(launch_skinny, S11), a_group_rows, beside);
     case ProductKernel::kStream16x64: return JT_DOWN(launch_skinny, S12), a_group_rows, beside);
@@ -458,7 +457,7 @@ int launch_down_fast(const void* act, const void* down, const int32_t* group_siz
     default: break;
   }
   // (at most half a tile of rows per group on the decode path: the rules above take all of it)
-  if (row_map) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: no down kernel reads blocks of rows per group at this size");
+  if (row_map || beside) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: no down kernel reads blocks of rows per group at this size");
   switch (k) {
     case ProductKernel::kHalf: return JT_DOWN(launch_stream, DownHalfCfg), 2);
     case ProductKernel::kHalfDeep: return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
@@ -573,14 +572,14 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
                 int64_t x_rows = 0, void* save_gate = nullptr, void* save_up = nullptr,
                 const SharedExperts* shared = nullptr) {
   if (rows == 0) return JTMOE_OK;
-  const RoutedProblem gu{x, gate, up, act, save_gate, save_up, group_sizes, offsets, row_map, rows, H, I, E, x_rows, 0, row_div};
-  const RoutedProblem dn{act, down, nullptr, y, nullptr, nullptr, group_sizes, offsets, nullptr, rows, I, H, E, 0, 0, 1};
+  const RoutedProblem gu{x, gate, up, act, save_gate, save_up, group_sizes, offsets, row_map, rows, H, I, E, x_rows, row_div};
+  const RoutedProblem dn{act, down, nullptr, y, nullptr, nullptr, group_sizes, offsets, nullptr, rows, I, H, E, 0, 1};
   int rc = JTMOE_OK;
   if (shared != nullptr) {
     const RoutedProblem sgu{x, shared->gate, shared->up, shared->act, shared->gate_pre, shared->up_pre, nullptr, nullptr,
-                            nullptr, x_rows, H, shared->Is, 1, 0, 0, 1};
+                            nullptr, x_rows, H, shared->Is, 1, 0, 1};
     const RoutedProblem sdn{shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, nullptr, nullptr, nullptr,
-                            x_rows, shared->Is, H, 1, 0, 0, 1};
+                            x_rows, shared->Is, H, 1, 0, 1};
     if (shared->gate_up_done) {
       // (a few tokens: the router has run the shared gate/up product, its down product goes beside the routed gate/up)
       const SkinnyProblem down_p = dense_skinny(shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, x_rows,
@@ -627,12 +626,8 @@ int launch_down_from_all_tokens(const void* act_full, const void* down, const in
   const SkinnyProblem p = dense_skinny(shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, T, shared->Is, H,
                                        BesideCfg::BM, BesideCfg::BN);
   const Beside beside{p, (int)gemm_grid(p.mtiles, p.ntiles_n)};
-  bool taken = false;
-  const int rc = launch_down_fast(act_full, down, group_sizes, offsets, T * K, H, I, E, packed_y, stream, source_order,
-                                  (int)K, /*a_group_rows=*/T, &beside, &taken);
-  // (every kernel that reads blocks of rows per group takes the shared tiles along)
-  if (rc || taken) return rc;
-  return launch_down_fast(shared->act, shared->down, nullptr, nullptr, T, H, shared->Is, 1, shared->y, stream);
+  return launch_down_fast(act_full, down, group_sizes, offsets, T * K, H, I, E, packed_y, stream, source_order, (int)K,
+                          /*a_group_rows=*/T, &beside);
 }
 
 bool shared_in_skinny_tiles(const void* x, const SharedExperts& s, int64_t T, int64_t H) {
