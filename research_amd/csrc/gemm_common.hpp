@@ -268,7 +268,10 @@ inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, doub
 // routed tiles of 1408 53; gate/up at 1024 tokens 41 and 57; dx of 2048 at 4096 tokens 41 and 99).  At equal
 // rounds a call gains or loses up to 3 % with few of them (less of a last round idle against a higher clock in two part-filled
 // ones) and gains up to 1 % from six on.  As for half tiles it has to pay by two estimates of how the groups spread (1300
-// tokens, 64 experts top-8: two rounds of routed tiles by one, 2.3 by the other; down jointly 3 % more a call).
+// tokens, 64 experts top-8: two rounds of routed tiles by one, 2.3 by the other; down jointly 3 % more a call), and with
+// three standard deviations more groups than are to be expected: with a few rows per group each is a tile, and a round more
+// streams the experts' matrices a second time (backward of 24 tokens, 64 experts top-8, 2048 x 1408, shared 2816: dX jointly
+// 194 us where 63 groups had a row, 121 + 39 apart; of 27 tokens 595 the pass against 555).
 inline HalfTiles joint_tiles(int64_t rows, int64_t E, int64_t N, int64_t T, int64_t N1, double longer, double cus,
                              double one_per_cu, bool dual = false) {
   auto across = [dual](int64_t n, int bn) { return (double)(dual ? (n + 127) / 128 : (n + bn - 1) / bn); };
@@ -280,9 +283,13 @@ inline HalfTiles joint_tiles(int64_t rows, int64_t E, int64_t N, int64_t T, int6
   if (expected_mtiles(rows, E, false, 128) * across(N, 128) + dense_tiles(128) <= cus) return HalfTiles::kOnePerCu;
   const HalfTiles routed = half_tiles(rows, E, false, N, cus);
   const double shared = longer * alone(half_tiles(T, 1, true, N1, cus), dense_tiles(128), dense_tiles(256));
+  const double mean = (double)rows / (double)E, empty = std::exp(-mean);
+  const double more_groups =
+      std::fmin((double)E * empty, 3.0 * std::sqrt((double)E * empty * (1.0 - (1.0 + mean) * empty)));
   auto pays = [&](auto mtiles) {
     const double full = mtiles(rows, E, false, 256) * across(N, 256), half = mtiles(rows, E, false, 128) * across(N, 128);
-    const double both = std::fmax(longer, std::ceil((full + longer * dense_tiles(256)) / cus));
+    const double both =
+        std::fmax(longer, std::ceil((full + more_groups * across(N, 256) + longer * dense_tiles(256)) / cus));
     const double apart = alone(routed, half, full) + shared;
     return both < apart || (both == apart && both > 6.0);
   };

@@ -72,6 +72,21 @@ def test_joint_shapes_take_the_kernels_they_name(tokens, hidden, experts, top_k,
     assert " ".join(joint_kernels(tokens, top_k, hidden, inter, shared, experts, MI355X_CUS)) == kernels
 
 
+@pytest.mark.parametrize("tokens,top_k,hidden,inter,shared,experts,dz,dx", [
+    # a few rows per group: a tile each, and how many groups have a row is chance.  Jointly where the rounds hold
+    # whatever happens, apart where a few groups more start another round
+    (12, 8, 2048, 1408, 2816, 64, "separate", "rows256"),
+    (16, 8, 2048, 1408, 2816, 64, "separate", "separate"),
+    (24, 8, 2048, 1408, 2816, 64, "separate", "separate"),
+    (27, 8, 2048, 1408, 2816, 64, "separate", "separate"),
+    (6, 8, 2048, 1408, 2816, 64, "rows256", "separate"),
+    (8, 8, 2048, 1408, 2816, 64, "separate", "separate"),
+    (21, 3, 1000, 2664, 2664, 24, "separate", "half_deep"),
+])
+def test_joint_gradients_of_a_few_rows_leave_room_for_more_groups(tokens, top_k, hidden, inter, shared, experts, dz, dx):
+    assert joint_kernels(tokens, top_k, hidden, inter, shared, experts, MI355X_CUS)[2:] == [dz, dx]
+
+
 def test_every_joint_kernel_is_held_to_separate_launches():
     for product, names in enumerate(zip(*(case[6].split() for case in joint.SHAPES))):
         assert set(names) == JOINT_KERNELS[product]
