@@ -9,6 +9,10 @@ point jtmoe_moe_forward bracketed by torch.cuda.synchronize().  After it, K more
 steps are run through jtmoe_moe_forward_timed, which records a hipEvent on the
 launch stream after every stage; the per-stage averages give the roofline
 figures.  Prints ONE JSON line.
+
+A stage of the timed call is a launch of its own.  The steps that are timed as a
+whole run a product of the routed experts and the same product of the shared ones
+in one launch where the library finds that faster; "joint_launches" names them.
 """
 
 from __future__ import annotations
@@ -440,6 +444,11 @@ def main() -> int:
         "roofline": roofline,
         "stages": stages,
     }
+    if shared is not None and code == _ffi.JTMOE_BF16:
+        # gate/up and down as the whole steps run them; the stages above are the launches of the timed call
+        inter = (cfg["I"], cfg["I"] * cfg["Ns"])
+        line["joint_launches"] = {name: lib.jtmoe_joint_kernel(product, T, cfg["K"], cfg["H"], *inter, cfg["E"], 0).decode()
+                                  for product, name in enumerate(("gate_up", "down"))}
     if lib.jtmoe_moe_forward_takes_decode_path(T, cfg["H"], cfg["E"], cfg["K"], cfg["I"], code):
         line["stages"]["note"] = ("decode path: the gate/up stage is one launch that runs every token through every "
                                   "expert and holds the router and the dispatch plan in a few of its workgroups")

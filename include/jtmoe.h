@@ -331,9 +331,9 @@ int jtmoe_moe_forward_sf(const void* x, const void* w_router, const float* exper
  *    shared gate/up GEMM + SwiGLU, shared down GEMM, combine}.
  * A stage without a launch of its own reads as zero: the row scatter wherever the GEMM fetches its
  * rows through the permutation, the router and the dispatch of a call that takes the decode path
- * (jtmoe_moe_forward_takes_decode_path), which run inside the gate/up launch.  The shared experts of a
- * call of up to 64 tokens, which jtmoe_moe_forward may run beside the router, have launches of their
- * own here; the outputs are the same bits.
+ * (jtmoe_moe_forward_takes_decode_path), which run inside the gate/up launch.  The shared experts, whose
+ * products jtmoe_moe_forward may run beside the router and in one launch with the routed ones
+ * (jtmoe_joint_kernel), have launches of their own here; the outputs are the same bits.
  */
 #define JTMOE_NUM_STAGES 8
 int jtmoe_moe_forward_timed(const void* x, const void* w_router, const float* expert_bias,

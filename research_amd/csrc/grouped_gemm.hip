@@ -329,16 +329,15 @@ int launch_skinny(const void* a, const void* b0, const void* b1, void* c, const 
 // 34 at 1 token, 36 at 64 (148 in 64-row LDS tiles), 43 at 130 with 32-row tiles (58 without them).  Tiles of 128
 // columns and 32 or 64 rows do not pay where half tiles can be had: 68 against 53 at 387 tokens, 91 against 63 at 700.
 // With more tiles than CUs, and up to four rows per group reached (a group's second tile reads its matrix again),
-// they compete with the 64-row LDS tiles over the number that is resident at once.  Gate/up: the LDS tiles are as
-// wide, three to a CU; streaming pays up to two tiles per CU: 74 against 76 us at 12 tokens top-8 of 128 experts,
-// 2048 -> 768 (426 tiles expected), 77 against 84 at 8 tokens of 64 experts, 2048 -> 1408 (448), but 104 against 98 at
-// 20 tokens (546) and 104 against 102 at 15 (605).  Down: the LDS tiles are 256 wide, two to a CU, and a second
-// round of them costs as much as the first (33 us for 480 tiles, 55 for 528); streaming pays while all of its
-// tiles are resident, three to a CU (8 tokens, 64 experts 48 against 56), and where the LDS tiles start that round (12
-// and 20 tokens, 128 experts 41 and 52 against 56 and 58; 37 with two thirds of the experts reached 39 against 55;
-// balanced 63 against 62), but not in between (15 tokens, 64 experts 63 against 54).
-// (These lines were drawn with three and two of the 64-row LDS tiles on a CU; four are resident now.
-// They have not been drawn again; what the fourth gave, the LDS tiles' side of them gained.)
+// they compete with the 64-row LDS tiles over the number that is resident at once.  Kernel times, us, LDS tiles, four to
+// a CU, / streaming; 64 experts of 2048 -> 1408 and 128 of 2048 -> 768, top-8:
+//   gate/up, LDS tiles as wide; streaming up to two tiles per CU.  64 experts: 8 tokens 76.1 / 74.0, 10 92.2 / 101.4, 15
+//   102.3 / 105.3; 128: 8 tokens 65.4 / 66.0, 12 75.2 / 75.0, 20 96.5 / 101.1, 64 123.9 / 121.7.
+//   down, LDS tiles 256 wide; streaming while all of its tiles are resident, three to a CU, and from more than two LDS tiles
+//   per CU on, but not in between.  64 experts: 8 tokens 49.0 / 46.8, 10 48.4 / 50.3, 15 50.8 / 61.6, 64 57.8 / 75.5; 128: 8
+//   tokens 28.8 / 33.8, 12 40.5 / 42.4, 20 45.9 / 47.3, 24 61.5 / 54.0, 37 66.2 / 63.2, 56 67.8 / 66.0.
+// (The lines were drawn with three and two LDS tiles on a CU, which took longer; where they stand now they cost 4 to 10 % of
+// a product at 10 tokens of 64 experts and 2 to 5 % of the down product at 12 to 20 tokens of 128.)
 inline bool pick_skinny(int64_t rows, int64_t E, bool dense, int64_t N, bool dual, double cus, ProductKernel* out) {
   struct Shape {
     ProductKernel id;

@@ -15,9 +15,9 @@ inline int64_t f32_mtiles(bool dense, int64_t rows, int64_t E, int BM) {
 }
 
 // Rounds over the CUs times the work of a tile, in units of a 64 x 64 tile.  With unequal groups about half a
-// tile per group is padding.  At 4096 rows in 8 groups, 512 x 1024 the rule takes the small tiles; when it was drawn,
-// before either lost 5 to 9 % of its time: gate/up 101 against 120 us, down 62 (544 tiles, three units) against 81 (144 tiles,
-// four units), data gradients 55 and 118 against 74 and 151 us.
+// tile per group is padding.  At 8 groups, 512 x 1024 the rule takes the small tiles, us against the large ones: 2048 rows
+// gate/up 57 and 73, down 38 and 72; 4096 rows 106 and 118, 61 (544 tiles, three units) and 77 (144 tiles, four units);
+// 8192 rows 170 and 179, 94 and 129.
 inline int64_t f32_cost(bool dense, int64_t rows, int64_t E, int64_t N, int BM, int BN, int units,
                         int64_t cus = persistent_grid_size()) {
   const int64_t mt = (rows + BM - 1) / BM + (dense ? 0 : std::min(E, rows) / 2);

@@ -236,8 +236,8 @@ __device__ __forceinline__ void select_by_rows(const RouterSmem& sm, int t, bool
 // workgroup of 1024 threads: 37 tokens, 128 experts 20.3 -> 13.0 us, 14 tokens, 64 experts 13.2 -> 9.4; of 256 threads
 // and 16 tokens: 17.5 -> 12.3 and 12.0 -> 9.0 (the sigmoid without a pass of its own among it, see add_slices).  Four
 // passes cost what one of four lanes does where waves fill each other's latency (1024 threads, 200 tokens: 28.5 and
-// 28.2) and more with a wave per SIMD (64-token workgroups 31.0 against 33.6 us), which therefore keep four lanes from
-// three passes on.
+// 28.2) and more with a wave per SIMD (64-token workgroups 31.0 against 33.6 us): 64 tokens to 256 threads are selected by
+// four lanes each.
 template <int kRouterTokens, int kRouterThreads>
 __device__ __forceinline__ void select_all(const RouterSmem& sm, int nrows, int E, int K) {
   constexpr int kGroups = kRouterThreads / 16;
