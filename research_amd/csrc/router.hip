@@ -1022,8 +1022,8 @@ __global__ __launch_bounds__(kThreads) void router_finish_blocks_kernel(
 // another 16, which keeps the two-byte writes of the transposed matrix at two lanes to a bank.
 // What lies outside the row or the matrix reads as zeros; columns of LDS past the last expert hold anything, and their
 // sums go nowhere.
-// Router calls, us, staged kernel -> here: 2000 x 1384 x 96 118 -> 41, 2931 x 1000 x 24 31 -> 18, 4096 x 1024 x 8 22 -> 16,
-// 300 x 1024 x 8 19 -> 13, 1 x 1024 x 8 19 -> 12, 16384 x 1024 x 8 44 -> 31.  bf16 products in slices of k take 35, 17, 15, 14,
+// Router calls, us, staged kernel -> here: 2000 x 1384 x 96 118 -> 33, 2931 x 1000 x 24 31 -> 18, 4096 x 1024 x 8 22 -> 16,
+// 300 x 1024 x 8 19 -> 13, 1 x 1024 x 8 19 -> 12, 16384 x 1024 x 8 44 -> 27.  bf16 products in slices of k take 35, 17, 15, 14,
 // 6 and 18, with other last bits in one to three of ten thousand logits.
 // ---------------------------------------------------------------------------
 constexpr int kChainColumns = 64;  // of a workgroup that only writes sums: a chain to a wave
@@ -1036,12 +1036,12 @@ inline size_t router_chain_smem_bytes(int cols) {
   return (size_t)2 * (24 + (cols + 15) / 16 * 16) * (kChainRow<NBW> + 2);  // (16 bytes to eight rows)
 }
 
-template <int NBW, int NL>
+template <int NBW, int NL, int D>
 __device__ __forceinline__ void router_chain(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int t0,
                                              int nrows, int H, int E, int col0, int cols, unsigned char* smem,
                                              f32x4_t (&acc)[NBW]) {
   constexpr int kThreads = 256, KC = kChainKC<NBW>, RS = kChainRow<NBW>, XP = KC / 8;  // XP pieces of a token's row
-  constexpr int D = NL == 1 ? 8 : (NL == 2 ? 4 : (NL <= 4 ? 3 : 2)), UNROLL = D % 2 ? 2 * D : D;
+  constexpr int UNROLL = D % 2 ? 2 * D : D;
   static_assert(16 * XP <= kThreads, "a piece of x per thread");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1187,7 +1187,7 @@ __device__ __forceinline__ void router_chain_sums(const uint16_t* __restrict__ x
   const int t0 = token_block * 16, nrows = min(16, tokens - t0), col0 = column_block * kChainColumns;
   const int lane = threadIdx.x & 63, col = col0 + ((int)threadIdx.x >> 6) * 16 + (lane & 15);
   f32x4_t acc[1];
-  router_chain<1, NL>(x, w, t0, nrows, H, E, col0, min(kChainColumns, E - col0), smem_raw, acc);
+  router_chain<1, NL, NL == 1 ? 8 : (NL == 2 ? 4 : 3)>(x, w, t0, nrows, H, E, col0, min(kChainColumns, E - col0), smem_raw, acc);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int t = 4 * (lane >> 4) + i;
@@ -1202,16 +1202,19 @@ __global__ __launch_bounds__(256) void router_chain_sums_kernel(const uint16_t* 
   router_chain_sums<NL>(x, w, tokens, H, E, partial, (int)blockIdx.x, (int)blockIdx.y);
 }
 
-// Projection and epilogue of 16 tokens.
+// Projection and epilogue of 16 tokens.  Held to four waves per SIMD up to 128 experts, with fewer chunks in flight than the
+// sums of a small batch, whose workgroups are alone on their CUs: us with the deep rings (two and three waves) and now,
+// 16384 x 1024 x 8 31.0 and 26.5, 2000 x 1384 x 96 41.1 and 33.4, 8192 x 1600 x 96 63.0 and 55.4; 16384 x 2048 x 248, in
+// chains that need the registers, 305 and 333 at two waves.
 template <int NBW, int NL>
-__global__ __launch_bounds__(256) void router_chain_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBW <= 2 ? 4 : 1))) void router_chain_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias, int tokens, int H,
     int E, int K, float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights,
     float* __restrict__ scores, float* __restrict__ logits_out, void* ws, int score_func) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int t0 = (int)blockIdx.x * 16, lane = threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
   f32x4_t acc[NBW];
-  router_chain<NBW, NL>(x, w, t0, min(16, tokens - t0), H, E, 0, E, smem_raw, acc);
+  router_chain<NBW, NL, NL <= 2 ? 4 : 2>(x, w, t0, min(16, tokens - t0), H, E, 0, E, smem_raw, acc);
   RouterSmem sm = router_smem(smem_raw, E, K, 16);  // (the stages are dead: the loop ends with a barrier)
 #pragma unroll
   for (int b = 0; b < NBW; ++b)
