@@ -237,13 +237,15 @@ __device__ __forceinline__ void select_by_rows(const RouterSmem& sm, int t, bool
 // and 16 tokens: 17.5 -> 12.3 and 12.0 -> 9.0 (the sigmoid without a pass of its own among it, see add_slices).  Four
 // passes cost what one of four lanes does where waves fill each other's latency (1024 threads, 200 tokens: 28.5 and
 // 28.2) and more with a wave per SIMD (64-token workgroups 31.0 against 33.6 us): 64 tokens to 256 threads are selected by
-// four lanes each.
+// four lanes each.  So are the tokens of 16 and 32 experts, of which four lanes hold as few as four and eight.  Router
+// calls, us, sixteen lanes / four: 16 experts top-2, 1 token 6.2 / 5.7, 64 7.1 / 6.7, 200 10.0 / 8.5; 32 experts top-2, 3
+// tokens 6.5 / 6.1, top-8 8.1 / 8.5, 200 tokens top-4 14.3 / 12.2.
 template <int kRouterTokens, int kRouterThreads>
 __device__ __forceinline__ void select_all(const RouterSmem& sm, int nrows, int E, int K) {
   constexpr int kGroups = kRouterThreads / 16;
   static_assert(4 * kRouterTokens <= kRouterThreads, "four lanes to a token");
   const int tid = threadIdx.x;
-  if (kRouterTokens > 2 * kGroups && kRouterThreads < 1024 &&
+  if (((kRouterTokens > 2 * kGroups && kRouterThreads < 1024) || E <= 32) &&
       (E == 16 || E == 32 || E == 64 || E == 128 || E == 256)) {
     const int t = tid >> 2, q = tid & 3, e_begin = q * (E >> 2);
     const bool row_ok = t < nrows;
