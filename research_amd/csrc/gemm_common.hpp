@@ -23,7 +23,28 @@ struct TileRows {
   int rows;  // valid rows in the tile (0 = no such tile)
 };
 
-// Tiles are counted expert by expert, ceil(group_size / BM) m-tiles each.  group_scan computes, in
+// m-tiles of a group of n rows.  With extra == 0: BM rows each, the last one what is left.  With extra rows to a tile
+// (beyond BM) the rows that whole tiles leave over are spread over these, `extra` to each from the first one on, and
+// only rows that do not fit in there start a tile of their own.
+__host__ __device__ __forceinline__ int group_mtiles(int n, int BM, int extra) {
+  if (n <= 0) return 0;
+  const int whole = n < BM ? 1 : n / BM;
+  return whole + (n - whole * BM > extra * whole ? 1 : 0);
+}
+// rows [first, first + rows) of the group: its m-tile i
+struct TileSpan {
+  int first, rows;
+};
+__host__ __device__ __forceinline__ TileSpan group_mtile(int n, int i, int BM, int extra) {
+  const int whole = n < BM ? 1 : n / BM, left = n - whole * BM;
+  const bool fits = left <= extra * whole;
+  const int spread = fits && left > 0 ? left : 0, tiles = whole + (fits ? 0 : 1);
+  auto start = [&](int t) { return t * BM + (t * extra < spread ? t * extra : spread); };
+  const int first = start(i);
+  return {first, (i + 1 < tiles ? start(i + 1) : n) - first};
+}
+
+// Tiles are counted expert by expert, group_mtiles each.  group_scan computes, in
 // every lane of the calling wave, the tile counts of the lane's own experts, their exclusive
 // prefix and the total; locate_tile then finds the expert and row range of m-tile `mt`.
 // E <= JTMOE_MAX_EXPERTS.
@@ -34,15 +55,14 @@ struct GroupScan {
   int total;  // tiles of all experts
 };
 
-__device__ __forceinline__ GroupScan group_scan(int BM, const int32_t* __restrict__ group_sizes, int E) {
+__device__ __forceinline__ GroupScan group_scan(int BM, const int32_t* __restrict__ group_sizes, int E, int extra, int lane) {
   GroupScan g;
-  const int lane = threadIdx.x & 63;
   int local = 0;
 #pragma unroll
   for (int j = 0; j < GroupScan::kPer; ++j) {
     const int e = lane * GroupScan::kPer + j;
     g.n[j] = e < E ? group_sizes[e] : 0;
-    g.tiles[j] = (g.n[j] + BM - 1) / BM;
+    g.tiles[j] = group_mtiles(g.n[j], BM, extra);
     local += g.tiles[j];
   }
   int incl = local;
@@ -56,13 +76,16 @@ __device__ __forceinline__ GroupScan group_scan(int BM, const int32_t* __restric
   return g;
 }
 
+__device__ __forceinline__ GroupScan group_scan(int BM, const int32_t* __restrict__ group_sizes, int E) {
+  return group_scan(BM, group_sizes, E, 0, threadIdx.x & 63);
+}
+
 __device__ __forceinline__ TileRows locate_tile(const GroupScan& g, int mt, int BM,
-                                                const int32_t* __restrict__ offsets) {
+                                                const int32_t* __restrict__ offsets, int extra, int lane) {
   TileRows r;
   r.expert = 0;
   r.row0 = 0;
   r.rows = 0;
-  const int lane = threadIdx.x & 63;
   int first = g.first;
   int last = first;
 #pragma unroll
@@ -85,9 +108,14 @@ __device__ __forceinline__ TileRows locate_tile(const GroupScan& g, int mt, int 
   local_tile = __shfl(local_tile, owner);
   rows_e = __shfl(rows_e, owner);
   r.expert = expert;
-  r.row0 = offsets[expert] + local_tile * BM;
-  r.rows = min(BM, rows_e - local_tile * BM);
+  const TileSpan span = group_mtile(rows_e, local_tile, BM, extra);
+  r.row0 = offsets[expert] + span.first;
+  r.rows = span.rows;
   return r;
+}
+
+__device__ __forceinline__ TileRows locate_tile(const GroupScan& g, int mt, int BM, const int32_t* __restrict__ offsets) {
+  return locate_tile(g, mt, BM, offsets, 0, threadIdx.x & 63);
 }
 
 // m-tile `mt` of a grouped (or, with group_sizes == nullptr, dense) row range.  Every lane of the
@@ -233,13 +261,32 @@ inline double spread_mtiles(int64_t rows, int64_t E, bool dense, int BM) {
   return groups * (tiles_upto(hi) - tiles_upto(lo)) / (hi - lo);
 }
 
+// m-tiles of 256 rows, each of up to 64 more where that spares tiles (group_mtiles; the stream kernel takes them only
+// where they spare a round), by the two estimates: what a group's
+// whole tiles leave over spread evenly over 256 rows, and groups spread evenly over mean +- 3 sqrt(mean).
+inline double tall_mtiles(int64_t rows, int64_t E, bool dense, bool spread) {
+  if (dense) return (double)group_mtiles((int)rows, 256, 64);
+  const double groups = (double)E * (1.0 - std::exp(-(double)rows / (double)E)), mean = (double)rows / groups;
+  const double reach = spread ? 3.0 * std::sqrt(mean) : 128.0;
+  double tiles = 0.0;
+  for (int i = 0; i < 32; ++i) {
+    const int n = (int)(mean + reach * ((i + 0.5) / 16.0 - 1.0));
+    tiles += n > 0 ? group_mtiles(n, 256, 64) : 1;
+  }
+  return groups * tiles / 32.0;
+}
+// what a launch of 256-row tiles of N columns counts, by either estimate
+inline double whole_tiles(int64_t rows, int64_t E, bool dense, double ntiles, double cus, bool spread, bool tall) {
+  const double plain = (spread ? spread_mtiles(rows, E, dense, 256) : expected_mtiles(rows, E, dense, 256)) * ntiles;
+  return plain <= cus || !tall ? plain : std::fmin(plain, tall_mtiles(rows, E, dense, spread) * ntiles);
+}
+
 // 128 x 128 tiles against 256 x 256 ones, by rounds over the CUs: a round of 512 half tiles takes 0.57 of a round of
 // 256 whole ones, a last round of at most 256 of them 0.42, the launch 0.12 more; half tiles read their operands
 // twice as often, so beyond one per CU they are taken only where that is 15 % less.  Down products: one half tile
 // per CU 40 us against 63 (2048 tokens, shared 2816; 64-deep steps 41), two per CU with 64-deep steps 55 against 64
 // (4096 tokens; 32-deep 69); 8192 rows x 2048 -> 1024 in 8 groups: 57 against 56 (576 tiles, whole ones kept);
-// 16384 rows in 16 groups x 2816 -> 1024 (1088 against 288 tiles: the whole ones start a second round for 32 of them):
-// 145 against 152 inside the layer call, whose gate/up launch then clocks lower: 372 against 374 for the call.  The data
+// 16384 rows in 16 groups x 2816 -> 1024 (1088 against 256 tiles of up to 320 rows): 109 against 87.  The data
 // gradients follow the same line (figures at DgradHalfCfg and DgradHalfDeepCfg); on the wrong side of it 32768
 // rows in 64 groups x 2048 -> 1408 would take 262 us against 228.
 enum class HalfTiles { kNone, kOnePerCu, kRounds };
@@ -248,12 +295,13 @@ inline double half_tile_rounds(double half, double cus) {
   const double rounds = std::floor(half / (2 * cus)), rest = half - rounds * 2 * cus;
   return 0.12 + 0.57 * rounds + (rest <= 0.0 ? 0.0 : (rest <= cus ? 0.42 : 0.57));
 }
-inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, double cus) {
+// (tall: with the 256-row tiles counted as the stream kernel takes them, of up to 320 rows)
+inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, double cus, bool tall = true) {
   const double half_n = (double)((N + 127) / 128), full_n = (double)((N + 255) / 256);
   if (expected_mtiles(rows, E, dense, 128) * half_n <= cus) return HalfTiles::kOnePerCu;
   auto pays = [cus](double half, double full) { return 1.15 * half_tile_rounds(half, cus) < std::ceil(full / cus); };
-  return pays(expected_mtiles(rows, E, dense, 128) * half_n, expected_mtiles(rows, E, dense, 256) * full_n) &&
-                 pays(spread_mtiles(rows, E, dense, 128) * half_n, spread_mtiles(rows, E, dense, 256) * full_n)
+  return pays(expected_mtiles(rows, E, dense, 128) * half_n, whole_tiles(rows, E, dense, full_n, cus, false, tall)) &&
+                 pays(spread_mtiles(rows, E, dense, 128) * half_n, whole_tiles(rows, E, dense, full_n, cus, true, tall))
              ? HalfTiles::kRounds
              : HalfTiles::kNone;
 }
@@ -271,7 +319,8 @@ inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, doub
 // tokens, 64 experts top-8: two rounds of routed tiles by one, 2.3 by the other; down jointly 3 % more a call), and with
 // three standard deviations more groups than are to be expected: with a few rows per group each is a tile, and a round more
 // streams the experts' matrices a second time (backward of 24 tokens, 64 experts top-8, 2048 x 1408, shared 2816: dX jointly
-// 194 us where 63 groups had a row, 121 + 39 apart; of 27 tokens 595 the pass against 555).
+// 194 us where 63 groups had a row, 121 + 39 apart; of 27 tokens 595 the pass against 555).  The 256-row tiles are counted
+// without rows beyond these, with which the lines were drawn.
 inline HalfTiles joint_tiles(int64_t rows, int64_t E, int64_t N, int64_t T, int64_t N1, double longer, double cus,
                              double one_per_cu, bool dual = false) {
   auto across = [dual](int64_t n, int bn) { return (double)(dual ? (n + 127) / 128 : (n + bn - 1) / bn); };
@@ -281,8 +330,8 @@ inline HalfTiles joint_tiles(int64_t rows, int64_t E, int64_t N, int64_t T, int6
     return h == HalfTiles::kRounds && !dual ? half_tile_rounds(half, cus) : std::ceil(full / cus);
   };
   if (expected_mtiles(rows, E, false, 128) * across(N, 128) + dense_tiles(128) <= cus) return HalfTiles::kOnePerCu;
-  const HalfTiles routed = half_tiles(rows, E, false, N, cus);
-  const double shared = longer * alone(half_tiles(T, 1, true, N1, cus), dense_tiles(128), dense_tiles(256));
+  const HalfTiles routed = half_tiles(rows, E, false, N, cus, /*tall=*/false);
+  const double shared = longer * alone(half_tiles(T, 1, true, N1, cus, /*tall=*/false), dense_tiles(128), dense_tiles(256));
   const double mean = (double)rows / (double)E, empty = std::exp(-mean);
   const double more_groups =
       std::fmin((double)E * empty, 3.0 * std::sqrt((double)E * empty * (1.0 - (1.0 + mean) * empty)));

@@ -19,7 +19,7 @@ enum class ProductKernel {
   kHalf,          // 128 x 128 tiles
   kHalfTail,
   kHalfDeep,
-  kRows256,       // 256-row tiles: gate/up in the four-stage kernel, the others persistent with two stages
+  kRows256,       // 256-row tiles, of up to 320 rows (grouped_gemm_stream.hpp)
   kRows256Tail,
   kRows256Short,  // gate/up whose reduction is too short for four stages
   kRows256ShortTail,

@@ -218,9 +218,10 @@ int launch_fast(const void* a, const void* b0, const void* b1, void* c, const in
 }
 
 
-// The stream kernel (grouped_gemm_stream.hpp) for the gate/up launch of the 256-row configurations: the
-// same tiles as one software pipeline through all tiles of a workgroup, results written straight from
-// the accumulators.  Its envelope is narrower than launch_fast's (see stream_ok).
+// The stream kernel (grouped_gemm_stream.hpp): one software pipeline through all tiles of a workgroup, results written
+// straight from the accumulators.  Its envelope is narrower than launch_fast's (see stream_ok).  256-row tiles run in
+// one workgroup per CU for the whole launch (0.5 to 2 % faster than in workgroups of four tiles each), half tiles in
+// workgroups of four.
 template <typename Cfg>
 int launch_stream(const void* a, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, hipStream_t stream,
@@ -241,11 +242,11 @@ int launch_stream(const void* a, const void* b0, const void* b1, void* c, const 
   const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles_grid = gemm_grid(mtiles, nt);
   if (tiles_grid >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: grid too large");
-  const PersistentSchedule ps = persistent_schedule(tiles_grid, workgroups_per_cu * persistent_grid_size(), 4);
+  const PersistentSchedule ps =
+      persistent_schedule(tiles_grid, workgroups_per_cu * persistent_grid_size(), Cfg::XROWS ? 0 : 4);
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes, stream>>>(
       static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
-      static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim, (int)N, (int)mtiles, (int)nt,
-      row_map, row_div, (int)a_rows, static_cast<uint16_t*>(save0), static_cast<uint16_t*>(save1), ps.window, ps.chunk);
+      static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim, (int)N, (int)nt, row_map, row_div, (int)a_rows, static_cast<uint16_t*>(save0), static_cast<uint16_t*>(save1), ps.window, ps.chunk);
   return JTMOE_OK;
 }
 
@@ -262,7 +263,7 @@ struct RoutedProblem {
 DenseProblem dense_problem(const RoutedProblem& s) {
   return {static_cast<const uint16_t*>(s.a), nullptr, static_cast<const uint16_t*>(s.b0), static_cast<const uint16_t*>(s.b1),
           static_cast<uint16_t*>(s.c), static_cast<uint16_t*>(s.save0), static_cast<uint16_t*>(s.save1), (int)s.rows,
-          (int)s.K, (int)s.N, 0, 0};
+          (int)s.K, (int)s.N, 0};
 }
 
 template <typename Cfg>
@@ -277,15 +278,14 @@ int launch_joint(const RoutedProblem& r, DenseProblem dp, hipStream_t stream) {
   if (attr_err != hipSuccess)
     return fail(JTMOE_ELAUNCH, "grouped gemm: kernel set-up: %s", hipGetErrorString(attr_err));
   const int64_t mtiles = max_m_tiles(r.rows, r.E, Cfg::BM), nt = (r.N + Cfg::BN - 1) / Cfg::BN;
-  dp.mtiles = (dp.rows + Cfg::BM - 1) / Cfg::BM;
   dp.ntiles = (dp.n + Cfg::BN - 1) / Cfg::BN;
-  const int64_t tiles_grid = gemm_grid(mtiles, nt) + gemm_grid(dp.mtiles, dp.ntiles);
+  const int64_t tiles_grid = gemm_grid(mtiles, nt) + gemm_grid((dp.rows + Cfg::BM - 1) / Cfg::BM, dp.ntiles);
   if (tiles_grid >= ((int64_t)1 << 28)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: grid too large");
   const int64_t grid = std::min<int64_t>(tiles_grid, persistent_grid_size());
   kernel<<<(unsigned)grid, Cfg::NT, kSmem, stream>>>(
       static_cast<const uint16_t*>(r.a), static_cast<const uint16_t*>(r.b0), static_cast<const uint16_t*>(r.b1),
-      static_cast<uint16_t*>(r.c), r.group_sizes, r.offsets, (int)r.E, (int)r.rows, (int)r.K, (int)r.N, (int)mtiles,
-      (int)nt, r.row_map, r.row_div, (int)r.a_rows, static_cast<uint16_t*>(r.save0), static_cast<uint16_t*>(r.save1), dp);
+      static_cast<uint16_t*>(r.c), r.group_sizes, r.offsets, (int)r.E, (int)r.rows, (int)r.K, (int)r.N, (int)nt,
+      r.row_map, r.row_div, (int)r.a_rows, static_cast<uint16_t*>(r.save0), static_cast<uint16_t*>(r.save1), dp);
   return JTMOE_OK;
 }
 
@@ -460,9 +460,16 @@ int launch_down_fast(const void* act, const void* down, const int32_t* group_siz
   switch (k) {
     case ProductKernel::kHalf: return JT_DOWN(launch_stream, DownHalfCfg), 2);
     case ProductKernel::kHalfDeep: return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
-    case ProductKernel::kRows256: return JT_DOWN(launch_fast, DownCfg));
-    default: return JT_DOWN(launch_fast, DownTailCfg));
+    default: break;
   }
+  // 256-row tiles; a reduction too short for the stream kernel, or a result past its limit: the kernel without it
+  const bool tail = k == ProductKernel::kRows256Tail;
+  if (stream_ok<DownStreamTailCfg>(rows, I, H, nullptr, 1)) {
+    if (tail) return JT_DOWN(launch_stream, DownStreamTailCfg));
+    return JT_DOWN(launch_stream, DownStreamCfg));
+  }
+  if (tail) return JT_DOWN(launch_fast, DownTailCfg));
+  return JT_DOWN(launch_fast, DownCfg));
 #undef JT_DOWN
 }
 

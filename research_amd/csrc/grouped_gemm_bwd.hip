@@ -185,11 +185,11 @@ int launch_nt_stream(const void* a0, const void* a1, const void* b0, const void*
   const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles_grid = gemm_grid(mtiles, nt);
   if (tiles_grid >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");
-  const PersistentSchedule ps = persistent_schedule(tiles_grid, persistent_grid_size(), 4);
+  const PersistentSchedule ps = persistent_schedule(tiles_grid, persistent_grid_size(), Cfg::XROWS ? 0 : 4);
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes, stream>>>(
       static_cast<const uint16_t*>(a0), static_cast<const uint16_t*>(a1), static_cast<const uint16_t*>(b0),
       static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim,
-      (int)N, (int)mtiles, (int)nt, row_map, row_div, (int)a_rows, segs, ps.window, ps.chunk);
+      (int)N, (int)nt, row_map, row_div, (int)a_rows, segs, ps.window, ps.chunk);
   return JTMOE_OK;
 }
 
@@ -204,8 +204,7 @@ ProductKernel data_gradient_kernel(int64_t rows, int64_t Kdim, int64_t N, int64_
   return Kdim % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
 }
 
-// 256-row tiles of the joint launch: 64-deep steps in two stages (as fast as grouped_gemm_nt_kernel there, see
-// DgradStreamCfg).  Both reductions fill its pipeline and both results stay below its limit.
+// (both reductions fill the stream kernel's pipeline and both results stay below its limit)
 ProductKernel joint_data_gradient_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t T, int64_t Is, int segs,
                                          double cus) {
   const int64_t k0 = segs == 1 ? H : I, k1 = segs == 1 ? H : Is, n0 = segs == 1 ? I : H, n1 = segs == 1 ? Is : H;
@@ -219,7 +218,7 @@ ProductKernel joint_data_gradient_kernel(int64_t rows, int64_t H, int64_t I, int
     case HalfTiles::kOnePerCu:
       return least >= 2 * DgradHalfDeepCfg::NSTAGE ? ProductKernel::kHalfDeep : ProductKernel::kGeneral;
     case HalfTiles::kRounds:
-      if (least < 2 * DgradJointCfg::NSTAGE) return ProductKernel::kGeneral;
+      if (least < 2 * DgradStreamCfg::NSTAGE) return ProductKernel::kGeneral;
       return k0 % 64 == 0 && k1 % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
     default: return ProductKernel::kGeneral;
   }
@@ -243,10 +242,10 @@ int launch_nt_joint(const NtProblem& p, const int32_t* group_sizes, const int32_
   const int64_t grid = std::min<int64_t>(tiles_grid, persistent_grid_size());
   auto in = [](const void* q) { return static_cast<const uint16_t*>(q); };
   const DenseProblem dp{in(s.a0), in(s.a1), in(s.b0), in(s.b1), static_cast<uint16_t*>(s.c), nullptr, nullptr,
-                        (int)s.rows, (int)s.Kdim, (int)s.N, (int)mt1, (int)nt1};
+                        (int)s.rows, (int)s.Kdim, (int)s.N, (int)nt1};
   kernel<<<(unsigned)grid, Cfg::NT, L::kSmemBytes, stream>>>(
       in(p.a0), in(p.a1), in(p.b0), in(p.b1), static_cast<uint16_t*>(p.c), group_sizes, offsets, (int)E, (int)p.rows,
-      (int)p.Kdim, (int)p.N, (int)mtiles, (int)nt, segs, dp);
+      (int)p.Kdim, (int)p.N, (int)nt, segs, dp);
   return JTMOE_OK;
 }
 }  // namespace
@@ -264,8 +263,8 @@ int launch_gemm_nt_joint(int dtype, const NtProblem& p, const int32_t* group_siz
                          const NtProblem& s, int segs, hipStream_t stream) {
   switch (gemm_nt_joint(dtype, p, E, s, segs)) {
     case ProductKernel::kHalfDeep: return launch_nt_joint<DgradHalfDeepCfg>(p, group_sizes, offsets, E, s, segs, stream);
-    case ProductKernel::kRows256: return launch_nt_joint<DgradJointCfg>(p, group_sizes, offsets, E, s, segs, stream);
-    case ProductKernel::kRows256Tail: return launch_nt_joint<DgradJointTailCfg>(p, group_sizes, offsets, E, s, segs, stream);
+    case ProductKernel::kRows256: return launch_nt_joint<DgradStreamCfg>(p, group_sizes, offsets, E, s, segs, stream);
+    case ProductKernel::kRows256Tail: return launch_nt_joint<DgradStreamTailCfg>(p, group_sizes, offsets, E, s, segs, stream);
     default: return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): no joint launch at this size");
   }
 }
@@ -277,13 +276,17 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
   const bool dense = group_sizes == nullptr;
   const bool fast = dtype == JTMOE_BF16 && (row_map ? a_rows : rows) * Kdim < kOperandLimit && aligned16(a0) &&
                     aligned16(b0) && (segs == 1 || (aligned16(a1) && aligned16(b1))) && aligned16(c);
+  const bool streams = (Kdim + 63) / 64 * segs >= 2 * DgradStreamCfg::NSTAGE && rows * N * 2 <= (int64_t)0x7ffe0000 &&
+                       (row_map == nullptr || (rows < ((int64_t)1 << 27) && row_div >= 1 && row_div <= 32));
 #define JT_NT(LAUNCH, CFG) \
   LAUNCH<CFG>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div, a_rows, segs, stream)
   switch (fast ? data_gradient_kernel(rows, Kdim, N, E, dense, segs, persistent_grid_size()) : ProductKernel::kGeneral) {
     case ProductKernel::kHalfDeep: return JT_NT(launch_nt_stream, DgradHalfDeepCfg);
     case ProductKernel::kHalf: return JT_NT(launch_nt_fast, DgradHalfCfg);
-    case ProductKernel::kRows256: return JT_NT(launch_nt_fast, DgradCfg);
-    case ProductKernel::kRows256Tail: return JT_NT(launch_nt_fast, DgradTailCfg);
+    // 256-row tiles; a reduction too short for the stream kernel, or a result past its limit: the kernel without it
+    case ProductKernel::kRows256: return streams ? JT_NT(launch_nt_stream, DgradStreamCfg) : JT_NT(launch_nt_fast, DgradCfg);
+    case ProductKernel::kRows256Tail:
+      return streams ? JT_NT(launch_nt_stream, DgradStreamTailCfg) : JT_NT(launch_nt_fast, DgradTailCfg);
     default: break;
   }
 #undef JT_NT

@@ -124,8 +124,10 @@ struct DmaGemmCfg {
   // 32 = raise the wave priority around the MFMA burst, 64 = ask the scheduler to interleave
   // one MFMA with up to three LDS reads, 128 = B tiles in 4 x 64 blocks, 2048 = (persistent kernel) results written
   // straight from transposed accumulators instead of through LDS, 4096 = non-temporal loads of B, 8192 / 16384 = 8 / 2 m-tiles per group of the tile order instead of 4, 32768 = non-temporal stores of the result,
-  // 65536 = (persistent and stream kernels) K may end inside a step; dual ones are for K % 64 != 0 only (silu_gate)
+  // 65536 = (persistent and stream kernels) K may end inside a step; dual ones are for K % 64 != 0 only (silu_gate),
+  // 131072 = (stream kernel) tiles of up to 64 rows more than BM
   static constexpr int OPT = OPT_;
+  static constexpr int XROWS = (OPT_ & 131072) ? 64 : 0;
   static constexpr bool kDual = kDual_;
   static constexpr int BNE = kDual ? 2 * BN : BN;  // columns of the B tile in LDS
   static constexpr int NSUB = BNE / 128;           // 128-column sub-tiles of B
@@ -135,7 +137,7 @@ struct DmaGemmCfg {
   static constexpr int TNO = kDual ? TN / 2 : TN;
   static constexpr int WNO = TNO * 32;
   static constexpr int CPRA = BK / 8;  // 16-byte chunks per A row
-  static constexpr int A_BYTES = BM * BK * 2;
+  static constexpr int A_BYTES = (BM + XROWS) * BK * 2;
   static constexpr int BSUB_BYTES = BK * 256;
   static constexpr int STAGE_BYTES = A_BYTES + NSUB * BSUB_BYTES;
   static constexpr int A_LOADS = BM * CPRA / NT;   // per thread per stage
@@ -162,6 +164,7 @@ struct DmaGemmCfg {
   static_assert(!kDual || (TN % 2 == 0 && BN == 128), "dual tiles: one sub-tile per matrix");
   static_assert(NSTAGE >= 2 && (NSTAGE - 2) * LPS < 64, "vmcnt is a 6-bit counter");
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
+  static_assert(XROWS == 0 || (WAVES_M == 2 && TM == 4 && NT == 512 && XROWS * CPRA <= NT), "a fifth row block per wave");
 };
 
 // two fp32 values -> their bf16 roundings packed in one dword (lo in the low half): one hardware conversion
@@ -181,13 +184,15 @@ __device__ __forceinline__ unsigned pack_bf16x2(float lo, float hi) {
 // 0x7ffe0000 bytes): one 32-bit offset per row, the column of each store as an immediate, and rows
 // past the end of the group (or columns past N) get the offset 0x7fff0000, which lies outside every
 // admitted result, so the hardware drops the store.
-// With save0 / save1 (dual tiles only) the two rounded products are written as well.
-template <typename Cfg>
-__device__ __forceinline__ void store_transposed_accumulators(const f32x16_t (&acc)[Cfg::TM][Cfg::TN], int wm, int wn,
-                                                              int row0, int rows, int n0, int N, int out_rows_total,
+// With save0 / save1 (dual tiles only) the two rounded products are written as well.  Block mi of the wave's TMX holds
+// the 32 rows from first_row + mi * row_step on.
+template <typename Cfg, int TMX>
+__device__ __forceinline__ void store_transposed_accumulators(const f32x16_t (&acc)[TMX][Cfg::TN], int first_row,
+                                                              int row_step, int wn, int row0, int rows, int n0, int N,
+                                                              int out_rows_total,
                                                               uint16_t* __restrict__ C, uint16_t* __restrict__ save0,
                                                               uint16_t* __restrict__ save1) {
-  constexpr int TM = Cfg::TM, TN = Cfg::TN, WM = Cfg::WM, TNO = Cfg::TNO, WNO = Cfg::WNO;
+  constexpr int TN = Cfg::TN, TNO = Cfg::TNO, WNO = Cfg::WNO;
   constexpr bool kDual = Cfg::kDual, kTail = (Cfg::OPT & 65536) != 0;
   // (the lane id is taken afresh so that nothing of the epilogue's addressing is kept in registers
   // through the k loops, where every register is spoken for)
@@ -201,8 +206,10 @@ __device__ __forceinline__ void store_transposed_accumulators(const f32x16_t (&a
     uint16_t* const out = pass == 0 ? C : (pass == 1 ? save0 : save1);
     const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, out_rows_total * N * 2, kBufferFlags);
 #pragma unroll
-    for (int mi = 0; mi < TM; ++mi) {
-      const int r = wm * WM + mi * 32 + (lane_e & 31);
+    for (int mi = 0; mi < TMX; ++mi) {
+      const int block_row = first_row + mi * row_step;
+      if (block_row >= rows) continue;
+      const int r = block_row + (lane_e & 31);
       const int row_off = r < rows ? ((row0 + r) * N + col0 + 8 * half) * 2 : 0x7fff0000;
 #pragma unroll
       for (int jj = 0; jj < TNO; ++jj) {
@@ -783,7 +790,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_dma_persistent_kernel(
     }
 
     if constexpr (kDirect) {
-      store_transposed_accumulators<Cfg>(acc, wm, wn, out_row0, out_rows, out_n0, N, dense_rows, C, save0, save1);
+      store_transposed_accumulators<Cfg, TM>(acc, wm * WM, 32, wn, out_row0, out_rows, out_n0, N, dense_rows, C, save0, save1);
       if (nxt.rows <= 0) break;
       cur = nxt;
       continue;

@@ -9,9 +9,12 @@
 //     stage: the first fragments of step c + 1 are read from LDS while the matrix cores work on the
 //     last sub-step of step c, so no wave starts a step by waiting for LDS.
 //   * The stream of k steps does not stop at the end of a tile: the loads of the next tile's first
-//     steps are issued during the last steps of the current one, and its first fragments are in
-//     registers before the epilogue.  The epilogue writes the accumulators straight to memory (they
-//     hold transposed blocks, so a lane owns runs of neighbouring columns): no LDS, no barrier.
+//     steps are issued during the last steps of the current one.  The epilogue writes the accumulators
+//     straight to memory (they hold transposed blocks, so a lane owns runs of neighbouring columns):
+//     no LDS, no barrier.
+//   * A tile takes up to 64 rows beyond BM (OPT & 131072) where that spares tiles: a fifth block of 32
+//     rows per wave, one more operand load per stage, read and multiplied only by the tiles that have
+//     such rows.  The accumulators are then 160 of a wave's 256 registers.
 //   * Nothing in the steady state returns data to vector registers through the memory pipe (the
 //     row map of the next tile arrives by LDS-DMA as well, group sizes and offsets are read from a copy
 //     in LDS), so the compiler never inserts a wait that drains the operand loads.
@@ -43,7 +46,7 @@ struct StreamLayout {
   static constexpr int kGroupBase = kRowBufBase + kRowBufBytes;  // group sizes, then first rows: 2 x JTMOE_MAX_EXPERTS ints
   static constexpr int kSmemBytes = kGroupBase + 2 * JTMOE_MAX_EXPERTS * 4;
   static_assert(kSmemBytes <= 160 * 1024, "LDS budget");
-  static_assert(Cfg::BM <= Cfg::NT, "one row-map entry per thread");
+  static_assert(Cfg::BM + Cfg::XROWS <= Cfg::NT, "one row-map entry per thread");
 };
 
 // A second product in the same launch: one dense group with its own matrices, width and reduction length, as the
@@ -51,7 +54,7 @@ struct StreamLayout {
 struct DenseProblem {
   const uint16_t *a0, *a1, *b0, *b1;  // a1 / b1: the up matrix or the second segment
   uint16_t *c, *save0, *save1;
-  int rows, k, n, mtiles, ntiles;
+  int rows, k, n, ntiles;
 };
 
 // How the workgroups of an XCD share out the tiles of two products (kJoint): the dense product's tiles first, dealt
@@ -84,13 +87,18 @@ template <typename Cfg, bool kNT, bool kJoint = false>
 __device__ __forceinline__ void stream_gemm_body(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes,
-    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n,
+    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int ntiles_n,
     const int32_t* __restrict__ row_map, int row_div, int a_rows, uint16_t* __restrict__ save0,
     uint16_t* __restrict__ save1, int segs, int window, int chunk, const DenseProblem& dp) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, NS = Cfg::NSTAGE;
-  constexpr int TM = Cfg::TM, TN = Cfg::TN, WM = Cfg::WM, WN = Cfg::WN;
+  constexpr int TM = Cfg::TM, TN = Cfg::TN, WN = Cfg::WN;
   constexpr int CPRA = Cfg::CPRA, KK = BK / 16, LPS = Cfg::LPS;
   constexpr bool kDual = Cfg::kDual;
+  // A wave's row blocks of 32 lie kRowStep apart, those of the waves above one another in turn, so that the rows of
+  // a tile that is not full are spread over all of them.  X: rows that a group's last tile may have beyond BM, a
+  // block more per wave.
+  constexpr int X = Cfg::XROWS, TMX = TM + (X ? 1 : 0), kRowStep = Cfg::WAVES_M * 32;
+  constexpr int kManyRounds = 8;
   using L = StreamLayout<Cfg>;
   static_assert(KK % 2 == 0, "fragment double buffer wants an even number of sub-steps");
   static_assert(kNT || (Cfg::OPT & 128) != 0, "weight tiles in 4 x 64 blocks");
@@ -110,6 +118,13 @@ __device__ __forceinline__ void stream_gemm_body(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WAVES_N, wn = wave - wm * Cfg::WAVES_N;
+  // What is computed from the lane once per tile takes the lane id afresh, so that none of it stays in registers
+  // through the k loops, which have none to spare.
+  auto fresh_lane = [] {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+  };
   const bool gather = row_map != nullptr;
   auto seg_steps = [](int k) { return kTail ? (k + BK - 1) / BK : k / BK; };  // k steps of one segment
   const int nk_segs = kNT ? segs : 1;
@@ -119,24 +134,43 @@ __device__ __forceinline__ void stream_gemm_body(
   // that no look-up touches global memory while operand loads are in flight.
   int* const gs_l = reinterpret_cast<int*>(smem_raw + L::kGroupBase);
   int* const row0_l = gs_l + JTMOE_MAX_EXPERTS;
-  int real_mtiles = mtiles;
   if (group_sizes) {
     for (int e = tid; e < JTMOE_MAX_EXPERTS; e += NT) {
       gs_l[e] = e < E ? group_sizes[e] : 0;
       row0_l[e] = e < E ? offsets[e] : 0;
     }
     __syncthreads();
-    real_mtiles = __builtin_amdgcn_readfirstlane(group_scan(BM, gs_l, JTMOE_MAX_EXPERTS).total);
+  }
+  auto mtiles_with = [&](int x) {
+    return group_sizes ? __builtin_amdgcn_readfirstlane(group_scan(BM, gs_l, JTMOE_MAX_EXPERTS, x, lane).total)
+                       : group_mtiles(dense_rows, BM, x);
+  };
+  const int lead = kJoint ? max(1, (2 * dp.k + Kdim) / (2 * Kdim)) : 0;  // how many grouped tiles last as long as a dense one
+  // Taller tiles where they spare a round (a tile with X rows takes up to a quarter longer: with 24 groups of 366 rows,
+  // two of them below 320, and four rounds either way they cost a forward pass 2.3 %), or where there are many rounds, of
+  // which they are the cheaper work.
+  int extra = 0, real_mtiles = mtiles_with(0), dense_mtiles = kJoint ? group_mtiles(dp.rows, BM, 0) : 0;
+  if (X != 0) {
+    const int workgroups = chunk > 0 ? 8 * window : (int)gridDim.x;
+    auto rounds = [&](int mt, int dense_mt) {
+      return (mt * ntiles_n + (kJoint ? dense_mt * dp.ntiles * lead : 0) + workgroups - 1) / workgroups;
+    };
+    const int tall = mtiles_with(X), dense_tall = kJoint ? group_mtiles(dp.rows, BM, X) : 0;
+    const int plain_rounds = rounds(real_mtiles, dense_mtiles);
+    if (plain_rounds >= kManyRounds || rounds(tall, dense_tall) < plain_rounds) {
+      extra = X;
+      real_mtiles = tall;
+      dense_mtiles = dense_tall;
+    }
   }
   const int total = real_mtiles * ntiles_n;
   const int per_xcd = (total + 7) >> 3;
   const int xcd = (int)blockIdx.x & 7;
   int idx = (int)blockIdx.x >> 3, stride = max(1, (int)gridDim.x >> 3), left = 0x7fffffff;
   // kJoint: this XCD's range of either product, the odd tiles of the two at opposite ends of the XCDs
-  const int total1 = kJoint ? dp.mtiles * dp.ntiles : 0;
+  const int total1 = kJoint ? dense_mtiles * dp.ntiles : 0;
   const int first0 = (xcd * total) >> 3, count0 = (((xcd + 1) * total) >> 3) - first0;
   const int first1 = (xcd * total1 + 7) >> 3, count1 = (((xcd + 1) * total1 + 7) >> 3) - first1;
-  const int lead = kJoint ? max(1, (2 * dp.k + Kdim) / (2 * Kdim)) : 0;
   int place = 0;  // kJoint: how many tiles this workgroup has looked up
   if (chunk > 0) {
     idx = (idx / window) * (window * chunk) + idx % window;
@@ -157,7 +191,7 @@ __device__ __forceinline__ void stream_gemm_body(
       if (j < 0) return t;
       second = j < count1;
       logical = second ? first1 + j : first0 + (j - count1);
-      mts = second ? dp.mtiles : real_mtiles;
+      mts = second ? dense_mtiles : real_mtiles;
       nts = second ? dp.ntiles : ntiles_n;
     } else if (i >= per_xcd || logical >= total) {
       return t;
@@ -170,16 +204,19 @@ __device__ __forceinline__ void stream_gemm_body(
     const int mt = group * Cfg::GROUP_M + (in_group - nt * gm);
     if (second) {
       t.expert = -1;
-      t.row0 = mt * BM;
-      t.rows = min(BM, dp.rows - mt * BM);
+      const TileSpan span = group_mtile(dp.rows, mt, BM, extra);
+      t.row0 = span.first;
+      t.rows = span.rows;
     } else if (group_sizes) {
-      const TileRows tr = locate_tile(group_scan(BM, gs_l, JTMOE_MAX_EXPERTS), mt, BM, row0_l);
+      const int l = fresh_lane();
+      const TileRows tr = locate_tile(group_scan(BM, gs_l, JTMOE_MAX_EXPERTS, extra, l), mt, BM, row0_l, extra, l);
       t.expert = __builtin_amdgcn_readfirstlane(tr.expert);
       t.row0 = __builtin_amdgcn_readfirstlane(tr.row0);
       t.rows = __builtin_amdgcn_readfirstlane(tr.rows);
     } else {
-      t.row0 = mt * BM;
-      t.rows = min(BM, dense_rows - mt * BM);
+      const TileSpan span = group_mtile(dense_rows, mt, BM, extra);
+      t.row0 = span.first;
+      t.rows = span.rows;
     }
     t.n0 = nt * BN;
     return t;
@@ -197,23 +234,30 @@ __device__ __forceinline__ void stream_gemm_body(
     i32x4_t b_rsrc[NBD];
     int a_voff[Cfg::A_LOADS];
     int b_voff[B_LOADS];
+    int x_voff;     // the chunk of the rows past BM
+    bool x;         // the tile has such rows: a stage has one load more
     int k, n, nk1;  // of the tile's product (constants of the launch unless kJoint)
   };
   // the tile's product, seen from the tile
   auto second_product = [](const Tile& t) { return kJoint && t.expert < 0; };
   auto tile_k = [&](const Tile& t) { return second_product(t) ? dp.k : Kdim; };
   auto tile_n = [&](const Tile& t) { return second_product(t) ? dp.n : N; };
-  const int a_r = tid / CPRA, a_slot = tid - a_r * CPRA;
-  const int a_c = a_slot ^ ((a_r / (16 / CPRA)) % CPRA);
-  const int b_blk_id = tid >> 5;
-  const int b_k = (b_blk_id >> 1) * 4 + ((tid >> 3) & 3);
-  const int b_c = (b_blk_id & 1) * 8 + ((tid & 7) ^ (((tid >> 4) & 1) << 2));
+  // thread t fetches 16-byte chunk chunk_of(t) of row t / CPRA of the A tile (and of the rows NT / CPRA further on)
+  auto chunk_of = [](int t) { return (t % CPRA) ^ ((t / CPRA / (16 / CPRA)) % CPRA); };
+  const int a_c = chunk_of(tid);
   const unsigned lds0 = lds_byte_addr(smem_raw);
   const unsigned wave_lds = lds0 + wave * 1024;
+  // The X rows have no more chunks than a load of the whole workgroup fetches: with fewer, several waves fetch the same.
+  constexpr int kXWaves = X ? X * CPRA / 64 : 1;
+  const unsigned wave_lds_x = lds0 + BM * BK * 2 + (wave % kXWaves) * 1024;
+  // the rows of the tile that thread t fetches chunks of: with its A loads, and past BM
+  auto load_row = [](int t, int j) { return t / CPRA + j * (NT / CPRA); };
+  auto x_row = [](int t) { return BM + t / CPRA % (X ? X : 1); };
   int* const rowbuf = reinterpret_cast<int*>(smem_raw + L::kRowBufBase);
 
   // everything of a plan but the A row offsets
   auto plan_tile = [&](Plan& p, const Tile& t) {
+    const int tid_f = wave * 64 + fresh_lane(), chunk = chunk_of(tid_f);
     const bool second = second_product(t), gathered = gather && !second;
     p.k = tile_k(t);
     p.n = tile_n(t);
@@ -231,16 +275,21 @@ __device__ __forceinline__ void stream_gemm_body(
       }
       // the B tile's rows are output columns: row n0 + r of B[e], the same slots and swizzle as the A tile
 #pragma unroll
-      for (int j = 0; j < B_LOADS; ++j) p.b_voff[j] = ((t.n0 + a_r + j * (NT / CPRA)) * p.k + a_c * 8) * 2;
+      for (int j = 0; j < B_LOADS; ++j) p.b_voff[j] = ((t.n0 + tid_f / CPRA + j * (NT / CPRA)) * p.k + chunk * 8) * 2;
     } else {
 #pragma unroll
       for (int u = 0; u < Cfg::NSUB; ++u) p.b_rsrc[u] = make_rsrc((kDual && u == 1 ? b1 : b0) + wofs, p.k * p.n * 2);
       p.a_rsrc[0] = gathered ? make_rsrc(a0, a_rows * Kdim * 2) : make_rsrc(a0 + (size_t)t.row0 * p.k, t.rows * p.k * 2);
+      // (B in 4 x 64 blocks: row and chunk of this thread)
+      const int b_blk_id = tid_f >> 5, b_k = (b_blk_id >> 1) * 4 + ((tid_f >> 3) & 3);
+      const int b_c = (b_blk_id & 1) * 8 + ((tid_f & 7) ^ (((tid_f >> 4) & 1) << 2));
 #pragma unroll
       for (int u = 0; u < Cfg::NSUB; ++u) p.b_voff[u] = (b_k * p.n + t.n0 + (kDual ? 0 : u * 128) + b_c * 8) * 2;
     }
 #pragma unroll
-    for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = ((a_r + j * (NT / CPRA)) * p.k + a_c * 8) * 2;
+    for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = (load_row(tid_f, j) * p.k + chunk * 8) * 2;
+    p.x = X != 0 && t.rows > BM;
+    p.x_voff = (x_row(tid_f) * p.k + chunk * 8) * 2;
   };
   // gathered rows: the offsets come from row ids (rows past the end of the group read as zeros)
   // row_map entries are divided by row_div (the top-k of the routing) with a multiply: for
@@ -248,12 +297,22 @@ __device__ __forceinline__ void stream_gemm_body(
   // below 2^60, and n * (d * ceil(2^32 / d) - 2^32) < 2^27 * 32 = 2^32)
   const unsigned long long div_magic = ((1ull << 32) + (unsigned)row_div - 1) / (unsigned)row_div;
   auto plan_rows = [&](Plan& p, const Tile& t, auto row_id) {
-#pragma unroll
-    for (int j = 0; j < Cfg::A_LOADS; ++j) {
-      const int r = a_r + j * (NT / CPRA);
+    const int tid_f = wave * 64 + fresh_lane(), chunk = chunk_of(tid_f);
+    auto offset_of = [&](int r) {
       const int src = (int)(((unsigned long long)(unsigned)row_id(r) * div_magic) >> 32);
-      p.a_voff[j] = r < t.rows ? (src * Kdim + a_c * 8) * 2 : 0x70000000;
-    }
+      return r < t.rows ? (src * Kdim + chunk * 8) * 2 : 0x70000000;
+    };
+#pragma unroll
+    for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = offset_of(load_row(tid_f, j));
+    if (p.x) p.x_voff = offset_of(x_row(tid_f));
+  };
+  // behind the last tile: loads that store zeros, so that every step has as many
+  auto plan_nothing = [](Plan& p) {
+#pragma unroll
+    for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = kOutside;
+#pragma unroll
+    for (int j = 0; j < B_LOADS; ++j) p.b_voff[j] = kOutside;
+    p.x = false;
   };
   // load i of the LPS loads of a stage (A loads first, then B) of k step kt of the planned tile
   auto issue_one = [&](const Plan& p, int kt, int stage, int i) {
@@ -280,13 +339,22 @@ __device__ __forceinline__ void stream_gemm_body(
       }
     }
   };
+  // ... and the one of the X rows, if the tile has any
+  auto issue_x = [&](const Plan& p, int kt, int stage) {
+    if (X == 0 || !p.x) return;
+    const bool second = kNT && kt >= p.nk1;
+    const int k0 = (second ? kt - p.nk1 : kt) * BK;
+    buffer_load_lds16(second ? p.a_rsrc[NSEG - 1] : p.a_rsrc[0], wave_lds_x + stage * Cfg::STAGE_BYTES,
+                      kTail && k0 + a_c * 8 >= p.k ? kOutside : p.x_voff, k0 * 2);
+  };
   auto issue = [&](const Plan& p, int kt, int stage) {
 #pragma unroll
     for (int i = 0; i < LPS; ++i) issue_one(p, kt, stage, i);
+    issue_x(p, kt, stage);
   };
 
   // ---- fragment addresses of this lane (bytes inside a stage) ----
-  const int a_row = wm * WM + (lane & 31);
+  const int a_row = wm * 32 + (lane & 31);
   const int a_sw = (a_row / (16 / CPRA)) % CPRA;
   const int a_rowoff = a_row * (BK * 2);
   const int b_laneoff = ((lane & 15) >> 2) * 128 + (lane & 3) * 8 + ((lane >> 4) & 1) * 32 + (lane >> 5) * 2048;
@@ -309,7 +377,7 @@ __device__ __forceinline__ void stream_gemm_body(
   }
   auto load_frag_a = [&](int stage, int kk, int mi) -> bf16x8_t {
     const unsigned char* st = smem_raw + stage * Cfg::STAGE_BYTES;
-    return *reinterpret_cast<const bf16x8_t*>(st + a_rowoff + mi * 32 * BK * 2 + (((kk * 2 + (lane >> 5)) ^ a_sw) << 4));
+    return *reinterpret_cast<const bf16x8_t*>(st + a_rowoff + mi * kRowStep * BK * 2 + (((kk * 2 + (lane >> 5)) ^ a_sw) << 4));
   };
   auto load_frag_b = [&](int stage, int kk, int jj) -> bf16x8_t {
     if constexpr (kNT) {
@@ -323,9 +391,11 @@ __device__ __forceinline__ void stream_gemm_body(
     const s16x8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(bf16x8_t, both);
   };
+  bf16x8_t ax[2];  // of the X rows' block
   auto load_frags = [&](int stage, int kk, bf16x8_t* af, bf16x8_t* bf) {
 #pragma unroll
     for (int mi = 0; mi < TM; ++mi) af[mi] = load_frag_a(stage, kk, mi);
+    if (X != 0) ax[0] = load_frag_a(stage, kk, TM);
 #pragma unroll
     for (int jj = 0; jj < TN; ++jj) bf[jj] = load_frag_b(stage, kk, jj);
   };
@@ -340,7 +410,6 @@ __device__ __forceinline__ void stream_gemm_body(
   int nk = pl.nk1 * nk_segs;  // k steps of the current tile
 #pragma unroll
   for (int s = 0; s < NS; ++s) issue(pl, s, s);
-  f32x16_t acc[TM][TN];
   bf16x8_t af[2][TM], bf[2][TN];
   wait_and_barrier<(NS - 1) * LPS>();
   load_frags(0, 0, af[0], bf[0]);
@@ -349,7 +418,8 @@ __device__ __forceinline__ void stream_gemm_body(
 
   while (true) {
     const int cur_n = tile_n(cur);
-    const bool wave_has_rows = wm * WM < cur.rows && cur.n0 + wn * Cfg::WNO < cur_n;
+    // row blocks of this wave that hold rows of the tile (none either if its columns lie past N)
+    const int blocks = cur.n0 + wn * Cfg::WNO < cur_n ? max(0, (cur.rows - wm * 32 + kRowStep - 1) / kRowStep) : 0;
     if constexpr (!kJoint) idx += stride;
     --left;
     const Tile nxt = locate(left > 0 ? idx : 0x3fffffff);
@@ -361,136 +431,128 @@ __device__ __forceinline__ void stream_gemm_body(
     // cover it)
     if (gather && have_next && !second_product(nxt)) {
       const i32x4_t map_rsrc = make_rsrc(row_map + nxt.row0, nxt.rows * 4);
-      buffer_load_lds4(map_rsrc, lds0 + L::kRowBufBase + wave * 256, lane * 4 + wave * 256);
+      buffer_load_lds4(map_rsrc, lds0 + L::kRowBufBase + wave * 256, (fresh_lane() + wave * 64) * 4);
     }
 
-    // MFMAs of one 16-deep sub-step on fragment set `cur_set`, interleaved by the scheduler with the
-    // LDS reads (two per MFMA) that were written before them
-    // (`first`: the tile's first sub-step, which accumulates onto zero instead of clearing 128 registers)
-    auto mfma_substep = [&](int cur_set, bool first = false) {
-      if (Cfg::OPT & 32) __builtin_amdgcn_s_setprio(1);
-      f32x16_t zero;
+    // The tile, written out for the number NB of the wave's row blocks that take part: a tile that is not full costs the
+    // matrix cores what its rows need, to two blocks of a wave.  (Accumulators that lived on from one of these forms to
+    // the next would not stay in the same registers, and hundreds would be spilled: each has its own, from the zeros to
+    // the epilogue.)
+    const bool x_rows = pl.x, second = second_product(cur);
+    auto run_tile = [&](auto nb) {
+      constexpr int NB = decltype(nb)::value, kMfmas = NB * TN;
+      f32x16_t acc[NB > 0 ? NB : 1][TN];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) zero[i] = 0.0f;
-#pragma unroll
-      for (int mi = 0; mi < TM; ++mi)
-#pragma unroll
-        for (int jj = 0; jj < TN; ++jj)
-          acc[mi][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[cur_set][jj], af[cur_set][mi],
-                                                                first ? zero : acc[mi][jj], 0, 0, 0);
-#pragma unroll
-      for (int g = 0; g < TM * TN; ++g) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-      }
-      if (Cfg::OPT & 32) __builtin_amdgcn_s_setprio(0);
-    };
-    // sub-steps 0 .. KK-2 of a step: fragments of the following sub-step are requested, then this one's MFMAs
-    auto leading_substeps = [&](auto first_tag) {
-#pragma unroll
-      for (int kk = 0; kk < KK - 1; ++kk) {
-        if (!kNoFragReads) load_frags(cs, kk + 1, af[(kk + 1) & 1], bf[(kk + 1) & 1]);
-        mfma_substep(kk & 1, decltype(first_tag)::value && kk == 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    };
-
-    // ---- steady part: every step has NS successors inside this tile ----
-    int j = 0;
-    if (wave_has_rows) {
-      auto steady_step = [&](auto first_tag) {
-        leading_substeps(first_tag);
-        // the next step's stage has arrived (own loads: the wait; everyone's: the barrier), and every
-        // wave holds its last fragments of the current stage, which is therefore free
-        wait_and_barrier<(NS - 2) * LPS>();
-        __builtin_amdgcn_sched_barrier(0);
-        // last sub-step, in a fixed order: after each of its MFMAs one operand load of step j + NS
-        // (into the stage just released) and one fragment read of step j + 1 are issued
-        const int ns = (cs + 1) & (NS - 1);
-        constexpr int cur_set = (KK - 1) & 1;
-        if (Cfg::OPT & 32) __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int g = 0; g < TM * TN; ++g) {
-          acc[g / TN][g % TN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[cur_set][g % TN], af[cur_set][g / TN],
-                                                                        acc[g / TN][g % TN], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          constexpr int kLoadsPer = (LPS + TM * TN - 1) / (TM * TN);
-#pragma unroll
-          for (int q = 0; q < kLoadsPer; ++q)
-            if (!kNoLoads && g * kLoadsPer + q < LPS) issue_one(pl, kSameTile ? 0 : j + NS, cs, g * kLoadsPer + q);
-          if (kNoFragReads) {
-          } else if (g < TM)
-            af[0][g] = load_frag_a(ns, 0, g);
-          else if (g < TM + TN)
-            bf[0][g - TM] = load_frag_b(ns, 0, g - TM);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (Cfg::OPT & 32) __builtin_amdgcn_s_setprio(0);
-        cs = ns;
-      };
-      steady_step(std::true_type{});  // nk >= 2 NS: the steady part has at least NS steps
-      for (j = 1; j < nk - NS; ++j) steady_step(std::false_type{});
-    } else {
-      // a tile at the end of a group: this wave's rows lie past it; it only keeps the loads going
-#pragma unroll
-      for (int mi = 0; mi < TM; ++mi)
+      for (int mi = 0; mi < NB; ++mi)
 #pragma unroll
         for (int jj = 0; jj < TN; ++jj)
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc[mi][jj][i] = 0.0f;
-      for (; j < nk - NS; ++j) {
-        wait_and_barrier<(NS - 2) * LPS>();
-        issue(pl, j + NS, cs);
-        cs = (cs + 1) & (NS - 1);
-      }
-    }
-
-    // ---- last NS steps: requests go to the next tile, if there is one ----
-    for (; j < nk; ++j) {
-      if (wave_has_rows) leading_substeps(std::false_type{});
-      // k steps of this workgroup's stream after this one (only the next tile counts: a load is
-      // never issued more than NS <= nk steps ahead)
-      const int rem = (nk - 1 - j) + (have_next ? nk_next : 0);
-      if (rem > 0) {
-        if (rem >= NS - 1)
-          wait_and_barrier<(NS - 2) * LPS>();
-        else if (NS > 3 && rem == NS - 2)
-          wait_and_barrier<(NS > 3 ? NS - 3 : 0) * LPS>();
+      // MFMA g of a sub-step on fragment set `set`
+      auto mfma = [&](int set, int g) {
+        acc[g / TN][g % TN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[set][g % TN], g / TN < TM ? af[set][g / TN] : ax[set],
+                                                                      acc[g / TN][g % TN], 0, 0, 0);
+      };
+      // fragment f of the NB + TN of a sub-step
+      auto read = [&](int set, int stage, int kk, int f) {
+        if (f < NB)
+          (f < TM ? af[set][f] : ax[set]) = load_frag_a(stage, kk, f);
         else
-          wait_and_barrier<0>();
-        if (rem >= NS) {
-          const int kt = j + NS - nk;  // a step of the next tile
-          if (kt == 0) {               // from here on the plan is the next tile's
+          bf[set][f - NB] = load_frag_b(stage, kk, f - NB);
+      };
+      // all steps but the last NS, then, with the next tile's plan, those: their loads are its first steps'
+#pragma unroll 1
+      for (int part = 0; part < 2; ++part) {
+        const int j0 = part ? nk - NS : 0, j1 = part ? nk : nk - NS, ahead = part ? NS - nk : NS;
+        if (part) {
+          if (have_next) {
             plan_tile(pl, nxt);
             if (gather && !second_product(nxt)) plan_rows(pl, nxt, [&](int r) { return rowbuf[r]; });
+          } else {
+            plan_nothing(pl);
           }
-          issue(pl, kt, cs);
+        }
+        const bool x_loads = x_rows && !part;  // (part 1: of some stages, then of others)
+        for (int j = j0; j < j1; ++j) {
+          // sub-steps 0 .. KK-2: the fragments of the following sub-step are requested, then this one's MFMAs, which the
+          // scheduler interleaves with the LDS reads (two per MFMA)
+#pragma unroll
+          for (int kk = 0; kk < KK - 1; ++kk) {
+            if (NB > 0 && !kNoFragReads)
+#pragma unroll
+              for (int f = 0; f < NB + TN; ++f) read((kk + 1) & 1, cs, kk + 1, f);
+#pragma unroll
+            for (int g = 0; g < kMfmas; ++g) mfma(kk & 1, g);
+#pragma unroll
+            for (int g = 0; g < kMfmas; ++g) {
+              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+              __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          // the next step's stage has arrived (own loads: the wait; everyone's: the barrier), and every
+          // wave holds its last fragments of the current stage, which is therefore free
+          // (a stage is LPS loads, with X rows one more)
+          if (X != 0 && NS > 2 && x_loads)
+            wait_and_barrier<(NS - 2) * (LPS + 1)>();
+          else
+            wait_and_barrier<(NS - 2) * LPS>();
+          __builtin_amdgcn_sched_barrier(0);
+          // last sub-step, in a fixed order: after each of its MFMAs operand loads of step j + ahead (into the stage just
+          // released) and fragment reads of step j + 1 are issued
+          const int ns = (cs + 1) & (NS - 1), kt = kSameTile ? 0 : j + ahead;
+          constexpr int kSlots = kMfmas > 0 ? kMfmas : 1;
+          constexpr int kLoadsPer = (LPS + kSlots - 1) / kSlots, kFragsPer = (NB + TN + kSlots - 1) / kSlots;
+#pragma unroll
+          for (int g = 0; g < kSlots; ++g) {
+            if (NB > 0) mfma((KK - 1) & 1, g);
+            __builtin_amdgcn_sched_barrier(0);
+            if (!kNoLoads) {
+#pragma unroll
+              for (int q = 0; q < kLoadsPer; ++q)
+                if (g * kLoadsPer + q < LPS) issue_one(pl, kt, cs, g * kLoadsPer + q);
+            }
+            if (NB > 0 && !kNoFragReads)
+#pragma unroll
+              for (int q = 0; q < kFragsPer; ++q)
+                if (g * kFragsPer + q < NB + TN) read(0, ns, 0, g * kFragsPer + q);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (!kNoLoads) issue_x(pl, kt, cs);
+          cs = ns;
         }
       }
-      __builtin_amdgcn_sched_barrier(0);
-      cs = (cs + 1) & (NS - 1);
-      if (rem > 0) load_frags(cs, 0, af[0], bf[0]);
-      if (wave_has_rows) mfma_substep((KK - 1) & 1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-
-    // ---- epilogue: straight from the accumulators to memory (no LDS, no barrier) ----
-    const bool second = second_product(cur);
-    store_transposed_accumulators<Cfg>(acc, wm, wn, cur.row0, cur.rows, cur.n0, cur_n, second ? dp.rows : dense_rows,
-                                       second ? dp.c : C, second ? dp.save0 : save0, second ? dp.save1 : save1);
+      // epilogue: straight from the accumulators to memory (no LDS, no barrier)
+      if constexpr (NB > 0)
+        store_transposed_accumulators<Cfg, NB>(acc, wm * 32, kRowStep, wn, cur.row0, cur.rows, cur.n0, cur_n,
+                                               second ? dp.rows : dense_rows, second ? dp.c : C,
+                                               second ? dp.save0 : save0, second ? dp.save1 : save1);
+    };
+    if (X != 0 && blocks > TM)
+      run_tile(std::integral_constant<int, TMX>{});
+    else if (TM > 2 && blocks > 2)
+      run_tile(std::integral_constant<int, TM>{});
+    else if (blocks > 0)
+      run_tile(std::integral_constant<int, 2>{});
+    else
+      run_tile(std::integral_constant<int, 0>{});
+    static_assert(TM == 2 || TM == 4, "row blocks per wave");
     if (!have_next) break;
+    // (only now: no fragment stays in registers through the epilogue)
+    load_frags(cs, 0, af[0], bf[0]);
     cur = nxt;
     nk = nk_next;
   }
+  wait_vmcnt<0>();  // (the loads of plan_nothing still write to LDS)
 }
 
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
     uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E,
-    int dense_rows, int Kdim, int N, int mtiles, int ntiles_n, const int32_t* __restrict__ row_map, int row_div,
+    int dense_rows, int Kdim, int N, int ntiles_n, const int32_t* __restrict__ row_map, int row_div,
     int a_rows, uint16_t* __restrict__ save0, uint16_t* __restrict__ save1, int window, int chunk) {
-  stream_gemm_body<Cfg, false>(A, nullptr, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, mtiles, ntiles_n,
+  stream_gemm_body<Cfg, false>(A, nullptr, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, ntiles_n,
                                row_map, row_div, a_rows, save0, save1, 1, window, chunk, DenseProblem{});
 }
 
@@ -500,9 +562,9 @@ template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_joint_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
     uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E,
-    int dense_rows, int Kdim, int N, int mtiles, int ntiles_n, const int32_t* __restrict__ row_map, int row_div,
+    int dense_rows, int Kdim, int N, int ntiles_n, const int32_t* __restrict__ row_map, int row_div,
     int a_rows, uint16_t* __restrict__ save0, uint16_t* __restrict__ save1, DenseProblem dp) {
-  stream_gemm_body<Cfg, false, true>(A, nullptr, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, mtiles,
+  stream_gemm_body<Cfg, false, true>(A, nullptr, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N,
                                      ntiles_n, row_map, row_div, a_rows, save0, save1, 1, 0, 0, dp);
 }
 
@@ -512,9 +574,9 @@ template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_nt_kernel(
     const uint16_t* __restrict__ A0, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes,
-    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n,
+    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int ntiles_n,
     const int32_t* __restrict__ row_map, int row_div, int a_rows, int segs, int window, int chunk) {
-  stream_gemm_body<Cfg, true>(A0, A1, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, mtiles, ntiles_n,
+  stream_gemm_body<Cfg, true>(A0, A1, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, ntiles_n,
                               row_map, row_div, a_rows, nullptr, nullptr, segs, window, chunk, DenseProblem{});
 }
 
@@ -522,18 +584,30 @@ template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_joint_nt_kernel(
     const uint16_t* __restrict__ A0, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes,
-    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n, int segs,
+    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int ntiles_n, int segs,
     DenseProblem dp) {
-  stream_gemm_body<Cfg, true, true>(A0, A1, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, mtiles, ntiles_n,
+  stream_gemm_body<Cfg, true, true>(A0, A1, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, ntiles_n,
                                     nullptr, 1, 0, nullptr, nullptr, segs, 0, 0, dp);
 }
 
-// The configuration the library launches for gate/up (routed and shared experts): the tile of GateUpCfg
-// with 32-deep steps and four stages.  Measured on 64 groups of 2048 gathered rows x 2048 x 1408
-// (alternating in one process): 1.306 ms against 1.400-1.409 ms for grouped_gemm_dma_persistent_kernel
-// and 1.315-1.320 ms for 64-deep steps with two stages.
-using GateUpStreamCfg = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128>;
-using GateUpStreamTailCfg = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 65536>;  // for K % 64 != 0
+// The 256-row tiles of the library, of up to 320 rows: gate/up, down and data gradients, each also for a reduction that is
+// no multiple of 64.  64-deep steps in two stages; with 32-deep ones in four, us (64-deep / 32-deep): 131072 rows in 64
+// groups, 2048 x 1408: gate/up 1313 / 1332, down 730 / 741, dZ 743 / 774, dX 1347 / 1406; 8192 rows in 8 groups, 1024 x
+// 2048: gate/up 71.6 / 72.9.  Eight waves of 128 x 64: with 64 x 128 there is no room for a block more per wave.
+//
+// Against 256 rows and a tile of its own for what is left of each group (uneven groups by random routing; us, before /
+// now; both products of a layer call alone, matrices not in the caches):
+//   16384 rows in 64 groups, 2048 x 1408    gate/up 271 / 213, down 134 / 117, dZ 161 / 149, dX 253 / 220
+//   16384 rows in 16 groups, 1024 x 2816    gate/up 195 / 196, down 131 (half tiles 110) / 87, dZ 116 / 107, dX 250 / 175
+//   8192 rows in 8 groups, 1024 x 2048      gate/up 80 / 72, dZ 54 / 40
+//   131072 rows in 64 groups, 2048 x 1408   gate/up 1343 / 1313, down 757 / 730, dZ 748 / 743, dX 1392 / 1347
+// (Bound by the matrix cores at the power limit at 131072 rows, by rounds over the CUs at the others.)
+using GateUpStreamCfg = DmaGemmCfg<256, 128, 64, 2, 4, true, 2, 16 + 128 + 131072>;
+using GateUpStreamTailCfg = DmaGemmCfg<256, 128, 64, 2, 4, true, 2, 16 + 128 + 65536 + 131072>;
+using DownStreamCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 32768 + 131072>;
+using DownStreamTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 32768 + 65536 + 131072>;
+using DgradStreamCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 131072>;
+using DgradStreamTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 65536 + 131072>;
 // Half-size tiles in four-wave workgroups for launches that would leave CUs without a 256-row tile: gate/up with
 // one workgroup per CU (99 KB of LDS), down with two.  The dispatch rules and what they measured stand in
 // grouped_gemm.hip.  (The check for a ragged last step costs nothing: 33.3 against 33.7 us without it for gate/up,
@@ -542,21 +616,7 @@ using GateUpHalfCfg = DmaGemmCfg<128, 128, 32, 2, 2, true, 4, 16 + 128>;
 using GateUpHalfTailCfg = DmaGemmCfg<128, 128, 32, 2, 2, true, 4, 16 + 128 + 65536>;  // for K % 64 != 0
 using DownHalfCfg = DmaGemmCfg<128, 128, 32, 2, 2, false, 4, 16 + 128 + 65536>;
 using DownHalfDeepCfg = DmaGemmCfg<128, 128, 64, 2, 2, false, 2, 16 + 128 + 65536>;
-// Variants kept for the stand-alone check and its timings (time_stream, time_down): 64-deep steps with
-// two stages, and the down projection's tile (within 2 % of grouped_gemm_dma_persistent_kernel, which
-// the library keeps for that launch, at 12, 22 and 44 k steps per tile).
-using GateUpStream2Cfg = DmaGemmCfg<256, 128, 64, 4, 2, true, 2, 16 + 128>;
-using DownStreamCfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768>;
-using DownStreamTailCfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + 65536>;
-using DownStream2Cfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 32768>;
-// The data-gradient products of the backward pass (transposed-B form): 256 x 256 tiles, 2 x 4 waves.
-// Checked and timed by the stand-alone check (time_stream_nt) against grouped_gemm_nt_kernel, which
-// the library launches: the transposed-B form measures equal or slower there.
-using DgradStreamCfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128>;
-// The 256-row tiles of the joint launch of routed and shared data gradients.
-using DgradJointCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128>;
-using DgradJointTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 65536>;
-// The same in half tiles, launched where a data gradient has at most one of them per CU: nothing else runs on the CU,
+// Data gradients in half tiles, launched where one has at most one of them per CU: nothing else runs on the CU,
 // so four 64-deep stages (131 KB) keep its loads going.  4096 rows x 4096 -> 1024: 40 us, two 64-deep stages with
 // two workgroups per CU 59, four 32-deep ones 49, 256 x 256 tiles 93; 2048 rows x 5632 -> 2048: 55, 79, 67 and 124.
 using DgradHalfDeepCfg = DmaGemmCfg<128, 128, 64, 2, 2, false, 4, 16 + 128 + 65536>;

@@ -86,6 +86,7 @@ struct Problem {
 
 // rows are spread over E groups (skewed, some empty); with top_k > 0 the A matrix has
 // rows/top_k rows and packed row j reads A row row_map[j] / top_k (gather on load)
+static std::vector<int> g_sizes;  // these group sizes instead of random ones
 static bool g_equal_groups = false;  // every group rows / E rows (no ragged last tiles) instead of random sizes
 static Problem make(int E, int rows, int K, int N, unsigned seed, bool skew, int top_k, float scale) {
   Problem p;
@@ -98,6 +99,7 @@ static Problem make(int E, int rows, int K, int N, unsigned seed, bool skew, int
     if (g_equal_groups) e = r % E;
     p.gs[e]++;
   }
+  if (!g_sizes.empty()) p.gs = g_sizes;
   p.off.assign(E, 0);
   for (int e = 1; e < E; ++e) p.off[e] = p.off[e - 1] + p.gs[e - 1];
   p.row_expert.resize(rows);
@@ -139,12 +141,17 @@ static void release(Problem& p) {
 // here), unless g_one_tile_per_workgroup asks for the plain kernel.
 static bool g_one_tile_per_workgroup = false;
 static int g_chunk = -1;  // tiles per workgroup of a persistent launch; -1: as the library chooses
+// the stream kernel's 256-row tiles with 32-deep steps in four stages (the library: 64-deep ones in two)
+using GateUpStream32Cfg = DmaGemmCfg<256, 128, 32, 2, 4, true, 4, 16 + 128 + 131072>;
+using DownStream32Cfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + 131072>;
+static int g_workgroups = 0;  // launch the stream kernel with so many persistent workgroups
+
 // the stream kernel (grouped_gemm_stream.hpp): one software pipeline through all tiles of a workgroup
 template <typename Cfg>
 static void launch_stream(Problem& p, bool dense) {
   using L = StreamLayout<Cfg>;
   if (p.K / Cfg::BK < 2 * Cfg::NSTAGE) { printf("stream kernel: K too short\n"); exit(1); }
-  const long mt = dense ? (p.rows + Cfg::BM - 1) / Cfg::BM
+  const long mt = dense ? group_mtiles(p.rows, Cfg::BM, Cfg::XROWS)
                         : (p.rows + Cfg::BM - 1) / Cfg::BM + (p.E < p.rows ? p.E : p.rows);
   const long nt = (p.N + Cfg::BN - 1) / Cfg::BN;
   const long tiles_grid = gemm_grid(mt, nt);
@@ -153,9 +160,10 @@ static void launch_stream(Problem& p, bool dense) {
                          (int)L::kSmemBytes));
   PersistentSchedule ps = persistent_schedule(tiles_grid, 256, g_chunk < 0 ? kTilesPerWorkgroup<Cfg> : g_chunk);
   if (tiles_grid <= 256) ps = {tiles_grid, 0, 0};
+  if (g_workgroups) ps = {g_workgroups, 0, 0};
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes>>>(
       p.A, p.B0, Cfg::kDual ? p.B1 : nullptr, p.C, dense ? nullptr : p.dgs, dense ? nullptr : p.doff, p.E, p.rows, p.K,
-      p.N, (int)mt, (int)nt, p.top_k > 0 ? p.dmap : nullptr, p.top_k > 0 ? p.top_k : 1, p.a_rows, nullptr, nullptr,
+      p.N, (int)nt, p.top_k > 0 ? p.dmap : nullptr, p.top_k > 0 ? p.top_k : 1, p.a_rows, nullptr, nullptr,
       ps.window, ps.chunk);
 }
 
@@ -332,9 +340,8 @@ static bool compare(const char* name, const float* dref, const uint16_t* dgot, s
 }
 
 // the transposed-B form of the stream kernel (what the library launches for the data gradients where it fits)
-static int g_stream_nt = 0;  // 0: the older kernel; 1: DgradStreamCfg; 2 and 3: its variants below
-using DgradStream42Cfg = DmaGemmCfg<256, 256, 32, 4, 2, false, 4, 16 + 128>;  // 4 x 2 waves of 64 x 128
-using DgradStream2Cfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128>;   // 64-deep steps, two stages
+static int g_stream_nt = 0;  // 0: the older kernel; 1: DgradStreamCfg; 2: 32-deep steps in four stages
+using DgradStream32Cfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 131072>;
 template <typename Cfg>
 static void launch_stream_nt_cfg(Problem& p, const uint16_t* A1, int segs, bool dense) {
   using L = StreamLayout<Cfg>;
@@ -345,19 +352,19 @@ static void launch_stream_nt_cfg(Problem& p, const uint16_t* A1, int segs, bool 
   auto kernel = grouped_gemm_stream_nt_kernel<Cfg>;
   CK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                          (int)L::kSmemBytes));
-  const long mt = dense ? (p.rows + Cfg::BM - 1) / Cfg::BM
+  const long mt = dense ? group_mtiles(p.rows, Cfg::BM, Cfg::XROWS)
                         : (p.rows + Cfg::BM - 1) / Cfg::BM + (p.E < p.rows ? p.E : p.rows);
   const long nt = (p.N + Cfg::BN - 1) / Cfg::BN;
   const long tiles_grid = gemm_grid(mt, nt);
   PersistentSchedule ps = persistent_schedule(tiles_grid, 256, g_chunk < 0 ? kTilesPerWorkgroup<Cfg> : g_chunk);
   if (tiles_grid <= 256) ps = {tiles_grid, 0, 0};
+  if (g_workgroups) ps = {g_workgroups, 0, 0};
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes>>>(
-      p.A, A1, p.B0, p.B1, p.C, dense ? nullptr : p.dgs, dense ? nullptr : p.doff, p.E, p.rows, p.K, p.N, (int)mt,
-      (int)nt, p.top_k > 0 ? p.dmap : nullptr, p.top_k > 0 ? p.top_k : 1, p.a_rows, segs, ps.window, ps.chunk);
+      p.A, A1, p.B0, p.B1, p.C, dense ? nullptr : p.dgs, dense ? nullptr : p.doff, p.E, p.rows, p.K, p.N, (int)nt,
+      p.top_k > 0 ? p.dmap : nullptr, p.top_k > 0 ? p.top_k : 1, p.a_rows, segs, ps.window, ps.chunk);
 }
 static void launch_stream_nt(Problem& p, const uint16_t* A1, int segs, bool dense) {
-  if (g_stream_nt == 2) return launch_stream_nt_cfg<DgradStream42Cfg>(p, A1, segs, dense);
-  if (g_stream_nt == 3) return launch_stream_nt_cfg<DgradStream2Cfg>(p, A1, segs, dense);
+  if (g_stream_nt == 2) return launch_stream_nt_cfg<DgradStream32Cfg>(p, A1, segs, dense);
   launch_stream_nt_cfg<DgradStreamCfg>(p, A1, segs, dense);
 }
 
@@ -602,7 +609,7 @@ static void time_decode() {
 }
 
 // "deal": host arithmetic only.  The workgroups of an XCD take every tile of the two products of a joint launch exactly
-// once, each workgroup the dense ones first, in rising order, and have no tile after their last.
+// once, each workgroup the dense ones first, in rising order, and have no tile after their last; and the m-tiles of a group.
 bool check_deal() {
   srand(1);
   const int cases = 20000;
@@ -630,6 +637,24 @@ bool check_deal() {
         return false;
       }
   }
+  // the m-tiles of a group hold every row once, no more than BM + extra each
+  for (int extra : {0, 64})
+    for (int BM : {128, 256})
+      for (int n = 0; n <= 3000; ++n) {
+        int row = 0;
+        for (int i = 0, tiles = group_mtiles(n, BM, extra); i < tiles; ++i) {
+          const TileSpan t = group_mtile(n, i, BM, extra);
+          if (t.first != row || t.rows <= 0 || t.rows > BM + extra || tiles > (n + BM - 1) / BM) {
+            printf("deal: BM=%d extra=%d: tile %d of %d rows: [%d, %d)\n", BM, extra, i, n, t.first, t.first + t.rows);
+            return false;
+          }
+          row += t.rows;
+        }
+        if (row != n) {
+          printf("deal: BM=%d extra=%d: %d of %d rows\n", BM, extra, row, n);
+          return false;
+        }
+      }
   printf("deal: %d cases\nPASS\n", cases);
   return true;
 }
@@ -756,12 +781,12 @@ int main(int argc, char** argv) {
     Problem p = make(7, 3001, 576, 392, 51, true, 0, 1.0f);
     ok &= check<GateUpStreamCfg>("stream gate/up ragged", p);
     ok &= check<DownStreamCfg>("stream down ragged", p);
-    ok &= check<GateUpStream2Cfg>("stream 2 x 64 gate/up ragged", p);
-    ok &= check<DownStream2Cfg>("stream 2 x 64 down ragged", p);
+    ok &= check<GateUpStream32Cfg>("stream 4 x 32 gate/up ragged", p);
+    ok &= check<DownStream32Cfg>("stream 4 x 32 down ragged", p);
     release(p);
     Problem q = make(5, 2400, 512, 384, 52, true, 3, 1.0f);
     ok &= check<GateUpStreamCfg>("stream gate/up gather on load", q);
-    ok &= check<GateUpStream2Cfg>("stream 2 x 64 gate/up gather on load", q);
+    ok &= check<GateUpStream32Cfg>("stream 4 x 32 gate/up gather on load", q);
     release(q);
     Problem r = make(1, 777, 512, 520, 53, false, 0, 1.0f);
     ok &= check<GateUpStreamCfg>("stream gate/up dense", r, true);
@@ -770,18 +795,46 @@ int main(int argc, char** argv) {
     Problem u = make(40, 70000, 256, 264, 54, true, 0, 1.0f);  // many more tiles than workgroups
     ok &= check<GateUpStreamCfg>("stream gate/up many tiles per workgroup", u);
     ok &= check<DownStreamCfg>("stream down many tiles per workgroup", u);
-    ok &= check<DownStream2Cfg>("stream 2 x 64 down many tiles per workgroup", u);
+    ok &= check<DownStream32Cfg>("stream 4 x 32 down many tiles per workgroup", u);
     release(u);
     Problem v = make(33, 90000, 256, 392, 55, true, 4, 1.0f);  // the same with gathered rows (row map by LDS-DMA)
     ok &= check<GateUpStreamCfg>("stream gate/up many tiles, gather", v);
-    ok &= check<GateUpStream2Cfg>("stream 2 x 64 gate/up many tiles, gather", v);
+    ok &= check<GateUpStream32Cfg>("stream 4 x 32 gate/up many tiles, gather", v);
     g_chunk = 0;
     ok &= check<GateUpStreamCfg>("stream gate/up many tiles, gather, one workgroup per CU", v);
     g_chunk = -1;
     release(v);
+    // groups either side of what tiles take beyond 256 rows (in few workgroups: with one per tile they take no more)
+    g_workgroups = 16;
+    g_sizes = {1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 192, 255, 256, 257, 287, 288, 289, 319, 320, 321, 0, 383, 384, 511, 512, 575, 576, 577, 832, 833};
+    int edge_rows = 0;
+    for (int n : g_sizes) edge_rows += n;
+    Problem x = make((int)g_sizes.size(), edge_rows, 512, 264, 56, false, 0, 1.0f);
+    ok &= check<GateUpStreamCfg>("stream gate/up, edges of tiles", x);
+    ok &= check<DownStreamCfg>("stream down, edges of tiles", x);
+    ok &= check<DownStream32Cfg>("stream 4 x 32 down, edges of tiles", x);
+    g_stream_nt = 1;
+    ok &= check_nt<DgradCfg>("stream dgrad, edges of tiles", x, 2);
+    g_stream_nt = 4;
+    ok &= check_nt<DgradCfg>("stream dgrad 4 x 32, edges of tiles", x, 2);
+    g_stream_nt = 0;
+    release(x);
+    Problem y = make((int)g_sizes.size(), edge_rows, 256, 392, 57, false, 2, 1.0f);
+    ok &= check<GateUpStreamCfg>("stream gate/up gather, edges of tiles", y);
+    release(y);
+    g_workgroups = 8;
+    for (int n : {900, 1024, 1200, 1279, 1281, 2800}) {
+      g_sizes = {n};
+      Problem z = make(1, n, 256, 264, 58, false, 0, 1.0f);
+      ok &= check<GateUpStreamCfg>("stream gate/up dense, edges of tiles", z, true);
+      ok &= check<DownStreamCfg>("stream down dense, edges of tiles", z, true);
+      release(z);
+    }
+    g_sizes.clear();
+    g_workgroups = 0;
     g_stream = false;
     // the transposed-B form of the stream kernel
-    for (g_stream_nt = 1; g_stream_nt <= 3; ++g_stream_nt) {
+    for (g_stream_nt = 1; g_stream_nt <= 2; ++g_stream_nt) {
     Problem w1 = make(7, 3001, 576, 392, 61, true, 0, 1.0f);  // ragged groups, N not a multiple of the tile
     ok &= check_nt<DgradCfg>("stream dgrad ragged", w1, 1);
     ok &= check_nt<DgradCfg>("stream dgrad ragged, two segments", w1, 2);
@@ -811,13 +864,13 @@ int main(int argc, char** argv) {
       timeit<GateUpCfg>("gate/up library", g, 20);
       timeit<DownCfg>("down library", d, 20);
       g_stream = true;
-      timeit<GateUpStreamCfg>("gate/up stream 4 x 32 (library)", g, 20);
-      timeit<DownStreamCfg>("down stream 4 x 32", d, 20);
-      timeit<GateUpStream2Cfg>("gate/up stream 2 x 64", g, 20);
-      timeit<DownStream2Cfg>("down stream 2 x 64", d, 20);
+      timeit<GateUpStreamCfg>("gate/up stream 2 x 64 (library)", g, 20);
+      timeit<DownStreamCfg>("down stream 2 x 64", d, 20);
+      timeit<GateUpStream32Cfg>("gate/up stream 4 x 32", g, 20);
+      timeit<DownStream32Cfg>("down stream 4 x 32", d, 20);
       g_chunk = 0;
-      timeit<GateUpStreamCfg>("gate/up stream 4 x 32, one wg per CU", g, 20);
-      timeit<DownStreamCfg>("down stream 4 x 32, 4 tiles per wg", d, 20);
+      timeit<GateUpStreamCfg>("gate/up stream 2 x 64, one wg per CU", g, 20);
+      timeit<DownStreamCfg>("down stream 2 x 64, 4 tiles per wg", d, 20);
       g_chunk = -1;
       g_stream = false;
     }
@@ -828,8 +881,8 @@ int main(int argc, char** argv) {
       g_stream = false;
       timeit<DownCfg>("8192^3 library", sq, 10);
       g_stream = true;
-      timeit<DownStreamCfg>("8192^3 stream 4 x 32", sq, 10);
-      timeit<DownStream2Cfg>("8192^3 stream 2 x 64", sq, 10);
+      timeit<DownStreamCfg>("8192^3 stream 2 x 64", sq, 10);
+      timeit<DownStream32Cfg>("8192^3 stream 4 x 32", sq, 10);
       g_stream = false;
     }
     release(sq);
@@ -841,8 +894,8 @@ int main(int argc, char** argv) {
     Problem x = make(E, rows, I, H, 22, false, 0, 1.0f);   // dXp = dG @ Wg^T + dU @ Wu^T : A [rows, I] twice, B [E, H, I] twice
     uint16_t* A1 = random_bf16((size_t)rows * I, 33, 1.0f);
     for (int rep = 0; rep < 3; ++rep) {
-      const char* names[4] = {"older kernel", "stream 4 x 32, 2 x 4 waves", "stream 4 x 32, 4 x 2 waves", "stream 2 x 64, 2 x 4 waves"};
-      for (g_stream_nt = 0; g_stream_nt <= 3; ++g_stream_nt) {
+      const char* names[3] = {"older kernel", "stream 2 x 64", "stream 4 x 32"};
+      for (g_stream_nt = 0; g_stream_nt <= 2; ++g_stream_nt) {
         char label[96];
         snprintf(label, sizeof label, "Z = dYp @ Wd^T, %s", names[g_stream_nt]);
         time_launches(label, 2.0 * rows * H * I, 10, [&] { launch_nt<DgradCfg>(z, nullptr, 1, false); });
@@ -886,8 +939,8 @@ int main(int argc, char** argv) {
       // the same launch with 64-deep steps in two stages, and with the older kernel
       for (int rep = 0; rep < 3; ++rep) {
         g_stream = true;
-        timeit_cold<GateUpStreamCfg>("C2 gate/up stream 4 x 32 (library)", g2, 20);
-        timeit_cold<GateUpStream2Cfg>("C2 gate/up stream 2 x 64", g2, 20);
+        timeit_cold<GateUpStreamCfg>("C2 gate/up stream 2 x 64 (library)", g2, 20);
+        timeit_cold<GateUpStream32Cfg>("C2 gate/up stream 4 x 32", g2, 20);
         g_stream = false;
         timeit_cold<GateUpCfg>("C2 gate/up, older kernel", g2, 20);
       }
@@ -980,7 +1033,7 @@ int main(int argc, char** argv) {
       launch<DownCfg>(sq, false);
       g_stream = true;
       launch<GateUpStreamCfg>(g, false);
-      launch<GateUpStream2Cfg>(g, false);
+      launch<GateUpStream32Cfg>(g, false);
       launch<DownStreamCfg>(sq, false);
       g_stream = false;
     }
@@ -1091,10 +1144,10 @@ int main(int argc, char** argv) {
         snprintf(name, sizeof name, "%s down, library", sh.name);
         timeit_cold<DownCfg>(name, d, 20);
         g_stream = true;
-        snprintf(name, sizeof name, "%s down, stream 4 x 32", sh.name);
-        timeit_cold<DownStreamCfg>(name, d, 20);
         snprintf(name, sizeof name, "%s down, stream 2 x 64", sh.name);
-        timeit_cold<DownStream2Cfg>(name, d, 20);
+        timeit_cold<DownStreamCfg>(name, d, 20);
+        snprintf(name, sizeof name, "%s down, stream 4 x 32", sh.name);
+        timeit_cold<DownStream32Cfg>(name, d, 20);
         g_stream = false;
         snprintf(name, sizeof name, "%s down, results from accumulators", sh.name);
         timeit_cold<DownDirect>(name, d, 20);
