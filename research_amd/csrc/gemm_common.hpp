@@ -287,7 +287,7 @@ inline double whole_tiles(int64_t rows, int64_t E, bool dense, double ntiles, do
 // per CU 40 us against 63 (2048 tokens, shared 2816; 64-deep steps 41), two per CU with 64-deep steps 55 against 64
 // (4096 tokens; 32-deep 69); 8192 rows x 2048 -> 1024 in 8 groups: 57 against 56 (576 tiles, whole ones kept);
 // 16384 rows in 16 groups x 2816 -> 1024 (1088 against 256 tiles of up to 320 rows): 109 against 87.  The data
-// gradients follow the same line (figures at DgradHalfCfg and DgradHalfDeepCfg); on the wrong side of it 32768
+// gradients follow the same line (figures at DgradHalfCfg); on the wrong side of it 32768
 // rows in 64 groups x 2048 -> 1408 would take 262 us against 228.
 enum class HalfTiles { kNone, kOnePerCu, kRounds };
 // what `half` half tiles take, in rounds of whole ones
@@ -304,6 +304,69 @@ inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, doub
                  pays(spread_mtiles(rows, E, dense, 128) * half_n, whole_tiles(rows, E, dense, full_n, cus, true, tall))
              ? HalfTiles::kRounds
              : HalfTiles::kNone;
+}
+
+// Tile of a product that has no streaming or 64-row tiles, for `rows` rows in E groups times N columns and, in the same
+// launch, dense_rows x dense_N.
+//
+// Where every tile finds a CU of its own nothing hides a step's latency but the loads in flight (operands arrive some
+// 1.3 us after their request, whatever the tile), so the smallest tiles that still do are the fastest.  Rows that may
+// end up in more tiles than the estimates say cost a second round: both have to fit.  us for 128 x 128 / 128 x 64 / 64 x
+// 64, matrices cold:
+//   one group, 2048 x 2816: 387 rows gate/up 30.3 / 21.7 (176 tiles) / 30.8 (308), down 23.7 / 19.1 / 16.6 (224); 700 rows
+//   32.5 / 38.7 (264) / 37.0, down 27.5 / 22.0 (192) / 29.0
+//   8 groups, 1024 x 2048: 400 rows gate/up 25.2 / 20.4 / 20.9, down 17.8 / 14.6 / 12.1
+// One output a tile: 256 x 128 and 128 x 256 ones in three stages take 0.6 of a round of 256 x 256 ones, whose two stages
+// drain once a step (us, 256 x 256 / 128 x 256 / 256 x 128): 2048 rows 2816 -> 2048 down 62 / 41 / 40, dX 127 / 83 / 77; 6000
+// rows in 16 groups, 2816 -> 1024, down 66 / 47 / 44, dX 129 / 91 / 87; two rounds of them are no less than one (8192 rows:
+// 73 / 75 / 81, 139 / 155 / 153).
+// kFewRows: groups that fit one tile of 128 rows.  Bound by the expert matrices, read once, and so by the bytes of them
+// in flight: half as many rows, and more stages or workgroups for it.  us, 256-row tiles / 128-row ones; 64 groups, 2048 x
+// 1408: 77 rows gate/up 146 / 140, dZ 105 / 94, dX 152 / 138, down 77.2 / 78.6; 128 groups, 2048 x 768: 93 rows 168 / 157 and 97
+// / 96, skewed by Zipf's law 198 / 180 and 111 / 106; at 137 rows gate/up 172 / 206, down 87 / 111.  Nearer to 128 rows a few
+// groups more than fit are likely: not where 5 % more tiles are a round more (96 groups of 100, 1304 x 904, four rounds for
+// three: gate/up 118 / 131).
+// Beyond, 128-row tiles (128 x 256 with one output) where they take no more rounds: 12 groups of 333 rows, 1280 x 1792,
+// two rounds either way: gate/up 62 / 50, three for two 53 / 55 (8192 rows, 1024 x 2048).
+// kTall: 256-row tiles of up to 320 rows where they spare a sixth of the rounds by the spread of the groups (such a tile
+// takes a fifth longer), or where there are many rounds (the kernel then decides from the real sizes); else plain ones.
+// us, plain / taller: 64 groups of 137 rows, gate/up 171 / 181, down 87 / 99, dZ 118 / 138; of 256 rows 262 / 213, 128 / 119,
+// 158 / 160, dX 247 / 239; of 325 333 / 336; of 400 308 / 317, 170 / 173, 178 / 199.
+enum class TileShape { k64x64, k128x64, k128x128, k128x128Short, k256x128, k128x256, kFewRows, kTall, kPlain };
+constexpr int64_t kFewGroupRows = 108, kFewGroupRowsSure = 94;  // mean + 3.5 standard deviations within 128
+constexpr double kManyRounds = 8.0;
+inline TileShape tile_shape(int64_t rows, int64_t E, bool dense, int64_t N, double cus, bool dual, int64_t dense_rows = 0,
+                            int64_t dense_N = 0) {
+  auto one_each = [&](int BM, int BN) {
+    const double mtiles = std::fmax(expected_mtiles(rows, E, dense, BM), spread_mtiles(rows, E, dense, BM));
+    return mtiles * (double)((N + BN - 1) / BN) + (double)((dense_rows + BM - 1) / BM * ((dense_N + BN - 1) / BN)) <= cus;
+  };
+  if (one_each(64, 64)) return TileShape::k64x64;
+  if (one_each(128, 64)) return TileShape::k128x64;
+  if (one_each(128, 128)) return TileShape::k128x128;
+  if (!dual && one_each(256, 128)) return TileShape::k256x128;
+  if (!dual && one_each(128, 256)) return TileShape::k128x256;
+  const int BN = dual ? 128 : 256;
+  const double nt = (double)((N + BN - 1) / BN), dense_nt = (double)((dense_N + BN - 1) / BN);
+  auto rounds = [cus](double tiles) { return std::ceil(tiles / cus); };
+  const double plain = spread_mtiles(rows, E, dense, 256) * nt + (double)((dense_rows + 255) / 256) * dense_nt;
+  if (!dense && dense_rows == 0 && rows <= kFewGroupRows * E && (rows <= kFewGroupRowsSure * E || rounds(1.05 * plain) == rounds(plain)))
+    return TileShape::kFewRows;
+  const double tall = tall_mtiles(rows, E, dense, true) * nt + (double)group_mtiles((int)dense_rows, 256, 64) * dense_nt;
+  if (rounds(plain) >= kManyRounds) return TileShape::kTall;
+  const double low = std::fmax(expected_mtiles(rows, E, dense, 128), spread_mtiles(rows, E, dense, 128)) * nt +
+                     (double)((dense_rows + 127) / 128) * dense_nt;
+  if (rounds(low) <= rounds(plain) && 0.72 * rounds(low) < 1.2 * rounds(tall)) return dual ? TileShape::k128x128 : TileShape::k128x256;
+  return 1.2 * rounds(tall) < rounds(plain) ? TileShape::kTall : TileShape::kPlain;
+}
+// ... with a reduction of `steps` 64-deep steps at least, of which a kernel wants twice as many as it has stages, and, for
+// launches of one half tile per CU, nothing larger than that.  k128x128Short: in 32-deep steps.
+inline TileShape tile_shape_for(TileShape s, bool half, int64_t steps, bool dual) {
+  const bool small = s == TileShape::k64x64 || s == TileShape::k128x64 || s == TileShape::k128x128;
+  if (half && !small) s = TileShape::k128x128;
+  const bool four = s == TileShape::k64x64 || s == TileShape::k128x64 || (s == TileShape::k128x128 && !dual);  // stages, or three
+  const bool fits = s == TileShape::kTall || s == TileShape::kPlain || steps >= 2 * (four ? 4 : 3);
+  return fits ? s : half ? TileShape::k128x128Short : TileShape::kTall;
 }
 
 // ---- routed and shared experts in one launch ----

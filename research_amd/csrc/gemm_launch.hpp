@@ -16,10 +16,10 @@ enum class ProductKernel {
   kStream32x64,
   kRows64,        // 64-row LDS tiles, non-temporal loads of the matrix
   kRows64Tail,
-  kHalf,          // 128 x 128 tiles
+  kHalf,          // 128 x 128 tiles, or smaller ones where these leave CUs idle (tile_shape)
   kHalfTail,
   kHalfDeep,
-  kRows256,       // 256-row tiles, of up to 320 rows (grouped_gemm_stream.hpp)
+  kRows256,       // 256-row tiles, or what suits the launch better (tile_shape)
   kRows256Tail,
   kRows256Short,  // gate/up whose reduction is too short for four stages
   kRows256ShortTail,

@@ -219,9 +219,9 @@ int launch_fast(const void* a, const void* b0, const void* b1, void* c, const in
 
 
 // The stream kernel (grouped_gemm_stream.hpp): one software pipeline through all tiles of a workgroup, results written
-// straight from the accumulators.  Its envelope is narrower than launch_fast's (see stream_ok).  256-row tiles run in
-// one workgroup per CU for the whole launch (0.5 to 2 % faster than in workgroups of four tiles each), half tiles in
-// workgroups of four.
+// straight from the accumulators.  Its envelope is narrower than launch_fast's (see stream_ok).  Tiles of up to
+// 320 rows run in one workgroup per CU for the whole launch (0.5 to 2 % faster than in workgroups of four tiles each), the
+// others in workgroups of four (skewed groups: 275 us for gate/up of 24000 rows in 128 groups, 2048 x 768, against 265).
 template <typename Cfg>
 int launch_stream(const void* a, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, hipStream_t stream,
@@ -382,7 +382,7 @@ ProductKernel gate_up_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, bool
   if (pick_skinny(rows, E, dense, I, true, cus, &k)) return k;
   if (!dense && rows <= kTinyGroupRows * E) return tail ? ProductKernel::kRows64Tail : ProductKernel::kRows64;
   if (half_tiles(rows, E, dense, I, cus) == HalfTiles::kOnePerCu &&
-      stream_ok<GateUpHalfTailCfg>(rows, H, I, row_map, row_div))
+      stream_ok<GateUpHalfShortCfg<true>>(rows, H, I, row_map, row_div))
     return tail ? ProductKernel::kHalfTail : ProductKernel::kHalf;
   if (stream_ok<GateUpStreamTailCfg>(rows, H, I, row_map, row_div))
     return tail ? ProductKernel::kRows256Tail : ProductKernel::kRows256;
@@ -394,7 +394,7 @@ ProductKernel down_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, bool de
   if (pick_skinny(rows, E, dense, H, false, cus, &k)) return k;
   if (!dense && rows <= kTinyGroupRows * E) return ProductKernel::kRows64;
   const HalfTiles half = half_tiles(rows, E, dense, H, cus);
-  if (half == HalfTiles::kOnePerCu && stream_ok<DownHalfCfg>(rows, I, H, nullptr, 1)) return ProductKernel::kHalf;
+  if (half == HalfTiles::kOnePerCu && stream_ok<HalfShortCfg>(rows, I, H, nullptr, 1)) return ProductKernel::kHalf;
   if (half != HalfTiles::kNone && stream_ok<DownHalfDeepCfg>(rows, I, H, nullptr, 1)) return ProductKernel::kHalfDeep;
   return I % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
 }
@@ -437,6 +437,15 @@ inline bool fast_ok(const void* a, const void* b0, const void* b1, const void* c
          aligned16(c);
 }
 
+// the tiles of a launch whose kernel the rules above have chosen (half: kHalf, kHalfTail)
+inline TileShape tiles_of(bool half, bool dual, int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense,
+                          const DenseProblem* dp = nullptr) {
+  const TileShape s = tile_shape(rows, E, dense, N, persistent_grid_size(), dual, dp ? dp->rows : 0, dp ? dp->n : 0);
+  const int64_t K = dp ? std::min<int64_t>(Kdim, dp->k) : Kdim;
+  // (plain tiles have four 32-deep stages here)
+  return tile_shape_for(s == TileShape::kPlain && (K + 31) / 32 < 8 ? TileShape::kTall : s, half, (K + 63) / 64, dual);
+}
+
 // y = act Wd[e] on the matrix cores (fast_ok holds); with a map, packed row j reads row row_map[j] / row_div of
 // its group's block of a_group_rows rows (the decode path), and the tiles of `beside` run in the same launch
 int launch_down_fast(const void* act, const void* down, const int32_t* group_sizes, const int32_t* offsets,
@@ -457,14 +466,20 @@ int launch_down_fast(const void* act, const void* down, const int32_t* group_siz
   }
   // (at most half a tile of rows per group on the decode path: the rules above take all of it)
   if (row_map || beside) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: no down kernel reads blocks of rows per group at this size");
-  switch (k) {
-    case ProductKernel::kHalf: return JT_DOWN(launch_stream, DownHalfCfg), 2);
-    case ProductKernel::kHalfDeep: return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
-    default: break;
-  }
-  // 256-row tiles; a reduction too short for the stream kernel, or a result past its limit: the kernel without it
-  const bool tail = k == ProductKernel::kRows256Tail;
-  if (stream_ok<DownStreamTailCfg>(rows, I, H, nullptr, 1)) {
+  const bool tail = k == ProductKernel::kRows256Tail, streams = stream_ok<DownStreamTailCfg>(rows, I, H, nullptr, 1);
+  TileShape tiles = tiles_of(k == ProductKernel::kHalf, false, rows, I, H, E, group_sizes == nullptr);
+  // Two half tiles per CU only where few CUs get a second one (4252 rows 2616 -> 1080, 306 of them: 50 us, 153 tiles of 256 x
+  // 128 57; groups of 250 rows, 296 of them, 55 and 46), or for want of steps (128 groups of 56 rows, skewed, 768 -> 2048: 92 us against 97 in half tiles).
+  const bool deep = k == ProductKernel::kHalfDeep && group_sizes == nullptr &&
+                    4 * ((rows + 127) / 128) * ((H + 127) / 128) <= 5 * persistent_grid_size();
+  if (deep) tiles = TileShape::kPlain;
+  if (k == ProductKernel::kHalfDeep && !deep && large_tiles(tiles))
+    tiles = tile_shape_for(TileShape::k128x256, false, (I + 63) / 64, false);
+  if (streams && !large_tiles(tiles))
+    return with_smaller_tiles<true>(tiles, [&](auto cfg) { return JT_DOWN(launch_stream, decltype(cfg))); });
+  if (k == ProductKernel::kHalfDeep) return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
+  // 256-row tiles; also for a reduction too short for the stream kernel, or a result past its limit: the kernel without it
+  if (streams && tiles == TileShape::kTall) {
     if (tail) return JT_DOWN(launch_stream, DownStreamTailCfg));
     return JT_DOWN(launch_stream, DownStreamCfg));
   }
@@ -497,10 +512,14 @@ int launch_gate_up(const RoutedProblem& p, hipStream_t stream, const Beside* bes
       case ProductKernel::kStream32x64: return JT_GATE_UP(launch_skinny, S22, JT_BESIDE);
       case ProductKernel::kRows64: return JT_GATE_UP(launch_fast, GateUpTinyCfg, JT_BESIDE64);
       case ProductKernel::kRows64Tail: return JT_GATE_UP(launch_fast, GateUpTinyTailCfg);
-      case ProductKernel::kHalf: return JT_GATE_UP(launch_stream, GateUpHalfCfg);
-      case ProductKernel::kHalfTail: return JT_GATE_UP(launch_stream, GateUpHalfTailCfg);
-      case ProductKernel::kRows256: return JT_GATE_UP(launch_stream, GateUpStreamCfg);
-      case ProductKernel::kRows256Tail: return JT_GATE_UP(launch_stream, GateUpStreamTailCfg);
+      case ProductKernel::kHalf:
+      case ProductKernel::kRows256:
+        return with_gate_up_tiles<false, false>(tiles_of(k == ProductKernel::kHalf, true, p.rows, p.K, p.N, p.E, dense),
+                                         [&](auto cfg) { return JT_GATE_UP(launch_stream, decltype(cfg)); });
+      case ProductKernel::kHalfTail:
+      case ProductKernel::kRows256Tail:
+        return with_gate_up_tiles<true, false>(tiles_of(k == ProductKernel::kHalfTail, true, p.rows, p.K, p.N, p.E, dense),
+                                        [&](auto cfg) { return JT_GATE_UP(launch_stream, decltype(cfg)); });
       case ProductKernel::kRows256Short: return JT_GATE_UP(launch_fast, GateUpCfg);
       default: return JT_GATE_UP(launch_fast, GateUpTailCfg);
     }
@@ -550,21 +569,34 @@ int launch_with_shared(const RoutedProblem& gu, const RoutedProblem& dn, const R
   const ProductKernel jd = Elem<T>::is_bf16 ? joint_down_of(dn, sdn) : ProductKernel::kGeneral;
   const bool joint_gu = jg != ProductKernel::kGeneral, joint_dn = jd != ProductKernel::kGeneral;
   const DenseProblem dgu = dense_problem(sgu), ddn = dense_problem(sdn);
+  auto gate_up = [&](auto cfg) { return launch_joint<decltype(cfg)>(gu, dgu, stream); };
+  auto down = [&](auto cfg) { return launch_joint<decltype(cfg)>(dn, ddn, stream); };
   int rc;
   switch (jg) {
     case ProductKernel::kGeneral: rc = launch_gate_up<T>(gu, stream); break;
-    case ProductKernel::kHalf: rc = launch_joint<GateUpHalfCfg>(gu, dgu, stream); break;
-    case ProductKernel::kHalfTail: rc = launch_joint<GateUpHalfTailCfg>(gu, dgu, stream); break;
-    case ProductKernel::kRows256: rc = launch_joint<GateUpStreamCfg>(gu, dgu, stream); break;
-    default: rc = launch_joint<GateUpStreamTailCfg>(gu, dgu, stream); break;
+    case ProductKernel::kHalf:
+    case ProductKernel::kRows256:
+      rc = with_gate_up_tiles<false, true>(tiles_of(jg == ProductKernel::kHalf, true, gu.rows, gu.K, gu.N, gu.E, false, &dgu), gate_up);
+      break;
+    default:
+      rc = with_gate_up_tiles<true, true>(tiles_of(jg == ProductKernel::kHalfTail, true, gu.rows, gu.K, gu.N, gu.E, false, &dgu), gate_up);
+      break;
   }
   if (!rc && !joint_gu && joint_dn) rc = launch_gate_up<T>(sgu, stream);
   if (rc) return rc;
   switch (jd) {
     case ProductKernel::kGeneral: rc = launch_down<T>(dn, stream); break;
-    case ProductKernel::kHalf: rc = launch_joint<DownHalfCfg>(dn, ddn, stream); break;
-    case ProductKernel::kRows256: rc = launch_joint<DownStreamCfg>(dn, ddn, stream); break;
-    default: rc = launch_joint<DownStreamTailCfg>(dn, ddn, stream); break;
+    default: {
+      const TileShape tiles = tiles_of(jd == ProductKernel::kHalf, false, dn.rows, dn.K, dn.N, dn.E, false, &ddn);
+      const bool tail = jd == ProductKernel::kRows256Tail;
+      if (!large_tiles(tiles))
+        rc = with_smaller_tiles<true>(tiles, down);
+      else if (tiles == TileShape::kPlain)
+        rc = tail ? down(DownPlainCfg<true>{}) : down(DownPlainCfg<false>{});
+      else
+        rc = tail ? down(DownStreamTailCfg{}) : down(DownStreamCfg{});
+      break;
+    }
   }
   if (!rc && !joint_gu && !joint_dn) rc = launch_gate_up<T>(sgu, stream);
   if (!rc && !joint_dn) rc = launch_down<T>(sdn, stream);

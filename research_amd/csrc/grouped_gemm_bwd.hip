@@ -261,12 +261,15 @@ ProductKernel gemm_nt_joint(int dtype, const NtProblem& p, int64_t E, const NtPr
 
 int launch_gemm_nt_joint(int dtype, const NtProblem& p, const int32_t* group_sizes, const int32_t* offsets, int64_t E,
                          const NtProblem& s, int segs, hipStream_t stream) {
-  switch (gemm_nt_joint(dtype, p, E, s, segs)) {
-    case ProductKernel::kHalfDeep: return launch_nt_joint<DgradHalfDeepCfg>(p, group_sizes, offsets, E, s, segs, stream);
-    case ProductKernel::kRows256: return launch_nt_joint<DgradStreamCfg>(p, group_sizes, offsets, E, s, segs, stream);
-    case ProductKernel::kRows256Tail: return launch_nt_joint<DgradStreamTailCfg>(p, group_sizes, offsets, E, s, segs, stream);
-    default: return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): no joint launch at this size");
-  }
+  const ProductKernel k = gemm_nt_joint(dtype, p, E, s, segs);
+  if (k == ProductKernel::kGeneral) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): no joint launch at this size");
+  auto launch = [&](auto cfg) { return launch_nt_joint<decltype(cfg)>(p, group_sizes, offsets, E, s, segs, stream); };
+  const TileShape tiles = tile_shape_for(tile_shape(p.rows, E, false, p.N, persistent_grid_size(), false, s.rows, s.N),
+                                         k == ProductKernel::kHalfDeep, (std::min(p.Kdim, s.Kdim) + 63) / 64 * segs, false);
+  if (!large_tiles(tiles)) return with_smaller_tiles<false>(tiles, launch);
+  const bool tail = k == ProductKernel::kRows256Tail;
+  if (tiles == TileShape::kPlain) return tail ? launch(DgradPlainCfg<true>{}) : launch(DgradPlainCfg<false>{});
+  return tail ? launch(DgradStreamTailCfg{}) : launch(DgradStreamCfg{});
 }
 
 int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, const void* b1, void* c,
@@ -280,14 +283,22 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
                        (row_map == nullptr || (rows < ((int64_t)1 << 27) && row_div >= 1 && row_div <= 32));
 #define JT_NT(LAUNCH, CFG) \
   LAUNCH<CFG>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div, a_rows, segs, stream)
-  switch (fast ? data_gradient_kernel(rows, Kdim, N, E, dense, segs, persistent_grid_size()) : ProductKernel::kGeneral) {
-    case ProductKernel::kHalfDeep: return JT_NT(launch_nt_stream, DgradHalfDeepCfg);
-    case ProductKernel::kHalf: return JT_NT(launch_nt_fast, DgradHalfCfg);
-    // 256-row tiles; a reduction too short for the stream kernel, or a result past its limit: the kernel without it
-    case ProductKernel::kRows256: return streams ? JT_NT(launch_nt_stream, DgradStreamCfg) : JT_NT(launch_nt_fast, DgradCfg);
-    case ProductKernel::kRows256Tail:
-      return streams ? JT_NT(launch_nt_stream, DgradStreamTailCfg) : JT_NT(launch_nt_fast, DgradTailCfg);
-    default: break;
+  const ProductKernel k = fast ? data_gradient_kernel(rows, Kdim, N, E, dense, segs, persistent_grid_size()) : ProductKernel::kGeneral;
+  if (k != ProductKernel::kGeneral) {
+    const TileShape tiles = tile_shape_for(tile_shape(rows, E, dense, N, persistent_grid_size(), false),
+                                           k == ProductKernel::kHalfDeep, (Kdim + 63) / 64 * segs, false);
+    // (few steps: two workgroups per CU; 3000 rows 1024 -> 2048 19 us against 22 in one round of 256 x 128 tiles, 2048 rows
+    // 2048 -> 2816 38 against 33)
+    const bool half = k == ProductKernel::kHalf && (Kdim + 63) / 64 * segs < 24;
+    if (half || tiles == TileShape::kFewRows) return JT_NT(launch_nt_fast, DgradHalfCfg);
+    if (streams && !large_tiles(tiles))
+      return with_smaller_tiles<false>(tiles, [&](auto cfg) { return JT_NT(launch_nt_stream, decltype(cfg)); });
+    const bool tail = k == ProductKernel::kRows256Tail;
+    if (k == ProductKernel::kHalf) return JT_NT(launch_nt_fast, DgradHalfCfg);
+    // 256-row tiles; also for a reduction too short for the stream kernel, or a result past its limit: the kernel without it
+    if (streams && tiles == TileShape::kTall)
+      return tail ? JT_NT(launch_nt_stream, DgradStreamTailCfg) : JT_NT(launch_nt_stream, DgradStreamCfg);
+    return tail ? JT_NT(launch_nt_fast, DgradTailCfg) : JT_NT(launch_nt_fast, DgradCfg);
   }
 #undef JT_NT
   if (dtype == JTMOE_F32 && f32_gemm_supported(a0, a1, b0, b1, c, row_map ? a_rows : rows, Kdim, N) &&

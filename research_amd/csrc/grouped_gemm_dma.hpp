@@ -130,7 +130,8 @@ struct DmaGemmCfg {
   static constexpr int XROWS = (OPT_ & 131072) ? 64 : 0;
   static constexpr bool kDual = kDual_;
   static constexpr int BNE = kDual ? 2 * BN : BN;  // columns of the B tile in LDS
-  static constexpr int NSUB = BNE / 128;           // 128-column sub-tiles of B
+  static constexpr int SUBW = BN == 64 ? 64 : 128;  // columns of a sub-tile of B (64: stream kernel)
+  static constexpr int NSUB = BNE / SUBW;
   static constexpr int NT = WAVES_M * WAVES_N * 64;
   static constexpr int WM = BM / WAVES_M, WN = BNE / WAVES_N;
   static constexpr int TM = WM / 32, TN = WN / 32;
@@ -138,10 +139,10 @@ struct DmaGemmCfg {
   static constexpr int WNO = TNO * 32;
   static constexpr int CPRA = BK / 8;  // 16-byte chunks per A row
   static constexpr int A_BYTES = (BM + XROWS) * BK * 2;
-  static constexpr int BSUB_BYTES = BK * 256;
+  static constexpr int BSUB_BYTES = BK * SUBW * 2;
   static constexpr int STAGE_BYTES = A_BYTES + NSUB * BSUB_BYTES;
   static constexpr int A_LOADS = BM * CPRA / NT;   // per thread per stage
-  static constexpr int BSUB_LOADS = BK * 16 / NT;  // per thread per sub-tile per stage
+  static constexpr int BSUB_LOADS = BK * (SUBW / 8) / NT;  // per thread per sub-tile per stage
   static constexpr int LPS = A_LOADS + NSUB * BSUB_LOADS;
   static constexpr int CS = WNO + 8;  // epilogue staging row stride (elements)
   static constexpr size_t EPI_BYTES = (size_t)WAVES_M * WAVES_N * WM * CS * 2;
@@ -156,12 +157,12 @@ struct DmaGemmCfg {
   // spilled) four really are resident, instead of three and two: gate/up at 37 tokens x 8 of 128 experts, 2048 -> 768
   // (800 workgroups) 79 -> 73.5 us, down of 64 tokens x 8 of 64 experts (576 workgroups) 58 -> 55.
   static constexpr int MIN_WAVES_PER_EU = NT != 256 ? 1 : (BM == 64 ? 4 : (TM * TN * 16 >= 128 ? 2 : 1));
-  static_assert(BNE % 128 == 0, "B tile is made of 128-column sub-tiles");
+  static_assert(BNE % SUBW == 0, "B tile is made of whole sub-tiles");
   static_assert(BK == 32 || BK == 64, "BK must be 32 or 64");
-  static_assert((BM * CPRA) % NT == 0 && (BK * 16) % NT == 0, "tile must divide evenly over the threads");
+  static_assert((BM * CPRA) % NT == 0 && (BK * (SUBW / 8)) % NT == 0, "tile must divide evenly over the threads");
   static_assert((NT / CPRA) % 16 == 0 && NT % 64 == 0, "swizzle must not depend on the load index");
   static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must be made of 32x32x16 MFMAs");
-  static_assert(!kDual || (TN % 2 == 0 && BN == 128), "dual tiles: one sub-tile per matrix");
+  static_assert(!kDual || (TN % 2 == 0 && BN == SUBW), "dual tiles: one sub-tile per matrix");
   static_assert(NSTAGE >= 2 && (NSTAGE - 2) * LPS < 64, "vmcnt is a 6-bit counter");
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
   static_assert(XROWS == 0 || (WAVES_M == 2 && TM == 4 && NT == 512 && XROWS * CPRA <= NT), "a fifth row block per wave");

@@ -93,12 +93,13 @@ __device__ __forceinline__ void stream_gemm_body(
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, NS = Cfg::NSTAGE;
   constexpr int TM = Cfg::TM, TN = Cfg::TN, WN = Cfg::WN;
   constexpr int CPRA = Cfg::CPRA, KK = BK / 16, LPS = Cfg::LPS;
+  constexpr int kBand = Cfg::SUBW / 64;  // 4 x 64 blocks of B side by side in a sub-tile
   constexpr bool kDual = Cfg::kDual;
-  // A wave's row blocks of 32 lie kRowStep apart, those of the waves above one another in turn, so that the rows of
-  // a tile that is not full are spread over all of them.  X: rows that a group's last tile may have beyond BM, a
-  // block more per wave.
-  constexpr int X = Cfg::XROWS, TMX = TM + (X ? 1 : 0), kRowStep = Cfg::WAVES_M * 32;
-  constexpr int kManyRounds = 8;
+  // X: rows that a group's last tile may have beyond BM, a block of 32 more per wave.  The row blocks of a wave then lie
+  // kRowStep apart, those of the waves above one another in turn; without such rows they are neighbours, so that waves
+  // without rows leave the LDS to the others (two blocks of each wave are bound by its reads: down of 333 rows a group 55.8
+  // us in turn, 54.3 as neighbours).
+  constexpr int X = Cfg::XROWS, TMX = TM + (X ? 1 : 0), kRowStep = X ? Cfg::WAVES_M * 32 : 32, kWaveStep = X ? 32 : TM * 32;
   using L = StreamLayout<Cfg>;
   static_assert(KK % 2 == 0, "fragment double buffer wants an even number of sub-steps");
   static_assert(kNT || (Cfg::OPT & 128) != 0, "weight tiles in 4 x 64 blocks");
@@ -157,7 +158,7 @@ __device__ __forceinline__ void stream_gemm_body(
     };
     const int tall = mtiles_with(X), dense_tall = kJoint ? group_mtiles(dp.rows, BM, X) : 0;
     const int plain_rounds = rounds(real_mtiles, dense_mtiles);
-    if (plain_rounds >= kManyRounds || rounds(tall, dense_tall) < plain_rounds) {
+    if (plain_rounds >= (int)kManyRounds || rounds(tall, dense_tall) < plain_rounds) {
       extra = X;
       real_mtiles = tall;
       dense_mtiles = dense_tall;
@@ -226,7 +227,7 @@ __device__ __forceinline__ void stream_gemm_body(
   // last NS steps of a tile request the next tile's first steps, so the plan switches over to the next
   // tile NS steps before the current tile ends; nothing else of the current tile depends on it. ----
   constexpr int NSEG = kNT ? 2 : 1;                        // A descriptors (one per segment)
-  constexpr int NBD = kNT ? 2 : Cfg::NSUB;                 // B descriptors (per segment / per 128-column sub-tile)
+  constexpr int NBD = kNT ? 2 : Cfg::NSUB;                 // B descriptors (per segment / per sub-tile)
   constexpr int B_LOADS = kNT ? BN * CPRA / NT : Cfg::NSUB;  // entries of b_voff
   static_assert(!kNT || B_LOADS == Cfg::NSUB * Cfg::BSUB_LOADS, "a stage has LPS loads in either form");
   struct Plan {
@@ -281,10 +282,10 @@ __device__ __forceinline__ void stream_gemm_body(
       for (int u = 0; u < Cfg::NSUB; ++u) p.b_rsrc[u] = make_rsrc((kDual && u == 1 ? b1 : b0) + wofs, p.k * p.n * 2);
       p.a_rsrc[0] = gathered ? make_rsrc(a0, a_rows * Kdim * 2) : make_rsrc(a0 + (size_t)t.row0 * p.k, t.rows * p.k * 2);
       // (B in 4 x 64 blocks: row and chunk of this thread)
-      const int b_blk_id = tid_f >> 5, b_k = (b_blk_id >> 1) * 4 + ((tid_f >> 3) & 3);
-      const int b_c = (b_blk_id & 1) * 8 + ((tid_f & 7) ^ (((tid_f >> 4) & 1) << 2));
+      const int b_blk_id = tid_f >> 5, b_k = (b_blk_id / kBand) * 4 + ((tid_f >> 3) & 3);
+      const int b_c = (b_blk_id % kBand) * 8 + ((tid_f & 7) ^ (((tid_f >> 4) & 1) << 2));
 #pragma unroll
-      for (int u = 0; u < Cfg::NSUB; ++u) p.b_voff[u] = (b_k * p.n + t.n0 + (kDual ? 0 : u * 128) + b_c * 8) * 2;
+      for (int u = 0; u < Cfg::NSUB; ++u) p.b_voff[u] = (b_k * p.n + t.n0 + (kDual ? 0 : u * Cfg::SUBW) + b_c * 8) * 2;
     }
 #pragma unroll
     for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = (load_row(tid_f, j) * p.k + chunk * 8) * 2;
@@ -306,7 +307,10 @@ __device__ __forceinline__ void stream_gemm_body(
     for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = offset_of(load_row(tid_f, j));
     if (p.x) p.x_voff = offset_of(x_row(tid_f));
   };
-  // behind the last tile: loads that store zeros, so that every step has as many
+  // The steps that end the launch.  With few accumulators they have a loop of their own, without loads (128 x 256 tiles,
+  // one each: 51.3 us against 53.5 for 2688 -> 1024); with many that loop would have hundreds of registers spilled, and
+  // they issue loads that store zeros.
+  constexpr bool kOwnEnd = X == 0 && TM * TN <= 4;
   auto plan_nothing = [](Plan& p) {
 #pragma unroll
     for (int j = 0; j < Cfg::A_LOADS; ++j) p.a_voff[j] = kOutside;
@@ -335,7 +339,7 @@ __device__ __forceinline__ void stream_gemm_body(
       } else {
         const int u = (i - Cfg::A_LOADS) / Cfg::BSUB_LOADS, jb = (i - Cfg::A_LOADS) % Cfg::BSUB_LOADS;
         buffer_load_lds16(p.b_rsrc[u], base + Cfg::A_BYTES + u * Cfg::BSUB_BYTES + jb * NT * 16,
-                          p.b_voff[u] + jb * (NT / 16) * p.n * 2 + (kTail ? k0 * p.n * 2 : 0), kTail ? 0 : k0 * p.n * 2);
+                          p.b_voff[u] + jb * (NT * 8 / Cfg::SUBW) * p.n * 2 + (kTail ? k0 * p.n * 2 : 0), kTail ? 0 : k0 * p.n * 2);
       }
     }
   };
@@ -354,10 +358,10 @@ __device__ __forceinline__ void stream_gemm_body(
   };
 
   // ---- fragment addresses of this lane (bytes inside a stage) ----
-  const int a_row = wm * 32 + (lane & 31);
+  const int a_row = wm * kWaveStep + (lane & 31);
   const int a_sw = (a_row / (16 / CPRA)) % CPRA;
   const int a_rowoff = a_row * (BK * 2);
-  const int b_laneoff = ((lane & 15) >> 2) * 128 + (lane & 3) * 8 + ((lane >> 4) & 1) * 32 + (lane >> 5) * 2048;
+  const int b_laneoff = ((lane & 15) >> 2) * 128 + (lane & 3) * 8 + ((lane >> 4) & 1) * 32 + (lane >> 5) * (2 * kBand * 512);
   const int half_swap = ((lane >> 3) & 1) * 64;
   int b_blk[TN];
   // kNT: the B tile in the A tile's layout, this lane's row = its output column
@@ -371,8 +375,8 @@ __device__ __forceinline__ void stream_gemm_body(
       col = (jj < TN / 2 ? 0 : BN) + wn * (WN / 2) + (jj % (TN / 2)) * 32;
     else
       col = wn * WN + jj * 32;
-    const int u = col >> 7;
-    b_blk[jj] = Cfg::A_BYTES + u * Cfg::BSUB_BYTES + ((col & 127) >> 6) * 512 + (col & 63) * 2 +
+    const int u = col / Cfg::SUBW;
+    b_blk[jj] = Cfg::A_BYTES + u * Cfg::BSUB_BYTES + (col % Cfg::SUBW / 64) * 512 + (col & 63) * 2 +
                 ((col & 32) ? -half_swap : half_swap);
   }
   auto load_frag_a = [&](int stage, int kk, int mi) -> bf16x8_t {
@@ -384,10 +388,10 @@ __device__ __forceinline__ void stream_gemm_body(
       const unsigned char* st = smem_raw + stage * Cfg::STAGE_BYTES;
       return *reinterpret_cast<const bf16x8_t*>(st + bt_rowoff + jj * 32 * BK * 2 + (((kk * 2 + (lane >> 5)) ^ bt_sw) << 4));
     }
-    const unsigned char* p = smem_raw + stage * Cfg::STAGE_BYTES + b_blk[jj] + b_laneoff + kk * (4 * 8 * 128);
+    const unsigned char* p = smem_raw + stage * Cfg::STAGE_BYTES + b_blk[jj] + b_laneoff + kk * (4 * kBand * 512);
     const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p));
     const s16x4_t hi =
-        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + 8 * 128));
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + kBand * 512));
     const s16x8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(bf16x8_t, both);
   };
@@ -419,7 +423,7 @@ __device__ __forceinline__ void stream_gemm_body(
   while (true) {
     const int cur_n = tile_n(cur);
     // row blocks of this wave that hold rows of the tile (none either if its columns lie past N)
-    const int blocks = cur.n0 + wn * Cfg::WNO < cur_n ? max(0, (cur.rows - wm * 32 + kRowStep - 1) / kRowStep) : 0;
+    const int blocks = cur.n0 + wn * Cfg::WNO < cur_n ? max(0, (cur.rows - wm * kWaveStep + kRowStep - 1) / kRowStep) : 0;
     if constexpr (!kJoint) idx += stride;
     --left;
     const Tile nxt = locate(left > 0 ? idx : 0x3fffffff);
@@ -460,6 +464,61 @@ __device__ __forceinline__ void stream_gemm_body(
         else
           bf[set][f - NB] = load_frag_b(stage, kk, f - NB);
       };
+      // a step: with the loads of step `ahead` of the planned tile, or (kLoads = false) as the one before `left` others that end
+      // the launch
+      auto step = [&](auto loads_tag, int ahead, bool x_loads, int left) {
+        constexpr bool kLoads = decltype(loads_tag)::value;
+        // sub-steps 0 .. KK-2: the fragments of the following sub-step are requested, then this one's MFMAs, which the
+        // scheduler interleaves with the LDS reads (two per MFMA)
+#pragma unroll
+        for (int kk = 0; kk < KK - 1; ++kk) {
+          if (NB > 0 && !kNoFragReads)
+#pragma unroll
+            for (int f = 0; f < NB + TN; ++f) read((kk + 1) & 1, cs, kk + 1, f);
+#pragma unroll
+          for (int g = 0; g < kMfmas; ++g) mfma(kk & 1, g);
+#pragma unroll
+          for (int g = 0; g < kMfmas; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // the next step's stage has arrived (own loads: the wait; everyone's: the barrier), and every
+        // wave holds its last fragments of the current stage, which is therefore free
+        // (a stage is LPS loads, with X rows one more)
+        if (X != 0 && NS > 2 && x_loads)
+          wait_and_barrier<(NS - 2) * (LPS + 1)>();
+        else if (kLoads || left == NS - 1)
+          wait_and_barrier<(NS - 2) * LPS>();
+        else if (NS > 3 && left == NS - 2)
+          wait_and_barrier<(NS > 3 ? NS - 3 : 0) * LPS>();
+        else
+          wait_and_barrier<0>();
+        __builtin_amdgcn_sched_barrier(0);
+        // last sub-step, in a fixed order: after each of its MFMAs operand loads of step `ahead` (into the stage just
+        // released) and fragment reads of the next step are issued
+        const int ns = (NS & (NS - 1)) == 0 ? (cs + 1) & (NS - 1) : cs + 1 == NS ? 0 : cs + 1, kt = kSameTile ? 0 : ahead;
+        constexpr int kSlots = kMfmas > 0 ? kMfmas : 1;
+        constexpr int kLoadsPer = (LPS + kSlots - 1) / kSlots, kFragsPer = (NB + TN + kSlots - 1) / kSlots;
+#pragma unroll
+        for (int g = 0; g < kSlots; ++g) {
+          if (NB > 0) mfma((KK - 1) & 1, g);
+          __builtin_amdgcn_sched_barrier(0);
+          if (kLoads && !kNoLoads) {
+#pragma unroll
+            for (int q = 0; q < kLoadsPer; ++q)
+              if (g * kLoadsPer + q < LPS) issue_one(pl, kt, cs, g * kLoadsPer + q);
+          }
+          if (NB > 0 && !kNoFragReads)
+#pragma unroll
+            for (int q = 0; q < kFragsPer; ++q)
+              if (g * kFragsPer + q < NB + TN) read(0, ns, 0, g * kFragsPer + q);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (kLoads && !kNoLoads) issue_x(pl, kt, cs);
+        cs = ns;
+      };
       // all steps but the last NS, then, with the next tile's plan, those: their loads are its first steps'
 #pragma unroll 1
       for (int part = 0; part < 2; ++part) {
@@ -468,63 +527,24 @@ __device__ __forceinline__ void stream_gemm_body(
           if (have_next) {
             plan_tile(pl, nxt);
             if (gather && !second_product(nxt)) plan_rows(pl, nxt, [&](int r) { return rowbuf[r]; });
+          } else if constexpr (kOwnEnd) {
+            break;
           } else {
             plan_nothing(pl);
           }
         }
         const bool x_loads = x_rows && !part;  // (part 1: of some stages, then of others)
-        for (int j = j0; j < j1; ++j) {
-          // sub-steps 0 .. KK-2: the fragments of the following sub-step are requested, then this one's MFMAs, which the
-          // scheduler interleaves with the LDS reads (two per MFMA)
-#pragma unroll
-          for (int kk = 0; kk < KK - 1; ++kk) {
-            if (NB > 0 && !kNoFragReads)
-#pragma unroll
-              for (int f = 0; f < NB + TN; ++f) read((kk + 1) & 1, cs, kk + 1, f);
-#pragma unroll
-            for (int g = 0; g < kMfmas; ++g) mfma(kk & 1, g);
-#pragma unroll
-            for (int g = 0; g < kMfmas; ++g) {
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-              __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          // the next step's stage has arrived (own loads: the wait; everyone's: the barrier), and every
-          // wave holds its last fragments of the current stage, which is therefore free
-          // (a stage is LPS loads, with X rows one more)
-          if (X != 0 && NS > 2 && x_loads)
-            wait_and_barrier<(NS - 2) * (LPS + 1)>();
-          else
-            wait_and_barrier<(NS - 2) * LPS>();
-          __builtin_amdgcn_sched_barrier(0);
-          // last sub-step, in a fixed order: after each of its MFMAs operand loads of step j + ahead (into the stage just
-          // released) and fragment reads of step j + 1 are issued
-          const int ns = (cs + 1) & (NS - 1), kt = kSameTile ? 0 : j + ahead;
-          constexpr int kSlots = kMfmas > 0 ? kMfmas : 1;
-          constexpr int kLoadsPer = (LPS + kSlots - 1) / kSlots, kFragsPer = (NB + TN + kSlots - 1) / kSlots;
-#pragma unroll
-          for (int g = 0; g < kSlots; ++g) {
-            if (NB > 0) mfma((KK - 1) & 1, g);
-            __builtin_amdgcn_sched_barrier(0);
-            if (!kNoLoads) {
-#pragma unroll
-              for (int q = 0; q < kLoadsPer; ++q)
-                if (g * kLoadsPer + q < LPS) issue_one(pl, kt, cs, g * kLoadsPer + q);
-            }
-            if (NB > 0 && !kNoFragReads)
-#pragma unroll
-              for (int q = 0; q < kFragsPer; ++q)
-                if (g * kFragsPer + q < NB + TN) read(0, ns, 0, g * kFragsPer + q);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          if (!kNoLoads) issue_x(pl, kt, cs);
-          cs = ns;
+        for (int j = j0; j < j1; ++j) step(std::true_type{}, j + ahead, x_loads, 0);
+      }
+      if constexpr (kOwnEnd) {
+        if (!have_next) {
+#pragma unroll 1
+          for (int left = NS - 1; left >= 0; --left) step(std::false_type{}, 0, false, left);
         }
       }
       // epilogue: straight from the accumulators to memory (no LDS, no barrier)
       if constexpr (NB > 0)
-        store_transposed_accumulators<Cfg, NB>(acc, wm * 32, kRowStep, wn, cur.row0, cur.rows, cur.n0, cur_n,
+        store_transposed_accumulators<Cfg, NB>(acc, wm * kWaveStep, kRowStep, wn, cur.row0, cur.rows, cur.n0, cur_n,
                                                second ? dp.rows : dense_rows, second ? dp.c : C,
                                                second ? dp.save0 : save0, second ? dp.save1 : save1);
     };
@@ -533,13 +553,13 @@ __device__ __forceinline__ void stream_gemm_body(
     else if (TM > 2 && blocks > 2)
       run_tile(std::integral_constant<int, TM>{});
     else if (blocks > 0)
-      run_tile(std::integral_constant<int, 2>{});
+      run_tile(std::integral_constant<int, TM < 2 ? TM : 2>{});
     else
       run_tile(std::integral_constant<int, 0>{});
-    static_assert(TM == 2 || TM == 4, "row blocks per wave");
+    static_assert(TM == 1 || TM == 2 || TM == 4, "row blocks per wave");
     if (!have_next) break;
-    // (only now: no fragment stays in registers through the epilogue)
-    load_frags(cs, 0, af[0], bf[0]);
+    // (with X rows no fragment stays in registers through the epilogue; without, a wave whose tile is full has read them)
+    if (X != 0 || blocks <= (TM > 2 ? 2 : 0)) load_frags(cs, 0, af[0], bf[0]);
     cur = nxt;
     nk = nk_next;
   }
@@ -608,17 +628,63 @@ using DownStreamCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 32768 
 using DownStreamTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 32768 + 65536 + 131072>;
 using DgradStreamCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 131072>;
 using DgradStreamTailCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + 65536 + 131072>;
-// Half-size tiles in four-wave workgroups for launches that would leave CUs without a 256-row tile: gate/up with
-// one workgroup per CU (99 KB of LDS), down with two.  The dispatch rules and what they measured stand in
-// grouped_gemm.hip.  (The check for a ragged last step costs nothing: 33.3 against 33.7 us without it for gate/up,
-// 39.8 against 40.4 for down, so that one variant of the latter serves every width.)
-using GateUpHalfCfg = DmaGemmCfg<128, 128, 32, 2, 2, true, 4, 16 + 128>;
-using GateUpHalfTailCfg = DmaGemmCfg<128, 128, 32, 2, 2, true, 4, 16 + 128 + 65536>;  // for K % 64 != 0
-using DownHalfCfg = DmaGemmCfg<128, 128, 32, 2, 2, false, 4, 16 + 128 + 65536>;
-using DownHalfDeepCfg = DmaGemmCfg<128, 128, 64, 2, 2, false, 2, 16 + 128 + 65536>;
-// Data gradients in half tiles, launched where one has at most one of them per CU: nothing else runs on the CU,
-// so four 64-deep stages (131 KB) keep its loads going.  4096 rows x 4096 -> 1024: 40 us, two 64-deep stages with
-// two workgroups per CU 59, four 32-deep ones 49, 256 x 256 tiles 93; 2048 rows x 5632 -> 2048: 55, 79, 67 and 124.
+// ... without the rows beyond 256, for launches in which no round is to be spared: gate/up in 32-deep steps and four
+// stages (figures at tile_shape).  Alone, the others then run in the kernels of grouped_gemm_dma.hpp and
+// grouped_gemm_bwd.hpp (64 groups of 180 rows, us: down 90 against 97 here, dZ 119 against 128); these are for joint
+// launches (down 60 against 63 us with them, 4096 tokens of 1024, 8 experts top-2 and one shared of 2048).
+template <bool kTail, bool kJoint>
+using GateUpPlainCfg = DmaGemmCfg<256, 128, 32, kJoint ? 4 : 2, kJoint ? 2 : 4, true, 4, 16 + 128 + (kTail ? 65536 : 0)>;
+template <bool kTail>
+using DownPlainCfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + (kTail ? 65536 : 0)>;
+template <bool kTail>
+using DgradPlainCfg = DmaGemmCfg<256, 256, 64, 2, 4, false, 2, 16 + 128 + (kTail ? 65536 : 0)>;
+// Smaller tiles (tile_shape).  128 x 128 ones in eight waves: gate/up of 1024 rows, 2048 x 2816, 33.8 us against 40.5 in
+// four waves and 32-deep steps, down 29.2 against 37.6; the
+// data gradients are up to 5 % faster in four.  (The check for a ragged last step costs nothing: one variant
+// serves every width where there is no SwiGLU.)
+template <bool kTail>
+using GateUpQuarterCfg = DmaGemmCfg<64, 64, 64, 2, 2, true, 4, 16 + 128 + (kTail ? 65536 : 0)>;
+template <bool kTail>
+using GateUpNarrowCfg = DmaGemmCfg<128, 64, 64, 2, 2, true, 4, 16 + 128 + (kTail ? 65536 : 0)>;
+template <bool kTail>
+using GateUpHalfCfg = DmaGemmCfg<128, 128, 64, 2, 4, true, 3, 16 + 128 + (kTail ? 65536 : 0)>;
+template <bool kTail>
+using GateUpHalfShortCfg = DmaGemmCfg<128, 128, 32, 2, 2, true, 4, 16 + 128 + (kTail ? 65536 : 0)>;
+using QuarterCfg = DmaGemmCfg<64, 64, 64, 2, 2, false, 4, 16 + 128 + 65536>;  // down and data gradients
+using NarrowCfg = DmaGemmCfg<128, 64, 64, 2, 2, false, 4, 16 + 128 + 65536>;
+using DownHalfCfg = DmaGemmCfg<128, 128, 64, 2, 4, false, 4, 16 + 128 + 65536>;
 using DgradHalfDeepCfg = DmaGemmCfg<128, 128, 64, 2, 2, false, 4, 16 + 128 + 65536>;
+using HalfShortCfg = DmaGemmCfg<128, 128, 32, 2, 2, false, 4, 16 + 128 + 65536>;
+using Rows256Cfg = DmaGemmCfg<256, 128, 64, 4, 2, false, 3, 16 + 128 + 65536>;
+using Rows128Cfg = DmaGemmCfg<128, 256, 64, 2, 4, false, 3, 16 + 128 + 65536>;
+// two workgroups per CU
+using DownHalfDeepCfg = DmaGemmCfg<128, 128, 64, 2, 2, false, 2, 16 + 128 + 65536>;
+
+// launch(Cfg{}) with the configuration of a shape
+template <bool kTail, bool kJoint, typename Launch>
+int with_gate_up_tiles(TileShape s, Launch launch) {
+  switch (s) {
+    case TileShape::k64x64: return launch(GateUpQuarterCfg<kTail>{});
+    case TileShape::k128x64: return launch(GateUpNarrowCfg<kTail>{});
+    case TileShape::k128x128:
+    case TileShape::kFewRows: return launch(GateUpHalfCfg<kTail>{});
+    case TileShape::k128x128Short: return launch(GateUpHalfShortCfg<kTail>{});
+    case TileShape::kPlain: return launch(GateUpPlainCfg<kTail, kJoint>{});
+    default: return launch(std::conditional_t<kTail, GateUpStreamTailCfg, GateUpStreamCfg>{});
+  }
+}
+// ... for down products and data gradients, all but the largest
+template <bool kDown, typename Launch>
+int with_smaller_tiles(TileShape s, Launch launch) {
+  switch (s) {
+    case TileShape::k64x64: return launch(QuarterCfg{});
+    case TileShape::k128x64: return launch(NarrowCfg{});
+    case TileShape::k128x128: return launch(std::conditional_t<kDown, DownHalfCfg, DgradHalfDeepCfg>{});
+    case TileShape::k256x128: return launch(Rows256Cfg{});
+    case TileShape::k128x128Short: return launch(HalfShortCfg{});
+    default: return launch(Rows128Cfg{});
+  }
+}
+inline bool large_tiles(TileShape s) { return s == TileShape::kTall || s == TileShape::kPlain; }
 
 }  // namespace jtmoe
