@@ -1,7 +1,12 @@
-// The dispatch plan of a small batch, computed by ONE workgroup: histogram of the expert ids in LDS,
-// exclusive scan over the experts, then the stable rank of every assignment (ballots inside a wave,
-// a per-wave table across the waves).  Same results as the three-pass plan of dispatch.hip
-// (local_dispatch of the reference at ep_size == 1, moe.py:583-602).
+// The dispatch plan of a small batch, computed by ONE workgroup: a histogram of the expert ids per wave in LDS, one
+// scan over experts and waves, then the stable rank of every assignment (ballots inside a wave, the wave's own next free
+// rows).  Same results as the three-pass plan of dispatch.hip (local_dispatch of the reference at ep_size == 1,
+// moe.py:583-602).
+//
+// Latency bounds it.  A wave owns a run of consecutive assignments, so that the waves meet three times in all,
+// whatever the number of assignments, and the ids arrive kDispatchBatch loads at a time.  (In rounds of the whole
+// workgroup, with two meetings and a load each, 3096 assignments to 64 experts with statistics took 11.0 us, now 7.1;
+// without them 4.4 us at 320, 6.4 at 4096, 9.7 at 8192.)
 //
 // The body is a device function so that two kernels can end in it: the stand-alone small dispatch,
 // and the last workgroup of the small-batch router, which then goes on from the ids it still holds
@@ -24,10 +29,12 @@ __device__ __forceinline__ unsigned long long importance_term(float w) {
   return (unsigned long long)(w * kImportanceScale);
 }
 
-// LDS of the body: cursor[E], wavehist[waves][E], wave_sums[waves] ints, then (kStats) imp[E] of 8 bytes
+constexpr int kDispatchBatch = 4;  // loads of a lane in flight
+
+// LDS of the body: next[waves][E], wave_sums[waves] ints, then (kStats) imp[E] of 8 bytes
 __host__ __device__ inline size_t dispatch_small_smem_bytes(int E, int threads, bool stats) {
   const int waves = threads / kWave;
-  size_t n = ((size_t)E * (1 + waves) + waves) * sizeof(int);
+  size_t n = ((size_t)E * waves + waves) * sizeof(int);
   n = (n + 7) / 8 * 8;
   if (stats) n += (size_t)E * 8;
   return n;
@@ -36,7 +43,7 @@ __host__ __device__ inline size_t dispatch_small_smem_bytes(int E, int threads, 
 // ids: A expert ids in assignment order (global memory or LDS); ids outside [0, E) are dropped.
 // kStats: also expert_counts[e] = number of assignments of e (as float) and importance[e] = the sum
 // of their route weights (the two vectors of _router_stats, moe.py:802-805).
-// Requires blockDim.x == kThreads and, for the scan, E <= kThreads.  Ends without a barrier.
+// Requires A > 0, blockDim.x == kThreads and, for the scan, E <= kThreads.  Ends without a barrier.
 template <int kThreads, bool kStats, typename WT>
 __device__ __forceinline__ void dispatch_small_body(const int32_t* ids, const WT* weights, int A, int E,
                                                     int32_t* __restrict__ group_sizes, int32_t* __restrict__ offsets,
@@ -44,28 +51,43 @@ __device__ __forceinline__ void dispatch_small_body(const int32_t* ids, const WT
                                                     float* __restrict__ expert_counts, float* __restrict__ importance,
                                                     unsigned char* smem_raw) {
   constexpr int kWaves = kThreads / kWave;
-  int* const cursor = reinterpret_cast<int*>(smem_raw);  // [E] histogram, then the next free packed row of expert e
-  int* const wavehist = cursor + E;                      // [kWaves][E]
-  int* const wave_sums = wavehist + kWaves * E;          // [kWaves]
+  int* const next = reinterpret_cast<int*>(smem_raw);  // [kWaves][E] assignments of the wave, then its next packed row
+  int* const wave_sums = next + kWaves * E;            // [kWaves]
   unsigned long long* const imp =
-      reinterpret_cast<unsigned long long*>(smem_raw + (((size_t)E * (1 + kWaves) + kWaves) * sizeof(int) + 7) / 8 * 8);
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-  for (int e = tid; e < E; e += kThreads) {
-    cursor[e] = 0;
-    if (kStats) imp[e] = 0ull;
-  }
-  for (int i = tid; i < kWaves * E; i += kThreads) wavehist[i] = 0;
+      reinterpret_cast<unsigned long long*>(smem_raw + (((size_t)E * kWaves + kWaves) * sizeof(int) + 7) / 8 * 8);
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  if (kStats)
+    for (int e = tid; e < E; e += kThreads) imp[e] = 0ull;
+  const int run = (A + kThreads - 1) / kThreads * kWave;                // assignments of a wave
+  const int waves = A <= kThreads ? (A + kWave - 1) / kWave : kWaves;  // no wave behind these has any
+  for (int i = tid; i < waves * E; i += kThreads) next[i] = 0;
   __syncthreads();
-  for (int a = tid; a < A; a += kThreads) {
-    const int id = ids[a];
-    if (id >= 0 && id < E) {
-      atomicAdd(&cursor[id], 1);
-      if (kStats) atomicAdd(&imp[id], importance_term(Elem<WT>::load(weights + a)));
+  const int first = wave * run, end = min(first + run, A);
+  int* const mine = next + wave * E;
+  for (int base = first; base < end; base += kDispatchBatch * kWave) {
+    int id[kDispatchBatch];
+    float w[kDispatchBatch];
+#pragma unroll
+    for (int i = 0; i < kDispatchBatch; ++i) {
+      const int a = base + i * kWave + lane;
+      id[i] = a < end ? ids[a] : -1;
+      if (kStats) w[i] = a < end ? Elem<WT>::load(weights + a) : 0.0f;
     }
+#pragma unroll
+    for (int i = 0; i < kDispatchBatch; ++i)
+      if (base + i * kWave < end && id[i] >= 0 && id[i] < E) {
+        atomicAdd(&mine[id[i]], 1);
+        if (kStats) atomicAdd(&imp[id[i]], importance_term(w[i]));
+      }
   }
   __syncthreads();
   // exclusive scan over the experts: thread e owns expert e
-  const int count = tid < E ? cursor[tid] : 0;
+  int of_wave[kWaves], count = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) of_wave[w] = tid < E && w < waves ? next[w * E + tid] : 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) count += of_wave[w];
   int incl = count;
 #pragma unroll
   for (int d = 1; d < kWave; d <<= 1) {
@@ -76,11 +98,15 @@ __device__ __forceinline__ void dispatch_small_body(const int32_t* ids, const WT
   __syncthreads();
   int before = 0;
   for (int w = 0; w < wave; ++w) before += wave_sums[w];
-  const int start = incl + before - count;
   if (tid < E) {
-    offsets[tid] = start;
+    int row = incl + before - count;
+    offsets[tid] = row;
     group_sizes[tid] = count;
-    cursor[tid] = start;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      if (w < waves) next[w * E + tid] = row;
+      row += of_wave[w];
+    }
     if (kStats) {
       expert_counts[tid] = (float)count;
       importance[tid] = (float)((double)imp[tid] * (1.0 / 4294967296.0));
@@ -89,43 +115,39 @@ __device__ __forceinline__ void dispatch_small_body(const int32_t* ids, const WT
   __syncthreads();
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
-  for (int base = 0; base < A; base += kThreads) {
-    const int a = base + tid;
-    int id = -1;
-    if (a < A) {
-      id = ids[a];
-      if (id < 0 || id >= E) id = -1;
-    }
-    const bool valid = id >= 0;
-    unsigned long long peers = __ballot(valid);  // lanes of this wave holding the same expert id
-    for (int b = 0; b < nbits; ++b) {
-      const bool bit = (id >> b) & 1;
-      const unsigned long long m = __ballot(valid && bit);
-      peers &= bit ? m : ~m;
-    }
-    const int rank = __popcll(peers & ((1ull << lane) - 1ull));
-    if (valid && rank == 0) wavehist[wave * E + id] = __popcll(peers);
-    __syncthreads();
-    if (valid) {
-      int pos = cursor[id] + rank;
-      for (int w = 0; w < wave; ++w) pos += wavehist[w * E + id];
-      inverse[a] = pos;
-      source_order[pos] = a;
-    } else if (a < A) {
-      inverse[a] = -1;
-    }
-    if (base + kThreads >= A) break;  // last round: the tables are not needed again
-    __syncthreads();
-    for (int e = tid; e < E; e += kThreads) {
-      int add = 0;
+  for (int base = first; base < end; base += kDispatchBatch * kWave) {
+    int id[kDispatchBatch];
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        add += wavehist[w * E + e];
-        wavehist[w * E + e] = 0;
-      }
-      cursor[e] += add;
+    for (int i = 0; i < kDispatchBatch; ++i) {
+      const int a = base + i * kWave + lane;
+      id[i] = a < end ? ids[a] : -1;
     }
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kDispatchBatch; ++i) {
+      const int a = base + i * kWave + lane;
+      const bool valid = id[i] >= 0 && id[i] < E;
+      unsigned long long peers = __ballot(valid);  // lanes of this wave holding the same expert id
+      for (int b = 0; b < nbits; ++b) {
+        const bool bit = (id[i] >> b) & 1;
+        const unsigned long long m = __ballot(valid && bit);
+        peers &= bit ? m : ~m;
+      }
+      const int rank = __popcll(peers & ((1ull << lane) - 1ull));
+      if (valid) {
+        const int pos = mine[id[i]] + rank;
+        inverse[a] = pos;
+        source_order[pos] = a;
+      } else if (a < end) {
+        inverse[a] = -1;
+      }
+      if (base + (i + 1) * kWave >= end) break;
+      // (the table is the wave's own, and its LDS accesses are done in order)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (valid && rank == 0) mine[id[i]] += __popcll(peers);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
   }
 }
 
