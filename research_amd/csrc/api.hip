@@ -667,7 +667,7 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
   // (a timed call keeps the shared experts in launches of their own, so that their stages are theirs)
   const bool offer_shared = Is > 0 && g_stage_timer == nullptr;
   SharedExperts shared{shared_gate, shared_up, shared_down, Is, w.shared_act, w.shared_y, shared_gate_pre,
-                       shared_up_pre, false};
+                       shared_up_pre, I, false, false, false};
   int rc;
   if (decode) {
     rc = launch_decode_gate_up_router(x, w_router, expert_bias, gate, up, w.act, T, H, E, K, I, route_scale,
@@ -691,7 +691,7 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
     stage_mark(kStageRouter, main_stream);
     rc = dispatch_for_layer(expert_ids, weights, (T > 0 && !gather) ? x : nullptr, T, H, E, K, dtype, group_sizes,
                             offsets, source_order, inverse, w.packed_x, expert_counts, importance, w.dispatch,
-                            !stats_done, plan_done, main_stream);
+                            !stats_done, plan_done, main_stream, x, offer_shared && gather ? &shared : nullptr);
   }
   if (rc) return rc;
   if (!decode) {  // (the decode path has enqueued both of its GEMM launches above)

@@ -116,21 +116,26 @@ void launch_dispatch_rows(const void* x, const int32_t* inverse, int64_t T, int6
 // dispatch.hip: the dispatch as the layer runs it.  want_stats (weights of element type = dtype): the
 // histogram pass also sums the route weights per expert, and expert_counts / importance get the
 // statistics that the router left out (router_for_layer).  The workspace holds
-// dispatch_layer_workspace_bytes(T*K, E) bytes.  plan_done: only the row scatter is left to do.
+// dispatch_layer_workspace_bytes(T*K, E) bytes.  plan_done: only the row scatter is left to do.  shared: experts of
+// which a product of the rows shared_x may run beside it.
+struct SharedExperts;
 size_t dispatch_layer_workspace_bytes(int64_t A, int64_t E);
 int dispatch_for_layer(const int32_t* expert_ids, const void* weights, const void* x, int64_t T, int64_t H, int64_t E,
                        int64_t K, int dtype, int32_t* group_sizes, int32_t* offsets, int32_t* source_order,
                        int32_t* inverse, void* packed_x, float* expert_counts, float* importance, void* workspace,
-                       bool want_stats, bool plan_done, hipStream_t stream);
+                       bool want_stats, bool plan_done, hipStream_t stream, const void* shared_x = nullptr,
+                       SharedExperts* shared = nullptr);
 
 // The shared experts of a layer call.  A router of a few tokens takes their gate/up product along in its launch (and sets
-// gate_up_done), the routed products then the down one: neither needs the other's results.
-// gate_pre / up_pre: where a training forward keeps the two rounded products, or null.
+// gate_up_done and few_rows), the routed products then the down one: neither needs the other's results.  With more tokens
+// the finishing launch of the router takes the one and the dispatch the other (down_done), or the dispatch the first.
+// gate_pre / up_pre: where a training forward keeps the two rounded products, or null.  routed_I: the routed experts' width.
 struct SharedExperts {
   const void *gate, *up, *down;
   int64_t Is;
   void *act, *y, *gate_pre, *up_pre;
-  bool gate_up_done;
+  int64_t routed_I;
+  bool gate_up_done, few_rows, down_done;
 };
 
 // router.hip: the router as the layer runs it, with the dispatch plan behind it where that is free.
@@ -157,6 +162,13 @@ int launch_swiglu_gather(const void* x, const int32_t* source_order, const void*
                          const void* down, const int32_t* group_sizes, const int32_t* offsets, int64_t T, int64_t K,
                          int64_t H, int64_t I, int64_t E, int dtype, void* act, void* packed_y, hipStream_t stream,
                          const SharedExperts* shared = nullptr, void* gate_pre = nullptr, void* up_pre = nullptr);
+
+// grouped_gemm.hip: the dispatch plan and its statistics (bf16 weights) in one workgroup with a product of the shared
+// experts beside it, where there is one that fits (*taken).
+int launch_dispatch_beside_shared(const int32_t* ids, const void* weights, const void* x, int64_t T, int64_t H, int64_t E,
+                                  int64_t K, int32_t* group_sizes, int32_t* offsets, int32_t* source_order,
+                                  int32_t* inverse, float* counts, float* importance, SharedExperts& shared, bool* taken,
+                                  hipStream_t stream);
 
 // The decode path of the layer (a handful of tokens, nearly every expert chosen by some token).  A tile is
 // 64 rows tall whether it holds an expert's few routed rows or all T <= 64 tokens, so ONE launch runs every

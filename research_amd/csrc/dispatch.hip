@@ -548,13 +548,18 @@ size_t dispatch_layer_workspace_bytes(int64_t A, int64_t E) {
 int dispatch_for_layer(const int32_t* expert_ids, const void* weights, const void* x, int64_t T, int64_t H, int64_t E,
                        int64_t K, int dtype, int32_t* group_sizes, int32_t* offsets, int32_t* source_order,
                        int32_t* inverse, void* packed_x, float* expert_counts, float* importance, void* workspace,
-                       bool want_stats, bool plan_done, hipStream_t s) {
-  const int rc = dispatch_validate("dispatch", expert_ids, x, T, H, E, K, dtype, group_sizes, offsets, source_order,
+                       bool want_stats, bool plan_done, hipStream_t s, const void* shared_x, SharedExperts* shared) {
+  int rc = dispatch_validate("dispatch", expert_ids, x, T, H, E, K, dtype, group_sizes, offsets, source_order,
                                    inverse, packed_x);
   if (rc) return rc;
   JT_REQUIRE(workspace != nullptr, "dispatch: null pointer argument");
   JT_REQUIRE(!want_stats || (expert_counts && importance && (weights || T == 0)), "dispatch: null pointer argument");
-  if (plan_done) {  // the router's finishing workgroup has written the plan
+  if (!plan_done && want_stats && shared && dtype == JTMOE_BF16 && T > 0 && T * K <= kSmallLayerAssignments) {
+    rc = launch_dispatch_beside_shared(expert_ids, weights, shared_x, T, H, E, K, group_sizes, offsets, source_order, inverse,
+                                       expert_counts, importance, *shared, &plan_done, s);
+    if (rc) return rc;
+  }
+  if (plan_done) {  // ... or the router's finishing workgroup has written the plan
     stage_mark(kStageDispatchMeta, s);
     if (x != nullptr && T > 0) launch_dispatch_rows(x, inverse, T, K, H, dtype, packed_x, s);
     stage_mark(kStageDispatchRows, s);

@@ -10,6 +10,7 @@
 // are accumulated in fp32 on the matrix cores (v_mfma_f32_32x32x16_bf16 for
 // bf16, v_mfma_f32_32x32x2_f32 for fp32).
 #include "common.hpp"
+#include "dispatch_small.hpp"
 #include "gemm_launch.hpp"
 #include "grouped_gemm_dma.hpp"
 #include "grouped_gemm_skinny.hpp"
@@ -564,9 +565,9 @@ ProductKernel joint_down_of(const RoutedProblem& p, const RoutedProblem& s) {
 // activations are then read while the caches hold them (800 and 1300 tokens, 64 experts top-8: 1.5 % of a call).
 template <typename T>
 int launch_with_shared(const RoutedProblem& gu, const RoutedProblem& dn, const RoutedProblem& sgu,
-                       const RoutedProblem& sdn, hipStream_t stream) {
-  const ProductKernel jg = Elem<T>::is_bf16 ? joint_gate_up_of(gu, sgu) : ProductKernel::kGeneral;
-  const ProductKernel jd = Elem<T>::is_bf16 ? joint_down_of(dn, sdn) : ProductKernel::kGeneral;
+                       const RoutedProblem& sdn, hipStream_t stream, bool gate_up_done, bool down_done) {
+  const ProductKernel jg = Elem<T>::is_bf16 && !gate_up_done ? joint_gate_up_of(gu, sgu) : ProductKernel::kGeneral;
+  const ProductKernel jd = Elem<T>::is_bf16 && !down_done ? joint_down_of(dn, sdn) : ProductKernel::kGeneral;
   const bool joint_gu = jg != ProductKernel::kGeneral, joint_dn = jd != ProductKernel::kGeneral;
   const DenseProblem dgu = dense_problem(sgu), ddn = dense_problem(sdn);
   auto gate_up = [&](auto cfg) { return launch_joint<decltype(cfg)>(gu, dgu, stream); };
@@ -582,7 +583,7 @@ int launch_with_shared(const RoutedProblem& gu, const RoutedProblem& dn, const R
       rc = with_gate_up_tiles<true, true>(tiles_of(jg == ProductKernel::kHalfTail, true, gu.rows, gu.K, gu.N, gu.E, false, &dgu), gate_up);
       break;
   }
-  if (!rc && !joint_gu && joint_dn) rc = launch_gate_up<T>(sgu, stream);
+  if (!rc && !gate_up_done && !joint_gu && joint_dn) rc = launch_gate_up<T>(sgu, stream);
   if (rc) return rc;
   switch (jd) {
     case ProductKernel::kGeneral: rc = launch_down<T>(dn, stream); break;
@@ -598,8 +599,8 @@ int launch_with_shared(const RoutedProblem& gu, const RoutedProblem& dn, const R
       break;
     }
   }
-  if (!rc && !joint_gu && !joint_dn) rc = launch_gate_up<T>(sgu, stream);
-  if (!rc && !joint_dn) rc = launch_down<T>(sdn, stream);
+  if (!rc && !gate_up_done && !joint_gu && !joint_dn) rc = launch_gate_up<T>(sgu, stream);
+  if (!rc && !down_done && !joint_dn) rc = launch_down<T>(sdn, stream);
   return rc;
 }
 
@@ -618,7 +619,7 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
                             nullptr, x_rows, H, shared->Is, 1, 0, 1};
     const RoutedProblem sdn{shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, nullptr, nullptr, nullptr,
                             x_rows, shared->Is, H, 1, 0, 1};
-    if (shared->gate_up_done) {
+    if (shared->few_rows) {
       // (a few tokens: the router has run the shared gate/up product, its down product goes beside the routed gate/up)
       const SkinnyProblem down_p = dense_skinny(shared->act, shared->down, nullptr, shared->y, nullptr, nullptr, x_rows,
                                                 shared->Is, H, BesideCfg::BM, BesideCfg::BN);
@@ -629,7 +630,7 @@ int launch_pair(const void* x, const void* gate, const void* up, const void* dow
       if (!rc && !taken) rc = launch_down<T>(sdn, stream);
       return rc ? rc : check_launch("grouped gemm");
     }
-    rc = launch_with_shared<T>(gu, dn, sgu, sdn, stream);
+    rc = launch_with_shared<T>(gu, dn, sgu, sdn, stream, shared->gate_up_done, shared->down_done);
     return rc ? rc : check_launch("grouped gemm");
   }
   rc = launch_gate_up<T>(gu, stream);
@@ -673,6 +674,97 @@ bool shared_in_skinny_tiles(const void* x, const SharedExperts& s, int64_t T, in
          aligned16(s.gate_pre) && aligned16(s.up_pre) &&
          gate_up_kernel(T, H, s.Is, 1, true, persistent_grid_size()) == ProductKernel::kStream16x64 &&
          down_kernel(T, H, s.Is, 1, true, persistent_grid_size()) == ProductKernel::kStream16x64;
+}
+
+// ---- products of the shared experts beside the small launches in front of the routed ones ----
+// Both take tiles that find a CU each; they run on as they would alone, and the launch beside them, a few workgroups and
+// 7 to 12 us, costs nothing.  Sizes whose products are parts of the routed launches (joint_gate_up, joint_down) stay there.
+namespace {
+
+SharedTiles beside_front(const RoutedProblem& s, bool dual, bool half, int front) {
+  const TileShape tiles = tiles_of(half, dual, s.rows, s.K, s.N, 1, true);
+  if (tiles != TileShape::k64x64 && tiles != TileShape::k128x64) return SharedTiles{};
+  const int BM = tiles == TileShape::k64x64 ? 64 : 128;
+  SharedTiles t{tiles, dense_problem(s), 0};
+  t.p.ntiles = (int)((s.N + 63) / 64);
+  const int64_t grid = gemm_grid((s.rows + BM - 1) / BM, t.p.ntiles);
+  if (front + grid <= persistent_grid_size()) t.grid = (int)grid;
+  return t;
+}
+
+struct DispatchPlan {
+  const int32_t* ids;
+  const bf16_raw* weights;
+  int A, E;
+  int32_t *group_sizes, *offsets, *source_order, *inverse;
+  float *counts, *importance;
+};
+constexpr int kDispatchFront = 8;
+
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) void dispatch_beside_kernel(DispatchPlan d, DenseProblem shared) {
+  static_assert(JTMOE_MAX_EXPERTS <= Cfg::NT, "an expert per thread of the dispatch");
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  if ((int)blockIdx.x >= kDispatchFront)
+    dense_stream_tiles<Cfg>(shared, kDispatchFront);
+  else if (blockIdx.x == 0)
+    dispatch_small_body<Cfg::NT, true, bf16_raw>(d.ids, d.weights, d.A, d.E, d.group_sizes, d.offsets, d.source_order,
+                                                 d.inverse, d.counts, d.importance, smem_raw);
+}
+
+}  // namespace
+
+SharedTiles shared_gate_up_beside(const void* x, const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front) {
+  const double cus = persistent_grid_size();
+  const ProductKernel k = gate_up_kernel(T, H, s.Is, 1, true, cus);
+  if ((k != ProductKernel::kHalf && k != ProductKernel::kRows256) || !fast_ok(x, s.gate, s.up, s.act, H, s.Is) ||
+      !aligned16(s.gate_pre) || !aligned16(s.up_pre) ||
+      joint_gate_up(T * K, H, s.routed_I, E, T, s.Is, cus) != ProductKernel::kGeneral)
+    return SharedTiles{};
+  return beside_front({x, s.gate, s.up, s.act, s.gate_pre, s.up_pre, nullptr, nullptr, nullptr, T, H, s.Is, 1, 0, 1}, true,
+                      k == ProductKernel::kHalf, front);
+}
+
+SharedTiles shared_down_beside(const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front) {
+  const double cus = persistent_grid_size();
+  const ProductKernel k = down_kernel(T, H, s.Is, 1, true, cus);
+  if ((k != ProductKernel::kHalf && k != ProductKernel::kRows256 && k != ProductKernel::kRows256Tail) ||
+      !fast_ok(s.act, s.down, nullptr, s.y, s.Is, H) || !stream_ok<DownStreamTailCfg>(T, s.Is, H, nullptr, 1) ||
+      joint_down(T * K, H, s.routed_I, E, T, s.Is, cus) != ProductKernel::kGeneral)
+    return SharedTiles{};
+  return beside_front({s.act, s.down, nullptr, s.y, nullptr, nullptr, nullptr, nullptr, nullptr, T, s.Is, H, 1, 0, 1}, false,
+                      k == ProductKernel::kHalf, front);
+}
+
+int launch_dispatch_beside_shared(const int32_t* ids, const void* weights, const void* x, int64_t T, int64_t H, int64_t E,
+                                  int64_t K, int32_t* group_sizes, int32_t* offsets, int32_t* source_order,
+                                  int32_t* inverse, float* counts, float* importance, SharedExperts& shared, bool* taken,
+                                  hipStream_t stream) {
+  const bool down = shared.gate_up_done;
+  const SharedTiles t = down ? shared_down_beside(shared, T, H, E, K, kDispatchFront)
+                             : shared_gate_up_beside(x, shared, T, H, E, K, kDispatchFront);
+  if (t.grid == 0) return JTMOE_OK;
+  const DispatchPlan plan{ids, static_cast<const bf16_raw*>(weights), (int)(T * K), (int)E, group_sizes, offsets,
+                          source_order, inverse, counts, importance};
+  auto launch = [&](auto cfg) {
+    using Cfg = decltype(cfg);
+    const size_t smem = std::max<size_t>(StreamLayout<Cfg>::kSmemBytes, dispatch_small_smem_bytes((int)E, Cfg::NT, true));
+    static std::once_flag once;
+    static hipError_t attr_err = hipSuccess;
+    auto kernel = &dispatch_beside_kernel<Cfg>;
+    std::call_once(once, [&] {
+      attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     160 * 1024);
+    });
+    if (attr_err != hipSuccess) return fail(JTMOE_ELAUNCH, "dispatch: kernel set-up: %s", hipGetErrorString(attr_err));
+    kernel<<<kDispatchFront + t.grid, Cfg::NT, smem, stream>>>(plan, t.p);
+    *taken = true;
+    (down ? shared.down_done : shared.gate_up_done) = true;
+    return check_launch("dispatch and shared experts");
+  };
+  const bool quarter = t.tiles == TileShape::k64x64;
+  if (down) return quarter ? launch(QuarterCfg{}) : launch(NarrowCfg{});
+  return quarter ? launch(GateUpQuarterCfg<false>{}) : launch(GateUpNarrowCfg<false>{});
 }
 
 // ---- the gathering launch pair as the layer uses it (declared in common.hpp) ----

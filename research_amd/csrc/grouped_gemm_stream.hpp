@@ -83,13 +83,14 @@ __host__ __device__ inline int joint_tile(int w, int W, int p, int n1, int n0, i
 //              lives in LDS in the same swizzled row layout and is read with ds_read_b128; the k loop
 //              runs through the segments one after the other.
 // kJoint: the tiles of `dp` run in the same launch (fully persistent workgroups, chunk 0).
+// first_block: the launch's workgroups in front of these (a multiple of 8: a tile's XCD stays the same).
 template <typename Cfg, bool kNT, bool kJoint = false>
 __device__ __forceinline__ void stream_gemm_body(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes,
     const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int ntiles_n,
     const int32_t* __restrict__ row_map, int row_div, int a_rows, uint16_t* __restrict__ save0,
-    uint16_t* __restrict__ save1, int segs, int window, int chunk, const DenseProblem& dp) {
+    uint16_t* __restrict__ save1, int segs, int window, int chunk, const DenseProblem& dp, int first_block = 0) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, NS = Cfg::NSTAGE;
   constexpr int TM = Cfg::TM, TN = Cfg::TN, WN = Cfg::WN;
   constexpr int CPRA = Cfg::CPRA, KK = BK / 16, LPS = Cfg::LPS;
@@ -152,7 +153,7 @@ __device__ __forceinline__ void stream_gemm_body(
   // which they are the cheaper work.
   int extra = 0, real_mtiles = mtiles_with(0), dense_mtiles = kJoint ? group_mtiles(dp.rows, BM, 0) : 0;
   if (X != 0) {
-    const int workgroups = chunk > 0 ? 8 * window : (int)gridDim.x;
+    const int workgroups = chunk > 0 ? 8 * window : (int)gridDim.x - first_block;
     auto rounds = [&](int mt, int dense_mt) {
       return (mt * ntiles_n + (kJoint ? dense_mt * dp.ntiles * lead : 0) + workgroups - 1) / workgroups;
     };
@@ -167,7 +168,7 @@ __device__ __forceinline__ void stream_gemm_body(
   const int total = real_mtiles * ntiles_n;
   const int per_xcd = (total + 7) >> 3;
   const int xcd = (int)blockIdx.x & 7;
-  int idx = (int)blockIdx.x >> 3, stride = max(1, (int)gridDim.x >> 3), left = 0x7fffffff;
+  int idx = ((int)blockIdx.x - first_block) >> 3, stride = max(1, ((int)gridDim.x - first_block) >> 3), left = 0x7fffffff;
   // kJoint: this XCD's range of either product, the odd tiles of the two at opposite ends of the XCDs
   const int total1 = kJoint ? dense_mtiles * dp.ntiles : 0;
   const int first0 = (xcd * total) >> 3, count0 = (((xcd + 1) * total) >> 3) - first0;
@@ -685,6 +686,23 @@ int with_smaller_tiles(TileShape s, Launch launch) {
     default: return launch(Rows128Cfg{});
   }
 }
+// A product of the shared experts beside the workgroups of a small launch in front of the routed products, each tile on
+// a CU of its own: behind `front` workgroups (a multiple of 8).  grid = 0: not at these sizes and pointers, or not where
+// the product is a part of the routed one's launch.  (grouped_gemm.hip; the tiles are 64 x 64 or 128 x 64.)
+struct SharedTiles {
+  TileShape tiles;
+  DenseProblem p;
+  int grid;
+};
+SharedTiles shared_gate_up_beside(const void* x, const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front);
+SharedTiles shared_down_beside(const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front);
+
+template <typename Cfg>
+__device__ __forceinline__ void dense_stream_tiles(const DenseProblem& p, int front) {
+  stream_gemm_body<Cfg, false>(p.a0, nullptr, p.b0, p.b1, p.c, nullptr, nullptr, 1, p.rows, p.k, p.n, p.ntiles, nullptr, 1,
+                               0, p.save0, p.save1, 1, 0, 0, DenseProblem{}, front);
+}
+
 inline bool large_tiles(TileShape s) { return s == TileShape::kTall || s == TileShape::kPlain; }
 
 }  // namespace jtmoe

@@ -14,6 +14,7 @@
 #include "dispatch_small.hpp"
 #include "grouped_gemm_dma.hpp"
 #include "grouped_gemm_skinny.hpp"
+#include "grouped_gemm_stream.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -991,20 +992,39 @@ __global__ __launch_bounds__(4 * kTok) void router_finish_kernel(
 
 // Second half of a middle-sized layer call: a workgroup per 16 tokens adds up their slices and runs the epilogue
 // (the statistics and the plan are the dispatch's).
-template <int kTok, int kThreads>
-__global__ __launch_bounds__(kThreads) void router_finish_blocks_kernel(
-    const float* __restrict__ partial, int slices, const float* __restrict__ bias, int tokens, int E, int K,
-    float route_scale, int32_t* __restrict__ ids, bf16_raw* __restrict__ weights, float* __restrict__ scores,
-    int score_func) {
+struct FinishBlocks {
+  const float *partial, *bias;
+  int slices, tokens, E, K, score_func;
+  float route_scale;
+  int32_t* ids;
+  bf16_raw* weights;
+  float* scores;
+};
+constexpr int kFinishBlockTokens = 16, kFinishBlockThreads = 256;
+__device__ __forceinline__ void router_finish_block(const FinishBlocks& f) {
+  constexpr int kTok = kFinishBlockTokens, kThreads = kFinishBlockThreads;
+  const int tokens = f.tokens, E = f.E, K = f.K;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   RouterSmem sm = router_smem(smem_raw, E, K, kTok);
   const int t0 = (int)blockIdx.x * kTok;
-  router_clear(sm, bias, E, kThreads);
-  add_slices<kThreads>(sm, partial + (size_t)t0 * E, slices, (size_t)tokens * E, min(kTok, tokens - t0), E, score_func,
-                       nullptr, scores + (size_t)t0 * E);
+  router_clear(sm, f.bias, E, kThreads);
+  add_slices<kThreads>(sm, f.partial + (size_t)t0 * E, f.slices, (size_t)tokens * E, min(kTok, tokens - t0), E,
+                       f.score_func, nullptr, f.scores + (size_t)t0 * E);
   __syncthreads();
-  router_epilogue<bf16_raw, kTok, kThreads, true>(sm, bias, t0, tokens, E, K, route_scale, ids, weights, scores, nullptr,
-                                                  RouterScratch{}, score_func);
+  router_epilogue<bf16_raw, kTok, kThreads, true>(sm, f.bias, t0, tokens, E, K, f.route_scale, f.ids, f.weights, f.scores,
+                                                  nullptr, RouterScratch{}, f.score_func);
+}
+__global__ __launch_bounds__(kFinishBlockThreads) void router_finish_blocks_kernel(FinishBlocks f) { router_finish_block(f); }
+
+// ... with the shared experts' gate/up tiles beside: the first `front` workgroups (a multiple of 8) are the router's.
+// The routed rows' 12 us of selection leave most CUs idle, and the tiles, a CU each, need nothing of it.
+template <typename Cfg>
+__global__ __launch_bounds__(Cfg::NT) void router_finish_blocks_beside_kernel(FinishBlocks f, DenseProblem shared, int front) {
+  static_assert(Cfg::NT == kFinishBlockThreads, "one workgroup size for both");
+  if ((int)blockIdx.x >= front)
+    dense_stream_tiles<Cfg>(shared, front);
+  else if ((int)blockIdx.x * kFinishBlockTokens < f.tokens)
+    router_finish_block(f);
 }
 
 // ---------------------------------------------------------------------------
@@ -1378,7 +1398,31 @@ struct LayerPlan {
   bool plan_done;
   void* scratch;  // memory of the layer that nothing uses until the router is done
   size_t scratch_bytes;
+  SharedExperts* shared;  // whose gate/up product may run beside the finishing launch, or null
 };
+
+// (the launch's LDS is the larger one's, and one of its workgroups fills a CU either way)
+int launch_finish_blocks(const FinishBlocks& f, const void* x, int64_t H, SharedExperts* shared, hipStream_t stream) {
+  const size_t smem = router_smem_bytes(f.E, f.K, kFinishBlockTokens);
+  const int blocks = (f.tokens + kFinishBlockTokens - 1) / kFinishBlockTokens, front = (blocks + 7) / 8 * 8;
+  const SharedTiles tiles = shared ? shared_gate_up_beside(x, *shared, f.tokens, H, f.E, f.K, front) : SharedTiles{};
+  auto beside = [&](auto cfg) {
+    using Cfg = decltype(cfg);
+    const size_t both = std::max<size_t>(smem, StreamLayout<Cfg>::kSmemBytes);
+    auto kernel = &router_finish_blocks_beside_kernel<Cfg>;
+    const int rc = set_max_smem(kernel, both);
+    if (rc) return rc;
+    kernel<<<front + tiles.grid, Cfg::NT, both, stream>>>(f, tiles.p, front);
+    shared->gate_up_done = true;
+    return check_launch("router and shared experts");
+  };
+  if (tiles.grid > 0 && tiles.tiles == TileShape::k64x64) return beside(GateUpQuarterCfg<false>{});
+  if (tiles.grid > 0) return beside(GateUpNarrowCfg<false>{});
+  const int rc = set_max_smem(&router_finish_blocks_kernel, smem);
+  if (rc) return rc;
+  router_finish_blocks_kernel<<<blocks, kFinishBlockThreads, smem, stream>>>(f);
+  return check_launch("router");
+}
 
 // bf16 routers whose experts and columns are multiples of 8 run on the matrix cores: those that fill the tiles with bf16
 // products in slices of k, the others (router_chained) as one chain in fp32.  The staged kernel takes what is left.
@@ -1473,13 +1517,8 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
         }
 #undef JT_PARTIAL_CASE
         if (layer && tokens * E >= kFinishInBlocks) {
-          const size_t bsmem = router_smem_bytes((int)E, (int)K, 16);
-          auto finish = router_finish_blocks_kernel<16, 256>;
-          const int rc = set_max_smem(finish, bsmem);
-          if (rc) return rc;
-          finish<<<blocks, 256, bsmem, stream>>>(partial, slices, bias, (int)tokens, (int)E, (int)K, (float)route_scale,
-                                                 ids, static_cast<bf16_raw*>(weights), scores, score_func);
-          return check_launch("router");
+          return launch_finish_blocks({partial, bias, slices, (int)tokens, (int)E, (int)K, score_func, (float)route_scale, ids,
+                                       static_cast<bf16_raw*>(weights), scores}, x, H, layer->shared, stream);
         }
         const size_t fsmem = router_smem_bytes((int)E, (int)K, finish_tok);
         const bool plan = layer != nullptr && tokens * K <= kSmallMaxAssignments && E <= 4 * finish_tok;
@@ -1549,8 +1588,7 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
     if (layer && tokens <= kMidMaxTokens && H % kSplitKC == 0 && H >= 1024 &&
         (size_t)slices * tokens * E * sizeof(float) <= layer->scratch_bytes) {
       const size_t smem = (size_t)2 * kSplitKC * router_w_stride((int)E) * 2;
-      const size_t fsmem = router_smem_bytes((int)E, (int)K, 16);
-      if (fsmem <= 160 * 1024) {
+      if (router_smem_bytes((int)E, (int)K, kFinishBlockTokens) <= 160 * 1024) {
         float* const partial = static_cast<float*>(layer->scratch);
         const int blocks = (int)((tokens + 15) / 16);
 #define JT_PARTIAL_CASE(NB)                                                                                  \
@@ -1571,12 +1609,8 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
           JT_PARTIAL_CASE(16)
         }
 #undef JT_PARTIAL_CASE
-        auto finish = router_finish_blocks_kernel<16, 256>;
-        const int rc = set_max_smem(finish, fsmem);
-        if (rc) return rc;
-        finish<<<blocks, 256, fsmem, stream>>>(partial, slices, bias, (int)tokens, (int)E, (int)K, (float)route_scale,
-                                               ids, static_cast<bf16_raw*>(weights), scores, score_func);
-        return check_launch("router");
+        return launch_finish_blocks({partial, bias, slices, (int)tokens, (int)E, (int)K, score_func, (float)route_scale, ids,
+                                     static_cast<bf16_raw*>(weights), scores}, x, H, layer->shared, stream);
       }
     }
     // four waves (64 tokens) per workgroup: the waves share the work of bringing in the router
@@ -1709,7 +1743,7 @@ int launch_decode_gate_up_router(const void* x, const void* w_router, const floa
     shared_gu = dense_skinny(x, shared->gate, shared->up, shared->act, shared->gate_pre, shared->up_pre, T, H, shared->Is,
                              SharedGateUpCfg::BM, SharedGateUpCfg::BN);
     shared_blocks = gemm_grid(shared_gu.mtiles, shared_gu.ntiles_n);
-    shared->gate_up_done = true;
+    shared->gate_up_done = shared->few_rows = true;
   }
   const int64_t grid = (int64_t)token_blocks * slices + shared_blocks + gemm_grid(mtiles, nt);
   if (token_blocks * slices > 255) return fail(JTMOE_EUNSUPPORTED, "moe_forward: decode launch with %d router workgroups", token_blocks * slices);
@@ -1789,7 +1823,7 @@ static int launch_router_with_shared(const void* x, const void* w_router, const 
     JT_SHARED_CASE(16)
   }
 #undef JT_SHARED_CASE
-  sh.gate_up_done = true;
+  sh.gate_up_done = sh.few_rows = true;
   return check_launch("router and shared experts");
 }
 
@@ -1807,7 +1841,7 @@ int router_for_layer(const void* x, const void* w_router, const float* expert_bi
   JT_REQUIRE(group_sizes && offsets && (T == 0 || (source_order && inverse)), "router: null pointer argument");
   if (workspace_bytes < jtmoe_router_workspace_bytes(E))
     return fail(JTMOE_EWORKSPACE, "router: workspace %zu < %zu bytes", workspace_bytes, jtmoe_router_workspace_bytes(E));
-  LayerPlan layer{group_sizes, offsets, source_order, inverse, false, false, scratch, scratch_bytes};
+  LayerPlan layer{group_sizes, offsets, source_order, inverse, false, false, scratch, scratch_bytes, shared};
   if (shared && router_takes_shared(x, w_router, *shared, T, H, E, K, dtype)) {
     *stats_done = *plan_done = true;
     return launch_router_with_shared(x, w_router, expert_bias, *shared, T, H, E, K, route_scale, score_func, expert_ids,
