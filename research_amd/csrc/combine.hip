@@ -43,9 +43,9 @@ __device__ __forceinline__ uint4 pack8_hw(const float* f) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// bf16, rows a multiple of 8 elements, 16-byte aligned.  One wave per token; a lane owns NV
-// 16-byte vectors of the row and requests them from all K source rows before it starts adding,
-// so K*NV independent loads are in flight per lane.  KT = K when K is one of the unrolled
+// bf16, rows a multiple of 8 elements, 16-byte aligned.  One wave per token (or per part of its row, kSplit);
+// a lane owns NV 16-byte vectors of the row and requests them from the K source rows before it starts
+// adding, as many as the compiler leaves registers for.  KT = K when K is one of the unrolled
 // values, 0 for a run-time loop.
 __device__ __forceinline__ float wave_sum_f32(float v) {
 #pragma unroll
@@ -53,8 +53,11 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
   return v;
 }
 
-template <int NV, int KT, bool kNorm>
-__global__ __launch_bounds__(256) void combine_bf16_vec_kernel(const uint4* __restrict__ packed_y,
+// kSplit (NV = 1): a workgroup per token, a wave per 64 vectors of its row; the norm's squares are then added up by every
+// wave, in the same order, from LDS.
+constexpr int kMaxRowWaves = 8;
+template <int NV, int KT, bool kNorm, bool kSplit>
+__global__ __launch_bounds__(kSplit ? 64 * kMaxRowWaves : 256) void combine_bf16_vec_kernel(const uint4* __restrict__ packed_y,
                                                                const int32_t* __restrict__ inverse,
                                                                const uint16_t* __restrict__ weights,
                                                                const uint4* __restrict__ shared_y, int tokens, int K,
@@ -62,9 +65,10 @@ __global__ __launch_bounds__(256) void combine_bf16_vec_kernel(const uint4* __re
                                                                const uint4* __restrict__ residual,
                                                                const float* __restrict__ post_scale, float eps) {
 #pragma clang fp contract(off)
-  const int t = blockIdx.x * blockDim.y + threadIdx.y;
+  static_assert(!kSplit || NV == 1, "a vector per lane");
+  const int t = kSplit ? blockIdx.x : blockIdx.x * blockDim.y + threadIdx.y;
   if (t >= tokens) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x, first = lane + (kSplit ? threadIdx.y * 64 : 0);
   float acc[NV][8];
 #pragma unroll
   for (int j = 0; j < NV; ++j)
@@ -98,7 +102,7 @@ __global__ __launch_bounds__(256) void combine_bf16_vec_kernel(const uint4* __re
       const bool ok = pos[s] >= 0 && pos[s] < A;
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const int v = lane + j * 64;
+        const int v = first + j * 64;
         rows[s][j] = (ok && v < row_vecs) ? load_stream(&packed_y[(size_t)pos[s] * row_vecs + v]) : make_uint4(0, 0, 0, 0);
       }
     }
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(256) void combine_bf16_vec_kernel(const uint4* __re
       uint4 r[NV];
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const int v = lane + j * 64;
+        const int v = first + j * 64;
         r[j] = v < row_vecs ? load_stream(&packed_y[(size_t)pos * row_vecs + v]) : make_uint4(0, 0, 0, 0);
       }
       add_row(r, w);
@@ -121,7 +125,7 @@ __global__ __launch_bounds__(256) void combine_bf16_vec_kernel(const uint4* __re
   float ss = 0.0f;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const int v = lane + j * 64;
+    const int v = first + j * 64;
     if (v >= row_vecs) continue;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[j][i] = round_bf16_hw(acc[j][i]);
@@ -137,16 +141,27 @@ __global__ __launch_bounds__(256) void combine_bf16_vec_kernel(const uint4* __re
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         acc[j][i] = round_bf16_hw(acc[j][i]);
-        ss += acc[j][i] * acc[j][i];
+        if (!kSplit) ss += acc[j][i] * acc[j][i];
       }
     }
   }
   if (kNorm) {
+    if (kSplit) {
+      __shared__ uint4 row[kMaxRowWaves][64];
+      row[threadIdx.y][lane] = first < row_vecs ? pack8_hw(acc[0]) : make_uint4(0, 0, 0, 0);
+      __syncthreads();
+      for (int p = 0; p < (int)blockDim.y; ++p) {
+        float f[8];
+        unpack8(row[p][lane], f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += f[i] * f[i];
+      }
+    }
     ss = wave_sum_f32(ss);
     const float inv = 1.0f / sqrtf(ss / (float)(row_vecs * 8) + eps);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int v = lane + j * 64;
+      const int v = first + j * 64;
       if (v >= row_vecs) continue;
       float r[8];
       unpack8(load_stream(&residual[(size_t)t * row_vecs + v]), r);
@@ -244,6 +259,13 @@ using namespace jtmoe;
 namespace jtmoe {
 namespace {
 
+// A wave per 64 vectors of a row (kSplit) while that is at most two rounds of the 8192 waves the chip holds: until then
+// latency and the CUs in use bound the kernel.  us, a wave per row / split; 2048 wide, top-8: 1 token 6.2 / 4.0, 37 5.8 /
+// 4.2, 387 with the norm 10.8 / 6.6, 2048 with the norm 23.5 / 17.4, 4096 27.0 / 25.4 and 30.6 / 28.2 with the norm; beyond,
+// at the memory's rate, either way within 4 %: 8192 tokens 54.0 / 53.7, of top-4 28.0 / 28.8, 4096 of 4096 columns 49.2 / 51.8,
+// 16384 of 1024 columns top-2 17.0 / 17.7.
+constexpr int64_t kSplitMaxWaves = 16384;
+
 // residual == nullptr: plain combine; otherwise the fused post-norm + residual variant
 int combine_launch(const char* what, const void* packed_y, const int32_t* inverse, const void* weights,
                    const void* shared_y, const void* residual, const float* post_scale, double eps, int64_t T,
@@ -265,19 +287,24 @@ int combine_launch(const char* what, const void* packed_y, const int32_t* invers
                    (!norm || (aligned16(residual) && aligned16(post_scale)));
   if (vec) {
     const int row_vecs = (int)(H / 8);
-    dim3 block(64, 4);
-    const int grid = (int)((T + block.y - 1) / block.y);
     const int nv = (row_vecs + 63) / 64;
-#define JT_COMBINE_N(NV, KT, NORM)                                                                          \
-  combine_bf16_vec_kernel<NV, KT, NORM><<<grid, block, 0, s>>>(                                             \
+    const bool split = nv > 1 && T * nv <= kSplitMaxWaves;
+    const dim3 block(64, split ? nv : 4);
+    const int grid = (int)(split ? T : (T + 3) / 4);
+#define JT_COMBINE_N(NV, KT, NORM, SPLIT)                                                                   \
+  combine_bf16_vec_kernel<NV, KT, NORM, SPLIT><<<grid, block, 0, s>>>(                                             \
       static_cast<const uint4*>(packed_y), inverse, static_cast<const uint16_t*>(weights),                   \
       static_cast<const uint4*>(shared_y), (int)T, (int)K, A, row_vecs, static_cast<uint4*>(y),              \
       static_cast<const uint4*>(residual), post_scale, epsf)
-#define JT_COMBINE(NV, KT)       \
-  if (norm)                      \
-    JT_COMBINE_N(NV, KT, true);  \
-  else                           \
-    JT_COMBINE_N(NV, KT, false)
+#define JT_COMBINE(NV, KT)                    \
+  if (split && norm)                          \
+    JT_COMBINE_N(1, KT, true, true);          \
+  else if (split)                             \
+    JT_COMBINE_N(1, KT, false, true);         \
+  else if (norm)                              \
+    JT_COMBINE_N(NV, KT, true, false);        \
+  else                                        \
+    JT_COMBINE_N(NV, KT, false, false)
 #define JT_COMBINE_K(NV)      \
   if (K == 8) {               \
     JT_COMBINE(NV, 8);        \
@@ -292,6 +319,8 @@ int combine_launch(const char* what, const void* packed_y, const int32_t* invers
       JT_COMBINE_K(2);
     } else if (nv <= 4) {
       JT_COMBINE_K(4);
+    } else if (split) {
+      JT_COMBINE_K(1);
     } else {
       JT_COMBINE(8, 0);
     }
