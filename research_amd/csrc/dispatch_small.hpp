@@ -3,7 +3,7 @@
 // rows).  Same results as the three-pass plan of dispatch.hip (local_dispatch of the reference at ep_size == 1,
 // moe.py:583-602).
 //
-// Latency bounds it.  A wave owns a run of consecutive assignments, so that the waves meet three times in all,
+// Latency bounds it.  A wave owns a run of consecutive assignments, so that the waves meet four times in all,
 // whatever the number of assignments, and the ids arrive kDispatchBatch loads at a time.  (In rounds of the whole
 // workgroup, with two meetings and a load each, 3096 assignments to 64 experts with statistics took 11.0 us, now 7.1;
 // without them 4.4 us at 320, 6.4 at 4096, 9.7 at 8192.)
