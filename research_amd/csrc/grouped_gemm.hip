@@ -239,6 +239,7 @@ int launch_stream(const void* a, const void* b0, const void* b1, void* c, const 
   if (attr_err != hipSuccess)
     return fail(JTMOE_ELAUNCH, "grouped gemm: kernel set-up: %s", hipGetErrorString(attr_err));
   const bool dense = group_sizes == nullptr;
+  if (!fills_pipeline<Cfg>(Kdim)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: reduction of %lld too short", (long long)Kdim);
   const int64_t mtiles = dense ? (rows + Cfg::BM - 1) / Cfg::BM : max_m_tiles(rows, E, Cfg::BM);
   const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles_grid = gemm_grid(mtiles, nt);
@@ -278,6 +279,8 @@ int launch_joint(const RoutedProblem& r, DenseProblem dp, hipStream_t stream) {
   });
   if (attr_err != hipSuccess)
     return fail(JTMOE_ELAUNCH, "grouped gemm: kernel set-up: %s", hipGetErrorString(attr_err));
+  const int64_t least = std::min<int64_t>(r.K, dp.k);
+  if (!fills_pipeline<Cfg>(least)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: reduction of %lld too short", (long long)least);
   const int64_t mtiles = max_m_tiles(r.rows, r.E, Cfg::BM), nt = (r.N + Cfg::BN - 1) / Cfg::BN;
   dp.ntiles = (dp.n + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles_grid = gemm_grid(mtiles, nt) + gemm_grid((dp.rows + Cfg::BM - 1) / Cfg::BM, dp.ntiles);
@@ -296,7 +299,7 @@ int launch_joint(const RoutedProblem& r, DenseProblem dp, hipStream_t stream) {
 // divisor of at most 32
 template <typename Cfg>
 inline bool stream_ok(int64_t rows, int64_t Kdim, int64_t N, const int32_t* row_map, int row_div) {
-  return ((Cfg::OPT & 65536) != 0 || Kdim % Cfg::BK == 0) && (Kdim + Cfg::BK - 1) / Cfg::BK >= 2 * Cfg::NSTAGE && rows * N * 2 <= (int64_t)0x7ffe0000 &&
+  return ((Cfg::OPT & 65536) != 0 || Kdim % Cfg::BK == 0) && fills_pipeline<Cfg>(Kdim) && rows * N * 2 <= (int64_t)0x7ffe0000 &&
          (row_map == nullptr || (rows < ((int64_t)1 << 27) && row_div >= 1 && row_div <= 32));
 }
 
@@ -416,7 +419,10 @@ ProductKernel joint_gate_up(int64_t rows, int64_t H, int64_t I, int64_t E, int64
     return ProductKernel::kGeneral;
   const bool tail = H % 64 != 0;
   switch (joint_tiles(rows, E, I, T, Is, 1.0, cus, 0.72, /*dual=*/true)) {
-    case HalfTiles::kOnePerCu: return tail ? ProductKernel::kHalfTail : ProductKernel::kHalf;
+    case HalfTiles::kOnePerCu:
+      // (H too short for the half tiles' deeper stages takes four 32-deep ones)
+      if (!stream_ok<GateUpHalfShortCfg<true>>(rows, H, I, row_map, row_div)) return ProductKernel::kGeneral;
+      return tail ? ProductKernel::kHalfTail : ProductKernel::kHalf;
     case HalfTiles::kRounds: return tail ? ProductKernel::kRows256Tail : ProductKernel::kRows256;
     default: return ProductKernel::kGeneral;
   }
@@ -427,7 +433,8 @@ ProductKernel joint_down(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t 
       !stream_ok<DownStreamTailCfg>(rows, I, H, nullptr, 1) || !stream_ok<DownStreamTailCfg>(T, Is, H, nullptr, 1))
     return ProductKernel::kGeneral;
   switch (joint_tiles(rows, E, H, T, H, (double)Is / (double)I, cus, 0.4)) {
-    case HalfTiles::kOnePerCu: return ProductKernel::kHalf;
+    case HalfTiles::kOnePerCu:
+      return stream_ok<HalfShortCfg>(rows, std::min(I, Is), H, nullptr, 1) ? ProductKernel::kHalf : ProductKernel::kGeneral;
     case HalfTiles::kRounds: return I % 64 == 0 && Is % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
     default: return ProductKernel::kGeneral;
   }

@@ -169,7 +169,7 @@ int launch_nt_fast(const void* a0, const void* a1, const void* b0, const void* b
   return JTMOE_OK;
 }
 
-// needs (K / 64, rounded up) * segs >= 2 * NSTAGE and a result of at most 0x7ffe0000 bytes
+// needs a result of at most 0x7ffe0000 bytes
 template <typename Cfg>
 int launch_nt_stream(const void* a0, const void* a1, const void* b0, const void* b1, void* c,
                      const int32_t* group_sizes, const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N,
@@ -181,6 +181,8 @@ int launch_nt_stream(const void* a0, const void* a1, const void* b0, const void*
   std::call_once(once, [&] { attr_err = allow_lds(kernel, L::kSmemBytes); });
   if (attr_err != hipSuccess)
     return fail(JTMOE_ELAUNCH, "grouped gemm (nt): hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
+  if (!fills_pipeline<Cfg>(Kdim, segs))
+    return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): reduction of %lld too short", (long long)Kdim);
   const int64_t mtiles = group_sizes == nullptr ? (rows + Cfg::BM - 1) / Cfg::BM : max_m_tiles(rows, E, Cfg::BM);
   const int64_t nt = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles_grid = gemm_grid(mtiles, nt);
@@ -235,6 +237,8 @@ int launch_nt_joint(const NtProblem& p, const int32_t* group_sizes, const int32_
   std::call_once(once, [&] { attr_err = allow_lds(kernel, L::kSmemBytes); });
   if (attr_err != hipSuccess)
     return fail(JTMOE_ELAUNCH, "grouped gemm (nt): hipFuncSetAttribute: %s", hipGetErrorString(attr_err));
+  if (!fills_pipeline<Cfg>(std::min(p.Kdim, s.Kdim), segs))
+    return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): reduction of %lld too short", (long long)std::min(p.Kdim, s.Kdim));
   const int64_t mtiles = max_m_tiles(p.rows, E, Cfg::BM), nt = (p.N + Cfg::BN - 1) / Cfg::BN;
   const int64_t mt1 = (s.rows + Cfg::BM - 1) / Cfg::BM, nt1 = (s.N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles_grid = gemm_grid(mtiles, nt) + gemm_grid(mt1, nt1);

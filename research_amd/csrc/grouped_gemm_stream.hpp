@@ -19,7 +19,8 @@
 //     row map of the next tile arrives by LDS-DMA as well, group sizes and offsets are read from a copy
 //     in LDS), so the compiler never inserts a wait that drains the operand loads.
 //
-// Requirements: those of grouped_gemm_dma.hpp, K % BK == 0 unless OPT & 65536, K / BK >= 2 * NSTAGE, a result of at most 0x7ffe0000
+// Requirements: those of grouped_gemm_dma.hpp, K % BK == 0 unless OPT & 65536, K / BK >= 2 * NSTAGE (fills_pipeline: with a
+// row map the next tile's has arrived after NSTAGE - 1 of the steps in front of the last NSTAGE), a result of at most 0x7ffe0000
 // bytes, with a row map fewer than 2^27 rows and row_div <= 32; launch with a multiple of 8 workgroups
 // (persistent schedule).
 #pragma once
@@ -48,6 +49,12 @@ struct StreamLayout {
   static_assert(kSmemBytes <= 160 * 1024, "LDS budget");
   static_assert(Cfg::BM + Cfg::XROWS <= Cfg::NT, "one row-map entry per thread");
 };
+
+// the reduction has the k steps that the kernel wants of it, in either segment or both together
+template <typename Cfg>
+inline bool fills_pipeline(int64_t Kdim, int segs = 1) {
+  return (Kdim + Cfg::BK - 1) / Cfg::BK * segs >= 2 * Cfg::NSTAGE;
+}
 
 // A second product in the same launch: one dense group with its own matrices, width and reduction length, as the
 // shared experts are beside the routed ones.

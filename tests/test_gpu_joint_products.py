@@ -30,6 +30,11 @@ SHAPES = [
     (3000, 1024, 5, 1, 768, 3072, "rows256 separate rows256 separate"),
     (2048, 1000, 8, 2, 2056, 2056, "rows256_tail rows256_tail rows256_tail rows256_tail"),
     (2600, 328, 12, 2, 1800, 4104, "rows256_tail half separate half_deep"),
+    # the shortest reductions that half tiles take, eight 32-deep steps, and the longest that they do not
+    (1000, 232, 8, 2, 512, 512, "half_tail half separate half_deep"),
+    (1000, 224, 8, 2, 512, 512, "separate half separate half_deep"),
+    (1000, 512, 8, 2, 232, 256, "half half half_deep half_deep"),
+    (1000, 512, 8, 2, 224, 232, "half separate half_deep half_deep"),
 ]
 
 

@@ -87,6 +87,15 @@ def test_joint_gradients_of_a_few_rows_leave_room_for_more_groups(tokens, top_k,
     assert joint_kernels(tokens, top_k, hidden, inter, shared, experts, MI355X_CUS)[2:] == [dz, dx]
 
 
+@pytest.mark.parametrize("reduction,gate_up,down", [(192, "separate", "separate"), (200, "separate", "separate"),
+                                                    (224, "separate", "separate"), (232, "half_tail", "half")])
+def test_joint_half_tiles_have_the_steps_their_pipeline_wants(reduction, gate_up, down):
+    """The shortest reductions in half tiles run in four 32-deep stages, which want eight steps, of either product."""
+    assert joint_kernels(1000, 2, reduction, 512, 512, 8, MI355X_CUS)[0] == gate_up
+    for inter, shared in ((reduction, reduction), (reduction, 512), (512, reduction)):
+        assert joint_kernels(1000, 2, 512, inter, shared, 8, MI355X_CUS)[1] == down
+
+
 def test_every_joint_kernel_is_held_to_separate_launches():
     for product, names in enumerate(zip(*(case[6].split() for case in joint.SHAPES))):
         assert set(names) == JOINT_KERNELS[product]
