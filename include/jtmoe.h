@@ -193,6 +193,21 @@ const char* jtmoe_product_kernel(int product, int64_t rows, int64_t K, int64_t N
 const char* jtmoe_joint_kernel(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is, int64_t E,
                                int compute_units);
 /*
+ * The tiles of the same launches: for kernels that choose them by the launch "64x64" to "256x128", "128x128_pair" (two
+ * workgroups to a compute unit), "tall" and "plain" (256 rows, of up to 320 or not), with "_tail" where a ragged
+ * reduction has a variant of its own; else the kernel's name.  Otherwise as above.
+ */
+const char* jtmoe_product_tiles(int product, int64_t rows, int64_t K, int64_t N, int64_t E, int compute_units);
+const char* jtmoe_joint_tiles(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is, int64_t E,
+                              int compute_units);
+/*
+ * Where a product (0 gate/up, 1 down) of the shared experts runs beside a launch in front of the routed products, and in
+ * which tiles, for aligned operands of a plain bf16 layer call of some hundred tokens: "router 128x64", "dispatch 64x64",
+ * ...; "" for none of these.  Otherwise as above.
+ */
+const char* jtmoe_shared_beside(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is, int64_t E,
+                                int compute_units);
+/*
  * Whether the single-precision backward pass of `rows` routed rows in E groups runs dXp and the three weight gradients
  * in one launch ("joint") or in launches of their own ("separate").  Otherwise as above.
  */

@@ -62,6 +62,9 @@ PROTOTYPES: dict[str, tuple] = {
     "jtmoe_grouped_swiglu_gather_supported": (c_int, [c_i64, c_i64, c_i64, c_int]),
     "jtmoe_product_kernel": (ctypes.c_char_p, [c_int, c_i64, c_i64, c_i64, c_i64, c_int]),
     "jtmoe_joint_kernel": (ctypes.c_char_p, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_int]),
+    "jtmoe_product_tiles": (ctypes.c_char_p, [c_int, c_i64, c_i64, c_i64, c_i64, c_int]),
+    "jtmoe_joint_tiles": (ctypes.c_char_p, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_int]),
+    "jtmoe_shared_beside": (ctypes.c_char_p, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_int]),
     "jtmoe_f32_backward_kernel": (ctypes.c_char_p, [c_i64, c_i64, c_i64, c_i64, c_int]),
     "jtmoe_moe_forward_takes_decode_path": (c_int, [c_i64, c_i64, c_i64, c_i64, c_i64, c_int]),
     "jtmoe_grouped_swiglu_gather": (

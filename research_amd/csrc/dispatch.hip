@@ -456,7 +456,6 @@ inline size_t partial_imp_offset(int64_t A, int64_t E) { return jtmoe_dispatch_w
 // batch; a training pass at 8192 takes the same time either way.  (Only in the
 // layer, whose workspace belongs to the call: the entry points of their own keep to one workgroup, which leaves
 // their scratch alone, up to kSmallMaxAssignments.)
-constexpr int64_t kSmallLayerAssignments = 4096;
 
 // The launches of a validated dispatch; `partial` holds jtmoe_dispatch_workspace_bytes(A, E) bytes
 // (dispatch_layer_workspace_bytes(A, E) when `weights` is given).

@@ -18,6 +18,7 @@
 namespace jtmoe {
 
 constexpr int kSmallMaxAssignments = 8192;
+constexpr int64_t kSmallLayerAssignments = 4096;  // in a layer call (dispatch.hip says why)
 constexpr int kSmallMaxExperts = JTMOE_MAX_EXPERTS;
 constexpr float kImportanceScale = 4294967296.0f;  // importance is summed in 32.32 fixed point: any order, same sum
 // A route weight as a 32.32 fixed-point term.  Route weights are finite, non-negative and far below 2^32

@@ -320,7 +320,7 @@ inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, doub
 // drain once a step (us, 256 x 256 / 128 x 256 / 256 x 128): 2048 rows 2816 -> 2048 down 62 / 41 / 40, dX 127 / 83 / 77; 6000
 // rows in 16 groups, 2816 -> 1024, down 66 / 47 / 44, dX 129 / 91 / 87; two rounds of them are no less than one (8192 rows:
 // 73 / 75 / 81, 139 / 155 / 153).
-// kFewRows: groups that fit one tile of 128 rows.  Bound by the expert matrices, read once, and so by the bytes of them
+// Groups that fit one tile of 128 rows (kFewGroupRows): bound by the expert matrices, read once, and so by the bytes of them
 // in flight: half as many rows, and more stages or workgroups for it.  us, 256-row tiles / 128-row ones; 64 groups, 2048 x
 // 1408: 77 rows gate/up 146 / 140, dZ 105 / 94, dX 152 / 138, down 77.2 / 78.6; 128 groups, 2048 x 768: 93 rows 168 / 157 and 97
 // / 96, skewed by Zipf's law 198 / 180 and 111 / 106; at 137 rows gate/up 172 / 206, down 87 / 111.  Nearer to 128 rows a few
@@ -332,11 +332,15 @@ inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, doub
 // takes a fifth longer), or where there are many rounds (the kernel then decides from the real sizes); else plain ones.
 // us, plain / taller: 64 groups of 137 rows, gate/up 171 / 181, down 87 / 99, dZ 118 / 138; of 256 rows 262 / 213, 128 / 119,
 // 158 / 160, dX 247 / 239; of 325 333 / 336; of 400 308 / 317, 170 / 173, 178 / 199.
-enum class TileShape { k64x64, k128x64, k128x128, k128x128Short, k256x128, k128x256, kFewRows, kTall, kPlain };
+// k128x128Pair: two workgroups to a CU.
+enum class TileShape { k64x64, k128x64, k128x128, k128x128Short, k128x128Pair, k256x128, k128x256, kTall, kPlain };
+enum class Product { kGateUp, kDown, kGradient, kGradientPair };  // the last: of two segments
+inline bool large_tiles(TileShape s) { return s == TileShape::kTall || s == TileShape::kPlain; }
 constexpr int64_t kFewGroupRows = 108, kFewGroupRowsSure = 94;  // mean + 3.5 standard deviations within 128
 constexpr double kManyRounds = 8.0;
-inline TileShape tile_shape(int64_t rows, int64_t E, bool dense, int64_t N, double cus, bool dual, int64_t dense_rows = 0,
-                            int64_t dense_N = 0) {
+inline TileShape tile_shape(Product product, int64_t rows, int64_t E, bool dense, int64_t N, double cus,
+                            int64_t dense_rows = 0, int64_t dense_N = 0) {
+  const bool dual = product == Product::kGateUp;
   auto one_each = [&](int BM, int BN) {
     const double mtiles = std::fmax(expected_mtiles(rows, E, dense, BM), spread_mtiles(rows, E, dense, BM));
     return mtiles * (double)((N + BN - 1) / BN) + (double)((dense_rows + BM - 1) / BM * ((dense_N + BN - 1) / BN)) <= cus;
@@ -351,7 +355,7 @@ inline TileShape tile_shape(int64_t rows, int64_t E, bool dense, int64_t N, doub
   auto rounds = [cus](double tiles) { return std::ceil(tiles / cus); };
   const double plain = spread_mtiles(rows, E, dense, 256) * nt + (double)((dense_rows + 255) / 256) * dense_nt;
   if (!dense && dense_rows == 0 && rows <= kFewGroupRows * E && (rows <= kFewGroupRowsSure * E || rounds(1.05 * plain) == rounds(plain)))
-    return TileShape::kFewRows;
+    return dual ? TileShape::k128x128 : product == Product::kDown ? TileShape::k128x256 : TileShape::k128x128Pair;
   const double tall = tall_mtiles(rows, E, dense, true) * nt + (double)group_mtiles((int)dense_rows, 256, 64) * dense_nt;
   if (rounds(plain) >= kManyRounds) return TileShape::kTall;
   const double low = std::fmax(expected_mtiles(rows, E, dense, 128), spread_mtiles(rows, E, dense, 128)) * nt +

@@ -33,6 +33,9 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
                    int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream);
 // ... and the kernel it takes for bf16 operands (16-byte aligned, below 2 GiB) on `cus` compute units
 ProductKernel data_gradient_kernel(int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense, int segs, double cus);
+// ... in which tiles
+enum class TileShape;
+TileShape data_gradient_tiles(ProductKernel k, int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense, int segs, double cus);
 
 // The routed product above and the shared experts' one (one dense group of s.rows rows) in one launch.  Operands as in
 // launch_gemm_nt, without a row map; gemm_nt_joint: the kernel, or kGeneral where launches of their own are faster or
@@ -49,6 +52,9 @@ int launch_gemm_nt_joint(int dtype, const NtProblem& p, const int32_t* group_siz
 // launches of their own
 ProductKernel joint_data_gradient_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t T, int64_t Is, int segs,
                                          double cus);
+// ... and its tiles: rows x N with a reduction of Kdim beside T x N1 with one of K1
+TileShape joint_data_gradient_tiles(ProductKernel k, int64_t rows, int64_t Kdim, int64_t N, int64_t E, int64_t T, int64_t K1,
+                                    int64_t N1, int segs, double cus);
 
 // C_i[e] = P[rows of group e, :]^T @ D_i[rows of group e, :]     (i = 0, and 1 if d1 is given)
 //   P: [rows, KA], D_i: [rows, N]; either may instead be [gathered_rows, .] read through row_map

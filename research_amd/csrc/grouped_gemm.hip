@@ -445,13 +445,31 @@ inline bool fast_ok(const void* a, const void* b0, const void* b1, const void* c
          aligned16(c);
 }
 
-// the tiles of a launch whose kernel the rules above have chosen (half: kHalf, kHalfTail)
-inline TileShape tiles_of(bool half, bool dual, int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense,
-                          const DenseProblem* dp = nullptr) {
-  const TileShape s = tile_shape(rows, E, dense, N, persistent_grid_size(), dual, dp ? dp->rows : 0, dp ? dp->n : 0);
-  const int64_t K = dp ? std::min<int64_t>(Kdim, dp->k) : Kdim;
-  // (plain tiles have four 32-deep stages here)
-  return tile_shape_for(s == TileShape::kPlain && (K + 31) / 32 < 8 ? TileShape::kTall : s, half, (K + 63) / 64, dual);
+// ---- the tiles of a launch whose kernel the rules above have chosen -----------------------------------------
+// (T rows times N1 columns with a reduction of K1 in the same launch, T = 0: none)
+inline TileShape stream_tiles(Product product, ProductKernel k, int64_t rows, int64_t K, int64_t N, int64_t E, bool dense,
+                              double cus, int64_t T = 0, int64_t K1 = 0, int64_t N1 = 0) {
+  const bool half = k == ProductKernel::kHalf || k == ProductKernel::kHalfTail;
+  const int64_t least = T ? std::min(K, K1) : K;
+  TileShape s = tile_shape(product, rows, E, dense, N, cus, T, N1);
+  if (s == TileShape::kPlain && (least + 31) / 32 < 8) s = TileShape::kTall;  // (plain tiles have four 32-deep stages here)
+  return tile_shape_for(s, half, (least + 63) / 64, product == Product::kGateUp);
+}
+
+// kHalf to kRows256Tail, with the activations as they are; kTall, kPlain: 256-row tiles of the stream kernel and of the other
+TileShape down_tiles(ProductKernel k, int64_t rows, int64_t H, int64_t I, int64_t E, bool dense, double cus) {
+  const TileShape tiles = stream_tiles(Product::kDown, k, rows, I, H, E, dense, cus);
+  const bool streams = stream_ok<DownStreamTailCfg>(rows, I, H, nullptr, 1);
+  if (k == ProductKernel::kHalfDeep) {
+    // Two half tiles per CU only where few CUs get a second one (4252 rows 2616 -> 1080, 306 of them: 50 us, 153 tiles of 256 x
+    // 128 57; groups of 250 rows, 296 of them, 55 and 46), or for want of steps (128 groups of 56 rows, skewed, 768 -> 2048: 92
+    // us against 97 in half tiles).
+    if (dense && 4 * ((rows + 127) / 128) * ((H + 127) / 128) <= 5 * (int64_t)cus) return TileShape::k128x128Pair;
+    const TileShape smaller = large_tiles(tiles) ? tile_shape_for(TileShape::k128x256, false, (I + 63) / 64, false) : tiles;
+    return streams && !large_tiles(smaller) ? smaller : TileShape::k128x128Pair;
+  }
+  if (streams && (!large_tiles(tiles) || tiles == TileShape::kTall)) return tiles;
+  return TileShape::kPlain;  // also for a reduction too short for the stream kernel, or a result past its limit
 }
 
 // y = act Wd[e] on the matrix cores (fast_ok holds); with a map, packed row j reads row row_map[j] / row_div of
@@ -474,25 +492,17 @@ int launch_down_fast(const void* act, const void* down, const int32_t* group_siz
   }
   // (at most half a tile of rows per group on the decode path: the rules above take all of it)
   if (row_map || beside) return fail(JTMOE_EUNSUPPORTED, "grouped gemm: no down kernel reads blocks of rows per group at this size");
-  const bool tail = k == ProductKernel::kRows256Tail, streams = stream_ok<DownStreamTailCfg>(rows, I, H, nullptr, 1);
-  TileShape tiles = tiles_of(k == ProductKernel::kHalf, false, rows, I, H, E, group_sizes == nullptr);
-  // Two half tiles per CU only where few CUs get a second one (4252 rows 2616 -> 1080, 306 of them: 50 us, 153 tiles of 256 x
-  // 128 57; groups of 250 rows, 296 of them, 55 and 46), or for want of steps (128 groups of 56 rows, skewed, 768 -> 2048: 92 us against 97 in half tiles).
-  const bool deep = k == ProductKernel::kHalfDeep && group_sizes == nullptr &&
-                    4 * ((rows + 127) / 128) * ((H + 127) / 128) <= 5 * persistent_grid_size();
-  if (deep) tiles = TileShape::kPlain;
-  if (k == ProductKernel::kHalfDeep && !deep && large_tiles(tiles))
-    tiles = tile_shape_for(TileShape::k128x256, false, (I + 63) / 64, false);
-  if (streams && !large_tiles(tiles))
-    return with_smaller_tiles<true>(tiles, [&](auto cfg) { return JT_DOWN(launch_stream, decltype(cfg))); });
-  if (k == ProductKernel::kHalfDeep) return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
-  // 256-row tiles; also for a reduction too short for the stream kernel, or a result past its limit: the kernel without it
-  if (streams && tiles == TileShape::kTall) {
-    if (tail) return JT_DOWN(launch_stream, DownStreamTailCfg));
-    return JT_DOWN(launch_stream, DownStreamCfg));
+  const bool tail = k == ProductKernel::kRows256Tail;
+  switch (const TileShape tiles = down_tiles(k, rows, H, I, E, group_sizes == nullptr, persistent_grid_size())) {
+    case TileShape::k128x128Pair: return JT_DOWN(launch_stream, DownHalfDeepCfg), 2);
+    case TileShape::kTall:
+      if (tail) return JT_DOWN(launch_stream, DownStreamTailCfg));
+      return JT_DOWN(launch_stream, DownStreamCfg));
+    case TileShape::kPlain:
+      if (tail) return JT_DOWN(launch_fast, DownTailCfg));
+      return JT_DOWN(launch_fast, DownCfg));
+    default: return with_smaller_tiles<true>(tiles, [&](auto cfg) { return JT_DOWN(launch_stream, decltype(cfg))); });
   }
-  if (tail) return JT_DOWN(launch_fast, DownTailCfg));
-  return JT_DOWN(launch_fast, DownCfg));
 #undef JT_DOWN
 }
 
@@ -514,6 +524,7 @@ int launch_gate_up(const RoutedProblem& p, hipStream_t stream, const Beside* bes
     using S22 = SkinnyCfg<2, 2, true>;
     const ProductKernel k = gate_up_kernel(p.rows, p.K, p.N, p.E, dense, persistent_grid_size(), p.row_map, p.row_div);
     if (beside) *beside_taken = streaming_or_rows64(k) && k != ProductKernel::kRows64Tail;
+    auto tiles = [&](ProductKernel k) { return stream_tiles(Product::kGateUp, k, p.rows, p.K, p.N, p.E, dense, persistent_grid_size()); };
     switch (k) {
       case ProductKernel::kStream16x128: return JT_GATE_UP(launch_skinny, S11, JT_BESIDE);
       case ProductKernel::kStream16x64: return JT_GATE_UP(launch_skinny, S12, JT_BESIDE);
@@ -522,12 +533,10 @@ int launch_gate_up(const RoutedProblem& p, hipStream_t stream, const Beside* bes
       case ProductKernel::kRows64Tail: return JT_GATE_UP(launch_fast, GateUpTinyTailCfg);
       case ProductKernel::kHalf:
       case ProductKernel::kRows256:
-        return with_gate_up_tiles<false, false>(tiles_of(k == ProductKernel::kHalf, true, p.rows, p.K, p.N, p.E, dense),
-                                         [&](auto cfg) { return JT_GATE_UP(launch_stream, decltype(cfg)); });
+        return with_gate_up_tiles<false, false>(tiles(k), [&](auto cfg) { return JT_GATE_UP(launch_stream, decltype(cfg)); });
       case ProductKernel::kHalfTail:
       case ProductKernel::kRows256Tail:
-        return with_gate_up_tiles<true, false>(tiles_of(k == ProductKernel::kHalfTail, true, p.rows, p.K, p.N, p.E, dense),
-                                        [&](auto cfg) { return JT_GATE_UP(launch_stream, decltype(cfg)); });
+        return with_gate_up_tiles<true, false>(tiles(k), [&](auto cfg) { return JT_GATE_UP(launch_stream, decltype(cfg)); });
       case ProductKernel::kRows256Short: return JT_GATE_UP(launch_fast, GateUpCfg);
       default: return JT_GATE_UP(launch_fast, GateUpTailCfg);
     }
@@ -580,31 +589,29 @@ int launch_with_shared(const RoutedProblem& gu, const RoutedProblem& dn, const R
   auto gate_up = [&](auto cfg) { return launch_joint<decltype(cfg)>(gu, dgu, stream); };
   auto down = [&](auto cfg) { return launch_joint<decltype(cfg)>(dn, ddn, stream); };
   int rc;
-  switch (jg) {
-    case ProductKernel::kGeneral: rc = launch_gate_up<T>(gu, stream); break;
-    case ProductKernel::kHalf:
-    case ProductKernel::kRows256:
-      rc = with_gate_up_tiles<false, true>(tiles_of(jg == ProductKernel::kHalf, true, gu.rows, gu.K, gu.N, gu.E, false, &dgu), gate_up);
-      break;
-    default:
-      rc = with_gate_up_tiles<true, true>(tiles_of(jg == ProductKernel::kHalfTail, true, gu.rows, gu.K, gu.N, gu.E, false, &dgu), gate_up);
-      break;
+  auto tiles_with = [](Product product, ProductKernel k, const RoutedProblem& p, const RoutedProblem& s) {
+    return stream_tiles(product, k, p.rows, p.K, p.N, p.E, false, persistent_grid_size(), s.rows, s.K, s.N);
+  };
+  if (!joint_gu) {
+    rc = launch_gate_up<T>(gu, stream);
+  } else {
+    const TileShape tiles = tiles_with(Product::kGateUp, jg, gu, sgu);
+    const bool tail = jg == ProductKernel::kHalfTail || jg == ProductKernel::kRows256Tail;
+    rc = tail ? with_gate_up_tiles<true, true>(tiles, gate_up) : with_gate_up_tiles<false, true>(tiles, gate_up);
   }
   if (!rc && !gate_up_done && !joint_gu && joint_dn) rc = launch_gate_up<T>(sgu, stream);
   if (rc) return rc;
-  switch (jd) {
-    case ProductKernel::kGeneral: rc = launch_down<T>(dn, stream); break;
-    default: {
-      const TileShape tiles = tiles_of(jd == ProductKernel::kHalf, false, dn.rows, dn.K, dn.N, dn.E, false, &ddn);
-      const bool tail = jd == ProductKernel::kRows256Tail;
-      if (!large_tiles(tiles))
-        rc = with_smaller_tiles<true>(tiles, down);
-      else if (tiles == TileShape::kPlain)
-        rc = tail ? down(DownPlainCfg<true>{}) : down(DownPlainCfg<false>{});
-      else
-        rc = tail ? down(DownStreamTailCfg{}) : down(DownStreamCfg{});
-      break;
-    }
+  if (!joint_dn) {
+    rc = launch_down<T>(dn, stream);
+  } else {
+    const TileShape tiles = tiles_with(Product::kDown, jd, dn, sdn);
+    const bool tail = jd == ProductKernel::kRows256Tail;
+    if (tiles == TileShape::kPlain)
+      rc = tail ? down(DownPlainCfg<true>{}) : down(DownPlainCfg<false>{});
+    else if (tiles == TileShape::kTall)
+      rc = tail ? down(DownStreamTailCfg{}) : down(DownStreamCfg{});
+    else
+      rc = with_smaller_tiles<true>(tiles, down);
   }
   if (!rc && !gate_up_done && !joint_gu && !joint_dn) rc = launch_gate_up<T>(sgu, stream);
   if (!rc && !down_done && !joint_dn) rc = launch_down<T>(sdn, stream);
@@ -686,16 +693,32 @@ bool shared_in_skinny_tiles(const void* x, const SharedExperts& s, int64_t T, in
 // ---- products of the shared experts beside the small launches in front of the routed ones ----
 // Both take tiles that find a CU each; they run on as they would alone, and the launch beside them, a few workgroups and
 // 7 to 12 us, costs nothing.  Sizes whose products are parts of the routed launches (joint_gate_up, joint_down) stay there.
+// (kPlain: none)
+TileShape tiles_beside(Product product, int64_t T, int64_t H, int64_t Is, int64_t I, int64_t E, int64_t K, int front,
+                       double cus) {
+  const bool dual = product == Product::kGateUp;
+  const ProductKernel k = dual ? gate_up_kernel(T, H, Is, 1, true, cus) : down_kernel(T, H, Is, 1, true, cus);
+  const bool joint = (dual ? joint_gate_up(T * K, H, I, E, T, Is, cus) : joint_down(T * K, H, I, E, T, Is, cus)) != ProductKernel::kGeneral;
+  // (gate/up of whole reductions only: see dense_stream_tiles)
+  const bool streams = k == ProductKernel::kHalf || (dual ? k == ProductKernel::kRows256
+                                                          : (k == ProductKernel::kRows256 || k == ProductKernel::kRows256Tail) &&
+                                                                stream_ok<DownStreamTailCfg>(T, Is, H, nullptr, 1));
+  if (joint || !streams) return TileShape::kPlain;
+  const int64_t N = dual ? Is : H;
+  const TileShape tiles = stream_tiles(product, k, T, dual ? H : Is, N, 1, true, cus);
+  if (tiles != TileShape::k64x64 && tiles != TileShape::k128x64) return TileShape::kPlain;
+  const int BM = tiles == TileShape::k64x64 ? 64 : 128;
+  return front + gemm_grid((T + BM - 1) / BM, (N + 63) / 64) <= (int64_t)cus ? tiles : TileShape::kPlain;
+}
+
 namespace {
 
-SharedTiles beside_front(const RoutedProblem& s, bool dual, bool half, int front) {
-  const TileShape tiles = tiles_of(half, dual, s.rows, s.K, s.N, 1, true);
-  if (tiles != TileShape::k64x64 && tiles != TileShape::k128x64) return SharedTiles{};
-  const int BM = tiles == TileShape::k64x64 ? 64 : 128;
+SharedTiles beside_front(const RoutedProblem& s, TileShape tiles) {
+  if (tiles == TileShape::kPlain) return SharedTiles{};
   SharedTiles t{tiles, dense_problem(s), 0};
   t.p.ntiles = (int)((s.N + 63) / 64);
-  const int64_t grid = gemm_grid((s.rows + BM - 1) / BM, t.p.ntiles);
-  if (front + grid <= persistent_grid_size()) t.grid = (int)grid;
+  const int BM = tiles == TileShape::k64x64 ? 64 : 128;
+  t.grid = (int)gemm_grid((s.rows + BM - 1) / BM, t.p.ntiles);
   return t;
 }
 
@@ -706,7 +729,6 @@ struct DispatchPlan {
   int32_t *group_sizes, *offsets, *source_order, *inverse;
   float *counts, *importance;
 };
-constexpr int kDispatchFront = 8;
 
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NT) void dispatch_beside_kernel(DispatchPlan d, DenseProblem shared) {
@@ -722,25 +744,15 @@ __global__ __launch_bounds__(Cfg::NT) void dispatch_beside_kernel(DispatchPlan d
 }  // namespace
 
 SharedTiles shared_gate_up_beside(const void* x, const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front) {
-  const double cus = persistent_grid_size();
-  const ProductKernel k = gate_up_kernel(T, H, s.Is, 1, true, cus);
-  if ((k != ProductKernel::kHalf && k != ProductKernel::kRows256) || !fast_ok(x, s.gate, s.up, s.act, H, s.Is) ||
-      !aligned16(s.gate_pre) || !aligned16(s.up_pre) ||
-      joint_gate_up(T * K, H, s.routed_I, E, T, s.Is, cus) != ProductKernel::kGeneral)
-    return SharedTiles{};
-  return beside_front({x, s.gate, s.up, s.act, s.gate_pre, s.up_pre, nullptr, nullptr, nullptr, T, H, s.Is, 1, 0, 1}, true,
-                      k == ProductKernel::kHalf, front);
+  if (!fast_ok(x, s.gate, s.up, s.act, H, s.Is) || !aligned16(s.gate_pre) || !aligned16(s.up_pre)) return SharedTiles{};
+  return beside_front({x, s.gate, s.up, s.act, s.gate_pre, s.up_pre, nullptr, nullptr, nullptr, T, H, s.Is, 1, 0, 1},
+                      tiles_beside(Product::kGateUp, T, H, s.Is, s.routed_I, E, K, front, persistent_grid_size()));
 }
 
 SharedTiles shared_down_beside(const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front) {
-  const double cus = persistent_grid_size();
-  const ProductKernel k = down_kernel(T, H, s.Is, 1, true, cus);
-  if ((k != ProductKernel::kHalf && k != ProductKernel::kRows256 && k != ProductKernel::kRows256Tail) ||
-      !fast_ok(s.act, s.down, nullptr, s.y, s.Is, H) || !stream_ok<DownStreamTailCfg>(T, s.Is, H, nullptr, 1) ||
-      joint_down(T * K, H, s.routed_I, E, T, s.Is, cus) != ProductKernel::kGeneral)
-    return SharedTiles{};
-  return beside_front({s.act, s.down, nullptr, s.y, nullptr, nullptr, nullptr, nullptr, nullptr, T, s.Is, H, 1, 0, 1}, false,
-                      k == ProductKernel::kHalf, front);
+  if (!fast_ok(s.act, s.down, nullptr, s.y, s.Is, H)) return SharedTiles{};
+  return beside_front({s.act, s.down, nullptr, s.y, nullptr, nullptr, nullptr, nullptr, nullptr, T, s.Is, H, 1, 0, 1},
+                      tiles_beside(Product::kDown, T, H, s.Is, s.routed_I, E, K, front, persistent_grid_size()));
 }
 
 int launch_dispatch_beside_shared(const int32_t* ids, const void* weights, const void* x, int64_t T, int64_t H, int64_t E,
@@ -834,34 +846,83 @@ static const char* const kProductKernelNames[] = {"general", "stream_16x128", "s
                                                   "rows64_tail", "half", "half_tail", "half_deep", "rows256",
                                                   "rows256_tail", "rows256_short", "rows256_short_tail"};
 
+static bool product_sizes_ok(int product, int64_t rows, int64_t K, int64_t N, int64_t E, int compute_units) {
+  return product >= 0 && product <= 3 && rows > 0 && K > 0 && N > 0 && E >= 0 && K < ((int64_t)1 << 24) &&
+         N < ((int64_t)1 << 24) && rows < ((int64_t)1 << 31) && compute_units >= 0;
+}
+
+static ProductKernel product_kernel(int product, int64_t rows, int64_t K, int64_t N, int64_t groups, bool dense, double cus) {
+  if (product >= 2) return data_gradient_kernel(rows, K, N, groups, dense, product - 1, cus);
+  if (!fast_ok(nullptr, nullptr, nullptr, nullptr, K, N)) return ProductKernel::kGeneral;
+  return product == 0 ? gate_up_kernel(rows, K, N, groups, dense, cus) : down_kernel(rows, N, K, groups, dense, cus);
+}
+
 extern "C" const char* jtmoe_product_kernel(int product, int64_t rows, int64_t K, int64_t N, int64_t E, int compute_units) {
+  if (!product_sizes_ok(product, rows, K, N, E, compute_units)) return "";
+  const double cus = compute_units > 0 ? compute_units : persistent_grid_size();
+  return kProductKernelNames[(int)product_kernel(product, rows, K, N, E == 0 ? 1 : E, E == 0, cus)];
+}
+
+// ... and their tiles; "_tail" where a ragged reduction has a variant of its own
+static const char* tile_name(TileShape s, bool tail) {
+  static const char* const names[][2] = {{"64x64", "64x64_tail"}, {"128x64", "128x64_tail"}, {"128x128", "128x128_tail"},
+                                         {"128x128_short", "128x128_short_tail"}, {"128x128_pair", "128x128_pair"},
+                                         {"256x128", "256x128"}, {"128x256", "128x256"}, {"tall", "tall_tail"},
+                                         {"plain", "plain_tail"}};
+  return names[(int)s][tail];
+}
+
+extern "C" const char* jtmoe_product_tiles(int product, int64_t rows, int64_t K, int64_t N, int64_t E, int compute_units) {
+  if (!product_sizes_ok(product, rows, K, N, E, compute_units)) return "";
   const bool dense = E == 0;
-  if (product < 0 || product > 3 || rows <= 0 || K <= 0 || N <= 0 || E < 0 || K >= ((int64_t)1 << 24) ||
-      N >= ((int64_t)1 << 24) || rows >= ((int64_t)1 << 31) || compute_units < 0)
-    return "";
   const double cus = compute_units > 0 ? compute_units : persistent_grid_size();
   const int64_t groups = dense ? 1 : E;
-  ProductKernel k = ProductKernel::kGeneral;
-  if (product >= 2)
-    k = data_gradient_kernel(rows, K, N, groups, dense, product - 1, cus);
-  else if (fast_ok(nullptr, nullptr, nullptr, nullptr, K, N))
-    k = product == 0 ? gate_up_kernel(rows, K, N, groups, dense, cus) : down_kernel(rows, N, K, groups, dense, cus);
-  return kProductKernelNames[(int)k];
+  const ProductKernel k = product_kernel(product, rows, K, N, groups, dense, cus);
+  if (k == ProductKernel::kGeneral || streaming_or_rows64(k) || k == ProductKernel::kRows256Short || k == ProductKernel::kRows256ShortTail)
+    return kProductKernelNames[(int)k];
+  if (product == 0)
+    return tile_name(stream_tiles(Product::kGateUp, k, rows, K, N, groups, dense, cus),
+                     k == ProductKernel::kHalfTail || k == ProductKernel::kRows256Tail);
+  const TileShape s = product == 1 ? down_tiles(k, rows, N, K, groups, dense, cus)
+                                   : data_gradient_tiles(k, rows, K, N, groups, dense, product - 1, cus);
+  return tile_name(s, k == ProductKernel::kRows256Tail && large_tiles(s));
+}
+
+static bool joint_sizes_ok(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is, int64_t E,
+                           int compute_units) {
+  const int64_t limit = (int64_t)1 << 24;
+  return product >= 0 && product <= 3 && T > 0 && top_k > 0 && H > 0 && I > 0 && Is > 0 && E > 0 && H < limit &&
+         I < limit && Is < limit && T * top_k < ((int64_t)1 << 31) && compute_units >= 0;
+}
+
+static ProductKernel joint_kernel(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is, int64_t E, double cus) {
+  if (product >= 2) return joint_data_gradient_kernel(T * top_k, H, I, E, T, Is, product - 1, cus);
+  if (!fast_ok(nullptr, nullptr, nullptr, nullptr, H, I) || !fast_ok(nullptr, nullptr, nullptr, nullptr, H, Is))
+    return ProductKernel::kGeneral;
+  return product == 0 ? joint_gate_up(T * top_k, H, I, E, T, Is, cus) : joint_down(T * top_k, H, I, E, T, Is, cus);
 }
 
 extern "C" const char* jtmoe_joint_kernel(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is,
                                           int64_t E, int compute_units) {
-  const int64_t limit = (int64_t)1 << 24;
-  if (product < 0 || product > 3 || T <= 0 || top_k <= 0 || H <= 0 || I <= 0 || Is <= 0 || E <= 0 || H >= limit ||
-      I >= limit || Is >= limit || T * top_k >= ((int64_t)1 << 31) || compute_units < 0)
-    return "";
+  if (!joint_sizes_ok(product, T, top_k, H, I, Is, E, compute_units)) return "";
   const double cus = compute_units > 0 ? compute_units : persistent_grid_size();
-  ProductKernel k = ProductKernel::kGeneral;
-  if (product >= 2)
-    k = joint_data_gradient_kernel(T * top_k, H, I, E, T, Is, product - 1, cus);
-  else if (fast_ok(nullptr, nullptr, nullptr, nullptr, H, I) && fast_ok(nullptr, nullptr, nullptr, nullptr, H, Is))
-    k = product == 0 ? joint_gate_up(T * top_k, H, I, E, T, Is, cus) : joint_down(T * top_k, H, I, E, T, Is, cus);
+  const ProductKernel k = joint_kernel(product, T, top_k, H, I, Is, E, cus);
   return k == ProductKernel::kGeneral ? "separate" : kProductKernelNames[(int)k];
+}
+
+extern "C" const char* jtmoe_joint_tiles(int product, int64_t T, int64_t top_k, int64_t H, int64_t I, int64_t Is,
+                                         int64_t E, int compute_units) {
+  if (!joint_sizes_ok(product, T, top_k, H, I, Is, E, compute_units)) return "";
+  const double cus = compute_units > 0 ? compute_units : persistent_grid_size();
+  const int64_t rows = T * top_k;
+  const ProductKernel k = joint_kernel(product, T, top_k, H, I, Is, E, cus);
+  if (k == ProductKernel::kGeneral) return "separate";
+  const bool tail = k == ProductKernel::kHalfTail || k == ProductKernel::kRows256Tail;
+  if (product == 0) return tile_name(stream_tiles(Product::kGateUp, k, rows, H, I, E, false, cus, T, H, Is), tail);
+  const TileShape s = product == 1   ? stream_tiles(Product::kDown, k, rows, I, H, E, false, cus, T, Is, H)
+                      : product == 2 ? joint_data_gradient_tiles(k, rows, H, I, E, T, H, Is, 1, cus)
+                                     : joint_data_gradient_tiles(k, rows, I, H, E, T, Is, H, 2, cus);
+  return tile_name(s, tail && large_tiles(s));
 }
 
 extern "C" int jtmoe_grouped_swiglu_gather_supported(int64_t T, int64_t H, int64_t I, int dtype) {

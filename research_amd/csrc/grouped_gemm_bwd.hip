@@ -206,6 +206,27 @@ ProductKernel data_gradient_kernel(int64_t rows, int64_t Kdim, int64_t N, int64_
   return Kdim % 64 == 0 ? ProductKernel::kRows256 : ProductKernel::kRows256Tail;
 }
 
+// its tiles (kTall, kPlain: 256-row ones of the stream kernel and of the other)
+static Product gradient_product(int segs) { return segs == 1 ? Product::kGradient : Product::kGradientPair; }
+TileShape data_gradient_tiles(ProductKernel k, int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense, int segs, double cus) {
+  const int64_t steps = (Kdim + 63) / 64 * segs;
+  const bool streams = steps >= 2 * DgradStreamCfg::NSTAGE && rows * N * 2 <= (int64_t)0x7ffe0000;
+  const TileShape tiles = tile_shape_for(tile_shape(gradient_product(segs), rows, E, dense, N, cus),
+                                         k == ProductKernel::kHalfDeep, steps, false);
+  // (few steps: two workgroups per CU; 3000 rows 1024 -> 2048 19 us against 22 in one round of 256 x 128 tiles, 2048 rows
+  // 2048 -> 2816 38 against 33)
+  if (k == ProductKernel::kHalf && steps < 24) return TileShape::k128x128Pair;
+  if (tiles == TileShape::k128x128Pair || (streams && !large_tiles(tiles))) return tiles;
+  if (k == ProductKernel::kHalf) return TileShape::k128x128Pair;
+  // also for a reduction too short for the stream kernel, or a result past its limit: the kernel without it
+  return streams && tiles == TileShape::kTall ? TileShape::kTall : TileShape::kPlain;
+}
+TileShape joint_data_gradient_tiles(ProductKernel k, int64_t rows, int64_t Kdim, int64_t N, int64_t E, int64_t T, int64_t K1,
+                                    int64_t N1, int segs, double cus) {
+  return tile_shape_for(tile_shape(gradient_product(segs), rows, E, false, N, cus, T, N1), k == ProductKernel::kHalfDeep,
+                        (std::min(Kdim, K1) + 63) / 64 * segs, false);
+}
+
 // (both reductions fill the stream kernel's pipeline and both results stay below its limit)
 ProductKernel joint_data_gradient_kernel(int64_t rows, int64_t H, int64_t I, int64_t E, int64_t T, int64_t Is, int segs,
                                          double cus) {
@@ -268,8 +289,8 @@ int launch_gemm_nt_joint(int dtype, const NtProblem& p, const int32_t* group_siz
   const ProductKernel k = gemm_nt_joint(dtype, p, E, s, segs);
   if (k == ProductKernel::kGeneral) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): no joint launch at this size");
   auto launch = [&](auto cfg) { return launch_nt_joint<decltype(cfg)>(p, group_sizes, offsets, E, s, segs, stream); };
-  const TileShape tiles = tile_shape_for(tile_shape(p.rows, E, false, p.N, persistent_grid_size(), false, s.rows, s.N),
-                                         k == ProductKernel::kHalfDeep, (std::min(p.Kdim, s.Kdim) + 63) / 64 * segs, false);
+  const TileShape tiles =
+      joint_data_gradient_tiles(k, p.rows, p.Kdim, p.N, E, s.rows, s.Kdim, s.N, segs, persistent_grid_size());
   if (!large_tiles(tiles)) return with_smaller_tiles<false>(tiles, launch);
   const bool tail = k == ProductKernel::kRows256Tail;
   if (tiles == TileShape::kPlain) return tail ? launch(DgradPlainCfg<true>{}) : launch(DgradPlainCfg<false>{});
@@ -283,26 +304,17 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
   const bool dense = group_sizes == nullptr;
   const bool fast = dtype == JTMOE_BF16 && (row_map ? a_rows : rows) * Kdim < kOperandLimit && aligned16(a0) &&
                     aligned16(b0) && (segs == 1 || (aligned16(a1) && aligned16(b1))) && aligned16(c);
-  const bool streams = (Kdim + 63) / 64 * segs >= 2 * DgradStreamCfg::NSTAGE && rows * N * 2 <= (int64_t)0x7ffe0000 &&
-                       (row_map == nullptr || (rows < ((int64_t)1 << 27) && row_div >= 1 && row_div <= 32));
 #define JT_NT(LAUNCH, CFG) \
   LAUNCH<CFG>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div, a_rows, segs, stream)
   const ProductKernel k = fast ? data_gradient_kernel(rows, Kdim, N, E, dense, segs, persistent_grid_size()) : ProductKernel::kGeneral;
   if (k != ProductKernel::kGeneral) {
-    const TileShape tiles = tile_shape_for(tile_shape(rows, E, dense, N, persistent_grid_size(), false),
-                                           k == ProductKernel::kHalfDeep, (Kdim + 63) / 64 * segs, false);
-    // (few steps: two workgroups per CU; 3000 rows 1024 -> 2048 19 us against 22 in one round of 256 x 128 tiles, 2048 rows
-    // 2048 -> 2816 38 against 33)
-    const bool half = k == ProductKernel::kHalf && (Kdim + 63) / 64 * segs < 24;
-    if (half || tiles == TileShape::kFewRows) return JT_NT(launch_nt_fast, DgradHalfCfg);
-    if (streams && !large_tiles(tiles))
-      return with_smaller_tiles<false>(tiles, [&](auto cfg) { return JT_NT(launch_nt_stream, decltype(cfg)); });
     const bool tail = k == ProductKernel::kRows256Tail;
-    if (k == ProductKernel::kHalf) return JT_NT(launch_nt_fast, DgradHalfCfg);
-    // 256-row tiles; also for a reduction too short for the stream kernel, or a result past its limit: the kernel without it
-    if (streams && tiles == TileShape::kTall)
-      return tail ? JT_NT(launch_nt_stream, DgradStreamTailCfg) : JT_NT(launch_nt_stream, DgradStreamCfg);
-    return tail ? JT_NT(launch_nt_fast, DgradTailCfg) : JT_NT(launch_nt_fast, DgradCfg);
+    switch (const TileShape tiles = data_gradient_tiles(k, rows, Kdim, N, E, dense, segs, persistent_grid_size())) {
+      case TileShape::k128x128Pair: return JT_NT(launch_nt_fast, DgradHalfCfg);
+      case TileShape::kTall: return tail ? JT_NT(launch_nt_stream, DgradStreamTailCfg) : JT_NT(launch_nt_stream, DgradStreamCfg);
+      case TileShape::kPlain: return tail ? JT_NT(launch_nt_fast, DgradTailCfg) : JT_NT(launch_nt_fast, DgradCfg);
+      default: return with_smaller_tiles<false>(tiles, [&](auto cfg) { return JT_NT(launch_nt_stream, decltype(cfg)); });
+    }
   }
 #undef JT_NT
   if (dtype == JTMOE_F32 && f32_gemm_supported(a0, a1, b0, b1, c, row_map ? a_rows : rows, Kdim, N) &&

@@ -674,14 +674,14 @@ int with_gate_up_tiles(TileShape s, Launch launch) {
   switch (s) {
     case TileShape::k64x64: return launch(GateUpQuarterCfg<kTail>{});
     case TileShape::k128x64: return launch(GateUpNarrowCfg<kTail>{});
-    case TileShape::k128x128:
-    case TileShape::kFewRows: return launch(GateUpHalfCfg<kTail>{});
+    case TileShape::k128x128: return launch(GateUpHalfCfg<kTail>{});
     case TileShape::k128x128Short: return launch(GateUpHalfShortCfg<kTail>{});
     case TileShape::kPlain: return launch(GateUpPlainCfg<kTail, kJoint>{});
     default: return launch(std::conditional_t<kTail, GateUpStreamTailCfg, GateUpStreamCfg>{});
   }
 }
-// ... for down products and data gradients, all but the largest
+// ... for down products and data gradients, all but the largest (no data gradient asks for the short ones: the deep kernel
+// would be refused)
 template <bool kDown, typename Launch>
 int with_smaller_tiles(TileShape s, Launch launch) {
   switch (s) {
@@ -689,7 +689,7 @@ int with_smaller_tiles(TileShape s, Launch launch) {
     case TileShape::k128x64: return launch(NarrowCfg{});
     case TileShape::k128x128: return launch(std::conditional_t<kDown, DownHalfCfg, DgradHalfDeepCfg>{});
     case TileShape::k256x128: return launch(Rows256Cfg{});
-    case TileShape::k128x128Short: return launch(HalfShortCfg{});
+    case TileShape::k128x128Short: return launch(std::conditional_t<kDown, HalfShortCfg, DgradHalfDeepCfg>{});
     default: return launch(Rows128Cfg{});
   }
 }
@@ -701,6 +701,9 @@ struct SharedTiles {
   DenseProblem p;
   int grid;
 };
+constexpr int kDispatchFront = 8;  // the workgroups of the dispatch in front of such tiles
+TileShape tiles_beside(Product product, int64_t T, int64_t H, int64_t Is, int64_t I, int64_t E, int64_t K, int front,
+                       double cus);  // by the sizes alone; kPlain: none
 SharedTiles shared_gate_up_beside(const void* x, const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front);
 SharedTiles shared_down_beside(const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front);
 
@@ -709,7 +712,5 @@ __device__ __forceinline__ void dense_stream_tiles(const DenseProblem& p, int fr
   stream_gemm_body<Cfg, false>(p.a0, nullptr, p.b0, p.b1, p.c, nullptr, nullptr, 1, p.rows, p.k, p.n, p.ntiles, nullptr, 1,
                                0, p.save0, p.save1, 1, 0, 0, DenseProblem{}, front);
 }
-
-inline bool large_tiles(TileShape s) { return s == TileShape::kTall || s == TileShape::kPlain; }
 
 }  // namespace jtmoe

@@ -1402,9 +1402,11 @@ struct LayerPlan {
 };
 
 // (the launch's LDS is the larger one's, and one of its workgroups fills a CU either way)
+inline int finish_blocks(int64_t tokens) { return (int)((tokens + kFinishBlockTokens - 1) / kFinishBlockTokens); }
+inline int finish_front(int64_t tokens) { return (finish_blocks(tokens) + 7) / 8 * 8; }
 int launch_finish_blocks(const FinishBlocks& f, const void* x, int64_t H, SharedExperts* shared, hipStream_t stream) {
   const size_t smem = router_smem_bytes(f.E, f.K, kFinishBlockTokens);
-  const int blocks = (f.tokens + kFinishBlockTokens - 1) / kFinishBlockTokens, front = (blocks + 7) / 8 * 8;
+  const int blocks = finish_blocks(f.tokens), front = finish_front(f.tokens);
   const SharedTiles tiles = shared ? shared_gate_up_beside(x, *shared, f.tokens, H, f.E, f.K, front) : SharedTiles{};
   auto beside = [&](auto cfg) {
     using Cfg = decltype(cfg);
@@ -1461,6 +1463,24 @@ int launch_router_chain(const void* x, const void* w, const float* bias, int64_t
   return check_launch("router");
 }
 
+// The forms of the matrix-core router: a few hundred tokens k slice by k slice (one chain of a padded size), then a
+// finishing launch where the epilogue of the whole call fits a workgroup's LDS ...
+inline bool router_split(int64_t tokens, int64_t H, int64_t E) {
+  return (router_chained(H, E) || H % kSplitKC == 0) && tokens <= kSplitMaxTokens;
+}
+inline int finish_tokens(int64_t E, int64_t K) { return router_smem_bytes((int)E, (int)K, 256) <= 160 * 1024 ? 256 : 64; }
+inline bool router_two_launches(int64_t tokens, int64_t E, int64_t K) {
+  const int finish_tok = finish_tokens(E, K);
+  return tokens > 0 && tokens <= finish_tok && router_smem_bytes((int)E, (int)K, finish_tok) <= 160 * 1024;
+}
+inline int router_slices(int64_t H) { return (int)((H + router_slice_rows((int)H) - 1) / router_slice_rows((int)H)); }
+// ... and, of a layer call with `scratch` bytes to spare, middle-sized ones, of what the former leave
+inline bool router_middle(int64_t tokens, int64_t H, int64_t E, int64_t K, size_t scratch) {
+  return tokens <= kMidMaxTokens && H % kSplitKC == 0 && H >= 1024 &&
+         (size_t)router_slices(H) * tokens * E * sizeof(float) <= scratch &&
+         router_smem_bytes((int)E, (int)K, kFinishBlockTokens) <= 160 * 1024;
+}
+
 template <typename T, bool kFromLogits>
 int launch_router(const void* x, const void* w, const float* logits_in, const float* bias, int64_t tokens,
                   int64_t H, int64_t E, int64_t K, double route_scale, int32_t* ids, void* weights,
@@ -1477,7 +1497,7 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
     // chain of chunks: the k-split kernel (16 tokens per workgroup, half as many and shorter
     // iterations) is used; beyond that the 64-token workgroups stage the router matrix four times
     // less often per token and win.
-    if ((chained || H % kSplitKC == 0) && tokens <= kSplitMaxTokens) {
+    if (router_split(tokens, H, E)) {
       const int blocks = (int)((tokens + 15) / 16);
       const size_t smem = chained ? router_chain_smem_bytes<1>(std::min((int)E, kChainColumns))
                                   : router_split_smem_bytes((int)E, (int)K);
@@ -1485,10 +1505,9 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
         return fail(JTMOE_EUNSUPPORTED, "router: E=%lld K=%lld needs %zu bytes of LDS", (long long)E, (long long)K, smem);
       // Two launches when one workgroup can hold the epilogue of the whole call: partial sums over
       // k slices from many workgroups, then the finishing workgroup.
-      const int finish_tok = router_smem_bytes((int)E, (int)K, 256) <= 160 * 1024 ? 256 : 64;
-      if (tokens > 0 && tokens <= finish_tok && router_smem_bytes((int)E, (int)K, finish_tok) <= 160 * 1024) {
-        const int slice_rows = router_slice_rows((int)H);
-        const int slices = chained ? 1 : (int)((H + slice_rows - 1) / slice_rows);
+      const int finish_tok = finish_tokens(E, K);
+      if (router_two_launches(tokens, E, K)) {
+        const int slices = chained ? 1 : router_slices(H);
         float* partial = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + router_scratch_bytes(E));
         if (chained) {
           const int pieces = chain_pieces(E);
@@ -1583,14 +1602,11 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
     // The walk grows with H and E, the second launch does not: a layer call gains, at 300 and 2560 tokens, E = 16: 5.4
     // and 4.0 us at 2048 columns, 1.7 and 1.6 at 1024, 0.8 and 0.2 at 768, 0 and -0.3 at 512; E = 256: 40 and 18, 20 and
     // 7, 13 and 6, 8 and 3.  The line is drawn where every expert count gains.
-    const int slice_rows = router_slice_rows((int)H);
-    const int slices = (int)((H + slice_rows - 1) / slice_rows);
-    if (layer && tokens <= kMidMaxTokens && H % kSplitKC == 0 && H >= 1024 &&
-        (size_t)slices * tokens * E * sizeof(float) <= layer->scratch_bytes) {
+    if (layer && router_middle(tokens, H, E, K, layer->scratch_bytes)) {
+      const int slices = router_slices(H);
       const size_t smem = (size_t)2 * kSplitKC * router_w_stride((int)E) * 2;
-      if (router_smem_bytes((int)E, (int)K, kFinishBlockTokens) <= 160 * 1024) {
-        float* const partial = static_cast<float*>(layer->scratch);
-        const int blocks = (int)((tokens + 15) / 16);
+      float* const partial = static_cast<float*>(layer->scratch);
+      const int blocks = (int)((tokens + 15) / 16);
 #define JT_PARTIAL_CASE(NB)                                                                                  \
   case NB * 16: {                                                                                            \
     auto kernel = router_mfma_split_kernel<NB, true>;                                                        \
@@ -1601,17 +1617,16 @@ int launch_router(const void* x, const void* w, const float* logits_in, const fl
         (float)route_scale, ids, static_cast<bf16_raw*>(weights), scores, logits_out, nullptr, partial,      \
         score_func);                                                                                         \
   } break;
-        switch ((int)E) {
-          JT_PARTIAL_CASE(1)
-          JT_PARTIAL_CASE(2)
-          JT_PARTIAL_CASE(4)
-          JT_PARTIAL_CASE(8)
-          JT_PARTIAL_CASE(16)
-        }
-#undef JT_PARTIAL_CASE
-        return launch_finish_blocks({partial, bias, slices, (int)tokens, (int)E, (int)K, score_func, (float)route_scale, ids,
-                                     static_cast<bf16_raw*>(weights), scores}, x, H, layer->shared, stream);
+      switch ((int)E) {
+        JT_PARTIAL_CASE(1)
+        JT_PARTIAL_CASE(2)
+        JT_PARTIAL_CASE(4)
+        JT_PARTIAL_CASE(8)
+        JT_PARTIAL_CASE(16)
       }
+#undef JT_PARTIAL_CASE
+      return launch_finish_blocks({partial, bias, slices, (int)tokens, (int)E, (int)K, score_func, (float)route_scale, ids,
+                                   static_cast<bf16_raw*>(weights), scores}, x, H, layer->shared, stream);
     }
     // four waves (64 tokens) per workgroup: the waves share the work of bringing in the router
     // matrix, which every workgroup reads in full
@@ -1866,6 +1881,41 @@ extern "C" size_t jtmoe_router_workspace_bytes(int64_t E) {
   if (E <= 0) return 0;
   // the statistics accumulators, the partial sums of the small-batch path, the arrival word of the decode launch
   return router_arrivals_offset(E) + 256;
+}
+
+extern "C" const char* jtmoe_shared_beside(int product, int64_t T, int64_t K, int64_t H, int64_t I, int64_t Is, int64_t E,
+                                           int compute_units) {
+  const int64_t limit = (int64_t)1 << 24;
+  if (product < 0 || product > 1 || T <= 0 || H <= 0 || I <= 0 || Is <= 0 || E <= 0 || K <= 0 || K > E || H >= limit ||
+      I >= limit || Is >= limit || E > JTMOE_MAX_EXPERTS || K > JTMOE_MAX_TOP_K || T * K >= ((int64_t)1 << 31) || compute_units < 0)
+    return "";
+  const double cus = compute_units > 0 ? compute_units : persistent_grid_size();
+  const SharedExperts none{nullptr, nullptr, nullptr, Is, nullptr, nullptr, nullptr, nullptr, I, false, false, false};
+  if (H % 8 != 0 || I % 8 != 0 || Is % 8 != 0 || decode_dense_supported(T, H, E, K, I, JTMOE_BF16) ||
+      router_takes_shared(nullptr, nullptr, none, T, H, E, K, JTMOE_BF16))
+    return "";
+  bool in_blocks = false, plan_done = false;  // as launch_router leaves the call
+  if (router_on_matrix_cores(nullptr, nullptr, H, E)) {
+    if (router_split(T, H, E)) {
+      const bool two = router_two_launches(T, E, K);
+      in_blocks = two && T * E >= kFinishInBlocks;
+      plan_done = two && !in_blocks;  // (or the statistics are)
+    } else {
+      in_blocks = !router_chained(H, E) && router_middle(T, H, E, K, (size_t)T * K * I * 2);
+    }
+  }
+  const bool dispatch = !plan_done && T * K <= kSmallLayerAssignments && T * H * 2 < ((int64_t)1 << 30);
+  const TileShape first = tiles_beside(Product::kGateUp, T, H, Is, I, E, K, in_blocks ? finish_front(T) : kDispatchFront, cus);
+  const bool by_router = in_blocks && first != TileShape::kPlain;
+  auto name = [](bool router, TileShape s) {
+    if (s == TileShape::kPlain) return "";
+    return s == TileShape::k64x64 ? (router ? "router 64x64" : "dispatch 64x64") : (router ? "router 128x64" : "dispatch 128x64");
+  };
+  if (product == 0) {
+    if (by_router) return name(true, first);
+    return dispatch ? name(false, tiles_beside(Product::kGateUp, T, H, Is, I, E, K, kDispatchFront, cus)) : "";
+  }
+  return dispatch && by_router ? name(false, tiles_beside(Product::kDown, T, H, Is, I, E, K, kDispatchFront, cus)) : "";
 }
 
 extern "C" int jtmoe_router(const void* x, const void* w_router, const float* expert_bias, int64_t T, int64_t H,

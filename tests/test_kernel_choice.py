@@ -12,11 +12,12 @@ import pytest
 
 import test_gpu_f32_gemm as f32
 import test_gpu_joint_products as joint
+import test_gpu_middle_batch_beside as beside
 import test_gpu_ragged_widths as ragged
 import test_gpu_row_bits as row_bits
 import test_gpu_tile_choice as tiles
 from kernel_choice import (DOWN, GATE_UP, MI355X_CUS, chosen, f32_backward_kernel, forward_kernels, gradient_kernels,
-                           joint_kernels)
+                           joint_kernels, joint_tiles, product_tiles, shared_beside, tiles as product_tile)
 from research_amd import build
 
 GATE_UP_KERNELS = {"stream_16x128", "stream_16x64", "stream_32x64", "rows64", "rows64_tail", "half", "half_tail", "rows256",
@@ -117,3 +118,27 @@ def test_joint_launches_deal_every_tile_once():
 def test_sizes_out_of_range_have_no_kernel():
     assert chosen(GATE_UP, 0, 64, 64, 1, MI355X_CUS) == chosen(4, 1, 64, 64, 1, MI355X_CUS) == ""
     assert chosen(GATE_UP, 1, 63, 64, 1, MI355X_CUS) == chosen(DOWN, 1, 64, 12, 1, MI355X_CUS) == "general"
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,top_k,d_ff,shared_width,gate_up,down", beside.SHAPES + [beside.RAGGED])
+def test_middle_batches_run_beside_the_launches_they_name(tokens, hidden, experts, top_k, d_ff, shared_width, gate_up, down):
+    assert shared_beside(tokens, top_k, hidden, d_ff, shared_width, experts) == [gate_up, down]
+
+
+def test_every_launch_and_tile_beside_it_is_checked():
+    launches = [f"{launch} {tile}" for launch in ("router", "dispatch") for tile in ("64x64", "128x64")]
+    assert {case[6] for case in beside.SHAPES} == {"", *launches}
+    assert {case[7] for case in beside.SHAPES} == {"", *launches[2:]}
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,top_k,inter,kernels,gradients", [case for case in tiles.GROUPED + ragged.SHAPES])
+def test_kernels_without_a_choice_of_tiles_name_themselves(tokens, hidden, experts, top_k, inter, kernels, gradients):
+    names = product_tiles(tokens * top_k, hidden, inter, experts)
+    for kernel, name in zip(kernels.split() + gradients.split(), names):
+        assert (name == kernel) == (kernel.startswith(("stream", "rows64", "rows256_short")))
+
+
+def test_sizes_out_of_range_have_no_tiles():
+    assert product_tile(GATE_UP, 0, 64, 64) == product_tile(4, 1, 64, 64) == ""
+    assert product_tile(GATE_UP, 1, 63, 64) == product_tile(DOWN, 1, 64, 12) == "general"
+    assert joint_tiles(0, 2, 512, 512, 512, 8) == [""] * 4 and shared_beside(300, 9, 512, 512, 512, 8) == ["", ""]
