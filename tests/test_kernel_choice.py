@@ -142,3 +142,22 @@ def test_sizes_out_of_range_have_no_tiles():
     assert product_tile(GATE_UP, 0, 64, 64) == product_tile(4, 1, 64, 64) == ""
     assert product_tile(GATE_UP, 1, 63, 64) == product_tile(DOWN, 1, 64, 12) == "general"
     assert joint_tiles(0, 2, 512, 512, 512, 8) == [""] * 4 and shared_beside(300, 9, 512, 512, 512, 8) == ["", ""]
+
+
+@pytest.mark.parametrize("rows,hidden,inter,experts,names", [
+    # what a taller tile spares against what it takes longer, by the measured sizes
+    (64 * 512, 2048, 1408, 64, "plain tall tall tall"),
+    (64 * 698, 2048, 1408, 64, "plain plain plain plain"),         # many rounds, hardly fewer tiles
+    (64 * 1024, 2048, 1408, 64, "tall tall plain plain"),          # fewer tiles; data gradients of many rounds
+    (128 * 688, 2048, 768, 128, "plain plain plain plain"),
+    (24 * 698, 1000, 2664, 24, "plain_tail 128x256 plain_tail 128x128_pair"),
+    (16 * 1375, 1024, 2816, 16, "tall plain plain plain"),         # five rounds for four of one data gradient
+])
+def test_taller_tiles_where_they_spare_more_than_they_cost(rows, hidden, inter, experts, names):
+    assert product_tiles(rows, hidden, inter, experts) == names.split()
+
+
+def test_taller_tiles_beside_dense_ones():
+    assert joint_tiles(2621, 8, 2048, 1408, 2816, 64) == ["separate", "plain", "separate", "plain"]  # five rounds for four
+    assert joint_tiles(2048, 8, 2048, 1408, 2816, 64)[0] == "tall"  # ... but with 3.4 rounds of tiles for 4.8
+    assert joint_tiles(4096, 8, 2048, 1408, 2816, 64)[0] == joint_tiles(5588, 8, 2048, 1408, 2816, 64)[0] == "tall"
