@@ -451,8 +451,8 @@ int dispatch_validate(const char* who, const int32_t* expert_ids, const void* x,
 // Where the fixed-point weight sums [E][chunks] of the layer's statistics start inside the scratch.
 inline size_t partial_imp_offset(int64_t A, int64_t E) { return jtmoe_dispatch_workspace_bytes(A, E); }
 
-// The one-workgroup dispatch takes, with the statistics, 7 us at 3096 assignments to 64 experts and 13.4 at 8192 to 8
-// (without them 6.4 and 8.5: their sums meet at few addresses), the two launches of the passes 12 and a gap whatever the
+// The one-workgroup dispatch takes, with the statistics, 7.6 us at 4096 assignments to 8 experts and 13 at 8192
+// (without them 5.4 and 8.4: their sums meet at few addresses), the two launches of the passes 12 and a gap whatever the
 // batch; a training pass at 8192 takes the same time either way.  (Only in the
 // layer, whose workspace belongs to the call: the entry points of their own keep to one workgroup, which leaves
 // their scratch alone, up to kSmallMaxAssignments.)

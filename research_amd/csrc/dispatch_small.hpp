@@ -4,9 +4,10 @@
 // moe.py:583-602).
 //
 // Latency bounds it.  A wave owns a run of consecutive assignments, so that the waves meet four times in all,
-// whatever the number of assignments, and the ids arrive kDispatchBatch loads at a time.  (In rounds of the whole
-// workgroup, with two meetings and a load each, 3096 assignments to 64 experts with statistics took 11.0 us, now 7.1;
-// without them 4.4 us at 320, 6.4 at 4096, 9.7 at 8192.)
+// whatever the number of assignments, and the ids arrive kDispatchBatch loads at a time.  us without statistics, in rounds
+// of the whole workgroup with two meetings and a load each / so; 64 experts, 6 assignments 3.3 / 3.2, 296 3.5 / 3.4, 3096
+// 8.4 / 5.5, 4096 9.1 / 6.0, 8192 16.3 / 9.4 (with the counts of the waves read one after the other and the ids a second time
+// 3.7, 3.8, 6.0, 6.4 and 9.7).
 //
 // The body is a device function so that two kernels can end in it: the stand-alone small dispatch,
 // and the last workgroup of the small-batch router, which then goes on from the ids it still holds
@@ -66,8 +67,8 @@ __device__ __forceinline__ void dispatch_small_body(const int32_t* ids, const WT
   __syncthreads();
   const int first = wave * run, end = min(first + run, A);
   int* const mine = next + wave * E;
+  int id[kDispatchBatch];  // (a run of one batch keeps its ids for the ranks)
   for (int base = first; base < end; base += kDispatchBatch * kWave) {
-    int id[kDispatchBatch];
     float w[kDispatchBatch];
 #pragma unroll
     for (int i = 0; i < kDispatchBatch; ++i) {
@@ -84,11 +85,15 @@ __device__ __forceinline__ void dispatch_small_body(const int32_t* ids, const WT
   }
   __syncthreads();
   // exclusive scan over the experts: thread e owns expert e
-  int of_wave[kWaves], count = 0;
+  // (the reads of a wave's threads without a condition, so that they are all on their way at once)
+  int of_wave[kWaves] = {}, count = 0;
+  if (wave * kWave < E) {
+    const int mine_or_last = min(tid, E - 1);
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) of_wave[w] = tid < E && w < waves ? next[w * E + tid] : 0;
+    for (int w = 0; w < kWaves; ++w) of_wave[w] = next[min(w, waves - 1) * E + mine_or_last];
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) count += of_wave[w];
+    for (int w = 0; w < kWaves; ++w) count += of_wave[w] = tid < E && w < waves ? of_wave[w] : 0;
+  }
   int incl = count;
 #pragma unroll
   for (int d = 1; d < kWave; d <<= 1) {
@@ -117,12 +122,12 @@ __device__ __forceinline__ void dispatch_small_body(const int32_t* ids, const WT
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   for (int base = first; base < end; base += kDispatchBatch * kWave) {
-    int id[kDispatchBatch];
+    if (run > kDispatchBatch * kWave)
 #pragma unroll
-    for (int i = 0; i < kDispatchBatch; ++i) {
-      const int a = base + i * kWave + lane;
-      id[i] = a < end ? ids[a] : -1;
-    }
+      for (int i = 0; i < kDispatchBatch; ++i) {
+        const int a = base + i * kWave + lane;
+        id[i] = a < end ? ids[a] : -1;
+      }
 #pragma unroll
     for (int i = 0; i < kDispatchBatch; ++i) {
       const int a = base + i * kWave + lane;
