@@ -295,7 +295,7 @@ int shared_backward_steps(const void* x, const void* dy, const SharedBackward& s
   const int64_t Is = sh.Is;
   int rc = JTMOE_OK;
   if (with_z)
-    rc = launch_gemm_nt(dtype, dy, nullptr, sh.down, nullptr, ws.dg, nullptr, nullptr, T, H, Is, 1, nullptr, 1, 0, 1, s);
+    rc = launch_gemm_nt(dtype, dy, nullptr, sh.down, nullptr, ws.dg, nullptr, nullptr, T, H, Is, 1, 1, s);
   if (rc) return rc;
   rc = dtype == JTMOE_BF16
            ? run_swiglu_backward<bf16_raw>(ws.dg, sh.gate_pre, sh.up_pre, nullptr, nullptr, T, Is, ws.du, ws.hw, nullptr, s)
@@ -307,7 +307,7 @@ int shared_backward_steps(const void* x, const void* dy, const SharedBackward& s
   rc = launch_gemm_tn(dtype, x, ws.dg, ws.du, sh.d_gate, sh.d_up, nullptr, nullptr, T, H, Is, 1, nullptr, 1, false,
                       false, 0, s, ws.split);
   if (rc || !with_dx) return rc;
-  rc = launch_gemm_nt(dtype, ws.dg, ws.du, sh.gate, sh.up, sh.dx, nullptr, nullptr, T, Is, H, 1, nullptr, 1, 0, 2, s);
+  rc = launch_gemm_nt(dtype, ws.dg, ws.du, sh.gate, sh.up, sh.dx, nullptr, nullptr, T, Is, H, 1, 2, s);
   return rc ? rc : check_launch("shared backward");
 }
 
@@ -343,8 +343,7 @@ int experts_backward_core(const void* x, const void* dy, const int32_t* source_o
   }
   // Z = dYp @ Wd[e]^T
   rc = joint_z ? launch_gemm_nt_joint(dtype, routed_z, group_sizes, offsets, E, shared_z, 1, s)
-               : launch_gemm_nt(dtype, ws.packed_dy, nullptr, down, nullptr, ws.dg, group_sizes, offsets, A, H, I, E,
-                                nullptr, 1, 0, 1, s);
+               : launch_gemm_nt(dtype, ws.packed_dy, nullptr, down, nullptr, ws.dg, group_sizes, offsets, A, H, I, E, 1, s);
   if (rc) return rc;
   rc = dtype == JTMOE_BF16 ? run_swiglu_backward<bf16_raw>(ws.dg, gate_pre, up_pre, source_order, weights, A, I, ws.du,
                                                            ws.hw, d_weights, s, group_sizes, offsets, E)
@@ -370,8 +369,7 @@ int experts_backward_core(const void* x, const void* dy, const int32_t* source_o
     }
     // dXp = dG @ Wg[e]^T + dU @ Wu[e]^T
     rc = joint_dx ? launch_gemm_nt_joint(dtype, routed_dx, group_sizes, offsets, E, shared_dx, 2, s)
-                  : launch_gemm_nt(dtype, ws.dg, ws.du, gate, up, ws.dxp, group_sizes, offsets, A, I, H, E, nullptr, 1, 0,
-                                   2, s);
+                  : launch_gemm_nt(dtype, ws.dg, ws.du, gate, up, ws.dxp, group_sizes, offsets, A, I, H, E, 2, s);
     if (rc) return rc;
   }
   if (shared && !joint_dx) {
@@ -411,8 +409,7 @@ int router_backward_impl(const void* x, const void* router_weight, const float* 
   rc = launch_gemm_tn(dtype, x, d_logits, nullptr, d_router_weight, nullptr, nullptr, nullptr, T, H, E, 1, nullptr, 1,
                       false, false, 0, s, ws.split);
   if (rc) return rc;
-  return launch_gemm_nt(dtype, d_logits, nullptr, router_weight, nullptr, dx, nullptr, nullptr, T, E, H, 1, nullptr, 1,
-                        0, 1, s);
+  return launch_gemm_nt(dtype, d_logits, nullptr, router_weight, nullptr, dx, nullptr, nullptr, T, E, H, 1, 1, s);
 }
 
 // the same for bf16, eight elements per thread, every byte touched once

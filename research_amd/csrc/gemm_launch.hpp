@@ -26,11 +26,10 @@ enum class ProductKernel {
 };
 
 // C[rows of group e, :] = sum over s < segs of A_s[rows of e, :] @ B_s[e]^T
-//   A_s: [rows, Kdim], or [a_rows, Kdim] read through row_map (row j -> row_map[j] / row_div)
-//   B_s: [E, N, Kdim]      C: [rows, N]      group_sizes == nullptr: one group holding every row
+//   A_s: [rows, Kdim]      B_s: [E, N, Kdim]      C: [rows, N]      group_sizes == nullptr: one group holding every row
 int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, const void* b1, void* c,
                    const int32_t* group_sizes, const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N,
-                   int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream);
+                   int64_t E, int segs, hipStream_t stream);
 // ... and the kernel it takes for bf16 operands (16-byte aligned, below 2 GiB) on `cus` compute units
 ProductKernel data_gradient_kernel(int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense, int segs, double cus);
 // ... in which tiles
@@ -38,7 +37,7 @@ enum class TileShape;
 TileShape data_gradient_tiles(ProductKernel k, int64_t rows, int64_t Kdim, int64_t N, int64_t E, bool dense, int segs, double cus);
 
 // The routed product above and the shared experts' one (one dense group of s.rows rows) in one launch.  Operands as in
-// launch_gemm_nt, without a row map; gemm_nt_joint: the kernel, or kGeneral where launches of their own are faster or
+// launch_gemm_nt; gemm_nt_joint: the kernel, or kGeneral where launches of their own are faster or
 // the operands ask for them.
 struct NtProblem {
   const void *a0, *a1, *b0, *b1;
@@ -77,8 +76,7 @@ int launch_f32_nn(const void* a, const void* b0, const void* b1, void* c, const 
                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, const int32_t* row_map,
                   int row_div, int64_t a_rows, void* save0, void* save1, hipStream_t stream);
 int launch_f32_nt(const void* a0, const void* a1, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
-                  const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, const int32_t* row_map,
-                  int row_div, int64_t a_rows, int segs, hipStream_t stream);
+                  const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, int segs, hipStream_t stream);
 int launch_f32_tn(const void* p, const void* d0, const void* d1, void* c0, void* c1, const int32_t* group_sizes,
                   const int32_t* offsets, int64_t rows, int64_t KA, int64_t N, int64_t E, void* split_ws,
                   hipStream_t stream);

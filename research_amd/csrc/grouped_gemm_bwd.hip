@@ -22,18 +22,15 @@ template <typename T>
 __global__ __launch_bounds__(256) void gemm_nt_staged_kernel(
     const T* __restrict__ A0, const T* __restrict__ A1, const T* __restrict__ B0, const T* __restrict__ B1,
     T* __restrict__ C, const int32_t* __restrict__ group_sizes, const int32_t* __restrict__ offsets, int E,
-    int dense_rows, int Kdim, int N, int ntiles_n, const int32_t* __restrict__ row_map, int row_div, int segs) {
+    int dense_rows, int Kdim, int N, int ntiles_n, int segs) {
   __shared__ float As[QK][QB + 1];
   __shared__ float Bs[QK][QB + 1];
-  __shared__ int a_row_of[QB];
   const int mt = blockIdx.x / ntiles_n;
   const int nt = blockIdx.x - mt * ntiles_n;
   const TileRows tr = find_tile_wave(mt, QB, group_sizes, offsets, E, dense_rows);
   if (tr.rows <= 0) return;
   const int n0 = nt * QB;
   const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-  if (tid < tr.rows) a_row_of[tid] = row_map ? row_map[tr.row0 + tid] / row_div : tr.row0 + tid;
-  __syncthreads();
   float acc[4][4] = {};
   for (int s = 0; s < segs; ++s) {
     const T* A = s ? A1 : A0;
@@ -42,7 +39,7 @@ __global__ __launch_bounds__(256) void gemm_nt_staged_kernel(
       for (int idx = tid; idx < QB * QK; idx += 256) {
         const int r = idx / QK, k = idx - r * QK;
         const int gk = k0 + k;
-        As[k][r] = (r < tr.rows && gk < Kdim) ? Elem<T>::load(A + (size_t)a_row_of[r] * Kdim + gk) : 0.0f;
+        As[k][r] = (r < tr.rows && gk < Kdim) ? Elem<T>::load(A + (size_t)(tr.row0 + r) * Kdim + gk) : 0.0f;
         Bs[k][r] = (n0 + r < N && gk < Kdim) ? Elem<T>::load(B + (size_t)(n0 + r) * Kdim + gk) : 0.0f;
       }
       __syncthreads();
@@ -147,8 +144,7 @@ constexpr int64_t kOperandLimit = (int64_t)1 << 30;  // elements: byte offsets s
 
 template <typename Cfg>
 int launch_nt_fast(const void* a0, const void* a1, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
-                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, const int32_t* row_map,
-                   int row_div, int64_t a_rows, int segs, hipStream_t stream) {
+                   const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, int segs, hipStream_t stream) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   auto kernel = grouped_gemm_nt_kernel<Cfg>;
@@ -165,7 +161,7 @@ int launch_nt_fast(const void* a0, const void* a1, const void* b0, const void* b
   kernel<<<(unsigned)grid, Cfg::NT, Cfg::SMEM_BYTES, stream>>>(
       static_cast<const uint16_t*>(a0), static_cast<const uint16_t*>(a1), static_cast<const uint16_t*>(b0),
       static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim,
-      (int)N, (int)mtiles, (int)nt, row_map, row_div, (int)a_rows, segs);
+      (int)N, (int)mtiles, (int)nt, segs);
   return JTMOE_OK;
 }
 
@@ -173,7 +169,7 @@ int launch_nt_fast(const void* a0, const void* a1, const void* b0, const void* b
 template <typename Cfg>
 int launch_nt_stream(const void* a0, const void* a1, const void* b0, const void* b1, void* c,
                      const int32_t* group_sizes, const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N,
-                     int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream) {
+                     int64_t E, int segs, hipStream_t stream) {
   using L = StreamLayout<Cfg>;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
@@ -191,7 +187,7 @@ int launch_nt_stream(const void* a0, const void* a1, const void* b0, const void*
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes, stream>>>(
       static_cast<const uint16_t*>(a0), static_cast<const uint16_t*>(a1), static_cast<const uint16_t*>(b0),
       static_cast<const uint16_t*>(b1), static_cast<uint16_t*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim,
-      (int)N, (int)nt, row_map, row_div, (int)a_rows, segs, ps.window, ps.chunk);
+      (int)N, (int)nt, segs, ps.window, ps.chunk);
   return JTMOE_OK;
 }
 
@@ -299,13 +295,13 @@ int launch_gemm_nt_joint(int dtype, const NtProblem& p, const int32_t* group_siz
 
 int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, const void* b1, void* c,
                    const int32_t* group_sizes, const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N,
-                   int64_t E, const int32_t* row_map, int row_div, int64_t a_rows, int segs, hipStream_t stream) {
+                   int64_t E, int segs, hipStream_t stream) {
   if (rows == 0) return JTMOE_OK;
   const bool dense = group_sizes == nullptr;
-  const bool fast = dtype == JTMOE_BF16 && (row_map ? a_rows : rows) * Kdim < kOperandLimit && aligned16(a0) &&
+  const bool fast = dtype == JTMOE_BF16 && rows * Kdim < kOperandLimit && aligned16(a0) &&
                     aligned16(b0) && (segs == 1 || (aligned16(a1) && aligned16(b1))) && aligned16(c);
 #define JT_NT(LAUNCH, CFG) \
-  LAUNCH<CFG>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div, a_rows, segs, stream)
+  LAUNCH<CFG>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, segs, stream)
   const ProductKernel k = fast ? data_gradient_kernel(rows, Kdim, N, E, dense, segs, persistent_grid_size()) : ProductKernel::kGeneral;
   if (k != ProductKernel::kGeneral) {
     const bool tail = k == ProductKernel::kRows256Tail;
@@ -317,10 +313,8 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
     }
   }
 #undef JT_NT
-  if (dtype == JTMOE_F32 && f32_gemm_supported(a0, a1, b0, b1, c, row_map ? a_rows : rows, Kdim, N) &&
-      !(row_map && segs > 1))
-    return launch_f32_nt(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map, row_div, a_rows, segs,
-                         stream);
+  if (dtype == JTMOE_F32 && f32_gemm_supported(a0, a1, b0, b1, c, rows, Kdim, N))
+    return launch_f32_nt(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, segs, stream);
   const int64_t mtiles = dense ? (rows + QB - 1) / QB : max_m_tiles(rows, E, QB);
   const int64_t nt = (N + QB - 1) / QB;
   if (mtiles * nt >= ((int64_t)1 << 31)) return fail(JTMOE_EUNSUPPORTED, "grouped gemm (nt): grid too large");
@@ -328,12 +322,12 @@ int launch_gemm_nt(int dtype, const void* a0, const void* a1, const void* b0, co
     gemm_nt_staged_kernel<bf16_raw><<<(unsigned)(mtiles * nt), 256, 0, stream>>>(
         static_cast<const bf16_raw*>(a0), static_cast<const bf16_raw*>(a1), static_cast<const bf16_raw*>(b0),
         static_cast<const bf16_raw*>(b1), static_cast<bf16_raw*>(c), group_sizes, offsets, (int)E, (int)rows,
-        (int)Kdim, (int)N, (int)nt, row_map, row_div, segs);
+        (int)Kdim, (int)N, (int)nt, segs);
   else
     gemm_nt_staged_kernel<float><<<(unsigned)(mtiles * nt), 256, 0, stream>>>(
         static_cast<const float*>(a0), static_cast<const float*>(a1), static_cast<const float*>(b0),
         static_cast<const float*>(b1), static_cast<float*>(c), group_sizes, offsets, (int)E, (int)rows, (int)Kdim,
-        (int)N, (int)nt, row_map, row_div, segs);
+        (int)N, (int)nt, segs);
   return JTMOE_OK;
 }
 

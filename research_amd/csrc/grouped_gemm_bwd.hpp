@@ -14,9 +14,7 @@
 //         reduction index as the row, so both tiles use the 4 x 16 block layout and are
 //         read with the transposing ds_read_b64_tr_b16.  An empty group yields zeros.
 //
-// Either kernel can fetch operand rows through a row map (packed row j reads row
-// row_map[j] / row_div), the way the forward gate/up launch does, so neither the
-// permuted activations nor the permuted output gradient are ever written to memory.
+// TN can fetch operand rows through a row map (packed row j reads row row_map[j] / row_div).
 //
 // NT: with OPT & 65536 K need not be a multiple of the 64-deep step (chunks past the end of a row read as zeros).
 //
@@ -48,14 +46,14 @@ struct NtGemmCfg {
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
 };
 
-// A0/A1: [rows, Kdim] (or [a_rows, Kdim] fetched through row_map); B0/B1: [E, N, Kdim];
+// A0/A1: [rows, Kdim]; B0/B1: [E, N, Kdim];
 // C: [rows, N].  segs = 1 uses A0/B0 only; segs = 2 adds A1 @ B1^T into the same output.
 template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_nt_kernel(
     const uint16_t* __restrict__ A0, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes,
     const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int mtiles, int ntiles_n,
-    const int32_t* __restrict__ row_map, int row_div, int a_rows, int segs) {
+    int segs) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT;
   constexpr int TM = Cfg::TM, TN = Cfg::TN, WM = Cfg::WM, WN = Cfg::WN;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -63,7 +61,6 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_nt_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WAVES_N, wn = wave - wm * Cfg::WAVES_N;
-  const bool gather = row_map != nullptr;
 
   // Persistent workgroups, as in grouped_gemm_dma_persistent_kernel: this one walks the tiles
   // idx, idx + stride, ... of its XCD's contiguous range of the logical order.
@@ -116,11 +113,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_nt_kernel(
   auto row_offsets = [&](const Tile& t, int* voff) {
 #pragma unroll
     for (int j = 0; j < Cfg::A_LOADS; ++j) {
-      const int r = l_r + j * (NT / 8);
-      if (gather)
-        voff[j] = r < t.rows ? ((row_map[t.row0 + r] / row_div) * Kdim + l_c * 8) * 2 : 0x70000000;
-      else
-        voff[j] = (r * Kdim + l_c * 8) * 2;
+      voff[j] = ((l_r + j * (NT / 8)) * Kdim + l_c * 8) * 2;
     }
   };
   auto plan = [&](const Tile& t, const int* voff) {
@@ -133,7 +126,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_nt_kernel(
         a = A0;
         b = B0;
       }
-      a_rsrc[s] = gather ? make_rsrc(a, a_rows * Kdim * 2) : make_rsrc(a + (size_t)t.row0 * Kdim, t.rows * Kdim * 2);
+      a_rsrc[s] = make_rsrc(a + (size_t)t.row0 * Kdim, t.rows * Kdim * 2);
       // rows of B past N lie outside the descriptor and read as zeros
       b_rsrc[s] = make_rsrc(b + wofs, N * Kdim * 2);
     }

@@ -99,12 +99,11 @@ int launch_f32_nn(const void* a, const void* b0, const void* b1, void* c, const 
 }
 
 int launch_f32_nt(const void* a0, const void* a1, const void* b0, const void* b1, void* c, const int32_t* group_sizes,
-                  const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, const int32_t* row_map,
-                  int row_div, int64_t a_rows, int segs, hipStream_t stream) {
+                  const int32_t* offsets, int64_t rows, int64_t Kdim, int64_t N, int64_t E, int segs, hipStream_t stream) {
   const bool dense = group_sizes == nullptr;
 #define JT_F32(BM, BN)                                                                                       \
-  launch_f32<F32Cfg<BM, BN, false, true>>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, row_map,    \
-                                          row_div, a_rows, segs, nullptr, nullptr, stream)
+  launch_f32<F32Cfg<BM, BN, false, true>>(a0, a1, b0, b1, c, group_sizes, offsets, rows, Kdim, N, E, nullptr, 1,  \
+                                          rows, segs, nullptr, nullptr, stream)
   return f32_cost(dense, rows, E, N, 128, 128, 4) <= f32_cost(dense, rows, E, N, 64, 64, 1) ? JT_F32(128, 128)
                                                                                             : JT_F32(64, 64);
 #undef JT_F32

@@ -602,10 +602,10 @@ template <typename Cfg>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_stream_nt_kernel(
     const uint16_t* __restrict__ A0, const uint16_t* __restrict__ A1, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, const int32_t* __restrict__ group_sizes,
-    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int ntiles_n,
-    const int32_t* __restrict__ row_map, int row_div, int a_rows, int segs, int window, int chunk) {
+    const int32_t* __restrict__ offsets, int E, int dense_rows, int Kdim, int N, int ntiles_n, int segs,
+    int window, int chunk) {
   stream_gemm_body<Cfg, true>(A0, A1, B0, B1, C, group_sizes, offsets, E, dense_rows, Kdim, N, ntiles_n,
-                              row_map, row_div, a_rows, nullptr, nullptr, segs, window, chunk, DenseProblem{});
+                              nullptr, 1, 0, nullptr, nullptr, segs, window, chunk, DenseProblem{});
 }
 
 template <typename Cfg>

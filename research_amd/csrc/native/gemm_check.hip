@@ -361,7 +361,7 @@ static void launch_stream_nt_cfg(Problem& p, const uint16_t* A1, int segs, bool 
   if (g_workgroups) ps = {g_workgroups, 0, 0};
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes>>>(
       p.A, A1, p.B0, p.B1, p.C, dense ? nullptr : p.dgs, dense ? nullptr : p.doff, p.E, p.rows, p.K, p.N, (int)nt,
-      p.top_k > 0 ? p.dmap : nullptr, p.top_k > 0 ? p.top_k : 1, p.a_rows, segs, ps.window, ps.chunk);
+      segs, ps.window, ps.chunk);
 }
 static void launch_stream_nt(Problem& p, const uint16_t* A1, int segs, bool dense) {
   if (g_stream_nt == 2) return launch_stream_nt_cfg<DgradStream32Cfg>(p, A1, segs, dense);
@@ -370,6 +370,7 @@ static void launch_stream_nt(Problem& p, const uint16_t* A1, int segs, bool dens
 
 template <typename Cfg>
 static void launch_nt(Problem& p, const uint16_t* A1, int segs, bool dense) {
+  if (p.a_rows != p.rows) { printf("nt kernels read a row per packed row\n"); exit(1); }
   if (g_stream_nt) return launch_stream_nt(p, A1, segs, dense);
   auto kernel = grouped_gemm_nt_kernel<Cfg>;
   CK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -381,7 +382,7 @@ static void launch_nt(Problem& p, const uint16_t* A1, int segs, bool dense) {
   const long tiles_grid = gemm_grid(mt, nt);
   kernel<<<(unsigned)(!g_one_tile_per_workgroup && tiles_grid > 256 ? 256 : tiles_grid), Cfg::NT, Cfg::SMEM_BYTES>>>(
       p.A, A1, p.B0, p.B1, p.C, dense ? nullptr : p.dgs, dense ? nullptr : p.doff, p.E, p.rows, p.K, p.N, (int)mt,
-      (int)nt, p.top_k > 0 ? p.dmap : nullptr, p.top_k > 0 ? p.top_k : 1, p.a_rows, segs);
+      (int)nt, segs);
 }
 
 // B0 / B1 of the problem are read as [E, N, K] here
@@ -499,10 +500,13 @@ static void time_backward() {
     hipFree(s0); hipFree(s1);
     release(p);
   }
-  {  // d act = dy[token of row] @ Wd^T : A gathered [T, H], B [E, I, H]
+  {  // d act = dy @ Wd^T : A [rows, H], B [E, I, H]
+    Problem p = make(E, rows, H, I, 21, false, 0, 1.0f);
+    time_launches("dgrad down (dy @ Wd^T)", 2.0 * rows * H * I, 10, [&] { launch_nt<DgradCfg>(p, nullptr, 1, false); });
+    release(p);
+  }
+  {  // dWg, dWu = x[token of row]^T @ (dG, dU) : P gathered [T, H]
     Problem p = make(E, rows, H, I, 21, false, topk, 1.0f);
-    time_launches("dgrad down (gathered dy @ Wd^T)", 2.0 * rows * H * I, 10, [&] { launch_nt<DgradCfg>(p, nullptr, 1, false); });
-    // dWg, dWu = x[token of row]^T @ (dG, dU)
     uint16_t* D0 = random_bf16((size_t)rows * I, 31, 1.0f);
     uint16_t* D1 = random_bf16((size_t)rows * I, 32, 1.0f);
     uint16_t *C0, *C1;
@@ -707,7 +711,6 @@ int main(int argc, char** argv) {
   }
   {
     Problem p = make(5, 2400, 512, 384, 12, true, 3, 1.0f);
-    ok &= check_nt<DgradCfg>("dgrad gather on load", p, 1);
     ok &= check_tn<WgradDualGatherCfg>("wgrad dual, transposed operand gathered", p, 1);
     ok &= check_tn<WgradGatherCfg>("wgrad, other operand gathered", p, 2);
     release(p);
@@ -753,8 +756,8 @@ int main(int argc, char** argv) {
     ok &= check_nt<DgradCfg>("dgrad many tiles per workgroup", u, 1);
     ok &= check_nt<DgradCfg>("dgrad many tiles per workgroup, two segments", u, 2);
     release(u);
-    Problem v = make(9, 20000, 64, 520, 29, true, 3, 1.0f);  // one k step, gathered rows
-    ok &= check_nt<DgradCfg>("dgrad one k step, gather on load", v, 1);
+    Problem v = make(9, 20000, 64, 520, 29, true, 0, 1.0f);
+    ok &= check_nt<DgradCfg>("dgrad one k step", v, 1);
     release(v);
   }
   {
@@ -839,9 +842,6 @@ int main(int argc, char** argv) {
     ok &= check_nt<DgradCfg>("stream dgrad ragged", w1, 1);
     ok &= check_nt<DgradCfg>("stream dgrad ragged, two segments", w1, 2);
     release(w1);
-    Problem w2 = make(5, 2400, 512, 384, 62, true, 3, 1.0f);
-    ok &= check_nt<DgradCfg>("stream dgrad gather on load", w2, 1);
-    release(w2);
     Problem w3 = make(1, 777, 512, 520, 63, false, 0, 1.0f);
     ok &= check_nt<DgradCfg>("stream dgrad dense, two segments", w3, 2, true);
     release(w3);
@@ -849,8 +849,8 @@ int main(int argc, char** argv) {
     ok &= check_nt<DgradCfg>("stream dgrad many tiles per workgroup", w4, 1);
     ok &= check_nt<DgradCfg>("stream dgrad many tiles per workgroup, two segments", w4, 2);
     release(w4);
-    Problem w5 = make(33, 90000, 128, 392, 65, true, 4, 1.0f);  // 4 k steps per segment: two segments just fill the pipeline
-    ok &= check_nt<DgradCfg>("stream dgrad short segments, gather", w5, 2);
+    Problem w5 = make(33, 90000, 128, 392, 65, true, 0, 1.0f);  // 4 k steps per segment: two segments just fill the pipeline
+    ok &= check_nt<DgradCfg>("stream dgrad short segments", w5, 2);
     release(w5);
     }
     g_stream_nt = 0;
