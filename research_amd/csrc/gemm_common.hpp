@@ -329,19 +329,18 @@ inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, doub
 // Beyond, 128-row tiles (128 x 256 with one output) where they take no more rounds: 12 groups of 333 rows, 1280 x 1792,
 // two rounds either way: gate/up 62 / 50, three for two 53 / 55 (8192 rows, 1024 x 2048).
 // kTall: 256-row tiles of up to 320 rows (a kernel of their own, which without such rows is slower than the others' by up to
-// 5 %, for data gradients by 8 % and more); else plain ones.  By the spread of the groups, where they spare rounds enough for
-// the time a taller tile takes: 1.2 of a plain one, 1.3 for one data gradient alone, 1.25 for products of one output beside
-// dense tiles, which fill the last round of either, unless the tiles themselves are fewer by as much.  us, plain / taller
-// (rounds): 64 groups of 256 rows, 2048 x 1408, gate/up 262 / 213, down 128 / 119, dX 247 / 239; of 328 gate/up 294 / 288 (6, 5),
-// beside shared tiles down 208 / 218 and dX 346 / 369 (5, 4; by tiles 4.3, 3.4); of 256, gate/up beside shared tiles, the forward
-// pass 493 / 460 (5, 4; 4.8, 3.4); of 512 down 212 / 189 and dX 414 / 357 (5, 4), dZ 221 / 194 (4, 3), but gate/up, which the line
-// leaves out, 383 / 336 (7, 6); dZ of 16 groups of 1375, 1024 x 2816, 135 / 145, of 40 of 1638, 1304 x 904, 228 / 260 (5, 4), of
-// 24 of 698, 1000 x 2664, 125 / 145 (4, 3, with 94 % of the tiles).
-// Forward products of eight rounds and more: the tiles that are left count, and the kernel decides from the real sizes.  64
-// groups of 698 rows (94 % of the tiles) gate/up 471 / 487, of 1024 (85 %) 700 / 652 and down 403 / 392, of 2048 (88 %) 1287 /
-// 1248 and 744 / 736; 128 skewed groups of 688 (93 %), 2048 x 768, down 341 / 357.  Beside shared tiles, where the plain kernel
-// is slower too, always, gradients as well: 64 groups of 698 590 / 581.  Gradients alone gain little there: 64 groups of 1024 dX
-// 758 / 732 (9, 8), of 2048 1337 / 1372 (18, 15), dZ of 1375 495 / 510 (9, 8), 128 skewed groups of 1024 dX 810 / 855 (18, 16).
+// 5 %); else plain ones.  By the spread of the groups, where they spare rounds enough for the time a taller tile takes: 1.2 of a
+// plain one, 1.25 for one data gradient alone, which has to spare a tenth of the tiles as well, and for products of one output
+// beside dense tiles, which fill the last round of either, unless the tiles themselves are fewer by as much.  us, plain /
+// taller (rounds): 64 groups of 256 rows, 2048 x 1408, gate/up 262 / 213, down 128 / 119, dX 247 / 239; of 328 gate/up 294 /
+// 288 (6, 5), beside shared tiles down 208 / 218 and dX 346 / 369 (5, 4; by tiles 4.3, 3.4); of 256, gate/up beside shared
+// tiles, the forward pass 493 / 460 (5, 4; 4.8, 3.4); of 512 down 212 / 189 and dX 419 / 356 (5, 4), dZ 229 / 200 (4, 3), but
+// gate/up, which the line leaves out, 383 / 336 (7, 6); dZ of 64 groups of 600 258 / 265, of 40 of 1638, 1304 x 904, 233 / 235 (5,
+// 4), of 24 of 698, 1000 x 2664, 134 / 138 (4, 3, with 94 % of the tiles).
+// With eight rounds and more the tiles that are left count, and the kernel decides from the real sizes: 64 groups of 698 rows
+// (94 % of the tiles) gate/up 471 / 487, of 1024 (85 %) 700 / 652, down 403 / 392 and dX 782 / 700, of 2048 (88 %) 1287 / 1248,
+// 744 / 736 and 1361 / 1307; 128 skewed groups of 688 (93 %), 2048 x 768, down 341 / 357, dX 591 / 606, of 1024 (85 %) dX 835 /
+// 817.  Beside shared tiles, where the plain kernel is slower too, always: 64 groups of 698 590 / 581.
 // k128x128Pair: two workgroups to a CU.
 enum class TileShape { k64x64, k128x64, k128x128, k128x128Short, k128x128Pair, k256x128, k128x256, kTall, kPlain };
 enum class Product { kGateUp, kDown, kGradient, kGradientPair };  // the last: of two segments
@@ -368,14 +367,12 @@ inline TileShape tile_shape(Product product, int64_t rows, int64_t E, bool dense
     return dual ? TileShape::k128x128 : product == Product::kDown ? TileShape::k128x256 : TileShape::k128x128Pair;
   const double tall = tall_mtiles(rows, E, dense, true) * nt + (double)group_mtiles((int)dense_rows, 256, 64) * dense_nt;
   const bool fewer = tall <= 0.9 * plain;
-  const bool gradient = product == Product::kGradient || product == Product::kGradientPair;
-  const bool many = rounds(plain) >= kManyRounds;
-  if (many && !(alone && gradient)) return !alone || fewer ? TileShape::kTall : TileShape::kPlain;
+  if (rounds(plain) >= kManyRounds) return !alone || fewer ? TileShape::kTall : TileShape::kPlain;
   const double low = std::fmax(expected_mtiles(rows, E, dense, 128), spread_mtiles(rows, E, dense, 128)) * nt +
                      (double)((dense_rows + 127) / 128) * dense_nt;
-  if (!many && rounds(low) <= rounds(plain) && 0.72 * rounds(low) < 1.2 * rounds(tall)) return dual ? TileShape::k128x128 : TileShape::k128x256;
+  if (rounds(low) <= rounds(plain) && 0.72 * rounds(low) < 1.2 * rounds(tall)) return dual ? TileShape::k128x128 : TileShape::k128x256;
   const bool one_gradient = alone && product == Product::kGradient;
-  const double longer = alone ? (one_gradient ? 1.3 : 1.2) : (dual || 1.3 * tall < plain ? 1.2 : 1.25);
+  const double longer = one_gradient || (!alone && !dual && 1.3 * tall >= plain) ? 1.25 : 1.2;
   return longer * rounds(tall) < rounds(plain) && (fewer || !one_gradient) ? TileShape::kTall : TileShape::kPlain;
 }
 // ... with a reduction of `steps` 64-deep steps at least, of which a kernel wants twice as many as it has stages, and, for

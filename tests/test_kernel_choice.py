@@ -148,7 +148,7 @@ def test_sizes_out_of_range_have_no_tiles():
     # what a taller tile spares against what it takes longer, by the measured sizes
     (64 * 512, 2048, 1408, 64, "plain tall tall tall"),
     (64 * 698, 2048, 1408, 64, "plain plain plain plain"),         # many rounds, hardly fewer tiles
-    (64 * 1024, 2048, 1408, 64, "tall tall plain plain"),          # fewer tiles; data gradients of many rounds
+    (64 * 1024, 2048, 1408, 64, "tall tall plain tall"),           # fewer tiles; seven rounds of dZ for six
     (128 * 688, 2048, 768, 128, "plain plain plain plain"),
     (24 * 698, 1000, 2664, 24, "plain_tail 128x256 plain_tail 128x128_pair"),
     (16 * 1375, 1024, 2816, 16, "tall plain plain plain"),         # five rounds for four of one data gradient
