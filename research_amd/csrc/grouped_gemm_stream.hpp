@@ -103,7 +103,7 @@ __device__ __forceinline__ void stream_gemm_body(
   constexpr int CPRA = Cfg::CPRA, KK = BK / 16, LPS = Cfg::LPS;
   constexpr int kBand = Cfg::SUBW / 64;  // 4 x 64 blocks of B side by side in a sub-tile
   constexpr bool kDual = Cfg::kDual;
-  // X: rows that a group's last tile may have beyond BM, a block of 32 more per wave.  The row blocks of a wave then lie
+  // X: rows that a tile may have beyond BM, a block of 32 more per wave.  The row blocks of a wave then lie
   // kRowStep apart, those of the waves above one another in turn; without such rows they are neighbours, so that waves
   // without rows leave the LDS to the others (two blocks of each wave are bound by its reads: down of 333 rows a group 55.8
   // us in turn, 54.3 as neighbours).
@@ -115,13 +115,7 @@ __device__ __forceinline__ void stream_gemm_body(
   // K may end inside a step (the interleaved steady part leaves no room for a branch: every load checks)
   constexpr bool kTail = (Cfg::OPT & 65536) != 0;
   static_assert(!kNT || (BN * CPRA) % NT == 0, "the B tile must divide evenly over the threads");
-  // Timing experiments of the stand-alone check's time_ablation mode, which bounds what any schedule of
-  // this loop can reach (wrong results by construction, never launched by the library): OPT & 256 leaves out the operand loads of the steady part of the k loop, OPT & 512 its
-  // fragment reads (the MFMAs then run on the fragments read once before the loop).
-  // OPT & 1024 makes every load of the steady part fetch the tile's first k step again (operands that
-  // are in the nearest cache: the cost of issuing the loads without the memory system behind them).
-  constexpr bool kNoLoads = (Cfg::OPT & 256) != 0, kNoFragReads = (Cfg::OPT & 512) != 0;
-  constexpr bool kSameTile = (Cfg::OPT & 1024) != 0;
+  static_assert(X == 0 || NS == 2, "the waits count the load of the X rows only where they drain everything");
   extern __shared__ __align__(16) unsigned char smem_raw[];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -160,7 +154,7 @@ __device__ __forceinline__ void stream_gemm_body(
   // which they are the cheaper work.
   int extra = 0, real_mtiles = mtiles_with(0), dense_mtiles = kJoint ? group_mtiles(dp.rows, BM, 0) : 0;
   if (X != 0) {
-    const int workgroups = chunk > 0 ? 8 * window : (int)gridDim.x - first_block;
+    const int workgroups = (int)gridDim.x - first_block;  // (one for the whole launch each: chunk 0)
     auto rounds = [&](int mt, int dense_mt) {
       return (mt * ntiles_n + (kJoint ? dense_mt * dp.ntiles * lead : 0) + workgroups - 1) / workgroups;
     };
@@ -425,7 +419,6 @@ __device__ __forceinline__ void stream_gemm_body(
   bf16x8_t af[2][TM], bf[2][TN];
   wait_and_barrier<(NS - 1) * LPS>();
   load_frags(0, 0, af[0], bf[0]);
-  if (kNoFragReads) load_frags(0, 1, af[1], bf[1]);
   int cs = 0;  // stage of the current k step
 
   while (true) {
@@ -450,7 +443,7 @@ __device__ __forceinline__ void stream_gemm_body(
     // matrix cores what its rows need, to two blocks of a wave.  (Accumulators that lived on from one of these forms to
     // the next would not stay in the same registers, and hundreds would be spilled: each has its own, from the zeros to
     // the epilogue.)
-    const bool x_rows = pl.x, second = second_product(cur);
+    const bool second = second_product(cur);
     auto run_tile = [&](auto nb) {
       constexpr int NB = decltype(nb)::value, kMfmas = NB * TN;
       f32x16_t acc[NB > 0 ? NB : 1][TN];
@@ -474,13 +467,13 @@ __device__ __forceinline__ void stream_gemm_body(
       };
       // a step: with the loads of step `ahead` of the planned tile, or (kLoads = false) as the one before `left` others that end
       // the launch
-      auto step = [&](auto loads_tag, int ahead, bool x_loads, int left) {
+      auto step = [&](auto loads_tag, int ahead, int left) {
         constexpr bool kLoads = decltype(loads_tag)::value;
         // sub-steps 0 .. KK-2: the fragments of the following sub-step are requested, then this one's MFMAs, which the
         // scheduler interleaves with the LDS reads (two per MFMA)
 #pragma unroll
         for (int kk = 0; kk < KK - 1; ++kk) {
-          if (NB > 0 && !kNoFragReads)
+          if (NB > 0)
 #pragma unroll
             for (int f = 0; f < NB + TN; ++f) read((kk + 1) & 1, cs, kk + 1, f);
 #pragma unroll
@@ -494,10 +487,7 @@ __device__ __forceinline__ void stream_gemm_body(
         }
         // the next step's stage has arrived (own loads: the wait; everyone's: the barrier), and every
         // wave holds its last fragments of the current stage, which is therefore free
-        // (a stage is LPS loads, with X rows one more)
-        if (X != 0 && NS > 2 && x_loads)
-          wait_and_barrier<(NS - 2) * (LPS + 1)>();
-        else if (kLoads || left == NS - 1)
+        if (kLoads || left == NS - 1)
           wait_and_barrier<(NS - 2) * LPS>();
         else if (NS > 3 && left == NS - 2)
           wait_and_barrier<(NS > 3 ? NS - 3 : 0) * LPS>();
@@ -506,25 +496,25 @@ __device__ __forceinline__ void stream_gemm_body(
         __builtin_amdgcn_sched_barrier(0);
         // last sub-step, in a fixed order: after each of its MFMAs operand loads of step `ahead` (into the stage just
         // released) and fragment reads of the next step are issued
-        const int ns = (NS & (NS - 1)) == 0 ? (cs + 1) & (NS - 1) : cs + 1 == NS ? 0 : cs + 1, kt = kSameTile ? 0 : ahead;
+        const int ns = (NS & (NS - 1)) == 0 ? (cs + 1) & (NS - 1) : cs + 1 == NS ? 0 : cs + 1;
         constexpr int kSlots = kMfmas > 0 ? kMfmas : 1;
         constexpr int kLoadsPer = (LPS + kSlots - 1) / kSlots, kFragsPer = (NB + TN + kSlots - 1) / kSlots;
 #pragma unroll
         for (int g = 0; g < kSlots; ++g) {
           if (NB > 0) mfma((KK - 1) & 1, g);
           __builtin_amdgcn_sched_barrier(0);
-          if (kLoads && !kNoLoads) {
+          if (kLoads) {
 #pragma unroll
             for (int q = 0; q < kLoadsPer; ++q)
-              if (g * kLoadsPer + q < LPS) issue_one(pl, kt, cs, g * kLoadsPer + q);
+              if (g * kLoadsPer + q < LPS) issue_one(pl, ahead, cs, g * kLoadsPer + q);
           }
-          if (NB > 0 && !kNoFragReads)
+          if (NB > 0)
 #pragma unroll
             for (int q = 0; q < kFragsPer; ++q)
               if (g * kFragsPer + q < NB + TN) read(0, ns, 0, g * kFragsPer + q);
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (kLoads && !kNoLoads) issue_x(pl, kt, cs);
+        if (kLoads) issue_x(pl, ahead, cs);
         cs = ns;
       };
       // all steps but the last NS, then, with the next tile's plan, those: their loads are its first steps'
@@ -541,13 +531,12 @@ __device__ __forceinline__ void stream_gemm_body(
             plan_nothing(pl);
           }
         }
-        const bool x_loads = x_rows && !part;  // (part 1: of some stages, then of others)
-        for (int j = j0; j < j1; ++j) step(std::true_type{}, j + ahead, x_loads, 0);
+        for (int j = j0; j < j1; ++j) step(std::true_type{}, j + ahead, 0);
       }
       if constexpr (kOwnEnd) {
         if (!have_next) {
 #pragma unroll 1
-          for (int left = NS - 1; left >= 0; --left) step(std::false_type{}, 0, false, left);
+          for (int left = NS - 1; left >= 0; --left) step(std::false_type{}, 0, left);
         }
       }
       // epilogue: straight from the accumulators to memory (no LDS, no barrier)

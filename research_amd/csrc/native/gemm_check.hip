@@ -141,9 +141,10 @@ static void release(Problem& p) {
 // here), unless g_one_tile_per_workgroup asks for the plain kernel.
 static bool g_one_tile_per_workgroup = false;
 static int g_chunk = -1;  // tiles per workgroup of a persistent launch; -1: as the library chooses
-// the stream kernel's 256-row tiles with 32-deep steps in four stages (the library: 64-deep ones in two)
-using GateUpStream32Cfg = DmaGemmCfg<256, 128, 32, 2, 4, true, 4, 16 + 128 + 131072>;
-using DownStream32Cfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + 131072>;
+static int stream_chunk(int xrows) { return xrows ? 0 : g_chunk < 0 ? 4 : g_chunk; }
+// the library's 256-row tiles without rows beyond these: gate/up and down with 32-deep steps in four stages
+using GateUpPlain = GateUpPlainCfg<false, false>;
+using DownPlain = DownPlainCfg<false>;
 static int g_workgroups = 0;  // launch the stream kernel with so many persistent workgroups
 
 // the stream kernel (grouped_gemm_stream.hpp): one software pipeline through all tiles of a workgroup
@@ -158,7 +159,7 @@ static void launch_stream(Problem& p, bool dense) {
   auto kernel = grouped_gemm_stream_kernel<Cfg>;
   CK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                          (int)L::kSmemBytes));
-  PersistentSchedule ps = persistent_schedule(tiles_grid, 256, g_chunk < 0 ? kTilesPerWorkgroup<Cfg> : g_chunk);
+  PersistentSchedule ps = persistent_schedule(tiles_grid, 256, stream_chunk(Cfg::XROWS));
   if (tiles_grid <= 256) ps = {tiles_grid, 0, 0};
   if (g_workgroups) ps = {g_workgroups, 0, 0};
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes>>>(
@@ -340,8 +341,7 @@ static bool compare(const char* name, const float* dref, const uint16_t* dgot, s
 }
 
 // the transposed-B form of the stream kernel (what the library launches for the data gradients where it fits)
-static int g_stream_nt = 0;  // 0: the older kernel; 1: DgradStreamCfg; 2: 32-deep steps in four stages
-using DgradStream32Cfg = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 131072>;
+static int g_stream_nt = 0;  // 0: the older kernel; 1: DgradStreamCfg; 2: DgradPlainCfg
 template <typename Cfg>
 static void launch_stream_nt_cfg(Problem& p, const uint16_t* A1, int segs, bool dense) {
   using L = StreamLayout<Cfg>;
@@ -356,7 +356,7 @@ static void launch_stream_nt_cfg(Problem& p, const uint16_t* A1, int segs, bool 
                         : (p.rows + Cfg::BM - 1) / Cfg::BM + (p.E < p.rows ? p.E : p.rows);
   const long nt = (p.N + Cfg::BN - 1) / Cfg::BN;
   const long tiles_grid = gemm_grid(mt, nt);
-  PersistentSchedule ps = persistent_schedule(tiles_grid, 256, g_chunk < 0 ? kTilesPerWorkgroup<Cfg> : g_chunk);
+  PersistentSchedule ps = persistent_schedule(tiles_grid, 256, stream_chunk(Cfg::XROWS));
   if (tiles_grid <= 256) ps = {tiles_grid, 0, 0};
   if (g_workgroups) ps = {g_workgroups, 0, 0};
   kernel<<<(unsigned)ps.grid, Cfg::NT, L::kSmemBytes>>>(
@@ -364,8 +364,11 @@ static void launch_stream_nt_cfg(Problem& p, const uint16_t* A1, int segs, bool 
       segs, ps.window, ps.chunk);
 }
 static void launch_stream_nt(Problem& p, const uint16_t* A1, int segs, bool dense) {
-  if (g_stream_nt == 2) return launch_stream_nt_cfg<DgradStream32Cfg>(p, A1, segs, dense);
-  launch_stream_nt_cfg<DgradStreamCfg>(p, A1, segs, dense);
+  switch (g_stream_nt) {
+    case 1: return launch_stream_nt_cfg<DgradStreamCfg>(p, A1, segs, dense);
+    case 2: return launch_stream_nt_cfg<DgradPlainCfg<false>>(p, A1, segs, dense);
+    default: printf("stream nt: no variant %d\n", g_stream_nt); exit(1);
+  }
 }
 
 template <typename Cfg>
@@ -784,12 +787,12 @@ int main(int argc, char** argv) {
     Problem p = make(7, 3001, 576, 392, 51, true, 0, 1.0f);
     ok &= check<GateUpStreamCfg>("stream gate/up ragged", p);
     ok &= check<DownStreamCfg>("stream down ragged", p);
-    ok &= check<GateUpStream32Cfg>("stream 4 x 32 gate/up ragged", p);
-    ok &= check<DownStream32Cfg>("stream 4 x 32 down ragged", p);
+    ok &= check<GateUpPlain>("stream plain gate/up ragged", p);
+    ok &= check<DownPlain>("stream plain down ragged", p);
     release(p);
     Problem q = make(5, 2400, 512, 384, 52, true, 3, 1.0f);
     ok &= check<GateUpStreamCfg>("stream gate/up gather on load", q);
-    ok &= check<GateUpStream32Cfg>("stream 4 x 32 gate/up gather on load", q);
+    ok &= check<GateUpPlain>("stream plain gate/up gather on load", q);
     release(q);
     Problem r = make(1, 777, 512, 520, 53, false, 0, 1.0f);
     ok &= check<GateUpStreamCfg>("stream gate/up dense", r, true);
@@ -798,11 +801,11 @@ int main(int argc, char** argv) {
     Problem u = make(40, 70000, 256, 264, 54, true, 0, 1.0f);  // many more tiles than workgroups
     ok &= check<GateUpStreamCfg>("stream gate/up many tiles per workgroup", u);
     ok &= check<DownStreamCfg>("stream down many tiles per workgroup", u);
-    ok &= check<DownStream32Cfg>("stream 4 x 32 down many tiles per workgroup", u);
+    ok &= check<DownPlain>("stream plain down many tiles per workgroup", u);
     release(u);
     Problem v = make(33, 90000, 256, 392, 55, true, 4, 1.0f);  // the same with gathered rows (row map by LDS-DMA)
     ok &= check<GateUpStreamCfg>("stream gate/up many tiles, gather", v);
-    ok &= check<GateUpStream32Cfg>("stream 4 x 32 gate/up many tiles, gather", v);
+    ok &= check<GateUpPlain>("stream plain gate/up many tiles, gather", v);
     g_chunk = 0;
     ok &= check<GateUpStreamCfg>("stream gate/up many tiles, gather, one workgroup per CU", v);
     g_chunk = -1;
@@ -815,11 +818,11 @@ int main(int argc, char** argv) {
     Problem x = make((int)g_sizes.size(), edge_rows, 512, 264, 56, false, 0, 1.0f);
     ok &= check<GateUpStreamCfg>("stream gate/up, edges of tiles", x);
     ok &= check<DownStreamCfg>("stream down, edges of tiles", x);
-    ok &= check<DownStream32Cfg>("stream 4 x 32 down, edges of tiles", x);
+    ok &= check<DownPlain>("stream plain down, edges of tiles", x);
     g_stream_nt = 1;
     ok &= check_nt<DgradCfg>("stream dgrad, edges of tiles", x, 2);
-    g_stream_nt = 4;
-    ok &= check_nt<DgradCfg>("stream dgrad 4 x 32, edges of tiles", x, 2);
+    g_stream_nt = 2;
+    ok &= check_nt<DgradCfg>("stream dgrad plain, edges of tiles", x, 2);
     g_stream_nt = 0;
     release(x);
     Problem y = make((int)g_sizes.size(), edge_rows, 256, 392, 57, false, 2, 1.0f);
@@ -861,17 +864,13 @@ int main(int argc, char** argv) {
     Problem d = make(64, 131072, 1408, 2048, 5, false, 0, 1.0f);
     for (int rep = 0; rep < 3; ++rep) {
       g_stream = false;
-      timeit<GateUpCfg>("gate/up library", g, 20);
-      timeit<DownCfg>("down library", d, 20);
+      timeit<GateUpCfg>("gate/up, older kernel", g, 20);
+      timeit<DownCfg>("down, older kernel", d, 20);
       g_stream = true;
-      timeit<GateUpStreamCfg>("gate/up stream 2 x 64 (library)", g, 20);
-      timeit<DownStreamCfg>("down stream 2 x 64", d, 20);
-      timeit<GateUpStream32Cfg>("gate/up stream 4 x 32", g, 20);
-      timeit<DownStream32Cfg>("down stream 4 x 32", d, 20);
-      g_chunk = 0;
-      timeit<GateUpStreamCfg>("gate/up stream 2 x 64, one wg per CU", g, 20);
-      timeit<DownStreamCfg>("down stream 2 x 64, 4 tiles per wg", d, 20);
-      g_chunk = -1;
+      timeit<GateUpStreamCfg>("gate/up stream, up to 320 rows (library)", g, 20);
+      timeit<DownStreamCfg>("down stream, up to 320 rows (library)", d, 20);
+      timeit<GateUpPlain>("gate/up stream, plain", g, 20);
+      timeit<DownPlain>("down stream, plain", d, 20);
       g_stream = false;
     }
     release(g); release(d);
@@ -879,10 +878,10 @@ int main(int argc, char** argv) {
     Problem sq = make(1, 8192, 8192, 8192, 6, false, 0, 1.0f);
     for (int rep = 0; rep < 2; ++rep) {
       g_stream = false;
-      timeit<DownCfg>("8192^3 library", sq, 10);
+      timeit<DownCfg>("8192^3, older kernel", sq, 10);
       g_stream = true;
-      timeit<DownStreamCfg>("8192^3 stream 2 x 64", sq, 10);
-      timeit<DownStream32Cfg>("8192^3 stream 4 x 32", sq, 10);
+      timeit<DownStreamCfg>("8192^3 stream, up to 320 rows", sq, 10);
+      timeit<DownPlain>("8192^3 stream, plain", sq, 10);
       g_stream = false;
     }
     release(sq);
@@ -894,7 +893,7 @@ int main(int argc, char** argv) {
     Problem x = make(E, rows, I, H, 22, false, 0, 1.0f);   // dXp = dG @ Wg^T + dU @ Wu^T : A [rows, I] twice, B [E, H, I] twice
     uint16_t* A1 = random_bf16((size_t)rows * I, 33, 1.0f);
     for (int rep = 0; rep < 3; ++rep) {
-      const char* names[3] = {"older kernel", "stream 2 x 64", "stream 4 x 32"};
+      const char* names[3] = {"older kernel", "stream, up to 320 rows", "stream, plain"};
       for (g_stream_nt = 0; g_stream_nt <= 2; ++g_stream_nt) {
         char label[96];
         snprintf(label, sizeof label, "Z = dYp @ Wd^T, %s", names[g_stream_nt]);
@@ -923,8 +922,8 @@ int main(int argc, char** argv) {
     }
     release(d);
     // the gate/up launch of the same configuration (gathered rows, K = 1024, N = 2816: 72 x 22 tiles of
-    // 256 x 128 + 128, 6.2 per CU) with the stream kernel's workgroups holding 4 tiles (library), 3, 2, 1,
-    // or one workgroup per CU walking its share (0)
+    // 256 x 128 + 128, 6.2 per CU) in plain tiles, with the stream kernel's workgroups holding 4 of them (as the library
+    // launches these), 3, 2, 1, or one workgroup per CU walking its share (0)
     {
       Problem g2 = make(16, 16384, 1024, 2816, 6, false, 2, 1.0f);
       g_stream = true;
@@ -932,15 +931,15 @@ int main(int argc, char** argv) {
         for (int chunk : {-1, 0, 1, 2, 3}) {
           g_chunk = chunk;
           char name[64];
-          snprintf(name, sizeof name, "C2 gate/up stream, %d tiles per workgroup", chunk < 0 ? 4 : chunk);
-          timeit_cold<GateUpStreamCfg>(name, g2, 20);
+          snprintf(name, sizeof name, "C2 gate/up stream, plain, %d tiles per workgroup", chunk < 0 ? 4 : chunk);
+          timeit_cold<GateUpPlain>(name, g2, 20);
         }
       g_chunk = -1;
-      // the same launch with 64-deep steps in two stages, and with the older kernel
+      // the same launch in tiles of up to 320 rows, and with the older kernel
       for (int rep = 0; rep < 3; ++rep) {
         g_stream = true;
-        timeit_cold<GateUpStreamCfg>("C2 gate/up stream 2 x 64 (library)", g2, 20);
-        timeit_cold<GateUpStream32Cfg>("C2 gate/up stream 4 x 32", g2, 20);
+        timeit_cold<GateUpStreamCfg>("C2 gate/up stream, up to 320 rows", g2, 20);
+        timeit_cold<GateUpPlain>("C2 gate/up stream, plain", g2, 20);
         g_stream = false;
         timeit_cold<GateUpCfg>("C2 gate/up, older kernel", g2, 20);
       }
@@ -953,17 +952,6 @@ int main(int argc, char** argv) {
       timeit<Half>("C3 down, 256 x 128 tiles", d3, 20);
     }
     release(d3);
-  }
-  if (ok && argc > 1 && !strcmp(argv[1], "time_prio")) {
-    using Prio = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 32>;
-    Problem g = make(64, 131072, 2048, 1408, 4, false, 8, 1.0f);
-    g_stream = true;
-    for (int rep = 0; rep < 3; ++rep) {
-      timeit<GateUpStreamCfg>("gate/up stream", g, 20);
-      timeit<Prio>("gate/up stream, wave priority around the MFMAs", g, 20);
-    }
-    g_stream = false;
-    release(g);
   }
   if (ok && argc > 1 && !strcmp(argv[1], "time_ragged")) {
     // What the ragged last tile of every group costs: the C3 launches on groups of random sizes
@@ -985,42 +973,6 @@ int main(int argc, char** argv) {
     }
     release(g); release(d); release(ge); release(de);
   }
-  if (ok && argc > 1 && !strcmp(argv[1], "time_ablation")) {
-    // What bounds the stream kernel: the same launch with parts of the k loop left out (results are
-    // wrong by construction), on N(0,1) x N(0,0.05) operands and on all-zero operands.  Dense problems
-    // (one group), one workgroup per CU.
-    using Full = GateUpStreamCfg;
-    using NoLoads = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 256>;
-    using NoFrags = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 512>;
-    using MfmaOnly = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 256 + 512>;
-    using SqFull = DownStreamCfg;
-    using SqNoLoads = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + 256>;
-    using SqNoFrags = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + 512>;
-    using SqMfmaOnly = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + 256 + 512>;
-    using SameTile = DmaGemmCfg<256, 128, 32, 4, 2, true, 4, 16 + 128 + 1024>;
-    using SqSameTile = DmaGemmCfg<256, 256, 32, 2, 4, false, 4, 16 + 128 + 32768 + 1024>;
-    g_stream = true;
-    g_chunk = 0;
-    for (float scale : {1.0f, 0.0f}) {
-      printf("-- operand data: %s\n", scale > 0 ? "N(0,1) activations, N(0,0.05) weights" : "all zeros");
-      Problem gd = make(1, 131072, 2048, 1408, 4, false, 0, scale);
-      timeit<Full>("gate/up dense: whole kernel", gd, 10);
-      timeit<NoLoads>("gate/up dense: no operand loads", gd, 10);
-      timeit<NoFrags>("gate/up dense: no fragment reads", gd, 10);
-      timeit<MfmaOnly>("gate/up dense: MFMAs and barriers only", gd, 10);
-      timeit<SameTile>("gate/up dense: loads of one cached k step", gd, 10);
-      release(gd);
-      Problem sq = make(1, 8192, 8192, 8192, 6, false, 0, scale);
-      timeit<SqFull>("8192^3: whole kernel", sq, 10);
-      timeit<SqNoLoads>("8192^3: no operand loads", sq, 10);
-      timeit<SqNoFrags>("8192^3: no fragment reads", sq, 10);
-      timeit<SqMfmaOnly>("8192^3: MFMAs and barriers only", sq, 10);
-      timeit<SqSameTile>("8192^3: loads of one cached k step", sq, 10);
-      release(sq);
-    }
-    g_chunk = -1;
-    g_stream = false;
-  }
   if (ok && argc > 1 && !strcmp(argv[1], "counters_stream")) {
     // a few launches of each kernel for a hardware-counter run (rocprofv3 --pmc ... -- gemm_check counters_stream nocheck)
     Problem g = make(64, 131072, 2048, 1408, 4, false, 8, 1.0f);
@@ -1033,7 +985,7 @@ int main(int argc, char** argv) {
       launch<DownCfg>(sq, false);
       g_stream = true;
       launch<GateUpStreamCfg>(g, false);
-      launch<GateUpStream32Cfg>(g, false);
+      launch<GateUpPlain>(g, false);
       launch<DownStreamCfg>(sq, false);
       g_stream = false;
     }
@@ -1144,10 +1096,10 @@ int main(int argc, char** argv) {
         snprintf(name, sizeof name, "%s down, library", sh.name);
         timeit_cold<DownCfg>(name, d, 20);
         g_stream = true;
-        snprintf(name, sizeof name, "%s down, stream 2 x 64", sh.name);
+        snprintf(name, sizeof name, "%s down, stream, up to 320 rows", sh.name);
         timeit_cold<DownStreamCfg>(name, d, 20);
-        snprintf(name, sizeof name, "%s down, stream 4 x 32", sh.name);
-        timeit_cold<DownStream32Cfg>(name, d, 20);
+        snprintf(name, sizeof name, "%s down, stream, plain", sh.name);
+        timeit_cold<DownPlain>(name, d, 20);
         g_stream = false;
         snprintf(name, sizeof name, "%s down, results from accumulators", sh.name);
         timeit_cold<DownDirect>(name, d, 20);
@@ -1182,8 +1134,8 @@ int main(int argc, char** argv) {
       for (int chunk : {0, 1, 2, 4, 8}) {
         g_chunk = chunk;
         char name[80];
-        snprintf(name, sizeof name, "gate/up stream, %d tiles per workgroup", chunk);
-        if (timing) timeit<GateUpStreamCfg>(name, g, 20); else launch<GateUpStreamCfg>(g, false);
+        snprintf(name, sizeof name, "gate/up stream, plain, %d tiles per workgroup", chunk);
+        if (timing) timeit<GateUpPlain>(name, g, 20); else launch<GateUpPlain>(g, false);
       }
       g_chunk = 4;
       if (timing) {
