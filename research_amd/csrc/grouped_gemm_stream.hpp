@@ -696,8 +696,11 @@ TileShape tiles_beside(Product product, int64_t T, int64_t H, int64_t Is, int64_
 SharedTiles shared_gate_up_beside(const void* x, const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front);
 SharedTiles shared_down_beside(const SharedExperts& s, int64_t T, int64_t H, int64_t E, int64_t K, int front);
 
+// (Also in router.hip, whose flags round divisions correctly and contract nothing.  A gate/up product of a whole reduction
+// has the same bits there: silu_rcp neither divides nor adds to a product.  One that divides would not.)
 template <typename Cfg>
 __device__ __forceinline__ void dense_stream_tiles(const DenseProblem& p, int front) {
+  static_assert(!Cfg::kDual || (Cfg::OPT & 65536) == 0, "gate/up of whole reductions only");
   stream_gemm_body<Cfg, false>(p.a0, nullptr, p.b0, p.b1, p.c, nullptr, nullptr, 1, p.rows, p.k, p.n, p.ntiles, nullptr, 1,
                                0, p.save0, p.save1, 1, 0, 0, DenseProblem{}, front);
 }
