@@ -1,5 +1,5 @@
-"""Norm and combine with a wave per 512 columns of a row: bits of a wave per row.  Rows of one wave and of eight, with
-ends inside a wave, and batches on either side of the line between the two forms of the combine."""
+"""Norm and combine with a wave per 512 columns of a row: bits of a wave per row.  Rows of two waves to eight, with
+ends inside a wave, and batches on either side of the line between the two forms of either."""
 
 from __future__ import annotations
 
@@ -11,13 +11,25 @@ from research_amd import ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("hidden", [8, 504, 512, 520, 2048, 3080, 4096])
+@pytest.mark.parametrize("hidden", [520, 1024, 2048, 3080, 4096])
 def test_norm(gpu, hidden):
     generator = torch.Generator(device=gpu).manual_seed(hidden)
     x = torch.randn(67, hidden, generator=generator, device=gpu).to(torch.bfloat16)
     scale = torch.randn(hidden + 1, generator=generator, device=gpu)
     # a scale that starts between two 16-byte boundaries takes the kernel of a wave per row
     assert torch.equal(ops.rmsnorm(x, scale[1:].clone(), 1e-6), ops.rmsnorm(x, scale[1:], 1e-6))
+
+
+@pytest.mark.parametrize("hidden", [520, 1032, 3080, 4096])
+def test_norm_of_the_most_rows(gpu, hidden):
+    """As many rows as a workgroup each takes, and one more: the bits of any of them alone."""
+    generator = torch.Generator(device=gpu).manual_seed(hidden)
+    most = 8192 // ((hidden + 511) // 512)
+    x = torch.randn(most + 1, hidden, generator=generator, device=gpu).to(torch.bfloat16)
+    scale = torch.randn(hidden, generator=generator, device=gpu)
+    over = ops.rmsnorm(x, scale, 1e-6)
+    assert torch.equal(ops.rmsnorm(x[:most].contiguous(), scale, 1e-6), over[:most])
+    assert torch.equal(ops.rmsnorm(x[most - 5:].contiguous(), scale, 1e-6), over[most - 5:])
 
 
 @pytest.mark.parametrize("top_k", [1, 2, 8])

@@ -1,7 +1,8 @@
 """256-row tiles of up to 320 rows, and part-filled ones beside them: every row has the bits of its group alone.
 
 The group sizes stand on either side of what tiles take beyond 256 rows (64 each, from a group's first tile on) and of
-the row blocks that a part-filled tile leaves out; taller tiles spare a round in each of the four products named.
+the row blocks that a part-filled tile leaves out; taller tiles spare a round in each of the products named, which
+tests/test_kernel_choice.py holds to the rules.
 """
 
 from __future__ import annotations
@@ -16,12 +17,16 @@ pytestmark = pytest.mark.gpu
 SIZES = (257, 320, 577, 1100, 0, 1279, 1025, 1, 300, 65, 2303, 33)
 
 
-@pytest.mark.parametrize("hidden,inter", [
-    (256, 4096),  # gate/up and dZ: the fewest whole steps
-    (264, 4104),  # ... whose last step holds one chunk
-    (4096, 256),  # down and dX
-    (4104, 264),
-])
+WIDTHS = [
+    # ..., the products (gate/up, down, dZ, dX) that take them
+    (256, 4096, (0, 2)),  # the fewest whole steps
+    (264, 4104, (0, 2)),  # ... whose last step holds one chunk
+    (4096, 256, (1, 3)),
+    (4104, 264, (1, 3)),
+]
+
+
+@pytest.mark.parametrize("hidden,inter", [widths[:2] for widths in WIDTHS])
 def test_rows_have_the_bits_of_their_group_alone(gpu, hidden, inter):
     generator = torch.Generator(device=gpu).manual_seed(hidden)
 

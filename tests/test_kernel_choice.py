@@ -1,7 +1,8 @@
 """The rules that deal the expert products to kernels, asked on the CPU for a device of 256 compute units.
 
 What the GPU tests say about the kernels they exercise is checked here without a GPU, and that between them they
-exercise every kernel, so that a change of a rule cannot take a kernel's last test away unseen.
+exercise every kernel, so that a change of a rule cannot take a kernel's last test away unseen.  The tiles within a
+kernel are held to one another's bits, each of them, and some of each product's to the oracle.
 """
 
 from __future__ import annotations
@@ -15,7 +16,9 @@ import test_gpu_joint_products as joint
 import test_gpu_middle_batch_beside as beside
 import test_gpu_ragged_widths as ragged
 import test_gpu_row_bits as row_bits
+import test_gpu_tall_tiles as tall
 import test_gpu_tile_choice as tiles
+import test_gpu_tile_shapes as shapes
 from kernel_choice import (DOWN, GATE_UP, MI355X_CUS, chosen, f32_backward_kernel, forward_kernels, gradient_kernels,
                            joint_kernels, joint_tiles, product_tiles, shared_beside, tiles as product_tile)
 from research_amd import build
@@ -161,3 +164,50 @@ def test_taller_tiles_beside_dense_ones():
     assert joint_tiles(2621, 8, 2048, 1408, 2816, 64) == ["separate", "plain", "separate", "plain"]  # five rounds for four
     assert joint_tiles(2048, 8, 2048, 1408, 2816, 64)[0] == "tall"  # ... but with 3.4 rounds of tiles for 4.8
     assert joint_tiles(4096, 8, 2048, 1408, 2816, 64)[0] == joint_tiles(5588, 8, 2048, 1408, 2816, 64)[0] == "tall"
+
+
+def with_tails(*names):
+    return {name + tail for name in names for tail in ("", "_tail")}
+
+
+LARGE = with_tails("tall", "plain")
+GATE_UP_TILES = with_tails("64x64", "128x64", "128x128", "128x128_short") | LARGE
+DOWN_TILES = {"64x64", "128x64", "128x128", "128x128_short", "128x128_pair", "256x128", "128x256"} | LARGE
+GRADIENT_TILES = DOWN_TILES - {"128x128_short"}
+
+
+def test_every_tile_is_held_to_the_bits_of_the_others():
+    """... which the GPU test takes, by the rows of a dense call and by the tokens of a layer call."""
+    alone, joint_ones = [set() for _ in range(4)], [set() for _ in range(4)]
+
+    def add(sets, names):
+        for seen, name in zip(sets, names):
+            seen.add(name)
+
+    for hidden, inter, rows in shapes.DENSE:
+        for n in rows:
+            add(alone, product_tiles(n, hidden, inter))
+    for hidden, inter, shared, experts, top_k, tokens in shapes.LAYERS:
+        for n in tokens:
+            add(alone, product_tiles(n * top_k, hidden, inter, experts))
+            if shared:
+                add(alone, product_tiles(n, hidden, shared))
+                add(joint_ones, joint_tiles(n, top_k, hidden, inter, shared, experts))
+    for seen, names in zip(alone, (GATE_UP_TILES, DOWN_TILES, GRADIENT_TILES, GRADIENT_TILES)):
+        assert seen >= names
+    pair = {"128x128_pair"}
+    for seen, names in zip(joint_ones, (GATE_UP_TILES, DOWN_TILES - pair, GRADIENT_TILES - pair, GRADIENT_TILES - pair)):
+        assert seen == names | {"separate"}
+
+
+@pytest.mark.parametrize("hidden,inter,tall_ones", tall.WIDTHS)
+def test_rows_beyond_256_spare_a_round_of_the_products_named(hidden, inter, tall_ones):
+    def mtiles(n, extra):  # as the kernels count them
+        whole = max(1, n // 256)
+        return whole + (n - whole * 256 > extra * whole) if n else 0
+
+    names = product_tiles(sum(tall.SIZES), hidden, inter, len(tall.SIZES))
+    columns = -(-inter // 128), -(-hidden // 256), -(-inter // 256), -(-hidden // 256)
+    for product, (name, across) in enumerate(zip(names, columns)):
+        plain, taller = (-(-across * sum(mtiles(n, extra) for n in tall.SIZES) // MI355X_CUS) for extra in (0, 64))
+        assert (name.startswith("tall") and taller < plain) == (product in tall_ones)
