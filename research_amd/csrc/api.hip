@@ -686,7 +686,7 @@ static int moe_forward_impl(const void* x, const void* w_router, const float* ex
     rc = router_for_layer(x, w_router, expert_bias, T, H, E, K, route_scale, dtype, expert_ids, weights, scores,
                           expert_counts, importance, group_sizes, offsets, source_order, inverse, w.router,
                           w.router_bytes, score_func, &stats_done, &plan_done, main_stream, w.act, w.act_bytes,
-                          offer_shared ? &shared : nullptr);
+                          offer_shared && gather ? &shared : nullptr);
     if (rc) return rc;
     stage_mark(kStageRouter, main_stream);
     rc = dispatch_for_layer(expert_ids, weights, (T > 0 && !gather) ? x : nullptr, T, H, E, K, dtype, group_sizes,

@@ -1891,7 +1891,7 @@ extern "C" const char* jtmoe_shared_beside(int product, int64_t T, int64_t K, in
     return "";
   const double cus = compute_units > 0 ? compute_units : persistent_grid_size();
   const SharedExperts none{nullptr, nullptr, nullptr, Is, nullptr, nullptr, nullptr, nullptr, I, false, false, false};
-  if (H % 8 != 0 || I % 8 != 0 || Is % 8 != 0 || decode_dense_supported(T, H, E, K, I, JTMOE_BF16) ||
+  if (H % 8 != 0 || I % 8 != 0 || Is % 8 != 0 || T * H * 2 >= ((int64_t)1 << 30) || decode_dense_supported(T, H, E, K, I, JTMOE_BF16) ||
       router_takes_shared(nullptr, nullptr, none, T, H, E, K, JTMOE_BF16))
     return "";
   bool in_blocks = false, plan_done = false;  // as launch_router leaves the call
@@ -1904,7 +1904,7 @@ extern "C" const char* jtmoe_shared_beside(int product, int64_t T, int64_t K, in
       in_blocks = !router_chained(H, E) && router_middle(T, H, E, K, (size_t)T * K * I * 2);
     }
   }
-  const bool dispatch = !plan_done && T * K <= kSmallLayerAssignments && T * H * 2 < ((int64_t)1 << 30);
+  const bool dispatch = !plan_done && T * K <= kSmallLayerAssignments;
   const TileShape first = tiles_beside(Product::kGateUp, T, H, Is, I, E, K, in_blocks ? finish_front(T) : kDispatchFront, cus);
   const bool by_router = in_blocks && first != TileShape::kPlain;
   auto name = [](bool router, TileShape s) {

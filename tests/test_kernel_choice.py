@@ -128,6 +128,12 @@ def test_middle_batches_run_beside_the_launches_they_name(tokens, hidden, expert
     assert shared_beside(tokens, top_k, hidden, d_ff, shared_width, experts) == [gate_up, down]
 
 
+@pytest.mark.parametrize("hidden,gate_up", [(2**19 - 128, "router 64x64"), (2**19, "")])
+def test_layers_that_copy_their_rows_leave_shared_products_alone(hidden, gate_up):
+    """x of 1 GiB or more: the routed products read a copy, and the shared ones run behind them."""
+    assert shared_beside(1024, 2, hidden, 1984, 576, 16)[0] == gate_up
+
+
 def test_every_launch_and_tile_beside_it_is_checked():
     launches = [f"{launch} {tile}" for launch in ("router", "dispatch") for tile in ("64x64", "128x64")]
     assert {case[6] for case in beside.SHAPES} == {"", *launches}
