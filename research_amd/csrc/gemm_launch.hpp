@@ -7,8 +7,9 @@
 
 namespace jtmoe {
 
-// The bf16 kernel of a product, as the dispatch rules choose it (jtmoe_product_kernel names them).  "Tail": K ends
-// inside a step, or a gate/up product that divides (silu_gate).
+// The bf16 kernel of a product, as the dispatch rules choose it (jtmoe_product_kernel names them), or a family of tiles of
+// which tile_shape then picks one (jtmoe_product_tiles).  "Tail": K ends inside a step, or a gate/up product that divides
+// (silu_gate).
 enum class ProductKernel {
   kGeneral,
   kStream16x128,  // grouped_gemm_skinny.hpp: tiles of 16 or 32 rows
@@ -16,12 +17,12 @@ enum class ProductKernel {
   kStream32x64,
   kRows64,        // 64-row LDS tiles, non-temporal loads of the matrix
   kRows64Tail,
-  kHalf,          // 128 x 128 tiles, or smaller ones where these leave CUs idle (tile_shape)
+  kHalf,          // where 128 x 128 tiles have a CU each; down and gradients in short steps, or two tiles to a CU
   kHalfTail,
-  kHalfDeep,
-  kRows256,       // 256-row tiles, or what suits the launch better (tile_shape)
+  kHalfDeep,      // down: two 128 x 128 tiles to a CU pay; gradients: they have a CU each
+  kRows256,       // beyond
   kRows256Tail,
-  kRows256Short,  // gate/up whose reduction is too short for four stages
+  kRows256Short,  // gate/up whose reduction is too short for the stream kernel
   kRows256ShortTail,
 };
 
