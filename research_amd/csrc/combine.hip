@@ -263,10 +263,11 @@ namespace {
 // latency and the CUs in use bound the kernel.  us, a wave per row / split; 2048 wide, top-8: 1 token 6.2 / 4.0, 37 5.8 /
 // 4.2, 387 with the norm 10.8 / 6.6, 2048 with the norm 23.5 / 17.4, 4096 27.0 / 25.4 and 30.6 / 28.2 with the norm; beyond,
 // at the memory's rate, either way within 4 %: 8192 tokens 54.0 / 53.7, of top-4 28.0 / 28.8, 4096 of 4096 columns 49.2 / 51.8,
-// 16384 of 1024 columns top-2 17.0 / 17.7.  Rows of two waves, in turn on one box, cold: 1024 columns top-2 with shared rows
-// 1200 tokens 4.9 / 4.2, 2931 6.5 / 5.7, 4000 7.9 / 7.1, 6000 10.0 / 10.0, 8190 12.9 / 13.1; 1000 columns top-3 with shared
-// rows 7.5 / 5.8, 9.1 / 7.4, 10.4 / 9.0, 13.2 / 12.7, 16.6 / 17.2.
-constexpr int64_t kSplitMaxWaves = 16384;
+// 16384 of 1024 columns top-2 17.0 / 17.7.  Rows of two waves for one round only: beyond, it is worth 3 % either way.  In
+// turn on one box, cold, at 1200, 2000, 2931, 4000, 6000 and 8190 tokens: 1024 columns top-2 with shared rows 4.9 / 4.2, 5.5 /
+// 4.9, 6.5 / 5.7, 7.9 / 7.1, 10.0 / 10.0, 12.9 / 13.1; 1000 columns top-3 with shared rows 7.5 / 5.8, 8.0 / 6.4, 9.1 / 7.4, 10.4
+// / 9.0, 13.2 / 12.7, 16.6 / 17.2; 640 columns top-8 7.1 / 5.5, 8.0 / 6.9, 9.7 / 8.3, 11.5 / 10.6, 15.6 / 15.0, 20.3 / 19.2.
+constexpr int64_t kSplitMaxWaves = 16384, kSplitMaxHalfRowWaves = 8192;
 
 // residual == nullptr: plain combine; otherwise the fused post-norm + residual variant
 int combine_launch(const char* what, const void* packed_y, const int32_t* inverse, const void* weights,
@@ -290,7 +291,7 @@ int combine_launch(const char* what, const void* packed_y, const int32_t* invers
   if (vec) {
     const int row_vecs = (int)(H / 8);
     const int nv = (row_vecs + 63) / 64;
-    const bool split = nv > 1 && T * nv <= kSplitMaxWaves;
+    const bool split = nv > 1 && T * nv <= (nv > 2 ? kSplitMaxWaves : kSplitMaxHalfRowWaves);
     const dim3 block(64, split ? nv : 4);
     const int grid = (int)(split ? T : (T + 3) / 4);
 #define JT_COMBINE_N(NV, KT, NORM, SPLIT)                                                                   \
