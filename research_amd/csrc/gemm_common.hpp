@@ -332,15 +332,15 @@ inline HalfTiles half_tiles(int64_t rows, int64_t E, bool dense, int64_t N, doub
 // 5 %); else plain ones.  By the spread of the groups, where they spare rounds enough for the time a taller tile takes: 1.2 of a
 // plain one, 1.25 for one data gradient alone, which has to spare a tenth of the tiles as well, and for products of one output
 // beside dense tiles, which fill the last round of either, unless the tiles themselves are fewer by as much.  us, plain /
-// taller (rounds): 64 groups of 256 rows, 2048 x 1408, gate/up 262 / 213, down 128 / 119, dX 247 / 239; of 328 gate/up 294 /
-// 288 (6, 5), beside shared tiles down 208 / 218 and dX 346 / 369 (5, 4; by tiles 4.3, 3.4); of 256, gate/up beside shared
-// tiles, the forward pass 493 / 460 (5, 4; 4.8, 3.4); of 512 down 212 / 189 and dX 419 / 356 (5, 4), dZ 229 / 200 (4, 3), but
-// gate/up, which the line leaves out, 383 / 336 (7, 6); dZ of 64 groups of 600 258 / 265, of 40 of 1638, 1304 x 904, 233 / 235 (5,
-// 4), of 24 of 698, 1000 x 2664, 134 / 138 (4, 3, with 94 % of the tiles).
+// taller (rounds), of passes without a pause: 64 groups of 256 rows, 2048 x 1408, gate/up 267 / 209, down 158 / 116, dX 305 /
+// 208 (5, 3 and 3, 2); of 328 gate/up 310 / 303 (6, 5), beside shared tiles down 188 / 202 and dX 352 / 373 (5, 4; by tiles
+// 4.3, 3.4); of 256, gate/up beside shared tiles 289 / 253 (5, 4; 4.8, 3.4); of 512 down 227 / 208 and dX 429 / 357 (5, 4), dZ
+// 235 / 203 (4, 3), but gate/up, which the line leaves out, 408 / 377 (7, 6); dZ of 64 groups of 600 271 / 271, of 40 of 1638,
+// 1304 x 904, 234 / 230 (5, 4), of 24 of 698, 1000 x 2664, 129 / 134 (4, 3, with 94 % of the tiles).
 // With eight rounds and more the tiles that are left count, and the kernel decides from the real sizes: 64 groups of 698 rows
-// (94 % of the tiles) gate/up 471 / 487, of 1024 (85 %) 700 / 652, down 403 / 392 and dX 782 / 700, of 2048 (88 %) 1287 / 1248,
-// 744 / 736 and 1361 / 1307; 128 skewed groups of 688 (93 %), 2048 x 768, down 341 / 357, dX 591 / 606, of 1024 (85 %) dX 835 /
-// 817.  Beside shared tiles, where the plain kernel is slower too, always: 64 groups of 698 590 / 581.
+// (94 % of the tiles) gate/up 509 / 542, of 1024 (85 %) 746 / 693, down 438 / 411 and dX 783 / 740, of 2048 (88 %) 1369 / 1314,
+// 792 / 755 and 1382 / 1343; 128 skewed groups of 750 (88 %), 2048 x 768, down 392 / 379, dX 625 / 635, of 1024 (85 %) dX 827 /
+// 829.  Beside shared tiles, where the plain kernel is slower too, always: 64 groups of 698 623 / 603.
 // k128x128Pair: two workgroups to a CU.
 enum class TileShape { k64x64, k128x64, k128x128, k128x128Short, k128x128Pair, k256x128, k128x256, kTall, kPlain };
 enum class Product { kGateUp, kDown, kGradient, kGradientPair };  // the last: of two segments

@@ -613,11 +613,11 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_joint_nt_kernel(
 // 2048: gate/up 71.6 / 72.9.  Eight waves of 128 x 64: with 64 x 128 there is no room for a block more per wave.
 //
 // Against 256 rows and a tile of its own for what is left of each group (uneven groups by random routing; us, before /
-// now; both products of a layer call alone, matrices not in the caches):
-//   16384 rows in 64 groups, 2048 x 1408    gate/up 271 / 213, down 134 / 117, dZ 161 / 149, dX 253 / 220
-//   16384 rows in 16 groups, 1024 x 2816    gate/up 195 / 196, down 131 (half tiles 110) / 87, dZ 116 / 107, dX 250 / 175
-//   8192 rows in 8 groups, 1024 x 2048      gate/up 80 / 72, dZ 54 / 40
-//   131072 rows in 64 groups, 2048 x 1408   gate/up 1343 / 1313, down 757 / 730, dZ 748 / 743, dX 1392 / 1347
+// now; both products of a layer call alone, matrices not in the caches; gradients in a training pass):
+//   16384 rows in 64 groups, 2048 x 1408    gate/up 271 / 213, down 134 / 117, dZ 151 (half tiles) / 137, dX 312 / 209
+//   16384 rows in 16 groups, 1024 x 2816    gate/up 195 / 196, down 131 (half tiles 110) / 87, dZ 113 / 104, dX 280 / 169
+//   8192 rows in 8 groups, 1024 x 2048      gate/up 80 / 72
+//   131072 rows in 64 groups, 2048 x 1408   gate/up 1343 / 1313, down 757 / 730, dZ 728 / 697, dX 1335 / 1261
 // (Bound by the matrix cores at the power limit at 131072 rows, by rounds over the CUs at the others.)
 using GateUpStreamCfg = DmaGemmCfg<256, 128, 64, 2, 4, true, 2, 16 + 128 + 131072>;
 using GateUpStreamTailCfg = DmaGemmCfg<256, 128, 64, 2, 4, true, 2, 16 + 128 + 65536 + 131072>;
